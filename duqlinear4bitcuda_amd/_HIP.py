@@ -36,6 +36,13 @@ def _launch(dev: torch.device, fn, *args):
         return fn(*args, _raw_stream(idx))
 
 
+def _host_for(entry: str):
+    """The native host module (csrc/duq_host.cpp) for calls that end in that entry point, or None where the function
+    on the loaded library was replaced by a Python one (a tracer's): the call then goes through that."""
+    lib = _lib.load()
+    return _lib.host() if type(getattr(lib, entry)) is lib._FuncPtr else None
+
+
 def _fast_check(name, what, t, dtype, dev):
     """Contiguity / device / dtype check of one tensor of a fused op."""
     if t.dtype is not dtype or not t.is_cuda or not t.is_contiguous() or (dev is not None and t.device != dev):
@@ -291,10 +298,21 @@ def get_dual_quant_col_k() -> int:
 
 # ---- additions over the reference module: fused ops -----------------------------------
 
+def _quantize_native(entry, x, kind, with_q=True, shadow=False, clip=1.0, qmax=6):
+    """The row quantizers through the native host module; None for what it does not take."""
+    if type(x) is not torch.Tensor or not x.is_cuda:
+        return None
+    host = _host_for(entry)
+    return None if host is None else _launch(x.device, host.quantize_rows, x, kind, bool(with_q), shadow, float(clip), qmax)
+
+
 def quantize_rows_sym(x: torch.Tensor, clip: float = 1.0, qmax: int = 6):
     """One-pass SymQuantizer (qlinear4bit/nn/quantizer.py:10-16) over the last dimension of a
     contiguous fp16 tensor [..., K]: returns (q uint8 [..., K/2], scales fp16 [..., 1]).
     Requires K % 32 == 0."""
+    r = _quantize_native("duq_quantize_rows_sym", x, 0, True, False, clip, qmax)
+    if r is not None:
+        return r
     if not isinstance(x, torch.Tensor):
         raise RuntimeError("quantize_rows_sym: argument #0 is not a tensor")
     _fast_check("quantize_rows_sym", "x", x, _F16, None)
@@ -315,6 +333,9 @@ def quantize_rows_sym(x: torch.Tensor, clip: float = 1.0, qmax: int = 6):
 def quantize_rows_asym(x: torch.Tensor):
     """One-pass AsymQuantizer (qlinear4bit/nn/quantizer.py:24-35) over the last dimension:
     returns (q, scale [..., 1], zeros [..., 1]).  Requires K % 32 == 0."""
+    r = _quantize_native("duq_quantize_rows_asym", x, 1)
+    if r is not None:
+        return r
     if not isinstance(x, torch.Tensor):
         raise RuntimeError("quantize_rows_asym: argument #0 is not a tensor")
     _fast_check("quantize_rows_asym", "x", x, _F16, None)
@@ -338,6 +359,16 @@ EPI_ASYM_ROWSUM = 4        # exact zero-point correction with row sums; not in t
 EPI_ASYM_DUAL_ROWSUM = 5   # the same for the dual-uniform layer (one-launch decode entry point only)
 
 
+def _linear4_native(entry, mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias, rowsum_x=None,
+                    w_rowsum_adj=None, shadows=False):
+    """GEMM + dequant through the native host module; None for what it does not take."""
+    if type(xq) is not torch.Tensor or not xq.is_cuda:
+        return None
+    host = _host_for(entry)
+    return None if host is None else _launch(xq.device, host.linear4, mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2,
+                                             w_zeros_2, bias, rowsum_x, w_rowsum_adj, shadows)
+
+
 def linear4bit_forward(mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1=None, w_scale_2=None, w_zeros_2=None,
                        bias=None):
     """matmul + dequant (+ bias) in one launch; bit-identical to the separate ops.
@@ -345,6 +376,9 @@ def linear4bit_forward(mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1=None,
     [N, K/2]; per-row tensors hold M, per-column tensors N fp16 values in any contiguous
     shape.  Returns fp16 [..., N]."""
     name = "linear4bit_forward"
+    y = _linear4_native("duq_linear4bit_forward", mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias)
+    if y is not None:
+        return y
     if not isinstance(xq, torch.Tensor) or not isinstance(w, torch.Tensor):
         raise RuntimeError(f"{name}: xq and w must be tensors")
     dev = xq.device
@@ -391,6 +425,12 @@ def batch_linear4bit_forward(mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1
     per-row tensors n * M and per-column tensors (and bias) n * N fp16 values, contiguous over the batch.
     Returns fp16 [n, M, N], entry i bit-identical to ``linear4bit_forward`` on the i-th slices."""
     name = "batch_linear4bit_forward"
+    if type(xq) is torch.Tensor and xq.is_cuda:
+        host = _host_for("duq_batch_linear4bit_forward")
+        y = None if host is None else _launch(xq.device, host.linear4_batched, mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1,
+                                              w_scale_2, w_zeros_2, bias)
+        if y is not None:
+            return y
     if not isinstance(xq, torch.Tensor) or not isinstance(w, torch.Tensor):
         raise RuntimeError(f"{name}: xq and w must be tensors")
     dev = xq.device
@@ -571,7 +611,7 @@ class FusedDecode:
     a caller can tell when the layer's buffers were replaced; a change of their contents in place needs no new
     object."""
 
-    __slots__ = ("mode", "N", "K", "device", "index", "tensors", "w_ptr", "_fn", "_ptrs", "_structs", "_one", "_lib")
+    __slots__ = ("mode", "N", "K", "device", "index", "tensors", "w_ptr", "_fn", "_ptrs", "_structs", "_one", "_lib", "native")
 
     def __init__(self, mode, w, w_scale_1, w_zeros_1=None, w_scale_2=None, w_zeros_2=None, w_rowsum_adj=None,
                  w_rowsum_adj_2=None, bias=None):
@@ -612,6 +652,20 @@ class FusedDecode:
         self._ptrs = ptrs
         self._structs = {}
         self._one = {}
+        self.native = None
+
+    def prepare_native(self, names):
+        """Make ``native``, the same prepared call in native code (``FusedCall`` of csrc/duq_host.cpp: take() and
+        take_rows() of a module), for a module whose buffers ``names`` (the weight first) are the tensors this object
+        was made of, given as (name, tensor or None) pairs.  It answers None when the module's buffers have changed
+        and for every input that is not the plain case."""
+        if type(self._fn) is self._lib._FuncPtr:
+            p = self._ptrs
+            self.native = _lib.host().FusedCall(
+                self.mode, self.N, self.K, self.index, self.max_rows,
+                (self.w_ptr, p["w_scale_1"], p["w_zeros_1"], p["w_scale_2"], p["w_zeros_2"], p["w_rowsum_adj"],
+                 p["w_rowsum_adj_2"], p["bias"]), tuple(n for n, _ in names), tuple(t for _, t in names))
+        return self
 
     def _layer(self, clip, qmax):
         key = (clip, qmax)
@@ -690,6 +744,9 @@ def quantize_rows_asym_shifted(x: torch.Tensor):
     """AsymQuantizer with signed-shifted storage: the codes of ``quantize_rows_asym`` minus 8
     (signed nibbles), zero points minus 8, and the per-row sums of the shifted codes.
     Returns (q uint8 [..., K/2], scale [..., 1], zeros [..., 1], rowsum int32 [...])."""
+    r = _quantize_native("duq_quantize_rows_asym_shifted", x, 2)
+    if r is not None:
+        return r
     if not isinstance(x, torch.Tensor):
         raise RuntimeError("quantize_rows_asym_shifted: argument #0 is not a tensor")
     _fast_check("quantize_rows_asym_shifted", "x", x, _F16, None)
@@ -732,6 +789,10 @@ def linear4bit_forward_rowsum(xq, scale_x, zeros_x, rowsum_x, w, w_scale, w_zero
     y = s_x*s_w * (acc - z_x*w_rowsum_adj - z_w*rowsum_x), w_rowsum_adj = sum_k c_w - K*z_w.
     ``xq`` uint8 [..., K/2]; returns fp16 [..., N]."""
     name = "linear4bit_forward_rowsum"
+    y = _linear4_native("duq_linear4bit_forward_rowsum", EPI_ASYM_ROWSUM, xq, scale_x, zeros_x, w, w_scale, w_zeros, None, None, bias,
+                        rowsum_x, w_rowsum_adj)
+    if y is not None:
+        return y
     if not isinstance(xq, torch.Tensor) or not isinstance(w, torch.Tensor):
         raise RuntimeError(f"{name}: xq and w must be tensors")
     dev = xq.device
@@ -881,6 +942,10 @@ def linear4bit_forward_bf6(mode, x_bf6, scale_x, zeros_x, w_bf6, w_scale_1, w_ze
     shadows: ``x_bf6`` uint8 [..., 3K/4], ``w_bf6`` uint8 [ceil(N/32)*32, 3K/4] from weight_shadow_bf6, N taken
     from ``w_scale_1``.  Bit-identical results."""
     name = "linear4bit_forward_bf6"
+    y = _linear4_native("duq_linear4bit_forward_bf6", mode, x_bf6, scale_x, zeros_x, w_bf6, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2,
+                        bias, rowsum_x, w_rowsum_adj, True)
+    if y is not None:
+        return y
     if not isinstance(x_bf6, torch.Tensor) or not isinstance(w_bf6, torch.Tensor):
         raise RuntimeError(f"{name}: x_bf6 and w_bf6 must be tensors")
     dev = x_bf6.device
@@ -957,6 +1022,9 @@ def quantize_rows_sym_bf6(x: torch.Tensor, clip: float = 1.0, qmax: int = 6, wit
     """``quantize_rows_sym`` that also writes the E3M2 shadow of the codes: returns
     (q or None, x_bf6 uint8 [..., 3K/4], scales).  K % 128 == 0."""
     name = "quantize_rows_sym_bf6"
+    r = _quantize_native("duq_quantize_rows_sym_bf6", x, 0, with_q, True, clip, qmax)
+    if r is not None:
+        return r
     if not isinstance(x, torch.Tensor):
         raise RuntimeError(f"{name}: argument #0 is not a tensor")
     _fast_check(name, "x", x, _F16, None)
@@ -979,6 +1047,9 @@ def quantize_rows_asym_bf6(x: torch.Tensor, shifted: bool = False, with_q: bool 
     """``quantize_rows_asym`` (or ``quantize_rows_asym_shifted``) that also writes the E3M2
     shadow: returns (q or None, x_bf6, scale, zeros[, rowsum])."""
     name = "quantize_rows_asym_bf6"
+    r = _quantize_native("duq_quantize_rows_asym_bf6", x, 2 if shifted else 1, with_q, True)
+    if r is not None:
+        return r
     if not isinstance(x, torch.Tensor):
         raise RuntimeError(f"{name}: argument #0 is not a tensor")
     _fast_check(name, "x", x, _F16, None)
@@ -1055,6 +1126,11 @@ def asym_dequant_hprec(q, scale_row, zeros_row, scale_col, zeros_col, bits: int 
 def quantize_rows_asym_8bit(x: torch.Tensor):
     """One-pass AsymQuantizer8bit (qlinear4bit/nn/quantizer.py:38-55) over the last dimension:
     (q int8 [..., K], scale [..., 1], zeros [..., 1]) float32.  Requires K % 4 == 0."""
+    if type(x) is torch.Tensor and x.is_cuda:
+        host = _host_for("duq_quantize_rows_asym_8bit")
+        r = None if host is None else _launch(x.device, host.quantize_rows_8bit, x)
+        if r is not None:
+            return r
     if not isinstance(x, torch.Tensor):
         raise RuntimeError("quantize_rows_asym_8bit: argument #0 is not a tensor")
     _fast_check("quantize_rows_asym_8bit", "x", x, _F32, None)
@@ -1088,6 +1164,13 @@ def linear8bit_forward(xq, scale_x, zeros_x, w, w_scale, w_zeros, bias=None, til
     """matmul_8bit + asym_dequant_hprec (+ bias) in one launch; xq [..., K] int8 -> float32 [..., N].
     ``w`` is the weight [N, K], or with ``tiled_rows=N`` its tiled copy from weight_tile_8bit (same bits)."""
     name = "linear8bit_forward"
+    if type(xq) is torch.Tensor and xq.is_cuda and type(w) is torch.Tensor and isinstance(scale_x, torch.Tensor):
+        host = _host_for("duq_linear8bit_forward" if tiled_rows is None else "duq_linear8bit_forward_tiled")
+        y = None if host is None else _launch(xq.device, host.linear8, xq, scale_x, zeros_x, w if tiled_rows is None else None,
+                                              None if tiled_rows is None else w, w_scale, w_zeros, bias,
+                                              w.shape[0] if tiled_rows is None else int(tiled_rows))
+        if y is not None:
+            return y
     if not isinstance(xq, torch.Tensor):
         raise RuntimeError(f"{name}: argument #0 is not a tensor")
     dev = xq.device
@@ -1127,6 +1210,11 @@ def quantize_linear8bit_forward(x, w, w_tiled, w_scale, w_zeros, bias=None):
     allocated here): x float32 [..., K] -> float32 [..., N], the bits of the two calls.  ``w`` the weight [N, K]
     int8, ``w_tiled`` its tiled copy from weight_tile_8bit or None."""
     name = "quantize_linear8bit_forward"
+    if type(x) is torch.Tensor and x.is_cuda and type(w) is torch.Tensor and w.dim() == 2:
+        host = _host_for("duq_quantize_linear8bit_forward")
+        y = None if host is None else _launch(x.device, host.linear8, x, None, None, w, w_tiled, w_scale, w_zeros, bias, w.shape[0])
+        if y is not None:
+            return y
     if not isinstance(x, torch.Tensor) or not isinstance(w, torch.Tensor):
         raise RuntimeError(f"{name}: x and w must be tensors")
     dev = x.device

@@ -11,6 +11,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libduq_hip.so")
+HOST_PATH = os.path.join(_HERE, "_duq_host.so")
 
 _c_u32 = ctypes.c_uint32
 _c_i32 = ctypes.c_int32
@@ -118,6 +119,23 @@ def load():
     lib.duq_status_string.restype = ctypes.c_char_p
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The native module of the host side (``csrc/duq_host.cpp``, built beside the library), imported once."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(f"{HOST_PATH} is missing: build it with `python -m duqlinear4bitcuda_amd.build`")
+        from . import _duq_host
+        from .tools.tensor_utils import PackedQuantizedTensor
+        _duq_host.setup(PackedQuantizedTensor, check)
+        _host = _duq_host
+    return _host
 
 
 def check(status: int, what: str):

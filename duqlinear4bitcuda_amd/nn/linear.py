@@ -74,7 +74,7 @@ class _Linear4bitBase(torch.nn.Module):
         held = tuple((buf, b.get(buf)) for _, buf in names)
         if not held[0][1].is_cuda:
             return None
-        d = self._decode = _ops.FusedDecode(spec[0], **{arg: t for (arg, _), (_, t) in zip(names, held)})
+        d = self._decode = _ops.FusedDecode(spec[0], **{arg: t for (arg, _), (_, t) in zip(names, held)}).prepare_native(held)
         self._decode_held = held
         return d
 
@@ -99,6 +99,11 @@ class _Linear4bitBase(torch.nn.Module):
     def _take_deferred(self, x):
         """A PackedQuantizedTensor that SymQuantizer handed on unquantized: the result of the one-call path, or None
         after quantizing it now (with the 6-bit float shadow when this layer will take that path)."""
+        d = self._decode
+        if d is not None and d.native is not None and self.fused:   # everything in native code; None: not the plain case
+            y = d.native.take(self._buffers, x)
+            if y is not None:
+                return y
         y = self._decode_forward(x.source(), x._clip, x._qmax, True)
         if y is None:
             src = x._src
@@ -144,6 +149,11 @@ class _Linear4bitBase(torch.nn.Module):
     def _own_quantizer_decode(self, x):
         """Layers with their own AsymQuantizer: a few contiguous binary16 rows on the GPU run quantizer + GEMM +
         dequant as one launch (the quantizer inside the GEMM kernel, same bits); None for anything else."""
+        d = self._decode
+        if d is not None and d.native is not None and self.fused:
+            y = d.native.take_rows(self._buffers, x)
+            if y is not None:
+                return y
         if type(x) is not torch.Tensor or x.dtype is not torch.float16 or not x.is_cuda or not x.is_contiguous() or \
                 x.data_ptr() % 16:
             return None

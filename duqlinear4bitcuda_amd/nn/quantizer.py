@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import torch
 
+from .. import _lib
 from ..tools import tensor_utils
 
 
@@ -46,6 +47,10 @@ class SymQuantizer(torch.nn.Module):
         self.shadow_min_rows = shadow_min_rows
 
     def forward(self, x, shadow=None) -> tensor_utils.PackedQuantizedTensor:
+        if shadow is None:   # the rule below in native code; None: not a plain case of it
+            p = _lib.host().defer(x, self.defer_rows, self.shadow, self.shadow_min_rows, self.input_clip_ratio, self.qmax)
+            if p is not None:
+                return p
         if not x.is_contiguous():
             x = x.contiguous()
         cols = x.shape[-1]

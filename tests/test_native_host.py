@@ -1,0 +1,60 @@
+"""The native host module (csrc/duq_host.cpp): it answers None for what it does not take, and where it does, the bits are
+those of the Python code that stands behind it."""
+import pytest
+import torch
+
+
+def test_declines_what_is_not_the_plain_case():
+    from duqlinear4bitcuda_amd import _lib
+
+    host = _lib.host()
+    x = torch.zeros(2, 128, dtype=torch.float16)                       # on the CPU
+    assert host.defer(x, 1024, False, 96, 1.0, 6) is None and host.defer(None, 1024, False, 96, 1.0, 6) is None
+    assert host.quantize_rows(x, 0, True, False, 1.0, 6, 0) is None
+    assert host.linear4(0, x, x, None, x, x, None, None, None, None, None, None, False, 0) is None
+    assert host.linear4_batched(0, x, x, None, x, x, None, None, None, None, 0) is None
+    assert host.linear8(x, None, None, x, None, x, x, None, 2, 0) is None and host.quantize_rows_8bit(x, 0) is None
+    w = torch.zeros(4, 64, dtype=torch.uint8)
+    call = host.FusedCall(0, 4, 128, 0, 1024, (w.data_ptr(),) + (None,) * 7, ("weight",), (w,))
+    assert call.take({"weight": w}, x) is None and call.take_rows({"weight": w}, x) is None
+    with pytest.raises(ValueError):
+        host.FusedCall(0, 4, 128, 0, 1024, (None,), ("weight",), (w,))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 9, 65, 1025])
+def test_native_and_python_host_code_give_the_same_bits(dev, monkeypatch, rows):
+    """The same module steps once natively and once with every library function replaced by a Python one."""
+    from duqlinear4bitcuda_amd import _lib
+    from duqlinear4bitcuda_amd import nn as qnn
+
+    K, N = 256, 96
+    gen = torch.Generator().manual_seed(rows)
+    lin = torch.nn.Linear(K, N, bias=True).half().to(dev).requires_grad_(False)
+    sw = lin.weight.abs().amax(1, keepdim=True) / 7
+    x = torch.randn(rows, K, generator=gen).half().to(dev)
+    b = torch.randn(3, 17, K, generator=gen).half().to(dev)
+
+    def steps():
+        sq = torch.nn.Sequential(qnn.SymQuantizer(0.95), qnn.Linear4bitSQ.from_float(lin, sw).to(dev))
+        fp6 = torch.nn.Sequential(qnn.SymQuantizer(shadow="only", shadow_min_rows=1), qnn.Linear4bitSQ.from_float(lin, sw).to(dev).enable_fp6())
+        fp6[1].fp6_min_tiles = 0
+        mods = [sq, fp6] + [c.from_linear(lin).to(dev) for c in (qnn.Linear4bitASQ, qnn.Linear4bitASQRowSum, qnn.LinearQuant4bitDUASQRowSum)]
+        out = [m(x) for m in mods for _ in range(2)]
+        l8 = qnn.LinearQuant8bitASQ.from_linear(lin.float()).to(dev)
+        lin.half()
+        for tiled in (True, False):
+            l8.tiled = tiled
+            out.append(l8(x.float()))
+        return out + [qnn.SymQuantMatMul()(b, b), qnn.AsymQuantMatMul()(b, b)]
+
+    native = steps()
+    lib, calls = _lib.load(), []
+    for name in _lib.PROTOTYPES:
+        if not name.endswith("_bytes"):
+            real = getattr(lib, name)
+            monkeypatch.setattr(lib, name, (lambda *a, _r=real, _n=name: (calls.append(_n), _r(*a))[1]), raising=False)
+    python = steps()
+    assert len(calls) >= len(python) and len(python) == len(native)
+    for p, n in zip(python, native):
+        assert p.dtype == n.dtype and p.shape == n.shape and torch.equal(p, n)
