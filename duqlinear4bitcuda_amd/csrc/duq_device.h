@@ -120,6 +120,19 @@ __device__ __forceinline__ T wave_reduce_dpp(T v, OP op)
     const T d = __builtin_bit_cast(T, (uint32_t)__builtin_amdgcn_readlane((int)bits, 48));
     return op(op(a, b), op(c, d));
 }
+// The same over aligned groups of N lanes (N = 4, 8, 16, 32 or 64), each group its own value in all its lanes.
+template <int N, typename OP>
+__device__ __forceinline__ uint32_t group_reduce(uint32_t v, OP op)
+{
+    static_assert(N == 4 || N == 8 || N == 16 || N == 32 || N == 64, "lanes per group");
+    v = op(v, dpp_get<0xB1>(v));
+    v = op(v, dpp_get<0x4E>(v));
+    if (N >= 8) v = op(v, dpp_get<0x141>(v));
+    if (N >= 16) v = op(v, dpp_get<0x140>(v));
+    if (N >= 32) v = op(v, (uint32_t)__shfl_xor((int)v, 16, kWave));
+    if (N >= 64) v = op(v, (uint32_t)__shfl_xor((int)v, 32, kWave));
+    return v;
+}
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
 {
     return wave_reduce_dpp(v, [](uint32_t x, uint32_t y) { return max(x, y); });

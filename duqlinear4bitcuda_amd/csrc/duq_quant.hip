@@ -407,10 +407,115 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
     }
 }
 
+// Short rows (at most 512 elements, no shadow: the operands of quantized attention).  With a workgroup per row such a
+// launch is bound by how fast workgroups start (65536 rows of 128 elements, asymmetric: 21.4 us for 21 MB, a quarter of a workgroup's
+// lanes at work).  Here LANES lanes hold a row, two units each, a workgroup takes 256 / LANES rows at a time and PASSES
+// times as many in all, every load of them requested up front; the same launch takes 7.4 us.  Two units per lane, not
+// one, because the constants of a row are computed by each of its lanes and cost as much as two units' codes.
+template <int LANES, int PASSES, bool ASYM>
+__global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL, RowParams tail)
+{
+    RowParams p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.x);
+    to_global(p.q);
+    to_global(p.scale);
+    to_global(p.zeros);
+    constexpr uint32_t kRows = 256 / LANES;
+    const bool shifted = ASYM && p.rowsum != nullptr;
+    const uint32_t nunits = p.cols >> 3;  // <= 2 * LANES
+    const uint32_t u0 = threadIdx.x % LANES, row0 = blockIdx.x * (kRows * PASSES) + threadIdx.x / LANES;
+    const v4u *x4 = reinterpret_cast<const v4u *>(p.x);
+    uint32_t *q32 = reinterpret_cast<uint32_t *>(p.q);
+
+    v4u regs[PASSES][2];
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t row = row0 + i * kRows, u = u0 + j * LANES;
+            regs[i][j] = row < p.rows && u < nunits ? __builtin_nontemporal_load(&x4[(uint64_t)row * nunits + u]) : v4u{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        const uint32_t row = row0 + i * kRows;
+        PkMinMax st;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            if (u0 + j * LANES < nunits) st.add8(regs[i][j]);
+        float a = 0.f, b = 0.f;
+        uint32_t m16;
+        if (!ASYM) {
+            m16 = group_reduce<LANES>(st.absmax_bits(), [](uint32_t x, uint32_t y) { return max(x, y); });
+        } else {
+            st.mx = group_reduce<LANES>(st.mx, [](uint32_t x, uint32_t y) {
+                asm("v_pk_maximum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
+                return x;
+            });
+            st.mn = group_reduce<LANES>(st.mn, [](uint32_t x, uint32_t y) {
+                asm("v_pk_minimum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
+                return x;
+            });
+            m16 = st.absmax_bits();
+            a = st.min_f32();
+            b = st.max_f32();
+            if (m16 > 0x7C00u) a = b = __builtin_nanf("");  // torch's min / max return NaN for a row that holds one
+        }
+        RowQuant<ASYM, false> rq;
+        rq.init(m16, a, b, p.clip, p.qmax);
+        uint32_t w[2];
+        rq.quant_units(regs[i], w);
+        if (shifted) {  // uniform branch: see quantize_rows_kernel
+            uint32_t sum = 0;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t pairs = (w[j] & 0x0F0F0F0Fu) + ((w[j] >> 4) & 0x0F0F0F0Fu);
+                if (u0 + j * LANES < nunits) sum = __builtin_amdgcn_udot4(pairs, 0x01010101u, sum, false);
+                w[j] ^= 0x88888888u;
+            }
+            sum = group_reduce<LANES>(sum, [](uint32_t x, uint32_t y) { return x + y; });
+            if (u0 == 0 && row < p.rows) p.rowsum[row] = (int)sum - 8 * (int)p.cols;
+        }
+        if (row < p.rows) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                if (u0 + j * LANES < nunits) DUQ_QSTORE(&q32[(uint64_t)row * nunits + u0 + j * LANES], w[j]);
+            if (u0 == 0) {
+                p.scale[row] = f16_to_bits(rq.s);
+                if (ASYM) p.zeros[row] = f16_to_bits(shifted ? rq.z - (f16)8.0f : rq.z);
+            }
+        }
+    }
+}
+
+template <bool ASYM>
+static int launch_short_rows(const RowParams &p, hipStream_t stream)
+{
+    // four passes where that still leaves two workgroups per CU, one otherwise (few rows: latency)
+#define DUQ_SHORT(L)                                                                                                  \
+    do {                                                                                                              \
+        const uint64_t groups = ((uint64_t)p.rows * L + 255) / 256;                                                   \
+        if (groups >= 2048)                                                                                           \
+            DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, 4, ASYM>), dim3((uint32_t)((groups + 3) / 4)), dim3(256), 0, stream, p); \
+        else                                                                                                          \
+            DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, 1, ASYM>), dim3((uint32_t)groups), dim3(256), 0, stream, p); \
+    } while (0)
+    if (p.cols <= 64)
+        DUQ_SHORT(4);
+    else if (p.cols <= 128)
+        DUQ_SHORT(8);
+    else if (p.cols <= 256)
+        DUQ_SHORT(16);
+    else
+        DUQ_SHORT(32);
+#undef DUQ_SHORT
+    return (int)hipGetLastError();
+}
+
 template <bool ASYM>
 static int launch_rows(const RowParams &p, hipStream_t stream)
 {
     if (p.rows == 0 || p.cols == 0) return 0;
+    if (p.cols <= 512 && !p.bf6) return launch_short_rows<ASYM>(p, stream);
     const uint32_t nunits = p.cols / 8;
     const dim3 grid(p.rows);
     // Wavefronts per row: enough that a lane holds at most `per_lane` units.  Four units per

@@ -80,7 +80,10 @@ __device__ __forceinline__ uint32_t quant8_exact(const v4u raw, float rcp, int q
 }
 
 // Statistics of one row -> scale, zero point and everything the quantization step needs.
-template <bool ASYM>
+// UNIFORM: all lanes of a wavefront hold the same row.  Otherwise a wavefront holds several rows, and one path is
+// taken for all of them: the element-wise one if a row of them needs it (it is right for every row), a clamp if a row
+// needs it (it changes nothing in one that does not).
+template <bool ASYM, bool UNIFORM = true>
 struct RowQuant {
     f16 s, z;
     float rcp, rcp_fast;
@@ -168,11 +171,16 @@ struct RowQuant {
             clamp_lo = false;
             clamp_hi = !(t + (float)zi <= 15.f);
         }
-        // every lane of a wavefront holds the same row statistics: tell the compiler, so that the choice of
-        // path is a scalar branch
-        fast = __builtin_amdgcn_readfirstlane((int)fast) != 0;
-        clamp_lo = __builtin_amdgcn_readfirstlane((int)clamp_lo) != 0;
-        clamp_hi = __builtin_amdgcn_readfirstlane((int)clamp_hi) != 0;
+        // (wavefront-uniform values either way: the choice of path is a scalar branch)
+        if (UNIFORM) {
+            fast = __builtin_amdgcn_readfirstlane((int)fast) != 0;
+            clamp_lo = __builtin_amdgcn_readfirstlane((int)clamp_lo) != 0;
+            clamp_hi = __builtin_amdgcn_readfirstlane((int)clamp_hi) != 0;
+        } else {
+            fast = __builtin_amdgcn_ballot_w64(!fast) == 0;
+            clamp_lo = __builtin_amdgcn_ballot_w64(clamp_lo) != 0;
+            clamp_hi = __builtin_amdgcn_ballot_w64(clamp_hi) != 0;
+        }
         lo2 = ASYM ? v2h{(f16)(float)(-zi), (f16)(float)(-zi)} : v2h{(f16)-8.0f, (f16)-8.0f};
         hi2 = ASYM ? v2h{(f16)(float)(15 - zi), (f16)(float)(15 - zi)} : v2h{(f16)(float)qmax, (f16)(float)qmax};
         zadd = ASYM ? (((uint32_t)zi & 0xFFFFu) * 0x00010001u) : 0u;
