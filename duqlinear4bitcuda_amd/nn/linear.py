@@ -9,6 +9,10 @@ asymmetric layers; optional ``bias`` [N].
 """
 from __future__ import annotations
 
+import contextlib
+import functools
+import threading
+
 import torch
 
 from .. import _HIP as _ops
@@ -19,8 +23,25 @@ from .quantizer import AsymQuantizer, AsymQuantizer8bit, SymQuantizer  # noqa: F
 _INT4_LEVELS = 2 ** 4
 
 
-def _placeholder_weight(out_features, in_features):
-    return torch.randint(1, 7, (out_features, in_features // 2), dtype=torch.uint8, requires_grad=False)
+_making = threading.local()
+
+
+def _placeholder_weight(shape, dtype):
+    """What a layer holds until weights are put in: small random codes, as in the reference."""
+    if getattr(_making, "unfilled", False):
+        return torch.empty(shape, dtype=dtype)
+    return torch.randint(1, 7, shape, dtype=dtype, requires_grad=False)
+
+
+def _unfilled(cls, *args, device=None, **kwargs):
+    """A layer (on ``device``) whose whole weight the caller writes: without the random codes (14 of the 15 ms that
+    converting a 4096 x 4096 layer took were the host's random numbers)."""
+    _making.unfilled = True
+    try:
+        with contextlib.nullcontext() if device is None else torch.device(device):
+            return cls(*args, **kwargs)
+    finally:
+        _making.unfilled = False
 
 
 def _asym_params(w: torch.Tensor):
@@ -173,7 +194,7 @@ class Linear4bitSQ(_Linear4bitBase):
         self.in_features = in_features
         self.out_features = out_features
         self.register_buffer("weight_scales", torch.zeros((out_features, 1), requires_grad=False))
-        self.register_buffer("weight", _placeholder_weight(out_features, in_features))
+        self.register_buffer("weight", _placeholder_weight((out_features, in_features // 2), torch.uint8))
         if bias:
             self.register_buffer("bias", torch.zeros((out_features), dtype=dtype))
         else:
@@ -202,8 +223,8 @@ class Linear4bitSQ(_Linear4bitBase):
         """Quantize ``module.weight`` with the given per-row scales: round(W / s), no clamp
         (pack_i4 rejects values outside [-8, 7]) (linear.py:58-78)."""
         w = module.weight.data
-        new = Linear4bitSQ(module.in_features, module.out_features, bias=module.bias is not None,
-                           dtype=w.dtype).to(w.dtype)
+        make = Linear4bitSQ if weight_scales is None else functools.partial(_unfilled, Linear4bitSQ)
+        new = make(module.in_features, module.out_features, bias=module.bias is not None, dtype=w.dtype).to(w.dtype)
         if weight_scales is not None:
             assert weight_scales.shape == (module.out_features, 1), "weight_scales should have shape (out_features, 1)"
             new.weight_scales.copy_(weight_scales.to(w.dtype))
@@ -224,7 +245,7 @@ class Linear4bitASQ(_Linear4bitBase):
         self.require_quantizer = require_quantizer
         self.register_buffer("weight_scales", torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float16))
         self.register_buffer("weight_zeros", torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float16))
-        self.register_buffer("weight", _placeholder_weight(out_features, in_features))
+        self.register_buffer("weight", _placeholder_weight((out_features, in_features // 2), torch.uint8))
         if bias:
             self.register_buffer("bias", torch.zeros((out_features), dtype=torch.float16))
         else:
@@ -254,8 +275,8 @@ class Linear4bitASQ(_Linear4bitBase):
 
     @classmethod
     def from_linear(cls, module: torch.nn.Linear, require_quantizer: bool = True):
-        new = cls(module.in_features, module.out_features, bias=module.bias is not None,
-                  require_quantizer=require_quantizer)
+        new = _unfilled(cls, module.in_features, module.out_features, bias=module.bias is not None,
+                        require_quantizer=require_quantizer)
         scale, zeros, codes = _asym_params(module.weight.data)
         new.weight.copy_(quant_utils.pack_i4(codes.to(torch.int8), sym=False))
         new.weight_scales.copy_(scale.to(torch.float16))
@@ -283,7 +304,7 @@ class Linear4bitASQRowSum(_Linear4bitBase):
         self.register_buffer("weight_scales", torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float16))
         self.register_buffer("weight_zeros", torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float16))
         self.register_buffer("weight_rowsum", torch.zeros((out_features,), requires_grad=False, dtype=torch.int32))
-        self.register_buffer("weight", _placeholder_weight(out_features, in_features))
+        self.register_buffer("weight", _placeholder_weight((out_features, in_features // 2), torch.uint8))
         if bias:
             self.register_buffer("bias", torch.zeros((out_features), dtype=torch.float16))
         else:
@@ -322,8 +343,8 @@ class Linear4bitASQRowSum(_Linear4bitBase):
         (the activation quantizer kernel, applied to the weight rows)."""
         w = module.weight.data
         assert w.is_cuda, "weight preparation runs on the GPU: move the layer there first"
-        new = cls(module.in_features, module.out_features, bias=module.bias is not None,
-                  require_quantizer=require_quantizer).to(w.device)
+        new = _unfilled(cls, module.in_features, module.out_features, bias=module.bias is not None,
+                        require_quantizer=require_quantizer, device=w.device)
         q, scale, zeros, rowsum = tensor_utils.quantize_asym_shifted(w.to(torch.float16).contiguous())
         new.weight.copy_(q)
         new.weight_scales.copy_(scale)
@@ -354,7 +375,7 @@ class LinearQuant4bitDUASQRowSum(_Linear4bitBase):
             self.register_buffer(f"weight_scales_{k}", torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float16))
             self.register_buffer(f"weight_zeros_{k}", torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float16))
             self.register_buffer(f"weight_rowsum_{k}", torch.zeros((out_features,), requires_grad=False, dtype=torch.int32))
-        self.register_buffer("weight", _placeholder_weight(out_features, in_features))
+        self.register_buffer("weight", _placeholder_weight((out_features, in_features // 2), torch.uint8))
         if bias:
             self.register_buffer("bias", torch.zeros((out_features), dtype=torch.float16))
         else:
@@ -407,7 +428,8 @@ class LinearQuant4bitDUASQRowSum(_Linear4bitBase):
         assert w.is_cuda, "weight preparation runs on the GPU: move the layer there first"
         K, split = module.in_features, tensor_utils.get_dual_quant_col()
         assert K > split and K % 2 == 0
-        new = cls(K, module.out_features, bias=module.bias is not None, require_quantizer=require_quantizer).to(w.device)
+        new = _unfilled(cls, K, module.out_features, bias=module.bias is not None, require_quantizer=require_quantizer,
+                        device=w.device)
         w = w.to(torch.float16)
         codes = []
         for k, (lo, hi) in enumerate(((0, split), (split, K)), start=1):
@@ -438,7 +460,7 @@ class Linear4bitDUSQ(_Linear4bitBase):
         self.out_features = out_features
         self.register_buffer("weight_scales_1", torch.zeros((out_features, 1), requires_grad=False))
         self.register_buffer("weight_scales_2", torch.zeros((out_features, 1), requires_grad=False))
-        self.register_buffer("weight", _placeholder_weight(out_features, in_features))
+        self.register_buffer("weight", _placeholder_weight((out_features, in_features // 2), torch.uint8))
         if bias:
             self.register_buffer("bias", torch.zeros((out_features), dtype=dtype))
         else:
@@ -465,8 +487,8 @@ class Linear4bitDUSQ(_Linear4bitBase):
     @staticmethod
     def from_float(module: torch.nn.Linear, weight_scales_1=None, weight_scales_2=None):
         w = module.weight.data
-        new = Linear4bitDUSQ(module.in_features, module.out_features, bias=module.bias is not None,
-                             dtype=w.dtype).to(w.dtype)
+        make = Linear4bitDUSQ if weight_scales_1 is None or weight_scales_2 is None else functools.partial(_unfilled, Linear4bitDUSQ)
+        new = make(module.in_features, module.out_features, bias=module.bias is not None, dtype=w.dtype).to(w.dtype)
         if weight_scales_1 is not None and weight_scales_2 is not None:
             shape = (module.out_features, 1)
             assert weight_scales_1.shape == shape, "weight_scales_1 should have shape (out_features, 1)"
@@ -493,7 +515,7 @@ class LinearQuant4bitDUASQ(_Linear4bitBase):
         self.require_quantizer = require_quantizer
         for name in ("weight_scales_1", "weight_zeros_1", "weight_scales_2", "weight_zeros_2"):
             self.register_buffer(name, torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float16))
-        self.register_buffer("weight", _placeholder_weight(out_features, in_features))
+        self.register_buffer("weight", _placeholder_weight((out_features, in_features // 2), torch.uint8))
         if bias:
             self.register_buffer("bias", torch.zeros((out_features), dtype=torch.float16))
         else:
@@ -528,8 +550,8 @@ class LinearQuant4bitDUASQ(_Linear4bitBase):
 
     @classmethod
     def from_linear(cls, module: torch.nn.Linear, require_quantizer=True):
-        new = cls(module.in_features, module.out_features, bias=module.bias is not None,
-                  require_quantizer=require_quantizer)
+        new = _unfilled(cls, module.in_features, module.out_features, bias=module.bias is not None,
+                        require_quantizer=require_quantizer)
         w = module.weight.data
         split = tensor_utils.get_dual_quant_col()
         s1, z1, c1 = _asym_params(w[:, :split])
@@ -571,8 +593,7 @@ class LinearQuant8bitASQ(torch.nn.Module):
         self.require_quantizer = require_quantizer
         self.register_buffer("weight_scales", torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float32))
         self.register_buffer("weight_zeros", torch.zeros((out_features, 1), requires_grad=False, dtype=torch.float32))
-        self.register_buffer("weight", torch.randint(1, 7, (out_features, in_features), dtype=torch.int8,
-                                                     requires_grad=False))
+        self.register_buffer("weight", _placeholder_weight((out_features, in_features), torch.int8))
         if bias:
             self.register_buffer("bias", torch.zeros((out_features), dtype=torch.float32))
         else:
@@ -613,8 +634,8 @@ class LinearQuant8bitASQ(torch.nn.Module):
     def from_linear(cls, module: torch.nn.Linear, require_quantizer: bool = True):
         """Per-row scale / zero over |W| with 127 steps, codes clamp(round(W / s) + z, 0, 127)
         (linear.py:338-368)."""
-        new = cls(module.in_features, module.out_features, bias=module.bias is not None,
-                  require_quantizer=require_quantizer)
+        new = _unfilled(cls, module.in_features, module.out_features, bias=module.bias is not None,
+                        require_quantizer=require_quantizer)
         w = module.weight.data
         levels = 2 ** 7
         aw = w.abs()
