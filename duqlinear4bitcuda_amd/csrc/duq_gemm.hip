@@ -10,14 +10,12 @@
 // 256*|C| stays below 2^31 for K <= 131008.  Integer accumulation is order-free, so the
 // k order inside a tile only has to be the same for A and B.
 //
-// Six kernels here, picked by shape in select_gemm_kernel() (up to 64 rows run the two kernels of
-// duq_decode.hip as far as they reach):
-//  * stream kernel (prefill, more than 64 rows; tiles of 128, 64 or 32 rows x 256 columns or of 128 or 64 rows x
-//    128, the shape picked per problem): weights go from global memory straight to registers, activations are
-//    expanded once into LDS, v_mfma_i32_32x32x32_i8 with a hand-ordered schedule (see the kernel);
-//  * short-row kernel (rows of at most 256 elements): the stream kernel's tile without its K pipeline;
-//  * tile kernel (what is left, and any tensor of 4 GiB or more): BM x BN x 128 tiles, 4 wavefronts (2 x 2),
-//    both operands expanded on the way into double-buffered LDS, v_mfma_i32_16x16x64_i8;
+// Five kernels here, and the prefill kernel in duq_prefill.hip, picked by shape in select_gemm_kernel() (up to 64 rows
+// run the two kernels of duq_decode.hip as far as they reach):
+//  * prefill kernel (duq_prefill.hip): more than 64 rows, long rows, tensors of 4 GiB or more, what is left;
+//  * stream kernel (the same shapes where rows are short): 64 x 128 tiles, weights from global memory straight to
+//    registers, activations expanded once into LDS, v_mfma_i32_32x32x32_i8 with a hand-ordered schedule;
+//  * short-row kernel (rows of at most 256 elements): the stream kernel's operand paths without its K pipeline;
 //  * ring kernel (17 <= M <= 256 on narrow problems or long rows, and 5..16 rows of 12289..16384 elements):
 //    packed activations of all rows in LDS, every wavefront streams whole weight rows through a ring of loads;
 //  * skinny kernel (9 <= M <= 16 with 1536 or more column tiles): one workgroup owns 16 output columns, its
@@ -26,9 +24,7 @@
 //    pure HBM stream.
 // In the MFMA kernels the weight operand goes to the MFMA "A" side, so each lane ends up
 // with four consecutive output columns of one row.
-#include "duq_epilogue.h"
-// Cache policy of the stream / short-row kernels' output stores: 2 = non-temporal (the output is written once and
-// read by nobody in the launch; measured at M = 2048, N = K = 4096: 30.2 against 31.5 us, M = 4096: 58.8 against 61.1)
+#include "duq_gemm_common.h"
 // Cache policy of the weight loads of the kernels that read every weight byte once: 2 = non-temporal.  Measured:
 // skinny kernel 16 x 28672 x 4096 13.2 against 14.1 us, dot kernel 1 x 8192 x 28672 20.9 against 22.8 and 4 x 4096 x
 // 20480 11.5 against 13.2; the ring kernel (row groups read the weights again; a lane fetches 16 bytes of a row, a
@@ -43,250 +39,35 @@
 #ifndef DUQ_DOT_WLOAD_AUX
 #define DUQ_DOT_WLOAD_AUX 2
 #endif
-#ifndef DUQ_STREAM_STORE_AUX
-#define DUQ_STREAM_STORE_AUX 2
-#endif
-#include "duq_launch.h"
-#include "duq_tiles.h"
 #include <type_traits>
 
 namespace duq {
 
-constexpr uint32_t kNibbleMask = 0xF0F0F0F0u;
-
-// The first 56 bytes (through tiles_n) reach the kernels in registers (DUQ_HEAD_DECL / with_head).
-struct GemmParams {
-    const uint8_t *A;  // activations [M, K/2]
-    const uint8_t *B;  // weights     [N, K/2]
-    uint32_t M, N, K;
-    uint32_t tiles_m;
-    int32_t *C;        // int32 out (EPI < 0)
-    uint16_t *y;       // fp16 out  (EPI >= 0)
-    uint32_t tiles_n;
-    Epilogue epi;
-};
-static_assert(offsetof(GemmParams, epi) == kHeadBytes, "the fields delivered in registers");
-
-// Batched launch: problem blockIdx.z of a batch whose tensors are contiguous ([batch, M, K/2], [batch, N, K/2],
-// [batch, M, N], per-row arrays [batch, M], per-column arrays [batch, N]).
-__device__ __forceinline__ void batch_shift(GemmParams &p, uint32_t b)
-{
-    p.A += (uint64_t)b * p.M * (p.K >> 1);
-    p.B += (uint64_t)b * p.N * (p.K >> 1);
-    if (p.C) p.C += (uint64_t)b * p.M * p.N;
-    if (p.y) p.y += (uint64_t)b * p.M * p.N;
-    batch_shift(p.epi, b, p.M, p.N);
-}
-
-__device__ __forceinline__ void expand_nibbles(const v4u w, v4u &even, v4u &odd)
-{
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        even[i] = (w[i] << 4) & kNibbleMask;
-        odd[i] = w[i] & kNibbleMask;
-    }
-}
-
-
-// Store four consecutive output columns of one row.
-template <int EPI, bool BIAS>
-__device__ __forceinline__ void store_quad(const GemmParams &p, uint32_t m, uint32_t n0, v4i acc, bool vec_ok)
-{
-    if (m >= p.M || n0 >= p.N) return;
-    if (EPI < 0) {
-        int32_t *dst = p.C + (uint64_t)m * p.N + n0;
-        if (vec_ok && n0 + 3 < p.N) {
-            *reinterpret_cast<v4i *>(dst) = acc;
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (n0 + r < p.N) dst[r] = acc[r];
-        }
-    } else {
-        constexpr int MODE = EPI < 0 ? 0 : EPI;
-        const RowEpi rp = load_row<MODE>(p.epi, m);
-        uint16_t out[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t n = min(n0 + r, p.N - 1);
-            const ColParams c = load_col<MODE, BIAS>(p.epi.s_col_1, p.epi.z_col_1, p.epi.s_col_2, p.epi.z_col_2,
-                                                     p.epi.bias, n, p.epi.rs_col);
-            out[r] = dequant_one<MODE, BIAS>(acc[r], rp, c);
-        }
-        uint16_t *dst = p.y + (uint64_t)m * p.N + n0;
-        if (vec_ok && n0 + 3 < p.N) {
-            *reinterpret_cast<v2u *>(dst) = v2u{(uint32_t)out[0] | ((uint32_t)out[1] << 16),
-                                                (uint32_t)out[2] | ((uint32_t)out[3] << 16)};
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (n0 + r < p.N) dst[r] = out[r];
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------------
-// tile kernel
-// ---------------------------------------------------------------------------------
-constexpr int kBK = 128;           // k elements per tile step (64 packed bytes per row)
-constexpr int kLdsStride = 144;    // bytes per LDS row: 128 expanded bytes + 16 pad
-
-template <int BM, int BN, int EPI, bool BIAS>
-__global__ __launch_bounds__(256) void gemm_s4_tile_kernel(DUQ_HEAD_DECL, GemmParams tail)
-{
-    GemmParams p = with_head(tail, DUQ_HEAD_USE);
-    to_global(p.A);
-    to_global(p.B);
-    to_global(p.C);
-    to_global(p.y);
-    constexpr int WTM = BM / 2, WTN = BN / 2;  // per-wavefront tile
-    constexpr int TM = WTM / 16, TN = WTN / 16;
-    constexpr int NA = BM / 64, NB = BN / 64;  // 16-byte global pieces per thread
-    static_assert(BM % 64 == 0 && BN % 64 == 0, "tile shape");
-
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2][(BM + BN) * kLdsStride];
-
-    if (blockIdx.z) batch_shift(p, blockIdx.z);
-    uint32_t tile_m, tile_n;
-    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-    const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u, wave = tid >> 6;
-    const uint32_t wm = wave >> 1, wn = wave & 1u;
-    const uint32_t l16 = lane & 15u, g = lane >> 4;
-    const uint32_t kbytes = p.K >> 1;
-    const uint32_t nk = (p.K + kBK - 1) / kBK;
-
-    // global source of each 16-byte piece this thread moves (row clamped to stay in bounds)
-    const uint8_t *srcA[NA];
-    const uint8_t *srcB[NB];
-    uint32_t ldsA[NA], ldsB[NB];
-    const uint32_t pj = tid & 3u;  // which 16-byte piece of the 64-byte row segment
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-        const uint32_t row = (tid >> 2) + i * 64;
-        const uint32_t gm = min(m0 + row, p.M - 1);
-        srcA[i] = p.A + (uint64_t)gm * kbytes + pj * 16;
-        ldsA[i] = row * kLdsStride + pj * 32;
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-        const uint32_t row = (tid >> 2) + i * 64;
-        const uint32_t gn = min(n0 + row, p.N - 1);
-        srcB[i] = p.B + (uint64_t)gn * kbytes + pj * 16;
-        ldsB[i] = (BM + row) * kLdsStride + pj * 32;
-    }
-
-    v4u ga[NA], gb[NB];
-    auto load_tile = [&](uint32_t kt) {
-        const uint32_t koff = kt * (kBK / 2);
-        const bool ok = koff + pj * 16 < kbytes;  // K % 64 == 0: a piece is all in or all out
-#pragma unroll
-        for (int i = 0; i < NA; ++i)
-            ga[i] = ok ? *reinterpret_cast<const v4u *>(srcA[i] + koff) : v4u{0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-            gb[i] = ok ? *reinterpret_cast<const v4u *>(srcB[i] + koff) : v4u{0u, 0u, 0u, 0u};
-    };
-    auto store_tile = [&](uint32_t buf) {
-        uint8_t *base = lds[buf];
-#pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            v4u ev, od;
-            expand_nibbles(ga[i], ev, od);
-            *reinterpret_cast<v4u *>(base + ldsA[i]) = ev;
-            *reinterpret_cast<v4u *>(base + ldsA[i] + 16) = od;
-        }
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            v4u ev, od;
-            expand_nibbles(gb[i], ev, od);
-            *reinterpret_cast<v4u *>(base + ldsB[i]) = ev;
-            *reinterpret_cast<v4u *>(base + ldsB[i] + 16) = od;
-        }
-    };
-
-    v4i acc[TN][TM];
-#pragma unroll
-    for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b) acc[a][b] = v4i{0, 0, 0, 0};
-
-    // fragment rows of this lane inside the LDS tile
-    const uint32_t fragX = (wm * WTM + l16) * kLdsStride + g * 16;         // activations
-    const uint32_t fragW = (BM + wn * WTN + l16) * kLdsStride + g * 16;    // weights
-
-    load_tile(0);
-    store_tile(0);
-    __syncthreads();
-
-    for (uint32_t kt = 0; kt < nk; ++kt) {
-        const uint32_t cur = kt & 1u;
-        const bool more = kt + 1 < nk;
-        if (more) load_tile(kt + 1);
-
-        const uint8_t *base = lds[cur];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            v4i fx[TM], fw[TN];
-#pragma unroll
-            for (int b = 0; b < TM; ++b)
-                fx[b] = *reinterpret_cast<const v4i *>(base + fragX + b * 16 * kLdsStride + s * 64);
-#pragma unroll
-            for (int a = 0; a < TN; ++a)
-                fw[a] = *reinterpret_cast<const v4i *>(base + fragW + a * 16 * kLdsStride + s * 64);
-#pragma unroll
-            for (int a = 0; a < TN; ++a)
-#pragma unroll
-                for (int b = 0; b < TM; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[a], fx[b], acc[a][b], 0, 0, 0);
-        }
-
-        if (more) store_tile(cur ^ 1u);
-        __syncthreads();
-    }
-
-    // lane holds, for every (a, b): rows n = 4*g + r of the weight fragment, column m = l16
-    const bool vec_ok = (EPI < 0) ? (p.N % 4 == 0 && reinterpret_cast<uintptr_t>(p.C) % 16 == 0)
-                                  : (p.N % 4 == 0 && reinterpret_cast<uintptr_t>(p.y) % 8 == 0);
-#pragma unroll
-    for (int b = 0; b < TM; ++b)
-#pragma unroll
-        for (int a = 0; a < TN; ++a) {
-            v4i v = acc[a][b];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] >>= 8;
-            store_quad<EPI, BIAS>(p, m0 + wm * WTM + b * 16 + l16, n0 + wn * WTN + a * 16 + g * 4, v, vec_ok);
-        }
-}
-
-typedef int v16i __attribute__((ext_vector_type(16)));
-
-// ---------------------------------------------------------------------------------
-// stream kernel (prefill): weights global -> registers, activations through LDS,
+// stream kernel (prefill on short rows): weights global -> registers, activations through LDS,
 // v_mfma_i32_32x32x32_i8
 // ---------------------------------------------------------------------------------
-// Tile 32*TM (M) x 256 (N), TM = 4 for large problems (described below; TM = 2 and 1 run the same
-// schedule with 4 and 2 MFMA slots per step and exist to give mid-size M one workgroup per
-// CU), 4 wavefronts side by side along N: every wavefront owns 64 weight
+// Tile 64 (M) x 128 (N), 4 wavefronts side by side along N: every wavefront owns 32 weight
 // rows that no other wavefront of the workgroup needs, so weight fragments never go through
 // LDS: lane (l32, h) loads 16-byte piece i (0..3) = bytes [i*32 + h*16, +16) of the 128-byte
-// row segment of a 256-k chunk straight into registers.  The 128 activation rows are shared
+// row segment of a 256-k chunk straight into registers.  The 64 activation rows are shared
 // by the four wavefronts: they are expanded to bytes once on the way into LDS (three
-// buffers, rows padded to 272 B) and read back as 128-bit fragments.  LDS traffic per chunk
-// is 32 KB written + 128 KB read.
+// buffers, rows padded to 272 B) and read back as 128-bit fragments.  What bounds it is the wait
+// for a chunk's activations, which are loaded and used within one chunk; with two or three workgroups
+// on a CU they cover for one another, and with few chunks it matters less than the prefill kernel's
+// longer start and end (select_stream_tile draws the line).
 //
 // The 32x32x32 MFMA keeps the matrix pipe full from a single wavefront per SIMD (32 cycles
 // per instruction, 16 per 32768 operations); the 16x16x64 form needs 18 and loses more to
-// interleaved vector work.  A chunk is 8 k-steps (piece i, nibble parity) of 8 MFMAs (2
-// weight tiles x 4 activation tiles).  The order is fixed by hand, a scheduling fence after
+// interleaved vector work.  A chunk is 8 k-steps (piece i, nibble parity) of 2 MFMAs (1
+// weight tile x 2 activation tiles).  The order is fixed by hand, a scheduling fence after
 // every MFMA, and everything else rides in the MFMA shadows, a few instructions per slot:
-//   every step    : the next step's four activation fragments (step 7: the next chunk's);
+//   every step    : the next step's two activation fragments (step 7: the next chunk's);
 //   step 2i       : refetch weight piece i for the next chunk (its registers were just
-//                   expanded), expand piece i+1 of weight tile 0;  step 2i+1: of tile 1;
+//                   expanded), expand piece i+1;
 //   step 1        : fetch the activations two chunks ahead;
-//   steps 4..7    : expand + store those activations into the third LDS buffer;
-//   steps 6, 7    : expand the next chunk's weight piece 0.
+//   steps 6, 7    : expand + store those activations into the third LDS buffer;
+//   step 6        : expand the next chunk's weight piece 0.
 // MFMAs are issued through inline assembly with the accumulators tied to the accumulation
 // register file, so they never move.
 //
@@ -298,7 +79,7 @@ constexpr int kCK = 256;         // k elements per chunk (128 packed bytes per r
 constexpr int kXStride = 272;    // LDS bytes per activation row: 256 expanded + 16 pad
 
 
-template <int TM, int EPI, bool BIAS, int TN = 2>
+template <int EPI, bool BIAS>
 __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, GemmParams tail)
 {
     GemmParams p = with_head(tail, DUQ_HEAD_USE);
@@ -306,10 +87,7 @@ __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, Gemm
     to_global(p.B);
     to_global(p.C);
     to_global(p.y);
-    static_assert(TM == 4 || TM == 2 || TM == 1, "32-row activation tiles per wavefront");
-    // TN = 32-column weight tiles per wavefront: tiles of 256 columns (TN = 2), or of 128 with 64 rows (TN = 1):
-    // as many outputs per workgroup as 32 x 256 with a third less operand bytes into the CU
-    static_assert(TN == 2 || (TN == 1 && TM >= 2), "column tiles per wavefront");
+    constexpr int TM = 2, TN = 1;      // 32-row activation and 32-column weight tiles per wavefront
     constexpr int BM = 32 * TM, BN = 128 * TN;
     constexpr int S = TM * TN;         // MFMA slots per step
     constexpr int NXP = TM;            // 16-byte activation pieces per thread and chunk
@@ -330,6 +108,7 @@ __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, Gemm
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     const uint32_t l32 = lane & 31u, h = lane >> 5;
+    const uint32_t wm0 = m0, wn0 = n0 + wave * (32 * TN);
     const uint32_t kbytes = p.K >> 1;
     const uint32_t nfull = p.K / kCK;
     const uint32_t nchunks = (p.K + kCK - 1) / kCK;
@@ -492,6 +271,7 @@ __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, Gemm
 
     // ---- epilogue parameters: fetched now so that their latency hides behind the main loop
 #include "duq_stream_epilogue_fetch.inc"
+    fetch_params();
 
     uint32_t cur = 0, nxt = kBuf, nx2 = 2 * kBuf;
     auto rotate = [&]() {
@@ -514,192 +294,7 @@ __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, Gemm
     asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
 
     constexpr bool kWideStore = false;
-#include "duq_stream_epilogue_store.inc"
-}
-
-// ---------------------------------------------------------------------------------
-// stream kernel, 256-row tiles: problems with at least one 256 x 256 tile per CU
-// ---------------------------------------------------------------------------------
-// The stream kernel's schedule with twice the activation rows per workgroup: the weight bytes a wavefront fetches
-// and expands (the loop's main side work: two vector instructions per packed word) meet eight activation tiles
-// instead of four, and a tile's prologue and epilogue are paid once per 65536 outputs instead of twice.  All 256
-// accumulation registers hold accumulators (2 weight tiles x 8 activation tiles x 16), so the epilogue parameters
-// are fetched after the loop, and a chunk is 128 k (three LDS buffers of 256 rows x 144 bytes; the epilogue's staging
-// area, 4 x 256 x 144 bytes, is what sizes the array).  A chunk is four steps (piece, nibble parity) of sixteen
-// MFMAs; per step: slots 0-7 read the next step's eight activation fragments, 8-9 refetch the weight piece just
-// consumed (even steps), 10-13 expand one weight piece of one tile, 8, 9, 14, 15 expand one activation piece (stored
-// in slot 15), and the activations ride two chunks of registers deep: a chunk's packed activations are requested a
-// whole chunk before they are expanded into the buffer that is read two chunks later.
-constexpr int kCK2 = 128;        // k elements per chunk
-constexpr int kXStride2 = 144;   // LDS bytes per activation row: 128 expanded + 16 pad
-
-template <int EPI, bool BIAS>
-__global__ __launch_bounds__(256) void gemm_s4_stream256_kernel(DUQ_HEAD_DECL, GemmParams tail)
-{
-    GemmParams p = with_head(tail, DUQ_HEAD_USE);
-    to_global(p.A);
-    to_global(p.B);
-    to_global(p.C);
-    to_global(p.y);
-    static_assert(EPI != 5, "the dual-uniform row-sum epilogue stages its parameters in LDS: stream kernel");
-    constexpr int TM = 8, TN = 2, BM = 256, BN = 256, S = TM * TN, NXP = 4;
-    constexpr uint32_t kBuf = BM * kXStride2;
-    constexpr uint32_t kLds = 4 * BM * 144 > 3 * kBuf ? 4 * BM * 144 : 3 * kBuf;
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
-    uint32_t *const dpar = nullptr;  // named by the shared epilogue text for an epilogue this kernel never runs
-    const uint32_t dwide = 0;
-
-    if (blockIdx.z) batch_shift(p, blockIdx.z);
-    uint32_t tile_m, tile_n;
-    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-    const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u, wave = tid >> 6;
-    const uint32_t l32 = lane & 31u, h = lane >> 5;
-    const uint32_t kbytes = p.K >> 1;
-    const uint32_t nchunks = (p.K + kCK2 - 1) / kCK2;
-
-    const __amdgpu_buffer_rsrc_t rW = make_rsrc(p.B + (uint64_t)n0 * kbytes, min(p.N - n0, (uint32_t)BN) * kbytes);
-    const __amdgpu_buffer_rsrc_t rX = make_rsrc(p.A + (uint64_t)m0 * kbytes, min(p.M - m0, (uint32_t)BM) * kbytes);
-
-    // weights: lane (l32, h) of tile t holds piece i = bytes [i*32 + h*16, +16) of the chunk's 64-byte row segment
-    uint32_t woff[TN];
-#pragma unroll
-    for (int t = 0; t < TN; ++t) woff[t] = (wave * (32 * TN) + t * 32 + l32) * kbytes + h * 16;
-    // activations: thread -> 16-byte piece xq of the segment of row xrow + 64 * i.  The sixteen lanes that an LDS
-    // write instruction serves together hold rows r, r + 1, r + 8, r + 9 (r even): with 144-byte rows their four
-    // pieces each land in sixteen different 16-byte columns of the banks (rows r .. r + 3 would collide in pairs)
-    uint32_t xoff[NXP], xlds[NXP];
-    const uint32_t xq = tid & 3u;
-    const uint32_t xrow = ((tid >> 2) & 1u) + 8u * ((tid >> 3) & 1u) + 2u * ((tid >> 4) & 3u) + 16u * (tid >> 6);
-#pragma unroll
-    for (int i = 0; i < NXP; ++i) {
-        const uint32_t row = xrow + i * 64;
-        xoff[i] = row * kbytes + xq * 16;
-        xlds[i] = row * kXStride2 + xq * 32;
-    }
-    // K % 64 == 0: a 16-byte piece is all inside the row or all outside (then redirected out of range: zero)
-    auto load_w = [&](int t, int i, uint32_t koff) {
-        return buf_load16(rW, koff + i * 32 + h * 16 < kbytes ? woff[t] + i * 32 : kOobOffset, koff);
-    };
-    auto load_x = [&](int j, uint32_t koff) {
-        return buf_load16(rX, koff + xq * 16 < kbytes ? xoff[j] : kOobOffset, koff);
-    };
-
-    v4u wreg[TN][2];      // raw weight pieces [tile][piece]
-    v4u xr[2][NXP];       // raw activation pieces, two chunks of them
-    v4u wexp[2][2][TN];   // expanded weights [piece][parity][tile]
-    v4i fx[2][TM];        // activation fragments [step & 1][tile]
-    v16i acc[TN][TM];
-#pragma unroll
-    for (int t = 0; t < TN; ++t)
-#pragma unroll
-        for (int b = 0; b < TM; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[t][b][r] = 0;
-
-    // fragment of step (i, par) for activation tile b: + b*32*kXStride2 + i*64 + par*16
-    const uint32_t fragX = l32 * kXStride2 + h * 32;
-    auto expand_word = [&](const v4u &raw, v4u &even, v4u &odd, int w) {
-        even[w] = (raw[w] << 4) & kNibbleMask;
-        odd[w] = raw[w] & kNibbleMask;
-    };
-
-    // chunk c; PAR = c & 1: xr[PAR] holds the packed activations of chunk c + 2, xr[PAR ^ 1] receives those of c + 3
-    auto body = [&](auto parity, uint32_t c, uint32_t cur, uint32_t nxt, uint32_t nx2) {
-        constexpr int PAR = decltype(parity)::value;
-        const uint32_t koff1 = (c + 1) * (kCK2 / 2), koff3 = (c + 3) * (kCK2 / 2);
-        v4u xe, xo;
-#pragma unroll
-        for (int step = 0; step < 4; ++step) {
-            const int i = step >> 1, par = step & 1;
-#pragma unroll
-            for (int slot = 0; slot < S; ++slot) {
-                const int b = slot / TN, t = slot % TN;
-                asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, %0"
-                             : "+a"(acc[t][b])
-                             : "v"(wexp[i][par][t]), "v"(fx[step & 1][b]));
-                __builtin_amdgcn_sched_barrier(0);
-                // ---- side work in the shadow of this MFMA
-                if (slot < TM) {  // next step's activation fragment for tile `slot`
-                    const uint8_t *src = step < 3 ? lds + cur + fragX + ((step + 1) >> 1) * 64 + ((step + 1) & 1) * 16
-                                                  : lds + nxt + fragX;
-                    fx[(step + 1) & 1][slot] = *reinterpret_cast<const v4i *>(src + slot * 32 * kXStride2);
-                }
-                if (par == 0 && slot >= 8 && slot < 8 + TN)  // piece i was expanded earlier: refetch it for the next chunk
-                    wreg[slot - 8][i] = load_w(slot - 8, i, koff1);
-                if (slot >= 10 && slot < 14)  // the next piece (this chunk's second, then the next chunk's first) of tile `par`
-                    expand_word(wreg[par][(i + 1) & 1], wexp[(i + 1) & 1][0][par], wexp[(i + 1) & 1][1][par], slot - 10);
-                if (step == 0 && slot >= 12) xr[PAR ^ 1][slot - 12] = load_x(slot - 12, koff3);
-                // chunk c + 2 -> third LDS buffer: piece `step`, its four words in the slots without a fragment read
-                // or a weight word, then both halves stored
-                if (slot == 8 || slot == 9 || slot == 14 || slot == 15) {
-                    const int w = slot < 10 ? slot - 8 : slot - 12;
-                    expand_word(xr[PAR][step], xe, xo, w);
-                    if (w == 3) {
-                        *reinterpret_cast<v4u *>(lds + nx2 + xlds[step]) = xe;
-                        *reinterpret_cast<v4u *>(lds + nx2 + xlds[step] + 16) = xo;
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        __syncthreads();
-    };
-
-    // ---- prologue: chunks 0 and 1 activations -> LDS, chunk 2 -> registers, chunk 0 weights -> registers
-    {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int t = 0; t < TN; ++t) wreg[t][i] = load_w(t, i, 0);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-#pragma unroll
-            for (int j = 0; j < NXP; ++j) xr[q][j] = load_x(j, q * (kCK2 / 2));
-        }
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int j = 0; j < NXP; ++j) {
-                v4u ev, od;
-                expand_nibbles(xr[q][j], ev, od);
-                *reinterpret_cast<v4u *>(lds + q * kBuf + xlds[j]) = ev;
-                *reinterpret_cast<v4u *>(lds + q * kBuf + xlds[j] + 16) = od;
-            }
-#pragma unroll
-        for (int j = 0; j < NXP; ++j) xr[0][j] = load_x(j, 2 * (kCK2 / 2));
-#pragma unroll
-        for (int t = 0; t < TN; ++t) expand_nibbles(wreg[t][0], wexp[0][0][t], wexp[0][1][t]);
-        __syncthreads();
-#pragma unroll
-        for (int b = 0; b < TM; ++b) fx[0][b] = *reinterpret_cast<const v4i *>(lds + fragX + b * 32 * kXStride2);
-    }
-
-    uint32_t cur = 0, nxt = kBuf, nx2 = 2 * kBuf;
-    auto rotate = [&]() {
-        const uint32_t t = cur;
-        cur = nxt;
-        nxt = nx2;
-        nx2 = t;
-    };
-    using P0 = std::integral_constant<int, 0>;
-    using P1 = std::integral_constant<int, 1>;
-    uint32_t c = 0;
-    for (; c + 1 < nchunks; c += 2) {
-        body(P0{}, c, cur, nxt, nx2);
-        rotate();
-        body(P1{}, c + 1, cur, nxt, nx2);
-        rotate();
-    }
-    if (c < nchunks) body(P0{}, c, cur, nxt, nx2);
-    // the MFMAs above are opaque to the compiler's hazard tracking: let the last ones retire
-    // before the accumulators are read
-    asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-
-    // ---- epilogue parameters (after the loop: no registers to spare inside it), then the epilogue
-#include "duq_stream_epilogue_fetch.inc"
-    constexpr bool kWideStore = false;
+    uint8_t *const wstage = lds + wave * (BM * (64 * TN + 16));
 #include "duq_stream_epilogue_store.inc"
 }
 
@@ -735,6 +330,7 @@ __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, G
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     const uint32_t l32 = lane & 31u, h = lane >> 5;
+    const uint32_t wm0 = m0, wn0 = n0 + wave * (32 * TN);
     const uint32_t kbytes = p.K >> 1;  // <= 128
 
     const __amdgpu_buffer_rsrc_t rW = make_rsrc(p.B + (uint64_t)n0 * kbytes, min(p.N - n0, (uint32_t)BN) * kbytes);
@@ -758,6 +354,7 @@ __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, G
         xreg[j] = buf_load16(rX, xq * 16 < kbytes ? row * kbytes + xq * 16 : kOobOffset, 0);
     }
 #include "duq_stream_epilogue_fetch.inc"
+    fetch_params();
 #pragma unroll
     for (int j = 0; j < NXP; ++j) {
         const uint32_t row = (tid >> 3) + j * 32;
@@ -803,6 +400,7 @@ __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, G
     if (kbytes > 64) steps(2, 4);  // rows of 192 or 256 elements
     // (the activation buffer becomes the staging area of the epilogue, which waits for every wavefront first)
     constexpr bool kWideStore = true;
+    uint8_t *const wstage = lds + wave * (BM * (64 * TN + 16));
 #include "duq_stream_epilogue_store.inc"
 }
 
@@ -1162,7 +760,7 @@ __global__ __launch_bounds__(256) void gemv_s4_dot_kernel(DUQ_HEAD_DECL, GemmPar
 // Which kernel family takes a shape.  Host arithmetic only, so that the rule can be tested without a GPU:
 // every kernel whose weight offsets are 32-bit (decode, dot, ring: row * K/2 + offset, and a buffer descriptor
 // over the whole tensor) is reachable only while the packed weights stay below 4 GiB - 256 (the out-of-range
-// marker); larger tensors go to the stream / tile kernels, whose descriptors and pointers are per tile
+// marker); larger tensors go to the stream / prefill kernels, whose descriptors and pointers are per tile
 // (64-bit base, 32-bit offsets inside 256 rows).
 int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
 {
@@ -1182,7 +780,11 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
     }
     if (M <= 64 && small_offsets) {
         if (K <= 4096 || (K <= 8192 && M <= 32)) return kKernelDecodeMfma;
-        if ((N + 15) / 16 >= 192 && (K <= 8192 || (K <= 12288 && M <= 48))) return kKernelDecodeMfma;
+        // (wide layers of more than 32 long rows: one round of 64 x 128 tiles of the prefill kernel, 64 x 11008 x 8192
+        // 16.3 against 21.1 us, 48 x 11008 x 11008 20.3 / 24.0, 33 x 11008 x 8192 15.9 / 16.8; at N = 4096 the decode
+        // kernel is ahead)
+        const bool wide = M > 32 && N >= 8192;
+        if ((N + 15) / 16 >= 192 && !wide && (K <= 8192 || (K <= 12288 && M <= 48))) return kKernelDecodeMfma;
     }
     const uint32_t xstride = ((K / 2 + 127) / 128) * 128;
     // dot kernel: up to four rows too long for the decode kernels
@@ -1206,7 +808,14 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
         const bool few_groups = row_groups <= 2 || (row_groups <= 6 && tiles32 < 64) || tiles32 < 48;
         const bool mid_rows = M > 16 && M <= 256 && few_groups && !(row_groups > 1 && tiles32 >= 128);
         const bool long_rows = M <= 16 && K > 8192;  // 5..16 rows of 12289..16384 elements
-        if ((long_rows || mid_rows) && K <= 16384 && small_offsets && !narrow_round) return kKernelRing;
+        // (16 x 16 tiles of the output from which the prefill kernel's 64 x 128 tiles are ahead although they leave CUs
+        // idle: a ring group re-streams the weights per 64, 32 or, for rows longer than 8192 elements, 16 rows.  64 x
+        // 4096 x 11008 18.9 against 26.3 us, 33 x 4096 x 14336 22.7 / 24.4, 17 x 11008 x 14336 23.2 / 38.6, 160 x 2048 x
+        // 4096 9.8 / 13.2, 200 x 1024 x 11008 18.9 / 24.8; but 17 x 4096 x 14336, 100 x 1000 x 4096, 100 x 2048 x 8192 and
+        // 200 x 520 x 8192 are the ring kernel's)
+        const bool many_tiles = (uint64_t)rb_all * ((N + 15) / 16) >= (K > 8192 ? 768u : 1280u);
+        if ((long_rows || (mid_rows && !many_tiles)) && K <= 16384 && small_offsets && !narrow_round) return kKernelRing;
+        if (mid_rows && many_tiles && K <= 16384) return kKernelStream;
     }
     auto tiles = [&](uint32_t bm, uint32_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     if (narrow_round || (M > 32 && tiles(32, 256) >= 32)) return kKernelStream;
@@ -1214,12 +823,11 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
 }
 
 // batch > 1: `batch` problems of one shape, tensors contiguous over the batch, one launch (blockIdx.z is the
-// problem): stream or tile kernel only, the choice made on the tiles of the whole batch.
+// problem): the short-row, stream and prefill kernels only, the tile chosen on the whole batch.
 template <int EPI, bool BIAS>
 static void launch_epi(GemmParams &p, hipStream_t stream, uint32_t batch = 1)
 {
-    const int kernel = batch > 1 ? (p.M > 32 && ((p.M + 31) / 32) * ((p.N + 255) / 256) * batch >= 32 ? kKernelStream : kKernelTile)
-                                 : select_gemm_kernel(p.M, p.N, p.K);
+    const int kernel = batch > 1 ? kKernelStream : select_gemm_kernel(p.M, p.N, p.K);
     // (EPI 5, the dual-uniform row-sum epilogue, exists in the stream kernel only: gemm_fuses_dual_rowsum)
     if constexpr (EPI != 5) {
     if (kernel == kKernelDot) {
@@ -1280,69 +888,29 @@ static void launch_epi(GemmParams &p, hipStream_t stream, uint32_t batch = 1)
         return;
     }
     }
-    // Stream kernel: the tile that select_stream_tile prices cheapest; small problems (few column tiles) stay on
-    // the tile kernels.
-    auto tiles = [&](uint32_t bm, uint32_t bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * batch; };
-    int best_tm = 0;
-    bool half_width = false;  // 128-column tiles
-    if (kernel == kKernelStream) {
-        const StreamTile tile = select_stream_tile(p.M, p.N, p.K, batch, EPI == 5);
-        if constexpr (EPI != 5) {
-            if (tile.rows == 256) {
-                p.tiles_m = (p.M + 255) / 256;
-                p.tiles_n = (p.N + 255) / 256;
-                DUQ_LAUNCH_HEAD((gemm_s4_stream256_kernel<EPI, BIAS>), dim3(p.tiles_m * p.tiles_n, 1, batch), dim3(256), 0,
-                                stream, p);
-                return;
-            }
-        }
-        best_tm = (int)(tile.rows / 32);
-        half_width = tile.cols == 128;
-    }
-    if constexpr (EPI != 5) if (best_tm && p.K <= 256) {
-        // rows of at most 256 elements: one chunk, the launch is its output stores: the short-row kernel with 64-row
-        // tiles (measured on 32 products of 2048 x 2048 x 128: 86 us against 95 us on the stream kernel's 64-row tiles)
-        p.tiles_m = (p.M + 63) / 64;
-        p.tiles_n = (p.N + 255) / 256;
-        DUQ_LAUNCH_HEAD((gemm_s4_shortk_kernel<2, EPI, BIAS>), dim3(p.tiles_m * p.tiles_n, 1, batch), dim3(256), 0,
-                           stream, p);
-        return;
-    }
-    if (best_tm && half_width) {
-        p.tiles_m = (p.M + 32 * best_tm - 1) / (32 * best_tm);
-        p.tiles_n = (p.N + 127) / 128;
-        const dim3 grid(p.tiles_m * p.tiles_n, 1, batch);
-        if (best_tm == 4)
-            DUQ_LAUNCH_HEAD((gemm_s4_stream_kernel<4, EPI, BIAS, 1>), grid, dim3(256), 0, stream, p);
-        else
-            DUQ_LAUNCH_HEAD((gemm_s4_stream_kernel<2, EPI, BIAS, 1>), grid, dim3(256), 0, stream, p);
-    } else if (best_tm) {
-        p.tiles_m = (p.M + 32 * best_tm - 1) / (32 * best_tm);
-        p.tiles_n = (p.N + 255) / 256;
-        const dim3 grid(p.tiles_m * p.tiles_n, 1, batch);
-        if (best_tm == 4)
-            DUQ_LAUNCH_HEAD((gemm_s4_stream_kernel<4, EPI, BIAS>), grid, dim3(256), 0, stream, p);
-        else if (best_tm == 2)
-            DUQ_LAUNCH_HEAD((gemm_s4_stream_kernel<2, EPI, BIAS>), grid, dim3(256), 0, stream, p);
-        else
-            DUQ_LAUNCH_HEAD((gemm_s4_stream_kernel<1, EPI, BIAS>), grid, dim3(256), 0, stream, p);
-    } else if constexpr (EPI != 5) {
-        if (tiles(128, 256) >= 256 && p.M > 64) {
-            p.tiles_m = (p.M + 127) / 128;
+    if constexpr (EPI != 5) {
+        if (p.K <= 256) {
+            // rows of at most 256 elements: one chunk, the launch is its output stores: the short-row kernel with 64-row
+            // tiles (measured on 32 products of 2048 x 2048 x 128: 86 us against 95 us on the stream kernel's 64-row tiles),
+            // 32-row ones for a few rows (one query per head)
+            const uint32_t bm = p.M <= 32 ? 32 : 64;
+            p.tiles_m = (p.M + bm - 1) / bm;
             p.tiles_n = (p.N + 255) / 256;
-            DUQ_LAUNCH_HEAD((gemm_s4_tile_kernel<128, 256, EPI, BIAS>), dim3(p.tiles_m * p.tiles_n, 1, batch), dim3(256),
-                               0, stream, p);
-        } else if (tiles(128, 128) >= 256 && p.M > 64) {
-            p.tiles_m = (p.M + 127) / 128;
-            p.tiles_n = (p.N + 127) / 128;
-            DUQ_LAUNCH_HEAD((gemm_s4_tile_kernel<128, 128, EPI, BIAS>), dim3(p.tiles_m * p.tiles_n, 1, batch), dim3(256),
-                               0, stream, p);
-        } else {
-            p.tiles_m = (p.M + 63) / 64;
-            p.tiles_n = (p.N + 63) / 64;
-            DUQ_LAUNCH_HEAD((gemm_s4_tile_kernel<64, 64, EPI, BIAS>), dim3(p.tiles_m * p.tiles_n, 1, batch), dim3(256), 0,
-                               stream, p);
+            const dim3 grid(p.tiles_m * p.tiles_n, 1, batch);
+            if (bm == 32)
+                DUQ_LAUNCH_HEAD((gemm_s4_shortk_kernel<1, EPI, BIAS>), grid, dim3(256), 0, stream, p);
+            else
+                DUQ_LAUNCH_HEAD((gemm_s4_shortk_kernel<2, EPI, BIAS>), grid, dim3(256), 0, stream, p);
+            return;
         }
+    }
+    const StreamTile tile = select_stream_tile(p.M, p.N, p.K, batch, EPI == 5);
+    if (tile.stream) {
+        p.tiles_m = (p.M + 63) / 64;
+        p.tiles_n = (p.N + 127) / 128;
+        DUQ_LAUNCH_HEAD((gemm_s4_stream_kernel<EPI, BIAS>), dim3(p.tiles_m * p.tiles_n, 1, batch), dim3(256), 0, stream, p);
+    } else {
+        (void)launch_prefill(p, tile, EPI >= 0, stream, batch);
     }
 }
 

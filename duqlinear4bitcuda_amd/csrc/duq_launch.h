@@ -75,53 +75,47 @@ enum GemmKernelId {
     kKernelDot = 3,         // duq_gemm.hip, M <= 4 with rows longer than 16384 elements
     kKernelRing = 4,        // duq_gemm.hip, 17 <= M <= 256 on narrow problems the decode kernel does not take
     kKernelSkinny = 5,      // duq_gemm.hip, 9 <= M <= 16 with 1536 or more column tiles, K <= 4096
-    kKernelStream = 6,      // duq_gemm.hip, prefill
-    kKernelTile = 7,        // duq_gemm.hip, everything else (per-tile 64-bit bases: any tensor size)
+    kKernelStream = 6,      // duq_prefill.hip (duq_gemm.hip for short rows), prefill
+    kKernelTile = 7,        // the same kernels on problems of few tiles or rows too long for the others
 };
 int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K);
 // Shapes whose GEMM can apply the dual-uniform row-sum epilogue itself (mode 5): those of the decode kernels, and those
-// of the stream kernel with rows longer than 256 elements and N % 8 == 0 (its staged stores); the others run the GEMM
-// into int32 and launch_dual_rowsum_dequant.
+// of the stream and prefill kernels with rows longer than 256 elements (512 where output rows are not 16-byte aligned:
+// there the accumulators' detour through memory, 8 bytes per output, is what a launch takes); the others run the GEMM into
+// int32 and launch_dual_rowsum_dequant.
 inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 {
     const int kernel = select_gemm_kernel(M, N, K);
     if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma) return true;
-    return kernel == kKernelStream && K > 256 && N % 8 == 0;
+    return (kernel == kKernelStream || kernel == kKernelTile) && (N % 8 == 0 ? K > 256 : K >= 512);
 }
-// Tile of the stream kernel for a problem select_gemm_kernel gives to it (rows 0: none, the tile kernels run).
-// Whole rounds of 256 workgroups (one per CU) cost about nchunks * c + f microseconds each, c (per 256 k) and f
-// measured per tile shape; the cheapest wins.  The L2 -> CU path bounds these tiles, so what counts is operand rows
-// per output: a 64 x 128 tile has the outputs of a 32 x 256 one with a third less operand bytes into the CU (192 rows
-// of K / 2 bytes against 288): 512 x 4096 x 4096 13.1 against 19.8 us, 512 x 4096 x 11008 (K) 34.1 against 52; a
-// 128 x 128 tile those of a 64 x 256 one with a fifth less (256 against 320): 1024 x 4096 x 4096 21.5 against 26.1 us
-// on one box, 768 rows 18.9 against 22.4, 1024 x 4096 x 11008 (K) 50.5 against 58.5.  A round of 256 x 256 tiles
-// (gemm_s4_stream256_kernel; not with the dual-uniform row-sum epilogue, `mode5`) costs 1.91 rounds of 128 x 256
-// ones for twice the outputs, measured (us, 256-row against 128-row tiles): 4096 x 4096 x 4096 56.5 / 58.9,
-// 4096 x 11008 x 4096 149 / 160, 2048 x 22016 x 4096 150 / 160, 4096 x 28672 x 8192 668 / 707,
-// 4096 x 8192 x 28672 (K) 634 / 667; and 4000 x 8200 x 4160, three ragged rounds against five: 160 / 145.
+// Tile for a problem select_gemm_kernel gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
+// 64 x 128 tiles (duq_gemm.hip).  Whole rounds of 256 workgroups (one per CU) cost about f + c * (K / 256) microseconds
+// each, measured per tile shape (N = 4096, one round, K = 1024 / 4096 / 16384): 64 x 128 6.6 / 11.9 / 33, 128 x 128 8.9 /
+// 17.5 / 55, 128 x 256 12.5 / 30 / 100, 256 x 256 21 / 52.7 / 178 (1.3 of it once per launch); the cheapest wins.  The
+// stream kernel has the longer loop but starts and ends faster (512 x 4096 x 512 4.8 against 5.9 us, x 1024 5.8 / 6.6, x
+// 2048 8.1 / 8.3, x 4096 13.3 / 11.9), and two or three of its workgroups share a CU, so its rounds need not be whole (32
+// products of 1216 x 64 x 1216, 608 tiles: 12.8 us).  The dual-uniform row-sum epilogue (`mode5`) has no 256 x 256 tile
+// (its staged parameters do not fit in LDS beside the operands).
 struct StreamTile {
     uint32_t rows, cols;
+    bool stream;
 };
 inline StreamTile select_stream_tile(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, bool mode5)
 {
-    auto tiles = [&](uint32_t bm, uint32_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
     const float nch = (float)((K + 255) / 256);
-    const uint32_t tm[5] = {4, 2, 1, 2, 4};
-    const bool hw[5] = {false, false, false, true, true};
-    const float c_us[5] = {1.5f, 1.0f, 0.8f, 0.78f, 0.9f}, f_us[5] = {9.f, 7.f, 6.f, 1.f, 4.5f};
-    StreamTile best{0, 0};
-    float best_cost = 0.f;
-    for (int k = 0; k < 5; ++k) {
-        const uint32_t t = tiles(32u * tm[k], hw[k] ? 128 : 256);
-        const float cost = (float)((t + 255) / 256) * (nch * c_us[k] + f_us[k]);
-        if (best.rows == 0 || cost < best_cost) {
+    const uint32_t bm[4] = {64, 128, 128, 256}, bn[4] = {128, 128, 256, 256};
+    const float c_us[4] = {0.44f, 0.76f, 1.47f, 2.62f}, f_us[4] = {3.6f, 4.3f, 5.5f, 9.5f};
+    auto tiles = [&](int k) { return (uint64_t)((M + bm[k] - 1) / bm[k]) * ((N + bn[k] - 1) / bn[k]) * batch; };
+    StreamTile best{64, 128, true};
+    float best_cost = std::max(1.f, (float)tiles(0) / 256.f) * (nch * 0.62f + 0.9f) + 1.3f;
+    for (int k = 0; k < (mode5 ? 3 : 4); ++k) {
+        const float cost = (float)((tiles(k) + 255) / 256) * (nch * c_us[k] + f_us[k]);
+        if (cost < best_cost) {
             best_cost = cost;
-            best = StreamTile{32u * tm[k], hw[k] ? 128u : 256u};
+            best = StreamTile{bm[k], bn[k], false};
         }
     }
-    const uint32_t t256 = tiles(256, 256);
-    if (!mode5 && K > 256 && t256 >= 256 && 1.91f * (float)((t256 + 255) / 256) * (nch * c_us[0] + f_us[0]) < best_cost)
-        best = StreamTile{256, 256};
     return best;
 }
 inline bool decode_uses_rows_kernel(uint32_t M) { return M <= 4; }
