@@ -152,6 +152,15 @@ __device__ __forceinline__ uint32_t dequant_pair(ACC acc0, ACC acc1, const RowEp
     return __builtin_bit_cast(uint32_t, y);
 }
 
+// The same for integer accumulators carried x 256: the factor goes in one instruction with the conversion to binary16
+// (exact: the float32 of 256 * acc is, below 2^24, and so is its 256th part) instead of a shift per accumulator.
+template <int MODE, bool BIAS>
+__device__ __forceinline__ uint32_t dequant_pair_x256(int acc0, int acc1, const RowEpi &r, const ColParams &c0, const ColParams &c1)
+{
+    if (MODE == 4) return dequant_pair<MODE, BIAS>(acc0 >> 8, acc1 >> 8, r, c0, c1);
+    return dequant_pair<MODE, BIAS>((float)acc0 * (1.0f / 256.0f), (float)acc1 * (1.0f / 256.0f), r, c0, c1);
+}
+
 // Row-sum epilogue of the dual-uniform layer for one output (definition: include/duq_hip.h,
 // duq_asym_dual_rowsum_dequant_host), shared by the stand-alone kernel and the fused GEMM so that both give
 // identical bits.  xlo / xhi and wlo / whi: the first eight bytes of the packed activation and weight rows, xhi

@@ -270,6 +270,7 @@ __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, Gemm
     }
 
     // ---- epilogue parameters: fetched now so that their latency hides behind the main loop
+    constexpr bool kLdsParams = false;
 #include "duq_stream_epilogue_fetch.inc"
     fetch_params();
 
@@ -305,10 +306,13 @@ __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, Gemm
 // registers, activations expanded into LDS, v_mfma_i32_32x32x32_i8, the same epilogue) without its K pipeline: a
 // problem whose rows hold at most 256 elements is one chunk, and a launch is its output stores (a 2048 x 2048 x 128
 // product moves 0.5 MB in and 8 MB out).  One activation buffer that doubles as the epilogue's staging area (37 KB
-// of LDS at 64 rows), only the steps the row length needs, whole-row stores; two workgroups share a CU (about 200
-// registers each) and overlap one another's loads, matrix work and stores.  (Persistent workgroups that request
-// the next tile's operands before the current tile's epilogue measured slower, 93 against 86 us on 32 products of
-// 2048 x 2048 x 128: the loop-carried wait for those loads also waits for the stores issued after them.)
+// of LDS at 64 rows), only the steps the row length needs, whole-row stores; up to four workgroups share a CU and
+// overlap one another's loads, matrix work and stores.  (Persistent workgroups that request the next tile's operands
+// before the current tile's epilogue measured slower, 93 against 86 us on 32 products of 2048 x 2048 x 128: the
+// loop-carried wait for those loads also waits for the stores issued after them.)  The epilogue's per-row parameters go
+// through LDS, one 16-byte read for four rows, instead of a register per row and parameter: 112 registers instead of
+// 148 and no loads of single values at the tile's head (32 products of 2048 x 2048 x 128, asymmetric: 71 -> 67 us;
+// K = 64: 60 -> 52).
 template <int TM, int EPI, bool BIAS>
 __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, GemmParams tail)
 {
@@ -353,6 +357,7 @@ __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, G
         const uint32_t row = (tid >> 3) + j * 32;
         xreg[j] = buf_load16(rX, xq * 16 < kbytes ? row * kbytes + xq * 16 : kOobOffset, 0);
     }
+    constexpr bool kLdsParams = true;
 #include "duq_stream_epilogue_fetch.inc"
     fetch_params();
 #pragma unroll

@@ -166,6 +166,7 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
     };
     // the part of the tile that this wavefront finishes
     const uint32_t wm0 = m0 + wm * (32 * WTM) + (ks >> 1) * (32 * TM), wn0 = n0 + wn * (32 * WTN) + (ks & 1u) * (32 * TN);
+    constexpr bool kLdsParams = false;
 #include "duq_stream_epilogue_fetch.inc"
     if (!LATE) fetch_params();
     wait_stages(std::integral_constant<int, NST - 1>{});
