@@ -1248,3 +1248,70 @@ def quantize_linear8bit_forward(x, w, w_tiled, w_scale, w_zeros, bias=None):
     if st:
         _lib.check(st, name)
     return y
+
+
+# ---- weight preparation (from_linear / from_float of the layers) ---------------------------------
+
+
+def _weight_rows(name, w, dtype, unit, split):
+    """Check of a weight [N, K] for the one-pass kernels; (N, K, its device)."""
+    if not isinstance(w, torch.Tensor):
+        raise RuntimeError(f"{name}: argument #0 is not a tensor")
+    _fast_check(name, "w", w, dtype, None)
+    if w.dim() != 2 or w.shape[1] % unit or split >= w.shape[1]:
+        raise RuntimeError(f"{name}: expected w [N, K] with K % {unit} == 0 and K > {split}, got {tuple(w.shape)}")
+    return w.shape[0], w.shape[1], w.device
+
+
+def weight_takes_one_pass(w: torch.Tensor, dtype=_F16) -> bool:
+    """Whether a weight can go through the one-pass kernels (the layers use torch's operators for others)."""
+    return w.is_cuda and w.dtype is dtype and w.dim() == 2 and w.is_contiguous() and w.data_ptr() % 16 == 0 and \
+        w.shape[1] % 8 == 0 and 2 * _QUANT_COL_K <= w.shape[1] <= 131072 and 0 < w.shape[0] <= 1 << 22
+
+
+def weight_quant_asym(w: torch.Tensor, split: int = 0, shifted: bool = False):
+    """binary16 weight [N, K] -> (packed codes [N, K/2], [(scale [N, 1], zeros [N, 1][, row sums [N]]) per range]): the
+    asymmetric quantization over |w| of ``from_linear`` (linear.py:123-145, 262-297), or ``shifted`` the activation
+    quantizer's signed-shifted form.  split > 0: two ranges of input columns."""
+    name = "weight_quant_asym"
+    N, K, dev = _weight_rows(name, w, _F16, 8, split)
+    q = torch.empty((N, K // 2), dtype=_U8, device=dev)
+    ranges = []
+    for _ in range(2 if split else 1):
+        r = (torch.empty((N, 1), dtype=_F16, device=dev), torch.empty((N, 1), dtype=_F16, device=dev))
+        ranges.append(r + (torch.empty((N,), dtype=_I32, device=dev),) if shifted else r)
+    n = 3 if shifted else 2
+    ptrs = [t.data_ptr() for r in ranges for t in r] + [None] * (2 * n - n * len(ranges))
+    lib = _lib.load()
+    st = _launch(dev, lib.duq_weight_quant_asym_shifted if shifted else lib.duq_weight_quant_asym, w.data_ptr(), N, K, split,
+                 q.data_ptr(), *ptrs)
+    _lib.check(st, name)
+    return q, ranges
+
+
+def weight_quant_sym(w: torch.Tensor, scale_1: torch.Tensor, scale_2: torch.Tensor = None, split: int = 0):
+    """rint(w / scale) packed, with the caller's per-channel scales (linear.py:58-78, 185-206): (packed codes [N, K/2],
+    int32 [1] that is not 0 where a code is outside the int4 range)."""
+    name = "weight_quant_sym"
+    N, K, dev = _weight_rows(name, w, _F16, 8, split)
+    for t, what in ((scale_1, "scale_1"),) + (((scale_2, "scale_2"),) if split else ()):
+        _fast_check(name, what, t, _F16, dev)
+        if t.numel() != N:
+            _check_size0(name, t.reshape(-1), what, N)
+    q = torch.empty((N, K // 2), dtype=_U8, device=dev)
+    bad = torch.zeros(1, dtype=_I32, device=dev)
+    st = _launch(dev, _lib.load().duq_weight_quant_sym, w.data_ptr(), N, K, split, scale_1.data_ptr(),
+                 scale_2.data_ptr() if split else None, q.data_ptr(), bad.data_ptr())
+    _lib.check(st, name)
+    return q, bad
+
+
+def weight_quant_asym_8bit(w: torch.Tensor):
+    """float32 weight [N, K] -> (int8 codes 0..127, scale [N, 1], zeros [N, 1]) over |w| (linear.py:338-368)."""
+    name = "weight_quant_asym_8bit"
+    N, K, dev = _weight_rows(name, w, _F32, 4, 0)
+    q = torch.empty((N, K), dtype=_I8, device=dev)
+    s, z = torch.empty((N, 1), dtype=_F32, device=dev), torch.empty((N, 1), dtype=_F32, device=dev)
+    st = _launch(dev, _lib.load().duq_weight_quant_asym_8bit, w.data_ptr(), N, K, q.data_ptr(), s.data_ptr(), z.data_ptr())
+    _lib.check(st, name)
+    return q, s, z

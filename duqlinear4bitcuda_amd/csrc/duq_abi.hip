@@ -801,4 +801,50 @@ int duq_quantize_linear8bit_forward(const float *x, const int8_t *w, const int8_
     return duq::launch_gemm_s8(q, weight, tiled, M, N, K, nullptr, sx, zx, w_scale, w_zeros, bias, y, as_stream(stream));
 }
 
+static int check_weight(const void *w, const void *q, uint32_t N, uint32_t K, uint32_t split, uint32_t unit)
+{
+    if (!w || !q) return DUQ_E_NULL;
+    if (K % unit != 0 || (split && split >= K)) return DUQ_E_SHAPE;
+    if (K > 131072u || N > (1u << 22)) return DUQ_E_TOO_LARGE;
+    if (!aligned(w, 16) || !aligned(q, 4)) return DUQ_E_ALIGN;
+    return DUQ_OK;
+}
+
+int duq_weight_quant_asym(const duq_half *w, uint32_t N, uint32_t K, uint32_t split, uint8_t *q, duq_half *scale_1,
+                          duq_half *zeros_1, duq_half *scale_2, duq_half *zeros_2, duq_stream_t stream)
+{
+    if (N == 0 || K == 0) return DUQ_OK;
+    if (int e = check_weight(w, q, N, K, split, 8)) return e;
+    if (!scale_1 || !zeros_1 || (split && (!scale_2 || !zeros_2))) return DUQ_E_NULL;
+    return duq::launch_weight_rows(0, w, N, K, split, q, scale_1, zeros_1, nullptr, scale_2, zeros_2, nullptr, nullptr, as_stream(stream));
+}
+
+int duq_weight_quant_asym_shifted(const duq_half *w, uint32_t N, uint32_t K, uint32_t split, uint8_t *q, duq_half *scale_1,
+                                  duq_half *zeros_1, int32_t *rowsum_1, duq_half *scale_2, duq_half *zeros_2,
+                                  int32_t *rowsum_2, duq_stream_t stream)
+{
+    if (N == 0 || K == 0) return DUQ_OK;
+    if (int e = check_weight(w, q, N, K, split, 8)) return e;
+    if (!scale_1 || !zeros_1 || !rowsum_1 || (split && (!scale_2 || !zeros_2 || !rowsum_2))) return DUQ_E_NULL;
+    return duq::launch_weight_rows(1, w, N, K, split, q, scale_1, zeros_1, rowsum_1, scale_2, zeros_2, rowsum_2, nullptr, as_stream(stream));
+}
+
+int duq_weight_quant_sym(const duq_half *w, uint32_t N, uint32_t K, uint32_t split, const duq_half *scale_1,
+                         const duq_half *scale_2, uint8_t *q, int32_t *bad, duq_stream_t stream)
+{
+    if (N == 0 || K == 0) return DUQ_OK;
+    if (int e = check_weight(w, q, N, K, split, 8)) return e;
+    if (!scale_1 || (split && !scale_2) || !bad) return DUQ_E_NULL;
+    return duq::launch_weight_rows(2, w, N, K, split, q, const_cast<duq_half *>(scale_1), nullptr, nullptr,
+                                   const_cast<duq_half *>(scale_2), nullptr, nullptr, bad, as_stream(stream));
+}
+
+int duq_weight_quant_asym_8bit(const float *w, uint32_t N, uint32_t K, int8_t *q, float *scale, float *zeros, duq_stream_t stream)
+{
+    if (N == 0 || K == 0) return DUQ_OK;
+    if (int e = check_weight(w, q, N, K, 0, 4)) return e;
+    if (!scale || !zeros) return DUQ_E_NULL;
+    return duq::launch_weight_rows8(w, N, K, q, scale, zeros, as_stream(stream));
+}
+
 }  // extern "C"

@@ -200,4 +200,10 @@ int launch_gemm_s8(const int8_t *A, const int8_t *B, bool b_tiled, uint32_t M, u
                    float *y, hipStream_t stream);
 int launch_weight_tile8(const int8_t *w, uint32_t N, uint32_t K, int8_t *out, hipStream_t stream);
 
+// Weight preparation (duq_weight.hip).  kind 0: asymmetric over |w|, 1: signed-shifted, 2: symmetric with given scales s1,
+// s2.  split: first column of the second range (0: one range, parameters s1, z1, r1).  cols % 8 == 0.
+int launch_weight_rows(int kind, const uint16_t *w, uint32_t rows, uint32_t cols, uint32_t split, uint8_t *q, uint16_t *s1,
+                       uint16_t *z1, int32_t *r1, uint16_t *s2, uint16_t *z2, int32_t *r2, int32_t *bad, hipStream_t stream);
+int launch_weight_rows8(const float *w, uint32_t rows, uint32_t cols, int8_t *q, float *scale, float *zero, hipStream_t stream);
+
 }  // namespace duq

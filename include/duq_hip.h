@@ -489,6 +489,30 @@ int duq_quantize_linear8bit_forward(const float *x, const int8_t *w, const int8_
                                     const float *w_zeros, const float *bias, uint32_t M, uint32_t N, uint32_t K, float *y,
                                     void *workspace, uint64_t workspace_bytes, duq_stream_t stream);
 
+/* ---- weight preparation ----------------------------------------------------------------- */
+
+/* A layer's binary16 weight [N,K] -> packed codes [N,K/2] and per-channel parameters [N] in one pass, with the bits that the
+ * torch statements of the reference's from_linear / from_float give on a GPU (qlinear4bit/nn/linear.py:58-78, 123-145,
+ * 185-206, 262-297).  split > 0: input columns below it take the first set of parameters, the others the second (the
+ * dual-uniform layers); split = 0: one range, its parameters in the first set, the second NULL.  K % 8 == 0, w 16-byte and
+ * q 4-byte aligned, split < K.
+ *   asym     statistics over |w|: scale = h(h(max - min) / 15), zero = rint(h(-min / scale)), unsigned codes
+ *            clamp(h(rint(h(w / scale)) + zero), 0, 15)
+ *   shifted  the signed-shifted form of duq_quantize_rows_asym_shifted per range, with the sums of the range's codes
+ *   sym      rint(h(w / scale)) as int8 with the given scales, packed; *bad (int32, set to 0 by the caller) becomes 1 where a
+ *            code is outside [-8, 7] */
+int duq_weight_quant_asym(const duq_half *w, uint32_t N, uint32_t K, uint32_t split, uint8_t *q, duq_half *scale_1,
+                          duq_half *zeros_1, duq_half *scale_2, duq_half *zeros_2, duq_stream_t stream);
+int duq_weight_quant_asym_shifted(const duq_half *w, uint32_t N, uint32_t K, uint32_t split, uint8_t *q, duq_half *scale_1,
+                                  duq_half *zeros_1, int32_t *rowsum_1, duq_half *scale_2, duq_half *zeros_2,
+                                  int32_t *rowsum_2, duq_stream_t stream);
+int duq_weight_quant_sym(const duq_half *w, uint32_t N, uint32_t K, uint32_t split, const duq_half *scale_1,
+                         const duq_half *scale_2, uint8_t *q, int32_t *bad, duq_stream_t stream);
+/* float32 weight [N,K] -> int8 codes 0..127 over |w| (qlinear4bit/nn/linear.py:338-368): scale = (max - min) / 127 (times the
+ * rounded reciprocal, as torch divides by a scalar on a GPU), zero = rint(-min / scale), clamp(rint(w / scale) + zero, 0,
+ * 127).  K % 4 == 0, w 16-byte and q 4-byte aligned. */
+int duq_weight_quant_asym_8bit(const float *w, uint32_t N, uint32_t K, int8_t *q, float *scale, float *zeros, duq_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
