@@ -36,6 +36,9 @@ def _launch(dev: torch.device, fn, *args):
         return fn(*args, _raw_stream(idx))
 
 
+_own_launch = _launch   # (a tracer may replace _launch to see every call: no call is then taken past it)
+
+
 def _host_for(entry: str):
     """The native host module (csrc/duq_host.cpp) for calls that end in that entry point, or None where the function
     on the loaded library was replaced by a Python one (a tracer's): the call then goes through that."""

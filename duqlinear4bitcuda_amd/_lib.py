@@ -33,6 +33,9 @@ PROTOTYPES = {
     "duq_asym_batch_dequant_host": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_u32, _c_u32, _c_u32, _c_p, _c_p],
     "duq_batch_linear4bit_forward": [_c_i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_u32, _c_u32,
                                      _c_u32, _c_u32, _c_p, _c_p],
+    "duq_quantize_product_workspace_bytes": [_c_i32, _c_u32, _c_u32, _c_u32, _c_u32],  # returns uint64_t
+    "duq_quantize_product": [_c_i32, _c_p, _c_p, _c_u32, _c_u32, _c_u32, _c_u32, ctypes.c_float, _c_i32, ctypes.c_float, _c_i32,
+                             _c_p, _c_p, ctypes.c_uint64, _c_p],
     "duq_sym_dequant_host": [_c_p, _c_p, _c_p, _c_u32, _c_u32, _c_p, _c_p],
     "duq_sym_dual_dequant_host": [_c_p, _c_p, _c_p, _c_p, _c_u32, _c_u32, _c_p, _c_p],
     "duq_asym_dequant_host": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_u32, _c_u32, _c_p, _c_p],
@@ -119,6 +122,7 @@ def load():
     lib.duq_linear4bit_dual_rowsum_workspace_bytes.restype = ctypes.c_uint64
     lib.duq_quantize_linear4bit_asym_workspace_bytes.restype = ctypes.c_uint64
     lib.duq_quantize_linear8bit_workspace_bytes.restype = ctypes.c_uint64
+    lib.duq_quantize_product_workspace_bytes.restype = ctypes.c_uint64
     lib.duq_status_string.argtypes = [ctypes.c_int]
     lib.duq_status_string.restype = ctypes.c_char_p
     _lib = lib
@@ -126,6 +130,22 @@ def load():
 
 
 _host = None
+
+
+def _install_calls(native):
+    """The native ``__call__`` of the module classes (``install`` in ``csrc/duq_host.cpp``)."""
+    from torch.nn.modules import module as m
+
+    from . import _HIP, nn
+    kinds = ((nn.SymQuantizer,), (nn.Linear4bitSQ, nn.Linear4bitDUSQ),
+             (nn.Linear4bitASQ, nn.LinearQuant4bitDUASQ, nn.Linear4bitASQRowSum, nn.LinearQuant4bitDUASQRowSum),
+             (nn.LinearQuant8bitASQ,), (nn.SymQuantMatMul,), (nn.AsymQuantMatMul,))
+    classes = [(cls, kind) for kind, group in enumerate(kinds) for cls in group] + [(nn.AsymQuantizer, -1)]
+    lib = load()
+    native.install(tuple(c for c in classes if c[0].forward.__module__ == c[0].__module__),   # (forwards as they are written there)
+                   (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks, m._global_backward_pre_hooks),
+                   m.Module, (_HIP, _HIP._own_launch), (lib, lib._FuncPtr),
+                   (nn.SymQuantizer, nn.AsymQuantizer, nn.AsymQuantizer8bit))
 
 
 def host():
@@ -138,6 +158,7 @@ def host():
         from . import _duq_host
         from .tools.tensor_utils import PackedQuantizedTensor
         _duq_host.setup(PackedQuantizedTensor, check)
+        _install_calls(_duq_host)
         _host = _duq_host
     return _host
 

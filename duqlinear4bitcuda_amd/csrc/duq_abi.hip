@@ -409,6 +409,45 @@ int duq_batch_linear4bit_forward(int32_t mode, const uint8_t *xq, const duq_half
     return DUQ_OK;
 }
 
+uint64_t duq_quantize_product_workspace_bytes(int32_t mode, uint32_t batch_count, uint32_t M, uint32_t N, uint32_t K)
+{
+    const uint64_t rows = (uint64_t)batch_count * ((uint64_t)M + N);
+    return up16(rows * (K / 2)) + up16(rows * 2) * (mode == DUQ_EPI_ASYM ? 2 : 1);
+}
+
+int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uint32_t batch_count, uint32_t M, uint32_t N, uint32_t K,
+                         float clip_a, int32_t qmax_a, float clip_b, int32_t qmax_b, duq_half *y, void *workspace,
+                         uint64_t workspace_bytes, duq_stream_t stream)
+{
+    if (mode != DUQ_EPI_SYM && mode != DUQ_EPI_ASYM) return DUQ_E_MODE;
+    if (int e = check_qmax(qmax_a)) return e;
+    if (int e = check_qmax(qmax_b)) return e;
+    if (batch_count == 0 || M == 0 || N == 0) return DUQ_OK;
+    if (int e = check_gemm(a, b, M, N, K)) return e;
+    if (K == 0) return DUQ_E_KALIGN;
+    const uint64_t rows_a = (uint64_t)batch_count * M, rows_b = (uint64_t)batch_count * N, rows = rows_a + rows_b;
+    if (rows > 0x7FFFFFFFull) return DUQ_E_TOO_LARGE;
+    if (!y || !workspace) return DUQ_E_NULL;
+    if (!aligned(workspace, 16)) return DUQ_E_ALIGN;
+    if (workspace_bytes < duq_quantize_product_workspace_bytes(mode, batch_count, M, N, K)) return DUQ_E_SHAPE;
+    const bool asym = mode == DUQ_EPI_ASYM;
+    uint8_t *q = static_cast<uint8_t *>(workspace);
+    duq_half *s = reinterpret_cast<duq_half *>(q + up16(rows * (K / 2)));
+    duq_half *z = asym ? s + up16(rows * 2) / 2 : nullptr;
+    if (asym || (clip_a == clip_b && qmax_a == qmax_b)) {
+        if (int e = duq::launch_quantize_two(a, (uint32_t)rows_a, b, (uint32_t)rows_b, K, asym, asym ? 1.0f : clip_a,
+                                             asym ? 15 : qmax_a, q, s, z, as_stream(stream)))
+            return e;
+    } else {
+        if (int e = duq::launch_quantize_rows_sym(a, (uint32_t)rows_a, K, clip_a, qmax_a, q, s, nullptr, as_stream(stream))) return e;
+        if (int e = duq::launch_quantize_rows_sym(b, (uint32_t)rows_b, K, clip_b, qmax_b, q + rows_a * (K / 2), s + rows_a, nullptr,
+                                                  as_stream(stream)))
+            return e;
+    }
+    return duq_batch_linear4bit_forward(mode, q, s, z, q + rows_a * (K / 2), s + rows_a, asym ? z + rows_a : nullptr, nullptr, nullptr,
+                                        nullptr, batch_count, M, N, K, y, stream);
+}
+
 int duq_probe_read(const void *src, uint64_t bytes, uint32_t *sink, duq_stream_t stream)
 {
     if (bytes == 0) return DUQ_OK;

@@ -159,17 +159,20 @@ bool still_current(FusedCall *c, PyObject *buffers)
     return THPVariable_Unpack(PyTuple_GET_ITEM(c->tensors, 0)).const_data_ptr() == c->layer.w;
 }
 
-PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip, int qmax)
+// min_tiles: the module's fp6_min_tiles, negative where the caller does not know it
+PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip, int qmax, int64_t min_tiles = -1)
 {
     duq_fused_layer l = c->layer;
     if (x.dim() == 0 || x.size(-1) != static_cast<int64_t>(l.K) || x.get_device() != c->dev || l.K % 64) return none();
     const int64_t M = x.numel() / l.K;
     if (M < 1 || M > c->max_rows || current_device() != c->dev) return none();
-    // more than 64 rows of a layer with a 6-bit float shadow: the Python side decides which path they take
+    // more than 64 rows of a layer with a 6-bit float shadow: those of the 6-bit float path are not run here (the rule
+    // of the layer's _fp6_wanted)
     static PyObject *const shadow_name = PyUnicode_InternFromString("weight_shadow");
     if (M > 64) {
         PyObject *s = PyDict_GetItemWithError(buffers, shadow_name);
-        if (s && s != Py_None) return none();
+        const int64_t tiles = (M + 63) / 64 * ((l.N + 255) / 256);
+        if (s && s != Py_None && (min_tiles < 0 || tiles >= min_tiles || (M > 256 && 8 * tiles >= 5 * min_tiles))) return none();
     }
     const int64_t bytes = staging_of(c, M);
     l.clip = clip;
@@ -187,27 +190,33 @@ PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip,
     return wrap(std::move(y));
 }
 
-// take(buffers, packed): the layer's result for a PackedQuantizedTensor that was handed on unquantized
+int64_t tiles_argument(PyObject *const *a, Py_ssize_t n)
+{
+    return n == 3 && PyLong_Check(a[2]) ? PyLong_AsLongLong(a[2]) : -1;
+}
+
+// take(buffers, packed[, the module's fp6_min_tiles]): the layer's result for a PackedQuantizedTensor that was handed on unquantized
 PyObject *fused_take(PyObject *self, PyObject *const *a, Py_ssize_t n)
 {
     FusedCall *c = reinterpret_cast<FusedCall *>(self);
-    if (n != 2 || !PyDict_Check(a[0]) || reinterpret_cast<PyObject *>(Py_TYPE(a[1])) != g_packed) return none();
+    if (n < 2 || n > 3 || !PyDict_Check(a[0]) || reinterpret_cast<PyObject *>(Py_TYPE(a[1])) != g_packed) return none();
     PyObject *src = slot(a[1], kSrc), *version = slot(a[1], kVersion), *clip = slot(a[1], kClip), *qmax = slot(a[1], kQmax);
     if (!src || !version || !clip || !qmax || !PyFloat_Check(clip) || !PyLong_Check(qmax)) return none();
     const Tensor *x = plain(src, ScalarType::Half, c->dev);
     if (!x || x->is_inference() || static_cast<long>(x->_version()) != PyLong_AsLong(version) || !still_current(c, a[0])) return none();
     const Tensor held = *x;  // (another thread may quantize the packed tensor, which drops its rows)
-    return guarded([&] { return run_rows(c, a[0], held, static_cast<float>(PyFloat_AS_DOUBLE(clip)), static_cast<int>(PyLong_AsLong(qmax))); });
+    return guarded([&] { return run_rows(c, a[0], held, static_cast<float>(PyFloat_AS_DOUBLE(clip)), static_cast<int>(PyLong_AsLong(qmax)),
+                                         tiles_argument(a, n)); });
 }
 
-// take_rows(buffers, x): the same for a layer with its own quantizer
+// take_rows(buffers, x[, fp6_min_tiles]): the same for a layer with its own quantizer
 PyObject *fused_take_rows(PyObject *self, PyObject *const *a, Py_ssize_t n)
 {
     FusedCall *c = reinterpret_cast<FusedCall *>(self);
-    if (n != 2 || !PyDict_Check(a[0])) return none();
+    if (n < 2 || n > 3 || !PyDict_Check(a[0])) return none();
     const Tensor *x = plain(a[1], ScalarType::Half, c->dev);
     if (!x || reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16 || !still_current(c, a[0])) return none();
-    return guarded([&] { return run_rows(c, a[0], *x, 1.0f, 6); });
+    return guarded([&] { return run_rows(c, a[0], *x, 1.0f, 6, tiles_argument(a, n)); });
 }
 
 // FusedCall(mode, N, K, device index, max_rows, addresses of (w, s1, z1, s2, z2, adj1, adj2, bias), names, tensors)
@@ -434,17 +443,15 @@ PyObject *m_linear4_batched(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
-// linear8(x, scale_x, zeros_x, w, w_tiled, w_scale, w_zeros, bias, N, stream): int8 codes with their scales and zeros
-// (w_tiled not None: the GEMM reads that copy and w is not looked at), or float32 rows (scale_x and zeros_x None) that
-// the call quantizes first
-PyObject *m_linear8(PyObject *, PyObject *const *a, Py_ssize_t n)
+// int8 codes with their scales and zeros (w_tiled not None: the GEMM reads that copy and w is not looked at), or float32
+// rows (scale_x and zeros_x None) that the call quantizes first.  null stream: the current one.
+PyObject *linear8(PyObject *const *a, int64_t N, const duq_stream_t *stream)
 {
-    if (n != 10 || !PyLong_Check(a[8])) return none();
     const bool quantize = a[1] == Py_None;
     const Tensor *x = plain(a[0], quantize ? ScalarType::Float : ScalarType::Char, -1);
     if (!x || x->dim() == 0 || x->numel() == 0) return none();
     const int dev = static_cast<int>(x->get_device());
-    const int64_t K = x->size(-1), M = x->numel() / K, N = PyLong_AsLongLong(a[8]);
+    const int64_t K = x->size(-1), M = x->numel() / K;
     if (N <= 0 || M > UINT32_MAX || N > UINT32_MAX || K > UINT32_MAX) return none();
     const void *p[8] = {};
     if (!operand(a[1], ScalarType::Float, dev, M, quantize, &p[1]) || !operand(a[2], ScalarType::Float, dev, M, quantize, &p[2]) ||
@@ -454,8 +461,8 @@ PyObject *m_linear8(PyObject *, PyObject *const *a, Py_ssize_t n)
         !operand(a[7], ScalarType::Float, dev, N, true, &p[7]))
         return none();
     if (p[3] && THPVariable_Unpack(a[3]).dim() != 2) return none();
-    const duq_stream_t st = stream_of(a[9]);
     return guarded([&]() -> PyObject * {
+        const duq_stream_t st = stream ? *stream : c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream();
         Tensor y = output(*x, N, ScalarType::Float);
         const uint32_t m = static_cast<uint32_t>(M), nn = static_cast<uint32_t>(N), k = static_cast<uint32_t>(K);
         const int8_t *w = static_cast<const int8_t *>(p[3]), *wt = static_cast<const int8_t *>(p[4]);
@@ -475,6 +482,365 @@ PyObject *m_linear8(PyObject *, PyObject *const *a, Py_ssize_t n)
         if (e) return finish(e, quantize ? "quantize_linear8bit_forward" : "linear8bit_forward", nullptr);
         return wrap(std::move(y));
     });
+}
+
+// linear8(x, scale_x, zeros_x, w, w_tiled, w_scale, w_zeros, bias, N, stream)
+PyObject *m_linear8(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    if (n != 10 || !PyLong_Check(a[8])) return none();
+    const duq_stream_t st = stream_of(a[9]);
+    return linear8(a, PyLong_AsLongLong(a[8]), &st);
+}
+
+// ---- calls of modules ----------------------------------------------------------------------------------------
+// `__call__` of the framework's module classes: what torch.nn.Module.__call__ and the class's forward do in the plain
+// case (no hooks, no compiled or replaced forward, plain tensors, buffers as they were when the layer's call was
+// prepared), in one piece of native code: 0.2 us where the two Python frames cost 1 (quantizer and layer of a decode
+// step 6.6 -> 5.5 us).  Anything else goes to torch.nn.Module.__call__ as it is at that moment.
+
+enum Kind { kSymQuant, kSymLayer, kOwnLayer, kEightBit, kSymProduct, kAsymProduct };
+struct Entry {
+    PyTypeObject *type;
+    PyObject *forward;
+    Kind kind;
+};
+std::vector<Entry> *g_entries = nullptr;
+PyTypeObject *g_module_type = nullptr;           // torch.nn.Module
+PyObject *g_module_call[3], *g_module_call_names[3];  // what stands behind its __call__, and under which names
+std::vector<PyObject *> *g_global_hooks = nullptr;    // torch's dicts of hooks for every module
+PyObject *g_ops_dict = nullptr, *g_launch = nullptr;  // _HIP's namespace and the _launch function defined there
+PyObject *g_lib_dict = nullptr;                  // attributes of the ctypes library object
+PyTypeObject *g_funcptr = nullptr;               // ... and the type of its functions
+PyTypeObject *g_quant8_type = nullptr, *g_asym_type = nullptr, *g_sym_type = nullptr;
+
+struct Names {
+#define NAME(n) PyObject *n = PyUnicode_InternFromString(#n)
+    NAME(_forward_hooks);
+    NAME(_forward_pre_hooks);
+    NAME(_backward_hooks);
+    NAME(_backward_pre_hooks);
+    NAME(_compiled_call_impl);
+    NAME(forward);
+    NAME(_buffers);
+    NAME(_modules);
+    NAME(_decode);
+    NAME(native);
+    NAME(fused);
+    NAME(input_clip_ratio);
+    NAME(qmax);
+    NAME(shadow);
+    NAME(shadow_min_rows);
+    NAME(shifted);
+    NAME(defer_rows);
+    NAME(require_quantizer);
+    NAME(quantizer);
+    NAME(quantizer_A);
+    NAME(quantizer_B);
+    NAME(tiled);
+    NAME(one_call_rows);
+    NAME(fp6_min_tiles);
+    NAME(transpose_B);
+    NAME(weight);
+    NAME(weight_tiled);
+    NAME(weight_scales);
+    NAME(weight_zeros);
+    NAME(bias);
+    NAME(_tiled_key);
+    NAME(_launch);
+    NAME(duq_quantize_linear8bit_forward);
+    NAME(duq_quantize_product);
+    NAME(__call__);
+#undef NAME
+};
+const Names *g_names = nullptr;
+
+PyObject *get(PyObject *dict, PyObject *name) { return dict ? PyDict_GetItemWithError(dict, name) : nullptr; }
+
+// attribute of an instance: its own dict, then its class (plain values only; borrowed)
+PyObject *attr(PyObject *self, PyObject *dict, PyObject *name)
+{
+    PyObject *v = get(dict, name);
+    return v ? v : _PyType_Lookup(Py_TYPE(self), name);
+}
+
+PyObject *dict_of(PyObject *o)
+{
+    PyObject **d = _PyObject_GetDictPtr(o);
+    return d ? *d : nullptr;
+}
+
+bool empty_dict(PyObject *d) { return d && PyDict_Check(d) && PyDict_GET_SIZE(d) == 0; }
+
+// The entry of a module whose call is its class's forward and nothing else, or null.
+const Entry *plain_module(PyObject *self, PyObject *dict)
+{
+    const Entry *e = nullptr;
+    for (const Entry &k : *g_entries)
+        if (k.type == Py_TYPE(self)) e = &k;
+    const Names &n = *g_names;
+    if (!e || !dict || get(e->type->tp_dict, n.forward) != e->forward || get(dict, n.forward)) return nullptr;
+    for (PyObject *h : {n._forward_hooks, n._forward_pre_hooks, n._backward_hooks, n._backward_pre_hooks})
+        if (!empty_dict(get(dict, h))) return nullptr;
+    PyObject *compiled = get(dict, n._compiled_call_impl);
+    return compiled && compiled != Py_None ? nullptr : e;
+}
+
+bool plain_torch()
+{
+    for (int i = 0; i < 3; ++i)
+        if (get(g_module_type->tp_dict, g_module_call_names[i]) != g_module_call[i]) return false;
+    for (PyObject *d : *g_global_hooks)
+        if (PyDict_GET_SIZE(d)) return false;
+    return true;
+}
+
+// the library's own function under that name (a tracer may have put a Python one there)
+bool library_function(PyObject *name)
+{
+    PyObject *f = get(g_lib_dict, name);
+    return f && Py_TYPE(f) == g_funcptr;
+}
+
+PyObject *call_sym_quantizer(PyObject *self, PyObject *dict, PyObject *x)
+{
+    const Names &n = *g_names;
+    PyObject *a[6] = {x,
+                      attr(self, dict, n.defer_rows),
+                      get(dict, n.shadow),
+                      get(dict, n.shadow_min_rows),
+                      get(dict, n.input_clip_ratio),
+                      get(dict, n.qmax)};
+    for (PyObject *v : a)
+        if (!v) return none();
+    return m_defer(nullptr, a, 6);
+}
+
+PyObject *call_layer(PyObject *self, PyObject *dict, PyObject *x, bool own_quantizer)
+{
+    const Names &n = *g_names;
+    PyObject *decode = get(dict, n._decode), *buffers = get(dict, n._buffers);
+    if (!decode || decode == Py_None || !buffers || attr(self, dict, n.fused) != Py_True) return none();
+    if (own_quantizer && get(dict, n.require_quantizer) != Py_True) return none();
+    PyObject *native = PyObject_GetAttr(decode, n.native);
+    if (!native) return nullptr;
+    PyObject *r = none();
+    if (Py_TYPE(native) == &g_fused_type) {
+        Py_DECREF(r);
+        PyObject *tiles = attr(self, dict, n.fp6_min_tiles), *a[3] = {buffers, x, tiles ? tiles : Py_None};
+        r = own_quantizer ? fused_take_rows(native, a, 3) : fused_take(native, a, 3);
+    }
+    Py_DECREF(native);
+    return r;
+}
+
+PyObject *call_eight_bit(PyObject *self, PyObject *dict, PyObject *x)
+{
+    const Names &n = *g_names;
+    PyObject *buffers = get(dict, n._buffers), *modules = get(dict, n._modules), *rows = attr(self, dict, n.one_call_rows);
+    if (!buffers || !modules || !rows || !PyLong_Check(rows) || get(dict, n.require_quantizer) != Py_True ||
+        attr(self, dict, n.fused) != Py_True || !library_function(n.duq_quantize_linear8bit_forward))
+        return none();
+    PyObject *q = get(modules, n.quantizer), *qd = q ? dict_of(q) : nullptr;
+    if (!q || Py_TYPE(q) != g_quant8_type || !qd || get(qd, n.fused) != Py_True) return none();
+    PyObject *tiled = attr(self, dict, n.tiled), *w = get(buffers, n.weight), *wt = Py_None;
+    if (!w || (tiled != Py_True && tiled != Py_False)) return none();
+    const Tensor *px = plain(x, ScalarType::Float, -1), *pw = plain(w, ScalarType::Char, -1);
+    if (!px || !pw || pw->dim() != 2 || px->dim() == 0 || px->size(-1) != pw->size(1) || pw->size(1) % 32 ||
+        reinterpret_cast<uintptr_t>(px->const_data_ptr()) % 16 || px->numel() > PyLong_AsLongLong(rows) * pw->size(1) ||
+        px->get_device() != current_device())
+        return none();
+    if (tiled == Py_True) {  // the copy is the weight's as it is now: version, address, device (the layer's _tiled_weight)
+        PyObject *key = get(dict, n._tiled_key);
+        wt = get(buffers, n.weight_tiled);
+        if (!wt || wt == Py_None || !key || !PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || pw->is_inference() ||
+            PyLong_AsLong(PyTuple_GET_ITEM(key, 0)) != static_cast<long>(pw->_version()) ||
+            PyLong_AsVoidPtr(PyTuple_GET_ITEM(key, 1)) != pw->const_data_ptr() || !THPVariable_CheckExact(wt) ||
+            THPVariable_Unpack(wt).get_device() != pw->get_device()) {
+            PyErr_Clear();
+            return none();
+        }
+    }
+    PyObject *s = get(buffers, n.weight_scales), *z = get(buffers, n.weight_zeros), *bias = get(buffers, n.bias);
+    if (!s || !z) return none();
+    PyObject *a[8] = {x, Py_None, Py_None, w, wt, s, z, bias ? bias : Py_None};
+    return linear8(a, pw->size(0), nullptr);
+}
+
+// A product of activations: both quantizers of the module in their plain form, operands of one batch.
+PyObject *call_product(PyObject *self, PyObject *dict, PyObject *pa, PyObject *pb, bool asym)
+{
+    const Names &n = *g_names;
+    PyObject *modules = get(dict, n._modules);
+    if (!modules || attr(self, dict, n.fused) != Py_True || get(g_ops_dict, n._launch) != g_launch ||
+        !library_function(n.duq_quantize_product) || (asym && get(dict, n.transpose_B) != Py_False))
+        return none();
+    float clip[2] = {1.0f, 1.0f};
+    long qmax[2] = {6, 6};
+    PyObject *const names[2] = {n.quantizer_A, n.quantizer_B};
+    for (int i = 0; i < 2; ++i) {
+        PyObject *q = get(modules, names[i]), *qd = q ? dict_of(q) : nullptr;
+        if (!q || Py_TYPE(q) != (asym ? g_asym_type : g_sym_type) || !plain_module(q, qd) || get(qd, n.shadow) != Py_False) return none();
+        if (asym) {
+            if (get(qd, n.shifted) != Py_False) return none();
+        } else {
+            PyObject *c = get(qd, n.input_clip_ratio), *m = get(qd, n.qmax);
+            if (!c || !m || !PyFloat_Check(c) || !PyLong_Check(m)) return none();
+            clip[i] = static_cast<float>(PyFloat_AS_DOUBLE(c));
+            qmax[i] = PyLong_AsLong(m);
+            if (qmax[i] < 0 || qmax[i] > 7) {
+                PyErr_Clear();
+                return none();
+            }
+        }
+    }
+    const Tensor *a = plain(pa, ScalarType::Half, -1);
+    if (!a || a->dim() < 2) return none();
+    const int dev = static_cast<int>(a->get_device());
+    const Tensor *b = plain(pb, ScalarType::Half, dev);
+    if (!b || b->dim() < 2 || dev != current_device() || a->numel() == 0 || b->numel() == 0) return none();
+    const int64_t K = a->size(-1), N = b->size(-2);
+    int64_t batch = 1, M = a->size(-2);
+    if (b->size(-1) != K || K % 64 || K > 131008 || reinterpret_cast<uintptr_t>(a->const_data_ptr()) % 16 ||
+        reinterpret_cast<uintptr_t>(b->const_data_ptr()) % 16)
+        return none();
+    if (b->dim() > 2 || asym) {  // one product per entry of the same leading dimensions
+        if (a->dim() != b->dim()) return none();
+        for (int64_t d = 0; d < a->dim() - 2; ++d) {
+            if (a->size(d) != b->size(d)) return none();
+            batch *= a->size(d);
+        }
+    } else {
+        M = a->numel() / K;  // every row of A against one B
+    }
+    if (M > (1 << 24) || N > (1 << 22) || batch > INT32_MAX || batch * (M + N) > INT32_MAX) return none();
+    return guarded([&]() -> PyObject * {
+        const int mode = asym ? DUQ_EPI_ASYM : DUQ_EPI_SYM;
+        const uint32_t nb = static_cast<uint32_t>(batch), m = static_cast<uint32_t>(M), nn = static_cast<uint32_t>(N),
+                       k = static_cast<uint32_t>(K);
+        Tensor y = output(*a, N, ScalarType::Half);
+        const uint64_t bytes = duq_quantize_product_workspace_bytes(mode, nb, m, nn, k);
+        Scratch ws(bytes);
+        int e;
+        {
+            Unlocked u;
+            e = duq_quantize_product(mode, half(a->const_data_ptr()), half(b->const_data_ptr()), nb, m, nn, k, clip[0],
+                                     static_cast<int>(qmax[0]), clip[1], static_cast<int>(qmax[1]), out<duq_half>(y), ws.get(), bytes,
+                                     c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream());
+        }
+        if (e) return finish(e, "quantize_product", nullptr);
+        return wrap(std::move(y));
+    });
+}
+
+struct ModuleCall {
+    PyObject_HEAD
+    vectorcallfunc call;
+};
+
+PyObject *module_call(PyObject *, PyObject *const *a, size_t nargsf, PyObject *kwnames)
+{
+    const Py_ssize_t n = PyVectorcall_NARGS(nargsf);
+    if (!kwnames && n >= 2 && n <= 3 && plain_torch()) {
+        PyObject *dict = dict_of(a[0]);
+        const Entry *e = plain_module(a[0], dict);
+        const bool product = e && (e->kind == kSymProduct || e->kind == kAsymProduct);
+        if (e && n == (product ? 3 : 2)) {
+            PyObject *r = e->kind == kSymQuant   ? call_sym_quantizer(a[0], dict, a[1])
+                          : e->kind == kSymLayer ? call_layer(a[0], dict, a[1], false)
+                          : e->kind == kOwnLayer ? call_layer(a[0], dict, a[1], true)
+                          : e->kind == kEightBit ? call_eight_bit(a[0], dict, a[1])
+                                                 : call_product(a[0], dict, a[1], a[2], e->kind == kAsymProduct);
+            if (r != Py_None) return r;
+            Py_DECREF(r);
+        }
+    }
+    // torch.nn.Module.__call__(self, ...)
+    PyObject *f = PyObject_GetAttr(reinterpret_cast<PyObject *>(g_module_type), g_names->__call__);
+    if (!f) return nullptr;
+    PyObject *r = PyObject_Vectorcall(f, a, static_cast<size_t>(n), kwnames);
+    Py_DECREF(f);
+    return r;
+}
+
+PyObject *module_call_get(PyObject *self, PyObject *obj, PyObject *)
+{
+    if (!obj || obj == Py_None) {
+        Py_INCREF(self);
+        return self;
+    }
+    return PyMethod_New(self, obj);
+}
+
+PyTypeObject g_module_call_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// install(classes, torch's hook dicts, torch.nn.Module, (_HIP module, its _launch), (ctypes library, type of its functions),
+// (SymQuantizer, AsymQuantizer, AsymQuantizer8bit)): `classes` is a tuple of (class, kind as in Kind, or -1 for a class
+// that only a product looks at); gives every one of them the native __call__
+PyObject *m_install(PyObject *, PyObject *args)
+{
+    PyObject *classes, *hooks, *module, *ops, *lib, *launch, *funcptr, *sym, *asym, *quant8;
+    if (!PyArg_ParseTuple(args, "O!O!O!(OO)(OO!)(O!O!O!)", &PyTuple_Type, &classes, &PyTuple_Type, &hooks, &PyType_Type, &module, &ops,
+                          &launch, &lib, &PyType_Type, &funcptr, &PyType_Type, &sym, &PyType_Type, &asym, &PyType_Type, &quant8))
+        return nullptr;
+    PyObject *lib_dict = dict_of(lib), *ops_dict = dict_of(ops);
+    if (g_names || !lib_dict || !ops_dict) {
+        PyErr_SetString(PyExc_RuntimeError, "install: once, with a module and a library object");
+        return nullptr;
+    }
+    const Names *names = new Names();
+    bool found = true;
+    static const char *const call_names[3] = {"__call__", "_wrapped_call_impl", "_call_impl"};
+    PyObject *module_dict = reinterpret_cast<PyTypeObject *>(module)->tp_dict;
+    for (int i = 0; i < 3; ++i) {
+        g_module_call_names[i] = PyUnicode_InternFromString(call_names[i]);
+        g_module_call[i] = get(module_dict, g_module_call_names[i]);
+        Py_XINCREF(g_module_call[i]);
+        if (!g_module_call[i]) found = false;
+    }
+    auto *global_hooks = new std::vector<PyObject *>();
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(hooks); ++i) {
+        PyObject *d = PyTuple_GET_ITEM(hooks, i);
+        if (!PyDict_Check(d)) found = false;
+        Py_INCREF(d);
+        global_hooks->push_back(d);
+    }
+    auto *entries = new std::vector<Entry>();
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(classes); ++i) {
+        PyObject *cls;
+        int kind;
+        if (!PyArg_ParseTuple(PyTuple_GET_ITEM(classes, i), "O!i", &PyType_Type, &cls, &kind)) return nullptr;
+        PyTypeObject *t = reinterpret_cast<PyTypeObject *>(cls);
+        PyObject *forward = get(t->tp_dict, names->forward);
+        if (!forward) found = false;
+        Py_INCREF(cls);
+        Py_XINCREF(forward);
+        entries->push_back(Entry{t, forward, static_cast<Kind>(kind)});
+    }
+    if (!found) {
+        PyErr_SetString(PyExc_RuntimeError, "install: a function or dictionary is not where it was expected");
+        return nullptr;
+    }
+    for (PyObject *o : {module, launch, ops_dict, lib_dict, funcptr, sym, asym, quant8}) Py_INCREF(o);
+    g_module_type = reinterpret_cast<PyTypeObject *>(module);
+    g_ops_dict = ops_dict;
+    g_launch = launch;
+    g_lib_dict = lib_dict;
+    g_funcptr = reinterpret_cast<PyTypeObject *>(funcptr);
+    g_sym_type = reinterpret_cast<PyTypeObject *>(sym);
+    g_asym_type = reinterpret_cast<PyTypeObject *>(asym);
+    g_quant8_type = reinterpret_cast<PyTypeObject *>(quant8);
+    g_global_hooks = global_hooks;
+    g_entries = entries;
+    g_names = names;
+    ModuleCall *call = PyObject_New(ModuleCall, &g_module_call_type);
+    if (!call) return nullptr;
+    call->call = module_call;
+    int bad = 0;
+    for (const Entry &e : *entries)
+        bad |= e.kind >= 0 ? PyObject_SetAttr(reinterpret_cast<PyObject *>(e.type), names->__call__, reinterpret_cast<PyObject *>(call)) : 0;
+    Py_DECREF(call);
+    if (bad) return nullptr;
+    Py_RETURN_NONE;
 }
 
 // setup(PackedQuantizedTensor, check): the class defer() makes instances of, and what raises for a status
@@ -505,6 +871,7 @@ PyMethodDef g_methods[] = {FAST("defer", m_defer),
                            FAST("linear4_batched", m_linear4_batched),
                            FAST("linear8", m_linear8),
                            {"setup", m_setup, METH_VARARGS, nullptr},
+                           {"install", m_install, METH_VARARGS, nullptr},
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_duq_host", "host side of the ops (csrc/duq_host.cpp)", -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
@@ -519,6 +886,13 @@ PyMODINIT_FUNC PyInit__duq_host(void)
     g_fused_type.tp_dealloc = fused_dealloc;
     g_fused_type.tp_methods = g_fused_methods;
     if (PyType_Ready(&g_fused_type) < 0) return nullptr;
+    g_module_call_type.tp_name = "_duq_host.ModuleCall";
+    g_module_call_type.tp_basicsize = sizeof(ModuleCall);
+    g_module_call_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL | Py_TPFLAGS_METHOD_DESCRIPTOR;
+    g_module_call_type.tp_vectorcall_offset = offsetof(ModuleCall, call);
+    g_module_call_type.tp_call = PyVectorcall_Call;
+    g_module_call_type.tp_descr_get = module_call_get;
+    if (PyType_Ready(&g_module_call_type) < 0) return nullptr;
     PyObject *m = PyModule_Create(&g_module);
     if (!m) return nullptr;
     Py_INCREF(&g_fused_type);

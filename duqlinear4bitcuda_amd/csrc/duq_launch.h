@@ -23,6 +23,10 @@ int launch_quantize_rows_sym(const uint16_t *x, uint32_t rows, uint32_t cols, fl
 // signed-shifted form (code - 8, zero - 8) plus the per-row sum of the shifted codes.
 int launch_quantize_rows_asym(const uint16_t *x, uint32_t rows, uint32_t cols, uint8_t *q, uint16_t *scale,
                               uint16_t *zeros, int32_t *rowsum, uint8_t *bf6, hipStream_t stream);
+// The rows of two tensors of one width in one launch, without the shadow: codes, scales (and zero points) of x2's rows
+// follow those of x's.
+int launch_quantize_two(const uint16_t *x, uint32_t rows, const uint16_t *x2, uint32_t rows2, uint32_t cols, bool asym, float clip,
+                        int qmax, uint8_t *q, uint16_t *scale, uint16_t *zeros, hipStream_t stream);
 
 // Epilogue description shared by the stand-alone dequant kernels and the fused GEMM.
 // mode: 0 sym, 1 asym, 2 sym-dual, 3 asym-dual, 4 asym with row-sum zero-point correction, 5 the same for the

@@ -214,6 +214,8 @@ struct RowParams {
     float clip;
     int qmax;
     int32_t *rowsum;  // asym only: non-null selects the signed-shifted form (code - 8, zero - 8, sum of codes)
+    const uint16_t *x2;  // two tensors in one launch (kTwo): rows from `split` on are those of x2, outputs go on after x's
+    uint32_t split;
 };
 static_assert(offsetof(RowParams, rowsum) == kHeadBytes, "the fields delivered in registers");
 
@@ -242,11 +244,29 @@ __device__ __forceinline__ v6u bf6_block(const uint32_t (&w)[4])
     return __builtin_amdgcn_cvt_scalef32_pk32_bf6_f16(__builtin_bit_cast(v32h, pairs), 1.0f);
 }
 
-// BF6: the kernel also writes the E3M2 shadow of the codes (blocks of 32 elements = four
+// What a row kernel writes and reads: the codes; codes and (or only) their E3M2 shadow; the codes of two tensors of one
+// width, as the operands of a product of activations are (one launch instead of two: 3.3 us of host time and a gap on
+// the GPU, more than the kernel itself takes for the products of one decode step).
+enum RowForm { kCodes = 0, kShadow = 1, kTwo = 2 };
+
+// the first unit of a row
+template <int FORM>
+__device__ __forceinline__ const v4u *row_units(const RowParams &p, uint32_t row)
+{
+    const uint16_t *x = p.x;
+    if (FORM == kTwo && row >= p.split) {
+        x = p.x2;
+        to_global(x);
+        row -= p.split;
+    }
+    return reinterpret_cast<const v4u *>(x + (uint64_t)row * p.cols);
+}
+
+// kShadow: the kernel also writes the E3M2 shadow of the codes (blocks of 32 elements = four
 // consecutive units); the packed words of a row meet in LDS so that the loads keep the
 // coalesced unit-per-lane pattern and a lane still converts whole blocks.  The packed nibbles
 // are written only when p.q is given.
-template <int WAVES, bool ASYM, bool CACHED, bool BF6 = false>
+template <int WAVES, bool ASYM, bool CACHED, int FORM>
 __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL, RowParams tail)
 {
     RowParams p = with_head(tail, DUQ_HEAD_USE);
@@ -256,6 +276,7 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
     to_global(p.zeros);
     to_global(p.bf6);
     constexpr int T = WAVES * 64;
+    constexpr bool BF6 = FORM == kShadow;
     __shared__ float red[3][WAVES];
     __shared__ int red_sum[WAVES];
     const bool shifted = ASYM && p.rowsum != nullptr;
@@ -263,7 +284,7 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
     const uint32_t row = blockIdx.x;
     const uint32_t tid = threadIdx.x;
     const uint32_t nunits = p.cols >> 3;  // units of 8 elements
-    const v4u *xrow = reinterpret_cast<const v4u *>(p.x + (uint64_t)row * p.cols);
+    const v4u *xrow = row_units<FORM>(p, row);
     uint32_t *qrow = reinterpret_cast<uint32_t *>(p.q + (uint64_t)row * (p.cols >> 1));
     __shared__ __attribute__((aligned(16))) uint32_t words[BF6 && CACHED ? T * kMaxUnits : 4];
     // unit held in register slot i
@@ -412,7 +433,7 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
 // lanes at work).  Here LANES lanes hold a row, two units each, a workgroup takes 256 / LANES rows at a time and PASSES
 // times as many in all, every load of them requested up front; the same launch takes 7.4 us.  Two units per lane, not
 // one, because the constants of a row are computed by each of its lanes and cost as much as two units' codes.
-template <int LANES, int PASSES, bool ASYM>
+template <int LANES, int PASSES, bool ASYM, int FORM>
 __global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL, RowParams tail)
 {
     RowParams p = with_head(tail, DUQ_HEAD_USE);
@@ -424,7 +445,6 @@ __global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL,
     const bool shifted = ASYM && p.rowsum != nullptr;
     const uint32_t nunits = p.cols >> 3;  // <= 2 * LANES
     const uint32_t u0 = threadIdx.x % LANES, row0 = blockIdx.x * (kRows * PASSES) + threadIdx.x / LANES;
-    const v4u *x4 = reinterpret_cast<const v4u *>(p.x);
     uint32_t *q32 = reinterpret_cast<uint32_t *>(p.q);
 
     v4u regs[PASSES][2];
@@ -433,7 +453,7 @@ __global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL,
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const uint32_t row = row0 + i * kRows, u = u0 + j * LANES;
-            regs[i][j] = row < p.rows && u < nunits ? __builtin_nontemporal_load(&x4[(uint64_t)row * nunits + u]) : v4u{0u, 0u, 0u, 0u};
+            regs[i][j] = row < p.rows && u < nunits ? __builtin_nontemporal_load(row_units<FORM>(p, row) + u) : v4u{0u, 0u, 0u, 0u};
         }
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
@@ -487,7 +507,7 @@ __global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL,
     }
 }
 
-template <bool ASYM>
+template <bool ASYM, int FORM>
 static int launch_short_rows(const RowParams &p, hipStream_t stream)
 {
     // four passes where that still leaves two workgroups per CU, one otherwise (few rows: latency)
@@ -495,9 +515,9 @@ static int launch_short_rows(const RowParams &p, hipStream_t stream)
     do {                                                                                                              \
         const uint64_t groups = ((uint64_t)p.rows * L + 255) / 256;                                                   \
         if (groups >= 2048)                                                                                           \
-            DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, 4, ASYM>), dim3((uint32_t)((groups + 3) / 4)), dim3(256), 0, stream, p); \
+            DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, 4, ASYM, FORM>), dim3((uint32_t)((groups + 3) / 4)), dim3(256), 0, stream, p); \
         else                                                                                                          \
-            DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, 1, ASYM>), dim3((uint32_t)groups), dim3(256), 0, stream, p); \
+            DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, 1, ASYM, FORM>), dim3((uint32_t)groups), dim3(256), 0, stream, p); \
     } while (0)
     if (p.cols <= 64)
         DUQ_SHORT(4);
@@ -511,11 +531,12 @@ static int launch_short_rows(const RowParams &p, hipStream_t stream)
     return (int)hipGetLastError();
 }
 
-template <bool ASYM>
+template <bool ASYM, int FORM>
 static int launch_rows(const RowParams &p, hipStream_t stream)
 {
     if (p.rows == 0 || p.cols == 0) return 0;
-    if (p.cols <= 512 && !p.bf6) return launch_short_rows<ASYM>(p, stream);
+    if constexpr (FORM != kShadow)
+        if (p.cols <= 512) return launch_short_rows<ASYM, FORM>(p, stream);
     const uint32_t nunits = p.cols / 8;
     const dim3 grid(p.rows);
     // Wavefronts per row: enough that a lane holds at most `per_lane` units.  Four units per
@@ -530,11 +551,7 @@ static int launch_rows(const RowParams &p, hipStream_t stream)
     if ((uint64_t)p.rows * waves < 2048) waves = waves_for(2);
     if ((uint64_t)p.rows * waves < 512) waves = waves_for(1);
     const bool cached = waves * 64 * kMaxUnits >= nunits;
-#define DUQ_ROWS_LAUNCH(W, C)                                                                                \
-    if (p.bf6)                                                                                               \
-        DUQ_LAUNCH_HEAD((quantize_rows_kernel<W, ASYM, C, true>), grid, dim3(W * 64), 0, stream, p);      \
-    else                                                                                                     \
-        DUQ_LAUNCH_HEAD((quantize_rows_kernel<W, ASYM, C, false>), grid, dim3(W * 64), 0, stream, p);
+#define DUQ_ROWS_LAUNCH(W, C) DUQ_LAUNCH_HEAD((quantize_rows_kernel<W, ASYM, C, FORM>), grid, dim3(W * 64), 0, stream, p);
 #define DUQ_ROWS_CASE(W)                                                                                     \
     case W:                                                                                                  \
         if (cached) {                                                                                        \
@@ -558,14 +575,20 @@ static int launch_rows(const RowParams &p, hipStream_t stream)
 int launch_quantize_rows_sym(const uint16_t *x, uint32_t rows, uint32_t cols, float clip, int qmax, uint8_t *q,
                              uint16_t *scale, uint8_t *bf6, hipStream_t stream)
 {
-    RowParams p{x, q, scale, nullptr, bf6, rows, cols, clip, qmax, nullptr};
-    return launch_rows<false>(p, stream);
+    RowParams p{x, q, scale, nullptr, bf6, rows, cols, clip, qmax, nullptr, nullptr, 0};
+    return bf6 ? launch_rows<false, kShadow>(p, stream) : launch_rows<false, kCodes>(p, stream);
 }
 int launch_quantize_rows_asym(const uint16_t *x, uint32_t rows, uint32_t cols, uint8_t *q, uint16_t *scale,
                               uint16_t *zeros, int32_t *rowsum, uint8_t *bf6, hipStream_t stream)
 {
-    RowParams p{x, q, scale, zeros, bf6, rows, cols, 1.0f, 15, rowsum};
-    return launch_rows<true>(p, stream);
+    RowParams p{x, q, scale, zeros, bf6, rows, cols, 1.0f, 15, rowsum, nullptr, 0};
+    return bf6 ? launch_rows<true, kShadow>(p, stream) : launch_rows<true, kCodes>(p, stream);
+}
+int launch_quantize_two(const uint16_t *x, uint32_t rows, const uint16_t *x2, uint32_t rows2, uint32_t cols, bool asym, float clip,
+                        int qmax, uint8_t *q, uint16_t *scale, uint16_t *zeros, hipStream_t stream)
+{
+    RowParams p{x, q, scale, zeros, nullptr, rows + rows2, cols, clip, qmax, nullptr, x2, rows};
+    return asym ? launch_rows<true, kTwo>(p, stream) : launch_rows<false, kTwo>(p, stream);
 }
 
 }  // namespace duq

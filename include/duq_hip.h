@@ -210,6 +210,17 @@ int duq_batch_linear4bit_forward(int32_t mode, const uint8_t *xq, const duq_half
                                  uint32_t batch_count, uint32_t M, uint32_t N, uint32_t K, duq_half *y,
                                  duq_stream_t stream);
 
+/* The whole forward of AsymQuantMatMul (mode DUQ_EPI_ASYM) and SymQuantMatMul (DUQ_EPI_SYM): both operands quantized per
+ * row, in one launch unless the symmetric settings of the two differ, then duq_batch_linear4bit_forward; the same bits
+ * as those steps (qlinear4bit/nn/matmul.py:38-63, 78-84).
+ *   a [batch_count, M, K], b [batch_count, N, K] fp16, 16-byte aligned, K % 64 == 0;  y [batch_count, M, N] fp16
+ *   clip, qmax   settings of the symmetric quantizers (not read by DUQ_EPI_ASYM, qmax has to be valid)
+ *   workspace    duq_quantize_product_workspace_bytes(...) bytes, 16-byte aligned */
+uint64_t duq_quantize_product_workspace_bytes(int32_t mode, uint32_t batch_count, uint32_t M, uint32_t N, uint32_t K);
+int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uint32_t batch_count, uint32_t M, uint32_t N, uint32_t K,
+                         float clip_a, int32_t qmax_a, float clip_b, int32_t qmax_b, duq_half *y, void *workspace,
+                         uint64_t workspace_bytes, duq_stream_t stream);
+
 /* Which kernel family duq_matmul_host_4bit / duq_linear4bit_forward run for a shape (no GPU work; for tests
  * and tuning): 1 decode rows kernel (M <= 4), 2 decode MFMA kernel (M <= 16; up to 64 rows of at most 8192
  * elements, 48 of at most 12288), 3 dot kernel (M <= 4, rows longer than 16384 elements), 4 ring kernel, 5 skinny

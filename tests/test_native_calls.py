@@ -1,0 +1,85 @@
+"""The native ``__call__`` of the module classes (csrc/duq_host.cpp): same bits as torch.nn.Module.__call__ with the
+class's forward, which it leaves to torch wherever a call is more than that."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("batch,M,N,K", [((1,), 1, 1, 64), ((3,), 1, 65, 64), ((2, 3), 7, 33, 128), ((5,), 129, 64, 512),
+                                         ((2,), 31, 130, 576), ((1,), 1, 257, 4160), ((9,), 400, 300, 192), ((2,), 3, 5, 16448)],
+                         ids=str)
+def test_products_of_activations_in_one_call(dev, monkeypatch, batch, M, N, K):
+    """Both operands quantized by one launch (rows of both kinds of row kernel, in and beyond the register cache) against
+    the module's separate steps, and settings of the two quantizers that differ."""
+    from duqlinear4bitcuda_amd import _HIP as ops
+    from duqlinear4bitcuda_amd import nn as qnn
+    print("product", batch, M, N, K, flush=True)
+    g = torch.Generator(device=dev).manual_seed(N)
+    a, b = (torch.randn(*batch, r, K, generator=g, device=dev).half() for r in (M, N))
+    asym, sym, other = qnn.AsymQuantMatMul(), qnn.SymQuantMatMul(), qnn.SymQuantMatMul()
+    other.quantizer_A.input_clip_ratio, other.quantizer_B.qmax = 0.8, 7
+    calls = ((asym, a, b), (sym, a, b), (other, a, b), (sym, a, b.view(-1, K)[:N].contiguous()))
+    asym(a, b)
+    steps = []
+    real = ops._launch
+    with monkeypatch.context() as m:
+        m.setattr(ops, "_launch", lambda *x: (steps.append(x[1]), real(*x))[1])
+        got = [f(x, y) for f, x, y in calls]
+        assert len(steps) == 3 * len(calls)
+    for (f, x, y), want in zip(calls, got):
+        out = f(x, y)
+        assert out.shape == want.shape and torch.equal(out, want)
+
+
+def test_calls_that_are_more_than_the_forward(dev, monkeypatch):
+    from duqlinear4bitcuda_amd import nn as qnn
+    K, N = 256, 96
+    lin = torch.nn.Linear(K, N).half().to(dev).requires_grad_(False)
+    sw = lin.weight.abs().amax(1, keepdim=True) / 7
+    x = torch.randn(5, K, device=dev).half()
+    l8 = qnn.LinearQuant8bitASQ.from_linear(lin.float()).to(dev)
+    lin.half()
+    pairs = [(torch.nn.Sequential(qnn.SymQuantizer(), qnn.Linear4bitSQ.from_float(lin, sw).to(dev)), (x,)),
+             (qnn.Linear4bitASQ.from_linear(lin).to(dev), (x,)), (l8, (x.float(),)),
+             (qnn.SymQuantMatMul(), (x, x)), (qnn.AsymQuantMatMul(), (x[None], x[None]))]
+    for mod, args in pairs:
+        inner = list(mod) if isinstance(mod, torch.nn.Sequential) else [mod]
+        mod(*args)
+        want = mod(*args)
+        seen = []
+        for m in inner:                                      # hooks of the instance
+            handle = m.register_forward_hook(lambda *a: seen.append(a))
+            assert torch.equal(mod(*args), want) and len(seen) == 1
+            handle.remove()
+            seen.clear()
+        handle = torch.nn.modules.module.register_module_forward_pre_hook(lambda *a: seen.append(a))   # of every module
+        assert torch.equal(mod(*args), want) and len(seen) >= len(inner)
+        handle.remove()
+        seen.clear()
+        for m in inner:                                      # a replaced forward, of the class and of the instance
+            real = type(m).forward
+            with monkeypatch.context() as c:
+                c.setattr(type(m), "forward", lambda self, *a: (seen.append(1), real(self, *a))[1])
+                assert torch.equal(mod(*args), want) and seen == [1]
+            seen.clear()
+            m.forward = lambda *a, _m=m, _r=real: (seen.append(1), _r(_m, *a))[1]
+            assert torch.equal(mod(*args), want) and seen == [1]
+            del m.forward
+            seen.clear()
+        assert torch.equal(mod(*args), want) and not seen
+    # the copy of an 8-bit weight follows changes in place; a layer's prepared call follows its buffers
+    before = l8(x.float())
+    l8.weight.add_(1)
+    assert not torch.equal(l8(x.float()), before)
+    l8.weight.sub_(1)
+    assert torch.equal(l8(x.float()), before)
+    sq = pairs[0][0]
+    before = sq(x)
+    sq[1].weight_scales = sq[1].weight_scales * 2
+    assert not torch.equal(sq(x), before)
+    # operands that do not fit raise what the steps raise
+    with pytest.raises(RuntimeError, match="same leading dimensions"):
+        qnn.SymQuantMatMul()(torch.zeros(2, 4, K, device=dev).half(), torch.zeros(3, 4, K, device=dev).half())
+    with pytest.raises(AssertionError, match="Batch dimensions"):
+        qnn.AsymQuantMatMul()(torch.zeros(2, 4, K, device=dev).half(), torch.zeros(3, 4, K, device=dev).half())
