@@ -12,11 +12,12 @@
 //
 // Five kernels here, and the prefill kernel in duq_prefill.hip, picked by shape in select_gemm_kernel() (up to 64 rows
 // run the two kernels of duq_decode.hip as far as they reach):
-//  * prefill kernel (duq_prefill.hip): more than 64 rows, long rows, tensors of 4 GiB or more, what is left;
+//  * prefill kernel (duq_prefill.hip): more than 64 rows, long rows, fewer rows on wide layers, tensors of 4 GiB or more,
+//    what is left;
 //  * stream kernel (the same shapes where rows are short): 64 x 128 tiles, weights from global memory straight to
 //    registers, activations expanded once into LDS, v_mfma_i32_32x32x32_i8 with a hand-ordered schedule;
 //  * short-row kernel (rows of at most 256 elements): the stream kernel's operand paths without its K pipeline;
-//  * ring kernel (17 <= M <= 256 on narrow problems or long rows, and 5..16 rows of 12289..16384 elements):
+//  * ring kernel (17 <= M <= 256 on problems of at most one round of its workgroups, and 5..16 rows of 12289..16384 elements):
 //    packed activations of all rows in LDS, every wavefront streams whole weight rows through a ring of loads;
 //  * skinny kernel (9 <= M <= 16 with 1536 or more column tiles): one workgroup owns 16 output columns, its
 //    wavefronts split K, whole-line weight loads turned into fragments through LDS;
@@ -784,44 +785,37 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
         if (K <= 12288) return kKernelDecodeMfma;
     }
     if (M <= 64 && small_offsets) {
+        // one round of 64 x 64 tiles of the prefill kernel, whose time hardly depends on rows and columns, is ahead of the
+        // decode kernel where that has many row tiles or several column tiles per workgroup.  More than 48 rows: 64 x
+        // 11008 x 4096 9.8 against 10.65 us, 64 x 13824 x 1024 6.6 / 8.2 (but N = 8192 8.6 either way), 64 x 4096 x 8192
+        // 11.5 / 13.5, 56 x 3072 x 5120 9.3 / 10.1; 40 x 5120 x 5120 9.3 / 11.2, 40 x 11008 x 8192 14.8 / 18.6 (but 48 x 4096
+        // x 8192 11.5 / 11.3); 32 x 13824 x 5120 11.8 / 13.6, 32 x 16384 x 8192 18.3 / 20.0 (but 17 x 16384 x 8192 19.3 /
+        // 18.4, 32 x 8192 x 5120 9.3 / 8.65).
+        const bool tiles = K <= 4096 ? M > 48 && N > 8192 && K >= 1024
+                         : K <= 8192 && (M > 48 ? N >= 3072 : M > 32 ? N >= 5120 : M > 24 && N > 10240);
+        if (tiles && N <= 16384) return kKernelStream;
         if (K <= 4096 || (K <= 8192 && M <= 32)) return kKernelDecodeMfma;
-        // (wide layers of more than 32 long rows: one round of 64 x 128 tiles of the prefill kernel, 64 x 11008 x 8192
-        // 16.3 against 21.1 us, 48 x 11008 x 11008 20.3 / 24.0, 33 x 11008 x 8192 15.9 / 16.8; at N = 4096 the decode
-        // kernel is ahead)
+        // (wide layers of more than 32 long rows: one round of tiles of the prefill kernel, 48 x 11008 x 11008 20.3 us
+        // against 24.0 with 64 x 128 tiles; at N = 4096 the decode kernel is ahead)
         const bool wide = M > 32 && N >= 8192;
         if ((N + 15) / 16 >= 192 && !wide && (K <= 8192 || (K <= 12288 && M <= 48))) return kKernelDecodeMfma;
     }
     const uint32_t xstride = ((K / 2 + 127) / 128) * 128;
     // dot kernel: up to four rows too long for the decode kernels
     if (M <= 4 && small_offsets && 4 * xstride <= 60 * 1024) return kKernelDot;
-    // more than 64 rows whose 64 x 128 tiles make one round of 64..256 workgroups: the stream kernel on those tiles
-    // (measured against the ring kernel, N = 4096: 128 x 4096 11.9 against 14.6 us, 192 x 4096 12.1 against 18.3,
-    // 128 x 11008 (K) 25.1 against 42.2; with fewer tiles the ring kernel, which splits K over workgroups, is far
-    // ahead: 200 x 520 x 8192 8.2 against 28.8 us)
+    // ring kernel: 17..256 rows in groups whose packed activations fit in LDS, while one column tile per CU and row group
+    // is one round of workgroups; every further round streams the weights again, and the prefill kernel's 64 x 64 tiles
+    // are ahead or equal (128 x 1024 x 8192, 256 workgroups: 8.2 against 11.4 us, 192 rows 14.5 / 11.5; 64 x 2048 x 8192
+    // 8.2 / 11.4, 100 rows 14.6 / 11.5; 72 x 1536 x 8192 13.4 / 11.3; 64 x 1024 x 16384 10.0 / 17.1, 100 rows 17.4 / 17.3, 192
+    // rows 26.1 / 17.4; 144 x 1536 x 4096 12.75 / 8.5).  More than 64 rows of at most 2048 elements: the tiles are ahead
+    // in any case (72 x 512 x 2048 7.2 / 6.4).  And 5..16 rows of 12289..16384 elements.
+    const uint32_t rb_max = K <= 4096 ? 4 : (K <= 8192 ? 2 : 1);  // 16-row blocks whose activations fit in LDS
+    const uint32_t row_groups = ((M + 15) / 16 + rb_max - 1) / rb_max;
+    const bool one_round = M > 16 && M <= 256 && (uint64_t)((N + 15) / 16) * row_groups <= 256 && (K > 2048 || M <= 64);
+    const bool long_rows = M <= 16 && K > 8192;
+    if ((long_rows || one_round) && K <= 16384 && small_offsets) return kKernelRing;
     const uint32_t narrow_tiles = ((M + 63) / 64) * ((N + 127) / 128);
     const bool narrow_round = M > 64 && narrow_tiles >= 64 && narrow_tiles <= 256;
-    {
-        // ring kernel: 17..256 rows in groups whose packed activations fit in LDS (a few groups only, or a
-        // problem too narrow to fill the chip with stream-kernel tiles)
-        const uint32_t rb_all = (M + 15) / 16;
-        const uint32_t rb_max = K <= 4096 ? 4 : (K <= 8192 ? 2 : 1);  // 16-row blocks whose activations fit in LDS
-        const uint32_t rb = std::min(rb_all, rb_max);
-        const uint32_t row_groups = (rb_all + rb - 1) / rb;
-        // (several row groups re-stream the weights: with enough column tiles to fill the chip the stream
-        // kernel's 32-row tiles are cheaper then)
-        const uint32_t tiles32 = ((M + 31) / 32) * ((N + 255) / 256);
-        const bool few_groups = row_groups <= 2 || (row_groups <= 6 && tiles32 < 64) || tiles32 < 48;
-        const bool mid_rows = M > 16 && M <= 256 && few_groups && !(row_groups > 1 && tiles32 >= 128);
-        const bool long_rows = M <= 16 && K > 8192;  // 5..16 rows of 12289..16384 elements
-        // (16 x 16 tiles of the output from which the prefill kernel's 64 x 128 tiles are ahead although they leave CUs
-        // idle: a ring group re-streams the weights per 64, 32 or, for rows longer than 8192 elements, 16 rows.  64 x
-        // 4096 x 11008 18.9 against 26.3 us, 33 x 4096 x 14336 22.7 / 24.4, 17 x 11008 x 14336 23.2 / 38.6, 160 x 2048 x
-        // 4096 9.8 / 13.2, 200 x 1024 x 11008 18.9 / 24.8; but 17 x 4096 x 14336, 100 x 1000 x 4096, 100 x 2048 x 8192 and
-        // 200 x 520 x 8192 are the ring kernel's)
-        const bool many_tiles = (uint64_t)rb_all * ((N + 15) / 16) >= (K > 8192 ? 768u : 1280u);
-        if ((long_rows || (mid_rows && !many_tiles)) && K <= 16384 && small_offsets && !narrow_round) return kKernelRing;
-        if (mid_rows && many_tiles && K <= 16384) return kKernelStream;
-    }
     auto tiles = [&](uint32_t bm, uint32_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     if (narrow_round || (M > 32 && tiles(32, 256) >= 32)) return kKernelStream;
     return kKernelTile;

@@ -96,10 +96,12 @@ inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 // Tile for a problem select_gemm_kernel gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
 // 64 x 128 tiles (duq_gemm.hip).  Whole rounds of 256 workgroups (one per CU) cost about f + c * (K / 256) microseconds
 // each, measured per tile shape (N = 4096, one round, K = 1024 / 4096 / 16384): 64 x 128 6.6 / 11.9 / 33, 128 x 128 8.9 /
-// 17.5 / 55, 128 x 256 12.5 / 30 / 100, 256 x 256 21 / 52.7 / 178 (1.3 of it once per launch); the cheapest wins.  The
+// 17.5 / 55, 128 x 256 12.5 / 30 / 100, 256 x 256 21 / 52.7 / 178 (1.3 of it once per launch); the cheapest wins.  64 x 64 and
+// 96 x 64 tiles (128 rows; 65 rows) 5.9 / 8.7 / 22 and - / 10 / 22.6: in one round only, where they halve the walk over K;
+// two rounds of them are behind (512 x 4096 x 4096 17 against 12.4, 96 x 28672 x 8192 38 against 34.7).  The
 // stream kernel has the longer loop but starts and ends faster (512 x 4096 x 512 4.8 against 5.9 us, x 1024 5.8 / 6.6, x
-// 2048 8.1 / 8.3, x 4096 13.3 / 11.9), and two or three of its workgroups share a CU, so its rounds need not be whole (32
-// products of 1216 x 64 x 1216, 608 tiles: 12.8 us).  The dual-uniform row-sum epilogue (`mode5`) has no 256 x 256 tile
+// 2048 8.1 / 8.3, x 4096 13.3 / 11.9; 32 products of 1216 x 64 x 1216, 608 tiles: 12.8 us; 250 x 11008 x 4096, 344 tiles:
+// 24.8 against 17.7 on 128 x 128: two or three of its workgroups share a CU, but a round begun takes a round's time).  The dual-uniform row-sum epilogue (`mode5`) has no 256 x 256 tile
 // (its staged parameters do not fit in LDS beside the operands).
 struct StreamTile {
     uint32_t rows, cols;
@@ -108,12 +110,13 @@ struct StreamTile {
 inline StreamTile select_stream_tile(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, bool mode5)
 {
     const float nch = (float)((K + 255) / 256);
-    const uint32_t bm[4] = {64, 128, 128, 256}, bn[4] = {128, 128, 256, 256};
-    const float c_us[4] = {0.44f, 0.76f, 1.47f, 2.62f}, f_us[4] = {3.6f, 4.3f, 5.5f, 9.5f};
+    const uint32_t bm[6] = {64, 64, 96, 128, 128, 256}, bn[6] = {128, 64, 64, 128, 256, 256};
+    const float c_us[6] = {0.44f, 0.2f, 0.258f, 0.76f, 1.47f, 2.62f}, f_us[6] = {3.6f, 5.5f, 6.1f, 4.3f, 5.5f, 9.5f};
     auto tiles = [&](int k) { return (uint64_t)((M + bm[k] - 1) / bm[k]) * ((N + bn[k] - 1) / bn[k]) * batch; };
     StreamTile best{64, 128, true};
-    float best_cost = std::max(1.f, (float)tiles(0) / 256.f) * (nch * 0.62f + 0.9f) + 1.3f;
-    for (int k = 0; k < (mode5 ? 3 : 4); ++k) {
+    float best_cost = (float)((tiles(0) + 255) / 256) * (nch * 0.62f + 0.9f) + 1.3f;
+    for (int k = 0; k < (mode5 ? 5 : 6); ++k) {
+        if (bn[k] == 64 && tiles(k) > 256) continue;
         const float cost = (float)((tiles(k) + 255) / 256) * (nch * c_us[k] + f_us[k]);
         if (cost < best_cost) {
             best_cost = cost;

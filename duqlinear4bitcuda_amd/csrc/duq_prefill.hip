@@ -16,6 +16,14 @@
 // them was 1100 of the 1700 cycles of a 256-k chunk): 512 x 4096 x 11008 (K) 34.7 -> 26.6 us, 77 x 13824 x 5120 19.0 ->
 // 14.3, 128 x 4096 x 11008 25.1 -> 19.9, 1024 x 11008 x 4096 55.5 -> 45, 4096 x 4096 x 4096 58 -> 53.5; rows of more than
 // 16384 elements, formerly on a kernel of 64 x 64 tiles, 9 x 11008 x 20480 79 -> 31 us, 2048 x 512 x 28672 81 -> 44.6.
+//
+// Few rows (65..256 on a few thousand columns, 17..64 long ones) leave most CUs without a 64 x 128 tile, and there a
+// launch lasts as long as one workgroup's walk over K.  64 x 64 tiles (96 x 64 for 65..96 rows on wide layers) whose eight
+// wavefronts each take an eighth of every stage: twice the workgroups, half the walk (0.2 us per 256 k against 0.44),
+// for a longer end, since eight partial tiles have to meet (5.5 us with the start against 3.6).  128 x 4096 x 4096 10.5 ->
+// 8.7 us, 128 x 4096 x 11008 22.5 -> 16.9, 64 x 4096 x 16384 30.6 -> 22.7, 77 x 4096 x 28672 43.4 -> 32.5; 72 x 3072 x 4096,
+// on the ring kernel before, 13.8 -> 8.5; 96 x 64: 77 x 13824 x 5120 15.1 -> 14.4 (3.9 TB/s of weights).  A 128 x 64 tile
+// measured behind 64 x 128 (512 x 4096 x 4096 13.4 against 12.4).
 #include "duq_gemm_common.h"
 #include <type_traits>
 
@@ -46,9 +54,10 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
     constexpr int H = WTM * WTN;              // MFMAs per nibble parity of a step
     constexpr int P = WTM + WTN;              // fragments per step
     constexpr int W = 4 * P;                  // words a lane expands per step and parity
-    constexpr int TM = KS == 4 ? WTM / 2 : WTM, TN = KS == 1 ? WTN : WTN / 2;    // what a wavefront finishes after the loop
+    constexpr int T = WTM * WTN;
+    constexpr int TM = KS == 8 ? 1 : KS == 4 ? WTM / 2 : WTM, TN = KS == 1 ? WTN : WTN / 2;  // what a wavefront finishes after the loop
     constexpr bool LATE = WTM * WTN == 8;     // no registers to spare in the loop: parameters after it
-    constexpr uint32_t kEpiLds = 8 * (32 * TM) * (64 * TN + 16), kXchg = KS == 1 ? 0 : 8 * KS * TM * TN * 4096;
+    constexpr uint32_t kEpiLds = 8 * (32 * TM) * (64 * TN + 16), kXchg = KS == 1 ? 0 : KS == 8 ? T * 4096 : 8 * KS * TM * TN * 4096;
     constexpr uint32_t kLds = NST * kStage > kEpiLds ? (NST * kStage > kXchg ? NST * kStage : kXchg) : (kEpiLds > kXchg ? kEpiLds : kXchg);
     __shared__ __attribute__((aligned(256))) uint8_t lds[kLds];
     __shared__ __attribute__((aligned(16))) uint32_t dpar[EPI == 5 ? (BN + BM) * 8 : 4];
@@ -165,15 +174,30 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
     };
     // the part of the tile that this wavefront finishes
-    const uint32_t wm0 = m0 + wm * (32 * WTM) + (ks >> 1) * (32 * TM), wn0 = n0 + wn * (32 * WTN) + (ks & 1u) * (32 * TN);
+    // (KS = 8: wavefronts T and up finish nothing, and fetch parameters of the last tile)
+    const uint32_t mine = KS == 8 ? min(ks, (uint32_t)T - 1) : ks;
+    const uint32_t wm0 = m0 + wm * (32 * WTM) + (mine >> 1) * (32 * TM), wn0 = n0 + wn * (32 * WTN) + (mine & 1u) * (32 * TN);
     constexpr bool kLdsParams = false;
 #include "duq_stream_epilogue_fetch.inc"
     if (!LATE) fetch_params();
-    wait_stages(std::integral_constant<int, NST - 1>{});
+    if constexpr (STEPS == 1) {
+        // a wavefront has one step of every stage, and reads two stages ahead into its registers: the stages of this chunk
+        // and the next are free to be loaded once every wavefront has read them
+        wait_stages(std::integral_constant<int, NST - 2>{});
 #pragma unroll
-    for (int f = 0; f < P; ++f) read(0, f, 0, 0);
+        for (int f = 0; f < P; ++f) read(0, f, 0, 0);
 #pragma unroll
-    for (int f = 0; f < P; ++f) read(1, f, 1, 0);
+        for (int f = 0; f < P; ++f) read(1, f, 0, kStage);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < L; ++j) load(j, NST, 0);
+    } else {
+        wait_stages(std::integral_constant<int, NST - 1>{});
+#pragma unroll
+        for (int f = 0; f < P; ++f) read(0, f, 0, 0);
+#pragma unroll
+        for (int f = 0; f < P; ++f) read(1, f, 1, 0);
+    }
 #pragma unroll
     for (int f = 0; f < P; ++f)
 #pragma unroll
@@ -183,40 +207,74 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
     // ones, in whose shadow the next step's even ones are expanded and the registers that leaves are read for the step
     // after it.  The first read of the next chunk is in step STEPS - 2: that is where the wavefronts wait for it.  All
     // reads of this chunk are done then (every wavefront waited for its own), and its stage takes the chunk NST further on.
-    uint32_t stage = 0;
+    if constexpr (STEPS == 1) {
+        // two chunks per turn for the two register sets; a chunk past the end is zeros
+        uint32_t st1 = kStage, st2 = 2 % NST * kStage;  // stages of the next chunk and the one after it
 #pragma unroll 1
-    for (uint32_t c = 0; c < nchunks; ++c) {
-        const uint32_t next = stage + kStage == NST * kStage ? 0 : stage + kStage;
+        for (uint32_t c = 0; c < nchunks; c += 2) {
 #pragma unroll
-        for (int i = 0; i < STEPS; ++i) {
-            const int set = i & 1;
+            for (int set = 0; set < 2; ++set) {
 #pragma unroll
-            for (int slot = 0; slot < 2 * H; ++slot) {
-                const int par = slot / H, q = slot % H, b = q / WTN, t = q % WTN;
-                if (i == STEPS - 2 && slot == H) {
-                    wait_stages(std::integral_constant<int, NST - 2>{});
+                for (int slot = 0; slot < 2 * H; ++slot) {
+                    const int par = slot / H, q = slot % H, b = q / WTN, t = q % WTN;
+                    if (slot == H) {
+                        wait_stages(std::integral_constant<int, NST - 2>{});
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, %0"
+                                 : "+a"(accw[t][b])
+                                 : "v"(ex[par][WTM + t]), "v"(ex[par][b]));
                     __builtin_amdgcn_sched_barrier(0);
-                }
-                asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, %0"
-                             : "+a"(accw[t][b])
-                             : "v"(ex[par][WTM + t]), "v"(ex[par][b]));
-                __builtin_amdgcn_sched_barrier(0);
-                // ---- side work in the shadow of this MFMA.  (The words expanded last belong to the last weight tile,
-                // which the MFMA behind them does not read: one that did would need two wait states first.)
 #pragma unroll
-                for (int w = q * W / H; w < (q + 1) * W / H; ++w) expand_word(par ^ 1, par ? set ^ 1 : set, w / 4, w % 4);
+                    for (int w = q * W / H; w < (q + 1) * W / H; ++w) expand_word(par ^ 1, par ? set ^ 1 : set, w / 4, w % 4);
 #pragma unroll
-                for (int f = 0; f < P; ++f)
-                    if (par && q == f * H / P) read(set, f, (i + 2) % STEPS, i < STEPS - 2 ? stage : next);
-                if (i >= STEPS - 2) {
+                    for (int f = 0; f < P; ++f)
+                        if (par && q == f * H / P) read(set, f, 0, st2);
 #pragma unroll
                     for (int j = 0; j < L; ++j)
-                        if ((i - STEPS + 2) * 2 * H + slot == H + j * 3 * H / L) load(j, c + NST, stage);
+                        if (par && q == j * H / L) load(j, c + set + 1 + NST, st1);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                __builtin_amdgcn_sched_barrier(0);
+                st1 = st2;
+                st2 = st2 + kStage == NST * kStage ? 0 : st2 + kStage;
             }
         }
-        stage = next;
+    } else {
+        uint32_t stage = 0;
+#pragma unroll 1
+        for (uint32_t c = 0; c < nchunks; ++c) {
+            const uint32_t next = stage + kStage == NST * kStage ? 0 : stage + kStage;
+#pragma unroll
+            for (int i = 0; i < STEPS; ++i) {
+                const int set = i & 1;
+#pragma unroll
+                for (int slot = 0; slot < 2 * H; ++slot) {
+                    const int par = slot / H, q = slot % H, b = q / WTN, t = q % WTN;
+                    if (i == STEPS - 2 && slot == H) {
+                        wait_stages(std::integral_constant<int, NST - 2>{});
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, %0"
+                                 : "+a"(accw[t][b])
+                                 : "v"(ex[par][WTM + t]), "v"(ex[par][b]));
+                    __builtin_amdgcn_sched_barrier(0);
+                    // ---- side work in the shadow of this MFMA.  (The words expanded last belong to the last weight tile,
+                    // which the MFMA behind them does not read: one that did would need two wait states first.)
+#pragma unroll
+                    for (int w = q * W / H; w < (q + 1) * W / H; ++w) expand_word(par ^ 1, par ? set ^ 1 : set, w / 4, w % 4);
+#pragma unroll
+                    for (int f = 0; f < P; ++f)
+                        if (par && q == f * H / P) read(set, f, (i + 2) % STEPS, i < STEPS - 2 ? stage : next);
+                    if (i >= STEPS - 2) {
+#pragma unroll
+                        for (int j = 0; j < L; ++j)
+                            if ((i - STEPS + 2) * 2 * H + slot == H + j * 3 * H / L) load(j, c + NST, stage);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            stage = next;
+        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
@@ -227,6 +285,27 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
         for (int t = 0; t < TN; ++t)
 #pragma unroll
             for (int b = 0; b < TM; ++b) acc[t][b] = accw[t][b];
+    } else if constexpr (KS == 8) {
+        // tile 2 * b + t is finished by the wavefront of that number: the others add to its sums in LDS (integers, in any
+        // order)
+        static_assert(WTN == 2 && T <= 8, "a tile per wavefront");
+        int32_t *const red = reinterpret_cast<int32_t *>(lds) + lane;
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < T; ++g)
+            if ((uint32_t)g == ks)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) red[(g * 16 + r) * 64] = accw[g & 1][g >> 1][r];
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < T; ++g)
+            if ((uint32_t)g != ks)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    __hip_atomic_fetch_add(red + (g * 16 + r) * 64, accw[g & 1][g >> 1][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][0][r] = red[(mine * 16 + r) * 64];
     } else {
         // the KS wavefronts of a tile share its outputs out: each hands the sums it does not finish to those that do
         auto at = [&](int dst, uint32_t src, int t, int b) {
@@ -269,6 +348,7 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
                     }
     }
     if (LATE) fetch_params();
+    if (KS == 8 && ks >= (uint32_t)T) p.M = 0;  // no rows of its own: stores nothing
     uint8_t *const wstage = lds + wave * (32 * TM) * (64 * TN + 16);
     constexpr bool kWideStore = false;
 #include "duq_stream_epilogue_store.inc"
@@ -281,7 +361,11 @@ static int launch_prefill_epi(GemmParams &p, StreamTile tile, hipStream_t stream
     p.tiles_m = (p.M + bm - 1) / bm;
     p.tiles_n = (p.N + bn - 1) / bn;
     const dim3 grid(p.tiles_m * p.tiles_n, 1, batch);
-    if (bm == 64 && bn == 128)
+    if (bm == 64 && bn == 64)
+        DUQ_LAUNCH_HEAD((gemm_s4_prefill_kernel<2, 2, 1, 1, 8, 256, EPI, BIAS>), grid, dim3(512), 0, stream, p);
+    else if (bm == 96 && bn == 64)
+        DUQ_LAUNCH_HEAD((gemm_s4_prefill_kernel<3, 2, 1, 1, 8, 256, EPI, BIAS>), grid, dim3(512), 0, stream, p);
+    else if (bm == 64 && bn == 128)
         DUQ_LAUNCH_HEAD((gemm_s4_prefill_kernel<2, 2, 1, 2, 4, 256, EPI, BIAS>), grid, dim3(512), 0, stream, p);
     else if (bm == 128 && bn == 128)
         DUQ_LAUNCH_HEAD((gemm_s4_prefill_kernel<2, 2, 2, 2, 2, 256, EPI, BIAS>), grid, dim3(512), 0, stream, p);

@@ -49,3 +49,21 @@ def test_prefill_tiles(dev, M, N, K, n):
         got = hip.linear4bit_forward_dual_rowsum(a[0], sr[0], zr[0], rr[0], b[0], s1[0], z1[0], s2[0], z1[0], r1[0], r1[0], bias[0])
         want = hip.asym_dual_rowsum_dequant(acc[0], a[0], sr[0], zr[0], rr[0], b[0], s1[0], z1[0], s2[0], z1[0], r1[0], r1[0], bias[0])
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# tiles whose eight wavefronts split every stage: odd and even numbers of stages, a k that ends inside a piece, few rows and
+# columns (tile 0: a shape the query names no tile for)
+SPLIT = [(65, 4100, 2112, 64064), (200, 1101, 4160, 64064), (17, 8201, 16448, 0), (6, 66, 20032, 0), (64, 11008, 4096, 64064),
+         (256, 4096, 4096, 64064), (96, 8193, 4160, 96064), (77, 13824, 5120, 96064), (65, 12001, 16448, 96064)]
+
+
+@pytest.mark.parametrize("M,N,K,tile", SPLIT)
+def test_tiles_split_over_k(dev, M, N, K, tile):
+    from duqlinear4bitcuda_amd import _HIP as hip
+    assert hip.gemm_stream_tile_for(M, N, K) == tile
+    test_prefill_tiles(dev, M, N, K, 1)
+
+
+@pytest.mark.parametrize("M,N,K,n", [(1, 130, 4160, 5), (63, 64, 2112, 7)])
+def test_tiles_split_over_k_batched(dev, M, N, K, n):
+    test_prefill_tiles(dev, M, N, K, n)
