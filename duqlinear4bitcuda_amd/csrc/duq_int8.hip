@@ -496,6 +496,172 @@ __global__ __launch_bounds__(256) void gemm_s8_kernel(DUQ_HEAD_DECL, Gemm8Params
 }
 
 // ---------------------------------------------------------------------------------
+// split kernel (17 to some hundred rows, one round of its tiles): a 64 x 64 tile per workgroup
+// ---------------------------------------------------------------------------------
+// Such launches have fewer 64 x 128 tiles than CUs and last as long as one workgroup's walk over K.  Here eight
+// wavefronts each take one of the eight 32-k steps of every 256-k chunk for the whole tile (2 x 2 MFMA tiles), which is
+// twice the workgroups and an eighth of the walk.  Both operands go to LDS without registers, four chunks in flight; a
+// row's sixteen 16-byte pieces lie at piece ^ (row % 16) (the load instruction puts lane l's bytes 16 * l behind its base,
+// so the lane's source swizzles), tiled weights in their own fragment order.  The sums meet in LDS with integer adds, laid
+// out so that neither the adds nor the reads that turn them to rows share a bank.
+template <bool FUSED, bool BIAS, bool TILED>
+__global__ __launch_bounds__(512) void gemm_s8_split_kernel(DUQ_HEAD_DECL, Gemm8Params tail)
+{
+    Gemm8Params p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.A);
+    to_global(p.B);
+    to_global(p.C);
+    to_global(p.y);
+    constexpr uint32_t kStage = 32768, kW = 16384;  // bytes of a chunk; offset of its weights
+    constexpr int NST = 4;
+    __shared__ __attribute__((aligned(256))) uint8_t lds[NST * kStage];
+    uint32_t tile_m, tile_n;
+    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    const uint32_t m0 = tile_m * 64, n0 = tile_n * 64;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t l32 = lane & 31u, h = lane >> 5;
+    const uint32_t nchunks = (p.K + 255) / 256;
+
+    // ---- global -> LDS: two instructions per operand, wavefront and chunk.  Row-major: rows 4 * (8 * j + wave) .. + 3 of
+    // the tile; tiled: this wavefront's own fragments, step `wave` of both 32-row tiles.  K % 32 == 0: a piece is all
+    // inside its row or past it, and then reads as zero (as do rows past the descriptor and chunks past the end).
+    auto desc = [](const void *base, uint32_t bytes) {
+        const uint64_t a = reinterpret_cast<uint64_t>(base);
+        return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
+                   (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+    };
+    const uint32_t wrows = TILED ? min((p.N + 31u) / 32u * 32u - n0, 64u) : min(p.N - n0, 64u);
+    const v4u dX = desc(p.A + (uint64_t)m0 * p.K, min(p.M - m0, 64u) * p.K);
+    const v4u dW = desc(p.B + (uint64_t)n0 * p.K, wrows * p.K);
+    const uint32_t lr = wave * 4 + (lane >> 4), piece = (lane & 15u) ^ (lr & 15u);  // (32 * j rows further on: the same)
+    const uint32_t row0 = lr * p.K + piece * 16;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    auto to_lds = [&](const v4u d, uint32_t dst, uint32_t off) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(off), "s"(d) : "memory", "m0");
+    };
+    auto load = [&](uint32_t c, uint32_t stage) {
+        const uint32_t k = c * 256;
+        [[maybe_unused]] const bool in_row = k + piece * 16 < p.K, in_step = k + wave * 32 < p.K;
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j) to_lds(dX, lds0 + stage + (j * 8 + wave) * 1024, in_row ? row0 + j * 32 * p.K + k : kOobOffset);
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j)
+            if (TILED)
+                to_lds(dW, lds0 + stage + kW + (j * 8 + wave) * 1024, in_step ? j * 32 * p.K + k * 32 + wave * 1024 + lane * 16 : kOobOffset);
+            else
+                to_lds(dW, lds0 + stage + kW + (j * 8 + wave) * 1024, in_row ? row0 + j * 32 * p.K + k : kOobOffset);
+    };
+    // ---- LDS -> registers: this wavefront's step of the chunk
+    const uint32_t pos = ((2 * wave + h) ^ (l32 & 15u)) * 16;
+    auto frag = [&](uint32_t base, uint32_t j) { return *reinterpret_cast<const v4i *>(lds + base + (j * 32 + l32) * 256 + pos); };
+    v4i fx[2][2], fw[2][2];
+    auto read = [&](int set, uint32_t stage) {
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j) {
+            fx[set][j] = frag(stage, j);
+            fw[set][j] = TILED ? *reinterpret_cast<const v4i *>(lds + stage + kW + (j * 8 + wave) * 1024 + lane * 16) : frag(stage + kW, j);
+        }
+    };
+    v16i32 acc[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[t][b][r] = 0;
+
+    static_assert(NST == 4, "the waits below: two later chunks (eight loads) may be in flight");
+#pragma unroll
+    for (uint32_t c = 0; c < NST; ++c) load(c, c * kStage);
+    // parameters of the outputs this thread stores: four columns, rows tid / 16 and 32 further on
+    const uint32_t cg = tid & 15u, n = n0 + cg * 4;
+    float sc[4], zc[4], bs[4], sr[2], zr[2];
+    if (FUSED) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t nn = min(n + r, p.N - 1);
+            sc[r] = p.epi.s_col[nn];
+            zc[r] = p.epi.z_col[nn];
+            bs[r] = BIAS ? p.epi.bias[nn] : 0.f;
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const uint32_t m = min(m0 + b * 32 + (tid >> 4), p.M - 1);
+            sr[b] = p.epi.s_row[m];
+            zr[b] = p.epi.z_row[m];
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");  // chunk 0 is here
+    read(0, 0);
+    uint32_t cur = 0;
+    for (uint32_t c = 0; c < nchunks; c += 2) {  // two chunks per turn for the two register sets; one past the end is zeros
+#pragma unroll
+        for (int set = 0; set < 2; ++set) {
+            // the next chunk is here, and every wavefront has read this one: its place takes the chunk NST further on
+            asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            const uint32_t nxt = cur + kStage == NST * kStage ? 0 : cur + kStage;
+            read(set ^ 1, nxt);
+            load(c + set + NST, cur);
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) acc[t][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[set][t], fx[set][b], acc[t][b], 0, 0, 0);
+            cur = nxt;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+    // ---- the eight partial tiles meet: register r of tile (t, b) of all lanes at 64 consecutive integers, lane l at
+    // l ^ (4 * (q + 4 * t)) (r = 4 * q + ..), so that the sixteen threads of an output row read sixteen banks apart
+    int32_t *const red = reinterpret_cast<int32_t *>(lds);
+    auto at = [&](uint32_t t, uint32_t b, uint32_t q, uint32_t r, uint32_t l) { return red + ((b * 2 + t) * 16 + q * 4 + r) * 64 + (l ^ ((q + 4 * t) * 4)); };
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            if (((uint32_t)g == wave) == (pass == 0))
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    int32_t *const d = at(g & 1, g >> 1, r >> 2, r & 3, lane);
+                    if (pass == 0)
+                        *d = acc[g & 1][g >> 1][r];
+                    else
+                        __hip_atomic_fetch_add(d, acc[g & 1][g >> 1][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+        __syncthreads();
+    }
+    const void *outp = FUSED ? (const void *)p.y : (const void *)p.C;
+    const bool vec_ok = p.N % 4 == 0 && reinterpret_cast<uintptr_t>(outp) % 16 == 0;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        const uint32_t m = m0 + b * 32 + (tid >> 4);
+        if (m >= p.M || n >= p.N) continue;
+        v4i a;
+        v4f32 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            a[r] = *at(cg >> 3, b, (cg >> 1) & 3u, r, (cg & 1u) * 32 + (tid >> 4));
+            if (FUSED) {
+                v[r] = dequant_hprec_one(a[r], sr[b], zr[b], sc[r], zc[r]);
+                if (BIAS) v[r] = v[r] + bs[r];
+            }
+        }
+        if (vec_ok) {  // (n is a multiple of four: the four columns end inside the row)
+            if (FUSED) __builtin_nontemporal_store(v, reinterpret_cast<v4f32 *>(p.y + (uint64_t)m * p.N + n));
+            else __builtin_nontemporal_store(a, reinterpret_cast<v4i *>(p.C + (uint64_t)m * p.N + n));
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (n + r < p.N) {
+                    if (FUSED) p.y[(uint64_t)m * p.N + n + r] = v[r];
+                    else p.C[(uint64_t)m * p.N + n + r] = a[r];
+                }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------
 // skinny kernel (M <= 32): bound by reading the weight once from HBM
 // ---------------------------------------------------------------------------------
 // A workgroup owns 16 weight rows; its four wavefronts split K in contiguous quarters and meet in LDS at the end, so
@@ -900,6 +1066,19 @@ static void launch_rows8(const Gemm8Params &p, hipStream_t stream)
 // shapes the rows kernel takes: row-major weight, up to four rows of at most 4096 elements (two rows: 8192), the
 // weight tensor within 32-bit offsets per descriptor (a descriptor covers one wavefront's rows)
 inline bool rows8_takes(uint32_t M, uint32_t K) { return M <= 4 && K <= (M <= 2 ? 8192u : 4096u); }
+// split kernel: problems of one round of its 64 x 64 tiles, from 33 rows on where the decode kernel does not reach (tiled
+// weights, against the 64 x 128, 64 x 256 and 32 x 256 tiles that ran them: 65 x 4096 x 4096 10.7 against 14.75 us, 128 x 4096
+// x 11008 29 / 55, 256 x 2048 x 8192 15.8 / 25.3, 256 x 4096 x 4096 11.3 / 12.4, 40 rows of 8192 on N = 8192 22 / 42), rows
+// of at least 1536 elements (x 1024: 6.4 - 7.3 us either way).  Of the decode kernel's shapes those of four row tiles on a
+// narrow layer (64 x 4096 x 4096 10.4 / 11.85, 64 x 1024 x 4096 10.3 / 11.1, but 64 x 8192 x 4096 15.0 / 13.9, 48 x 4096 x 4096
+// 10.1 / 9.3); of the skinny kernel's 17 rows and more on a wide layer (20 x 11008 x 8192 21.5 / 29.2, but 20 x 8192 x 8192
+// 22.5 / 21.75).
+inline bool split8_takes(uint32_t M, uint32_t N, uint32_t K)
+{
+    if (M <= 16 || (uint64_t)((M + 63) / 64) * ((N + 63) / 64) > 256) return false;
+    if (decode8_takes(M, N, K)) return M > 48 && K > 2048 && N <= 4096;
+    return M <= 32 ? N > 8192 : K >= 1536;
+}
 
 // a round of 256 x 256 tiles in rounds of 128 x 256 ones (measured 1.86 - 1.97: 4096 x 4096 x 4096 73.4 against
 // 74.4 us, 4096 x 11008 x 4096 188 against 202, 4096 x 8192 x 8192 240 against 251)
@@ -913,6 +1092,12 @@ static void launch_gemm8_variant(Gemm8Params &p, hipStream_t stream)
         if (p.M == 1) launch_rows8<1, FUSED, BIAS>(p, stream);
         else if (p.M == 2) launch_rows8<2, FUSED, BIAS>(p, stream);
         else launch_rows8<4, FUSED, BIAS>(p, stream);
+        return;
+    }
+    if (split8_takes(p.M, p.N, p.K)) {
+        p.tiles_m = (p.M + 63) / 64;
+        p.tiles_n = (p.N + 63) / 64;
+        DUQ_LAUNCH_HEAD((gemm_s8_split_kernel<FUSED, BIAS, TILED>), dim3(p.tiles_m * p.tiles_n), dim3(512), 0, stream, p);
         return;
     }
     if (decode8_takes(p.M, p.N, p.K)) {
