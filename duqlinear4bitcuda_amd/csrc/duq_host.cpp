@@ -60,6 +60,24 @@ PyObject *guarded(F f)
     END_HANDLE_TH_ERRORS
 }
 
+// The entries of the module: what throws on the way to the library (a tensor without memory of its own: a vmap or
+// functional wrapper, a sparse tensor) is not the plain case, and goes to the Python code like the rest of those.
+template <class F>
+PyObject *plain_case(F f)
+{
+    try {
+        return f();
+    } catch (const std::exception &) {
+        PyErr_Clear();
+        return none();
+    }
+}
+template <PyObject *(*F)(PyObject *, PyObject *const *, Py_ssize_t)>
+PyObject *entry(PyObject *self, PyObject *const *a, Py_ssize_t n)
+{
+    return plain_case([&] { return F(self, a, n); });
+}
+
 int current_device()
 {
     int d = -1;
@@ -71,6 +89,7 @@ const Tensor *plain(PyObject *o, ScalarType type, int dev)
 {
     if (!THPVariable_CheckExact(o)) return nullptr;
     const Tensor &t = THPVariable_Unpack(o);
+    if (t.layout() != at::kStrided || !t.has_storage()) return nullptr;
     if (!t.is_cuda() || t.scalar_type() != type || !t.is_contiguous() || (dev >= 0 && t.get_device() != dev)) return nullptr;
     return &t;
 }
@@ -265,8 +284,8 @@ void fused_dealloc(PyObject *self)
 }
 
 PyMethodDef g_fused_methods[] = {
-    {"take", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fused_take)), METH_FASTCALL, nullptr},
-    {"take_rows", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fused_take_rows)), METH_FASTCALL, nullptr},
+    {"take", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<fused_take>)), METH_FASTCALL, nullptr},
+    {"take_rows", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<fused_take_rows>)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyTypeObject g_fused_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
@@ -745,11 +764,13 @@ PyObject *module_call(PyObject *, PyObject *const *a, size_t nargsf, PyObject *k
         const Entry *e = plain_module(a[0], dict);
         const bool product = e && (e->kind == kSymProduct || e->kind == kAsymProduct);
         if (e && n == (product ? 3 : 2)) {
-            PyObject *r = e->kind == kSymQuant   ? call_sym_quantizer(a[0], dict, a[1])
-                          : e->kind == kSymLayer ? call_layer(a[0], dict, a[1], false)
-                          : e->kind == kOwnLayer ? call_layer(a[0], dict, a[1], true)
-                          : e->kind == kEightBit ? call_eight_bit(a[0], dict, a[1])
-                                                 : call_product(a[0], dict, a[1], a[2], e->kind == kAsymProduct);
+            PyObject *r = plain_case([&] {
+                return e->kind == kSymQuant   ? call_sym_quantizer(a[0], dict, a[1])
+                       : e->kind == kSymLayer ? call_layer(a[0], dict, a[1], false)
+                       : e->kind == kOwnLayer ? call_layer(a[0], dict, a[1], true)
+                       : e->kind == kEightBit ? call_eight_bit(a[0], dict, a[1])
+                                              : call_product(a[0], dict, a[1], a[2], e->kind == kAsymProduct);
+            });
             if (r != Py_None) return r;
             Py_DECREF(r);
         }
@@ -863,7 +884,7 @@ PyObject *m_setup(PyObject *, PyObject *args)
     Py_RETURN_NONE;
 }
 
-#define FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(fn)), METH_FASTCALL, nullptr}
+#define FAST(name, fn) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<fn>)), METH_FASTCALL, nullptr}
 PyMethodDef g_methods[] = {FAST("defer", m_defer),
                            FAST("quantize_rows", m_quantize_rows),
                            FAST("quantize_rows_8bit", m_quantize_rows_8bit),

@@ -83,3 +83,22 @@ def test_calls_that_are_more_than_the_forward(dev, monkeypatch):
         qnn.SymQuantMatMul()(torch.zeros(2, 4, K, device=dev).half(), torch.zeros(3, 4, K, device=dev).half())
     with pytest.raises(AssertionError, match="Batch dimensions"):
         qnn.AsymQuantMatMul()(torch.zeros(2, 4, K, device=dev).half(), torch.zeros(3, 4, K, device=dev).half())
+
+
+def test_tensors_without_memory_of_their_own(dev):
+    """What has no address (a vmap wrapper, a sparse tensor) is refused with a Python error by modules and ops, as by the Python
+    code that the native calls stand for."""
+    from duqlinear4bitcuda_amd import _HIP as hip, nn as qnn
+    x = torch.randn(3, 4, 128, device=dev).half()
+    lin = torch.nn.Linear(128, 64, bias=False, device=dev, dtype=torch.float16)
+    with torch.device(dev):
+        layer = qnn.Linear4bitASQ.from_linear(lin)
+    layer = layer.to(dev)
+    product = qnn.AsymQuantMatMul()
+    layer(x[0]), product(x, x)   # (the plain case, prepared)
+    refused = (RuntimeError, ValueError, TypeError, NotImplementedError)
+    for f in (layer, hip.quantize_rows_sym, lambda v: product(v, v)):
+        with pytest.raises(refused):
+            torch.func.vmap(lambda v: (f(v), v)[1])(x)
+        with pytest.raises(refused):
+            f(x[0].to_sparse())
