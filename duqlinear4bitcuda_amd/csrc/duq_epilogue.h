@@ -161,6 +161,15 @@ __device__ __forceinline__ uint32_t dequant_pair_x256(int acc0, int acc1, const 
     return dequant_pair<MODE, BIAS>((float)acc0 * (1.0f / 256.0f), (float)acc1 * (1.0f / 256.0f), r, c0, c1);
 }
 
+// The same for accumulators that started at the bits of kF32Base (short rows: |256 * acc| <= 2^22): read as a float they are
+// kF32Base + acc, whose last place is 2^-8 up to 2^16.
+constexpr float kF32Base = 49152.0f;  // 1.5 * 2^15
+template <int MODE, bool BIAS>
+__device__ __forceinline__ uint32_t dequant_pair_based(int acc0, int acc1, const RowEpi &r, const ColParams &c0, const ColParams &c1)
+{
+    return dequant_pair<MODE, BIAS>(__builtin_bit_cast(float, acc0) - kF32Base, __builtin_bit_cast(float, acc1) - kF32Base, r, c0, c1);
+}
+
 // Row-sum epilogue of the dual-uniform layer for one output (definition: include/duq_hip.h,
 // duq_asym_dual_rowsum_dequant_host), shared by the stand-alone kernel and the fused GEMM so that both give
 // identical bits.  xlo / xhi and wlo / whi: the first eight bytes of the packed activation and weight rows, xhi

@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, Gemm
     // before the accumulators are read
     asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
 
-    constexpr bool kWideStore = false;
+    constexpr bool kWideStore = false, kFloatBits = false;
     uint8_t *const wstage = lds + wave * (BM * (64 * TN + 16));
 #include "duq_stream_epilogue_store.inc"
 }
@@ -313,7 +313,8 @@ __global__ __launch_bounds__(256) void gemm_s4_stream_kernel(DUQ_HEAD_DECL, Gemm
 // loop-carried wait for those loads also waits for the stores issued after them.)  The epilogue's per-row parameters go
 // through LDS, one 16-byte read for four rows, instead of a register per row and parameter: 112 registers instead of
 // 148 and no loads of single values at the tile's head (32 products of 2048 x 2048 x 128, asymmetric: 71 -> 67 us;
-// K = 64: 60 -> 52).
+// K = 64: 60 -> 52).  What bounds it now is the mix: 268 MB of stores take 39 us at the rate of a plain fill, the vector
+// work 30 us of issue, and the launch 48 - 58 (into buffers already in the last-level cache, or not).
 template <int TM, int EPI, bool BIAS>
 __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, GemmParams tail)
 {
@@ -330,8 +331,11 @@ __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, G
     const uint32_t dwide = 0;
 
     if (blockIdx.z) batch_shift(p, blockIdx.z);
-    // column blocks fastest: neighbouring workgroups share an activation tile
-    const uint32_t m0 = (blockIdx.x / p.tiles_n) * BM, n0 = (blockIdx.x % p.tiles_n) * BN;
+    // every XCD a contiguous range of tiles, column blocks fastest: whole output rows leave from one XCD (8 products of 4000 x
+    // 4000 x 128: 52.0 -> 48.4 us, 12 of 1111 x 1111 x 128 14.5 -> 14.0, 32 of 2048 x 2048 x 128 49.0 -> 47.9)
+    const uint32_t ntiles = p.tiles_m * p.tiles_n, per = ntiles / 8, rem = ntiles % 8, xcd = blockIdx.x % 8, local = blockIdx.x / 8;
+    const uint32_t id = xcd < rem ? xcd * (per + 1) + local : rem * (per + 1) + (xcd - rem) * per + local;
+    const uint32_t m0 = (id / p.tiles_n) * BM, n0 = (id % p.tiles_n) * BN;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     const uint32_t l32 = lane & 31u, h = lane >> 5;
@@ -371,13 +375,20 @@ __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, G
     }
     __syncthreads();
 
+    // The accumulators of the binary16 epilogues start at the bits of kF32Base: at most 256 products of at most 64, carried x
+    // 256, stay within 2^22, so that they are the float kF32Base + sum all along (one subtraction in place of a conversion
+    // and a scaling per output).
+    constexpr bool kFloatBits = EPI >= 0 && EPI != 4;
+    uint32_t start = kFloatBits ? __builtin_bit_cast(uint32_t, kF32Base) : 0u;
+    v16i acc0;
+    if (kFloatBits) asm volatile("" : "+v"(start));  // (one tuple for all four, not sixteen constants each)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc0[r] = (int)start;
     v16i acc[TN][TM];
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int b = 0; b < TM; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[j][b][r] = 0;
+        for (int b = 0; b < TM; ++b) acc[j][b] = acc0;
     // step (i, par): weight operand = even (par 0) or odd (par 1) nibbles of piece i, activation fragment at
     // + i*64 + par*16 of the row; both sides pair the same k values
     const uint32_t fragX = l32 * kXStride + h * 32;

@@ -350,7 +350,7 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
     if (LATE) fetch_params();
     if (KS == 8 && ks >= (uint32_t)T) p.M = 0;  // no rows of its own: stores nothing
     uint8_t *const wstage = lds + wave * (32 * TM) * (64 * TN + 16);
-    constexpr bool kWideStore = false;
+    constexpr bool kWideStore = false, kFloatBits = false;
 #include "duq_stream_epilogue_store.inc"
 }
 

@@ -2,6 +2,7 @@
 rows that need the element-wise path beside ordinary ones in one wavefront."""
 import numpy as np
 import pytest
+import torch
 
 from oracle import duq_oracle as orc
 from tests import cases
@@ -36,3 +37,28 @@ def test_quantize_short_rows(dev, M, K):
         got = [t.cpu().numpy() for t in hip.quantize_rows_asym_shifted(X)]
         assert np.array_equal(got[0], want[0]) and cases.bits_equal(got[1], want[1]) and cases.bits_equal(got[2], want[2])
         assert np.array_equal(got[3].reshape(-1), want[3].reshape(-1))
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 256])
+def test_products_of_extreme_codes(dev, K):
+    """Short rows, whose accumulators start at a float's bits: sums at both ends of their range (every code -8, and -8 against
+    7) and around zero, through the four epilogues that read them so, against the stand-alone ones on int32."""
+    from duqlinear4bitcuda_amd import _HIP as hip
+    M, N = 70, 300
+    a = torch.randint(0, 256, (M, K // 2), dtype=torch.uint8, device=dev)
+    b = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, device=dev)
+    a[:20], a[20:40], b[:99], b[99:180] = 0x88, 0x77, 0x88, 0x77
+    acc = hip.matmul(a, b)
+    assert int(acc.max()) == 64 * K and int(acc.min()) == -56 * K
+    h = lambda n: (torch.rand(n, device=dev) * 4 - 2).half()
+    sr, zr, s1, z1, s2, z2, bias = h(M), h(M).round(), h(N), h(N).round(), h(N), h(N).round(), h(N)
+    steps = ((hip.EPI_SYM, (sr, None), (s1, None, None, None), hip.sym_dequant(acc, sr, s1)),
+             (hip.EPI_ASYM, (sr, zr), (s1, z1, None, None), hip.asym_dequant(acc, sr, zr, s1, z1)),
+             (hip.EPI_SYM_DUAL, (sr, None), (s1, None, s2, None), hip.sym_dual_dequant(acc, sr, s1, s2)),
+             (hip.EPI_ASYM_DUAL, (sr, zr), (s1, z1, s2, z2), hip.asym_dual_dequant(acc, sr, zr, s1, z1, s2, z2)))
+    for mode, r, c, y in steps:
+        for add in (None, bias):
+            got = hip.batch_linear4bit_forward(mode, a[None], *(t if t is None else t[None] for t in r), b[None],
+                                               *(t if t is None else t[None] for t in c), bias=None if add is None else add[None])
+            want = y if add is None else y + add
+            assert torch.equal(got[0].view(torch.int16), want.view(torch.int16)), (mode, add is None)
