@@ -770,16 +770,16 @@ def main():
                                    PREWARM_STEPS + args.warmup)
     i8_quant_us = graph_time_us([lambda: hip.quantize_rows_sym(x)] * 40)
     integer_path = {"ms_per_step": round(i8_ms_per_step, 5), "TOPS": round(ops / (i8_ms_per_step * 1e-3) / 1e12, 2),
-                    "kernel": "gemm_s4_stream_kernel<4,0,false,2> (v_mfma_i32_32x32x32_i8, 128 x 256 tiles)", "gemm_fused_us": round(i8_gemm_us, 2),
+                    "kernel": "gemm_s4_prefill_kernel<2,2,2,4,1,128,0,false> (v_mfma_i32_32x32x32_i8, 128 x 256 tiles)", "gemm_fused_us": round(i8_gemm_us, 2),
                     "quantize_rows_sym_us": round(i8_quant_us, 2),
-                    "roofline": {"bound": "mfma", "kernel": "gemm_s4_stream_kernel (fused GEMM + dequant on v_mfma_i32_32x32x32_i8)",
+                    "roofline": {"bound": "mfma", "kernel": "gemm_s4_prefill_kernel (fused GEMM + dequant on v_mfma_i32_32x32x32_i8)",
                                  "achieved": round(ops / i8_gemm_us / 1e6, 1), "peak": PEAK_INT8_TOPS,
                                  "unit": "TOP/s", "frac": round(ops / i8_gemm_us / 1e6 / PEAK_INT8_TOPS, 4),
                                  "avg_kernel_us": round(i8_gemm_us, 2), "launches_timed": n_timed,
                                  "shader_clock_during_timing": clk_i8.summary(),
-                                 "traffic": profile_traffic_bytes("gemm_s4_stream_kernel__prefill_M2048_K4096_N4096.txt",
-                                                                  "gemm_s4_stream_kernel"),
-                                 "traffic_source": "profiles/gemm_s4_stream_kernel__prefill_M2048_K4096_N4096.txt"}}
+                                 "traffic": profile_traffic_bytes("gemm_s4_prefill_kernel__prefill_M2048_K4096_N4096.txt",
+                                                                  "gemm_s4_prefill_kernel"),
+                                 "traffic_source": "profiles/gemm_s4_prefill_kernel__prefill_M2048_K4096_N4096.txt"}}
     # the driver record keeps `roofline`: the integer path's figures ride inside it as a second entry
     roofline["integer_path"] = integer_path["roofline"]
 

@@ -223,13 +223,13 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
 
 /* Which kernel family duq_matmul_host_4bit / duq_linear4bit_forward run for a shape (no GPU work; for tests
  * and tuning): 1 decode rows kernel (M <= 4), 2 decode MFMA kernel (M <= 16; up to 64 rows of at most 8192
- * elements, 48 of at most 12288), 3 dot kernel (M <= 4, rows longer than 16384 elements), 4 ring kernel, 5 skinny
+ * elements, 48 of at most 12288, where family 6 is not ahead), 3 dot kernel (M <= 4, rows longer than 16384 elements), 4 ring kernel, 5 skinny
  * kernel (9 <= M <= 16, very wide problems), 6 prefill kernel (short rows: stream kernel),
  * 7 the same on problems of few tiles or long rows.  Families 1-5 address the weight tensor with 32-bit byte offsets and are only picked while
  * N * K / 2 < 2^32 - 256; larger tensors run families 6 and 7, whose bases are 64-bit per tile.  No
  * counterpart in the reference (CUTLASS picks its own tile, src/kernels/gemm.cu:17-42). */
 int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
-/* For a shape of family 6: its tile as rows * 1000 + columns (256256, 128256, 128128, 64128); 0 for the other families.  (The dual-uniform row-sum epilogue never runs the 256-row tile.) */
+/* For a shape of family 6: its tile as rows * 1000 + columns (256256, 128256, 128128, 64128, 96064, 64064); 0 for the other families.  (The dual-uniform row-sum epilogue never runs the 256-row tile.) */
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
 
 /* Measurement aid, no counterpart in the reference: reads `bytes` (16-byte aligned, < 4 GiB) of device memory
