@@ -137,14 +137,11 @@ def _install_calls(native):
     from torch.nn.modules import module as m
 
     from . import _HIP, nn
-    kinds = ((nn.SymQuantizer,), (nn.Linear4bitSQ, nn.Linear4bitDUSQ),
-             (nn.Linear4bitASQ, nn.LinearQuant4bitDUASQ, nn.Linear4bitASQRowSum, nn.LinearQuant4bitDUASQRowSum),
-             (nn.LinearQuant8bitASQ,), (nn.SymQuantMatMul,), (nn.AsymQuantMatMul,))
-    classes = [(cls, kind) for kind, group in enumerate(kinds) for cls in group] + [(nn.AsymQuantizer, -1)]
+    from .nn import _calls
     lib = load()
-    native.install(tuple(c for c in classes if c[0].forward.__module__ == c[0].__module__),   # (forwards as they are written there)
+    native.install(tuple(_calls.classes),
                    (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks, m._global_backward_pre_hooks),
-                   m.Module, (_HIP, _HIP._own_launch), (lib, lib._FuncPtr),
+                   (m.Module, _calls.module_call, _calls.module_call_impl), (_HIP, _HIP._own_launch), (lib, lib._FuncPtr),
                    (nn.SymQuantizer, nn.AsymQuantizer, nn.AsymQuantizer8bit))
 
 

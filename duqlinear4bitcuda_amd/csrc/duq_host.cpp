@@ -525,7 +525,7 @@ struct Entry {
 };
 std::vector<Entry> *g_entries = nullptr;
 PyTypeObject *g_module_type = nullptr;           // torch.nn.Module
-PyObject *g_module_call[3], *g_module_call_names[3];  // what stands behind its __call__, and under which names
+PyObject *g_module_call[2], *g_module_call_names[2];  // what stands behind its __call__, and under which names
 std::vector<PyObject *> *g_global_hooks = nullptr;    // torch's dicts of hooks for every module
 PyObject *g_ops_dict = nullptr, *g_launch = nullptr;  // _HIP's namespace and the _launch function defined there
 PyObject *g_lib_dict = nullptr;                  // attributes of the ctypes library object
@@ -606,7 +606,7 @@ const Entry *plain_module(PyObject *self, PyObject *dict)
 
 bool plain_torch()
 {
-    for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 2; ++i)
         if (get(g_module_type->tp_dict, g_module_call_names[i]) != g_module_call[i]) return false;
     for (PyObject *d : *g_global_hooks)
         if (PyDict_GET_SIZE(d)) return false;
@@ -794,14 +794,16 @@ PyObject *module_call_get(PyObject *self, PyObject *obj, PyObject *)
 
 PyTypeObject g_module_call_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-// install(classes, torch's hook dicts, torch.nn.Module, (_HIP module, its _launch), (ctypes library, type of its functions),
-// (SymQuantizer, AsymQuantizer, AsymQuantizer8bit)): `classes` is a tuple of (class, kind as in Kind, or -1 for a class
-// that only a product looks at); gives every one of them the native __call__
+// install(classes, torch's hook dicts, (torch.nn.Module, its own __call__ and _call_impl, None for one that is not torch's: no
+// call is then run natively), (_HIP module, its _launch), (ctypes library, type of its functions), (SymQuantizer, AsymQuantizer,
+// AsymQuantizer8bit)): `classes` is a tuple of (class, kind as in Kind, or -1 for a class that only a product looks at, the
+// forward it was defined with); gives every one of them the native __call__ that has no __call__ of its own
 PyObject *m_install(PyObject *, PyObject *args)
 {
-    PyObject *classes, *hooks, *module, *ops, *lib, *launch, *funcptr, *sym, *asym, *quant8;
-    if (!PyArg_ParseTuple(args, "O!O!O!(OO)(OO!)(O!O!O!)", &PyTuple_Type, &classes, &PyTuple_Type, &hooks, &PyType_Type, &module, &ops,
-                          &launch, &lib, &PyType_Type, &funcptr, &PyType_Type, &sym, &PyType_Type, &asym, &PyType_Type, &quant8))
+    PyObject *classes, *hooks, *module, *call[2], *ops, *lib, *launch, *funcptr, *sym, *asym, *quant8;
+    if (!PyArg_ParseTuple(args, "O!O!(O!OO)(OO)(OO!)(O!O!O!)", &PyTuple_Type, &classes, &PyTuple_Type, &hooks, &PyType_Type, &module,
+                          &call[0], &call[1], &ops, &launch, &lib, &PyType_Type, &funcptr, &PyType_Type, &sym, &PyType_Type, &asym,
+                          &PyType_Type, &quant8))
         return nullptr;
     PyObject *lib_dict = dict_of(lib), *ops_dict = dict_of(ops);
     if (g_names || !lib_dict || !ops_dict) {
@@ -810,13 +812,11 @@ PyObject *m_install(PyObject *, PyObject *args)
     }
     const Names *names = new Names();
     bool found = true;
-    static const char *const call_names[3] = {"__call__", "_wrapped_call_impl", "_call_impl"};
-    PyObject *module_dict = reinterpret_cast<PyTypeObject *>(module)->tp_dict;
-    for (int i = 0; i < 3; ++i) {
+    static const char *const call_names[2] = {"__call__", "_call_impl"};
+    for (int i = 0; i < 2; ++i) {
         g_module_call_names[i] = PyUnicode_InternFromString(call_names[i]);
-        g_module_call[i] = get(module_dict, g_module_call_names[i]);
-        Py_XINCREF(g_module_call[i]);
-        if (!g_module_call[i]) found = false;
+        Py_INCREF(call[i]);
+        g_module_call[i] = call[i];
     }
     auto *global_hooks = new std::vector<PyObject *>();
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(hooks); ++i) {
@@ -827,14 +827,13 @@ PyObject *m_install(PyObject *, PyObject *args)
     }
     auto *entries = new std::vector<Entry>();
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(classes); ++i) {
-        PyObject *cls;
+        PyObject *cls, *forward;
         int kind;
-        if (!PyArg_ParseTuple(PyTuple_GET_ITEM(classes, i), "O!i", &PyType_Type, &cls, &kind)) return nullptr;
+        if (!PyArg_ParseTuple(PyTuple_GET_ITEM(classes, i), "O!iO", &PyType_Type, &cls, &kind, &forward)) return nullptr;
         PyTypeObject *t = reinterpret_cast<PyTypeObject *>(cls);
-        PyObject *forward = get(t->tp_dict, names->forward);
-        if (!forward) found = false;
+        if (get(t->tp_dict, names->__call__)) continue;   // (somebody's wrapper: every call of the class goes through it)
         Py_INCREF(cls);
-        Py_XINCREF(forward);
+        Py_INCREF(forward);
         entries->push_back(Entry{t, forward, static_cast<Kind>(kind)});
     }
     if (!found) {
@@ -853,15 +852,22 @@ PyObject *m_install(PyObject *, PyObject *args)
     g_global_hooks = global_hooks;
     g_entries = entries;
     g_names = names;
-    ModuleCall *call = PyObject_New(ModuleCall, &g_module_call_type);
-    if (!call) return nullptr;
-    call->call = module_call;
+    ModuleCall *own = PyObject_New(ModuleCall, &g_module_call_type);
+    if (!own) return nullptr;
+    own->call = module_call;
     int bad = 0;
     for (const Entry &e : *entries)
-        bad |= e.kind >= 0 ? PyObject_SetAttr(reinterpret_cast<PyObject *>(e.type), names->__call__, reinterpret_cast<PyObject *>(call)) : 0;
-    Py_DECREF(call);
+        bad |= e.kind >= 0 ? PyObject_SetAttr(reinterpret_cast<PyObject *>(e.type), names->__call__, reinterpret_cast<PyObject *>(own)) : 0;
+    Py_DECREF(own);
     if (bad) return nullptr;
     Py_RETURN_NONE;
+}
+
+// plain_call(module): whether a call of it is its class's forward as it was written and nothing else, so that it may be
+// run natively
+PyObject *m_plain_call(PyObject *, PyObject *module)
+{
+    return PyBool_FromLong(g_names && plain_torch() && plain_module(module, dict_of(module)));
 }
 
 // setup(PackedQuantizedTensor, check): the class defer() makes instances of, and what raises for a status
@@ -893,6 +899,7 @@ PyMethodDef g_methods[] = {FAST("defer", m_defer),
                            FAST("linear8", m_linear8),
                            {"setup", m_setup, METH_VARARGS, nullptr},
                            {"install", m_install, METH_VARARGS, nullptr},
+                           {"plain_call", m_plain_call, METH_O, nullptr},
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_duq_host", "host side of the ops (csrc/duq_host.cpp)", -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

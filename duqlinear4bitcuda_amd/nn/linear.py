@@ -18,6 +18,7 @@ import torch
 from .. import _HIP as _ops
 from ..tools import quantization as quant_utils
 from ..tools import tensor_utils
+from ._calls import native_call
 from .quantizer import AsymQuantizer, AsymQuantizer8bit, SymQuantizer  # noqa: F401  (re-exported like the reference)
 
 _INT4_LEVELS = 2 ** 4
@@ -247,6 +248,7 @@ class _Linear4bitBase(torch.nn.Module):
         return self.quantizer(x, shadow="only" if self._fp6_wanted(rows) else False)
 
 
+@native_call("sym_layer")
 class Linear4bitSQ(_Linear4bitBase):
     """Symmetric 4-bit linear layer; takes a PackedQuantizedTensor (linear.py:24-78)."""
 
@@ -293,6 +295,7 @@ class Linear4bitSQ(_Linear4bitBase):
         return new
 
 
+@native_call("own_layer")
 class Linear4bitASQ(_Linear4bitBase):
     """Asymmetric 4-bit linear layer with its own AsymQuantizer (linear.py:80-145)."""
 
@@ -346,6 +349,7 @@ class Linear4bitASQ(_Linear4bitBase):
         return new
 
 
+@native_call("own_layer")
 class Linear4bitASQRowSum(_Linear4bitBase):
     """Asymmetric 4-bit linear layer with the exact zero-point correction.  Not in the
     reference: its Linear4bitASQ stores unsigned codes that the signed GEMM misreads
@@ -415,6 +419,7 @@ class Linear4bitASQRowSum(_Linear4bitBase):
         return new
 
 
+@native_call("own_layer")
 class LinearQuant4bitDUASQRowSum(_Linear4bitBase):
     """Dual-uniform asymmetric layer with the exact zero-point correction.  Not in the reference: its
     LinearQuant4bitDUASQ (linear.py:209-297) quantizes input columns 0..9 of every weight row with one
@@ -519,6 +524,7 @@ class LinearQuant4bitDUASQRowSum(_Linear4bitBase):
         return new
 
 
+@native_call("sym_layer")
 class Linear4bitDUSQ(_Linear4bitBase):
     """Symmetric layer with two per-row weight scales: input columns < 10 were quantized
     with scale 1, the rest with scale 2; the epilogue picks per OUTPUT column < 10
@@ -572,6 +578,7 @@ class Linear4bitDUSQ(_Linear4bitBase):
         return new
 
 
+@native_call("own_layer")
 class LinearQuant4bitDUASQ(_Linear4bitBase):
     """Asymmetric dual-uniform layer (linear.py:209-297)."""
 
@@ -632,6 +639,7 @@ class LinearQuant4bitDUASQ(_Linear4bitBase):
         return new
 
 
+@native_call("eight_bit")
 class LinearQuant8bitASQ(torch.nn.Module):
     """Asymmetric 8-bit linear layer on float32 activations (linear.py:300-368): buffers ``weight`` int8
     [N, K] (codes 0..127), ``weight_scales`` / ``weight_zeros`` float32 [N, 1], optional ``bias``

@@ -17,9 +17,11 @@ import torch
 
 from .. import _HIP as _ops
 from ..tools import tensor_utils
+from ._calls import native_call
 from .quantizer import AsymQuantizer, SymQuantizer
 
 
+@native_call("sym_product")
 class SymQuantMatMul(torch.nn.Module):
     """sym_dequant(matmul(q(A), q(B)), s_A, s_B) (matmul.py:69-84): A [..., M, K] against a 2-D B [N, K] gives
     [..., M, N], as in the reference (its wrappers flatten the leading dimensions of A).
@@ -61,6 +63,7 @@ class SymQuantMatMul(torch.nn.Module):
         return tensor_utils.sym_dequant(out, A.scales_x, B.scales_x)
 
 
+@native_call("asym_product")
 class AsymQuantMatMul(torch.nn.Module):
     """Batched asymmetric product (matmul.py:19-66): A [..., HA, W], B [..., HB, W] (or [..., W, HB] with
     ``transpose_B``), leading dimensions equal; returns fp16 [..., HA, HB] with the reference's asymmetric

@@ -7,6 +7,7 @@ import torch
 
 from .. import _lib
 from ..tools import tensor_utils
+from ._calls import LOOKED_AT, native_call
 
 
 def _shadow_choice(quantizer, x, override):
@@ -21,6 +22,7 @@ def _shadow_choice(quantizer, x, override):
     return False
 
 
+@native_call("sym_quantizer")
 class SymQuantizer(torch.nn.Module):
     """x fp16 [..., K] -> PackedQuantizedTensor(q u8 [..., K/2], scales fp16 [..., 1]).
 
@@ -70,6 +72,7 @@ class SymQuantizer(torch.nn.Module):
         return tensor_utils.PackedQuantizedTensor(q, scales)
 
 
+@native_call(LOOKED_AT)
 class AsymQuantizer(torch.nn.Module):
     """scale = (max - min) / 15, zero = round(-min / scale), unsigned codes 0..15
     (quantizer.py:24-35).  ``input_clip_ratio`` is accepted and unused, as in the
