@@ -7,6 +7,7 @@ loading raises and every op of this package fails.
 from __future__ import annotations
 
 import ctypes
+import inspect
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -143,6 +144,11 @@ def _install_calls(native):
                    (m._global_forward_hooks, m._global_forward_pre_hooks, m._global_backward_hooks, m._global_backward_pre_hooks),
                    (m.Module, _calls.module_call, _calls.module_call_impl), (_HIP, _HIP._own_launch), (lib, lib._FuncPtr),
                    (nn.SymQuantizer, nn.AsymQuantizer, nn.AsymQuantizer8bit))
+    for cls, kind, _ in _calls.classes:
+        call = cls.__dict__.get("__call__")
+        if type(call) is native.ModuleCall:   # (what inspect and help show is torch's)
+            call.__name__, call.__qualname__, call.__module__ = "__call__", f"{cls.__qualname__}.__call__", cls.__module__
+            call.__doc__, call.__signature__ = m.Module.__call__.__doc__, inspect.signature(m.Module.__call__)
 
 
 def host():

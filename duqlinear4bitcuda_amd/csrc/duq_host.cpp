@@ -9,6 +9,7 @@
 // word the errors.  Nothing is computed or kept here, outputs and staging come from torch's allocator, and the
 // interpreter lock is given up around the calls that launch (a full queue makes a launch wait).
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
@@ -513,19 +514,23 @@ PyObject *m_linear8(PyObject *, PyObject *const *a, Py_ssize_t n)
 
 // ---- calls of modules ----------------------------------------------------------------------------------------
 // `__call__` of the framework's module classes: what torch.nn.Module.__call__ and the class's forward do in the plain
-// case (no hooks, no compiled or replaced forward, plain tensors, buffers as they were when the layer's call was
-// prepared), in one piece of native code: 0.2 us where the two Python frames cost 1 (quantizer and layer of a decode
-// step 6.6 -> 5.5 us).  Anything else goes to torch.nn.Module.__call__ as it is at that moment.
+// case (no hooks, no compiled or replaced forward, no other __call__ or _call_impl on the way, plain tensors, buffers as
+// they were when the layer's call was prepared), in one piece of native code: 0.2 us where the two Python frames cost 1
+// (quantizer and layer of a decode step 6.6 -> 5.5 us).  Anything else goes to the __call__ that comes next in the method
+// order of the object's class, as super().__call__ would: mostly torch.nn.Module's.
 
 enum Kind { kSymQuant, kSymLayer, kOwnLayer, kEightBit, kSymProduct, kAsymProduct };
 struct Entry {
     PyTypeObject *type;
     PyObject *forward;
     Kind kind;
+    PyObject *call = nullptr;          // the __call__ that its instances have: a ModuleCall, or torch's for kind -1
+    PyObject *mro = nullptr;           // the method order at the time,
+    std::vector<PyTypeObject *> bases; // and what stands between the class and torch.nn.Module there
 };
 std::vector<Entry> *g_entries = nullptr;
 PyTypeObject *g_module_type = nullptr;           // torch.nn.Module
-PyObject *g_module_call[2], *g_module_call_names[2];  // what stands behind its __call__, and under which names
+PyObject *g_module_call = nullptr, *g_call_impl = nullptr;  // its __call__, and the _call_impl that this one calls
 std::vector<PyObject *> *g_global_hooks = nullptr;    // torch's dicts of hooks for every module
 PyObject *g_ops_dict = nullptr, *g_launch = nullptr;  // _HIP's namespace and the _launch function defined there
 PyObject *g_lib_dict = nullptr;                  // attributes of the ctypes library object
@@ -539,6 +544,7 @@ struct Names {
     NAME(_backward_hooks);
     NAME(_backward_pre_hooks);
     NAME(_compiled_call_impl);
+    NAME(_call_impl);
     NAME(forward);
     NAME(_buffers);
     NAME(_modules);
@@ -590,27 +596,37 @@ PyObject *dict_of(PyObject *o)
 
 bool empty_dict(PyObject *d) { return d && PyDict_Check(d) && PyDict_GET_SIZE(d) == 0; }
 
-// The entry of a module whose call is its class's forward and nothing else, or null.
+// The entry of a module for which torch's __call__ would run its class's forward and nothing else, or null.
 const Entry *plain_module(PyObject *self, PyObject *dict)
 {
     const Entry *e = nullptr;
     for (const Entry &k : *g_entries)
         if (k.type == Py_TYPE(self)) e = &k;
     const Names &n = *g_names;
-    if (!e || !dict || get(e->type->tp_dict, n.forward) != e->forward || get(dict, n.forward)) return nullptr;
+    if (!e || !dict || e->type->tp_mro != e->mro) return nullptr;
+    if (_PyType_Lookup(e->type, n.forward) != e->forward || get(dict, n.forward)) return nullptr;
+    if (_PyType_Lookup(e->type, n._call_impl) != g_call_impl || get(dict, n._call_impl)) return nullptr;
+    if (attr(self, dict, n._compiled_call_impl) != Py_None) return nullptr;
+    for (PyTypeObject *base : e->bases)
+        if (get(base->tp_dict, n.__call__)) return nullptr;
     for (PyObject *h : {n._forward_hooks, n._forward_pre_hooks, n._backward_hooks, n._backward_pre_hooks})
         if (!empty_dict(get(dict, h))) return nullptr;
-    PyObject *compiled = get(dict, n._compiled_call_impl);
-    return compiled && compiled != Py_None ? nullptr : e;
+    return e;
+}
+
+// The same for a module that is not being called already: its class's __call__ has to be the one known too.
+const Entry *plain_call(PyObject *self, PyObject *dict)
+{
+    const Entry *e = plain_module(self, dict);
+    return e && _PyType_Lookup(e->type, g_names->__call__) == e->call ? e : nullptr;
 }
 
 bool plain_torch()
 {
-    for (int i = 0; i < 2; ++i)
-        if (get(g_module_type->tp_dict, g_module_call_names[i]) != g_module_call[i]) return false;
+    if (get(g_module_type->tp_dict, g_names->__call__) != g_module_call) return false;
     for (PyObject *d : *g_global_hooks)
         if (PyDict_GET_SIZE(d)) return false;
-    return true;
+    return !torch::jit::tracer::isTracing();   // (torch then calls _slow_forward)
 }
 
 // the library's own function under that name (a tracer may have put a Python one there)
@@ -698,7 +714,7 @@ PyObject *call_product(PyObject *self, PyObject *dict, PyObject *pa, PyObject *p
     PyObject *const names[2] = {n.quantizer_A, n.quantizer_B};
     for (int i = 0; i < 2; ++i) {
         PyObject *q = get(modules, names[i]), *qd = q ? dict_of(q) : nullptr;
-        if (!q || Py_TYPE(q) != (asym ? g_asym_type : g_sym_type) || !plain_module(q, qd) || get(qd, n.shadow) != Py_False) return none();
+        if (!q || Py_TYPE(q) != (asym ? g_asym_type : g_sym_type) || !plain_call(q, qd) || get(qd, n.shadow) != Py_False) return none();
         if (asym) {
             if (get(qd, n.shifted) != Py_False) return none();
         } else {
@@ -754,12 +770,46 @@ PyObject *call_product(PyObject *self, PyObject *dict, PyObject *pa, PyObject *p
 struct ModuleCall {
     PyObject_HEAD
     vectorcallfunc call;
+    PyTypeObject *owner;   // the class whose __call__ it is
+    PyObject *dict;        // __name__, __doc__, __signature__: those of torch.nn.Module's
 };
 
-PyObject *module_call(PyObject *, PyObject *const *a, size_t nargsf, PyObject *kwnames)
+// super(owner, self).__call__(...)
+PyObject *next_call(PyTypeObject *owner, PyObject *const *a, Py_ssize_t n, PyObject *kwnames)
 {
+    PyTypeObject *type = n && PyType_IsSubtype(Py_TYPE(a[0]), owner) ? Py_TYPE(a[0]) : owner;
+    PyObject *mro = type->tp_mro, *f = nullptr;
+    bool behind = false;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(mro) && !f; ++i) {
+        PyTypeObject *t = reinterpret_cast<PyTypeObject *>(PyTuple_GET_ITEM(mro, i));
+        if (behind) f = get(t->tp_dict, g_names->__call__);
+        behind |= t == owner;
+    }
+    if (!f) {
+        PyErr_Format(PyExc_TypeError, "'%.200s' object is not callable", type->tp_name);
+        return nullptr;
+    }
+    Py_INCREF(f);
+    PyObject *r = nullptr;
+    if (!n || Py_TYPE(f)->tp_flags & Py_TPFLAGS_METHOD_DESCRIPTOR) {   // (a function: takes the object as its first argument)
+        r = PyObject_Vectorcall(f, a, static_cast<size_t>(n), kwnames);
+    } else if (descrgetfunc bind = Py_TYPE(f)->tp_descr_get) {
+        if (PyObject *bound = bind(f, a[0], reinterpret_cast<PyObject *>(Py_TYPE(a[0])))) {
+            r = PyObject_Vectorcall(bound, a + 1, static_cast<size_t>(n - 1), kwnames);
+            Py_DECREF(bound);
+        }
+    } else {
+        r = PyObject_Vectorcall(f, a + 1, static_cast<size_t>(n - 1), kwnames);
+    }
+    Py_DECREF(f);
+    return r;
+}
+
+PyObject *module_call(PyObject *self, PyObject *const *a, size_t nargsf, PyObject *kwnames)
+{
+    PyTypeObject *owner = reinterpret_cast<ModuleCall *>(self)->owner;
     const Py_ssize_t n = PyVectorcall_NARGS(nargsf);
-    if (!kwnames && n >= 2 && n <= 3 && plain_torch()) {
+    if (!kwnames && n >= 2 && n <= 3 && Py_TYPE(a[0]) == owner && plain_torch()) {
         PyObject *dict = dict_of(a[0]);
         const Entry *e = plain_module(a[0], dict);
         const bool product = e && (e->kind == kSymProduct || e->kind == kAsymProduct);
@@ -775,12 +825,7 @@ PyObject *module_call(PyObject *, PyObject *const *a, size_t nargsf, PyObject *k
             Py_DECREF(r);
         }
     }
-    // torch.nn.Module.__call__(self, ...)
-    PyObject *f = PyObject_GetAttr(reinterpret_cast<PyObject *>(g_module_type), g_names->__call__);
-    if (!f) return nullptr;
-    PyObject *r = PyObject_Vectorcall(f, a, static_cast<size_t>(n), kwnames);
-    Py_DECREF(f);
-    return r;
+    return next_call(owner, a, n, kwnames);
 }
 
 PyObject *module_call_get(PyObject *self, PyObject *obj, PyObject *)
@@ -806,18 +851,13 @@ PyObject *m_install(PyObject *, PyObject *args)
                           &PyType_Type, &quant8))
         return nullptr;
     PyObject *lib_dict = dict_of(lib), *ops_dict = dict_of(ops);
+    PyTypeObject *module_type = reinterpret_cast<PyTypeObject *>(module);
     if (g_names || !lib_dict || !ops_dict) {
         PyErr_SetString(PyExc_RuntimeError, "install: once, with a module and a library object");
         return nullptr;
     }
     const Names *names = new Names();
     bool found = true;
-    static const char *const call_names[2] = {"__call__", "_call_impl"};
-    for (int i = 0; i < 2; ++i) {
-        g_module_call_names[i] = PyUnicode_InternFromString(call_names[i]);
-        Py_INCREF(call[i]);
-        g_module_call[i] = call[i];
-    }
     auto *global_hooks = new std::vector<PyObject *>();
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(hooks); ++i) {
         PyObject *d = PyTuple_GET_ITEM(hooks, i);
@@ -834,14 +874,21 @@ PyObject *m_install(PyObject *, PyObject *args)
         if (get(t->tp_dict, names->__call__)) continue;   // (somebody's wrapper: every call of the class goes through it)
         Py_INCREF(cls);
         Py_INCREF(forward);
-        entries->push_back(Entry{t, forward, static_cast<Kind>(kind)});
+        Entry e{t, forward, static_cast<Kind>(kind)};
+        e.mro = t->tp_mro;
+        Py_INCREF(e.mro);
+        for (Py_ssize_t k = 1; k < PyTuple_GET_SIZE(e.mro) && PyTuple_GET_ITEM(e.mro, k) != module; ++k)
+            e.bases.push_back(reinterpret_cast<PyTypeObject *>(PyTuple_GET_ITEM(e.mro, k)));
+        entries->push_back(e);
     }
     if (!found) {
         PyErr_SetString(PyExc_RuntimeError, "install: a function or dictionary is not where it was expected");
         return nullptr;
     }
-    for (PyObject *o : {module, launch, ops_dict, lib_dict, funcptr, sym, asym, quant8}) Py_INCREF(o);
-    g_module_type = reinterpret_cast<PyTypeObject *>(module);
+    for (PyObject *o : {module, call[0], call[1], launch, ops_dict, lib_dict, funcptr, sym, asym, quant8}) Py_INCREF(o);
+    g_module_type = module_type;
+    g_module_call = call[0];
+    g_call_impl = call[1];
     g_ops_dict = ops_dict;
     g_launch = launch;
     g_lib_dict = lib_dict;
@@ -852,14 +899,17 @@ PyObject *m_install(PyObject *, PyObject *args)
     g_global_hooks = global_hooks;
     g_entries = entries;
     g_names = names;
-    ModuleCall *own = PyObject_New(ModuleCall, &g_module_call_type);
-    if (!own) return nullptr;
-    own->call = module_call;
-    int bad = 0;
-    for (const Entry &e : *entries)
-        bad |= e.kind >= 0 ? PyObject_SetAttr(reinterpret_cast<PyObject *>(e.type), names->__call__, reinterpret_cast<PyObject *>(own)) : 0;
-    Py_DECREF(own);
-    if (bad) return nullptr;
+    for (Entry &e : *entries) {
+        e.call = g_module_call;
+        if (e.kind < 0) continue;
+        ModuleCall *own = PyObject_New(ModuleCall, &g_module_call_type);
+        if (!own) return nullptr;
+        own->call = module_call;
+        own->owner = e.type;
+        own->dict = nullptr;
+        e.call = reinterpret_cast<PyObject *>(own);   // (kept for good)
+        if (PyObject_SetAttr(reinterpret_cast<PyObject *>(e.type), names->__call__, e.call) < 0) return nullptr;
+    }
     Py_RETURN_NONE;
 }
 
@@ -867,7 +917,7 @@ PyObject *m_install(PyObject *, PyObject *args)
 // run natively
 PyObject *m_plain_call(PyObject *, PyObject *module)
 {
-    return PyBool_FromLong(g_names && plain_torch() && plain_module(module, dict_of(module)));
+    return PyBool_FromLong(g_names && plain_torch() && plain_call(module, dict_of(module)));
 }
 
 // setup(PackedQuantizedTensor, check): the class defer() makes instances of, and what raises for a status
@@ -920,10 +970,15 @@ PyMODINIT_FUNC PyInit__duq_host(void)
     g_module_call_type.tp_vectorcall_offset = offsetof(ModuleCall, call);
     g_module_call_type.tp_call = PyVectorcall_Call;
     g_module_call_type.tp_descr_get = module_call_get;
+    g_module_call_type.tp_dictoffset = offsetof(ModuleCall, dict);
+    g_module_call_type.tp_getattro = PyObject_GenericGetAttr;
+    g_module_call_type.tp_setattro = PyObject_GenericSetAttr;
     if (PyType_Ready(&g_module_call_type) < 0) return nullptr;
     PyObject *m = PyModule_Create(&g_module);
     if (!m) return nullptr;
     Py_INCREF(&g_fused_type);
     if (PyModule_AddObject(m, "FusedCall", reinterpret_cast<PyObject *>(&g_fused_type)) < 0) return nullptr;
+    Py_INCREF(&g_module_call_type);
+    if (PyModule_AddObject(m, "ModuleCall", reinterpret_cast<PyObject *>(&g_module_call_type)) < 0) return nullptr;
     return m;
 }

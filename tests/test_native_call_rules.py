@@ -29,7 +29,7 @@ def modules():
 def call(m):
     x = torch.zeros(2, 128, dtype=torch.float16)
     try:
-        m(x, x) if "MatMul" in type(m).__name__ else m(x)
+        m(x, x) if hasattr(m, "quantizer_B") else m(x)
     except (RuntimeError, AssertionError):
         pass
 def plain():
@@ -94,3 +94,87 @@ def run(body):
 @pytest.mark.parametrize("what", CASES)
 def test_what_was_replaced_before_the_first_call_is_called(what):
     run(CASES[what])
+
+
+# put in place before or after the first call: what a call does must not depend on that
+METHOD_ORDER = {
+    "a class behind in the method order": """
+class Mixin(torch.nn.Module):
+    def __call__(self, *a, **k):
+        seen.append("mixin")
+        return super().__call__(*a, **k)
+for m in modules():
+    cls = type(m)
+    sub = type("Sub", (cls, Mixin), {})
+    s = sub(128, 64) if hasattr(m, "in_features") else sub()
+    seen.clear()
+    call(s)
+    assert seen == ["mixin"], (cls, seen)
+""",
+    "a base class": """
+from duqlinear4bitcuda_amd.nn.linear import _Linear4bitBase as base
+base.__call__ = wrapped(torch.nn.Module.__call__)
+for m in modules():
+    below = isinstance(m, base)
+    seen.clear()
+    call(m)
+    assert (seen == [base.__call__]) == below and (first or host.plain_call(m) != below), type(m)
+del base.__call__
+base._call_impl = wrapped(torch.nn.Module._call_impl)
+for m in modules():
+    below = isinstance(m, base)
+    seen.clear()
+    call(m)
+    assert (seen == [base._call_impl]) == below and (first or host.plain_call(m) != below), type(m)
+del base._call_impl
+""",
+    "an instance": """
+for m in modules():
+    m._call_impl = wrapped(m._call_impl)
+    seen.clear()
+    call(m)
+    assert seen == [m._call_impl] and (first or not host.plain_call(m)), type(m)
+    del m._call_impl
+    m.compile(backend=lambda g, x: g)
+    assert first or not host.plain_call(m)
+""",
+    "a callable that is no function": """
+class Next:
+    def __call__(self, *a, **k):
+        seen.append(a)
+class Binds:
+    def __get__(self, obj, cls):
+        return lambda *a, **k: seen.append((obj, *a))
+for behind in (Next(), Binds(), staticmethod(lambda *a, **k: seen.append(a))):
+    Mixin = type("Mixin", (torch.nn.Module,), {"__call__": behind})
+    for m in modules():
+        sub = type("Sub", (type(m), Mixin), {})
+        s = sub(128, 64) if hasattr(m, "in_features") else sub()
+        seen.clear()
+        s(5)
+        assert seen == [(s, 5)] if isinstance(behind, Binds) else seen == [(5,)], (type(m), behind)
+""",
+    "calls through the class": """
+import inspect
+for m in modules():
+    cls = type(m)
+    for bad in ((), (5,)):
+        try:
+            cls.__call__(*bad)
+        except (TypeError, AttributeError):
+            pass
+        else:
+            raise AssertionError(bad)
+    other = torch.nn.Identity()
+    assert cls.__call__(other, 3) == 3 and cls.__call__(other, input=4) == 4
+    assert str(inspect.signature(cls.__call__)) == "(self, *args, **kwargs)" and str(inspect.signature(m)) == "(*args, **kwargs)"
+    assert cls.__call__.__name__ in ("__call__", "_wrapped_call_impl")
+""",
+}
+
+
+@pytest.mark.parametrize("first", (True, False), ids=("before the first call", "after it"))
+@pytest.mark.parametrize("what", METHOD_ORDER)
+def test_the_next_call_in_the_method_order(what, first):
+    loaded = "" if first else "from duqlinear4bitcuda_amd import _lib\nhost = _lib.host()\n"
+    run(f"first = {first}\n" + loaded + METHOD_ORDER[what])
