@@ -512,6 +512,26 @@ PyObject *m_linear8(PyObject *, PyObject *const *a, Py_ssize_t n)
     return linear8(a, PyLong_AsLongLong(a[8]), &st);
 }
 
+// References of one's own to what was read from a module: while the interpreter lock is given up, or a finalizer runs,
+// other code may put something else there, and a tensor that nobody else holds goes back to the allocator before the launch
+// that was given its address is queued.
+template <size_t N>
+struct Held {
+    PyObject *o[N];
+    explicit Held(PyObject *const (&from)[N])
+    {
+        for (size_t i = 0; i < N; ++i) {
+            o[i] = from[i];
+            Py_INCREF(o[i]);
+        }
+    }
+    ~Held()
+    {
+        for (PyObject *p : o) Py_DECREF(p);
+    }
+    Held(const Held &) = delete;
+};
+
 // ---- calls of modules ----------------------------------------------------------------------------------------
 // `__call__` of the framework's module classes: what torch.nn.Module.__call__ and the class's forward do in the plain
 // case (no hooks, no compiled or replaced forward, no other __call__ or _call_impl on the way, plain tensors, buffers as
@@ -697,8 +717,9 @@ PyObject *call_eight_bit(PyObject *self, PyObject *dict, PyObject *x)
     }
     PyObject *s = get(buffers, n.weight_scales), *z = get(buffers, n.weight_zeros), *bias = get(buffers, n.bias);
     if (!s || !z) return none();
-    PyObject *a[8] = {x, Py_None, Py_None, w, wt, s, z, bias ? bias : Py_None};
-    return linear8(a, pw->size(0), nullptr);
+    const int64_t N = pw->size(0);
+    const Held<8> a({x, Py_None, Py_None, w, wt, s, z, bias ? bias : Py_None});
+    return linear8(a.o, N, nullptr);
 }
 
 // A product of activations: both quantizers of the module in their plain form, operands of one batch.

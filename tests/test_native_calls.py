@@ -102,3 +102,40 @@ def test_tensors_without_memory_of_their_own(dev):
             torch.func.vmap(lambda v: (f(v), v)[1])(x)
         with pytest.raises(refused):
             f(x[0].to_sparse())
+
+
+def test_eight_bit_call_holds_its_tensors(dev):
+    """What the layer's buffers held when a call was made lives until the library has returned, whoever replaces it meanwhile:
+    looked at from inside the call, at the status of a copy of the weight that the library refuses unlaunched (misaligned)."""
+    import weakref
+
+    from duqlinear4bitcuda_amd import _lib, nn as qnn
+    from duqlinear4bitcuda_amd.tools.tensor_utils import PackedQuantizedTensor
+    K, N = 256, 96
+    layer = qnn.LinearQuant8bitASQ.from_linear(torch.nn.Linear(K, N)).to(dev)
+    x = torch.randn(8, K, device=dev)
+    want = layer(x)
+    copy = layer._buffers["weight_tiled"]
+    layer._buffers["weight_tiled"] = torch.empty(copy.numel() + 1, dtype=copy.dtype, device=dev)[1:]
+    names = ("weight_tiled", "weight_scales", "weight_zeros", "bias")
+    saved = {n: layer._buffers[n].clone() for n in names[1:]}
+    there = []
+
+    class Refused(Exception):
+        pass
+
+    def status(code, name):
+        refs = [weakref.ref(layer._buffers.pop(n)) for n in names]
+        there.extend(r() is not None for r in refs)
+        raise Refused(name)
+
+    host = _lib.host()
+    host.setup(PackedQuantizedTensor, status)
+    try:
+        with pytest.raises(Refused, match="quantize_linear8bit_forward"):
+            layer(x)
+    finally:
+        host.setup(PackedQuantizedTensor, _lib.check)
+    assert there == [True] * 4
+    layer._buffers.update(saved, weight_tiled=copy)
+    assert torch.equal(layer(x), want)
