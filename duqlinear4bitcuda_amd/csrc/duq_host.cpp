@@ -79,6 +79,26 @@ PyObject *entry(PyObject *self, PyObject *const *a, Py_ssize_t n)
     return plain_case([&] { return F(self, a, n); });
 }
 
+// References of one's own to what was read from a module: while the interpreter lock is given up, or a finalizer runs,
+// other code may put something else there, and a tensor that nobody else holds goes back to the allocator before the launch
+// that was given its address is queued.
+template <size_t N>
+struct Held {
+    PyObject *o[N];
+    explicit Held(PyObject *const (&from)[N])
+    {
+        for (size_t i = 0; i < N; ++i) {
+            o[i] = from[i];
+            Py_INCREF(o[i]);
+        }
+    }
+    ~Held()
+    {
+        for (PyObject *p : o) Py_DECREF(p);
+    }
+    Held(const Held &) = delete;
+};
+
 int current_device()
 {
     int d = -1;
@@ -304,6 +324,7 @@ PyObject *m_defer(PyObject *, PyObject *const *a, Py_ssize_t n)
         return none();
     if (a[2] != Py_False && cols % 128 == 0 && (!PyLong_Check(a[3]) || numel >= PyLong_AsLongLong(a[3]) * cols)) return none();
     PyTypeObject *type = reinterpret_cast<PyTypeObject *>(g_packed);
+    const Held<3> h({a[0], a[4], a[5]});   // (the allocation may run the garbage collector)
     PyObject *p = type->tp_alloc(type, 0);
     if (!p) return nullptr;
     for (Slot s : {kQ, kS, kZeros, kRowsum, kShadow}) slot(p, s) = none();
@@ -311,10 +332,10 @@ PyObject *m_defer(PyObject *, PyObject *const *a, Py_ssize_t n)
         Py_INCREF(v);
         slot(p, s) = v;
     };
-    put(kSrc, a[0]);
+    put(kSrc, h.o[0]);
     slot(p, kVersion) = PyLong_FromLong(static_cast<long>(x->_version()));
-    put(kClip, a[4]);
-    put(kQmax, a[5]);
+    put(kClip, h.o[1]);
+    put(kQmax, h.o[2]);
     return p;
 }
 
@@ -511,26 +532,6 @@ PyObject *m_linear8(PyObject *, PyObject *const *a, Py_ssize_t n)
     const duq_stream_t st = stream_of(a[9]);
     return linear8(a, PyLong_AsLongLong(a[8]), &st);
 }
-
-// References of one's own to what was read from a module: while the interpreter lock is given up, or a finalizer runs,
-// other code may put something else there, and a tensor that nobody else holds goes back to the allocator before the launch
-// that was given its address is queued.
-template <size_t N>
-struct Held {
-    PyObject *o[N];
-    explicit Held(PyObject *const (&from)[N])
-    {
-        for (size_t i = 0; i < N; ++i) {
-            o[i] = from[i];
-            Py_INCREF(o[i]);
-        }
-    }
-    ~Held()
-    {
-        for (PyObject *p : o) Py_DECREF(p);
-    }
-    Held(const Held &) = delete;
-};
 
 // ---- calls of modules ----------------------------------------------------------------------------------------
 // `__call__` of the framework's module classes: what torch.nn.Module.__call__ and the class's forward do in the plain

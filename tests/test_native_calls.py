@@ -139,3 +139,31 @@ def test_eight_bit_call_holds_its_tensors(dev):
     assert there == [True] * 4
     layer._buffers.update(saved, weight_tiled=copy)
     assert torch.equal(layer(x), want)
+
+
+def test_quantizer_settings_replaced_by_a_finalizer(dev):
+    """The object that hands the rows on is allocated with the settings in hand; the garbage collector may run there."""
+    import gc
+
+    from duqlinear4bitcuda_amd import nn as qnn
+    q = qnn.SymQuantizer(float("0.75"))
+    x = torch.randn(2, 256, device=dev).half()
+    q(x)
+    there = []
+
+    def replaced(phase, info):
+        q.input_clip_ratio = float("0.5")
+        there.append([float(i) for i in range(1000)])   # (what was freed is in use again)
+
+    before = gc.get_threshold()
+    gc.callbacks.append(replaced)
+    gc.set_threshold(1)
+    try:
+        for _ in range(20):
+            q.input_clip_ratio = float("0.75")
+            p = q(x)
+            assert p._clip in (0.5, 0.75)
+    finally:
+        gc.set_threshold(*before)
+        gc.callbacks.remove(replaced)
+    assert there
