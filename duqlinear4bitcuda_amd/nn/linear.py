@@ -199,14 +199,17 @@ class _Linear4bitBase(torch.nn.Module):
         nibbles; not part of the state_dict; rebuilt when ``weight`` changes).  Results are bit-identical;
         large inputs run 20-25 % faster.  Needs out_features % 16 == 0 and in_features % 128 == 0."""
         assert self.weight.is_cuda, "the shadow is built on the GPU: move the layer there first"
+        assert not self.weight.is_inference(), "the weight was made in torch.inference_mode() and counts no versions: a change " \
+            "of it could not be told; build or move the layer outside"
         assert self.out_features % 16 == 0 and self.in_features % 128 == 0, \
             "the 6-bit float path needs out_features % 16 == 0 and in_features % 128 == 0"
-        self.register_buffer("weight_shadow", tensor_utils.weight_shadow(self.weight), persistent=False)
+        with torch.inference_mode(False):
+            self.register_buffer("weight_shadow", tensor_utils.weight_shadow(self.weight), persistent=False)
         self._shadow_key = (self.weight._version, self.weight.data_ptr())
         return self
 
     def _fp6_ready(self):
-        if self._buffers.get("weight_shadow") is None:
+        if self._buffers.get("weight_shadow") is None or self.weight.is_inference():
             return False
         if self._shadow_key != (self.weight._version, self.weight.data_ptr()) or \
                 self.weight_shadow.device != self.weight.device:
@@ -648,14 +651,19 @@ class LinearQuant8bitASQ(torch.nn.Module):
     fused = True
     # the fused forward reads a copy of ``weight`` arranged for the MFMA operand layout (as many bytes again; not
     # part of the state_dict; rebuilt when ``weight`` changes).  tiled = False reads ``weight`` itself: same bits,
-    # about half the speed on large inputs
+    # about half the speed on large inputs; so does a layer whose weight was made in torch.inference_mode(): such a
+    # tensor counts no versions, and a copy could not follow its changes
     tiled = True
     _tiled_key = None
 
     def _tiled_weight(self):
+        """The copy of ``weight`` for the fused forward, None for a layer that reads ``weight`` itself."""
+        if not self.tiled or self.weight.is_inference():
+            return None
         key = (self.weight._version, self.weight.data_ptr(), self.weight.device)
         if self._tiled_key != key or self._buffers.get("weight_tiled") is None:
-            self.register_buffer("weight_tiled", tensor_utils.weight_tile_8bit(self.weight), persistent=False)
+            with torch.inference_mode(False):
+                self.register_buffer("weight_tiled", tensor_utils.weight_tile_8bit(self.weight), persistent=False)
             self._tiled_key = key
         return self.weight_tiled
 
@@ -684,8 +692,8 @@ class LinearQuant8bitASQ(torch.nn.Module):
                     and x.shape[-1] == self.in_features and self.in_features % 32 == 0 and x.data_ptr() % 16 == 0 \
                     and 0 < x.numel() <= self.one_call_rows * self.in_features and type(self.quantizer) is AsymQuantizer8bit \
                     and self.quantizer.fused:
-                return _ops.quantize_linear8bit_forward(x, self.weight, self._tiled_weight() if self.tiled else None,
-                                                        self.weight_scales, self.weight_zeros, self.bias)
+                return _ops.quantize_linear8bit_forward(x, self.weight, self._tiled_weight(), self.weight_scales,
+                                                        self.weight_zeros, self.bias)
             x = self.quantizer(x)
         assert type(x) == tensor_utils.PackedQuantizedTensor, \
             "Input should be quantized tensor, or require_quantizer should be passed as initial argument"
@@ -693,8 +701,9 @@ class LinearQuant8bitASQ(torch.nn.Module):
         rows = xq.numel() // xq.shape[-1] if xq.shape[-1] else 0
         # up to four rows (two for rows longer than 4096 elements) run a kernel that reads `weight` itself
         few_rows = rows <= 4 and self.in_features <= (8192 if rows <= 2 else 4096)
-        if self.fused and self.tiled and not few_rows:
-            return tensor_utils.linear8bit_forward(xq, scales_x, zeros_x, self._tiled_weight(), self.weight_scales,
+        copy = self._tiled_weight() if self.fused and not few_rows else None
+        if copy is not None:
+            return tensor_utils.linear8bit_forward(xq, scales_x, zeros_x, copy, self.weight_scales,
                                                    self.weight_zeros, self.bias, tiled_rows=self.out_features)
         if self.fused:
             return tensor_utils.linear8bit_forward(xq, scales_x, zeros_x, self.weight, self.weight_scales,

@@ -35,7 +35,9 @@ class SymQuantizer(torch.nn.Module):
     # quantizer + GEMM + dequant are ONE launch; above, the quantizer launch and the GEMM launch of one call: at
     # these sizes a step costs more on the host than on the GPU, and a call less is most of it), and anything
     # else that reads quantized_x / scales_x triggers this quantizer's launch then, with the same bits.  Not for
-    # inputs this quantizer is set to write the 6-bit float shadow for.  0 switches that off.
+    # inputs this quantizer is set to write the 6-bit float shadow for, and not for tensors made in
+    # torch.inference_mode(): these count no versions, so that a change between the quantizer and the layer could not
+    # be told.  0 switches that off.
     defer_rows = 1024
 
     def __init__(self, input_clip_ratio=1.0, qmax: int = 6, shadow=False, shadow_min_rows: int = 96):
@@ -57,7 +59,7 @@ class SymQuantizer(torch.nn.Module):
             x = x.contiguous()
         cols = x.shape[-1]
         if shadow is None and self.defer_rows and cols % 64 == 0 and 0 < x.numel() <= self.defer_rows * cols and \
-                x.is_cuda and x.dtype is torch.float16 and x.data_ptr() % 16 == 0 and \
+                x.is_cuda and x.dtype is torch.float16 and x.data_ptr() % 16 == 0 and not x.is_inference() and \
                 not (self.shadow and x.numel() >= self.shadow_min_rows * cols and cols % 128 == 0):
             return tensor_utils.PackedQuantizedTensor.deferred(x, self.input_clip_ratio, self.qmax)
         shadow = _shadow_choice(self, x, shadow)

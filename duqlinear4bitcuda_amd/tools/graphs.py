@@ -26,7 +26,12 @@ class GraphedForward:
         if not example.is_cuda:
             raise RuntimeError("GraphedForward: the example input must be on a GPU")
         self.module = module
-        self.input = example.detach().clone()
+        with torch.inference_mode(False):   # (static tensors that are written to in either mode, and count versions)
+            self._record(example, warmup)
+
+    def _record(self, example, warmup):
+        module = self.module
+        self.input = example.clone().detach()
         side = torch.cuda.Stream(device=example.device)
         side.wait_stream(torch.cuda.current_stream(example.device))
         with torch.cuda.stream(side), torch.no_grad():

@@ -36,8 +36,8 @@ class PackedQuantizedTensor:
 
     @classmethod
     def deferred(cls, x: torch.Tensor, clip: float, qmax: int):
-        """The symmetric quantization of ``x`` (contiguous binary16 [..., K], K % 32 == 0, 16-byte aligned), not
-        yet computed."""
+        """The symmetric quantization of ``x`` (contiguous binary16 [..., K], K % 32 == 0, 16-byte aligned, no inference
+        tensor), not yet computed."""
         self = cls.__new__(cls)
         self._q = self._s = self.zeros_x = self.rowsum_x = self.shadow_x = None
         self._src = x
