@@ -40,8 +40,8 @@ _own_launch = _launch   # (a tracer may replace _launch to see every call: no ca
 
 
 def _host_for(entry: str):
-    """The native host module (csrc/duq_host.cpp) for calls that end in that entry point, or None where the function
-    on the loaded library was replaced by a Python one (a tracer's): the call then goes through that."""
+    """The native host module (csrc/duq_host.cpp) for calls that end in that entry point, or None where there is none and
+    where the function on the loaded library was replaced by a Python one (a tracer's): the call then goes through that."""
     lib = _lib.load()
     return _lib.host() if type(getattr(lib, entry)) is lib._FuncPtr else None
 
@@ -661,10 +661,11 @@ class FusedDecode:
         """Make ``native``, the same prepared call in native code (``FusedCall`` of csrc/duq_host.cpp: take() and
         take_rows() of a module), for a module whose buffers ``names`` (the weight first) are the tensors this object
         was made of, given as (name, tensor or None) pairs.  It answers None when the module's buffers have changed
-        and for every input that is not the plain case."""
-        if type(self._fn) is self._lib._FuncPtr:
+        and for every input that is not the plain case.  Without the native module ``native`` stays None."""
+        host = _lib.host() if type(self._fn) is self._lib._FuncPtr else None
+        if host is not None:
             p = self._ptrs
-            self.native = _lib.host().FusedCall(
+            self.native = host.FusedCall(
                 self.mode, self.N, self.K, self.index, self.max_rows,
                 (self.w_ptr, p["w_scale_1"], p["w_zeros_1"], p["w_scale_2"], p["w_zeros_2"], p["w_rowsum_adj"],
                  p["w_rowsum_adj_2"], p["bias"]), tuple(n for n, _ in names), tuple(t for _, t in names))

@@ -2,13 +2,17 @@
 
 The shared library is built in-tree by ``duqlinear4bitcuda_amd/csrc/Makefile`` (see
 ``duqlinear4bitcuda_amd.build``).  There is no fallback: if the library is missing,
-loading raises and every op of this package fails.
+loading raises and every op of this package fails.  The host side of its calls exists
+twice: as Python code over ctypes, and in native code as ``_duq_host.so``, which is tied
+to one Python and one torch.  Without that module everything runs through the former, with
+the same results and kernels and more host time per call.
 """
 from __future__ import annotations
 
 import ctypes
 import inspect
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libduq_hip.so")
@@ -130,7 +134,7 @@ def load():
     return lib
 
 
-_host = None
+_host = None   # (False: looked for, and not to be had)
 
 
 def _install_calls(native):
@@ -152,18 +156,26 @@ def _install_calls(native):
 
 
 def host():
-    """The native module of the host side (``csrc/duq_host.cpp``, built beside the library), imported once."""
+    """The native module of the host side (``csrc/duq_host.cpp``, built beside the library), imported once; None, with a
+    warning the first time, where it is missing or was built for another Python or torch: the callers' Python code does
+    the same."""
     global _host
     if _host is None:
         load()
-        if not os.path.exists(HOST_PATH):
-            raise ImportError(f"{HOST_PATH} is missing: build it with `python -m duqlinear4bitcuda_amd.build`")
-        from . import _duq_host
+        try:
+            if not os.path.exists(HOST_PATH):
+                raise ImportError(f"{HOST_PATH} is missing")
+            from . import _duq_host
+        except ImportError as e:
+            _host = False
+            warnings.warn(f"{e}: calls take some microseconds more of host time each; build it with "
+                          "`python -m duqlinear4bitcuda_amd.build`", RuntimeWarning, stacklevel=3)
+            return None
         from .tools.tensor_utils import PackedQuantizedTensor
         _duq_host.setup(PackedQuantizedTensor, check)
         _install_calls(_duq_host)
         _host = _duq_host
-    return _host
+    return _host or None
 
 
 def check(status: int, what: str):

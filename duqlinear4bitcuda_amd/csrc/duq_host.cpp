@@ -16,7 +16,10 @@
 #include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <structmember.h>
+#include <torch/version.h>
 
+#include <cstdio>
+#include <cstring>
 #include <vector>
 
 #include "../../include/duq_hip.h"
@@ -977,8 +980,28 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_duq_host", "host side of the op
 
 }  // namespace
 
+// Whether the process is of the Python and the torch that this file was compiled with: it looks into objects of both.
+static bool built_for_this_process()
+{
+    int major = 0, minor = 0;
+    if (std::sscanf(Py_GetVersion(), "%d.%d", &major, &minor) != 2 || major != PY_MAJOR_VERSION || minor != PY_MINOR_VERSION) {
+        PyErr_Format(PyExc_ImportError, "_duq_host was built for Python %d.%d", PY_MAJOR_VERSION, PY_MINOR_VERSION);
+        return false;
+    }
+    PyObject *torch = PyImport_ImportModule("torch");
+    PyObject *version = torch ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+    const char *v = version ? PyUnicode_AsUTF8(version) : nullptr;
+    const size_t len = std::strlen(TORCH_VERSION);
+    const bool same = v && !std::strncmp(v, TORCH_VERSION, len) && (v[len] == 0 || v[len] == '+');   // (2.10.0+rocm7.0)
+    if (v && !same) PyErr_Format(PyExc_ImportError, "_duq_host was built for torch %s, this is %s", TORCH_VERSION, v);
+    Py_XDECREF(version);
+    Py_XDECREF(torch);
+    return same;
+}
+
 PyMODINIT_FUNC PyInit__duq_host(void)
 {
+    if (!built_for_this_process()) return nullptr;
     g_fused_type.tp_name = "_duq_host.FusedCall";
     g_fused_type.tp_basicsize = sizeof(FusedCall);
     g_fused_type.tp_flags = Py_TPFLAGS_DEFAULT;

@@ -51,8 +51,9 @@ class SymQuantizer(torch.nn.Module):
         self.shadow_min_rows = shadow_min_rows
 
     def forward(self, x, shadow=None) -> tensor_utils.PackedQuantizedTensor:
-        if shadow is None:   # the rule below in native code; None: not a plain case of it
-            p = _lib.host().defer(x, self.defer_rows, self.shadow, self.shadow_min_rows, self.input_clip_ratio, self.qmax)
+        host = _lib.host() if shadow is None else None
+        if host is not None:   # the rule below in native code; None: not a plain case of it
+            p = host.defer(x, self.defer_rows, self.shadow, self.shadow_min_rows, self.input_clip_ratio, self.qmax)
             if p is not None:
                 return p
         if not x.is_contiguous():

@@ -58,3 +58,52 @@ def test_native_and_python_host_code_give_the_same_bits(dev, monkeypatch, rows):
     assert len(calls) >= len(python) and len(python) == len(native)
     for p, n in zip(python, native):
         assert p.dtype == n.dtype and p.shape == n.shape and torch.equal(p, n)
+
+
+BROKEN = {
+    "missing": "_lib.HOST_PATH = '/nonexistent/_duq_host.so'",
+    "another torch": "torch.__version__ = torch.torch_version.TorchVersion('2.99.0+x')",
+}
+
+
+@pytest.mark.parametrize("what", BROKEN)
+def test_the_package_runs_without_the_native_module(what):
+    """Without it the calls reach the Python code behind them (here: its refusal of tensors on the CPU), after one warning."""
+    import os
+    import subprocess
+    import sys
+    code = f"""
+import warnings, torch
+from duqlinear4bitcuda_amd import _HIP, _lib, nn as qnn
+{BROKEN[what]}
+x = torch.zeros(2, 128, dtype=torch.float16)
+mods = [qnn.SymQuantizer(), qnn.Linear4bitASQ(128, 64), qnn.SymQuantMatMul(), qnn.AsymQuantMatMul()]
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    for m in mods:
+        try:
+            m(x, x) if hasattr(m, "quantizer_B") else m(x)
+        except RuntimeError as e:
+            assert "to be on a GPU device" in str(e), e
+        else:
+            raise AssertionError(m)
+seen = [w for w in seen if "_duq_host" in str(w.message)]
+assert len(seen) == 1 and seen[0].category is RuntimeWarning, seen
+assert _lib.host() is None and _HIP._host_for("duq_linear4bit_forward") is None
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.gpu
+def test_prepared_calls_without_the_native_module(dev, monkeypatch):
+    from duqlinear4bitcuda_amd import _lib
+    from duqlinear4bitcuda_amd import nn as qnn
+    lin = torch.nn.Linear(256, 96).half().to(dev).requires_grad_(False)
+    x = torch.randn(5, 256, device=dev).half()
+    want = qnn.Linear4bitASQ.from_linear(lin).to(dev)(x)
+    monkeypatch.setattr(_lib, "host", lambda: None)
+    layer = qnn.Linear4bitASQ.from_linear(lin).to(dev)
+    for _ in range(2):
+        assert torch.equal(layer(x), want) and layer._decode.native is None
