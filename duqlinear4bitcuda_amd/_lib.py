@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import inspect
 import os
+import threading
 import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -102,6 +103,7 @@ class FusedLayer(ctypes.Structure):
 
 
 _lib = None
+_loading = threading.RLock()   # (first calls may come from several threads)
 
 
 class DuqError(RuntimeError):
@@ -111,9 +113,14 @@ class DuqError(RuntimeError):
 
 def load():
     """Load the shared library once and attach prototypes."""
-    global _lib
     if _lib is not None:
         return _lib
+    with _loading:
+        return _lib if _lib is not None else _load()
+
+
+def _load():
+    global _lib
     if not os.path.exists(LIB_PATH):
         raise ImportError(
             f"{LIB_PATH} is missing: build it with `python -m duqlinear4bitcuda_amd.build` "
@@ -159,23 +166,29 @@ def host():
     """The native module of the host side (``csrc/duq_host.cpp``, built beside the library), imported once; None, with a
     warning the first time, where it is missing or was built for another Python or torch: the callers' Python code does
     the same."""
-    global _host
     if _host is None:
-        load()
-        try:
-            if not os.path.exists(HOST_PATH):
-                raise ImportError(f"{HOST_PATH} is missing")
-            from . import _duq_host
-        except ImportError as e:
-            _host = False
-            warnings.warn(f"{e}: calls take some microseconds more of host time each; build it with "
-                          "`python -m duqlinear4bitcuda_amd.build`", RuntimeWarning, stacklevel=3)
-            return None
-        from .tools.tensor_utils import PackedQuantizedTensor
-        _duq_host.setup(PackedQuantizedTensor, check)
-        _install_calls(_duq_host)
-        _host = _duq_host
+        with _loading:
+            if _host is None:
+                _load_host()
     return _host or None
+
+
+def _load_host():
+    global _host
+    load()
+    try:
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(f"{HOST_PATH} is missing")
+        from . import _duq_host
+    except ImportError as e:
+        _host = False
+        warnings.warn(f"{e}: calls take some microseconds more of host time each; build it with "
+                      "`python -m duqlinear4bitcuda_amd.build`", RuntimeWarning, stacklevel=4)
+        return
+    from .tools.tensor_utils import PackedQuantizedTensor
+    _duq_host.setup(PackedQuantizedTensor, check)
+    _install_calls(_duq_host)
+    _host = _duq_host
 
 
 def check(status: int, what: str):

@@ -107,3 +107,31 @@ def test_prepared_calls_without_the_native_module(dev, monkeypatch):
     layer = qnn.Linear4bitASQ.from_linear(lin).to(dev)
     for _ in range(2):
         assert torch.equal(layer(x), want) and layer._decode.native is None
+
+
+def test_first_calls_from_several_threads():
+    """The library and the native module are loaded once, whoever comes first."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import sys, threading
+sys.setswitchinterval(1e-6)
+from duqlinear4bitcuda_amd import _lib, nn
+start, got, errors = threading.Barrier(8), [], []
+def first():
+    start.wait()
+    try:
+        got.append((_lib.host(), _lib.load()))
+    except BaseException as e:
+        errors.append(e)
+threads = [threading.Thread(target=first) for _ in range(8)]
+[t.start() for t in threads]
+[t.join() for t in threads]
+assert not errors, errors
+assert len(got) == 8 and len({id(h) for h, _ in got}) == 1 and len({id(lib) for _, lib in got}) == 1
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    for _ in range(3):
+        r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
