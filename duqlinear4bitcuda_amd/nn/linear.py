@@ -138,6 +138,13 @@ class _Linear4bitBase(torch.nn.Module):
     _decode = None
     _decode_held = ()
 
+    def __getstate__(self):
+        """A copy or a saved file of the layer goes without its prepared call, which holds addresses of this process."""
+        state = self.__dict__.copy()
+        for name in ("_decode", "_decode_held"):
+            state.pop(name, None)
+        return state
+
     def _decode_call(self):
         """The layer's prepared one-launch call (``_HIP.FusedDecode``), rebuilt when a buffer was replaced (moved,
         cast, reloaded into a new tensor); None for a layer that has none or is not on a GPU."""

@@ -135,3 +135,34 @@ assert len(got) == 8 and len({id(h) for h, _ in got}) == 1 and len({id(lib) for 
     for _ in range(3):
         r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
         assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("called", [False, pytest.param(True, marks=pytest.mark.gpu)])
+def test_a_layer_with_a_prepared_call_is_copied_and_saved(called):
+    """The prepared call holds addresses of this process and stays behind: a copy prepares its own."""
+    import copy
+    import io
+
+    from duqlinear4bitcuda_amd import _lib
+    from duqlinear4bitcuda_amd import nn as qnn
+    lin = torch.nn.Linear(256, 96).half().requires_grad_(False)
+    sq = qnn.Linear4bitSQ.from_float(lin, lin.weight.abs().amax(1, keepdim=True) / 7)
+    for layer, model in ((sq, torch.nn.Sequential(qnn.SymQuantizer(), sq)), (a := qnn.Linear4bitASQ.from_linear(lin), a)):
+        if called:
+            model.to("cuda:0")
+            x = torch.randn(3, 256, device="cuda:0").half()
+            want = model(x)
+            assert layer._decode is not None
+        else:
+            layer._decode = _lib.load()
+        file = io.BytesIO()
+        torch.save(model, file)
+        file.seek(0)
+        for other in (copy.deepcopy(model), torch.load(file, weights_only=False)):
+            new = other[1] if isinstance(other, torch.nn.Sequential) else other
+            assert new._decode is None and layer._decode is not None
+            assert torch.equal(new.weight, layer.weight) and new.weight.data_ptr() != layer.weight.data_ptr()
+            if called:
+                assert torch.equal(other(x), want)
+                new.weight.zero_()
+                assert not torch.equal(other(x), want) and torch.equal(model(x), want)
