@@ -610,11 +610,10 @@ class FusedDecode:
     modes and ``duq_quantize_linear4bit_forward_asym`` for the asymmetric and row-sum modes), checked once and kept
     as a ``duq_fused_layer`` struct for ``duq_quantize_linear4bit_forward_layer``: a decode step of a module then
     costs one ``torch.empty`` (two for the shapes of two launches: the staging buffer) and one foreign call with seven
-    arguments.  The tensors are held (``tensors``) so that
-    a caller can tell when the layer's buffers were replaced; a change of their contents in place needs no new
-    object."""
+    arguments.  The tensors are held, for a module under the names of its buffers (``prepare_for``), so that it can tell
+    when they were replaced (``holds``); a change of their contents in place needs no new object."""
 
-    __slots__ = ("mode", "N", "K", "device", "index", "tensors", "w_ptr", "_fn", "_ptrs", "_structs", "_one", "_lib", "native")
+    __slots__ = ("mode", "N", "K", "device", "index", "tensors", "w_ptr", "_fn", "_ptrs", "_structs", "_one", "_lib", "held", "native")
 
     def __init__(self, mode, w, w_scale_1, w_zeros_1=None, w_scale_2=None, w_zeros_2=None, w_rowsum_adj=None,
                  w_rowsum_adj_2=None, bias=None):
@@ -655,21 +654,31 @@ class FusedDecode:
         self._ptrs = ptrs
         self._structs = {}
         self._one = {}
-        self.native = None
+        self.held, self.native = (), None
 
-    def prepare_native(self, names):
-        """Make ``native``, the same prepared call in native code (``FusedCall`` of csrc/duq_host.cpp: take() and
-        take_rows() of a module), for a module whose buffers ``names`` (the weight first) are the tensors this object
-        was made of, given as (name, tensor or None) pairs.  It answers None when the module's buffers have changed
-        and for every input that is not the plain case.  Without the native module ``native`` stays None."""
+    def prepare_for(self, names):
+        """For a module whose buffers ``names`` (the weight first) are the tensors this object was made of, given as
+        (name, tensor or None) pairs: keep them for ``holds``, and make ``native``, the same prepared call in native code
+        (``FusedCall`` of csrc/duq_host.cpp: take() and take_rows() of a module).  It answers None when the module's
+        buffers have changed and for every input that is not the plain case.  Without the native module ``native`` stays
+        None."""
+        at = {id(t): p for t, p in zip(self.tensors, (self.w_ptr, *self._ptrs.values())) if t is not None}
+        self.held = tuple((n, t, None if t is None else at[id(t)]) for n, t in names)
         host = _lib.host() if type(self._fn) is self._lib._FuncPtr else None
         if host is not None:
             p = self._ptrs
             self.native = host.FusedCall(
                 self.mode, self.N, self.K, self.index, self.max_rows,
                 (self.w_ptr, p["w_scale_1"], p["w_zeros_1"], p["w_scale_2"], p["w_zeros_2"], p["w_rowsum_adj"],
-                 p["w_rowsum_adj_2"], p["bias"]), tuple(n for n, _ in names), tuple(t for _, t in names))
+                 p["w_rowsum_adj_2"], p["bias"]), *zip(*self.held))
         return self
+
+    def holds(self, buffers) -> bool:
+        """Whether a module's buffers are still the tensors this object was made of, in the memory they had then."""
+        for name, t, ptr in self.held:
+            if buffers.get(name) is not t or (t is not None and t.data_ptr() != ptr):
+                return False
+        return True
 
     def _layer(self, clip, qmax):
         key = (clip, qmax)

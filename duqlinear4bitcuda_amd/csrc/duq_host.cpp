@@ -173,6 +173,7 @@ struct FusedCall {
     int dev;
     int64_t max_rows;
     PyObject *names, *tensors;        // tuples: the buffers' names in the module and the tensors the call was made of
+    std::vector<const void *> *at;    // and where these were then
     std::vector<int64_t> *staging;    // bytes the library stages at M rows, -1: not asked yet
 };
 
@@ -191,15 +192,17 @@ int64_t staging_of(FusedCall *c, int64_t M)
     return b;
 }
 
-// Whether `buffers` (the module's dict) still holds the tensors the call was made of, where it found them.
+// Whether `buffers` (the module's dict) still holds the tensors the call was made of, in the memory they had then (a tensor
+// is given other memory by an assignment to its .data).
 bool still_current(FusedCall *c, PyObject *buffers)
 {
     const Py_ssize_t n = PyTuple_GET_SIZE(c->names);
     for (Py_ssize_t i = 0; i < n; ++i) {
         PyObject *t = PyDict_GetItemWithError(buffers, PyTuple_GET_ITEM(c->names, i));
         if ((t ? t : Py_None) != PyTuple_GET_ITEM(c->tensors, i)) return false;
+        if (t && t != Py_None && THPVariable_Unpack(t).const_data_ptr() != (*c->at)[static_cast<size_t>(i)]) return false;
     }
-    return THPVariable_Unpack(PyTuple_GET_ITEM(c->tensors, 0)).const_data_ptr() == c->layer.w;
+    return true;
 }
 
 // min_tiles: the module's fp6_min_tiles, negative where the caller does not know it
@@ -262,28 +265,37 @@ PyObject *fused_take_rows(PyObject *self, PyObject *const *a, Py_ssize_t n)
     return guarded([&] { return run_rows(c, a[0], *x, 1.0f, 6, tiles_argument(a, n)); });
 }
 
-// FusedCall(mode, N, K, device index, max_rows, addresses of (w, s1, z1, s2, z2, adj1, adj2, bias), names, tensors)
+// FusedCall(mode, N, K, device index, max_rows, addresses of (w, s1, z1, s2, z2, adj1, adj2, bias), names, tensors[, the
+// address of each tensor, else where they are now])
 PyObject *fused_new(PyTypeObject *type, PyObject *args, PyObject *)
 {
     int mode, dev;
     unsigned N, K;
     long long max_rows;
-    PyObject *addr, *names, *tensors;
-    if (!PyArg_ParseTuple(args, "iIIiLO!O!O!", &mode, &N, &K, &dev, &max_rows, &PyTuple_Type, &addr, &PyTuple_Type, &names,
-                          &PyTuple_Type, &tensors))
+    PyObject *addr, *names, *tensors, *at = nullptr;
+    if (!PyArg_ParseTuple(args, "iIIiLO!O!O!|O!", &mode, &N, &K, &dev, &max_rows, &PyTuple_Type, &addr, &PyTuple_Type, &names,
+                          &PyTuple_Type, &tensors, &PyTuple_Type, &at))
         return nullptr;
     const Py_ssize_t n = PyTuple_GET_SIZE(names);
-    if (PyTuple_GET_SIZE(addr) != 8 || n < 1 || PyTuple_GET_SIZE(tensors) != n || !THPVariable_Check(PyTuple_GET_ITEM(tensors, 0)) ||
-        max_rows < 1 || max_rows > 65536) {
+    bool fits = PyTuple_GET_SIZE(addr) == 8 && n >= 1 && PyTuple_GET_SIZE(tensors) == n && (!at || PyTuple_GET_SIZE(at) == n) &&
+                max_rows >= 1 && max_rows <= 65536;
+    for (Py_ssize_t i = 0; fits && i < n; ++i)
+        fits = THPVariable_Check(PyTuple_GET_ITEM(tensors, i)) || (i > 0 && PyTuple_GET_ITEM(tensors, i) == Py_None);
+    if (!fits) {
         PyErr_SetString(PyExc_ValueError, "FusedCall: eight addresses, and a tensor (the weight first) for every name");
         return nullptr;
     }
     void *p[8];
-    for (int i = 0; i < 8; ++i) {
-        PyObject *o = PyTuple_GET_ITEM(addr, i);
-        p[i] = o == Py_None ? nullptr : PyLong_AsVoidPtr(o);
-        if (PyErr_Occurred()) return nullptr;
+    std::vector<const void *> where(static_cast<size_t>(n));
+    auto address = [](PyObject *o) { return o == Py_None ? nullptr : PyLong_AsVoidPtr(o); };
+    for (Py_ssize_t i = 0; i < 8 && !PyErr_Occurred(); ++i) p[i] = address(PyTuple_GET_ITEM(addr, i));
+    for (Py_ssize_t i = 0; i < n && !PyErr_Occurred(); ++i) {
+        PyObject *t = PyTuple_GET_ITEM(tensors, i);
+        where[static_cast<size_t>(i)] = at             ? address(PyTuple_GET_ITEM(at, i))
+                                        : t == Py_None ? nullptr
+                                                       : THPVariable_Unpack(t).const_data_ptr();
     }
+    if (PyErr_Occurred()) return nullptr;
     FusedCall *c = reinterpret_cast<FusedCall *>(type->tp_alloc(type, 0));
     if (!c) return nullptr;
     c->layer = duq_fused_layer{mode, 1.0f, 6, N, K, static_cast<const uint8_t *>(p[0]), half(p[1]), half(p[2]), half(p[3]),
@@ -294,6 +306,7 @@ PyObject *fused_new(PyTypeObject *type, PyObject *args, PyObject *)
     Py_INCREF(tensors);
     c->names = names;
     c->tensors = tensors;
+    c->at = new std::vector<const void *>(std::move(where));
     c->staging = new std::vector<int64_t>();
     return reinterpret_cast<PyObject *>(c);
 }
@@ -304,6 +317,7 @@ void fused_dealloc(PyObject *self)
     Py_XDECREF(c->names);
     Py_XDECREF(c->tensors);
     delete c->staging;
+    delete c->at;
     Py_TYPE(self)->tp_free(self);
 }
 

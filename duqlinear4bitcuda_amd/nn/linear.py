@@ -136,27 +136,21 @@ class _Linear4bitBase(torch.nn.Module):
     # one-launch form; the weight comes first.
     _decode_spec = None
     _decode = None
-    _decode_held = ()
 
     def __getstate__(self):
         """A copy or a saved file of the layer goes without its prepared call, which holds addresses of this process."""
         state = self.__dict__.copy()
-        for name in ("_decode", "_decode_held"):
-            state.pop(name, None)
+        state.pop("_decode", None)
         return state
 
     def _decode_call(self):
         """The layer's prepared one-launch call (``_HIP.FusedDecode``), rebuilt when a buffer was replaced (moved,
-        cast, reloaded into a new tensor); None for a layer that has none or is not on a GPU."""
+        cast, reloaded into a new tensor) or given other memory (``.data``); None for a layer that has none or is not on
+        a GPU."""
         d = self._decode
         b = self._buffers
-        if d is not None:
-            for name, t in self._decode_held:
-                if b.get(name) is not t:
-                    break
-            else:
-                if d.w_ptr == self._decode_held[0][1].data_ptr():
-                    return d
+        if d is not None and d.holds(b):
+            return d
         spec = self._decode_spec
         if spec is None:
             return None
@@ -164,8 +158,7 @@ class _Linear4bitBase(torch.nn.Module):
         held = tuple((buf, b.get(buf)) for _, buf in names)
         if not held[0][1].is_cuda:
             return None
-        d = self._decode = _ops.FusedDecode(spec[0], **{arg: t for (arg, _), (_, t) in zip(names, held)}).prepare_native(held)
-        self._decode_held = held
+        d = self._decode = _ops.FusedDecode(spec[0], **{arg: t for (arg, _), (_, t) in zip(names, held)}).prepare_for(held)
         return d
 
     def _decode_forward(self, x, clip=1.0, qmax=6, checked=False):

@@ -167,3 +167,27 @@ def test_quantizer_settings_replaced_by_a_finalizer(dev):
         gc.set_threshold(*before)
         gc.callbacks.remove(replaced)
     assert there
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_buffers_given_other_memory(dev, monkeypatch, native):
+    """An assignment to a buffer's .data leaves the tensor and changes its memory: the prepared call must not keep the old."""
+    from duqlinear4bitcuda_amd import _lib, nn as qnn
+    if not native:
+        monkeypatch.setattr(_lib, "host", lambda: None)
+    gen = torch.Generator(device=dev).manual_seed(3)
+    lin = torch.nn.Linear(256, 96, bias=True, device=dev, dtype=torch.float16).requires_grad_(False)
+    x = torch.randn(5, 256, generator=gen, device=dev).half()
+    for cls in (qnn.Linear4bitASQ, qnn.LinearQuant4bitDUASQ, qnn.Linear4bitASQRowSum, qnn.LinearQuant4bitDUASQRowSum):
+        layer, fresh = (cls.from_linear(lin).to(dev) for _ in range(2))
+        layer(x)
+        assert (layer._decode.native is not None) == native
+        for name, buf in layer._buffers.items():
+            before = layer(x)
+            other = torch.flip(buf, (0,)) if name == "weight" else buf + 1
+            buf.data = other.clone()
+            fresh._buffers[name] = other
+            got = layer(x)
+            fresh._decode = None
+            same, changed = torch.equal(got, fresh(x)), not torch.equal(got, before)
+            assert same and changed, (cls, name)
