@@ -25,6 +25,13 @@ _INT4_LEVELS = 2 ** 4
 
 
 _making = threading.local()
+_copying = threading.RLock()   # held where a layer's copy of its weight and the key it goes by are put in place
+
+
+def _weight_key(layer):
+    """What a copy of the layer's weight goes by: the copy is the weight's while this is what it was before it was made."""
+    w = layer.weight
+    return w._version, w.data_ptr(), w.device
 
 
 def _placeholder_weight(shape, dtype):
@@ -203,18 +210,24 @@ class _Linear4bitBase(torch.nn.Module):
             "of it could not be told; build or move the layer outside"
         assert self.out_features % 16 == 0 and self.in_features % 128 == 0, \
             "the 6-bit float path needs out_features % 16 == 0 and in_features % 128 == 0"
-        with torch.inference_mode(False):
-            self.register_buffer("weight_shadow", tensor_utils.weight_shadow(self.weight), persistent=False)
-        self._shadow_key = (self.weight._version, self.weight.data_ptr())
+        with _copying:
+            key = _weight_key(self)
+            with torch.inference_mode(False):
+                self.register_buffer("weight_shadow", tensor_utils.weight_shadow(self.weight), persistent=False)
+            self._shadow_key = key
         return self
 
     def _fp6_ready(self):
         if self._buffers.get("weight_shadow") is None or self.weight.is_inference():
             return False
-        if self._shadow_key != (self.weight._version, self.weight.data_ptr()) or \
-                self.weight_shadow.device != self.weight.device:
-            self.enable_fp6()  # weights were loaded or moved since
+        if self._shadow_stale():   # weights were loaded or moved since
+            with _copying:
+                if self._shadow_stale():
+                    self.enable_fp6()
         return True
+
+    def _shadow_stale(self):
+        return self._shadow_key != _weight_key(self) or self.weight_shadow.device != self.weight.device
 
     def _fp6_wanted(self, rows):
         tiles = -(-rows // 64) * -(-self.out_features // 256)
@@ -660,11 +673,13 @@ class LinearQuant8bitASQ(torch.nn.Module):
         """The copy of ``weight`` for the fused forward, None for a layer that reads ``weight`` itself."""
         if not self.tiled or self.weight.is_inference():
             return None
-        key = (self.weight._version, self.weight.data_ptr(), self.weight.device)
-        if self._tiled_key != key or self._buffers.get("weight_tiled") is None:
-            with torch.inference_mode(False):
-                self.register_buffer("weight_tiled", tensor_utils.weight_tile_8bit(self.weight), persistent=False)
-            self._tiled_key = key
+        if self._tiled_key != _weight_key(self) or self._buffers.get("weight_tiled") is None:
+            with _copying:
+                key = _weight_key(self)
+                if self._tiled_key != key or self._buffers.get("weight_tiled") is None:
+                    with torch.inference_mode(False):
+                        self.register_buffer("weight_tiled", tensor_utils.weight_tile_8bit(self.weight), persistent=False)
+                    self._tiled_key = key
         return self.weight_tiled
 
     def __init__(self, in_features, out_features, bias=False, require_quantizer=True):

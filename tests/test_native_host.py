@@ -166,3 +166,48 @@ def test_a_layer_with_a_prepared_call_is_copied_and_saved(called):
                 assert torch.equal(other(x), want)
                 new.weight.zero_()
                 assert not torch.equal(other(x), want) and torch.equal(model(x), want)
+
+
+@pytest.mark.parametrize("what", ["weight_tiled", "weight_shadow"])
+def test_copies_of_a_weight_made_by_two_threads_at_once(monkeypatch, what):
+    """A thread that is behind with the copy of an older weight must not leave it in the place of the newer one."""
+    import threading
+
+    from duqlinear4bitcuda_amd import nn as qnn
+    from duqlinear4bitcuda_amd.nn import linear
+    monkeypatch.setattr(linear.tensor_utils, "weight_tile_8bit", lambda w: w.clone())
+    monkeypatch.setattr(linear.tensor_utils, "weight_shadow", lambda w: w.clone())
+    if what == "weight_tiled":
+        layer = qnn.LinearQuant8bitASQ(128, 64)
+        make = layer._tiled_weight
+    else:
+        layer = qnn.Linear4bitASQ(128, 64)
+        monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+        layer.enable_fp6()
+        make = layer._fp6_ready
+    layer.weight.fill_(1)
+    real, older_made, newer_put, older_done = layer.register_buffer, threading.Event(), threading.Event(), threading.Event()
+
+    def put(name, t, persistent):
+        if threading.current_thread() is older:
+            older_made.set()
+            newer_put.wait(1)
+        real(name, t, persistent=persistent)
+        if threading.current_thread() is newer:
+            newer_put.set()
+            older_done.wait(1)
+
+    def first():
+        make()
+        older_done.set()
+
+    older, newer = threading.Thread(target=first), threading.Thread(target=make)
+    layer.register_buffer = put
+    older.start()
+    older_made.wait()
+    layer.weight.fill_(2)
+    newer.start()
+    older.join()
+    newer.join()
+    make()
+    assert (layer._buffers[what] == 2).all()
