@@ -34,6 +34,23 @@ def _weight_key(layer):
     return w._version, w.data_ptr(), w.device
 
 
+def _put_copy(layer, name, key_name, make):
+    """Make the layer's copy of its weight (buffer ``name``) and the key it goes by.  Another stream may read the copy as soon
+    as the key is there, and knows nothing of the launch that writes it: it is waited for, once per weight.  While a graph is
+    recorded nothing is written yet: the recording gets a copy without a key, and calls outside of it make their own."""
+    with _copying:
+        key = _weight_key(layer)
+        with torch.inference_mode(False):
+            copy = make(layer.weight)
+        if copy.is_cuda:
+            if torch.cuda.is_current_stream_capturing():
+                key = None
+            else:
+                torch.cuda.current_stream(copy.device).synchronize()
+        layer.register_buffer(name, copy, persistent=False)
+        setattr(layer, key_name, key)
+
+
 def _placeholder_weight(shape, dtype):
     """What a layer holds until weights are put in: small random codes, as in the reference."""
     if getattr(_making, "unfilled", False):
@@ -210,11 +227,7 @@ class _Linear4bitBase(torch.nn.Module):
             "of it could not be told; build or move the layer outside"
         assert self.out_features % 16 == 0 and self.in_features % 128 == 0, \
             "the 6-bit float path needs out_features % 16 == 0 and in_features % 128 == 0"
-        with _copying:
-            key = _weight_key(self)
-            with torch.inference_mode(False):
-                self.register_buffer("weight_shadow", tensor_utils.weight_shadow(self.weight), persistent=False)
-            self._shadow_key = key
+        _put_copy(self, "weight_shadow", "_shadow_key", tensor_utils.weight_shadow)
         return self
 
     def _fp6_ready(self):
@@ -673,14 +686,14 @@ class LinearQuant8bitASQ(torch.nn.Module):
         """The copy of ``weight`` for the fused forward, None for a layer that reads ``weight`` itself."""
         if not self.tiled or self.weight.is_inference():
             return None
-        if self._tiled_key != _weight_key(self) or self._buffers.get("weight_tiled") is None:
+        if self._tiled_stale():
             with _copying:
-                key = _weight_key(self)
-                if self._tiled_key != key or self._buffers.get("weight_tiled") is None:
-                    with torch.inference_mode(False):
-                        self.register_buffer("weight_tiled", tensor_utils.weight_tile_8bit(self.weight), persistent=False)
-                    self._tiled_key = key
+                if self._tiled_stale():
+                    _put_copy(self, "weight_tiled", "_tiled_key", tensor_utils.weight_tile_8bit)
         return self.weight_tiled
+
+    def _tiled_stale(self):
+        return self._tiled_key != _weight_key(self) or self._buffers.get("weight_tiled") is None
 
     def __init__(self, in_features, out_features, bias=False, require_quantizer=True):
         super().__init__()
