@@ -7,9 +7,9 @@ pytestmark = pytest.mark.gpu
 K, N = 4096, 1024
 
 
-def layers(dev):
+def layers(dev, seed=1):
     from duqlinear4bitcuda_amd import nn as qnn
-    gen = torch.Generator(device=dev).manual_seed(1)
+    gen = torch.Generator(device=dev).manual_seed(seed)
     lin = torch.nn.Linear(K, N, bias=False, device=dev, dtype=torch.float16).requires_grad_(False)
     lin.weight.copy_(torch.randn(N, K, generator=gen, device=dev) * 0.02)
     x = torch.randn(128, K, generator=gen, device=dev)
@@ -26,6 +26,12 @@ def test_a_copy_made_on_one_stream_is_read_on_another(dev, k):
     want = layer(x)                                         # without any copy
     layer.fused = fused
     one, other = torch.cuda.Stream(dev), torch.cuda.Stream(dev)
+    for stream in (one, other):                             # (memory for each stream, so that no call has to wait for it,
+        with torch.cuda.stream(stream):                     # with another weight's copy in it)
+            warm, y = layers(dev, 2)[k]
+            warm.weight.mul_(1)
+            warm(y), warm(y), torch.empty(1 << 24, device=dev)
+            del warm, y
     torch.cuda.synchronize()
     with torch.cuda.stream(one):
         torch.cuda._sleep(20_000_000)                       # some ms of work in front of what makes the copy
