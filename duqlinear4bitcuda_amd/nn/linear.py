@@ -34,9 +34,10 @@ def _weight_key(layer):
     return w._version, w.data_ptr(), w.device
 
 
-def _put_copy(layer, name, key_name, make):
+def _put_copy(layer, name, key_name, make, wait):
     """Make the layer's copy of its weight (buffer ``name``) and the key it goes by.  Another stream may read the copy as soon
-    as the key is there, and knows nothing of the launch that writes it: it is waited for, once per weight.  While a graph is
+    as the key is there, and its user knows nothing of the launch that writes a copy made on the way in a forward: that one is
+    waited for (``wait``), once per weight (a first 8-bit call of 8 rows, 4096 x 4096: 62 -> 90 us).  While a graph is
     recorded nothing is written yet: the recording gets a copy without a key, and calls outside of it make their own."""
     with _copying:
         key = _weight_key(layer)
@@ -45,7 +46,7 @@ def _put_copy(layer, name, key_name, make):
         if copy.is_cuda:
             if torch.cuda.is_current_stream_capturing():
                 key = None
-            else:
+            elif wait:
                 torch.cuda.current_stream(copy.device).synchronize()
         layer.register_buffer(name, copy, persistent=False)
         setattr(layer, key_name, key)
@@ -220,15 +221,18 @@ class _Linear4bitBase(torch.nn.Module):
 
     def enable_fp6(self):
         """Build the E3M2 shadow of ``weight`` (3/4 byte per element next to the 1/2 byte of the packed
-        nibbles; not part of the state_dict; rebuilt when ``weight`` changes).  Results are bit-identical;
-        large inputs run 20-25 % faster.  Needs out_features % 16 == 0 and in_features % 128 == 0."""
+        nibbles; not part of the state_dict; rebuilt when ``weight`` changes) on the current stream.  Results are
+        bit-identical; large inputs run 20-25 % faster.  Needs out_features % 16 == 0 and in_features % 128 == 0."""
+        self._build_shadow(wait=False)
+        return self
+
+    def _build_shadow(self, wait):
         assert self.weight.is_cuda, "the shadow is built on the GPU: move the layer there first"
         assert not self.weight.is_inference(), "the weight was made in torch.inference_mode() and counts no versions: a change " \
             "of it could not be told; build or move the layer outside"
         assert self.out_features % 16 == 0 and self.in_features % 128 == 0, \
             "the 6-bit float path needs out_features % 16 == 0 and in_features % 128 == 0"
-        _put_copy(self, "weight_shadow", "_shadow_key", tensor_utils.weight_shadow)
-        return self
+        _put_copy(self, "weight_shadow", "_shadow_key", tensor_utils.weight_shadow, wait)
 
     def _fp6_ready(self):
         if self._buffers.get("weight_shadow") is None or self.weight.is_inference():
@@ -236,7 +240,7 @@ class _Linear4bitBase(torch.nn.Module):
         if self._shadow_stale():   # weights were loaded or moved since
             with _copying:
                 if self._shadow_stale():
-                    self.enable_fp6()
+                    self._build_shadow(wait=True)
         return True
 
     def _shadow_stale(self):
@@ -689,7 +693,7 @@ class LinearQuant8bitASQ(torch.nn.Module):
         if self._tiled_stale():
             with _copying:
                 if self._tiled_stale():
-                    _put_copy(self, "weight_tiled", "_tiled_key", tensor_utils.weight_tile_8bit)
+                    _put_copy(self, "weight_tiled", "_tiled_key", tensor_utils.weight_tile_8bit, True)
         return self.weight_tiled
 
     def _tiled_stale(self):
