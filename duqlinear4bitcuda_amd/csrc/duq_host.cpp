@@ -102,6 +102,14 @@ struct Held {
     Held(const Held &) = delete;
 };
 
+// A Python int, which has no largest value: what does not fit is the nearest that does.
+int64_t whole(PyObject *o)
+{
+    int over = 0;
+    const long long v = PyLong_AsLongLongAndOverflow(o, &over);
+    return over > 0 ? INT64_MAX : over < 0 ? INT64_MIN : v;
+}
+
 int current_device()
 {
     int d = -1;
@@ -238,7 +246,7 @@ PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip,
 
 int64_t tiles_argument(PyObject *const *a, Py_ssize_t n)
 {
-    return n == 3 && PyLong_Check(a[2]) ? PyLong_AsLongLong(a[2]) : -1;
+    return n == 3 && PyLong_Check(a[2]) ? whole(a[2]) : -1;
 }
 
 // take(buffers, packed[, the module's fp6_min_tiles]): the layer's result for a PackedQuantizedTensor that was handed on unquantized
@@ -249,9 +257,9 @@ PyObject *fused_take(PyObject *self, PyObject *const *a, Py_ssize_t n)
     PyObject *src = slot(a[1], kSrc), *version = slot(a[1], kVersion), *clip = slot(a[1], kClip), *qmax = slot(a[1], kQmax);
     if (!src || !version || !clip || !qmax || !PyFloat_Check(clip) || !PyLong_Check(qmax)) return none();
     const Tensor *x = plain(src, ScalarType::Half, c->dev);
-    if (!x || x->is_inference() || static_cast<long>(x->_version()) != PyLong_AsLong(version) || !still_current(c, a[0])) return none();
+    if (!x || x->is_inference() || x->_version() != whole(version) || !still_current(c, a[0])) return none();
     const Tensor held = *x;  // (another thread may quantize the packed tensor, which drops its rows)
-    return guarded([&] { return run_rows(c, a[0], held, static_cast<float>(PyFloat_AS_DOUBLE(clip)), static_cast<int>(PyLong_AsLong(qmax)),
+    return guarded([&] { return run_rows(c, a[0], held, static_cast<float>(PyFloat_AS_DOUBLE(clip)), static_cast<int>(whole(qmax)),
                                          tiles_argument(a, n)); });
 }
 
@@ -337,9 +345,8 @@ PyObject *m_defer(PyObject *, PyObject *const *a, Py_ssize_t n)
     const Tensor *x = plain(a[0], ScalarType::Half, -1);
     if (!x || x->dim() == 0 || x->is_inference() || !PyLong_Check(a[1])) return none();  // (inference tensors count no versions)
     const int64_t cols = x->size(-1), numel = x->numel();
-    if (cols % 64 || numel <= 0 || numel > PyLong_AsLongLong(a[1]) * cols || reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16)
-        return none();
-    if (a[2] != Py_False && cols % 128 == 0 && (!PyLong_Check(a[3]) || numel >= PyLong_AsLongLong(a[3]) * cols)) return none();
+    if (cols % 64 || numel <= 0 || numel / cols > whole(a[1]) || reinterpret_cast<uintptr_t>(x->const_data_ptr()) % 16) return none();
+    if (a[2] != Py_False && cols % 128 == 0 && (!PyLong_Check(a[3]) || numel / cols >= whole(a[3]))) return none();
     PyTypeObject *type = reinterpret_cast<PyTypeObject *>(g_packed);
     const Held<3> h({a[0], a[4], a[5]});   // (the allocation may run the garbage collector)
     PyObject *p = type->tp_alloc(type, 0);
@@ -366,7 +373,7 @@ PyObject *m_quantize_rows(PyObject *, PyObject *const *a, Py_ssize_t n)
     const long kind = PyLong_AsLong(a[1]);
     const bool with_q = a[2] == Py_True, shadow = a[3] == Py_True;
     const float clip = static_cast<float>(PyFloat_AS_DOUBLE(a[4]));
-    const int qmax = static_cast<int>(PyLong_AsLong(a[5]));
+    const int qmax = static_cast<int>(whole(a[5]));
     const duq_stream_t st = stream_of(a[6]);
     return guarded([&]() -> PyObject * {
         const int64_t cols = x->size(-1), rows64 = x->numel() / cols;
@@ -718,15 +725,15 @@ PyObject *call_eight_bit(PyObject *self, PyObject *dict, PyObject *x)
     PyObject *tiled = attr(self, dict, n.tiled), *w = get(buffers, n.weight), *wt = Py_None;
     if (!w || (tiled != Py_True && tiled != Py_False)) return none();
     const Tensor *px = plain(x, ScalarType::Float, -1), *pw = plain(w, ScalarType::Char, -1);
-    if (!px || !pw || pw->dim() != 2 || px->dim() == 0 || px->size(-1) != pw->size(1) || pw->size(1) % 32 ||
-        reinterpret_cast<uintptr_t>(px->const_data_ptr()) % 16 || px->numel() > PyLong_AsLongLong(rows) * pw->size(1) ||
+    if (!px || !pw || pw->dim() != 2 || px->dim() == 0 || px->size(-1) != pw->size(1) || pw->size(1) % 32 || px->numel() == 0 ||
+        reinterpret_cast<uintptr_t>(px->const_data_ptr()) % 16 || px->numel() / pw->size(1) > whole(rows) ||
         px->get_device() != current_device())
         return none();
     if (tiled == Py_True) {  // the copy is the weight's as it is now: version, address, device (the layer's _tiled_weight)
         PyObject *key = get(dict, n._tiled_key);
         wt = get(buffers, n.weight_tiled);
         if (!wt || wt == Py_None || !key || !PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || pw->is_inference() ||
-            PyLong_AsLong(PyTuple_GET_ITEM(key, 0)) != static_cast<long>(pw->_version()) ||
+            whole(PyTuple_GET_ITEM(key, 0)) != pw->_version() ||
             PyLong_AsVoidPtr(PyTuple_GET_ITEM(key, 1)) != pw->const_data_ptr() || !THPVariable_CheckExact(wt) ||
             THPVariable_Unpack(wt).get_device() != pw->get_device()) {
             PyErr_Clear();
@@ -749,7 +756,7 @@ PyObject *call_product(PyObject *self, PyObject *dict, PyObject *pa, PyObject *p
         !library_function(n.duq_quantize_product) || (asym && get(dict, n.transpose_B) != Py_False))
         return none();
     float clip[2] = {1.0f, 1.0f};
-    long qmax[2] = {6, 6};
+    int64_t qmax[2] = {6, 6};
     PyObject *const names[2] = {n.quantizer_A, n.quantizer_B};
     for (int i = 0; i < 2; ++i) {
         PyObject *q = get(modules, names[i]), *qd = q ? dict_of(q) : nullptr;
@@ -760,11 +767,8 @@ PyObject *call_product(PyObject *self, PyObject *dict, PyObject *pa, PyObject *p
             PyObject *c = get(qd, n.input_clip_ratio), *m = get(qd, n.qmax);
             if (!c || !m || !PyFloat_Check(c) || !PyLong_Check(m)) return none();
             clip[i] = static_cast<float>(PyFloat_AS_DOUBLE(c));
-            qmax[i] = PyLong_AsLong(m);
-            if (qmax[i] < 0 || qmax[i] > 7) {
-                PyErr_Clear();
-                return none();
-            }
+            qmax[i] = whole(m);
+            if (qmax[i] < 0 || qmax[i] > 7) return none();
         }
     }
     const Tensor *a = plain(pa, ScalarType::Half, -1);

@@ -191,3 +191,27 @@ def test_buffers_given_other_memory(dev, monkeypatch, native):
             fresh._decode = None
             same, changed = torch.equal(got, fresh(x)), not torch.equal(got, before)
             assert same and changed, (cls, name)
+
+
+@pytest.mark.parametrize("most", [10 ** 30, 2 ** 62, -10 ** 30, 0])
+def test_settings_of_any_size(dev, most):
+    """Row counts that a C integer does not hold, or whose product with the row length it does not, and layers of no columns."""
+    from duqlinear4bitcuda_amd import nn as qnn
+    K, N = 256, 96
+    lin = torch.nn.Linear(K, N).half().to(dev).requires_grad_(False)
+    x = torch.randn(70, K, device=dev).half()
+    sq = torch.nn.Sequential(qnn.SymQuantizer(), qnn.Linear4bitSQ.from_float(lin, lin.weight.abs().amax(1, keepdim=True) / 7).to(dev))
+    asq = qnn.Linear4bitASQ.from_linear(lin).to(dev)
+    l8 = qnn.LinearQuant8bitASQ.from_linear(lin.float()).to(dev)
+    want = [sq(x), asq(x), l8(x.float())]
+    sq[0].defer_rows = most
+    assert (sq[0](x)._src is not None) == (most > 0)
+    asq.enable_fp6().fp6_min_tiles = most
+    l8.one_call_rows = most
+    for _ in range(2):
+        assert all(torch.equal(m(a), w) for m, a, w in zip((sq, asq, l8), (x, x, x.float()), want))
+    sq[0].shadow, sq[0].shadow_min_rows = True, most
+    assert torch.equal(sq(x), want[0])
+    empty = qnn.LinearQuant8bitASQ(0, 8).to(dev)
+    with pytest.raises((RuntimeError, IndexError, ZeroDivisionError)):
+        empty(torch.zeros(3, 0, device=dev))
