@@ -83,6 +83,22 @@ for m in mods:
     call(m)
     assert seen and seen[0] is put
 """,
+    "tracing, hooks of every module, hooks of an instance": """
+plain()
+from duqlinear4bitcuda_amd import _lib
+for m in modules():
+    seen.clear()
+    torch.jit.trace(lambda x: (seen.append(_lib.host().plain_call(m)), x + 1)[1], torch.zeros(2), check_trace=False)
+    assert seen == [False] and _lib.host().plain_call(m)
+    for register in (torch.nn.modules.module.register_module_forward_hook, torch.nn.modules.module.register_module_forward_pre_hook,
+                     torch.nn.modules.module.register_module_full_backward_hook,
+                     torch.nn.modules.module.register_module_full_backward_pre_hook, m.register_forward_hook,
+                     m.register_forward_pre_hook, m.register_full_backward_hook, m.register_full_backward_pre_hook):
+        handle = register(lambda *a: None)
+        assert not _lib.host().plain_call(m), register
+        handle.remove()
+        assert _lib.host().plain_call(m)
+""",
 }
 
 
