@@ -838,7 +838,8 @@ template <int EPI, bool BIAS>
 static void launch_epi(GemmParams &p, hipStream_t stream, uint32_t batch = 1)
 {
     const int kernel = batch > 1 ? kKernelStream : select_gemm_kernel(p.M, p.N, p.K);
-    // (EPI 5, the dual-uniform row-sum epilogue, exists in the stream kernel only: gemm_fuses_dual_rowsum)
+    // (EPI 5, the dual-uniform row-sum epilogue: of the kernels launched here, the stream and prefill kernels have it, and
+    // only their shapes come here with it: gemm_fuses_dual_rowsum)
     if constexpr (EPI != 5) {
     if (kernel == kKernelDot) {
         const uint32_t xstride = ((p.K / 2 + 127) / 128) * 128;

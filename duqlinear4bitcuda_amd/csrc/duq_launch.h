@@ -98,7 +98,9 @@ inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 // each, measured per tile shape (N = 4096, one round, K = 1024 / 4096 / 16384): 64 x 128 6.6 / 11.9 / 33, 128 x 128 8.9 /
 // 17.5 / 55, 128 x 256 12.5 / 30 / 100, 256 x 256 21 / 52.7 / 178 (1.3 of it once per launch); the cheapest wins.  64 x 64 and
 // 96 x 64 tiles (128 rows; 65 rows) 5.9 / 8.7 / 22 and - / 10 / 22.6: in one round only, where they halve the walk over K;
-// two rounds of them are behind (512 x 4096 x 4096 17 against 12.4, 96 x 28672 x 8192 38 against 34.7).  The
+// two rounds of them are behind (512 x 4096 x 4096 17 against 12.4, 96 x 28672 x 8192 38 against 34.7).  96 x 64 against the
+// next best on 65..96 rows, 8200..16384 columns of 4096..8192 elements: 1 - 11 % ahead on 47 of 48 shapes, level on one (65 x
+// 8200 x 4096 10.9 / 11.5, 65 x 13824 x 8192 19.3 / 21.1, 96 x 16384 x 5120 16.7 / 17.6, 96 x 11008 x 4096 11.9 / 12.1).  The
 // stream kernel has the longer loop but starts and ends faster (512 x 4096 x 512 4.8 against 5.9 us, x 1024 5.8 / 6.6, x
 // 2048 8.1 / 8.3, x 4096 13.3 / 11.9; 32 products of 1216 x 64 x 1216, 608 tiles: 12.8 us; 250 x 11008 x 4096, 344 tiles:
 // 24.8 against 17.7 on 128 x 128: two or three of its workgroups share a CU, but a round begun takes a round's time).  The dual-uniform row-sum epilogue (`mode5`) has no 256 x 256 tile
