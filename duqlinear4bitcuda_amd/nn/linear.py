@@ -43,11 +43,12 @@ def _put_copy(layer, name, key_name, make, wait):
         key = _weight_key(layer)
         with torch.inference_mode(False):
             copy = make(layer.weight)
-        if copy.is_cuda:
-            if torch.cuda.is_current_stream_capturing():
-                key = None
-            elif wait:
-                torch.cuda.current_stream(copy.device).synchronize()
+        if copy.device.type == "cuda":
+            with torch.cuda.device(copy.device):
+                if torch.cuda.is_current_stream_capturing():
+                    key = None
+                elif wait:
+                    torch.cuda.current_stream().synchronize()
         layer.register_buffer(name, copy, persistent=False)
         setattr(layer, key_name, key)
 

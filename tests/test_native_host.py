@@ -172,7 +172,6 @@ def test_a_layer_with_a_prepared_call_is_copied_and_saved(called):
 def test_copies_of_a_weight_made_by_two_threads_at_once(monkeypatch, what):
     """A thread that is behind with the copy of an older weight must not leave it in the place of the newer one."""
     import threading
-    from types import SimpleNamespace
 
     from duqlinear4bitcuda_amd import nn as qnn
     from duqlinear4bitcuda_amd.nn import linear
@@ -184,8 +183,6 @@ def test_copies_of_a_weight_made_by_two_threads_at_once(monkeypatch, what):
     else:
         layer = qnn.Linear4bitASQ(128, 64)
         monkeypatch.setattr(torch.Tensor, "is_cuda", True)
-        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
-        monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: SimpleNamespace(synchronize=lambda: None))
         layer.enable_fp6()
         make = layer._fp6_ready
     layer.weight.fill_(1)
