@@ -39,6 +39,75 @@ __device__ __forceinline__ uint32_t asym8_code(float x, float s, int zi)
 }
 __device__ __forceinline__ int asym8_zero_int(float z) { return rint_i32((float)(f16)z); }
 
+// Scale, zero point and code arithmetic of one row from its smallest and largest element (NaN if the row holds one).
+//
+// x / s has to be the float32 quotient, rounded once, and then rounded to binary16.  The division the compiler makes of it
+// is a dozen instructions per element and was the longest of the quantizer's three phases (load, arithmetic, store).  A row
+// has one divisor: y = 1 / s is computed once, q0 = x y is within 1.5 units in the last place, and q = q0 + (x - q0 s) y
+// (Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990) misses the correctly
+// rounded quotient only where x / s is closer than 2^-21 such units to the middle between two float32 numbers.  After the
+// rounding to binary16 that could show only beside the middle of two binary16 numbers; the pairs (x, s) with a quotient
+// that close to such a place are few enough to try them all (tests/test_int8_quotient.py), and none is rounded otherwise.
+// (No operand near the ends of the exponent range: `fast`.  Quotients so small that a remainder underflows give the code of
+// zero either way.)
+// From there two elements go together: both roundings to binary16 in one conversion, and in rows whose quotients stay
+// below 500 (all but rows far off zero for their spread) the rounding to an integer is the addition of 1536, which leaves
+// the integer in the low bits.  2048 x 4096 11.1 -> 8.4 us (5.0 TB/s), 512 x 11008 8.9 -> 7.3, 8 x 4096 3.2 -> 2.3.
+struct RowCode8 {
+    float s, z, y;
+    int zi;
+    bool fast;
+    __device__ __forceinline__ RowCode8(float lo, float hi)
+    {
+        // scale = (max - min) / 127, zeros = round(-min / scale)  (quantizer.py:50-51), float32.  torch evaluates
+        // tensor / scalar on a GPU as tensor * float32(1 / scalar), which is what the reference's scale is
+        const float d = hi - lo;
+        s = d * (1.0f / 127.0f);
+        z = __builtin_rintf((-lo) / s);
+        zi = asym8_zero_int(z);
+        y = 1.0f / s;
+        // (a NaN fails every comparison, an infinity the second)
+        fast = s >= 0x1p-100f && s <= 0x1p100f && fmaxf(__builtin_fabsf(lo), __builtin_fabsf(hi)) <= 500.0f * s;
+    }
+    __device__ __forceinline__ float quotient(float x) const
+    {
+        const float q0 = x * y;
+        float q = __builtin_fmaf(__builtin_fmaf(-q0, s, x), y, q0);
+        asm("" : "+v"(q));  // round to float32 here, then to binary16 (no mixed multiply-add with a single rounding)
+        return q;
+    }
+    __device__ __forceinline__ uint32_t quick4(const v4f32 g) const
+    {
+        const uint16_t off = (uint16_t)(0x6600 - zi);  // 0x6600: the bits of 1536
+        v2us c[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const v2h h = v2h{(f16)quotient(g[2 * i]), (f16)quotient(g[2 * i + 1])} + v2h{(f16)1536.0f, (f16)1536.0f};
+            c[i] = __builtin_elementwise_min(__builtin_elementwise_sub_sat(__builtin_bit_cast(v2us, h), v2us{off, off}),
+                                             v2us{kQmaxAsym8, kQmaxAsym8});
+        }
+        return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, c[1]), __builtin_bit_cast(uint32_t, c[0]), 0x06040200u);
+    }
+    __device__ __forceinline__ uint32_t slow4(const v4f32 g) const
+    {
+        uint32_t w = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w |= asym8_code(g[e], s, zi) << (8 * e);
+        return w;
+    }
+};
+
+// smallest and largest element so far, and whether a NaN was met (fminf / fmaxf pass one over)
+__device__ __forceinline__ void row_stats8(const v4f32 &g, float &lo, float &hi, bool &nan_seen)
+{
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+        lo = fminf(fminf(lo, g[e]), g[e + 1]);
+        hi = fmaxf(fmaxf(hi, g[e]), g[e + 1]);
+        nan_seen |= __builtin_isunordered(g[e], g[e + 1]);
+    }
+}
+
 // ---------------------------------------------------------------------------------
 // given-scale quantizer (asym_quant_host_8bit): 4 elements per lane step when the row
 // length allows, else one
@@ -84,38 +153,30 @@ int launch_asym_quant8(const float *x, const float *scale, const float *zeros, u
 // held in registers between the min / max reduction and the quantization (up to 8 x 4
 // elements per lane; longer rows are read a second time, from L2)
 // ---------------------------------------------------------------------------------
-constexpr int kMaxVec8 = 8;
 
-template <int WAVES, bool CACHED>
+// NV: 16-byte pieces of a row that a lane holds (0: none, the row is read twice).  Pieces past the row end are copies of
+// its last one, which change no statistic, and their codes are stored nowhere (beyond the descriptor): no piece hangs on a
+// branch of its own, so the chains of the quotients run side by side.
+template <int WAVES, int NV>
 __global__ __launch_bounds__(WAVES * 64) void quantize_rows_asym8_kernel(const float *x, uint32_t rows, uint32_t cols,
                                                                          int8_t *q, float *scale, float *zeros)
 {
     constexpr int T = WAVES * 64;
+    constexpr bool CACHED = NV > 0;
     __shared__ float red[2][WAVES];
     const uint32_t row = blockIdx.x, tid = threadIdx.x;
     const uint32_t nvec = cols >> 2;
     const v4f32 *xrow = reinterpret_cast<const v4f32 *>(x + (uint64_t)row * cols);
     uint32_t *qrow = reinterpret_cast<uint32_t *>(q + (uint64_t)row * cols);
-    v4f32 regs[kMaxVec8];
+    v4f32 regs[CACHED ? NV : 1];
     float lo = INFINITY, hi = -INFINITY;
     bool nan_seen = false;
-    auto reduce = [&](const v4f32 &g) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            lo = fminf(lo, g[e]);
-            hi = fmaxf(hi, g[e]);
-            nan_seen |= g[e] != g[e];
-        }
-    };
+    auto reduce = [&](const v4f32 &g) { row_stats8(g, lo, hi, nan_seen); };
     if (CACHED) {
 #pragma unroll
-        for (int i = 0; i < kMaxVec8; ++i) {
-            const uint32_t u = tid + i * T;
-            regs[i] = u < nvec ? __builtin_nontemporal_load(&xrow[u]) : v4f32{0.f, 0.f, 0.f, 0.f};
-        }
+        for (int i = 0; i < NV; ++i) regs[i] = __builtin_nontemporal_load(&xrow[min(tid + i * T, nvec - 1)]);
 #pragma unroll
-        for (int i = 0; i < kMaxVec8; ++i)
-            if (tid + i * T < nvec) reduce(regs[i]);
+        for (int i = 0; i < NV; ++i) reduce(regs[i]);
     } else {
         for (uint32_t u = tid; u < nvec; u += T) reduce(xrow[u]);
     }
@@ -139,31 +200,27 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_asym8_kernel(const f
         }
     }
     if (nan_seen) lo = hi = __builtin_nanf("");  // torch's min / max return NaN for a row that holds one
-    // scale = (max - min) / 127, zeros = round(-min / scale)  (quantizer.py:50-51), float32.  torch evaluates
-    // tensor / scalar on a GPU as tensor * float32(1 / scalar), which is what the reference's scale is
-    const float d = hi - lo;
-    const float s = d * (1.0f / 127.0f);
-    const float z = __builtin_rintf((-lo) / s);
+    const RowCode8 rc(lo, hi);
     if (tid == 0) {
-        scale[row] = s;
-        zeros[row] = z;
+        scale[row] = rc.s;
+        zeros[row] = rc.z;
     }
-    const int zi = asym8_zero_int(z);
-    auto quant4 = [&](const v4f32 &g) -> uint32_t {
-        uint32_t w = 0;
+    auto quantize = [&](auto code4) {
+        if (CACHED) {
+            const __amdgpu_buffer_rsrc_t rQ = make_rsrc(qrow, cols);
+            uint32_t c[CACHED ? NV : 1];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w |= asym8_code(g[e], s, zi) << (8 * e);
-        return w;
-    };
-    if (CACHED) {
+            for (int i = 0; i < NV; ++i) c[i] = code4(regs[i]);
 #pragma unroll
-        for (int i = 0; i < kMaxVec8; ++i) {
-            const uint32_t u = tid + i * T;
-            if (u < nvec) qrow[u] = quant4(regs[i]);
+            for (int i = 0; i < NV; ++i) __builtin_amdgcn_raw_buffer_store_b32(c[i], rQ, (int)((tid + i * T) * 4), 0, 0);
+        } else {
+            for (uint32_t u = tid; u < nvec; u += T) qrow[u] = code4(xrow[u]);
         }
-    } else {
-        for (uint32_t u = tid; u < nvec; u += T) qrow[u] = quant4(xrow[u]);
-    }
+    };
+    if (__builtin_amdgcn_readfirstlane(rc.fast))  // (one row, one answer)
+        quantize([&](const v4f32 &g) { return rc.quick4(g); });
+    else
+        quantize([&](const v4f32 &g) { return rc.slow4(g); });
 }
 
 int launch_quantize_rows_asym8(const float *x, uint32_t rows, uint32_t cols, int8_t *q, float *scale, float *zeros,
@@ -173,21 +230,18 @@ int launch_quantize_rows_asym8(const float *x, uint32_t rows, uint32_t cols, int
     const uint32_t nvec = cols / 4;
     uint32_t waves = 1;
     while (waves < 16 && waves * 64 * 4 < nvec) waves *= 2;  // four 128-bit loads per lane when the row allows
-    const bool cached = waves * 64 * kMaxVec8 >= nvec;
     const dim3 grid(rows);
-#define DUQ_ROWS8(W)                                                                                              \
-    case W:                                                                                                       \
-        if (cached)                                                                                               \
-            hipLaunchKernelGGL((quantize_rows_asym8_kernel<W, true>), grid, dim3(W * 64), 0, stream, x, rows, cols, q, scale, zeros); \
-        else                                                                                                      \
-            hipLaunchKernelGGL((quantize_rows_asym8_kernel<W, false>), grid, dim3(W * 64), 0, stream, x, rows, cols, q, scale, zeros); \
-        break;
+#define DUQ_ROWS8(W, V) \
+    hipLaunchKernelGGL((quantize_rows_asym8_kernel<W, V>), grid, dim3(W * 64), 0, stream, x, rows, cols, q, scale, zeros)
     switch (waves) {
-        DUQ_ROWS8(1)
-        DUQ_ROWS8(2)
-        DUQ_ROWS8(4)
-        DUQ_ROWS8(8)
-        DUQ_ROWS8(16)
+    case 1: DUQ_ROWS8(1, 4); break;
+    case 2: DUQ_ROWS8(2, 4); break;
+    case 4: DUQ_ROWS8(4, 4); break;
+    case 8: DUQ_ROWS8(8, 4); break;
+    default:
+        if (nvec <= 16 * 64 * 4) DUQ_ROWS8(16, 4);
+        else if (nvec <= 16 * 64 * 8) DUQ_ROWS8(16, 8);
+        else DUQ_ROWS8(16, 0);
     }
 #undef DUQ_ROWS8
     return (int)hipGetLastError();
@@ -831,18 +885,17 @@ __global__ __launch_bounds__(512) void gemm_s8_decode_kernel(DUQ_HEAD_DECL, Gemm
     // loads in the order their data is needed: activations, the first tile's weights, the finishing threads' row
     // parameters
     v4i x[MT][SEGS];
+    v4i w0[SEGS], w1[SEGS];
+    // thread (mt = tid / 64, lane) finishes C[mt*16 + l16][tile*16 + 4*g + (0..3)]
+    const bool finisher = tid < MT * 64;
+    const uint32_t m = wave * 16 + l16;
+    float sr = 0.f, zr = 0.f;
 #pragma unroll
     for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int u = 0; u < SEGS; ++u)
             x[t][u] = __builtin_bit_cast(v4i, buf_load16(rX, koff[u] != kOobOffset ? (t * 16 + l16) * p.K + koff[u] : kOobOffset, 0));
-    v4i w0[SEGS], w1[SEGS];
     load_tile(tile0, w0);
-
-    // thread (mt = tid / 64, lane) finishes C[mt*16 + l16][tile*16 + 4*g + (0..3)]
-    const bool finisher = tid < MT * 64;
-    const uint32_t m = wave * 16 + l16;
-    float sr = 0.f, zr = 0.f;
     if (FUSED && finisher) {
         const uint32_t mm = min(m, p.M - 1);
         sr = p.epi.s_row[mm], zr = p.epi.z_row[mm];
