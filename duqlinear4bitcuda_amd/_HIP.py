@@ -1219,8 +1219,8 @@ def linear8bit_forward(xq, scale_x, zeros_x, w, w_scale, w_zeros, bias=None, til
 
 
 def quantize_linear8bit_forward(x, w, w_tiled, w_scale, w_zeros, bias=None):
-    """AsymQuantizer8bit + linear8bit_forward in one library call (two launches, the codes staged in a workspace
-    allocated here): x float32 [..., K] -> float32 [..., N], the bits of the two calls.  ``w`` the weight [N, K]
+    """AsymQuantizer8bit + linear8bit_forward in one library call (one launch up to eight rows of at most 4096
+    elements, else two, the codes staged in a workspace allocated here): x float32 [..., K] -> float32 [..., N], the bits of the two calls.  ``w`` the weight [N, K]
     int8, ``w_tiled`` its tiled copy from weight_tile_8bit or None."""
     name = "quantize_linear8bit_forward"
     if type(x) is torch.Tensor and x.is_cuda and type(w) is torch.Tensor and w.dim() == 2:

@@ -843,9 +843,16 @@ __global__ __launch_bounds__(256) void gemm_s8_skinny_kernel(DUQ_HEAD_DECL, Gemm
 // with two tiles' weights in flight (two register sets alternate), so a launch is one round of at most 256
 // workgroups and the activations (as many bytes as a tile's weights at 16 rows) enter a CU once.  The partial
 // tiles meet in LDS; MT * 64 threads finish four consecutive columns of one row each.
-template <int SEGS, int MT, bool FUSED, bool BIAS, bool TILED>
+//
+// RQ > 0 (1, 2, 4 or 8 rows): p.A holds float32 rows and the workgroup quantizes all of them itself, with the arithmetic of
+// the row quantizer, while its weights are on the way: 8 / RQ wavefronts per row, which hold it in registers between the
+// statistics and the codes; the codes meet in LDS in place of a launch, a write and a read of their own.  What it costs over
+// the GEMM alone is the way of M * K floats into every CU (8 x 4096: 1.8 us of 7.1; the arithmetic is 0.5, in the time of
+// the weights).  Weights are requested right behind the rows (with a barrier between the two 7.75).
+template <int SEGS, int MT, bool FUSED, bool BIAS, bool TILED, int RQ = 0>
 __global__ __launch_bounds__(512) void gemm_s8_decode_kernel(DUQ_HEAD_DECL, Gemm8Params tail)
 {
+    static_assert(RQ == 0 || (MT == 1 && FUSED), "rows quantized here: one row tile");
     Gemm8Params p = with_head(tail, DUQ_HEAD_USE);
     to_global(p.A);
     to_global(p.B);
@@ -890,15 +897,67 @@ __global__ __launch_bounds__(512) void gemm_s8_decode_kernel(DUQ_HEAD_DECL, Gemm
     const bool finisher = tid < MT * 64;
     const uint32_t m = wave * 16 + l16;
     float sr = 0.f, zr = 0.f;
+    if constexpr (RQ == 0) {
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+        for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int u = 0; u < SEGS; ++u)
-            x[t][u] = __builtin_bit_cast(v4i, buf_load16(rX, koff[u] != kOobOffset ? (t * 16 + l16) * p.K + koff[u] : kOobOffset, 0));
-    load_tile(tile0, w0);
-    if (FUSED && finisher) {
-        const uint32_t mm = min(m, p.M - 1);
-        sr = p.epi.s_row[mm], zr = p.epi.z_row[mm];
+            for (int u = 0; u < SEGS; ++u)
+                x[t][u] = __builtin_bit_cast(v4i, buf_load16(rX, koff[u] != kOobOffset ? (t * 16 + l16) * p.K + koff[u] : kOobOffset, 0));
+        load_tile(tile0, w0);
+        if (FUSED && finisher) {
+            const uint32_t mm = min(m, p.M - 1);
+            sr = p.epi.s_row[mm], zr = p.epi.z_row[mm];
+        }
+    } else {
+        constexpr uint32_t kStride = 512 * SEGS + 16;  // bytes of a row of codes: sixteen rows' pieces on all banks
+        constexpr int WPR = WAVES / RQ, NV = 2 * SEGS / WPR;
+        __shared__ __attribute__((aligned(16))) uint8_t codes[RQ * kStride];
+        __shared__ float stat[2][WAVES], rowp[2][RQ];
+        const uint32_t r = wave / WPR, part = wave % WPR, nvec = p.K >> 2;
+        const __amdgpu_buffer_rsrc_t rF = make_rsrc(p.A, p.M * p.K * 4);
+        v4f32 v[NV];  // (pieces past the row end are copies of its last one: no statistic changes, no weight meets their codes)
+        auto piece = [&](int i) { return (part * NV + i) * 64 + lane; };
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            v[i] = __builtin_bit_cast(v4f32, buf_load16(rF, (min(r, p.M - 1) * nvec + min(piece(i), nvec - 1)) * 16, 0));
+        load_tile(tile0, w0);
+        load_tile(tile0 + 1, w1);
+        float lo = INFINITY, hi = -INFINITY;
+        bool nan_seen = false;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) row_stats8(v[i], lo, hi, nan_seen);
+        lo = wave_min_f32(lo);
+        hi = wave_max_f32(hi);
+        if (__builtin_amdgcn_ballot_w64(nan_seen) != 0) lo = hi = __builtin_nanf("");
+        if constexpr (WPR > 1) {
+            if (lane == 0) stat[0][wave] = lo, stat[1][wave] = hi;
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (no wait for the weights)
+#pragma unroll
+            for (int k = 0; k < WPR; ++k) {
+                const float l = stat[0][r * WPR + k], h = stat[1][r * WPR + k];
+                nan_seen |= l != l;
+                lo = fminf(lo, l);
+                hi = fmaxf(hi, h);
+            }
+            if (__builtin_amdgcn_ballot_w64(nan_seen) != 0) lo = hi = __builtin_nanf("");
+        }
+        const RowCode8 rc(lo, hi);
+        if (part == 0 && lane == 0) rowp[0][r] = rc.s, rowp[1][r] = rc.z;
+        auto quantize = [&](auto code4) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                *reinterpret_cast<uint32_t *>(codes + r * kStride + piece(i) * 4) = code4(v[i]);
+        };
+        if (__builtin_amdgcn_readfirstlane(rc.fast))
+            quantize([&](const v4f32 &q) { return rc.quick4(q); });
+        else
+            quantize([&](const v4f32 &q) { return rc.slow4(q); });
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int u = 0; u < SEGS; ++u) {
+            x[0][u] = *reinterpret_cast<const v4i *>(codes + min(l16, (uint32_t)RQ - 1) * kStride + (wave * SEGS + u) * 64 + g * 16);
+        }
+        sr = rowp[0][min(m, (uint32_t)RQ - 1)], zr = rowp[1][min(m, (uint32_t)RQ - 1)];
     }
     const void *outp = FUSED ? (const void *)p.y : (const void *)p.C;
     const bool vec_all = p.N % 4 == 0 && reinterpret_cast<uintptr_t>(outp) % 16 == 0;
@@ -967,7 +1026,7 @@ __global__ __launch_bounds__(512) void gemm_s8_decode_kernel(DUQ_HEAD_DECL, Gemm
 
     // the partial-sum buffers alternate with the register sets: one barrier per tile
     for (uint32_t t = tile0; t < tile_end; t += 2) {
-        load_tile(t + 1, w1);
+        if (RQ == 0 || t > tile0) load_tile(t + 1, w1);
         compute_tile(t, w0, 0);
         load_tile(t + 2, w0);
         if (t + 1 < tile_end) compute_tile(t + 1, w1, 1);
@@ -1006,6 +1065,45 @@ static void launch_decode8(Gemm8Params &p, hipStream_t stream)
         else DUQ_DEC8(4, 4);
     }
 #undef DUQ_DEC8
+}
+
+// Up to eight float32 rows of at most 4096 elements: quantizer and GEMM in one launch of the decode kernel.  Against two
+// launches with the present quantizer, on the tiled copy (up to four rows: on the weight as stored, whose kernel is the faster
+// one there), weights rotated over > 512 MB: 1 x 4096 x 4096 5.4 / 6.5 us, 2 rows 5.65 / 6.75, 4 rows 6.2 / 7.4, 8 rows 7.1 / 8.0,
+// 8 x 4096 x 2048 4.35 / 6.3, 8 x 11008 x 4096 11.1 / 12.2, 8 x 28672 x 4096 20.7 / 22.0.
+bool quantize_gemm8_fuses(uint32_t M, uint32_t N, uint32_t K) { return M <= 8 && K <= 4096 && decode8_takes(M, N, K); }
+
+template <bool BIAS, bool TILED>
+static void launch_decode8_rq(Gemm8Params &p, hipStream_t stream)
+{
+    const uint32_t ntiles = (p.N + 15) / 16;
+    p.tiles_n = (ntiles + 255) / 256;
+    const dim3 grid((ntiles + p.tiles_n - 1) / p.tiles_n);
+#define DUQ_DEC8(S, R) DUQ_LAUNCH_HEAD((gemm_s8_decode_kernel<S, 1, true, BIAS, TILED, R>), grid, dim3(512), 0, stream, p)
+#define DUQ_DEC8R(S)                                                                                                    \
+    if (p.M == 1) DUQ_DEC8(S, 1);                                                                                       \
+    else if (p.M == 2) DUQ_DEC8(S, 2);                                                                                  \
+    else if (p.M <= 4) DUQ_DEC8(S, 4);                                                                                  \
+    else DUQ_DEC8(S, 8)
+    if (p.K > 2048) {
+        DUQ_DEC8R(8);
+    } else {
+        DUQ_DEC8R(4);
+    }
+#undef DUQ_DEC8R
+#undef DUQ_DEC8
+}
+
+// x [M,K] float32, 16-byte aligned; a shape that quantize_gemm8_fuses takes
+int launch_quantize_gemm_s8(const float *x, const int8_t *B, bool b_tiled, uint32_t M, uint32_t N, uint32_t K, const float *s_col,
+                            const float *z_col, const float *bias, float *y, hipStream_t stream)
+{
+    Gemm8Params p{reinterpret_cast<const int8_t *>(x), B, M, N, K, 0, nullptr, y, 0, Epi8{nullptr, nullptr, s_col, z_col, bias}};
+    if (b_tiled)
+        bias ? launch_decode8_rq<true, true>(p, stream) : launch_decode8_rq<false, true>(p, stream);
+    else
+        bias ? launch_decode8_rq<true, false>(p, stream) : launch_decode8_rq<false, false>(p, stream);
+    return (int)hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------------

@@ -199,6 +199,10 @@ int launch_asym_quant8(const float *x, const float *scale, const float *zeros, u
                        hipStream_t stream);
 int launch_quantize_rows_asym8(const float *x, uint32_t rows, uint32_t cols, int8_t *q, float *scale, float *zeros,
                                hipStream_t stream);
+// up to eight rows: the same and the GEMM in one launch (duq_int8.hip)
+bool quantize_gemm8_fuses(uint32_t M, uint32_t N, uint32_t K);
+int launch_quantize_gemm_s8(const float *x, const int8_t *B, bool b_tiled, uint32_t M, uint32_t N, uint32_t K, const float *s_col,
+                            const float *z_col, const float *bias, float *y, hipStream_t stream);
 int launch_dequant_hprec(const int32_t *acc, const float *s_row, const float *z_row, const float *s_col,
                          const float *z_col, const float *bias, uint32_t rows, uint32_t cols, float *x,
                          hipStream_t stream);

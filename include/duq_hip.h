@@ -493,8 +493,8 @@ int duq_linear8bit_forward_tiled(const int8_t *xq, const float *scale_x, const f
  * bits as the two calls.  x [M,K] float32, 16-byte aligned, K % 32 == 0; w the weight as stored and / or w_tiled its
  * tiled copy (one may be NULL): up to four rows (two of more than 4096 elements) read w when it is given, everything
  * else w_tiled when it is given.  workspace: duq_quantize_linear8bit_workspace_bytes(M, K) bytes (codes, scales,
- * zero points), 16-byte aligned.  What a step of the layer costs at a few rows is mostly the host's share of a
- * call; this halves it. */
+ * zero points), 16-byte aligned.  Up to eight rows of at most 4096 elements are one launch, which quantizes the rows itself
+ * (and reads w_tiled when it is given); the workspace is asked for all the same. */
 uint64_t duq_quantize_linear8bit_workspace_bytes(uint32_t M, uint32_t K);
 int duq_quantize_linear8bit_forward(const float *x, const int8_t *w, const int8_t *w_tiled, const float *w_scale,
                                     const float *w_zeros, const float *bias, uint32_t M, uint32_t N, uint32_t K, float *y,

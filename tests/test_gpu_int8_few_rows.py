@@ -1,4 +1,5 @@
-"""The 8-bit layer's row quantizer: rows of every kind, lengths that end inside a wavefront's share."""
+"""The 8-bit layer on up to eight rows (quantizer inside the GEMM's launch) and its row quantizer: rows of every kind, lengths
+that end inside a wavefront's share, both weight layouts."""
 import numpy as np
 import pytest
 import torch
@@ -36,3 +37,25 @@ def test_row_quantizer(dev, M, K):
     assert np.array_equal(s.cpu().numpy().reshape(-1), s_want.reshape(-1), equal_nan=True)
     assert np.array_equal(z.cpu().numpy().reshape(-1), z_want.reshape(-1), equal_nan=True)
     assert np.array_equal(q.cpu().numpy(), q_want)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (1, 40, 4096), (2, 17, 64), (2, 4100, 2048), (3, 33, 2080), (4, 300, 1056), (5, 16, 96),
+                                   (7, 4113, 4064), (8, 4096, 4096), (8, 129, 2048), (8, 70, 32), (6, 9000, 512)])
+def test_quantizer_inside_the_gemm(dev, M, N, K):
+    """The same bits as the two launches, whose kernels the oracle tests cover."""
+    from duqlinear4bitcuda_amd import _HIP as hip
+    print("8-bit few rows", M, N, K, flush=True)
+    gen = torch.Generator(device=dev).manual_seed(M * 31 + K)
+    w = torch.randint(0, 128, (N, K), generator=gen, device=dev, dtype=torch.int8)
+    sw = torch.rand(N, generator=gen, device=dev) * 0.01
+    zw = torch.randint(0, 127, (N,), generator=gen, device=dev).float()
+    bias = torch.randn(N, generator=gen, device=dev)
+    tiled = hip.weight_tile_8bit(w)
+    for seed in (0, 3, 6):
+        x = torch.from_numpy(_rows(M, K, seed)).to(dev)
+        q, s, z = hip.quantize_rows_asym_8bit(x)
+        for b in (None, bias):
+            want = hip.linear8bit_forward(q, s, z, w, sw, zw, b)
+            for t in (None, tiled):
+                got = hip.quantize_linear8bit_forward(x, w, t, sw, zw, b)
+                assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (seed, b is None, t is None)
