@@ -16,6 +16,7 @@
 #include "duq_device.h"
 #include "duq_launch.h"
 #include "duq_rowquant.h"
+#include "duq_tiles.h"
 
 namespace duq {
 
@@ -187,10 +188,9 @@ int launch_asym_dual_quant(const uint16_t *x, const uint16_t *s1, const uint16_t
 // A row of `cols` elements is split into units of 8 (one 128-bit load, one 32-bit store).
 // WAVES wavefronts share one row; lane t owns units t, t+T, t+2T, ... (T = 64*WAVES), so
 // every load and store instruction of a wavefront covers one contiguous 1 KB / 256 B span,
-// and keeps up to kMaxUnits of them in registers between the reduction and the
-// quantization: x is read from HBM exactly once.  Rows longer than 8*kMaxUnits*T elements
-// run the same code with CACHED = false: the units are read a second time (from L2).
-constexpr int kMaxUnits = 8;  // 64 elements = 32 VGPRs of row data per lane
+// and keeps up to eight of them (32 VGPRs) in registers between the reduction and the
+// quantization: x is read from HBM exactly once.  Rows longer than 8 * 8 * 1024 elements
+// run the same code with NV = 0: the units are read a second time (from L2).
 
 // The fused row quantizer writes its codes / shadow with non-temporal stores (nobody reads them in this launch;
 // measured at 2048 x 4096: shadow 6.6 against 7.15 us, nibbles level).
@@ -266,7 +266,11 @@ __device__ __forceinline__ const v4u *row_units(const RowParams &p, uint32_t row
 // consecutive units); the packed words of a row meet in LDS so that the loads keep the
 // coalesced unit-per-lane pattern and a lane still converts whole blocks.  The packed nibbles
 // are written only when p.q is given.
-template <int WAVES, bool ASYM, bool CACHED, int FORM>
+//
+// NV: units that a lane holds (0: none, the row is read twice).  Those past the row end are copies of its last one, which
+// change no statistic, and their codes go beyond the descriptor of the row: no unit hangs on a branch of its own, and the
+// chains of a lane's units run side by side.
+template <int WAVES, int NV, bool ASYM, int FORM>
 __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL, RowParams tail)
 {
     RowParams p = with_head(tail, DUQ_HEAD_USE);
@@ -276,7 +280,7 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
     to_global(p.zeros);
     to_global(p.bf6);
     constexpr int T = WAVES * 64;
-    constexpr bool BF6 = FORM == kShadow;
+    constexpr bool BF6 = FORM == kShadow, CACHED = NV > 0;
     __shared__ float red[3][WAVES];
     __shared__ int red_sum[WAVES];
     const bool shifted = ASYM && p.rowsum != nullptr;
@@ -286,24 +290,20 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
     const uint32_t nunits = p.cols >> 3;  // units of 8 elements
     const v4u *xrow = row_units<FORM>(p, row);
     uint32_t *qrow = reinterpret_cast<uint32_t *>(p.q + (uint64_t)row * (p.cols >> 1));
-    __shared__ __attribute__((aligned(16))) uint32_t words[BF6 && CACHED ? T * kMaxUnits : 4];
+    __shared__ __attribute__((aligned(16))) uint32_t words[BF6 && CACHED ? T * NV : 4];
     // unit held in register slot i
     auto unit_of = [&](int i) -> uint32_t { return tid + i * T; };
 
-    v4u regs[kMaxUnits];
+    v4u regs[CACHED ? NV : 1];
     PkMinMax st;  // packed running maximum and minimum of this lane's elements
 
     auto reduce_unit = [&](const v4u &g) { st.add8(g); };
 
     if (CACHED) {
 #pragma unroll
-        for (int i = 0; i < kMaxUnits; ++i) {
-            const uint32_t u = unit_of(i);
-            regs[i] = u < nunits ? __builtin_nontemporal_load(&xrow[u]) : v4u{0u, 0u, 0u, 0u};
-        }
+        for (int i = 0; i < NV; ++i) regs[i] = __builtin_nontemporal_load(&xrow[min(unit_of(i), nunits - 1)]);
 #pragma unroll
-        for (int i = 0; i < kMaxUnits; ++i)
-            if (unit_of(i) < nunits) reduce_unit(regs[i]);
+        for (int i = 0; i < NV; ++i) reduce_unit(regs[i]);
     } else {
         for (uint32_t u = tid; u < nunits; u += T) reduce_unit(xrow[u]);
     }
@@ -356,16 +356,30 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
     }
 
     // ---- quantize + pack: 8 elements -> one 32-bit store ----
-    auto quant_unit = [&](const v4u &g) -> uint32_t {
-        uint32_t w = rq.quant8(g);
-        if (shifted) {
-            // eight unsigned codes: sum them, then u - 8 as a signed nibble is u with bit 3 flipped
-            const uint32_t pairs = (w & 0x0F0F0F0Fu) + ((w >> 4) & 0x0F0F0F0Fu);
-            code_sum = (int)__builtin_amdgcn_udot4(pairs, 0x01010101u, (uint32_t)code_sum, false);
-            w ^= 0x88888888u;
-        }
-        return w;
+    // shifted form, eight unsigned codes: sum them, then u - 8 as a signed nibble is u with bit 3 flipped
+    auto shift_codes = [&](uint32_t w, bool counts) -> uint32_t {
+        const uint32_t pairs = (w & 0x0F0F0F0Fu) + ((w >> 4) & 0x0F0F0F0Fu);
+        const uint32_t sum = __builtin_amdgcn_udot4(pairs, 0x01010101u, (uint32_t)code_sum, false);
+        code_sum = counts ? (int)sum : code_sum;
+        return w ^ 0x88888888u;
     };
+    auto quant_unit = [&](const v4u &g) -> uint32_t {  // (rows that are not held)
+        const uint32_t w = rq.quant8(g);
+        return shifted ? shift_codes(w, true) : w;
+    };
+    uint32_t w[CACHED ? NV : 1];
+    if constexpr (CACHED) {
+        rq.quant_units(regs, w);
+        if (shifted)
+#pragma unroll
+            for (int i = 0; i < NV; ++i) w[i] = shift_codes(w[i], unit_of(i) < nunits);
+        if (!BF6 || p.q) {
+            const __amdgpu_buffer_rsrc_t rQ = make_rsrc(qrow, nunits * 4);
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                __builtin_amdgcn_raw_buffer_store_b32(w[i], rQ, (int)(unit_of(i) * 4), 0, DUQ_QUANT_NT_STORE ? 2 : 0);
+        }
+    }
     if (BF6) {
         // cols % 32 == 0: a block is all inside the row or all outside
         const uint32_t nblk = p.cols >> 5;
@@ -378,17 +392,10 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
         };
         if (CACHED) {
 #pragma unroll
-            for (int i = 0; i < kMaxUnits; ++i) {
-                const uint32_t u = tid + i * T;
-                if (u < nunits) {
-                    const uint32_t w = quant_unit(regs[i]);
-                    words[u] = w;
-                    if (p.q) DUQ_QSTORE(&qrow[u], w);
-                }
-            }
+            for (int i = 0; i < NV; ++i) words[unit_of(i)] = w[i];
             __syncthreads();
 #pragma unroll
-            for (int g = 0; g < kMaxUnits / 4; ++g) {
+            for (int g = 0; g < (NV + 3) / 4; ++g) {
                 const uint32_t b = tid + g * T;
                 if (b < nblk) {
                     const v4u w4 = *reinterpret_cast<const v4u *>(&words[4 * b]);
@@ -406,13 +413,7 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
                 put_block(b, w);
             }
         }
-    } else if (CACHED) {
-#pragma unroll
-        for (int i = 0; i < kMaxUnits; ++i) {
-            const uint32_t u = tid + i * T;
-            if (u < nunits) DUQ_QSTORE(&qrow[u], quant_unit(regs[i]));
-        }
-    } else {
+    } else if constexpr (!CACHED) {
         for (uint32_t u = tid; u < nunits; u += T) DUQ_QSTORE(&qrow[u], quant_unit(xrow[u]));
     }
     if (shifted) {  // uniform branch: sum of (u - 8) over the row
@@ -430,10 +431,14 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
 
 // Short rows (at most 512 elements, no shadow: the operands of quantized attention).  With a workgroup per row such a
 // launch is bound by how fast workgroups start (65536 rows of 128 elements, asymmetric: 21.4 us for 21 MB, a quarter of a workgroup's
-// lanes at work).  Here LANES lanes hold a row, two units each, a workgroup takes 256 / LANES rows at a time and PASSES
-// times as many in all, every load of them requested up front; the same launch takes 7.4 us.  Two units per lane, not
-// one, because the constants of a row are computed by each of its lanes and cost as much as two units' codes.
-template <int LANES, int PASSES, bool ASYM, int FORM>
+// lanes at work).  Here LANES lanes hold a row, two units each, and a workgroup takes 256 / LANES rows; the same launch takes
+// 5.9 us.  Two units per lane, not one, because the constants of a row are computed by each of its lanes and cost as much as
+// two units' codes.  One set of rows per workgroup, not several whose loads are all requested up front: workgroups that
+// start while others compute and store overlap the three (131072 x 128 9.2 us = 4.6 TB/s against 10.35 with four sets, 131072
+// x 64 6.5 / 7.9, 40960 x 256 7.2 / 8.6, 16384 x 512 5.9 / 7.7).
+constexpr uint32_t kShortGrid = 1u << 22;  // workgroups in x (a launch has less than 2^32 threads in a dimension)
+
+template <int LANES, bool ASYM, int FORM>
 __global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL, RowParams tail)
 {
     RowParams p = with_head(tail, DUQ_HEAD_USE);
@@ -441,68 +446,61 @@ __global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL,
     to_global(p.q);
     to_global(p.scale);
     to_global(p.zeros);
-    constexpr uint32_t kRows = 256 / LANES;
     const bool shifted = ASYM && p.rowsum != nullptr;
     const uint32_t nunits = p.cols >> 3;  // <= 2 * LANES
-    const uint32_t u0 = threadIdx.x % LANES, row0 = blockIdx.x * (kRows * PASSES) + threadIdx.x / LANES;
+    const uint32_t u0 = threadIdx.x % LANES, row = (blockIdx.y * kShortGrid + blockIdx.x) * (256 / LANES) + threadIdx.x / LANES;
     uint32_t *q32 = reinterpret_cast<uint32_t *>(p.q);
 
-    v4u regs[PASSES][2];
+    v4u regs[2];
 #pragma unroll
-    for (int i = 0; i < PASSES; ++i)
+    for (int j = 0; j < 2; ++j) {
+        const uint32_t u = u0 + j * LANES;
+        regs[j] = row < p.rows && u < nunits ? __builtin_nontemporal_load(row_units<FORM>(p, row) + u) : v4u{0u, 0u, 0u, 0u};
+    }
+    PkMinMax st;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+        if (u0 + j * LANES < nunits) st.add8(regs[j]);
+    float a = 0.f, b = 0.f;
+    uint32_t m16;
+    if (!ASYM) {
+        m16 = group_reduce<LANES>(st.absmax_bits(), [](uint32_t x, uint32_t y) { return max(x, y); });
+    } else {
+        st.mx = group_reduce<LANES>(st.mx, [](uint32_t x, uint32_t y) {
+            asm("v_pk_maximum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
+            return x;
+        });
+        st.mn = group_reduce<LANES>(st.mn, [](uint32_t x, uint32_t y) {
+            asm("v_pk_minimum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
+            return x;
+        });
+        m16 = st.absmax_bits();
+        a = st.min_f32();
+        b = st.max_f32();
+        if (m16 > 0x7C00u) a = b = __builtin_nanf("");  // torch's min / max return NaN for a row that holds one
+    }
+    RowQuant<ASYM, false> rq;
+    rq.init(m16, a, b, p.clip, p.qmax);
+    uint32_t w[2];
+    rq.quant_units(regs, w);
+    if (shifted) {  // uniform branch: see quantize_rows_kernel
+        uint32_t sum = 0;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const uint32_t row = row0 + i * kRows, u = u0 + j * LANES;
-            regs[i][j] = row < p.rows && u < nunits ? __builtin_nontemporal_load(row_units<FORM>(p, row) + u) : v4u{0u, 0u, 0u, 0u};
+            const uint32_t pairs = (w[j] & 0x0F0F0F0Fu) + ((w[j] >> 4) & 0x0F0F0F0Fu);
+            if (u0 + j * LANES < nunits) sum = __builtin_amdgcn_udot4(pairs, 0x01010101u, sum, false);
+            w[j] ^= 0x88888888u;
         }
-#pragma unroll
-    for (int i = 0; i < PASSES; ++i) {
-        const uint32_t row = row0 + i * kRows;
-        PkMinMax st;
+        sum = group_reduce<LANES>(sum, [](uint32_t x, uint32_t y) { return x + y; });
+        if (u0 == 0 && row < p.rows) p.rowsum[row] = (int)sum - 8 * (int)p.cols;
+    }
+    if (row < p.rows) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            if (u0 + j * LANES < nunits) st.add8(regs[i][j]);
-        float a = 0.f, b = 0.f;
-        uint32_t m16;
-        if (!ASYM) {
-            m16 = group_reduce<LANES>(st.absmax_bits(), [](uint32_t x, uint32_t y) { return max(x, y); });
-        } else {
-            st.mx = group_reduce<LANES>(st.mx, [](uint32_t x, uint32_t y) {
-                asm("v_pk_maximum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
-                return x;
-            });
-            st.mn = group_reduce<LANES>(st.mn, [](uint32_t x, uint32_t y) {
-                asm("v_pk_minimum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
-                return x;
-            });
-            m16 = st.absmax_bits();
-            a = st.min_f32();
-            b = st.max_f32();
-            if (m16 > 0x7C00u) a = b = __builtin_nanf("");  // torch's min / max return NaN for a row that holds one
-        }
-        RowQuant<ASYM, false> rq;
-        rq.init(m16, a, b, p.clip, p.qmax);
-        uint32_t w[2];
-        rq.quant_units(regs[i], w);
-        if (shifted) {  // uniform branch: see quantize_rows_kernel
-            uint32_t sum = 0;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint32_t pairs = (w[j] & 0x0F0F0F0Fu) + ((w[j] >> 4) & 0x0F0F0F0Fu);
-                if (u0 + j * LANES < nunits) sum = __builtin_amdgcn_udot4(pairs, 0x01010101u, sum, false);
-                w[j] ^= 0x88888888u;
-            }
-            sum = group_reduce<LANES>(sum, [](uint32_t x, uint32_t y) { return x + y; });
-            if (u0 == 0 && row < p.rows) p.rowsum[row] = (int)sum - 8 * (int)p.cols;
-        }
-        if (row < p.rows) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                if (u0 + j * LANES < nunits) DUQ_QSTORE(&q32[(uint64_t)row * nunits + u0 + j * LANES], w[j]);
-            if (u0 == 0) {
-                p.scale[row] = f16_to_bits(rq.s);
-                if (ASYM) p.zeros[row] = f16_to_bits(shifted ? rq.z - (f16)8.0f : rq.z);
-            }
+            if (u0 + j * LANES < nunits) DUQ_QSTORE(&q32[(uint64_t)row * nunits + u0 + j * LANES], w[j]);
+        if (u0 == 0) {
+            p.scale[row] = f16_to_bits(rq.s);
+            if (ASYM) p.zeros[row] = f16_to_bits(shifted ? rq.z - (f16)8.0f : rq.z);
         }
     }
 }
@@ -510,14 +508,11 @@ __global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL,
 template <bool ASYM, int FORM>
 static int launch_short_rows(const RowParams &p, hipStream_t stream)
 {
-    // four passes where that still leaves two workgroups per CU, one otherwise (few rows: latency)
 #define DUQ_SHORT(L)                                                                                                  \
     do {                                                                                                              \
-        const uint64_t groups = ((uint64_t)p.rows * L + 255) / 256;                                                   \
-        if (groups >= 2048)                                                                                           \
-            DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, 4, ASYM, FORM>), dim3((uint32_t)((groups + 3) / 4)), dim3(256), 0, stream, p); \
-        else                                                                                                          \
-            DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, 1, ASYM, FORM>), dim3((uint32_t)groups), dim3(256), 0, stream, p); \
+        const uint32_t groups = (uint32_t)(((uint64_t)p.rows * L + 255) / 256);                                       \
+        const dim3 grid(std::min(groups, kShortGrid), (groups + kShortGrid - 1) / kShortGrid);                        \
+        DUQ_LAUNCH_HEAD((quantize_short_rows_kernel<L, ASYM, FORM>), grid, dim3(256), 0, stream, p);                  \
     } while (0)
     if (p.cols <= 64)
         DUQ_SHORT(4);
@@ -550,15 +545,16 @@ static int launch_rows(const RowParams &p, hipStream_t stream)
     uint32_t waves = waves_for(4);
     if ((uint64_t)p.rows * waves < 2048) waves = waves_for(2);
     if ((uint64_t)p.rows * waves < 512) waves = waves_for(1);
-    const bool cached = waves * 64 * kMaxUnits >= nunits;
-#define DUQ_ROWS_LAUNCH(W, C) DUQ_LAUNCH_HEAD((quantize_rows_kernel<W, ASYM, C, FORM>), grid, dim3(W * 64), 0, stream, p);
+    const uint32_t held = (nunits + waves * 64 - 1) / (waves * 64);  // units per lane
+#define DUQ_ROWS_LAUNCH(W, V) DUQ_LAUNCH_HEAD((quantize_rows_kernel<W, V, ASYM, FORM>), grid, dim3(W * 64), 0, stream, p)
 #define DUQ_ROWS_CASE(W)                                                                                     \
     case W:                                                                                                  \
-        if (cached) {                                                                                        \
-            DUQ_ROWS_LAUNCH(W, true)                                                                         \
-        } else {                                                                                             \
-            DUQ_ROWS_LAUNCH(W, false)                                                                        \
-        }                                                                                                    \
+        if (held <= 1) DUQ_ROWS_LAUNCH(W, 1);                                                                \
+        else if (held <= 2) DUQ_ROWS_LAUNCH(W, 2);                                                           \
+        else if (held <= 4) DUQ_ROWS_LAUNCH(W, 4);                                                           \
+        else if constexpr (W < 16) return (int)hipErrorInvalidValue;  /* (waves_for: at most four) */        \
+        else if (held <= 8) DUQ_ROWS_LAUNCH(W, 8);                                                           \
+        else DUQ_ROWS_LAUNCH(W, 0);                                                                          \
         break;
     switch (waves) {
         DUQ_ROWS_CASE(1)
