@@ -309,6 +309,31 @@ struct Gemm8Params {
 };
 static_assert(offsetof(Gemm8Params, epi) == kHeadBytes, "the fields delivered in registers");
 
+// Outputs of prefill-sized tiles.  Descriptor of `rows` rows (at most 64: 32-bit offsets) from row m on: those past M are
+// beyond it.
+template <bool FUSED>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t out_rows(const Gemm8Params &p, uint32_t m, uint32_t rows)
+{
+    const uint32_t here = m < p.M ? min(p.M - m, rows) : 0u;
+    return make_rsrc(FUSED ? (const void *)(p.y + (uint64_t)m * p.N) : (const void *)(p.C + (uint64_t)m * p.N), here * p.N * 4);
+}
+// Four neighbouring outputs, columns n .. n + 3 (`whole`: all inside the row) of the descriptor's row `row`.  One store
+// without a branch, at whatever alignment the row has (the hardware splits it); the last columns of an N that is no multiple
+// of four one by one, on a branch that other widths do not take.  With four stores per lane for such N, and
+// a branch around every store that the conversion sank into: 2048 x 11007 x 4096 109.6 us, now 99.1; 700 x 8191 x 4096 34.8 / 28.6;
+// 2048 x 3001 x 512 18.2 / 13.7; and 2048 x 11008 x 4096 93.6 / 91.6, 4096 x 11008 x 4096 169 / 164.6, but 1500 x 5000 x 4096 34.6 /
+// 35.4 (2048 x 5000 x 2048 39.5 / 38.7).
+__device__ __forceinline__ void store_quad8(const Gemm8Params &p, __amdgpu_buffer_rsrc_t r, uint32_t row, uint32_t n, bool whole, v4i v)
+{
+    const uint32_t off = (row * p.N + n) * 4;
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), r, (int)(whole ? off : kOobOffset), 0, 2);
+    if (p.N % 4 != 0) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            __builtin_amdgcn_raw_buffer_store_b32((uint32_t)v[e], r, (int)(!whole && n + e < p.N ? off + e * 4 : kOobOffset), 0, 0);
+    }
+}
+
 __device__ __forceinline__ void lds_barrier8() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 template <int TM, int TN, bool FUSED, bool BIAS, bool TILED>
@@ -501,9 +526,7 @@ __global__ __launch_bounds__(256) void gemm_s8_kernel(DUQ_HEAD_DECL, Gemm8Params
     // bytes each.  Each wavefront turns its 32 x 64 block around in its own piece of LDS (the loop's buffers are free
     // after the last barrier) so that a store instruction writes whole rows of 256 (128) contiguous bytes.
     uint8_t *stage = lds + wave * (32 * kEStride);
-    const uint32_t n = n_out;
-    const void *outp = FUSED ? (const void *)p.y : (const void *)p.C;
-    const bool vec_ok = p.N % 4 == 0 && reinterpret_cast<uintptr_t>(outp) % 16 == 0;
+    const bool whole = n_out + 3 < p.N;
 #pragma unroll
     for (int b = 0; b < TM; ++b) {
 #pragma unroll
@@ -512,39 +535,22 @@ __global__ __launch_bounds__(256) void gemm_s8_kernel(DUQ_HEAD_DECL, Gemm8Params
             for (int q = 0; q < 4; ++q)
                 *reinterpret_cast<v4i *>(stage + l32 * kEStride + (t * 32 + q * 8 + h * 4) * 4) =
                     v4i{acc[t][b][q * 4], acc[t][b][q * 4 + 1], acc[t][b][q * 4 + 2], acc[t][b][q * 4 + 3]};
+        const uint32_t mb = m0 + b * 32;
+        const __amdgpu_buffer_rsrc_t rY = out_rows<FUSED>(p, mb, 32);
 #pragma unroll
         for (int it = 0; it < 32 / (int)kRowsPerStore; ++it) {
             const uint32_t row = it * kRowsPerStore + r4;
-            const v4i a = *reinterpret_cast<const v4i *>(stage + row * kEStride + c16 * 16);
-            const uint32_t m = m0 + b * 32 + row;
-            if (m >= p.M || n >= p.N) continue;
+            v4i a = *reinterpret_cast<const v4i *>(stage + row * kEStride + c16 * 16);
             if (FUSED) {
                 const float sr = row_par[0][b * 32 + row], zr = row_par[1][b * 32 + row];
-                v4f32 v;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     float o = dequant_hprec_one(a[r], sr, zr, sc[r], zc[r]);
                     if (BIAS) o = o + bs[r];
-                    v[r] = o;
-                }
-                float *dst = p.y + (uint64_t)m * p.N + n;
-                if (vec_ok && n + 3 < p.N) {
-                    __builtin_nontemporal_store(v, reinterpret_cast<v4f32 *>(dst));
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (n + r < p.N) dst[r] = v[r];
-                }
-            } else {
-                int32_t *dst = p.C + (uint64_t)m * p.N + n;
-                if (vec_ok && n + 3 < p.N) {
-                    __builtin_nontemporal_store(a, reinterpret_cast<v4i *>(dst));
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (n + r < p.N) dst[r] = a[r];
+                    a[r] = __builtin_bit_cast(int, o);
                 }
             }
+            store_quad8(p, rY, row, n_out, whole, a);
         }
     }
 }
@@ -685,33 +691,21 @@ __global__ __launch_bounds__(512) void gemm_s8_split_kernel(DUQ_HEAD_DECL, Gemm8
                 }
         __syncthreads();
     }
-    const void *outp = FUSED ? (const void *)p.y : (const void *)p.C;
-    const bool vec_ok = p.N % 4 == 0 && reinterpret_cast<uintptr_t>(outp) % 16 == 0;
+    const bool whole = n + 3 < p.N;
+    const __amdgpu_buffer_rsrc_t rY = out_rows<FUSED>(p, m0, 64);
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-        const uint32_t m = m0 + b * 32 + (tid >> 4);
-        if (m >= p.M || n >= p.N) continue;
         v4i a;
-        v4f32 v;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             a[r] = *at(cg >> 3, b, (cg >> 1) & 3u, r, (cg & 1u) * 32 + (tid >> 4));
             if (FUSED) {
-                v[r] = dequant_hprec_one(a[r], sr[b], zr[b], sc[r], zc[r]);
-                if (BIAS) v[r] = v[r] + bs[r];
+                float o = dequant_hprec_one(a[r], sr[b], zr[b], sc[r], zc[r]);
+                if (BIAS) o = o + bs[r];
+                a[r] = __builtin_bit_cast(int, o);
             }
         }
-        if (vec_ok) {  // (n is a multiple of four: the four columns end inside the row)
-            if (FUSED) __builtin_nontemporal_store(v, reinterpret_cast<v4f32 *>(p.y + (uint64_t)m * p.N + n));
-            else __builtin_nontemporal_store(a, reinterpret_cast<v4i *>(p.C + (uint64_t)m * p.N + n));
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (n + r < p.N) {
-                    if (FUSED) p.y[(uint64_t)m * p.N + n + r] = v[r];
-                    else p.C[(uint64_t)m * p.N + n + r] = a[r];
-                }
-        }
+        store_quad8(p, rY, b * 32 + (tid >> 4), n, whole, a);
     }
 }
 

@@ -59,3 +59,26 @@ def test_quantizer_inside_the_gemm(dev, M, N, K):
             for t in (None, tiled):
                 got = hip.quantize_linear8bit_forward(x, w, t, sw, zw, b)
                 assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (seed, b is None, t is None)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 2561, 64), (257, 2303, 96), (130, 5122, 64), (65, 4095, 1536), (70, 131, 1536), (640, 515, 64),
+                                   (8200, 2050, 32)])
+def test_ragged_columns_of_the_tiles(dev, M, N, K):
+    """Prefill-sized tiles whose rows end inside a group of four columns: every output against torch, none past the end."""
+    from duqlinear4bitcuda_amd import _HIP as hip
+    print("8-bit ragged", M, N, K, flush=True)
+    gen = torch.Generator(device=dev).manual_seed(N)
+    a = torch.randint(-128, 128, (M, K), generator=gen, device=dev, dtype=torch.int8)
+    w = torch.randint(-128, 128, (N, K), generator=gen, device=dev, dtype=torch.int8)
+    want = (a.double() @ w.double().T).to(torch.int32)   # (exact: |sum| < 2^53)
+    acc = hip.matmul_8bit(a, w)
+    assert torch.equal(acc, want)
+    sx, zx = torch.rand(M, generator=gen, device=dev), torch.randint(0, 127, (M,), generator=gen, device=dev).float()
+    sw, zw = torch.rand(N, generator=gen, device=dev), torch.randint(0, 127, (N,), generator=gen, device=dev).float()
+    bias = torch.randn(N, generator=gen, device=dev)
+    for b in (None, bias):
+        y = (sx[:, None] * sw) * (want.float() - (zx[:, None] + zw))
+        y = y if b is None else y + b
+        for t, wt in ((None, w), (N, hip.weight_tile_8bit(w))):
+            got = hip.linear8bit_forward(a, sx, zx, wt, sw, zw, b, tiled_rows=t)
+            assert torch.equal(got.view(torch.int32), y.view(torch.int32)), (b is None, t)
