@@ -96,7 +96,10 @@ inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 // Tile for a problem select_gemm_kernel gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
 // 64 x 128 tiles (duq_gemm.hip).  Whole rounds of 256 workgroups (one per CU) cost about f + c * (K / 256) microseconds
 // each, measured per tile shape (N = 4096, one round, K = 1024 / 4096 / 16384): 64 x 128 6.6 / 11.9 / 33, 128 x 128 8.9 /
-// 17.5 / 55, 128 x 256 12.5 / 30 / 100, 256 x 256 21 / 52.7 / 178 (1.3 of it once per launch); the cheapest wins.  64 x 64 and
+// 17.5 / 55, 128 x 256 12.5 / 30 / 100, 256 x 256 21 / 52.7 / 178 (1.3 of it once per launch); the cheapest wins.  192 x 128
+// tiles (11.5 / 25.4 / 80) in one round only, where larger ones would leave CUs without any (1536 x 4096 x 4096 28.4 -> 25.4 us,
+// x 16384 95 -> 80) and the walk over K is long enough for their end, stores of 64 bytes a row (2422 x 2312 x 1088 13.9 / 17.2).
+// 64 x 64 and
 // 96 x 64 tiles (128 rows; 65 rows) 5.9 / 8.7 / 22 and - / 10 / 22.6: in one round only, where they halve the walk over K;
 // two rounds of them are behind (512 x 4096 x 4096 17 against 12.4, 96 x 28672 x 8192 38 against 34.7).  96 x 64 against the
 // next best on 65..96 rows, 8200..16384 columns of 4096..8192 elements: 1 - 11 % ahead on 47 of 48 shapes, level on one (65 x
@@ -108,24 +111,50 @@ inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 struct StreamTile {
     uint32_t rows, cols;
     bool stream;
+    uint32_t main_cols = 0, rest_rows = 0;  // main_cols > 0: from that column on, tiles of rest_rows x 128
 };
+// Rounds that do not come out even: tiles of 128 x 256 over as many columns as fill whole rounds, and the columns that are
+// left in one round of smaller tiles, 192 x 128, 128 x 128 or 64 x 128, in the same launch (a launch of their own would start
+// when the last large tile has ended).  Taken where the model above has it 4 % ahead of every uniform choice; measured, in
+// turn: 2048 x 6144 x 4096 50.9 -> 46.4 us, 4000 x 8200 x 4160 150 -> 137, 1999 x 11008 x 4096 81.3 -> 79.7.  (192 x 256 tiles are
+// ahead of it there, 77.9, but behind on 3000 x 5000 x 2048 and 2500 x 12000 x 5120, 46.7 against 34.5 and 134 against 119.)
+// Of 75 shapes drawn at random (128..4096 rows, 700..20000 columns) it and the 192 x 128 tiles alone change fifteen, by 1.02 to
+// 1.34 (147 x 24961 x 14464); rows of less than 2048 elements lose by it (1234 x 6658 x 832 0.87).
+inline StreamTile with_rest(StreamTile best, float best_cost, uint32_t M, uint32_t N, float nch)
+{
+    const uint32_t tm = (M + 127) / 128, rounds = (uint32_t)((uint64_t)tm * ((N + 255) / 256) / 256), cols = rounds * 256 / tm * 256;
+    if (rounds == 0 || cols >= N || nch < 8.0f) return best;
+    best_cost *= 0.96f;
+    const uint32_t rm[3] = {192, 128, 64};
+    const float c_us[3] = {1.146f, 0.76f, 0.44f}, f_us[3] = {7.1f, 4.3f, 3.6f};
+    for (int k = 0; k < 3; ++k) {
+        if ((uint64_t)((M + rm[k] - 1) / rm[k]) * ((N - cols + 127) / 128) > 256) continue;
+        const float cost = (float)rounds * (nch * 1.47f + 5.5f) + nch * c_us[k] + f_us[k];
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = StreamTile{128, 256, false, cols, rm[k]};
+        }
+    }
+    return best;
+}
 inline StreamTile select_stream_tile(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, bool mode5)
 {
     const float nch = (float)((K + 255) / 256);
-    const uint32_t bm[6] = {64, 64, 96, 128, 128, 256}, bn[6] = {128, 64, 64, 128, 256, 256};
-    const float c_us[6] = {0.44f, 0.2f, 0.258f, 0.76f, 1.47f, 2.62f}, f_us[6] = {3.6f, 5.5f, 6.1f, 4.3f, 5.5f, 9.5f};
+    const uint32_t bm[7] = {64, 64, 96, 192, 128, 128, 256}, bn[7] = {128, 64, 64, 128, 128, 256, 256};
+    const float c_us[7] = {0.44f, 0.2f, 0.258f, 1.146f, 0.76f, 1.47f, 2.62f}, f_us[7] = {3.6f, 5.5f, 6.1f, 7.1f, 4.3f, 5.5f, 9.5f};
     auto tiles = [&](int k) { return (uint64_t)((M + bm[k] - 1) / bm[k]) * ((N + bn[k] - 1) / bn[k]) * batch; };
     StreamTile best{64, 128, true};
     float best_cost = (float)((tiles(0) + 255) / 256) * (nch * 0.62f + 0.9f) + 1.3f;
-    for (int k = 0; k < (mode5 ? 5 : 6); ++k) {
-        if (bn[k] == 64 && tiles(k) > 256) continue;
+    for (int k = 0; k < (mode5 ? 6 : 7); ++k) {
+        if ((bn[k] == 64 || bm[k] == 192) && tiles(k) > 256) continue;
+        if (bm[k] == 192 && nch < 8.0f) continue;
         const float cost = (float)((tiles(k) + 255) / 256) * (nch * c_us[k] + f_us[k]);
         if (cost < best_cost) {
             best_cost = cost;
             best = StreamTile{bm[k], bn[k], false};
         }
     }
-    return best;
+    return batch == 1 && !mode5 ? with_rest(best, best_cost, M, N, nch) : best;
 }
 inline bool decode_uses_rows_kernel(uint32_t M) { return M <= 4; }
 // MFMA decode kernel: one round of at most 256 workgroups, each with its share of the 16-column tiles.  The

@@ -34,19 +34,26 @@ constexpr int stages_of(int bytes) { return 147456 / bytes > 6 ? 6 : 147456 / by
 
 // WTM x WTN: 32 x 32 tiles of a wavefront.  WM x WN: wavefronts over the rows and columns of the workgroup's tile, KS of
 // them over k.  kRowB: bytes of a row in a stage (128 = 256 elements, or 256 where the tile is small: half the barriers).
-template <int WTM, int WTN, int WM, int WN, int KS, int kRowB, int EPI, bool BIAS>
-__global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, GemmParams tail)
+template <int WTM_, int WTN_, int WM_, int WN_, int KS_, int kRowB_>
+struct PrefillTile {
+    static constexpr int WTM = WTM_, WTN = WTN_, WM = WM_, WN = WN_, KS = KS_, kRowB = kRowB_;
+    static constexpr int BM = 32 * WTM * WM, BN = 32 * WTN * WN;
+    static constexpr int NST = stages_of((BM + BN) * kRowB);
+    static constexpr uint32_t kStage = (BM + BN) * kRowB;
+    static constexpr int TM = KS == 8 ? 1 : KS == 4 ? WTM / 2 : WTM, TN = KS == 1 ? WTN : WTN / 2;  // what a wavefront finishes after the loop
+    static constexpr uint32_t kEpiLds = 8 * (32 * TM) * (64 * TN + 16), kXchg = KS == 1 ? 0 : KS == 8 ? WTM * WTN * 4096 : 8 * (KS - 1) * TM * TN * 4096;
+    static constexpr uint32_t kLds = NST * kStage > kEpiLds ? (NST * kStage > kXchg ? NST * kStage : kXchg) : (kEpiLds > kXchg ? kEpiLds : kXchg);
+};
+
+// The tile of rows m0 .. and columns n0 ...  lds: Tile::kLds bytes; dpar, dwide: staged parameters of EPI 5.
+template <typename Tile, int EPI, bool BIAS>
+__device__ __forceinline__ void prefill_tile(GemmParams &p, uint8_t *lds, uint32_t *dpar, uint32_t &dwide, const uint32_t m0, const uint32_t n0)
 {
-    GemmParams p = with_head(tail, DUQ_HEAD_USE);
-    to_global(p.A);
-    to_global(p.B);
-    to_global(p.C);
-    to_global(p.y);
+    constexpr int WTM = Tile::WTM, WTN = Tile::WTN, WM = Tile::WM, WN = Tile::WN, KS = Tile::KS, kRowB = Tile::kRowB;
     static_assert(WM * WN * KS == 8, "eight wavefronts");
     static_assert(WTN >= 2 && 4 * (WTM + WTN) / (WTM * WTN) <= 4, "the last slot expands words of the last weight tile only");
-    constexpr int BM = 32 * WTM * WM, BN = 32 * WTN * WN;
-    constexpr int NST = stages_of((BM + BN) * kRowB);
-    constexpr uint32_t kStage = (BM + BN) * kRowB;
+    constexpr int BM = Tile::BM, BN = Tile::BN, NST = Tile::NST;
+    constexpr uint32_t kStage = Tile::kStage;
     constexpr int RPL = 1024 / kRowB, LPR = 64 / RPL;  // rows per load instruction, lanes per row
     constexpr int L = (BM + BN) / (8 * RPL);  // loads per wavefront and stage
     constexpr int LX = BM / (8 * RPL);               // ... of which bring activation rows
@@ -55,18 +62,8 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
     constexpr int P = WTM + WTN;              // fragments per step
     constexpr int W = 4 * P;                  // words a lane expands per step and parity
     constexpr int T = WTM * WTN;
-    constexpr int TM = KS == 8 ? 1 : KS == 4 ? WTM / 2 : WTM, TN = KS == 1 ? WTN : WTN / 2;  // what a wavefront finishes after the loop
+    constexpr int TM = Tile::TM, TN = Tile::TN;
     constexpr bool LATE = WTM * WTN == 8;     // no registers to spare in the loop: parameters after it
-    constexpr uint32_t kEpiLds = 8 * (32 * TM) * (64 * TN + 16), kXchg = KS == 1 ? 0 : KS == 8 ? T * 4096 : 8 * KS * TM * TN * 4096;
-    constexpr uint32_t kLds = NST * kStage > kEpiLds ? (NST * kStage > kXchg ? NST * kStage : kXchg) : (kEpiLds > kXchg ? kEpiLds : kXchg);
-    __shared__ __attribute__((aligned(256))) uint8_t lds[kLds];
-    __shared__ __attribute__((aligned(16))) uint32_t dpar[EPI == 5 ? (BN + BM) * 8 : 4];
-    __shared__ uint32_t dwide;
-
-    if (blockIdx.z) batch_shift(p, blockIdx.z);
-    uint32_t tile_m, tile_n;
-    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-    const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t l32 = lane & 31u, h = lane >> 5;
@@ -151,8 +148,12 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
     auto read = [&](int set, int f, int i, uint32_t stage) {
         raw[set][f] = *reinterpret_cast<const v4u *>(lds + stage + (f < WTM ? rx + f * 32 * kRowB : rw + (f - WTM) * 32 * kRowB) + pos[i]);
     };
+    // (expanded where it stands: an MFMA is opaque to the compiler, which may otherwise leave an expansion until right before
+    // the MFMA that reads it, where it would need two wait states)
     auto expand_word = [&](int par, int set, int f, int w) {
-        ex[par][f][w] = (par ? raw[set][f][w] : raw[set][f][w] << 4) & kNibbleMask;
+        uint32_t e = (par ? raw[set][f][w] : raw[set][f][w] << 4) & kNibbleMask;
+        asm volatile("" : "+v"(e));
+        ex[par][f][w] = e;
     };
 
     v16i accw[WTN][WTM];
@@ -309,7 +310,8 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
     } else {
         // the KS wavefronts of a tile share its outputs out: each hands the sums it does not finish to those that do
         auto at = [&](int dst, uint32_t src, int t, int b) {
-            return reinterpret_cast<v4i *>(lds + ((((uint32_t)dst * KS + src) * (WM * WN) + w4) * (TM * TN) + t * TM + b) * 4096) + lane;
+            const uint32_t from = src > (uint32_t)dst ? src - 1 : src;  // (nobody hands itself anything)
+            return reinterpret_cast<v4i *>(lds + ((((uint32_t)dst * (KS - 1) + from) * (WM * WN) + w4) * (TM * TN) + t * TM + b) * 4096) + lane;
         };
         __syncthreads();
 #pragma unroll
@@ -354,10 +356,74 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, Gem
 #include "duq_stream_epilogue_store.inc"
 }
 
+template <int WTM, int WTN, int WM, int WN, int KS, int kRowB, int EPI, bool BIAS>
+__global__ __launch_bounds__(512) void gemm_s4_prefill_kernel(DUQ_HEAD_DECL, GemmParams tail)
+{
+    using Tile = PrefillTile<WTM, WTN, WM, WN, KS, kRowB>;
+    GemmParams p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.A);
+    to_global(p.B);
+    to_global(p.C);
+    to_global(p.y);
+    __shared__ __attribute__((aligned(256))) uint8_t lds[Tile::kLds];
+    __shared__ __attribute__((aligned(16))) uint32_t dpar[EPI == 5 ? (Tile::BN + Tile::BM) * 8 : 4];
+    __shared__ uint32_t dwide;
+    if (blockIdx.z) batch_shift(p, blockIdx.z);
+    uint32_t tile_m, tile_n;
+    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    prefill_tile<Tile, EPI, BIAS>(p, lds, dpar, dwide, tile_m * Tile::BM, tile_n * Tile::BN);
+}
+
+using Tile64x128 = PrefillTile<2, 2, 1, 2, 4, 256>;
+using Tile128x128 = PrefillTile<2, 2, 2, 2, 2, 256>;
+using Tile192x128 = PrefillTile<3, 2, 2, 2, 2, 128>;
+using Tile128x256 = PrefillTile<2, 2, 2, 4, 1, 128>;
+
+// Rounds that do not come out even: p.tiles_m x p.tiles_n tiles of 128 x 256, as many as fill whole rounds of 256 workgroups,
+// and behind them the columns that are left in tiles of another kind.
+template <typename Rest, int EPI, bool BIAS>
+__global__ __launch_bounds__(512) void gemm_s4_prefill_mixed_kernel(DUQ_HEAD_DECL, GemmParams tail)
+{
+    using Tile = Tile128x256;
+    GemmParams p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.A);
+    to_global(p.B);
+    to_global(p.C);
+    to_global(p.y);
+    __shared__ __attribute__((aligned(256))) uint8_t lds[Tile::kLds > Rest::kLds ? Tile::kLds : Rest::kLds];
+    uint32_t none = 0, tile_m, tile_n;
+    const uint32_t whole = p.tiles_m * p.tiles_n;
+    if (blockIdx.x < whole) {
+        tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+        prefill_tile<Tile, EPI, BIAS>(p, lds, &none, none, tile_m * Tile::BM, tile_n * Tile::BN);
+    } else {
+        const uint32_t n1 = p.tiles_n * Tile::BN;
+        tile_of_block(blockIdx.x - whole, (p.M + Rest::BM - 1) / Rest::BM, (p.N - n1 + Rest::BN - 1) / Rest::BN, tile_m, tile_n);
+        prefill_tile<Rest, EPI, BIAS>(p, lds, &none, none, tile_m * Rest::BM, n1 + tile_n * Rest::BN);
+    }
+}
+
+// Whole rounds of 128 x 256 tiles over the first tile.main_cols columns, the rest in other tiles behind them.
+template <typename Rest, int EPI, bool BIAS>
+static int launch_mixed(GemmParams &p, const StreamTile &tile, hipStream_t stream)
+{
+    p.tiles_m = (p.M + 127) / 128;
+    p.tiles_n = tile.main_cols / 256;
+    const uint32_t rest = ((p.M + Rest::BM - 1) / Rest::BM) * ((p.N - tile.main_cols + Rest::BN - 1) / Rest::BN);
+    DUQ_LAUNCH_HEAD((gemm_s4_prefill_mixed_kernel<Rest, EPI, BIAS>), dim3(p.tiles_m * p.tiles_n + rest), dim3(512), 0, stream, p);
+    return (int)hipGetLastError();
+}
+
 template <int EPI, bool BIAS>
 static int launch_prefill_epi(GemmParams &p, StreamTile tile, hipStream_t stream, uint32_t batch)
 {
     const uint32_t bm = tile.rows, bn = tile.cols;
+    if constexpr (EPI >= 0 && EPI != 5) {
+        if (tile.main_cols)
+            return tile.rest_rows == 192   ? launch_mixed<Tile192x128, EPI, BIAS>(p, tile, stream)
+                   : tile.rest_rows == 128 ? launch_mixed<Tile128x128, EPI, BIAS>(p, tile, stream)
+                                           : launch_mixed<Tile64x128, EPI, BIAS>(p, tile, stream);
+    }
     p.tiles_m = (p.M + bm - 1) / bm;
     p.tiles_n = (p.N + bn - 1) / bn;
     const dim3 grid(p.tiles_m * p.tiles_n, 1, batch);
@@ -367,6 +433,8 @@ static int launch_prefill_epi(GemmParams &p, StreamTile tile, hipStream_t stream
         DUQ_LAUNCH_HEAD((gemm_s4_prefill_kernel<3, 2, 1, 1, 8, 256, EPI, BIAS>), grid, dim3(512), 0, stream, p);
     else if (bm == 64 && bn == 128)
         DUQ_LAUNCH_HEAD((gemm_s4_prefill_kernel<2, 2, 1, 2, 4, 256, EPI, BIAS>), grid, dim3(512), 0, stream, p);
+    else if (bm == 192 && bn == 128)
+        DUQ_LAUNCH_HEAD((gemm_s4_prefill_kernel<3, 2, 2, 2, 2, 128, EPI, BIAS>), grid, dim3(512), 0, stream, p);
     else if (bm == 128 && bn == 128)
         DUQ_LAUNCH_HEAD((gemm_s4_prefill_kernel<2, 2, 2, 2, 2, 256, EPI, BIAS>), grid, dim3(512), 0, stream, p);
     else if (bm == 128 && bn == 256)

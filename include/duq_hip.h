@@ -229,7 +229,8 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
  * N * K / 2 < 2^32 - 256; larger tensors run families 6 and 7, whose bases are 64-bit per tile.  No
  * counterpart in the reference (CUTLASS picks its own tile, src/kernels/gemm.cu:17-42). */
 int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
-/* For a shape of family 6: its tile as rows * 1000 + columns (256256, 128256, 128128, 64128, 96064, 64064); 0 for the other families.  (The dual-uniform row-sum epilogue never runs the 256-row tile.) */
+/* For a shape of family 6: its tile as rows * 1000 + columns (256256, 128256, 192128, 128128, 64128, 96064, 64064; the fused
+ * entry points may cover the last columns of a problem in smaller tiles); 0 for the other families.  (The dual-uniform row-sum epilogue never runs the 256-row tile.) */
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
 
 /* Measurement aid, no counterpart in the reference: reads `bytes` (16-byte aligned, < 4 GiB) of device memory
