@@ -336,37 +336,33 @@ __device__ __forceinline__ void store_quad8(const Gemm8Params &p, __amdgpu_buffe
 
 __device__ __forceinline__ void lds_barrier8() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+template <int TM, int TN>
+struct Tile8 {
+    static constexpr int BM = 32 * TM, BN = 128 * TN;
+    // steps (of 32 k) per chunk: 8, or 4 with 256-row tiles (TM = 8: all 256 accumulation registers hold accumulators
+    // and three activation buffers of 256-k chunks would not fit in LDS)
+    static constexpr int NS = TM == 8 ? 4 : 8;
+    static constexpr uint32_t kStride = 32 * NS + 16, kEStride = 32 * TN * 4 + 16;  // epilogue staging: 32 rows of 32*TN int32 per wavefront
+    static constexpr uint32_t kLds = 3 * BM * kStride > 4 * 32 * kEStride ? 3 * BM * kStride : 4 * 32 * kEStride;
+};
+
+// The tile of rows m0 .. and columns n0 ...  lds: Tile8::kLds bytes; row_par: [2][BM], its per-row scale and zero point.
 template <int TM, int TN, bool FUSED, bool BIAS, bool TILED>
-__global__ __launch_bounds__(256) void gemm_s8_kernel(DUQ_HEAD_DECL, Gemm8Params tail)
+__device__ __forceinline__ void gemm8_tile(const Gemm8Params &p, uint8_t *lds, float *row_par, const uint32_t m0, const uint32_t n0)
 {
-    Gemm8Params p = with_head(tail, DUQ_HEAD_USE);
-    to_global(p.A);
-    to_global(p.B);
-    to_global(p.C);
-    to_global(p.y);
-    static_assert(TM == 8 || TM == 4 || TM == 2 || TM == 1, "32-row MFMA tiles per wavefront along M");
+    static_assert(TM == 8 || TM == 4 || TM == 3 || TM == 2 || TM == 1, "32-row MFMA tiles per wavefront along M");
     // TN = 32-column MFMA tiles per wavefront: tiles of 256 columns (TN = 2), or of 128 (TN = 1, with 64-row tiles:
     // twice the workgroups for problems that leave CUs without a 64 x 256 tile)
     static_assert(TN == 2 || (TN == 1 && TM == 2), "column tiles per wavefront");
-    constexpr int BM = 32 * TM, BN = 128 * TN;
-    // steps (of 32 k) per chunk: 8, or 4 with 256-row tiles (TM = 8: all 256 accumulation registers hold accumulators
-    // and three activation buffers of 256-k chunks would not fit in LDS)
-    constexpr int NS = TM == 8 ? 4 : 8;
+    constexpr int BM = Tile8<TM, TN>::BM, BN = Tile8<TM, TN>::BN, NS = Tile8<TM, TN>::NS;
     constexpr uint32_t kChunk = 32 * NS;  // 256 (128)
-    constexpr uint32_t kStride = kChunk + 16;
+    constexpr uint32_t kStride = Tile8<TM, TN>::kStride;
     constexpr uint32_t kBuf = BM * kStride;
     constexpr int PPR = kChunk / 16;      // 16-byte pieces per row of a chunk
     constexpr int NXP = BM * PPR / 256;   // 16-byte activation pieces per thread and chunk: 8, 4, 2 (TM = 8: 8)
 
-    constexpr uint32_t kEStride = 32 * TN * 4 + 16;  // epilogue staging: 32 rows of 32*TN int32 per wavefront
-    constexpr uint32_t kLds = 3 * kBuf > 4 * 32 * kEStride ? 3 * kBuf : 4 * 32 * kEStride;
+    constexpr uint32_t kEStride = Tile8<TM, TN>::kEStride;
 
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
-    __shared__ float row_par[2][BM];  // the tile's per-row scale and zero point, fetched before the loop
-
-    uint32_t tile_m, tile_n;
-    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-    const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     const uint32_t l32 = lane & 31u, h = lane >> 5;
@@ -426,8 +422,8 @@ __global__ __launch_bounds__(256) void gemm_s8_kernel(DUQ_HEAD_DECL, Gemm8Params
     if (FUSED) {
         if (tid < BM) {
             const uint32_t m = min(m0 + tid, p.M - 1);
-            row_par[0][tid] = p.epi.s_row[m];
-            row_par[1][tid] = p.epi.z_row[m];
+            row_par[tid] = p.epi.s_row[m];
+            row_par[BM + tid] = p.epi.z_row[m];
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -542,7 +538,7 @@ __global__ __launch_bounds__(256) void gemm_s8_kernel(DUQ_HEAD_DECL, Gemm8Params
             const uint32_t row = it * kRowsPerStore + r4;
             v4i a = *reinterpret_cast<const v4i *>(stage + row * kEStride + c16 * 16);
             if (FUSED) {
-                const float sr = row_par[0][b * 32 + row], zr = row_par[1][b * 32 + row];
+                const float sr = row_par[b * 32 + row], zr = row_par[BM + b * 32 + row];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     float o = dequant_hprec_one(a[r], sr, zr, sc[r], zc[r]);
@@ -552,6 +548,47 @@ __global__ __launch_bounds__(256) void gemm_s8_kernel(DUQ_HEAD_DECL, Gemm8Params
             }
             store_quad8(p, rY, row, n_out, whole, a);
         }
+    }
+}
+
+template <int TM, int TN, bool FUSED, bool BIAS, bool TILED>
+__global__ __launch_bounds__(256) void gemm_s8_kernel(DUQ_HEAD_DECL, Gemm8Params tail)
+{
+    Gemm8Params p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.A);
+    to_global(p.B);
+    to_global(p.C);
+    to_global(p.y);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[Tile8<TM, TN>::kLds];
+    __shared__ float row_par[2 * Tile8<TM, TN>::BM];
+    uint32_t tile_m, tile_n;
+    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    gemm8_tile<TM, TN, FUSED, BIAS, TILED>(p, lds, row_par, tile_m * Tile8<TM, TN>::BM, tile_n * Tile8<TM, TN>::BN);
+}
+
+// Rounds that do not come out even: p.tiles_m x p.tiles_n tiles of 128 x 256, as many as fill whole rounds of 256 workgroups,
+// and behind them the columns that are left in tiles of 32 * TM x 128 * TN.
+template <int TM, int TN, bool BIAS, bool TILED>
+__global__ __launch_bounds__(256) void gemm_s8_mixed_kernel(DUQ_HEAD_DECL, Gemm8Params tail)
+{
+    Gemm8Params p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.A);
+    to_global(p.B);
+    to_global(p.C);
+    to_global(p.y);
+    using Rest = Tile8<TM, TN>;
+    static_assert(TM < 4, "fits beside nothing larger than the 128 x 256 tile's share of LDS");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[Tile8<4, 2>::kLds];
+    __shared__ float row_par[2 * 128];
+    const uint32_t whole = p.tiles_m * p.tiles_n;
+    uint32_t tile_m, tile_n;
+    if (blockIdx.x < whole) {
+        tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+        gemm8_tile<4, 2, true, BIAS, TILED>(p, lds, row_par, tile_m * 128, tile_n * 256);
+    } else {
+        const uint32_t n1 = p.tiles_n * 256;
+        tile_of_block(blockIdx.x - whole, (p.M + Rest::BM - 1) / Rest::BM, (p.N - n1 + Rest::BN - 1) / Rest::BN, tile_m, tile_n);
+        gemm8_tile<TM, TN, true, BIAS, TILED>(p, lds, row_par, tile_m * Rest::BM, n1 + tile_n * Rest::BN);
     }
 }
 
@@ -1230,6 +1267,66 @@ inline bool split8_takes(uint32_t M, uint32_t N, uint32_t K)
 #ifndef DUQ_S8_COST256
 #define DUQ_S8_COST256 1.95f
 #endif
+// More than 64 rows on at least 160 tiles of 128 x 256.  A round of 256 workgroups lasts as long as its tile, however few
+// tiles it has: about f + c * (K / 256) microseconds, measured (one round, K = 1024 / 4096): 128 x 256 14.8 / 34.5, 96 x 256 12.7 /
+// 28.2, 64 x 256 10.6 / 23.2, 64 x 128 6.8 / 14.4; the constants below are of a round among others.  So the cheapest of: 128 x 256 tiles; 96 x 256 tiles (2000 x 6000 x 4096 62.5 -> 54.5
+// us, 1536 x 4096 x 4096 30.7 -> 28.2); and, where rows are long enough for the ends not to decide and the model has it 5 % ahead,
+// whole rounds of 128 x 256 tiles with the columns that are left in one round of smaller tiles behind them, in the same launch
+// (2048 x 11008 x 4096 100.4 -> 94.3, 2048 x 5000 x 8192 105 -> 84.5, 1024 x 11008 x 4096 61 -> 52).
+struct Plan8 {
+    uint32_t rows;                                        // 128 or 96
+    uint32_t cols = 0, rest_rows = 0, rest_cols = 0;      // cols > 0: tiles of 256 columns in whole rounds, and the rest's tile
+};
+inline Plan8 plan_gemm8(uint32_t M, uint32_t N, uint32_t K, bool fused)
+{
+    const float n = (float)((K + 255) / 256);
+    auto tiles = [&](uint32_t rows, uint32_t width, uint32_t from) { return ((M + rows - 1) / rows) * ((N - from + width - 1) / width); };
+    auto rounds = [&](uint32_t t) { return (float)((t + 255) / 256); };
+    const float round = n * 1.67f + 6.8f, c128 = rounds(tiles(128, 256, 0)) * round, c96 = rounds(tiles(96, 256, 0)) * (n * 1.29f + 5.4f);
+    Plan8 best{c96 < c128 ? 96u : 128u};
+    float cost = 0.95f * std::min(c96, c128);
+    const uint32_t tm = (M + 127) / 128, whole = tiles(128, 256, 0) / 256, cols = whole * 256 / tm;
+    if (!fused || whole == 0 || cols * 256 >= N || K < 2048) return best;
+    const uint32_t rr[3] = {96, 64, 64}, rc[3] = {256, 256, 128};
+    const float c_us[3] = {1.29f, 1.05f, 0.63f}, f_us[3] = {7.5f, 6.4f, 4.4f};
+    for (int k = 0; k < 3; ++k) {
+        const float c = (float)whole * round + n * c_us[k] + f_us[k];
+        if (tiles(rr[k], rc[k], cols * 256) <= 256 && c < cost) {
+            cost = c;
+            best = Plan8{128, cols, rr[k], rc[k]};
+        }
+    }
+    return best;
+}
+
+template <bool FUSED, bool BIAS, bool TILED>
+static void launch_plan8(Gemm8Params &p, hipStream_t stream)
+{
+    const Plan8 plan = plan_gemm8(p.M, p.N, p.K, FUSED);
+    p.tiles_m = (p.M + plan.rows - 1) / plan.rows;
+    p.tiles_n = (p.N + 255) / 256;
+    if constexpr (FUSED) {
+        if (plan.cols) {
+            p.tiles_n = plan.cols;
+            const uint32_t left = p.N - plan.cols * 256;
+            const dim3 grid(p.tiles_m * p.tiles_n +
+                            ((p.M + plan.rest_rows - 1) / plan.rest_rows) * ((left + plan.rest_cols - 1) / plan.rest_cols));
+            if (plan.rest_rows == 96)
+                DUQ_LAUNCH_HEAD((gemm_s8_mixed_kernel<3, 2, BIAS, TILED>), grid, dim3(256), 0, stream, p);
+            else if (plan.rest_cols == 256)
+                DUQ_LAUNCH_HEAD((gemm_s8_mixed_kernel<2, 2, BIAS, TILED>), grid, dim3(256), 0, stream, p);
+            else
+                DUQ_LAUNCH_HEAD((gemm_s8_mixed_kernel<2, 1, BIAS, TILED>), grid, dim3(256), 0, stream, p);
+            return;
+        }
+    }
+    const dim3 grid(p.tiles_m * p.tiles_n);
+    if (plan.rows == 96)
+        DUQ_LAUNCH_HEAD((gemm_s8_kernel<3, 2, FUSED, BIAS, TILED>), grid, dim3(256), 0, stream, p);
+    else
+        DUQ_LAUNCH_HEAD((gemm_s8_kernel<4, 2, FUSED, BIAS, TILED>), grid, dim3(256), 0, stream, p);
+}
+
 template <bool FUSED, bool BIAS, bool TILED>
 static void launch_gemm8_variant(Gemm8Params &p, hipStream_t stream)
 {
@@ -1267,8 +1364,7 @@ static void launch_gemm8_variant(Gemm8Params &p, hipStream_t stream)
         p.tiles_m = (p.M + 255) / 256;
         DUQ_LAUNCH_HEAD((gemm_s8_kernel<8, 2, FUSED, BIAS, TILED>), dim3(p.tiles_m * p.tiles_n), dim3(256), 0, stream, p);
     } else if (p.M > 64 && t128 >= 160) {
-        p.tiles_m = (p.M + 127) / 128;
-        DUQ_LAUNCH_HEAD((gemm_s8_kernel<4, 2, FUSED, BIAS, TILED>), dim3(p.tiles_m * p.tiles_n), dim3(256), 0, stream, p);
+        launch_plan8<FUSED, BIAS, TILED>(p, stream);
     } else if (p.M > 32 && t64 >= 48) {
         p.tiles_m = (p.M + 63) / 64;
         // one round of 64 x 256 tiles would leave CUs idle: 64 x 128 tiles, twice as many (measured 21-24 % faster at

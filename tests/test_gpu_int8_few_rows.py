@@ -82,3 +82,10 @@ def test_ragged_columns_of_the_tiles(dev, M, N, K):
         for t, wt in ((None, w), (N, hip.weight_tile_8bit(w))):
             got = hip.linear8bit_forward(a, sx, zx, wt, sw, zw, b, tiled_rows=t)
             assert torch.equal(got.view(torch.int32), y.view(torch.int32)), (b is None, t)
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 11008, 2048), (1999, 11007, 2080),    # 96 x 256 tiles behind whole rounds
+                                   (2040, 6100, 4096),                          # 96 x 256 tiles alone
+                                   (1024, 10500, 4096), (1950, 5005, 4096), (2048, 8300, 2112)])  # 64 x 256, 64 x 128 behind
+def test_uneven_rounds_of_the_tiles(dev, M, N, K):
+    test_ragged_columns_of_the_tiles(dev, M, N, K)
