@@ -461,7 +461,7 @@ int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K) { return duq::select
 
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K)
 {
-    if (duq::select_gemm_kernel(M, N, K) != duq::kKernelStream) return 0;
+    if (duq::select_gemm_kernel(M, N, K) != duq::kKernelStream || duq::takes_lds_kernel(M, N, K)) return 0;
     const duq::StreamTile t = duq::select_stream_tile(M, N, K, 1, false);
     return (int)(t.rows * 1000 + t.cols);
 }

@@ -1,10 +1,10 @@
-// Decode kernels (M <= 64 activation rows, K <= 16384): weight streaming for problems of a few MB,
+// Decode kernels (M <= 64 activation rows): weight streaming for problems of a few MB,
 // where a launch lives for two or three microseconds and what counts is that every byte is requested
 // in the kernel's first instructions and nothing else sits on the critical path.
 //
 //   C[m,n] = sum_k s4(A[m,k]) * s4(B[n,k])        (src/kernels/gemm.cu:8-43 of the reference, at M <= 16)
 //
-// Both kernels
+// The first two
 //  * issue every weight load of the workgroup before anything else (no ring: the whole share of a
 //    workgroup, 16-32 KB, is in flight at once),
 //  * fetch the epilogue parameters of the outputs a lane will store right behind them, so that no
@@ -20,9 +20,11 @@
 //    whole K range: lane l holds bytes [i*1024 + l*16, +16) of each row, so a load instruction covers 1 KB
 //    of one row and an activation register serves four rows.  The 4*M partial sums of a lane meet the other
 //    lanes' through the wavefront's own piece of LDS (no barrier) and a few DPP steps.
-//  MFMA kernel (5 <= M <= 64): v_mfma_i32_16x16x64_i8, eight wavefronts split K for one 16-column tile, one to
+//  MFMA kernel (5 <= M <= 64, several column tiles per CU, K <= 8192): v_mfma_i32_16x16x64_i8, eight wavefronts split K for one 16-column tile, one to
 //    four tiles of 16 rows against the same weight fragments, the partial tiles meet in LDS, 256 threads finish
 //    one output each per row tile; one round of at most 256 workgroups with several column tiles each.
+//  LDS kernel (M <= 64, one or two column tiles per workgroup, any K): the same MFMAs, both operands through LDS in whole
+//    cache lines, K in a loop.
 #include <cstddef>
 
 #include "duq_epilogue.h"
@@ -477,7 +479,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_s4_rows_kernel(DUQ_HEAD_DECL,
 // 16 / WAVES whole rows per wavefront (so a row's statistics never leave its wavefront), into LDS; the fragments
 // then come from there.  Every workgroup repeats that work: it pays while the quantizer's own launch (about 2.6 us
 // with the wait between the two) costs more than sixteen rows on a CU's vector units.
-template <int WAVES, int SEGS, int EPI, int MT = 1, bool DB = true, bool FUSEQ = false>
+template <int WAVES, int SEGS, int EPI, int MT = 1, bool FUSEQ = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DECL, DecodeParams tail)
 {
     const DecodeParams p = with_head(tail, DUQ_HEAD_USE);
@@ -548,7 +550,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DEC
         // every wavefront requests its activations before any requests weights (requests are served in order)
         __builtin_amdgcn_s_barrier();
     }
-    v4u w0[SEGS], w1[DB ? SEGS : 1];
+    v4u w0[SEGS], w1[SEGS];
     load_tile(tile0, w0);
 
     // threads finish one output per row tile they own: element er of MFMA lane src_lane; the 256-thread group
@@ -713,19 +715,191 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DEC
     };
 
     // two register sets alternate so that one tile's loads are in flight during the other's MFMAs; the
-    // partial-sum buffers alternate too: one barrier per tile.  (DB = false: one set, for the long rows whose
-    // fragments leave no room for a second; their layers have at most 256 column tiles, one per workgroup.)
-    if constexpr (DB) {
-        for (uint32_t t = tile0; t < tile_end; t += 2) {
-            load_tile(t + 1, w1);
-            compute_tile(t, w0, 0);
-            load_tile(t + 2, w0);
-            if (t + 1 < tile_end) compute_tile(t + 1, w1, 1);
+    // partial-sum buffers alternate too: one barrier per tile
+    for (uint32_t t = tile0; t < tile_end; t += 2) {
+        load_tile(t + 1, w1);
+        compute_tile(t, w0, 0);
+        load_tile(t + 2, w0);
+        if (t + 1 < tile_end) compute_tile(t + 1, w1, 1);
+    }
+}
+
+// ---------------------------------------------------------------------------------
+// LDS kernel: up to 64 rows of any length (what takes_lds_kernel gives it)
+// ---------------------------------------------------------------------------------
+// A fragment of the MFMA takes sixteen bytes of each of sixteen rows from sixteen neighbouring lanes, and a load in that
+// layout touches a cache line per lane: the kernel above requests its operands at about 29 bytes per ns and CU, a quarter of
+// what a CU can take in (131 KB a workgroup at 16 x 4096 x 8192), and a launch of few rows lasts as long as that.  Here both
+// operands come through LDS without registers, in instructions of whole 128- or 512-byte pieces of a row; eight wavefronts
+// split K, each reads its fragments out of LDS, and the walk over K is a loop, so that rows may be of any length.  Sixteen
+// columns per workgroup (up to 4096 columns, one round of workgroups): a wavefront's stages are its own, 128 bytes of every
+// kilobyte of a row, and nothing waits for another wavefront until the sums meet.  32 columns (up to 8192 in one round): the
+// activations are a third less of what enters a CU, and the wavefronts share stages of 512 bytes a row, which 64 rows need
+// (8192 x 28672: 29 us against 42 with 64-byte pieces of their own, which are half lines).  Measured against what ran before
+// (N x K, us): 16 rows 4096 x 4096 4.1 -> 3.8, x 8192 6.9 -> 5.5, x 11008 8.5 -> 6.2, 2606 x 26944 31.9 -> 14.1, 8192 x 28672
+// 31.0 -> 21.3; 64 rows 7.4 -> 5.7, 11.2 -> 8.0, 15.2 -> 10.4, 40.6 -> 27.4, 39.2 -> 29.1.
+template <int MT, int NT>
+struct LdsTile {
+    static constexpr int G = NT == 1 ? 1 : 8;            // wavefronts that share a stage
+    static constexpr int RB = G == 1 ? 128 : 512;        // bytes of a row in it
+    static constexpr int DEPTH = G == 1 ? 2 : 3;         // stages
+    static constexpr int U = RB / (64 * G);              // a wavefront's 64-byte fragments of a row in a stage
+    static constexpr int L = (MT + NT) * U;              // load instructions of a wavefront and stage, a kilobyte each
+    static constexpr int kStage = G * L * 1024, kLds = 8 / G * DEPTH * kStage, kPart = NT * MT * 8 * 1024;
+    static_assert(kLds <= 160 * 1024 && kPart <= kLds, "LDS");
+};
+template <int MT, int NT, int EPI>
+__global__ __launch_bounds__(512) void gemm_s4_lds_kernel(DUQ_HEAD_DECL, DecodeParams tail)
+{
+    const DecodeParams p = with_head(tail, DUQ_HEAD_USE);
+    using Tile = LdsTile<MT, NT>;
+    constexpr int MODE = EPI < 0 ? 0 : EPI;
+    constexpr int WAVES = 8, G = Tile::G, U = Tile::U, L = Tile::L, DEPTH = Tile::DEPTH, NG = WAVES / 4;
+    constexpr uint32_t RB = Tile::RB, kStage = Tile::kStage;
+    constexpr int FT = (MT * NT + NG - 1) / NG;  // output tiles a group of 256 threads finishes
+    static_assert(DEPTH >= 2 && DEPTH * L <= 63, "vmcnt");
+    __shared__ __attribute__((aligned(256))) uint8_t lds[Tile::kLds];
+    using ColRec = typename EpiRec<MODE>::Col;
+    using RowRec = typename EpiRec<MODE>::Row;
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t l16 = lane & 15u, g = lane >> 4;
+    const uint32_t kbytes = p.K >> 1;
+    const uint32_t col0 = blockIdx.x * (16 * NT);
+    const auto desc = [](const uint8_t *base, uint32_t bytes) {
+        const uint64_t a = reinterpret_cast<uint64_t>(base);
+        return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
+                   (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+    };
+    const v4u dX = desc(p.A, p.M * kbytes);  // rows past M and N read as zero
+    const v4u dW = desc(p.B + (uint64_t)col0 * kbytes, min(p.N - col0, 16u * NT) * kbytes);
+
+    // ---- global -> LDS: instruction j of a group's wavefront v takes kilobyte j * G + v of the stage, activations first; a
+    // row's 16-byte pieces lie at piece ^ (row / Q), so that the sixteen rows of a fragment read sixteen places
+    constexpr uint32_t PR = RB / 16, RPI = 64 / PR, Q = RB < 256 ? 256 / RB : 1;  // pieces a row, rows an instruction
+    const uint32_t group = G == 1 ? wave : 0, v = G == 1 ? 0 : wave;
+    const uint32_t r0 = v * RPI + lane / PR, row0 = r0 * kbytes;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds + group * (DEPTH * kStage) + v * 1024;
+    auto load = [&](uint32_t step, uint32_t slot) {
+        const uint32_t k = (step * (WAVES / G) + group) * RB;
+        uint32_t at[2];  // (of even and odd instructions: rows 16 apart swizzle alike)
+        bool in[2];
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+            at[o] = k + ((lane % PR) ^ ((o * (G * RPI) + r0) % 16 / Q)) * 16;
+            in[o] = at[o] < kbytes;  // K % 64 == 0: a 16-byte piece is all in or all out
         }
-    } else {
-        for (uint32_t t = tile0; t < tile_end; ++t) {
-            if (t != tile0) load_tile(t, w0);
-            compute_tile(t, w0, (t - tile0) & 1u);
+#pragma unroll
+        for (int j = 0; j < L; ++j) {
+            const uint32_t rows = (j < MT * U ? j : j - MT * U) * (G * RPI);
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds0 + slot + j * (G * 1024)),
+                         "v"(in[j % 2] ? row0 + rows * kbytes + at[j % 2] : kOobOffset), "s"(j < MT * U ? dX : dW)
+                         : "memory", "m0");
+        }
+    };
+    static_assert(G * RPI == 8 || G * RPI == 16, "the two swizzles above");
+    // ---- LDS -> registers: 64 bytes of a row make a fragment (two MFMAs)
+    v4u x[MT][U], w[NT][U];
+    const uint8_t *const own = lds + group * (DEPTH * kStage) + l16 * RB;
+    auto read = [&](uint32_t slot) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint8_t *const at = own + slot + (((v * U + u) * 4 + g) ^ (l16 / Q)) * 16;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) w[n][u] = *reinterpret_cast<const v4u *>(at + (MT + n) * (16 * RB));
+#pragma unroll
+            for (int m = 0; m < MT; ++m) x[m][u] = *reinterpret_cast<const v4u *>(at + m * (16 * RB));
+        }
+    };
+    v4i acc[NT][MT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[n][m] = v4i{0, 0, 0, 0};
+    auto compute = [&]() {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v4u we[NT], wo[NT];
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    we[n][q] = (w[n][u][q] << 4) & kNibbleMaskD;
+                    wo[n][q] = w[n][u][q] & kNibbleMaskD;
+                }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                v4u xe, xo;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    xe[q] = (x[m][u][q] << 4) & kNibbleMaskD;
+                    xo[q] = x[m][u][q] & kNibbleMaskD;
+                }
+#pragma unroll
+                for (int n = 0; n < NT; ++n) {
+                    acc[n][m] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, we[n]), __builtin_bit_cast(v4i, xe), acc[n][m], 0, 0, 0);
+                    acc[n][m] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, wo[n]), __builtin_bit_cast(v4i, xo), acc[n][m], 0, 0, 0);
+                }
+            }
+        }
+    };
+    const uint32_t steps = (kbytes + WAVES / G * RB - 1) / (WAVES / G * RB);
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s) load(s, s * kStage);
+
+    // the parameters of the outputs this thread finishes, behind the first steps' operands
+    const uint32_t src_lane = (tid >> 2) & 63u, er = tid & 3u, fg = tid >> 8;
+    const uint32_t my_m = src_lane & 15u, my_c = (src_lane >> 4) * 4 + er;
+    const bool bias = p.epi.bias != nullptr;
+    const auto c_out = as_global(p.C);
+    const auto y_out = as_global(p.y);
+    ColRec cp[FT];
+    RowRec rp[FT];
+#pragma unroll
+    for (int f = 0; f < FT; ++f) {
+        const uint32_t t = min(fg + NG * f, (uint32_t)(MT * NT - 1));
+        cp[f] = ColRec{};
+        rp[f] = RowRec{};
+        if (EPI >= 0) {
+            cp[f] = load_col_rt<MODE>(p.epi, min(col0 + t / MT * 16 + my_c, p.N - 1), bias, p.B, kbytes);
+            rp[f] = load_row_rt<MODE>(p.epi, min(t % MT * 16 + my_m, p.M - 1), p.A, kbytes);
+        }
+    }
+    uint32_t slot = 0;
+    for (uint32_t st = 0; st < steps; ++st) {
+        // this step's loads are here (those of the next DEPTH - 1 may be in flight; other loads only make the wait longer)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * L) : "memory");
+        if (G > 1) asm volatile("s_barrier" ::: "memory");  // (and everybody's)
+        read(slot);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the place takes the step DEPTH further on
+        if (G > 1) asm volatile("s_barrier" ::: "memory");
+        load(st + DEPTH, slot);
+        compute();
+        slot = slot + kStage == DEPTH * kStage ? 0 : slot + kStage;
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    v4i *const part = reinterpret_cast<v4i *>(lds);
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) part[((n * MT + m) * WAVES + wave) * 64 + lane] = acc[n][m];
+    __syncthreads();
+    const int *const sums = reinterpret_cast<const int *>(lds) + src_lane * 4 + er;
+#pragma unroll
+    for (int f = 0; f < FT; ++f) {
+        const uint32_t t = fg + NG * f;
+        if (t < (uint32_t)(MT * NT)) {
+            int sum = 0;
+#pragma unroll
+            for (int v = 0; v < WAVES; ++v) sum += sums[(t * WAVES + v) * 256];
+            sum >>= 8;
+            const uint32_t m = t % MT * 16 + my_m, n = col0 + t / MT * 16 + my_c;
+            if (m < p.M && n < p.N) {
+                if (EPI < 0)
+                    c_out[(uint64_t)m * p.N + n] = sum;
+                else
+                    y_out[(uint64_t)m * p.N + n] = dequant_rt<MODE>(sum, rp[f], cp[f], bias);
+            }
         }
     }
 }
@@ -796,13 +970,13 @@ bool launch_rows_xs(DecodeParams &p, int epi, hipStream_t stream)
     return false;
 }
 
-template <int WAVES, int SEGS, int MT = 1, bool DB = true, bool FUSEQ = false>
+template <int WAVES, int SEGS, int MT = 1, bool FUSEQ = false>
 bool launch_mfma_mode(const DecodeParams &p, int epi, hipStream_t stream)
 {
     const uint32_t ntiles = (p.N + 15) / 16;
     const dim3 grid((ntiles + p.tiles_per_wg - 1) / p.tiles_per_wg);
 #define DUQ_DEC(E) \
-    DUQ_LAUNCH_HEAD((gemm_s4_decode_kernel<WAVES, SEGS, E, MT, DB, FUSEQ>), grid, dim3(WAVES * 64), 0, stream, p)
+    DUQ_LAUNCH_HEAD((gemm_s4_decode_kernel<WAVES, SEGS, E, MT, FUSEQ>), grid, dim3(WAVES * 64), 0, stream, p)
     switch (epi) {
     case -1:
         if constexpr (FUSEQ) return false;
@@ -837,33 +1011,60 @@ bool launch_decode_any(DecodeParams &p, int epi, hipStream_t stream)
         // 9..16 rows: the MFMA kernel, rows quantized by every workgroup
         constexpr int W = DUQ_DEC_MFMA_FUSEQ_WAVES;
         p.tiles_per_wg = decode_tiles_per_workgroup((p.N + 15) / 16);
-        if (kbytes <= 1024) return launch_mfma_mode<W, 16 / W, 1, true, true>(p, epi, stream);
-        return launch_mfma_mode<W, 32 / W, 1, true, true>(p, epi, stream);
+        if (kbytes <= 1024) return launch_mfma_mode<W, 16 / W, 1, true>(p, epi, stream);
+        return launch_mfma_mode<W, 32 / W, 1, true>(p, epi, stream);
     } else {
         const uint32_t ntiles = (p.N + 15) / 16;
         p.tiles_per_wg = decode_tiles_per_workgroup(ntiles);
         constexpr int W = DUQ_DEC_WAVES, S = 32 / W;  // 64-byte segments per wavefront for 2 KB of a row
         const uint32_t mt = (p.M + 15) / 16;
-        // rows of up to 4096 / 8192 / 12288 elements: S, 2 S, 12 segments per wavefront; the row tiles whose
-        // fragments fit in registers next to two sets of weights (what select_gemm_kernel sends here)
-        if (mt > 4 || kbytes > 6144) return false;
+        // rows of up to 4096 / 8192 elements: S, 2 S segments per wavefront; the row tiles whose fragments fit in registers
+        // next to two sets of weights (what select_gemm_kernel leaves here)
+        if (mt > 4 || kbytes > 4096) return false;
         if (kbytes <= 2048) {
             if (mt == 1) return launch_mfma_mode<W, S, 1>(p, epi, stream);
             if (mt == 2) return launch_mfma_mode<W, S, 2>(p, epi, stream);
             if (mt == 3) return launch_mfma_mode<W, S, 3>(p, epi, stream);
             return launch_mfma_mode<W, S, 4>(p, epi, stream);
         }
-        if (kbytes <= 4096) {
-            if (mt == 1) return launch_mfma_mode<W, 2 * S, 1>(p, epi, stream);
-            if (mt == 2) return launch_mfma_mode<W, 2 * S, 2>(p, epi, stream);
-            if (mt == 3) return launch_mfma_mode<W, 2 * S, 3>(p, epi, stream);
-            return launch_mfma_mode<W, 2 * S, 4>(p, epi, stream);
-        }
-        if (mt == 1) return launch_mfma_mode<8, 12, 1>(p, epi, stream);
-        if (mt == 2) return launch_mfma_mode<8, 12, 2, false>(p, epi, stream);
-        if (mt == 3) return launch_mfma_mode<8, 12, 3, false>(p, epi, stream);
+        if (mt == 1) return launch_mfma_mode<W, 2 * S, 1>(p, epi, stream);
+        if (mt == 2) return launch_mfma_mode<W, 2 * S, 2>(p, epi, stream);
         return false;
     }
+}
+
+template <int MT, int NT>
+bool launch_lds_mode(const DecodeParams &p, int epi, hipStream_t stream)
+{
+    const dim3 grid((p.N + 16 * NT - 1) / (16 * NT));
+#define DUQ_DEC(E) DUQ_LAUNCH_HEAD((gemm_s4_lds_kernel<MT, NT, E>), grid, dim3(512), 0, stream, p)
+    switch (epi) {
+    case -1: DUQ_DEC(-1); break;
+    case 0: DUQ_DEC(0); break;
+    case 1: DUQ_DEC(1); break;
+    case 2: DUQ_DEC(2); break;
+    case 3: DUQ_DEC(3); break;
+    case 4: DUQ_DEC(4); break;
+    case 5: DUQ_DEC(5); break;
+    default: return false;
+    }
+#undef DUQ_DEC
+    return true;
+}
+
+bool launch_lds_any(const DecodeParams &p, int epi, hipStream_t stream)
+{
+    const uint32_t mt = (p.M + 15) / 16;
+    const bool two = p.N > 4096;  // one round of workgroups up to 8192 columns
+#define DUQ_LDS(MT) (two ? launch_lds_mode<MT, 2>(p, epi, stream) : launch_lds_mode<MT, 1>(p, epi, stream))
+    switch (mt) {
+    case 1: return DUQ_LDS(1);
+    case 2: return DUQ_LDS(2);
+    case 3: return DUQ_LDS(3);
+    case 4: return DUQ_LDS(4);
+    default: return false;
+    }
+#undef DUQ_LDS
 }
 
 }  // namespace
@@ -910,7 +1111,8 @@ int launch_decode_s4(const uint8_t *A, const uint8_t *B, uint32_t M, uint32_t N,
     p.C = out_acc;
     p.y = y;
     if (epi) p.epi = *epi;
-    if (!launch_decode_any<false>(p, out_acc ? -1 : epi->mode, stream)) return (int)hipErrorInvalidValue;
+    const int mode = out_acc ? -1 : epi->mode;
+    if (!(takes_lds_kernel(M, N, K) ? launch_lds_any(p, mode, stream) : launch_decode_any<false>(p, mode, stream))) return (int)hipErrorInvalidValue;
     return (int)hipGetLastError();
 }
 

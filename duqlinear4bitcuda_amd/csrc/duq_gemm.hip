@@ -892,8 +892,6 @@ static void launch_epi(GemmParams &p, hipStream_t stream, uint32_t batch = 1)
 #define DUQ_RING(X, R) DUQ_LAUNCH_HEAD((gemm_s4_ring_kernel<X, R, EPI, BIAS>), grid, dim3(256), 0, stream, p)
         if (xbytes == 8192) DUQ_RING(8192, 1);
         else if (xbytes == 4096) DUQ_RING(4096, 2);
-        else if (rb == 2) DUQ_RING(2048, 2);
-        else if (rb == 3) DUQ_RING(2048, 3);
         else DUQ_RING(2048, 4);
 #undef DUQ_RING
         return;
@@ -937,7 +935,7 @@ int launch_gemm_s4_batched(const uint8_t *A, const uint8_t *B, uint32_t M, uint3
     if (M == 0 || N == 0 || batch == 0) return 0;
     if (batch == 1) {
         const int kernel = select_gemm_kernel(M, N, K);
-        if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma)
+        if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma || takes_lds_kernel(M, N, K))
             return launch_decode_s4(A, B, M, N, K, out_acc, epi, y, stream);
     }
     GemmParams p{};

@@ -83,6 +83,26 @@ enum GemmKernelId {
     kKernelTile = 7,        // the same kernels on problems of few tiles or rows too long for the others
 };
 int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K);
+// Shapes of the LDS kernel (duq_decode.hip), asked before select_gemm_kernel's families (whose number such a shape keeps:
+// the buckets there are by size).  Measured against those on 900 shapes, us:
+//  - 5..64 rows: every length on up to 4096 columns (7 - 75 % less; 16 x 512 x 1024 3.2 -> 2.9, 64 x 1024 x 8192 7.9 -> 6.7, 16
+//    x 512 x 28672 25.6 -> 7.2).  Up to 8192 columns where the rows are many or long (64 x 5120 x 5120 9.6 -> 7.9, 16 x 8192 x
+//    8192 9.2 -> 8.5, but 16 x 8192 x 4096 5.1 -> 5.4 and 24 x 8192 x 4096 6.1 -> 6.3: the MFMA kernel keeps its activations in
+//    registers over several column tiles, one fetch of them per CU).  More columns: the lengths that the MFMA kernel does not
+//    hold and for which the ring kernel streams the weights twice (16 x 12288 x 14336 26.8 -> 20.0, 32 x 16384 x 11008 26.9 ->
+//    23.0; 48 x 11008 x 11008 19.8 -> 22.6).
+//  - up to 4 rows longer than the rows kernel's 16384 (the dot kernel, one weight row per wavefront pair, or beyond 30720 a
+//    prefill tile): up to 4096 columns (4 x 2606 x 28672 13.4 -> 8.1, 1 x 1024 x 40000 34.2 -> 8.3), above for 3 and 4 rows (4 x
+//    8192 x 28672 28.9 -> 21.8, but 4 x 8192 x 16448 18.6 -> 20.1) and beyond 30720 (1 x 8192 x 40000 49.4 -> 31.1; 1 x 8192 x
+//    28672 21.5 against 22.0).
+inline bool takes_lds_kernel(uint32_t M, uint32_t N, uint32_t K)
+{
+    if (M == 0 || M > 64 || K == 0 || K > 65536 || (uint64_t)N * (K / 2) >= 0xFFFFFF00ull) return false;
+    if (M <= 4) return K > 16384 && (N <= 4096 || (N <= 16384 && K > (M > 2 ? 18432 : 30720)));
+    if (N <= 4096) return true;
+    if (N <= 8192) return M > 32 || K > 4096 || (M > 16 && (N <= 6144 || K <= 2048));
+    return K > 8192 && (K <= 12288 ? M <= 32 : K <= 16384 && M <= 16);
+}
 // Shapes whose GEMM can apply the dual-uniform row-sum epilogue itself (mode 5): those of the decode kernels, and those
 // of the stream and prefill kernels with rows longer than 256 elements (512 where output rows are not 16-byte aligned:
 // there the accumulators' detour through memory, 8 bytes per output, is what a launch takes); the others run the GEMM into
@@ -90,7 +110,7 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K);
 inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 {
     const int kernel = select_gemm_kernel(M, N, K);
-    if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma) return true;
+    if (takes_lds_kernel(M, N, K) || kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma) return true;
     return (kernel == kKernelStream || kernel == kKernelTile) && (N % 8 == 0 ? K > 256 : K >= 512);
 }
 // Tile for a problem select_gemm_kernel gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
