@@ -20,9 +20,10 @@
 //    whole K range: lane l holds bytes [i*1024 + l*16, +16) of each row, so a load instruction covers 1 KB
 //    of one row and an activation register serves four rows.  The 4*M partial sums of a lane meet the other
 //    lanes' through the wavefront's own piece of LDS (no barrier) and a few DPP steps.
-//  MFMA kernel (5 <= M <= 64, several column tiles per CU, K <= 8192): v_mfma_i32_16x16x64_i8, eight wavefronts split K for one 16-column tile, one to
-//    four tiles of 16 rows against the same weight fragments, the partial tiles meet in LDS, 256 threads finish
+//  MFMA kernel (5 <= M <= 64, several column tiles per CU, K <= 8192): v_mfma_i32_16x16x64_i8, eight wavefronts split K
+//    for one 16-column tile, one to four tiles of 16 rows against the same weight fragments, the partial tiles meet in LDS, 256 threads finish
 //    one output each per row tile; one round of at most 256 workgroups with several column tiles each.
+//  wide kernel (5 <= M <= 64, many column tiles per CU, K <= 8192): the MFMA kernel's plan with the weights through LDS.
 //  LDS kernel (M <= 64, one or two column tiles per workgroup, any K): the same MFMAs, both operands through LDS in whole
 //    cache lines, K in a loop.
 #include <cstddef>
@@ -905,6 +906,159 @@ __global__ __launch_bounds__(512) void gemm_s4_lds_kernel(DUQ_HEAD_DECL, DecodeP
 }
 
 // ---------------------------------------------------------------------------------
+// wide kernel: 5 <= M <= 64, more than 8192 columns, K <= 8192 (what takes_wide_kernel gives it)
+// ---------------------------------------------------------------------------------
+// The MFMA kernel's plan, several column tiles per workgroup against activations held in registers, with the LDS kernel's way
+// in: weights arrive in whole cache lines, without registers, and six to eight steps of 2 KB per wavefront are in flight
+// whatever tile they belong to, so that no tile begins with a wait.  The activations take the same way, as the first steps of
+// the sequence.  What bounds a launch is the reading of the weights, 4.9 TB/s at 16 x 28672 x 8192 (4.1 before).  A load whose
+// result the compiler waits for would empty that queue: eight wavefronts only load and multiply, and four others fetch the
+// parameters, add up the eight partial tiles and store, one tile behind.  Measured (us): 16 x 28672 x 8192 28.6 -> 24.1, x
+// 16384 x 8192 15.4 -> 14.1, 24 x 28672 x 8192 30.3 -> 26.6, 32 x 11008 x 4096 8.5 -> 7.4, 48 x 11008 x 2048 7.7 -> 6.6.
+template <int MT, int KS>
+struct WideTile {
+    static constexpr int kPart = MT * 8 * 1024;                              // one tile's partial sums
+    static constexpr int DEPTH = (160 * 1024 - 2 * kPart) / (8 * 2048) < 8 ? (160 * 1024 - 2 * kPart) / (8 * 2048) : 8;  // steps in flight
+    static constexpr int kLds = 2 * kPart + 8 * DEPTH * 2048;
+    static_assert(kLds <= 160 * 1024, "LDS");
+};
+template <int MT, int KS, int EPI>
+__global__ __launch_bounds__(768) void gemm_s4_wide_kernel(DUQ_HEAD_DECL, DecodeParams tail)
+{
+    const DecodeParams p = with_head(tail, DUQ_HEAD_USE);
+    using Tile = WideTile<MT, KS>;
+    constexpr int MODE = EPI < 0 ? 0 : EPI;
+    constexpr int DEPTH = Tile::DEPTH;
+    constexpr uint32_t kStage = 2048, kPart = Tile::kPart;
+    __shared__ __attribute__((aligned(256))) uint8_t lds[Tile::kLds];
+    using ColRec = typename EpiRec<MODE>::Col;
+    using RowRec = typename EpiRec<MODE>::Row;
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t kbytes = p.K >> 1;
+    const uint32_t ntiles = (p.N + 15) / 16;
+    const uint32_t tile0 = blockIdx.x * p.tiles_per_wg, count = min(p.tiles_per_wg, ntiles - tile0);
+    if (wave < 8) {
+        const uint32_t l16 = lane & 15u, g = lane >> 4;
+        const auto desc = [](const uint8_t *base, uint32_t bytes) {
+            const uint64_t a = reinterpret_cast<uint64_t>(base);
+            return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
+                       (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+        };
+        const v4u dX = desc(p.A, p.M * kbytes);  // rows past M and N read as zero
+        const v4u dW = desc(p.B + (uint64_t)tile0 * 16 * kbytes, min(p.N - tile0 * 16, count * 16) * kbytes);
+        // ---- global -> LDS, two instructions of eight rows: sixteen rows' 128 bytes of kilobyte ks; pieces lie at piece ^ (row / 2)
+        const uint32_t r0 = lane >> 3, even = ((lane & 7u) ^ (r0 >> 1)) * 16, odd = even ^ 64u;
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds + 2 * kPart + wave * (DEPTH * kStage);
+        auto load = [&](const v4u d, uint32_t tile, uint32_t ks, uint32_t slot) {
+            const uint32_t k = ks * 1024 + wave * 128, row0 = (tile * 16 + r0) * kbytes;
+            const uint32_t off0 = k + even < kbytes ? row0 + k + even : kOobOffset;  // K % 64 == 0: a piece is all in or all out
+            const uint32_t off1 = k + odd < kbytes ? row0 + 8 * kbytes + k + odd : kOobOffset;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds0 + slot), "v"(off0), "s"(d) : "memory", "m0");
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds0 + slot + 1024), "v"(off1), "s"(d) : "memory", "m0");
+        };
+        // the sequence of steps: KS of every row tile of the activations, then KS of every column tile
+        const uint8_t *const own = lds + 2 * kPart + wave * (DEPTH * kStage) + l16 * 128;
+        uint32_t slot = 0;
+        auto step = [&](v4u(&f)[2], auto &&next) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * 2) : "memory");
+#pragma unroll
+            for (int u = 0; u < 2; ++u) f[u] = *reinterpret_cast<const v4u *>(own + slot + ((u * 4 + g) ^ (l16 >> 1)) * 16);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the place takes the step DEPTH further on
+            next(slot);
+            slot = slot + kStage == DEPTH * kStage ? 0 : slot + kStage;
+        };
+        auto load_step = [&](uint32_t i, uint32_t to) {  // i: constant in the two loops below
+            if (i < MT * KS)
+                load(dX, i / KS, i % KS, to);
+            else
+                load(dW, (i - MT * KS) / KS, (i - MT * KS) % KS, to);
+        };
+#pragma unroll
+        for (int i = 0; i < DEPTH; ++i) load_step(i, i * kStage);
+        v4u x[MT][KS][2];
+#pragma unroll
+        for (int i = 0; i < MT * KS; ++i) step(x[i / KS][i % KS], [&](uint32_t to) { load_step(i + DEPTH, to); });
+        for (uint32_t t = 0; t < count; ++t) {
+            v4i acc[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m] = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                v4u w[2];
+                step(w, [&](uint32_t to) { load(dW, t + (ks + DEPTH) / KS, (ks + DEPTH) % KS, to); });
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    v4u we, wo;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        we[q] = (w[u][q] << 4) & kNibbleMaskD;
+                        wo[q] = w[u][q] & kNibbleMaskD;
+                    }
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) {
+                        v4u xe, xo, xv = x[m][ks][u];
+                        if (MT * KS > 4) asm volatile("" : "+v"(xv));  // (expanded here: hoisted out of the loop it would double the registers)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            xe[q] = (xv[q] << 4) & kNibbleMaskD;
+                            xo[q] = xv[q] & kNibbleMaskD;
+                        }
+                        acc[m] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, we), __builtin_bit_cast(v4i, xe), acc[m], 0, 0, 0);
+                        acc[m] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, wo), __builtin_bit_cast(v4i, xo), acc[m], 0, 0, 0);
+                        if (MT * KS > 4) __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            v4i *const part = reinterpret_cast<v4i *>(lds + (t & 1u) * kPart);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) part[(m * 8 + wave) * 64 + lane] = acc[m];
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the loads past the end)
+    } else {
+        // ---- four wavefronts finish the tiles: one output per thread and row tile, element er of MFMA lane src_lane
+        const uint32_t src_lane = (tid >> 2) & 63u, er = tid & 3u;
+        const uint32_t my_m = src_lane & 15u, my_c = (src_lane >> 4) * 4 + er;
+        const bool bias = p.epi.bias != nullptr;
+        const auto c_out = as_global(p.C);
+        const auto y_out = as_global(p.y);
+        RowRec rp[MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            rp[m] = RowRec{};
+            if (EPI >= 0) rp[m] = load_row_rt<MODE>(p.epi, min(m * 16 + my_m, p.M - 1), p.A, kbytes);
+        }
+        auto load_cp = [&](uint32_t t) {
+            ColRec c{};
+            if (EPI >= 0) c = load_col_rt<MODE>(p.epi, min((tile0 + t) * 16 + my_c, p.N - 1), bias, p.B, kbytes);
+            return c;
+        };
+        ColRec cp = load_cp(0);
+        for (uint32_t t = 0; t < count; ++t) {
+            const ColRec next = load_cp(min(t + 1, count - 1));
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            const int *const sums = reinterpret_cast<const int *>(lds + (t & 1u) * kPart) + src_lane * 4 + er;
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                int sum = 0;
+#pragma unroll
+                for (int v = 0; v < 8; ++v) sum += sums[(m * 8 + v) * 256];
+                sum >>= 8;
+                const uint32_t row = m * 16 + my_m, n = (tile0 + t) * 16 + my_c;
+                if (row < p.M && n < p.N) {
+                    if (EPI < 0)
+                        c_out[(uint64_t)row * p.N + n] = sum;
+                    else
+                        y_out[(uint64_t)row * p.N + n] = dequant_rt<MODE>(sum, rp[m], cp, bias);
+                }
+            }
+            cp = next;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------
 // dispatch
 // ---------------------------------------------------------------------------------
 // Every dispatcher below returns whether it launched a kernel: a shape or mode that no instantiated template
@@ -1052,6 +1206,39 @@ bool launch_lds_mode(const DecodeParams &p, int epi, hipStream_t stream)
     return true;
 }
 
+template <int MT, int KS>
+bool launch_wide_mode(DecodeParams &p, int epi, hipStream_t stream)
+{
+    const uint32_t ntiles = (p.N + 15) / 16;
+    p.tiles_per_wg = decode_tiles_per_workgroup(ntiles);
+    const dim3 grid((ntiles + p.tiles_per_wg - 1) / p.tiles_per_wg);
+#define DUQ_DEC(E) DUQ_LAUNCH_HEAD((gemm_s4_wide_kernel<MT, KS, E>), grid, dim3(768), 0, stream, p)
+    switch (epi) {
+    case -1: DUQ_DEC(-1); break;
+    case 0: DUQ_DEC(0); break;
+    case 1: DUQ_DEC(1); break;
+    case 2: DUQ_DEC(2); break;
+    case 3: DUQ_DEC(3); break;
+    case 4: DUQ_DEC(4); break;
+    case 5: DUQ_DEC(5); break;
+    default: return false;
+    }
+#undef DUQ_DEC
+    return true;
+}
+
+bool launch_wide_any(DecodeParams &p, int epi, hipStream_t stream)
+{
+    const uint32_t mt = (p.M + 15) / 16, ks = p.K <= 2048 ? 1 : p.K <= 4096 ? 2 : 4;  // kilobytes of a row
+    if (mt == 1 && ks == 4) return launch_wide_mode<1, 4>(p, epi, stream);
+    if (mt == 2 && ks == 4) return launch_wide_mode<2, 4>(p, epi, stream);
+    if (mt == 2 && ks == 2) return launch_wide_mode<2, 2>(p, epi, stream);
+    if (mt == 2) return launch_wide_mode<2, 1>(p, epi, stream);
+    if (mt == 3 && ks == 1) return launch_wide_mode<3, 1>(p, epi, stream);
+    if (mt == 4 && ks == 1) return launch_wide_mode<4, 1>(p, epi, stream);
+    return false;
+}
+
 bool launch_lds_any(const DecodeParams &p, int epi, hipStream_t stream)
 {
     const uint32_t mt = (p.M + 15) / 16;
@@ -1112,7 +1299,7 @@ int launch_decode_s4(const uint8_t *A, const uint8_t *B, uint32_t M, uint32_t N,
     p.y = y;
     if (epi) p.epi = *epi;
     const int mode = out_acc ? -1 : epi->mode;
-    if (!(takes_lds_kernel(M, N, K) ? launch_lds_any(p, mode, stream) : launch_decode_any<false>(p, mode, stream))) return (int)hipErrorInvalidValue;
+    if (!(takes_wide_kernel(M, N, K) ? launch_wide_any(p, mode, stream) : takes_lds_kernel(M, N, K) ? launch_lds_any(p, mode, stream) : launch_decode_any<false>(p, mode, stream))) return (int)hipErrorInvalidValue;
     return (int)hipGetLastError();
 }
 

@@ -935,7 +935,7 @@ int launch_gemm_s4_batched(const uint8_t *A, const uint8_t *B, uint32_t M, uint3
     if (M == 0 || N == 0 || batch == 0) return 0;
     if (batch == 1) {
         const int kernel = select_gemm_kernel(M, N, K);
-        if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma || takes_lds_kernel(M, N, K))
+        if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma || takes_wide_kernel(M, N, K) || takes_lds_kernel(M, N, K))
             return launch_decode_s4(A, B, M, N, K, out_acc, epi, y, stream);
     }
     GemmParams p{};

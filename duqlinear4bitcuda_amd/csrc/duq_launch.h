@@ -87,7 +87,8 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K);
 // the buckets there are by size).  Measured against those on 900 shapes, us:
 //  - 5..64 rows: every length on up to 4096 columns (7 - 75 % less; 16 x 512 x 1024 3.2 -> 2.9, 64 x 1024 x 8192 7.9 -> 6.7, 16
 //    x 512 x 28672 25.6 -> 7.2).  Up to 8192 columns where the rows are many or long (64 x 5120 x 5120 9.6 -> 7.9, 16 x 8192 x
-//    8192 9.2 -> 8.5, but 16 x 8192 x 4096 5.1 -> 5.4 and 24 x 8192 x 4096 6.1 -> 6.3: the MFMA kernel keeps its activations in
+//    8192 9.2 -> 8.5, but 16 x 8192 x 4096 5.1 -> 5.4 and 24 x 8192 x 4096 6.1 -> 6.3, and where rows begin inside a cache line, 19 x 5332 x 3648 5.0
+//    -> 5.5: the MFMA kernel keeps its activations in
 //    registers over several column tiles, one fetch of them per CU).  More columns: the lengths that the MFMA kernel does not
 //    hold and for which the ring kernel streams the weights twice (16 x 12288 x 14336 26.8 -> 20.0, 32 x 16384 x 11008 26.9 ->
 //    23.0; 48 x 11008 x 11008 19.8 -> 22.6).
@@ -100,8 +101,22 @@ inline bool takes_lds_kernel(uint32_t M, uint32_t N, uint32_t K)
     if (M == 0 || M > 64 || K == 0 || K > 65536 || (uint64_t)N * (K / 2) >= 0xFFFFFF00ull) return false;
     if (M <= 4) return K > 16384 && (N <= 4096 || (N <= 16384 && K > (M > 2 ? 18432 : 30720)));
     if (N <= 4096) return true;
-    if (N <= 8192) return M > 32 || K > 4096 || (M > 16 && (N <= 6144 || K <= 2048));
-    return K > 8192 && (K <= 12288 ? M <= 32 : K <= 16384 && M <= 16);
+    if (N <= 8192) return M > 32 || K > 4096 || (M > 16 && (K <= 2048 || (N <= 6144 && K % 256 == 0)));
+    return K > 8192 && (M <= 16 ? K <= 16384 : M <= 32 && K <= 12288);
+}
+// Shapes of the wide kernel (duq_decode.hip), asked first.  Measured against the MFMA kernel, us: up to 16 rows longer than 6144
+// elements, from 5120 on above 16384 columns (16 x 28672 x 5120 18.1 -> 16.3, 8 x 20000 x 8192 19.2 -> 17.1, but 8 x 16384 x 6144
+// 10.2 -> 10.8, and up to 4096 elements it is level or behind, 16 x 16384 x 4096 7.8 -> 8.3); 17..32 rows of up to 4096 elements
+// on up to 14336 columns (24 x 9000 x 4096 7.7 -> 6.8; 24 x 20000 x 3072 9.6 -> 10.0), of more than 6144 above 16384 (32 x
+// 28672 x 8192 31.1 -> 27.3, but 18 x 33087 x 4160 20.6 -> 22.3, half of whose steps are padding; of fewer columns, tiles of the prefill kernel, 32 x 11008 x 8192 12.3 against 12.9); 33 and more rows of up to
+// 2048 elements (48 x 28672 x 1024 10.7 -> 9.9, longer ones 48 x 13824 x 3072 9.5 -> 10.3), from 49 on above 16384 columns
+// (64 x 28672 x 2048 13.3 -> 12.6, 64 x 13824 x 2048 8.3 -> 8.8).
+inline bool takes_wide_kernel(uint32_t M, uint32_t N, uint32_t K)
+{
+    if (M < 5 || M > 64 || N <= 8192 || K == 0 || K > 8192 || (uint64_t)N * (K / 2) >= 0xFFFFFF00ull) return false;
+    if (M <= 16) return K > 6144 || (K >= 5120 && N > 16384);
+    if (M <= 32) return K <= 4096 ? N <= 14336 : K > 6144 && N > 16384;
+    return K <= 2048 && (M <= 48 || N > 16384);
 }
 // Shapes whose GEMM can apply the dual-uniform row-sum epilogue itself (mode 5): those of the decode kernels, and those
 // of the stream and prefill kernels with rows longer than 256 elements (512 where output rows are not 16-byte aligned:
@@ -110,7 +125,7 @@ inline bool takes_lds_kernel(uint32_t M, uint32_t N, uint32_t K)
 inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 {
     const int kernel = select_gemm_kernel(M, N, K);
-    if (takes_lds_kernel(M, N, K) || kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma) return true;
+    if (takes_wide_kernel(M, N, K) || takes_lds_kernel(M, N, K) || kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma) return true;
     return (kernel == kKernelStream || kernel == kKernelTile) && (N % 8 == 0 ? K > 256 : K >= 512);
 }
 // Tile for a problem select_gemm_kernel gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
