@@ -24,7 +24,7 @@
 //    for one 16-column tile, one to four tiles of 16 rows against the same weight fragments, the partial tiles meet in LDS, 256 threads finish
 //    one output each per row tile; one round of at most 256 workgroups with several column tiles each.
 //  wide kernel (5 <= M <= 64, many column tiles per CU, K <= 8192): the MFMA kernel's plan with the weights through LDS.
-//  LDS kernel (M <= 64, one or two column tiles per workgroup, any K): the same MFMAs, both operands through LDS in whole
+//  LDS kernel (one or two column tiles and up to four row tiles per workgroup, any K): the same MFMAs, both operands through LDS in whole
 //    cache lines, K in a loop.
 #include <cstddef>
 
@@ -726,19 +726,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DEC
 }
 
 // ---------------------------------------------------------------------------------
-// LDS kernel: up to 64 rows of any length (what takes_lds_kernel gives it)
+// LDS kernel: up to 64 rows of any length, more on narrow problems (what takes_lds_kernel gives it)
 // ---------------------------------------------------------------------------------
 // A fragment of the MFMA takes sixteen bytes of each of sixteen rows from sixteen neighbouring lanes, and a load in that
 // layout touches a cache line per lane: the kernel above requests its operands at about 29 bytes per ns and CU, a quarter of
 // what a CU can take in (131 KB a workgroup at 16 x 4096 x 8192), and a launch of few rows lasts as long as that.  Here both
 // operands come through LDS without registers, in instructions of whole 128- or 512-byte pieces of a row; eight wavefronts
 // split K, each reads its fragments out of LDS, and the walk over K is a loop, so that rows may be of any length.  Sixteen
-// columns per workgroup (up to 4096 columns, one round of workgroups): a wavefront's stages are its own, 128 bytes of every
-// kilobyte of a row, and nothing waits for another wavefront until the sums meet.  32 columns (up to 8192 in one round): the
+// columns per workgroup: a wavefront's stages are its own, 128 bytes of every
+// kilobyte of a row, and nothing waits for another wavefront until the sums meet.  32 columns: the
 // activations are a third less of what enters a CU, and the wavefronts share stages of 512 bytes a row, which 64 rows need
 // (8192 x 28672: 29 us against 42 with 64-byte pieces of their own, which are half lines).  Measured against what ran before
 // (N x K, us): 16 rows 4096 x 4096 4.1 -> 3.8, x 8192 6.9 -> 5.5, x 11008 8.5 -> 6.2, 2606 x 26944 31.9 -> 14.1, 8192 x 28672
-// 31.0 -> 21.3; 64 rows 7.4 -> 5.7, 11.2 -> 8.0, 15.2 -> 10.4, 40.6 -> 27.4, 39.2 -> 29.1.
+// 31.0 -> 21.3; 64 rows 7.4 -> 5.6, 11.2 -> 7.6, 15.2 -> 8.9, 40.6 -> 16.4, 39.2 -> 29.1.  Groups of rows in workgroups of their
+// own, where a column range leaves compute units without work: 64 x 1024 x 8192 7.9 -> 4.4, 128 x 1024 x 8192 8.2 -> 5.4, 256 x
+// 2048 x 4096 9.0 -> 7.4, 96 x 4096 x 11008 14.3 -> 10.4 (64 x 64 tiles of the prefill kernel: half the workgroups and twice the
+// operands each).
 template <int MT, int NT>
 struct LdsTile {
     static constexpr int G = NT == 1 ? 1 : 8;            // wavefronts that share a stage
@@ -766,13 +769,17 @@ __global__ __launch_bounds__(512) void gemm_s4_lds_kernel(DUQ_HEAD_DECL, DecodeP
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t l16 = lane & 15u, g = lane >> 4;
     const uint32_t kbytes = p.K >> 1;
-    const uint32_t col0 = blockIdx.x * (16 * NT);
+    // groups of 16 * MT rows share the weights of a column tile: consecutive in `at`, an eighth of which runs on one XCD
+    const uint32_t groups = p.tiles_per_wg & 0x1FFu, per_xcd = ((p.N + 16 * NT - 1) / (16 * NT) * groups + 7) / 8;
+    const uint32_t at = blockIdx.x % 8 * per_xcd + blockIdx.x / 8, tile = at * (p.tiles_per_wg >> 9) >> 16;  // (tile = at / groups)
+    const uint32_t col0 = tile * (16 * NT), m0 = (at - tile * groups) * (16 * MT);
+    if (col0 >= p.N) return;
     const auto desc = [](const uint8_t *base, uint32_t bytes) {
         const uint64_t a = reinterpret_cast<uint64_t>(base);
         return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
     };
-    const v4u dX = desc(p.A, p.M * kbytes);  // rows past M and N read as zero
+    const v4u dX = desc(p.A + (uint64_t)m0 * kbytes, min(p.M - m0, 16u * MT) * kbytes);  // rows past M and N read as zero
     const v4u dW = desc(p.B + (uint64_t)col0 * kbytes, min(p.N - col0, 16u * NT) * kbytes);
 
     // ---- global -> LDS: instruction j of a group's wavefront v takes kilobyte j * G + v of the stage, activations first; a
@@ -863,7 +870,7 @@ __global__ __launch_bounds__(512) void gemm_s4_lds_kernel(DUQ_HEAD_DECL, DecodeP
         rp[f] = RowRec{};
         if (EPI >= 0) {
             cp[f] = load_col_rt<MODE>(p.epi, min(col0 + t / MT * 16 + my_c, p.N - 1), bias, p.B, kbytes);
-            rp[f] = load_row_rt<MODE>(p.epi, min(t % MT * 16 + my_m, p.M - 1), p.A, kbytes);
+            rp[f] = load_row_rt<MODE>(p.epi, min(m0 + t % MT * 16 + my_m, p.M - 1), p.A, kbytes);
         }
     }
     uint32_t slot = 0;
@@ -894,7 +901,7 @@ __global__ __launch_bounds__(512) void gemm_s4_lds_kernel(DUQ_HEAD_DECL, DecodeP
 #pragma unroll
             for (int v = 0; v < WAVES; ++v) sum += sums[(t * WAVES + v) * 256];
             sum >>= 8;
-            const uint32_t m = t % MT * 16 + my_m, n = col0 + t / MT * 16 + my_c;
+            const uint32_t m = m0 + t % MT * 16 + my_m, n = col0 + t / MT * 16 + my_c;
             if (m < p.M && n < p.N) {
                 if (EPI < 0)
                     c_out[(uint64_t)m * p.N + n] = sum;
@@ -1188,9 +1195,13 @@ bool launch_decode_any(DecodeParams &p, int epi, hipStream_t stream)
 }
 
 template <int MT, int NT>
-bool launch_lds_mode(const DecodeParams &p, int epi, hipStream_t stream)
+bool launch_lds_mode(DecodeParams &p, int epi, hipStream_t stream)
 {
-    const dim3 grid((p.N + 16 * NT - 1) / (16 * NT));
+    // groups of rows, and 2^16 over them: (at * m) >> 16 == at / groups while at * (groups - 1) < 2^16
+    const uint32_t groups = (p.M + 16 * MT - 1) / (16 * MT), tiles = (p.N + 16 * NT - 1) / (16 * NT);
+    if (groups > 1 && groups * tiles > 256) return false;
+    p.tiles_per_wg = groups | ((65535 + groups) / groups) << 9;
+    const dim3 grid((tiles * groups + 7) / 8 * 8);
 #define DUQ_DEC(E) DUQ_LAUNCH_HEAD((gemm_s4_lds_kernel<MT, NT, E>), grid, dim3(512), 0, stream, p)
     switch (epi) {
     case -1: DUQ_DEC(-1); break;
@@ -1239,12 +1250,11 @@ bool launch_wide_any(DecodeParams &p, int epi, hipStream_t stream)
     return false;
 }
 
-bool launch_lds_any(const DecodeParams &p, int epi, hipStream_t stream)
+bool launch_lds_any(DecodeParams &p, int epi, hipStream_t stream)
 {
-    const uint32_t mt = (p.M + 15) / 16;
-    const bool two = p.N > 4096;  // one round of workgroups up to 8192 columns
-#define DUQ_LDS(MT) (two ? launch_lds_mode<MT, 2>(p, epi, stream) : launch_lds_mode<MT, 1>(p, epi, stream))
-    switch (mt) {
+    const LdsShape tile = lds_shape(p.M, p.N);
+#define DUQ_LDS(MT) (tile.cols == 2 ? launch_lds_mode<MT, 2>(p, epi, stream) : launch_lds_mode<MT, 1>(p, epi, stream))
+    switch (tile.rows) {
     case 1: return DUQ_LDS(1);
     case 2: return DUQ_LDS(2);
     case 3: return DUQ_LDS(3);

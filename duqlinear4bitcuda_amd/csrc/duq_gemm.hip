@@ -10,32 +10,25 @@
 // 256*|C| stays below 2^31 for K <= 131008.  Integer accumulation is order-free, so the
 // k order inside a tile only has to be the same for A and B.
 //
-// Five kernels here, and the prefill kernel in duq_prefill.hip, picked by shape in select_gemm_kernel() (up to 64 rows
-// run the two kernels of duq_decode.hip as far as they reach):
+// Four kernels here, and the prefill kernel in duq_prefill.hip, picked by shape in select_gemm_kernel() (up to 64 rows,
+// and more on narrow problems, run the kernels of duq_decode.hip as far as they reach):
 //  * prefill kernel (duq_prefill.hip): more than 64 rows, long rows, fewer rows on wide layers, tensors of 4 GiB or more,
 //    what is left;
 //  * stream kernel (the same shapes where rows are short): 64 x 128 tiles, weights from global memory straight to
 //    registers, activations expanded once into LDS, v_mfma_i32_32x32x32_i8 with a hand-ordered schedule;
 //  * short-row kernel (rows of at most 256 elements): the stream kernel's operand paths without its K pipeline;
-//  * ring kernel (17 <= M <= 256 on problems of at most one round of its workgroups, and 5..16 rows of 12289..16384 elements):
-//    packed activations of all rows in LDS, every wavefront streams whole weight rows through a ring of loads;
 //  * skinny kernel (9 <= M <= 16 with 1536 or more column tiles): one workgroup owns 16 output columns, its
 //    wavefronts split K, whole-line weight loads turned into fragments through LDS;
-//  * dot kernel (M <= 4 with rows longer than 16384 elements): v_dot8_i32_i4 on the packed nibbles, a
+//  * dot kernel (M <= 4 with rows of 16385 to 30720 elements, more than 4096 columns): v_dot8_i32_i4 on the packed nibbles, a
 //    pure HBM stream.
 // In the MFMA kernels the weight operand goes to the MFMA "A" side, so each lane ends up
 // with four consecutive output columns of one row.
 #include "duq_gemm_common.h"
 // Cache policy of the weight loads of the kernels that read every weight byte once: 2 = non-temporal.  Measured:
 // skinny kernel 16 x 28672 x 4096 13.2 against 14.1 us, dot kernel 1 x 8192 x 28672 20.9 against 22.8 and 4 x 4096 x
-// 20480 11.5 against 13.2; the ring kernel (row groups read the weights again; a lane fetches 16 bytes of a row, a
-// quarter of a cache line, per instruction) loses on most shapes (100 x 1000 x 4096: 7.9 against 7.3) and keeps the
-// default.
+// 20480 11.5 against 13.2.
 #ifndef DUQ_SKINNY_WLOAD_AUX
 #define DUQ_SKINNY_WLOAD_AUX 2
-#endif
-#ifndef DUQ_RING_WLOAD_AUX
-#define DUQ_RING_WLOAD_AUX 0
 #endif
 #ifndef DUQ_DOT_WLOAD_AUX
 #define DUQ_DOT_WLOAD_AUX 2
@@ -542,131 +535,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_skinny_kernel(DUQ_HEAD_DEC
 }
 
 // ---------------------------------------------------------------------------------
-// ring kernel (17 <= M <= 256 on narrow problems, and M <= 16 with rows of 12289..16384 elements)
-// ---------------------------------------------------------------------------------
-// The packed activations of all 16*RB rows sit in LDS for the whole K range (rows padded so that
-// 16 rows x 16 bytes cover every bank once); a wavefront owns a 16-column tile and a K slice
-// and streams the weights of that slice through a ring of kRing 128-bit loads per lane that is
-// refilled slot by slot, across tile boundaries too, so the loads in flight never drain.  Every
-// weight fragment is expanded once and multiplied with the RB activation fragments read from
-// LDS (one expansion each).  No barrier inside the K loop; when several wavefronts split K for
-// a tile their partial sums meet in LDS once per tile.  More rows than 16*RB are covered by
-// blockIdx.y (groups of 16*RB rows, each streaming the weights again).
-constexpr int kRing = 8;  // 128-bit weight loads in flight per lane
-
-template <int XBYTES, int RB, int EPI, bool BIAS>
-__global__ __launch_bounds__(256) void gemm_s4_ring_kernel(DUQ_HEAD_DECL, GemmParams tail)
-{
-    GemmParams p = with_head(tail, DUQ_HEAD_USE);
-    to_global(p.A);
-    to_global(p.B);
-    to_global(p.C);
-    to_global(p.y);
-    constexpr uint32_t WAVES = 4, T = WAVES * 64;
-    constexpr uint32_t XS = XBYTES + 16;  // LDS row stride = 16 (mod 256)
-    __shared__ __attribute__((aligned(16))) uint8_t xs[16 * RB * XS];
-    __shared__ v4i part[WAVES][RB][64];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u, wave = tid >> 6;
-    const uint32_t l16 = lane & 15u, g = lane >> 4;
-    const uint32_t kbytes = p.K >> 1;
-    const uint32_t segs = (kbytes + 63) / 64;
-    const uint32_t kslices = p.tiles_m;  // (fields reused) wavefronts that split K for one tile: 1, 2 or 4
-    const uint32_t items = p.tiles_n;    // tiles each wavefront walks through
-    const uint32_t tiles_per_wg = WAVES / kslices;
-    const uint32_t slice = wave % kslices, tsub = wave / kslices;
-    const uint32_t sps = (segs + kslices - 1) / kslices;  // 64-byte segments per slice
-    const uint32_t seg_lo = slice * sps;
-    const uint32_t nblk = (sps + kRing - 1) / kRing;
-    const uint32_t m_base = blockIdx.y * (16 * RB);
-
-    const __amdgpu_buffer_rsrc_t rW = make_rsrc(p.B, p.N * kbytes);  // rows past N read as zero
-    const __amdgpu_buffer_rsrc_t rX = make_rsrc(p.A, p.M * kbytes);  // rows past M read as zero
-
-    v4u ring[kRing];
-    auto tile_of = [&](uint32_t it) { return (blockIdx.x * items + it) * tiles_per_wg + tsub; };
-    auto issue = [&](uint32_t it, uint32_t blk, int j) {
-        const uint32_t row = tile_of(it) * 16 + l16;
-        const uint32_t sg = blk * kRing + j;
-        const uint32_t off = (seg_lo + sg) * 64 + g * 16;
-        const bool ok = it < items && row < p.N && sg < sps && off < kbytes;
-        ring[j] = buf_load16_aux<DUQ_RING_WLOAD_AUX>(rW, ok ? row * kbytes + off : kOobOffset, 0);
-    };
-#pragma unroll
-    for (int j = 0; j < kRing; ++j) issue(0, 0, j);  // the first weights are under way before the activations
-
-    {
-        const uint32_t ppr = kbytes >> 4;  // 16-byte pieces per row
-        for (uint32_t c = tid; c < ppr; c += T) {
-#pragma unroll
-            for (int r0 = 0; r0 < 16 * RB; r0 += 16) {
-                v4u v[16];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) v[r] = buf_load16(rX, (m_base + r0 + r) * kbytes + c * 16, 0);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) *reinterpret_cast<v4u *>(xs + (r0 + r) * XS + c * 16) = v[r];
-            }
-        }
-    }
-    __syncthreads();
-
-    const bool vec_ok = (EPI < 0) ? (p.N % 4 == 0 && reinterpret_cast<uintptr_t>(p.C) % 16 == 0)
-                                  : (p.N % 4 == 0 && reinterpret_cast<uintptr_t>(p.y) % 8 == 0);
-    const uint32_t xbase = l16 * XS + g * 16;
-    for (uint32_t it = 0; it < items; ++it) {
-        v4i acc[RB];
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) acc[rb] = v4i{0, 0, 0, 0};
-        for (uint32_t blk = 0; blk < nblk; ++blk) {
-            const bool last = blk + 1 == nblk;
-            const uint32_t nit = last ? it + 1 : it, nb = last ? 0 : blk + 1;
-#pragma unroll
-            for (int j = 0; j < kRing; ++j) {
-                const v4u w = ring[j];
-                issue(nit, nb, j);
-                // segments past the slice carry zero weights; their activation read only has to stay inside the row
-                const uint32_t xoff = min((seg_lo + blk * kRing + j) * 64, (uint32_t)XBYTES - 64);
-                v4u we, wo;
-                expand_nibbles(w, we, wo);
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                    const v4u x = *reinterpret_cast<const v4u *>(xs + rb * 16 * XS + xbase + xoff);
-                    v4u xe, xo;
-                    expand_nibbles(x, xe, xo);
-                    acc[rb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, we),
-                                                                   __builtin_bit_cast(v4i, xe), acc[rb], 0, 0, 0);
-                    acc[rb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, wo),
-                                                                   __builtin_bit_cast(v4i, xo), acc[rb], 0, 0, 0);
-                }
-            }
-        }
-        const uint32_t tile = tile_of(it);
-        if (kslices > 1) {
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) part[wave][rb][lane] = acc[rb];
-            __syncthreads();
-            if (slice == 0)
-                for (uint32_t s2 = 1; s2 < kslices; ++s2)
-#pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) {
-                        const v4i o = part[wave + s2][rb][lane];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[rb][r] += o[r];
-                    }
-            __syncthreads();  // the partial sums are consumed before the next tile overwrites them
-        }
-        if (slice == 0) {
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[rb][r] >>= 8;
-                store_quad<EPI, BIAS>(p, m_base + rb * 16 + l16, tile * 16 + g * 4, acc[rb], vec_ok);
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------------
 // dot kernel (M <= 4, rows longer than 16384 elements): weight streaming on v_dot8_i32_i4
 // ---------------------------------------------------------------------------------
 // The signed 4-bit dot product instruction consumes packed nibbles as they lie in memory,
@@ -775,7 +643,7 @@ __global__ __launch_bounds__(256) void gemv_s4_dot_kernel(DUQ_HEAD_DECL, GemmPar
 // dispatch
 // ---------------------------------------------------------------------------------
 // Which kernel family takes a shape.  Host arithmetic only, so that the rule can be tested without a GPU:
-// every kernel whose weight offsets are 32-bit (decode, dot, ring: row * K/2 + offset, and a buffer descriptor
+// every kernel whose weight offsets are 32-bit (decode, dot: row * K/2 + offset, and a buffer descriptor
 // over the whole tensor) is reachable only while the packed weights stay below 4 GiB - 256 (the out-of-range
 // marker); larger tensors go to the stream / prefill kernels, whose descriptors and pointers are per tile
 // (64-bit base, 32-bit offsets inside 256 rows).
@@ -783,13 +651,11 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
 {
     const uint64_t wbytes = (uint64_t)N * (K / 2);
     const bool small_offsets = wbytes < 0xFFFFFF00ull && K > 0;
-    // decode.  Rows kernel for up to four rows (8 KB of every weight row per wavefront); above, the MFMA decode
-    // kernel (6 KB per row over eight wavefronts), with two to four row tiles against the same weight fragments
-    // for 17..64 rows as far as the fragments fit in registers (64 rows of at most 8192 elements, 48 of at most
-    // 12288).  Two exceptions, both measured: 9..16 rows on very wide layers run the skinny kernel (whole-line
-    // weight loads, 5 % faster at N = 28672, K = 4096), and the long-row forms (more than 32 rows of more than 4096
-    // elements, any of more than 8192) need 192 column tiles: on narrower layers the ring kernel, which splits K
-    // over workgroups, is ahead (48 x 1024 x 8192: 7.9 against 10.2 us; 48 x 3072 x 12288: 20.6 against 14.1).
+    // The launcher asks takes_wide_kernel and takes_lds_kernel first; what is said here of up to 64 rows and of narrow problems
+    // holds for the shapes that those leave.  Decode: rows kernel for up to four rows (8 KB of every weight row per
+    // wavefront); above, the MFMA decode kernel (rows of up to 8192 elements), with two to four row tiles against the same
+    // weight fragments for 17..64 rows.  9..16 rows on very wide layers run the skinny kernel (whole-line weight loads, 5 %
+    // faster at N = 28672, K = 4096).
     if (M <= 4 && K <= 16384 && small_offsets) return kKernelDecodeRows;
     if (M <= 16 && small_offsets) {
         if (M > 8 && (N + 15) / 16 >= 1536 && K <= 4096) return kKernelSkinny;
@@ -798,10 +664,8 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
     if (M <= 64 && small_offsets) {
         // one round of 64 x 64 tiles of the prefill kernel, whose time hardly depends on rows and columns, is ahead of the
         // decode kernel where that has many row tiles or several column tiles per workgroup.  More than 48 rows: 64 x
-        // 11008 x 4096 9.8 against 10.65 us, 64 x 13824 x 1024 6.6 / 8.2 (but N = 8192 8.6 either way), 64 x 4096 x 8192
-        // 11.5 / 13.5, 56 x 3072 x 5120 9.3 / 10.1; 40 x 5120 x 5120 9.3 / 11.2, 40 x 11008 x 8192 14.8 / 18.6 (but 48 x 4096
-        // x 8192 11.5 / 11.3); 32 x 13824 x 5120 11.8 / 13.6, 32 x 16384 x 8192 18.3 / 20.0 (but 17 x 16384 x 8192 19.3 /
-        // 18.4, 32 x 8192 x 5120 9.3 / 8.65).
+        // 11008 x 4096 9.8 against 10.65 us, 64 x 13824 x 1024 6.6 / 8.2; 40 x 11008 x 8192 14.8 / 18.6; 32 x 13824 x 5120 11.8 /
+        // 13.6, 32 x 16384 x 8192 18.3 / 20.0 (but 17 x 16384 x 8192 19.3 / 18.4).
         const bool tiles = K <= 4096 ? M > 48 && N > 8192 && K >= 1024
                          : K <= 8192 && (M > 48 ? N >= 3072 : M > 32 ? N >= 5120 : M > 24 && N > 10240);
         if (tiles && N <= 16384) return kKernelStream;
@@ -814,13 +678,9 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
     const uint32_t xstride = ((K / 2 + 127) / 128) * 128;
     // dot kernel: up to four rows too long for the decode kernels
     if (M <= 4 && small_offsets && 4 * xstride <= 60 * 1024) return kKernelDot;
-    // ring kernel: 17..256 rows in groups whose packed activations fit in LDS, while one column tile per CU and row group
-    // is one round of workgroups; every further round streams the weights again, and the prefill kernel's 64 x 64 tiles
-    // are ahead or equal (128 x 1024 x 8192, 256 workgroups: 8.2 against 11.4 us, 192 rows 14.5 / 11.5; 64 x 2048 x 8192
-    // 8.2 / 11.4, 100 rows 14.6 / 11.5; 72 x 1536 x 8192 13.4 / 11.3; 64 x 1024 x 16384 10.0 / 17.1, 100 rows 17.4 / 17.3, 192
-    // rows 26.1 / 17.4; 144 x 1536 x 4096 12.75 / 8.5).  More than 64 rows of at most 2048 elements: the tiles are ahead
-    // in any case (72 x 512 x 2048 7.2 / 6.4).  And 5..16 rows of 12289..16384 elements.
-    const uint32_t rb_max = K <= 4096 ? 4 : (K <= 8192 ? 2 : 1);  // 16-row blocks whose activations fit in LDS
+    // a bucket of narrow problems, all of which the LDS kernel takes: 17..256 rows in groups of 64, 32 or 16 whose column tiles
+    // are one round of workgroups, and 5..16 rows of 8193..16384 elements
+    const uint32_t rb_max = K <= 4096 ? 4 : (K <= 8192 ? 2 : 1);
     const uint32_t row_groups = ((M + 15) / 16 + rb_max - 1) / rb_max;
     const bool one_round = M > 16 && M <= 256 && (uint64_t)((N + 15) / 16) * row_groups <= 256 && (K > 2048 || M <= 64);
     const bool long_rows = M <= 16 && K > 8192;
@@ -869,31 +729,6 @@ static void launch_epi(GemmParams &p, hipStream_t stream, uint32_t batch = 1)
             DUQ_LAUNCH_HEAD((gemm_s4_skinny_kernel<4, EPI, BIAS>), grid, dim3(256), 0, stream, p);
         else
             DUQ_LAUNCH_HEAD((gemm_s4_skinny_kernel<8, EPI, BIAS>), grid, dim3(512), 0, stream, p);
-        return;
-    }
-    if (kernel == kKernelRing) {
-        const uint32_t rb_all = (p.M + 15) / 16;
-        const uint32_t rb_max = p.K <= 4096 ? 4 : (p.K <= 8192 ? 2 : 1);
-        const uint32_t rb = std::min(rb_all, rb_max);
-        const uint32_t row_groups = (rb_all + rb - 1) / rb;
-        const uint32_t ntiles = (p.N + 15) / 16;
-        const uint32_t segs = (p.K / 2 + 63) / 64;
-        // wavefronts splitting K for one tile: as few as give the chip ~2048 wavefronts, slices of at
-        // least 512 bytes per row
-        uint32_t kslices = 1;
-        while (ntiles * kslices < 2048 && kslices < 4 && segs / (kslices * 2) >= (uint32_t)kRing) kslices *= 2;
-        const uint32_t groups = (ntiles + 4 / kslices - 1) / (4 / kslices);
-        const uint32_t xbytes = p.K <= 4096 ? 2048 : (p.K <= 8192 ? 4096 : 8192);
-        const uint32_t lds = 16 * rb * (xbytes + 16) + 4 * rb * 1024;
-        const uint32_t slots = 256 * std::max(1u, std::min(8u, (160u * 1024) / lds));
-        p.tiles_m = kslices;
-        p.tiles_n = (groups + slots - 1) / slots;
-        const dim3 grid((groups + p.tiles_n - 1) / p.tiles_n, row_groups);
-#define DUQ_RING(X, R) DUQ_LAUNCH_HEAD((gemm_s4_ring_kernel<X, R, EPI, BIAS>), grid, dim3(256), 0, stream, p)
-        if (xbytes == 8192) DUQ_RING(8192, 1);
-        else if (xbytes == 4096) DUQ_RING(4096, 2);
-        else DUQ_RING(2048, 4);
-#undef DUQ_RING
         return;
     }
     }

@@ -77,13 +77,28 @@ enum GemmKernelId {
     kKernelDecodeRows = 1,  // duq_decode.hip, v_dot8_i32_i4, M <= 4
     kKernelDecodeMfma = 2,  // duq_decode.hip, MFMA, 5 <= M <= 16 (K <= 12288), 17 <= M <= 64 (K <= 8192; 48 rows: 12288)
     kKernelDot = 3,         // duq_gemm.hip, M <= 4 with rows longer than 16384 elements
-    kKernelRing = 4,        // duq_gemm.hip, 17 <= M <= 256 on narrow problems the decode kernel does not take
+    kKernelRing = 4,        // 17 <= M <= 256 on narrow problems: all of them shapes of the LDS kernel
     kKernelSkinny = 5,      // duq_gemm.hip, 9 <= M <= 16 with 1536 or more column tiles, K <= 4096
     kKernelStream = 6,      // duq_prefill.hip (duq_gemm.hip for short rows), prefill
     kKernelTile = 7,        // the same kernels on problems of few tiles or rows too long for the others
 };
 int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K);
-// Shapes of the LDS kernel (duq_decode.hip), asked before select_gemm_kernel's families (whose number such a shape keeps:
+// Tile of the LDS kernel in 16 x 16 units: the first of these, in the order of their time (64 x 4096 x 4096, one round of 256
+// workgroups: 4.0, 4.4, 4.5, 5.2, 5.4, 5.9, 6.1, 6.8 us), whose workgroups, a column range and a group of rows each, are one
+// round.  More row groups read the weights again, from their XCD's cache: 64 x 1024 x 8192 6.6 us with four row tiles each,
+// 4.4 with one; 128 x 1024 x 16384 9.1 with two row tiles, 17.2 on tiles of the prefill kernel.  rows = 0: none.
+struct LdsShape {
+    uint32_t rows, cols;
+};
+inline LdsShape lds_shape(uint32_t M, uint32_t N)
+{
+    const LdsShape order[8] = {{1, 1}, {2, 1}, {1, 2}, {3, 1}, {2, 2}, {4, 1}, {3, 2}, {4, 2}};
+    const uint64_t rows = (M + 15) / 16, cols = (N + 15) / 16;
+    for (const LdsShape &t : order)
+        if ((rows + t.rows - 1) / t.rows * ((cols + t.cols - 1) / t.cols) <= 256) return t;
+    return rows <= 4 ? LdsShape{(uint32_t)rows, 2} : LdsShape{0, 0};
+}
+// Shapes of the LDS kernel (duq_decode.hip), asked next and before select_gemm_kernel's families (whose number such a shape keeps:
 // the buckets there are by size).  Measured against those on 900 shapes, us:
 //  - 5..64 rows: every length on up to 4096 columns (7 - 75 % less; 16 x 512 x 1024 3.2 -> 2.9, 64 x 1024 x 8192 7.9 -> 6.7, 16
 //    x 512 x 28672 25.6 -> 7.2).  Up to 8192 columns where the rows are many or long (64 x 5120 x 5120 9.6 -> 7.9, 16 x 8192 x
@@ -92,13 +107,20 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K);
 //    registers over several column tiles, one fetch of them per CU).  More columns: the lengths that the MFMA kernel does not
 //    hold and for which the ring kernel streams the weights twice (16 x 12288 x 14336 26.8 -> 20.0, 32 x 16384 x 11008 26.9 ->
 //    23.0; 48 x 11008 x 11008 19.8 -> 22.6).
+//  - more rows while one round of its workgroups covers them (lds_shape), from 512 elements on, in its largest tile from
+//    1024 elements on and up to 1024 rows (128 x 1024 x 512 4.4 -> 3.6, x 28672 25.8 -> 11.3; 200 x 2048 x 1024 5.5 -> 5.0, but 128 x
+//    4000 x 512 4.6 -> 5.1 and 7787 x 58 x 6528 11.9 -> 12.5).
 //  - up to 4 rows longer than the rows kernel's 16384 (the dot kernel, one weight row per wavefront pair, or beyond 30720 a
 //    prefill tile): up to 4096 columns (4 x 2606 x 28672 13.4 -> 8.1, 1 x 1024 x 40000 34.2 -> 8.3), above for 3 and 4 rows (4 x
 //    8192 x 28672 28.9 -> 21.8, but 4 x 8192 x 16448 18.6 -> 20.1) and beyond 30720 (1 x 8192 x 40000 49.4 -> 31.1; 1 x 8192 x
 //    28672 21.5 against 22.0).
 inline bool takes_lds_kernel(uint32_t M, uint32_t N, uint32_t K)
 {
-    if (M == 0 || M > 64 || K == 0 || K > 65536 || (uint64_t)N * (K / 2) >= 0xFFFFFF00ull) return false;
+    if (M == 0 || K == 0 || K > 65536 || (uint64_t)N * (K / 2) >= 0xFFFFFF00ull) return false;
+    if (M > 64) {
+        const LdsShape t = lds_shape(M, N);
+        return t.rows > 0 && (t.rows * t.cols < 8 ? K >= 512 : K >= 1024 && M <= 1024);
+    }
     if (M <= 4) return K > 16384 && (N <= 4096 || (N <= 16384 && K > (M > 2 ? 18432 : 30720)));
     if (N <= 4096) return true;
     if (N <= 8192) return M > 32 || K > 4096 || (M > 16 && (K <= 2048 || (N <= 6144 && K % 256 == 0)));

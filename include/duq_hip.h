@@ -223,12 +223,13 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
 
 /* Which kernel family duq_matmul_host_4bit / duq_linear4bit_forward run for a shape (no GPU work; for tests
  * and tuning): 1 decode rows kernel (M <= 4), 2 decode MFMA kernel (M <= 16; up to 64 rows of at most 8192
- * elements, 48 of at most 12288, where family 6 is not ahead), 3 dot kernel (M <= 4, rows longer than 16384 elements), 4 ring kernel, 5 skinny
- * kernel (9 <= M <= 16, very wide problems), 6 prefill kernel (short rows: stream kernel),
- * 7 the same on problems of few tiles or long rows.  Families 1-5 address the weight tensor with 32-bit byte offsets and are only picked while
- * N * K / 2 < 2^32 - 256; larger tensors run families 6 and 7, whose bases are 64-bit per tile.  The families are buckets
- * by size: of those with up to 64 rows, the problems of up to 4096 columns (8192 where the rows are many or long), some
- * of very long rows and some of more columns run the decode kernels' LDS and wide forms, whatever the bucket.  No
+ * elements, 48 of at most 12288, where family 6 is not ahead), 3 dot kernel (M <= 4, rows longer than 16384 elements),
+ * 4 narrow problems, 5 skinny kernel (9 <= M <= 16, very wide problems), 6 prefill kernel (short rows: stream kernel),
+ * 7 the same on problems of few tiles or long rows.  Families 1-5 address the weight tensor with 32-bit byte offsets and are
+ * only picked while N * K / 2 < 2^32 - 256; larger tensors run families 6 and 7, whose bases are 64-bit per tile.  The
+ * families are buckets by size: below that limit the decode kernels' LDS form (5..64 rows on up to 4096 columns, 8192 where the
+ * rows are many or long, more rows while its tiles are one round of workgroups, very long rows) and wide form (some problems
+ * of up to 64 rows and more than 8192 columns) come first, whatever the bucket.  No
  * counterpart in the reference (CUTLASS picks its own tile, src/kernels/gemm.cu:17-42). */
 int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
 /* For a shape of family 6: its tile as rows * 1000 + columns (256256, 128256, 192128, 128128, 64128, 96064, 64064; the fused
