@@ -596,13 +596,15 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
     for (int ni = 0; ni < TNI; ++ni) {
         const uint32_t ncol = ni * 16 + kb * 4;
         const uint32_t nq = min(n0 + wave * (16 * TNI) + ncol, p.N - 4);
-        const QuadCols<MODE, BIAS> cols =
-            quad_cols_from_raw<MODE, BIAS>(raw_s1[ni], raw_z1[ni], raw_s2[ni], raw_z2[ni], raw_bias[ni], nq, raw_rs[ni]);
+        PairCols<MODE, BIAS> cols[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            cols[k] = pair_cols_from_raw<MODE, BIAS>(raw_s1[ni], raw_z1[ni], raw_s2[ni], raw_z2[ni], raw_bias[ni], nq, k, raw_rs[ni]);
 #pragma unroll
         for (int mi = 0; mi < TMI; ++mi) {
             *reinterpret_cast<v2u *>(stage + (mi * 16 + l16) * kYStride + ncol * 2) =
-                v2u{dequant_pair<MODE, BIAS>(acc[mi][ni][0], acc[mi][ni][1], rowp[mi], cols.c[0], cols.c[1]),
-                    dequant_pair<MODE, BIAS>(acc[mi][ni][2], acc[mi][ni][3], rowp[mi], cols.c[2], cols.c[3])};
+                v2u{dequant_pair<MODE, BIAS>(acc[mi][ni][0], acc[mi][ni][1], rowp[mi], cols[0]),
+                    dequant_pair<MODE, BIAS>(acc[mi][ni][2], acc[mi][ni][3], rowp[mi], cols[1])};
         }
     }
     }

@@ -131,43 +131,72 @@ __device__ __forceinline__ uint16_t dequant_one(float acc, const RowEpi &r, cons
     return f16_to_bits(y);
 }
 
+// Column-side parameters of two neighbouring columns, packed as the binary16 instructions take them.  (As two ColParams, whose
+// three halves the compiler packs and unpacks through memory where there are zero points and a bias, they end up in LDS, at an
+// address for which the kernel reads its dispatch packet, in host memory: 11 to 16 us a launch.  512 x 4096 x 4096, asymmetric
+// with bias, 27.6 -> 11.8 us, 100 x 11008 x 4096 23.5 -> 10.5, 2048 x 4096 x 4096 47.1 -> 31.8.)
+template <int MODE, bool BIAS>
+struct PairCols {
+    v2h s, z, bias;
+    int rs0, rs1;  // mode 4
+};
+
+// Columns n0 + 2 * half and the next one, from raw 64-bit words fetched earlier (four binary16 values per word, column n0
+// first); the column's range chooses between the two sets of the dual modes (as load_col).
+template <int MODE, bool BIAS>
+__device__ __forceinline__ PairCols<MODE, BIAS> pair_cols_from_raw(v2u s1, v2u z1, v2u s2, v2u z2, v2u bias, uint32_t n0, int half,
+                                                                   v4i rs = v4i{0, 0, 0, 0})
+{
+    const uint32_t col = n0 + 2 * half, first = MODE == 2 ? (uint32_t)kQuantColK : 1u;  // columns of the first set
+    const uint32_t set1 = (col < first ? 0xFFFFu : 0u) | (col + 1 < first ? 0xFFFF0000u : 0u);
+    auto pick = [&](v2u a, v2u b) { return (MODE == 2 || MODE == 3) ? (a[half] & set1) | (b[half] & ~set1) : (uint32_t)a[half]; };
+    PairCols<MODE, BIAS> c;
+    c.s = __builtin_bit_cast(v2h, pick(s1, s2));
+    c.z = __builtin_bit_cast(v2h, (MODE == 1 || MODE == 3 || MODE == 4) ? pick(z1, z2) : 0u);
+    const uint32_t b = BIAS ? bias[half] : 0u;
+    c.bias = __builtin_bit_cast(v2h, b);
+    c.rs0 = MODE == 4 ? rs[2 * half] : 0;
+    c.rs1 = MODE == 4 ? rs[2 * half + 1] : 0;
+    return c;
+}
+
 // Two neighbouring columns of one row at once, on the packed binary16 instructions (each lane of a
-// packed operation rounds like the scalar one): the low half of the result is column c0.
+// packed operation rounds like the scalar one): the low half of the result is the first column.
 template <int MODE, bool BIAS, typename ACC>
-__device__ __forceinline__ uint32_t dequant_pair(ACC acc0, ACC acc1, const RowEpi &r, const ColParams &c0,
-                                                 const ColParams &c1)
+__device__ __forceinline__ uint32_t dequant_pair(ACC acc0, ACC acc1, const RowEpi &r, const PairCols<MODE, BIAS> &c)
 {
     if (MODE == 4)
-        return (uint32_t)dequant_one<MODE, BIAS>(acc0, r, c0) | ((uint32_t)dequant_one<MODE, BIAS>(acc1, r, c1) << 16);
+        return (uint32_t)dequant_one<MODE, BIAS>(acc0, r, ColParams{c.s[0], c.z[0], c.bias[0], c.rs0}) |
+               ((uint32_t)dequant_one<MODE, BIAS>(acc1, r, ColParams{c.s[1], c.z[1], c.bias[1], c.rs1}) << 16);
     const v2h e = v2h{(f16)(float)acc0, (f16)(float)acc1};  // int32 or integer-valued float32: one rounding
-    const v2h ss = v2h{r.s, r.s} * v2h{c0.s, c1.s};
+    const v2h ss = v2h{r.s, r.s} * c.s;
     v2h y;
     if (MODE == 0 || MODE == 2) {
         y = ss * e;
     } else {
-        const v2h t = (e - v2h{r.z, r.z}) - v2h{c0.z, c1.z};
+        const v2h t = (e - v2h{r.z, r.z}) - c.z;
         y = ss * t;
     }
-    if (BIAS) y = y + v2h{c0.bias, c1.bias};
+    if (BIAS) y = y + c.bias;
     return __builtin_bit_cast(uint32_t, y);
 }
 
 // The same for integer accumulators carried x 256: the factor goes in one instruction with the conversion to binary16
 // (exact: the float32 of 256 * acc is, below 2^24, and so is its 256th part) instead of a shift per accumulator.
 template <int MODE, bool BIAS>
-__device__ __forceinline__ uint32_t dequant_pair_x256(int acc0, int acc1, const RowEpi &r, const ColParams &c0, const ColParams &c1)
+__device__ __forceinline__ uint32_t dequant_pair_x256(int acc0, int acc1, const RowEpi &r, const PairCols<MODE, BIAS> &c)
 {
-    if (MODE == 4) return dequant_pair<MODE, BIAS>(acc0 >> 8, acc1 >> 8, r, c0, c1);
-    return dequant_pair<MODE, BIAS>((float)acc0 * (1.0f / 256.0f), (float)acc1 * (1.0f / 256.0f), r, c0, c1);
+    if (MODE == 4) return dequant_pair<MODE, BIAS>(acc0 >> 8, acc1 >> 8, r, c);
+    return dequant_pair<MODE, BIAS>((float)acc0 * (1.0f / 256.0f), (float)acc1 * (1.0f / 256.0f), r, c);
 }
 
 // The same for accumulators that started at the bits of kF32Base (short rows: |256 * acc| <= 2^22): read as a float they are
 // kF32Base + acc, whose last place is 2^-8 up to 2^16.
 constexpr float kF32Base = 49152.0f;  // 1.5 * 2^15
 template <int MODE, bool BIAS>
-__device__ __forceinline__ uint32_t dequant_pair_based(int acc0, int acc1, const RowEpi &r, const ColParams &c0, const ColParams &c1)
+__device__ __forceinline__ uint32_t dequant_pair_based(int acc0, int acc1, const RowEpi &r, const PairCols<MODE, BIAS> &c)
 {
-    return dequant_pair<MODE, BIAS>(__builtin_bit_cast(float, acc0) - kF32Base, __builtin_bit_cast(float, acc1) - kF32Base, r, c0, c1);
+    return dequant_pair<MODE, BIAS>(__builtin_bit_cast(float, acc0) - kF32Base, __builtin_bit_cast(float, acc1) - kF32Base, r, c);
 }
 
 // Row-sum epilogue of the dual-uniform layer for one output (definition: include/duq_hip.h,
@@ -255,81 +284,6 @@ __device__ __forceinline__ uint16_t dual_finish(int acc, const DualRow &r, const
 {
     return dual_rowsum_one<false>(acc, r.xlo, r.xhi, r.zx, r.rxl, r.rxr, r.sx, c.wlo, c.whi, c.s1, c.s2, c.z1, c.z2, c.a1, c.a2,
                                   bias, c.bias);
-}
-
-// Column parameters of four consecutive output columns n0 .. n0+3, fetched with 64-bit
-// loads when the arrays allow it (`vec`: 8-byte aligned bases and n0 + 3 < cols).
-template <int MODE, bool BIAS>
-struct QuadCols {
-    ColParams c[4];
-};
-
-__device__ __forceinline__ void load4_f16(const uint16_t *ptr, uint32_t n0, uint32_t cols, bool vec, uint16_t (&out)[4])
-{
-    if (vec && n0 + 3 < cols) {
-        const v2u v = *reinterpret_cast<const v2u *>(ptr + n0);
-        out[0] = (uint16_t)(v[0] & 0xFFFFu);
-        out[1] = (uint16_t)(v[0] >> 16);
-        out[2] = (uint16_t)(v[1] & 0xFFFFu);
-        out[3] = (uint16_t)(v[1] >> 16);
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) out[r] = ptr[min(n0 + r, cols - 1)];
-    }
-}
-
-template <int MODE, bool BIAS>
-__device__ __forceinline__ QuadCols<MODE, BIAS> load_quad_cols(const uint16_t *s1, const uint16_t *z1,
-                                                               const uint16_t *s2, const uint16_t *z2,
-                                                               const uint16_t *bias, uint32_t n0, uint32_t cols,
-                                                               bool vec, const int32_t *rs = nullptr)
-{
-    QuadCols<MODE, BIAS> q;
-    uint16_t a[4], b[4];
-    load4_f16(s1, n0, cols, vec, a);
-    if (MODE == 2 || MODE == 3) load4_f16(s2, n0, cols, vec, b);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t col = n0 + r;
-        const bool first = MODE == 2 ? col < (uint32_t)kQuantColK : col == 0;  // see load_col
-        q.c[r].s = bits_to_f16((MODE == 2 || MODE == 3) ? (first ? a[r] : b[r]) : a[r]);
-        q.c[r].z = (f16)0;
-        q.c[r].bias = (f16)0;
-        q.c[r].rs = MODE == 4 ? rs[min(col, cols - 1)] : 0;
-    }
-    if (MODE == 1 || MODE == 3 || MODE == 4) {
-        load4_f16(z1, n0, cols, vec, a);
-        if (MODE == 3) load4_f16(z2, n0, cols, vec, b);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) q.c[r].z = bits_to_f16(MODE == 3 ? ((n0 + r) == 0 ? a[r] : b[r]) : a[r]);
-    }
-    if (BIAS) {
-        load4_f16(bias, n0, cols, vec, a);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) q.c[r].bias = bits_to_f16(a[r]);
-    }
-    return q;
-}
-
-// Same selection as load_quad_cols, from raw 64-bit words fetched earlier (four binary16
-// values per word, column n0 first).
-template <int MODE, bool BIAS>
-__device__ __forceinline__ QuadCols<MODE, BIAS> quad_cols_from_raw(v2u s1, v2u z1, v2u s2, v2u z2, v2u bias, uint32_t n0,
-                                                                   v4i rs = v4i{0, 0, 0, 0})
-{
-    auto pick = [](v2u v, int r) -> uint16_t { return (uint16_t)((r & 1) ? (v[r >> 1] >> 16) : (v[r >> 1] & 0xFFFFu)); };
-    QuadCols<MODE, BIAS> q;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t col = n0 + r;
-        const bool first = MODE == 2 ? col < (uint32_t)kQuantColK : col == 0;
-        q.c[r].s = bits_to_f16((MODE == 2 || MODE == 3) ? (first ? pick(s1, r) : pick(s2, r)) : pick(s1, r));
-        q.c[r].rs = MODE == 4 ? rs[r] : 0;
-        q.c[r].z = (MODE == 1 || MODE == 4) ? bits_to_f16(pick(z1, r))
-                               : (MODE == 3 ? bits_to_f16(col == 0 ? pick(z1, r) : pick(z2, r)) : (f16)0);
-        q.c[r].bias = BIAS ? bits_to_f16(pick(bias, r)) : (f16)0;
-    }
-    return q;
 }
 
 }  // namespace duq
