@@ -178,7 +178,9 @@ __device__ __forceinline__ void prefill_tile(GemmParams &p, uint8_t *lds, uint32
     // (KS = 8: wavefronts T and up finish nothing, and fetch parameters of the last tile)
     const uint32_t mine = KS == 8 ? min(ks, (uint32_t)T - 1) : ks;
     const uint32_t wm0 = m0 + wm * (32 * WTM) + (mine >> 1) * (32 * TM), wn0 = n0 + wn * (32 * WTN) + (mine & 1u) * (32 * TN);
-    constexpr bool kLdsParams = false;
+    // (the 256 x 256 tile stages its parameters in LDS: next to 128 accumulators the eight quads of up to five arrays do not fit
+    // in registers, and spilled or not by form: 4096 x 8192 x 4096, dual scales and zero points, 124 us spilled, 104 staged)
+    constexpr bool kLdsParams = LATE;
 #include "duq_stream_epilogue_fetch.inc"
     if (!LATE) fetch_params();
     if constexpr (STEPS == 1) {
