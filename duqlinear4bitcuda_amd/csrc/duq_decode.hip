@@ -742,16 +742,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DEC
 // own, where a column range leaves compute units without work: 64 x 1024 x 8192 7.9 -> 4.4, 128 x 1024 x 8192 8.2 -> 5.4, 256 x
 // 2048 x 4096 9.0 -> 7.4, 96 x 4096 x 11008 14.3 -> 10.4 (64 x 64 tiles of the prefill kernel: half the workgroups and twice the
 // operands each).
-template <int MT, int NT>
-struct LdsTile {
-    static constexpr int G = NT == 1 ? 1 : 8;            // wavefronts that share a stage
-    static constexpr int RB = G == 1 ? 128 : 512;        // bytes of a row in it
-    static constexpr int DEPTH = G == 1 ? 2 : 3;         // stages
-    static constexpr int U = RB / (64 * G);              // a wavefront's 64-byte fragments of a row in a stage
-    static constexpr int L = (MT + NT) * U;              // load instructions of a wavefront and stage, a kilobyte each
-    static constexpr int kStage = G * L * 1024, kLds = 8 / G * DEPTH * kStage, kPart = NT * MT * 8 * 1024;
-    static_assert(kLds <= 160 * 1024 && kPart <= kLds, "LDS");
-};
 template <int MT, int NT, int EPI>
 __global__ __launch_bounds__(512) void gemm_s4_lds_kernel(DUQ_HEAD_DECL, DecodeParams tail)
 {

@@ -747,6 +747,193 @@ __global__ __launch_bounds__(512) void gemm_s8_split_kernel(DUQ_HEAD_DECL, Gemm8
 }
 
 // ---------------------------------------------------------------------------------
+// LDS kernel: few rows, and more on narrow problems (what lds8_takes gives it)
+// ---------------------------------------------------------------------------------
+// The kernels below take their activations (and row-major weights) in the layout of the matrix instruction, sixteen bytes of
+// each of sixteen rows from neighbouring lanes, a cache line per lane, which a CU serves at a quarter of its rate; and long
+// rows on few columns leave most compute units without a workgroup.  Here both operands come through LDS without registers, in
+// whole pieces of a row (tiled weights: in runs of 256 bytes), as in the 4-bit LDS kernel, whose tiles, stages and groups of rows
+// these are.  Measured (N x K, tiled weights, us): 16 rows 4096 x 4096 6.5 -> 5.5, 4096 x 11008 14.8 -> 9.2, 250 x 8192 8.7 -> 4.5; 32
+// rows 8.1 -> 5.8, 20.4 -> 10.4 (45 MB: 4.3 TB/s), 12.8 -> 4.5; 128 rows 10.9 -> 9.4, 20.6 -> 18.7, 15.6 -> 5.7.
+template <int MT, int NT, bool FUSED, bool BIAS, bool TILED>
+__global__ __launch_bounds__(512) void gemm_s8_lds_kernel(DUQ_HEAD_DECL, Gemm8Params tail)
+{
+    Gemm8Params p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.A);
+    to_global(p.B);
+    to_global(p.C);
+    to_global(p.y);
+    using Tile = LdsTile<MT, NT>;
+    constexpr int G = Tile::G, U = Tile::U, L = Tile::L, DEPTH = Tile::DEPTH;
+    constexpr uint32_t RB = Tile::RB, kStage = Tile::kStage;
+    constexpr int FT = (MT * NT + 1) / 2;  // output tiles a group of 256 threads finishes
+    static_assert(DEPTH >= 2 && DEPTH * L <= 63, "vmcnt");
+    __shared__ __attribute__((aligned(256))) uint8_t lds[Tile::kLds];
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t l16 = lane & 15u, g = lane >> 4;
+    // groups of 16 * MT rows share the weights of a column tile: consecutive in `at`, an eighth of which runs on one XCD
+    const uint32_t groups = p.tiles_m & 0x1FFu, per_xcd = ((p.N + 16 * NT - 1) / (16 * NT) * groups + 7) / 8;
+    const uint32_t at = blockIdx.x % 8 * per_xcd + blockIdx.x / 8, tile = at * (p.tiles_m >> 9) >> 16;  // (tile = at / groups)
+    const uint32_t n0 = tile * (16 * NT), m0 = (at - tile * groups) * (16 * MT);
+    if (n0 >= p.N) return;
+    const auto desc = [](const int8_t *base, uint32_t bytes) {
+        const uint64_t a = reinterpret_cast<uint64_t>(base);
+        return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
+                   (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+    };
+    const v4u dX = desc(p.A + (uint64_t)m0 * p.K, min(p.M - m0, 16u * MT) * p.K);  // rows past M and N read as zero
+    // (tiled: the whole 32-row tile, zero-padded past N, of which NT = 1 takes the lower or the upper half)
+    const v4u dW = TILED ? desc(p.B + (uint64_t)(n0 / 32) * 32 * p.K, 32u * p.K) : desc(p.B + (uint64_t)n0 * p.K, min(p.N - n0, 16u * NT) * p.K);
+
+    // ---- global -> LDS: instruction j of a group's wavefront v takes kilobyte j * G + v of the stage, activations first; a
+    // row's 16-byte pieces lie at piece ^ (row / Q).  Tiled weights: sixteen rows of a piece side by side, as they come.
+    constexpr uint32_t PR = RB / 16, RPI = 64 / PR, Q = RB < 256 ? 256 / RB : 1;  // pieces a row, rows an instruction
+    const uint32_t group = G == 1 ? wave : 0, v = G == 1 ? 0 : wave;
+    const uint32_t r0 = v * RPI + lane / PR, row0 = r0 * p.K;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds + group * (DEPTH * kStage) + v * 1024;
+    auto load = [&](uint32_t step, uint32_t slot) {
+        const uint32_t k = (step * (8 / G) + group) * RB;
+        uint32_t off[2];  // (of even and odd instructions: rows 16 apart swizzle alike)
+        bool in[2];
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+            off[o] = k + ((lane % PR) ^ ((o * (G * RPI) + r0) % 16 / Q)) * 16;
+            in[o] = off[o] < p.K;  // K % 32 == 0: a 16-byte piece is all in or all out
+        }
+#pragma unroll
+        for (int j = 0; j < L; ++j) {
+            const int jw = j - MT * U;
+            uint32_t from = kOobOffset;
+            if (TILED && jw >= 0) {
+                const uint32_t piece = (uint32_t)(jw % U * G + v) * 4 + (lane >> 4), half = NT == 2 ? (uint32_t)(jw / U) : n0 / 16 & 1u;
+                if (k + piece * 16 < p.K) from = (k / 32 + piece / 2) * 1024 + ((piece & 1u) * 32 + half * 16 + l16) * 16;
+            } else if (in[j % 2]) {
+                from = row0 + (uint32_t)(jw < 0 ? j : jw) * (G * RPI) * p.K + off[j % 2];
+            }
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds0 + slot + j * (G * 1024)), "v"(from),
+                         "s"(jw < 0 ? dX : dW)
+                         : "memory", "m0");
+        }
+    };
+    static_assert(G * RPI == 8 || G * RPI == 16, "the two swizzles above");
+    // ---- LDS -> registers: 64 bytes of a row make a fragment
+    v4i x[MT][U], w[NT][U];
+    const uint8_t *const own = lds + group * (DEPTH * kStage);
+    auto read = [&](uint32_t slot) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t piece = (v * U + u) * 4 + g, swizzled = l16 * RB + (piece ^ (l16 / Q)) * 16;
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                w[n][u] = *reinterpret_cast<const v4i *>(own + slot + (MT + n) * (16 * RB) + (TILED ? piece * 256 + l16 * 16 : swizzled));
+#pragma unroll
+            for (int m = 0; m < MT; ++m) x[m][u] = *reinterpret_cast<const v4i *>(own + slot + m * (16 * RB) + swizzled);
+        }
+    };
+    v4i acc[NT][MT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[n][m] = v4i{0, 0, 0, 0};
+    const uint32_t steps = (p.K + 8 / G * RB - 1) / (8 / G * RB);
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s) load(s, s * kStage);
+
+    // the parameters of the outputs this thread finishes, behind the first steps' operands
+    const uint32_t src_lane = (tid >> 2) & 63u, er = tid & 3u, fg = tid >> 8;
+    const uint32_t my_m = m0 + (src_lane & 15u), my_c = n0 + (src_lane >> 4) * 4 + er;
+    float sc[FT], zc[FT], bs[FT], sr[FT], zr[FT];
+    if (FUSED) {
+#pragma unroll
+        for (int f = 0; f < FT; ++f) {
+            const uint32_t t = min(fg + 2 * f, (uint32_t)(MT * NT - 1));
+            const uint32_t n = min(my_c + t / MT * 16, p.N - 1), m = min(my_m + t % MT * 16, p.M - 1);
+            sc[f] = p.epi.s_col[n];
+            zc[f] = p.epi.z_col[n];
+            bs[f] = BIAS ? p.epi.bias[n] : 0.f;
+            sr[f] = p.epi.s_row[m];
+            zr[f] = p.epi.z_row[m];
+        }
+    }
+    uint32_t slot = 0;
+    for (uint32_t st = 0; st < steps; ++st) {
+        // this step's loads are here (those of the next DEPTH - 1 may be in flight; other loads only make the wait longer)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * L) : "memory");
+        if (G > 1) asm volatile("s_barrier" ::: "memory");  // (and everybody's)
+        read(slot);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the place takes the step DEPTH further on
+        if (G > 1) asm volatile("s_barrier" ::: "memory");
+        load(st + DEPTH, slot);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) acc[n][m] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[n][u], x[m][u], acc[n][m], 0, 0, 0);
+        slot = slot + kStage == DEPTH * kStage ? 0 : slot + kStage;
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    v4i *const part = reinterpret_cast<v4i *>(lds);
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) part[((n * MT + m) * 8 + wave) * 64 + lane] = acc[n][m];
+    __syncthreads();
+    const int *const sums = reinterpret_cast<const int *>(lds) + src_lane * 4 + er;
+#pragma unroll
+    for (int f = 0; f < FT; ++f) {
+        const uint32_t t = fg + 2 * f;
+        if (t < (uint32_t)(MT * NT)) {
+            int sum = 0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum += sums[(t * 8 + i) * 256];
+            const uint32_t m = my_m + t % MT * 16, n = my_c + t / MT * 16;
+            if (m < p.M && n < p.N) {
+                if (FUSED) {
+                    float o = dequant_hprec_one(sum, sr[f], zr[f], sc[f], zc[f]);
+                    if (BIAS) o = o + bs[f];
+                    p.y[(uint64_t)m * p.N + n] = o;
+                } else {
+                    p.C[(uint64_t)m * p.N + n] = sum;
+                }
+            }
+        }
+    }
+}
+
+// LDS kernel: what one round of its workgroups covers, and up to 16 rows on more columns where the decode kernel's registers
+// full of activations do not pay: 16 x 11008 x 4096 10.9 -> 10.4 us, 16 x 16384 x 8192 33.8 -> 21.5, x 512 6.2 -> 4.8, but 16 x 16384
+// x 4096 14.0 -> 14.2; 32 x 11008 x 4096 12.9 -> 13.4.  Of 288 shapes of one round, 8..500 rows, 250..16384 columns and 512..11008
+// elements, 283 are ahead, by up to 75 % of their time, and the others level but for 8 x 250 x 512 (3.2 -> 3.4).  Up to four rows: only those too long for the decode kernel.
+inline bool lds8_takes(uint32_t M, uint32_t N, uint32_t K)
+{
+    if (M == 0 || (M < 5 && K <= 4096) || K == 0 || K > 65536 || ((uint64_t)N + 32) * K >= 0xFFFFFF00ull) return false;
+    const LdsShape t = lds_shape(M, N);
+    if (t.rows == 0) return false;
+    if ((uint64_t)((M + 16 * t.rows - 1) / (16 * t.rows)) * ((N + 16 * t.cols - 1) / (16 * t.cols)) <= 256) return true;
+    return M <= 16 && N <= 65536 && (N <= 12288 || K <= 2560 || K > 4096);
+}
+
+template <bool FUSED, bool BIAS, bool TILED>
+static void launch_lds8(Gemm8Params &p, hipStream_t stream)
+{
+    const LdsShape t = lds_shape(p.M, p.N);
+    // groups of rows, and 2^16 over them: (at * m) >> 16 == at / groups while at * (groups - 1) < 2^16 (one round)
+    const uint32_t groups = (p.M + 16 * t.rows - 1) / (16 * t.rows), tiles = (p.N + 16 * t.cols - 1) / (16 * t.cols);
+    p.tiles_m = groups | ((65535 + groups) / groups) << 9;
+    const dim3 grid((tiles * groups + 7) / 8 * 8);
+#define DUQ_LDS8(MT)                                                                                                            \
+    if (t.rows == MT && t.cols == 1) DUQ_LAUNCH_HEAD((gemm_s8_lds_kernel<MT, 1, FUSED, BIAS, TILED>), grid, dim3(512), 0, stream, p); \
+    if (t.rows == MT && t.cols == 2) DUQ_LAUNCH_HEAD((gemm_s8_lds_kernel<MT, 2, FUSED, BIAS, TILED>), grid, dim3(512), 0, stream, p);
+    DUQ_LDS8(1)
+    DUQ_LDS8(2)
+    DUQ_LDS8(3)
+    DUQ_LDS8(4)
+#undef DUQ_LDS8
+}
+
+// ---------------------------------------------------------------------------------
 // skinny kernel (M <= 32): bound by reading the weight once from HBM
 // ---------------------------------------------------------------------------------
 // A workgroup owns 16 weight rows; its four wavefronts split K in contiguous quarters and meet in LDS at the end, so
@@ -1334,6 +1521,10 @@ static void launch_gemm8_variant(Gemm8Params &p, hipStream_t stream)
         if (p.M == 1) launch_rows8<1, FUSED, BIAS>(p, stream);
         else if (p.M == 2) launch_rows8<2, FUSED, BIAS>(p, stream);
         else launch_rows8<4, FUSED, BIAS>(p, stream);
+        return;
+    }
+    if (lds8_takes(p.M, p.N, p.K)) {
+        launch_lds8<FUSED, BIAS, TILED>(p, stream);
         return;
     }
     if (split8_takes(p.M, p.N, p.K)) {

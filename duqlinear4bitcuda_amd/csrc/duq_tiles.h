@@ -43,4 +43,17 @@ __device__ __forceinline__ v4u buf_load16_aux(__amdgpu_buffer_rsrc_t r, uint32_t
     return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, AUX));
 }
 
+// Stages of the LDS kernels (duq_decode.hip, duq_int8.hip): MT row tiles and NT column tiles of 16 per workgroup of eight
+// wavefronts.
+template <int MT, int NT>
+struct LdsTile {
+    static constexpr int G = NT == 1 ? 1 : 8;            // wavefronts that share a stage
+    static constexpr int RB = G == 1 ? 128 : 512;        // bytes of a row in it
+    static constexpr int DEPTH = G == 1 ? 2 : 3;         // stages
+    static constexpr int U = RB / (64 * G);              // a wavefront's 64-byte fragments of a row in a stage
+    static constexpr int L = (MT + NT) * U;              // load instructions of a wavefront and stage, a kilobyte each
+    static constexpr int kStage = G * L * 1024, kLds = 8 / G * DEPTH * kStage, kPart = NT * MT * 8 * 1024;
+    static_assert(kLds <= 160 * 1024 && kPart <= kLds, "LDS");
+};
+
 }  // namespace duq

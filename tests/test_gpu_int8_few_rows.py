@@ -89,3 +89,11 @@ def test_ragged_columns_of_the_tiles(dev, M, N, K):
                                    (1024, 10500, 4096), (1950, 5005, 4096), (2048, 8300, 2112)])  # 64 x 256, 64 x 128 behind
 def test_uneven_rounds_of_the_tiles(dev, M, N, K):
     test_ragged_columns_of_the_tiles(dev, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 1, 32), (16, 4100, 1056), (31, 1031, 4128), (40, 2400, 96), (60, 1600, 2080), (64, 8190, 544),
+                                   (129, 1040, 1088), (190, 1025, 2080), (250, 1500, 160), (129, 2600, 992), (96, 4000, 1024),
+                                   (4081, 16, 64), (12810, 10, 64), (3, 50, 8224), (12, 9000, 4192)])
+def test_rows_through_lds(dev, M, N, K):
+    """Every tile of the LDS kernel, groups of rows, ends inside a tile and a stage, up to the most groups there can be."""
+    test_ragged_columns_of_the_tiles(dev, M, N, K)
