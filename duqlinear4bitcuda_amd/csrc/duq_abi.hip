@@ -147,7 +147,7 @@ int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t
     e.s_row = out.scale;
     e.z_row = asym ? out.zeros : nullptr;
     e.rs_row = rowsum ? out.rowsum : nullptr;
-    if (acc_ws) {  // GEMM into int32, then the stand-alone epilogue
+    if (acc_ws && !duq::gemm_applies_dual_rowsum(M, N, K)) {  // GEMM into int32, then the stand-alone epilogue
         if (int st2 = duq::launch_gemm_s4(out.q, w, M, N, K, acc, nullptr, nullptr, as_stream(stream))) return st2;
         duq::DualRowsumParams dp{acc,       out.q,     w,         K / 2,    out.scale, out.zeros, out.rowsum, e.s_col_1, e.z_col_1,
                                  e.s_col_2, e.z_col_2, e.rs_col,  e.rs_col_2, e.bias,  M,         N,          y};
@@ -461,7 +461,7 @@ int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K) { return duq::select
 
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K)
 {
-    if (duq::select_gemm_kernel(M, N, K) != duq::kKernelStream || duq::takes_lds_kernel(M, N, K)) return 0;
+    if (duq::select_gemm_kernel(M, N, K) != duq::kKernelStream) return 0;
     const duq::StreamTile t = duq::select_stream_tile(M, N, K, 1, false);
     return (int)(t.rows * 1000 + t.cols);
 }
@@ -609,14 +609,16 @@ int duq_linear4bit_forward_dual_rowsum(const uint8_t *xq, const duq_half *scale_
         return DUQ_E_NULL;
     if (!aligned(y, 16)) return DUQ_E_ALIGN;
     const uint64_t need = duq_linear4bit_dual_rowsum_workspace_bytes(M, N, K);
-    if (need == 0) {
+    if (need != 0) {
+        if (!acc_workspace) return DUQ_E_NULL;
+        if (workspace_bytes < need) return DUQ_E_SHAPE;
+        if (!aligned(acc_workspace, 16)) return DUQ_E_ALIGN;
+    }
+    if (duq::gemm_applies_dual_rowsum(M, N, K)) {
         duq::Epilogue e{DUQ_EPI_ASYM_DUAL_ROWSUM, scale_x, zeros_x, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias, rowsum_x,
                         w_adj_1,                  w_adj_2};
         return duq::launch_gemm_s4(xq, w, M, N, K, nullptr, &e, y, as_stream(stream));
     }
-    if (!acc_workspace) return DUQ_E_NULL;
-    if (workspace_bytes < need) return DUQ_E_SHAPE;
-    if (!aligned(acc_workspace, 16)) return DUQ_E_ALIGN;
     int32_t *acc = static_cast<int32_t *>(acc_workspace);
     if (int e = duq::launch_gemm_s4(xq, w, M, N, K, acc, nullptr, nullptr, as_stream(stream))) return e;
     duq::DualRowsumParams p{acc,       xq,        w,         K / 2,   scale_x, zeros_x, rowsum_x, w_scale_1, w_zeros_1,

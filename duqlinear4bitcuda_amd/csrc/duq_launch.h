@@ -147,8 +147,14 @@ inline bool takes_wide_kernel(uint32_t M, uint32_t N, uint32_t K)
 inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 {
     const int kernel = select_gemm_kernel(M, N, K);
-    if (takes_wide_kernel(M, N, K) || takes_lds_kernel(M, N, K) || kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma) return true;
+    if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma) return true;
     return (kernel == kKernelStream || kernel == kKernelTile) && (N % 8 == 0 ? K > 256 : K >= 512);
+}
+// (the entry points ask callers for room for the accumulators by that rule; the LDS and wide kernels apply the epilogue
+// themselves all the same)
+inline bool gemm_applies_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
+{
+    return takes_wide_kernel(M, N, K) || takes_lds_kernel(M, N, K) || gemm_fuses_dual_rowsum(M, N, K);
 }
 // Tile for a problem select_gemm_kernel gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
 // 64 x 128 tiles (duq_gemm.hip).  Whole rounds of 256 workgroups (one per CU) cost about f + c * (K / 256) microseconds

@@ -232,7 +232,7 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
  * of up to 64 rows and more than 8192 columns) come first, whatever the bucket.  No
  * counterpart in the reference (CUTLASS picks its own tile, src/kernels/gemm.cu:17-42). */
 int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
-/* For a shape of family 6: its tile as rows * 1000 + columns (256256, 128256, 192128, 128128, 64128, 96064, 64064; the fused
+/* For a shape of family 6 (where the LDS and wide forms do not come first): its tile as rows * 1000 + columns (256256, 128256, 192128, 128128, 64128, 96064, 64064; the fused
  * entry points may cover the last columns of a problem in smaller tiles); 0 for the other families.  (The dual-uniform row-sum epilogue never runs the 256-row tile.) */
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
 
