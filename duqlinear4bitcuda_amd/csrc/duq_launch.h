@@ -72,7 +72,8 @@ struct DualRowsumParams {
 int launch_dual_rowsum_dequant(const DualRowsumParams &p, hipStream_t stream);
 
 // Kernel families of the int4 GEMM and the host-side rule that picks one (select_gemm_kernel: host arithmetic
-// only, exported as duq_gemm_kernel_for so that the rule can be tested without a GPU).
+// only, exported as duq_gemm_kernel_for so that the rule can be tested without a GPU).  Buckets by size: a shape that
+// takes_wide_kernel or takes_lds_kernel takes runs those kernels of duq_decode.hip whatever its bucket.
 enum GemmKernelId {
     kKernelDecodeRows = 1,  // duq_decode.hip, v_dot8_i32_i4, M <= 4
     kKernelDecodeMfma = 2,  // duq_decode.hip, MFMA, 5 <= M <= 16 (K <= 12288), 17 <= M <= 64 (K <= 8192; 48 rows: 12288)
