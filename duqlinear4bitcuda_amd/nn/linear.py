@@ -104,7 +104,7 @@ def _store(*pairs):
             at, fill = at + n, min(-(-(fill + n) // 256) * 256, _STAGE_BYTES)
     most = _STAGE_BYTES if len(pieces) > 1 else fill
     with torch.cuda.device(staged[0][1].device):
-        pins = [torch.empty(most, dtype=torch.uint8, pin_memory=True) for _ in pieces[:2]]
+        pins = [torch.empty(most, dtype=torch.uint8, device="cpu", pin_memory=True) for _ in pieces[:2]]
         arrived = [torch.cuda.Event() for _ in pins]
         for k in range(len(pieces) + 1):
             if k < len(pieces):
@@ -154,7 +154,8 @@ class _MovesTogether(torch.nn.Module):
 
 def _fetch(tensors, move):
     """{id(t): move(t)} of the host tensors that ``move`` takes to a GPU as they are."""
-    like = {dtype: move(torch.empty(0, dtype=dtype)) for dtype in {t.dtype for t in tensors}}
+    # (device="cpu", here and below: the caller may have set another default device)
+    like = {dtype: move(torch.empty(0, dtype=dtype, device="cpu")) for dtype in {t.dtype for t in tensors}}
     tensors = [t for t in {id(t): t for t in tensors}.values() if like[t.dtype].is_cuda and like[t.dtype].dtype == t.dtype]
     if not tensors:
         return {}
@@ -164,7 +165,7 @@ def _fetch(tensors, move):
         if torch.cuda.is_current_stream_capturing():
             return {}
         size = min(_STAGE_BYTES, sum(-(-t.nbytes // 256) * 256 for t in tensors))
-        pins = [torch.empty(size, dtype=torch.uint8, pin_memory=True)]
+        pins = [torch.empty(size, dtype=torch.uint8, device="cpu", pin_memory=True)]
         left = [torch.cuda.Event(), torch.cuda.Event()]
         k = fill = 0
         for t in tensors:
@@ -176,7 +177,7 @@ def _fetch(tensors, move):
                     left[k].record()
                     k, fill = k ^ 1, 0
                     if len(pins) == 1:
-                        pins.append(torch.empty(size, dtype=torch.uint8, pin_memory=True))
+                        pins.append(torch.empty(size, dtype=torch.uint8, device="cpu", pin_memory=True))
                     left[k].synchronize()
                 n = min(size - fill, src.numel() - at)
                 pin = pins[k][fill:fill + n]

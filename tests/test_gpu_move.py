@@ -57,3 +57,40 @@ def test_moves(dev, stage, monkeypatch):
     with torch.inference_mode():
         m = _layer()
         assert torch.equal(m.to(dev).weight.cpu(), want["weight"])
+
+
+def test_a_default_device_is_not_asked():
+    """Where a move leads is told by a host tensor, whatever device a caller has made the default one."""
+    t, seen = torch.zeros(4, 8), []
+    with torch.device("meta"):
+        assert impl._fetch([t], lambda t: (seen.append(t.device.type), t)[1]) == {}
+    assert seen == ["cpu"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stage", [1 << 24, 768 * 256])
+def test_moves_under_a_default_device(dev, stage, monkeypatch):
+    """The device of the pinned buffers and of the probe is named: under torch.device("cuda") and set_default_device layers
+    move as they do without, and a cast of a layer on the host stays there."""
+    monkeypatch.setattr(impl, "_STAGE_BYTES", stage)
+    want = {k: t.clone() for k, t in _layer().state_dict().items()}
+    same = lambda m: all(torch.equal(t.cpu(), want[k]) for k, t in m.state_dict().items())
+
+    def check():
+        for move in (lambda m: m.to("cuda"), lambda m: m.cuda()):
+            m = move(hosts.pop())
+            assert all(t.is_cuda for t in m.state_dict().values()) and same(m)
+        m = hosts.pop().to(torch.float16)
+        assert all(t.device.type == "cpu" for t in m.state_dict().values()) and same(m)
+        back = [torch.empty_like(t) for t in want.values()]   # (device results into host tensors, as a conversion stores them)
+        impl._store(*((d, t.to(dev)) for d, t in zip(back, want.values())))
+        assert all(not d.is_cuda and torch.equal(d, t) for d, t in zip(back, want.values()))
+
+    hosts = [_layer() for _ in range(6)]
+    with torch.device("cuda"):
+        check()
+    torch.set_default_device("cuda")
+    try:
+        check()
+    finally:
+        torch.set_default_device(None)
