@@ -838,8 +838,11 @@ int duq_quantize_linear8bit_forward(const float *x, const int8_t *w, const int8_
     if (int e = check_gemm8(q, weight, M, N, K)) return e;
     if (!w_scale || !w_zeros || !y) return DUQ_E_NULL;
     if (!aligned(y, 4)) return DUQ_E_ALIGN;
-    if (duq::quantize_gemm8_fuses(M, N, K))
-        return duq::launch_quantize_gemm_s8(x, w_tiled ? w_tiled : w, w_tiled != nullptr, M, N, K, w_scale, w_zeros, bias, y, as_stream(stream));
+    if (duq::quantize_gemm8_fuses(M, N, K)) {
+        // (up to four rows, where `weight` is w: a copy that is not aligned is no reason to refuse the call, only not to read it)
+        const bool copy = w_tiled && aligned(w_tiled, 16);
+        return duq::launch_quantize_gemm_s8(x, copy ? w_tiled : w, copy, M, N, K, w_scale, w_zeros, bias, y, as_stream(stream));
+    }
     if (int e = duq::launch_quantize_rows_asym8(x, M, K, q, sx, zx, as_stream(stream))) return e;
     return duq::launch_gemm_s8(q, weight, tiled, M, N, K, nullptr, sx, zx, w_scale, w_zeros, bias, y, as_stream(stream));
 }

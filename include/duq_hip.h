@@ -495,10 +495,12 @@ int duq_linear8bit_forward_tiled(const int8_t *xq, const float *scale_x, const f
 /* No counterpart in the reference: LinearQuant8bitASQ.forward with its own quantizer (qlinear4bit/nn/linear.py:323-335)
  * in one call: duq_quantize_rows_asym_8bit into `workspace`, then duq_linear8bit_forward(_tiled) on it; the same
  * bits as the two calls.  x [M,K] float32, 16-byte aligned, K % 32 == 0; w the weight as stored and / or w_tiled its
- * tiled copy (one may be NULL): up to four rows (two of more than 4096 elements) read w when it is given, everything
- * else w_tiled when it is given.  workspace: duq_quantize_linear8bit_workspace_bytes(M, K) bytes (codes, scales,
- * zero points), 16-byte aligned.  Up to eight rows of at most 4096 elements are one launch, which quantizes the rows itself
- * (and reads w_tiled when it is given); the workspace is asked for all the same. */
+ * tiled copy (one may be NULL).  Up to eight rows of at most 4096 elements are one launch, which quantizes the rows itself and
+ * reads w_tiled when it is given (up to four rows with both: when w_tiled is 16-byte aligned, else w); up to two rows of
+ * 4097..8192 elements read w when it is given; everything else reads w_tiled when it is given.  What is read has to be 16-byte
+ * aligned; so has w where up to four rows (two above 4096 elements) come with both.  workspace:
+ * duq_quantize_linear8bit_workspace_bytes(M, K) bytes (codes, scales, zero points), 16-byte aligned; the one launch does not
+ * write it, but it is asked for all the same. */
 uint64_t duq_quantize_linear8bit_workspace_bytes(uint32_t M, uint32_t K);
 int duq_quantize_linear8bit_forward(const float *x, const int8_t *w, const int8_t *w_tiled, const float *w_scale,
                                     const float *w_zeros, const float *bias, uint32_t M, uint32_t N, uint32_t K, float *y,

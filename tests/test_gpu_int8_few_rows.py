@@ -61,6 +61,30 @@ def test_quantizer_inside_the_gemm(dev, M, N, K):
                 assert torch.equal(got.view(torch.int32), want.view(torch.int32)), (seed, b is None, t is None)
 
 
+@pytest.mark.parametrize("M", [1, 3, 4])
+def test_a_misaligned_copy_is_not_read(dev, M):
+    """Up to four rows with both weights take the weight as stored where the tiled copy is not 16-byte aligned (a buffer of
+    zeros here, which would show); more rows, which have to read the copy, are refused."""
+    from duqlinear4bitcuda_amd import _HIP as hip
+    from duqlinear4bitcuda_amd import _lib
+    print("8-bit misaligned copy", M, flush=True)
+    lib, (N, K) = _lib.load(), (96, 256)
+    gen = torch.Generator(device=dev).manual_seed(M)
+    w = torch.randint(1, 128, (N, K), generator=gen, device=dev, dtype=torch.int8)
+    sw, zw = torch.rand(N, generator=gen, device=dev), torch.randint(0, 127, (N,), generator=gen, device=dev).float()
+    x = torch.randn(8, K, generator=gen, device=dev)
+    y = torch.empty(8, N, device=dev)
+    copy = torch.zeros(N * K + 16, device=dev, dtype=torch.int8)[4:]
+    ws = torch.empty(lib.duq_quantize_linear8bit_workspace_bytes(8, K), device=dev, dtype=torch.uint8)
+    call = lambda m, copy: lib.duq_quantize_linear8bit_forward(
+        x.data_ptr(), w.data_ptr(), copy.data_ptr(), sw.data_ptr(), zw.data_ptr(), None, m, N, K, y.data_ptr(), ws.data_ptr(),
+        ws.numel(), torch.cuda.current_stream().cuda_stream)
+    assert call(M, copy) == 0
+    want = hip.quantize_linear8bit_forward(x[:M], w, None, sw, zw)
+    assert torch.equal(y[:M].view(torch.int32), want.view(torch.int32))
+    assert call(8, copy) == -5
+
+
 @pytest.mark.parametrize("M,N,K", [(129, 2561, 64), (257, 2303, 96), (130, 5122, 64), (65, 4095, 1536), (70, 131, 1536), (640, 515, 64),
                                    (8200, 2050, 32)])
 def test_ragged_columns_of_the_tiles(dev, M, N, K):
