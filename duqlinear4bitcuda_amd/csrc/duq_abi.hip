@@ -814,6 +814,12 @@ int duq_linear8bit_forward_tiled(const int8_t *xq, const float *scale_x, const f
                                as_stream(stream));
 }
 
+int duq_gemm8_kernel_for(uint32_t M, uint32_t N, uint32_t K, int32_t tiled)
+{
+    if (M == 0 || N == 0 || K == 0) return 0;
+    return duq::select_gemm8_kernel(M, N, K, tiled != 0);
+}
+
 uint64_t duq_quantize_linear8bit_workspace_bytes(uint32_t M, uint32_t K)
 {
     return up16((uint64_t)M * K) + 2 * up16((uint64_t)M * 4);

@@ -753,8 +753,8 @@ __global__ __launch_bounds__(512) void gemm_s8_split_kernel(DUQ_HEAD_DECL, Gemm8
 // each of sixteen rows from neighbouring lanes, a cache line per lane, which a CU serves at a quarter of its rate; and long
 // rows on few columns leave most compute units without a workgroup.  Here both operands come through LDS without registers, in
 // whole pieces of a row (tiled weights: in runs of 256 bytes), as in the 4-bit LDS kernel, whose tiles, stages and groups of rows
-// these are.  Measured (N x K, tiled weights, us): 16 rows 4096 x 4096 6.5 -> 5.5, 4096 x 11008 14.8 -> 9.2, 250 x 8192 8.7 -> 4.5; 32
-// rows 8.1 -> 5.8, 20.4 -> 10.4 (45 MB: 4.3 TB/s), 12.8 -> 4.5; 128 rows 10.9 -> 9.4, 20.6 -> 18.7, 15.6 -> 5.7.
+// these are.  Measured (N x K, tiled weights out of the caches, us): 16 rows 4096 x 4096 6.0 -> 5.4, 4096 x 11008 13.4 -> 11.0 (45 MB: 4.1
+// TB/s), 250 x 8192 8.3 -> 6.8; 32 rows 7.2 -> 6.5, 19.6 -> 13.6, 12.6 -> 6.6.
 template <int MT, int NT, bool FUSED, bool BIAS, bool TILED>
 __global__ __launch_bounds__(512) void gemm_s8_lds_kernel(DUQ_HEAD_DECL, Gemm8Params tail)
 {
@@ -902,17 +902,39 @@ __global__ __launch_bounds__(512) void gemm_s8_lds_kernel(DUQ_HEAD_DECL, Gemm8Pa
     }
 }
 
-// LDS kernel: what one round of its workgroups covers, and up to 16 rows on more columns where the decode kernel's registers
-// full of activations do not pay: 16 x 11008 x 4096 10.9 -> 10.4 us, 16 x 16384 x 8192 33.8 -> 21.5, x 512 6.2 -> 4.8, but 16 x 16384
-// x 4096 14.0 -> 14.2; 32 x 11008 x 4096 12.9 -> 13.4.  Of 288 shapes of one round, 8..500 rows, 250..16384 columns and 512..11008
-// elements, 283 are ahead, by up to 75 % of their time, and the others level but for 8 x 250 x 512 (3.2 -> 3.4).  Up to four rows: only those too long for the decode kernel.
-inline bool lds8_takes(uint32_t M, uint32_t N, uint32_t K)
+// Shapes of the LDS kernel.  Measured against the kernels that would run otherwise, every weight out of the caches (a pool of 720 MB,
+// 640 MB of other data read before each run: with a few copies of the weight 16 x 11008 x 4096 seemed 10.9 -> 10.4 us and is
+// 10.7 -> 12.8), on 5400 shapes each of the tiled copy and the weight as stored, times as fast:
+//  - one round of workgroups: the weight as stored, a cache line per lane in the other kernels, 1.0 - 3.6; the copy with rows in
+//    several groups 1.05 - 3.0, and with rows longer than 4096 elements, which the decode kernel does not hold, 1.0 - 3.5 (up
+//    to four rows of 16384 elements 0.9 - 1.15).
+//  - tiled, rows in one group of up to 4096 elements, whose decode kernel keeps the activations of up to 2048 or 4096 elements in
+//    registers: ahead or level where those are not full (16 x 4096 columns: K 512 / 1024 / 1536 / 2080 / 4096 1.04 / 1.07 / 1.02 /
+//    1.12 / 1.11, but 2048 0.93; 24 rows 1.0 / 1.0 / 0.98 / 1.10 / 1.08, 2048 0.91), with two column tiles a workgroup (more than 4096 columns) only for short
+//    rows, registers that are half empty, or many rows (8192 columns: 16 x 1024 1.03, x 2080 1.05, x 4096 0.95; 32 x 512 1.03, x 2560
+//    1.05, x 4096 0.93; 64 x 2560 1.24, x 4096 1.18; 40 x 3072 1.03, x 4096 0.96).
+//  - up to 16 rows in several rounds, the last of which may leave most compute units idle (9000 columns: 282 workgroups): the weight as
+//    stored 0.97 - 2.0 (16384 x 4096 0.93); the copy 1.01 - 1.25 up to 768 elements and 16384 columns (1024 .. 4096: 0.8 - 1.1)
+//    and 1.0 - 1.6 from 4097 to 6144; longer rows, against the skinny kernel, 0.94 - 1.2 at eight rows (11008 x 8192 0.98, 13824
+//    x 8192 1.13, x 16384 0.85 - 1.12) and 1.0 - 1.35 at sixteen, less where the second round is a few workgroups (8200 columns:
+//    0.88 at eight, 0.93 - 1.1 at twelve).
+inline bool lds8_takes(uint32_t M, uint32_t N, uint32_t K, bool tiled)
 {
     if (M == 0 || (M < 5 && K <= 4096) || K == 0 || K > 65536 || ((uint64_t)N + 32) * K >= 0xFFFFFF00ull) return false;
     const LdsShape t = lds_shape(M, N);
     if (t.rows == 0) return false;
-    if ((uint64_t)((M + 16 * t.rows - 1) / (16 * t.rows)) * ((N + 16 * t.cols - 1) / (16 * t.cols)) <= 256) return true;
-    return M <= 16 && N <= 65536 && (N <= 12288 || K <= 2560 || K > 4096);
+    const uint32_t groups = (M + 16 * t.rows - 1) / (16 * t.rows);
+    const uint64_t workgroups = (uint64_t)groups * ((N + 16 * t.cols - 1) / (16 * t.cols));
+    if (workgroups > 256) {
+        if (M > 16 || N > 65536) return false;
+        if (!tiled) return N <= 12288 || K <= 2560 || K > 4096;
+        if (K <= 4096) return K <= 768 && N <= 16384;
+        return K <= 7168 || M > 8 || (workgroups > 272 && K <= 12288);
+    }
+    if (!tiled || groups > 1) return true;
+    if (K > 4096) return M > 4 || K <= 12288;
+    if (K > 2048) return t.cols == 1 || K <= 2560 || M > 40 || (M > 32 && K <= 3072);
+    return K <= (t.cols == 1 || M <= 16 || M > 48 ? 1024u : 512u) || (t.cols == 1 && M <= 16 && (K <= 1920 || M <= 12));
 }
 
 template <bool FUSED, bool BIAS, bool TILED>
@@ -1514,36 +1536,46 @@ static void launch_plan8(Gemm8Params &p, hipStream_t stream)
         DUQ_LAUNCH_HEAD((gemm_s8_kernel<4, 2, FUSED, BIAS, TILED>), grid, dim3(256), 0, stream, p);
 }
 
+int select_gemm8_kernel(uint32_t M, uint32_t N, uint32_t K, bool tiled)
+{
+    if (!tiled && rows8_takes(M, K)) return kKernel8Rows;
+    if (lds8_takes(M, N, K, tiled)) return kKernel8Lds;
+    if (split8_takes(M, N, K)) return kKernel8Split;
+    if (decode8_takes(M, N, K)) return kKernel8Decode;
+    return M <= 32 ? kKernel8Skinny : kKernel8Tile;
+}
+
 template <bool FUSED, bool BIAS, bool TILED>
 static void launch_gemm8_variant(Gemm8Params &p, hipStream_t stream)
 {
-    if (!TILED && rows8_takes(p.M, p.K)) {
-        if (p.M == 1) launch_rows8<1, FUSED, BIAS>(p, stream);
-        else if (p.M == 2) launch_rows8<2, FUSED, BIAS>(p, stream);
-        else launch_rows8<4, FUSED, BIAS>(p, stream);
+    switch (select_gemm8_kernel(p.M, p.N, p.K, TILED)) {
+    case kKernel8Rows:
+        if constexpr (!TILED) {
+            if (p.M == 1) launch_rows8<1, FUSED, BIAS>(p, stream);
+            else if (p.M == 2) launch_rows8<2, FUSED, BIAS>(p, stream);
+            else launch_rows8<4, FUSED, BIAS>(p, stream);
+        }
         return;
-    }
-    if (lds8_takes(p.M, p.N, p.K)) {
+    case kKernel8Lds:
         launch_lds8<FUSED, BIAS, TILED>(p, stream);
         return;
-    }
-    if (split8_takes(p.M, p.N, p.K)) {
+    case kKernel8Split:
         p.tiles_m = (p.M + 63) / 64;
         p.tiles_n = (p.N + 63) / 64;
         DUQ_LAUNCH_HEAD((gemm_s8_split_kernel<FUSED, BIAS, TILED>), dim3(p.tiles_m * p.tiles_n), dim3(512), 0, stream, p);
         return;
-    }
-    if (decode8_takes(p.M, p.N, p.K)) {
+    case kKernel8Decode:
         launch_decode8<FUSED, BIAS, TILED>(p, stream);
         return;
-    }
-    if (p.M <= 32) {
+    case kKernel8Skinny: {
         const dim3 grid((p.N + 15) / 16);
         if (p.M <= 16)
             DUQ_LAUNCH_HEAD((gemm_s8_skinny_kernel<1, FUSED, BIAS, TILED>), grid, dim3(256), 0, stream, p);
         else
             DUQ_LAUNCH_HEAD((gemm_s8_skinny_kernel<2, FUSED, BIAS, TILED>), grid, dim3(256), 0, stream, p);
         return;
+    }
+    default: break;
     }
     p.tiles_n = (p.N + 255) / 256;
     // the tallest tile that still gives most of the 256 CUs a workgroup

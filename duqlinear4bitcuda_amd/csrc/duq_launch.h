@@ -305,6 +305,16 @@ int launch_gemm_s8(const int8_t *A, const int8_t *B, bool b_tiled, uint32_t M, u
                    const float *s_row, const float *z_row, const float *s_col, const float *z_col, const float *bias,
                    float *y, hipStream_t stream);
 int launch_weight_tile8(const int8_t *w, uint32_t N, uint32_t K, int8_t *out, hipStream_t stream);
+// The kernel it runs, by shape and weight layout (host arithmetic only; exported as duq_gemm8_kernel_for).
+enum Gemm8KernelId {
+    kKernel8Rows = 1,    // up to four rows on the weight as stored
+    kKernel8Decode = 2,  // up to 64 rows of at most 4096 elements, activations in registers
+    kKernel8Lds = 3,     // few rows, and more on narrow problems, through LDS
+    kKernel8Skinny = 4,  // up to 32 longer rows
+    kKernel8Split = 5,   // one round of 64 x 64 tiles, wavefronts side by side along K
+    kKernel8Tile = 6,    // prefill tiles
+};
+int select_gemm8_kernel(uint32_t M, uint32_t N, uint32_t K, bool tiled);
 
 // Weight preparation (duq_weight.hip).  kind 0: asymmetric over |w|, 1: signed-shifted, 2: symmetric with given scales s1,
 // s2.  split: first column of the second range (0: one range, parameters s1, z1, r1).  cols % 8 == 0.

@@ -492,6 +492,11 @@ int duq_linear8bit_forward_tiled(const int8_t *xq, const float *scale_x, const f
                                  const float *w_scale, const float *w_zeros, const float *bias, uint32_t M, uint32_t N,
                                  uint32_t K, float *y, duq_stream_t stream);
 
+/* Which kernel duq_matmul_host_8bit / duq_linear8bit_forward (tiled 0) and duq_linear8bit_forward_tiled (tiled 1) run for a
+ * shape (no GPU work; for tests and tuning): 1 rows kernel, 2 decode kernel, 3 LDS kernel, 4 skinny kernel, 5 split kernel, 6
+ * prefill tiles; 0 for an empty problem.  No counterpart in the reference. */
+int duq_gemm8_kernel_for(uint32_t M, uint32_t N, uint32_t K, int32_t tiled);
+
 /* No counterpart in the reference: LinearQuant8bitASQ.forward with its own quantizer (qlinear4bit/nn/linear.py:323-335)
  * in one call: duq_quantize_rows_asym_8bit into `workspace`, then duq_linear8bit_forward(_tiled) on it; the same
  * bits as the two calls.  x [M,K] float32, 16-byte aligned, K % 32 == 0; w the weight as stored and / or w_tiled its

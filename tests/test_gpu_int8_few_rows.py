@@ -117,7 +117,12 @@ def test_uneven_rounds_of_the_tiles(dev, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [(9, 1, 32), (16, 4100, 1056), (31, 1031, 4128), (40, 2400, 96), (60, 1600, 2080), (64, 8190, 544),
                                    (129, 1040, 1088), (190, 1025, 2080), (250, 1500, 160), (129, 2600, 992), (96, 4000, 1024),
-                                   (4081, 16, 64), (12810, 10, 64), (3, 50, 8224), (12, 9000, 4192)])
+                                   (4081, 16, 64), (12810, 10, 64), (3, 50, 8224), (12, 9000, 4192),
+                                   # and on both weight layouts: one column tile a workgroup and two, one to four row tiles
+                                   (16, 4090, 992), (31, 4090, 2112), (40, 4090, 2112), (16, 4100, 992), (31, 8190, 4128),
+                                   (48, 8190, 2144), (64, 8190, 2112), (64, 4090, 544), (190, 1353, 992), (64, 8190, 480), (16, 8200, 480)])
 def test_rows_through_lds(dev, M, N, K):
     """Every tile of the LDS kernel, groups of rows, ends inside a tile and a stage, up to the most groups there can be."""
+    from duqlinear4bitcuda_amd import _lib
+    assert _lib.load().duq_gemm8_kernel_for(M, N, K, 0) == 3
     test_ragged_columns_of_the_tiles(dev, M, N, K)

@@ -281,6 +281,33 @@ def test_abi_validation_8bit_entries():
     assert ql(None, None, None, None, None, None, 0, 8, 32, None, None, 0, None) == 0
 
 
+def test_gemm8_kernel_rule():
+    """Which kernel a shape runs (host arithmetic, duq_gemm8_kernel_for): a row of 16 tokens on 11008 columns stays with the
+    decode kernel, whose workgroups share the columns evenly; kernels with 32-bit offsets only while the weight has them."""
+    from duqlinear4bitcuda_amd import _lib
+    f = _lib.load().duq_gemm8_kernel_for
+    rows, decode, lds, skinny, split, tile = 1, 2, 3, 4, 5, 6
+    # (tokens, columns, elements): tiled copy, weight as stored
+    for shape, want in {(4, 4096, 4096): (decode, rows), (2, 4096, 8192): (lds, rows), (5, 4096, 4096): (lds, lds),
+                        (16, 4096, 4096): (lds, lds), (16, 4096, 2048): (decode, lds), (16, 4097, 4096): (decode, lds),
+                        (16, 8192, 1024): (lds, lds), (16, 8193, 1024): (decode, lds), (16, 8193, 768): (lds, lds),
+                        (8, 11008, 4096): (decode, lds), (16, 11008, 4096): (decode, lds), (16, 12288, 4096): (decode, lds),
+                        (16, 11008, 6144): (lds, lds), (8, 8200, 8192): (skinny, lds), (8, 11008, 8192): (lds, lds), (16, 11008, 8192): (lds, lds), (8, 13824, 16384): (skinny, lds), (16, 13824, 4096): (decode, decode),
+                        (64, 8192, 1024): (lds, lds), (64, 8192, 2048): (decode, lds),
+                        (32, 2048, 2048): (lds, lds), (32, 2049, 2048): (decode, lds), (32, 4096, 4096): (lds, lds),
+                        (32, 8192, 4096): (decode, lds), (40, 8192, 3072): (lds, lds), (40, 8192, 4096): (decode, lds),
+                        (64, 8192, 4096): (lds, lds), (32, 8193, 8192): (split, split), (256, 2048, 4096): (lds, lds),
+                        (256, 4096, 4096): (split, split), (2048, 4096, 4096): (tile, tile), (1, 1024, 16384): (skinny, lds)}.items():
+        assert (f(*shape, 1), f(*shape, 0)) == want, shape
+    assert f(0, 64, 64, 0) == 0 and f(64, 64, 0, 1) == 0
+    for M in (1, 5, 16, 33, 64, 65, 300):
+        for K in (32, 4096, 4128, 65536, 131040):
+            for N in (1, 4096, 70000, 2 ** 32 // K - 33, 2 ** 32 // K, 1 << 22):
+                for tiled in (0, 1):
+                    if N <= 1 << 22 and (N + 32) * K >= 0xFFFFFF00:
+                        assert f(M, N, K, tiled) not in (decode, lds), (M, N, K)
+
+
 def test_python_ops_reject_bad_arguments():
     import torch
     from duqlinear4bitcuda_amd import _HIP
