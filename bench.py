@@ -377,7 +377,7 @@ def decode_section(dev, quick, eager=True):
                     "gemm_only_us": round(us_gemm, 3),
                     "gemm_only_GBps": round((byts - 2 * M * K + M * K // 2 + 2 * M) / us_gemm / 1e3, 1),
                     "read_floor_us": round(us_read, 3), "read_floor_GBps": round(wbytes / us_read / 1e3, 1),
-                    "frac_of_read_floor": round(us_read / us, 4), "gemm_kernel_family": hip.gemm_kernel_for(M, N, K),
+                    "frac_of_read_floor": round(us_read / us, 4), "gemm_kernel": hip.gemm_kernel_for(M, N, K),
                     "weight_buffers": nbuf})
         del ws, models
     return out
@@ -795,7 +795,7 @@ def main():
     rows_7b = [d for d in decode if (d["M"], d["N"], d["K"]) in LLAMA7B_DECODE]
     worst = min(rows_7b, key=lambda d: d["frac_hbm"])
     roofline_decode = {"bound": "hbm", "kernel": "gemv_s4_rows_kernel (M <= 8, quantizer inside) / quantize_rows_kernel + "
-                                                 "gemm_s4_decode_kernel (M <= 64)",
+                                                 "gemm_s4_lds_kernel (N <= 4096), gemm_s4_decode_kernel (wider)",
                        "what": "worst of the Llama-2-7B decode rows (M in {1,4,16}, K=4096, N in {4096,11008}), binary16 "
                                "activations in, quantize + GEMM + dequant, weights never in a cache",
                        "achieved": worst["GBps"], "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": worst["frac_hbm"],

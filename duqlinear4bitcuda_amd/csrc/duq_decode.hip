@@ -1170,7 +1170,7 @@ bool launch_decode_any(DecodeParams &p, int epi, hipStream_t stream)
         constexpr int W = DUQ_DEC_WAVES, S = 32 / W;  // 64-byte segments per wavefront for 2 KB of a row
         const uint32_t mt = (p.M + 15) / 16;
         // rows of up to 4096 / 8192 elements: S, 2 S segments per wavefront; the row tiles whose fragments fit in registers
-        // next to two sets of weights (what select_gemm_kernel leaves here)
+        // next to two sets of weights (what gemm_kernel_for leaves here)
         if (mt > 4 || kbytes > 4096) return false;
         if (kbytes <= 2048) {
             if (mt == 1) return launch_mfma_mode<W, S, 1>(p, epi, stream);

@@ -10,7 +10,7 @@
 // 256*|C| stays below 2^31 for K <= 131008.  Integer accumulation is order-free, so the
 // k order inside a tile only has to be the same for A and B.
 //
-// Four kernels here, and the prefill kernel in duq_prefill.hip, picked by shape in select_gemm_kernel() (up to 64 rows,
+// Four kernels here, and the prefill kernel in duq_prefill.hip, picked by shape in gemm_kernel_for() (up to 64 rows,
 // and more on narrow problems, run the kernels of duq_decode.hip as far as they reach):
 //  * prefill kernel (duq_prefill.hip): more than 64 rows, long rows, fewer rows on wide layers, tensors of 4 GiB or more,
 //    what is left;
@@ -642,7 +642,7 @@ __global__ __launch_bounds__(256) void gemv_s4_dot_kernel(DUQ_HEAD_DECL, GemmPar
 // ---------------------------------------------------------------------------------
 // dispatch
 // ---------------------------------------------------------------------------------
-// Which kernel family takes a shape.  Host arithmetic only, so that the rule can be tested without a GPU:
+// Which of the kernels by size takes a shape.  Host arithmetic only, so that the rule can be tested without a GPU:
 // every kernel whose weight offsets are 32-bit (decode, dot: row * K/2 + offset, and a buffer descriptor
 // over the whole tensor) is reachable only while the packed weights stay below 4 GiB - 256 (the out-of-range
 // marker); larger tensors go to the stream / prefill kernels, whose descriptors and pointers are per tile
@@ -651,8 +651,8 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
 {
     const uint64_t wbytes = (uint64_t)N * (K / 2);
     const bool small_offsets = wbytes < 0xFFFFFF00ull && K > 0;
-    // The launcher asks takes_wide_kernel and takes_lds_kernel first; what is said here of up to 64 rows and of narrow problems
-    // holds for the shapes that those leave.  Decode: rows kernel for up to four rows (8 KB of every weight row per
+    // (gemm_kernel_for asks takes_wide_kernel and takes_lds_kernel first: what is said here of up to 64 rows and of narrow problems
+    // holds for the shapes that those leave.)  Decode: rows kernel for up to four rows (8 KB of every weight row per
     // wavefront); above, the MFMA decode kernel (rows of up to 8192 elements), with two to four row tiles against the same
     // weight fragments for 17..64 rows.  9..16 rows on very wide layers run the skinny kernel (whole-line weight loads, 5 %
     // faster at N = 28672, K = 4096).
@@ -678,13 +678,13 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
     const uint32_t xstride = ((K / 2 + 127) / 128) * 128;
     // dot kernel: up to four rows too long for the decode kernels
     if (M <= 4 && small_offsets && 4 * xstride <= 60 * 1024) return kKernelDot;
-    // a bucket of narrow problems, all of which the LDS kernel takes: 17..256 rows in groups of 64, 32 or 16 whose column tiles
-    // are one round of workgroups, and 5..16 rows of 8193..16384 elements
+    // narrow problems, all of which takes_lds_kernel takes: 17..256 rows in groups of 64, 32 or 16 whose column tiles are one
+    // round of workgroups, and 5..16 rows of 8193..16384 elements
     const uint32_t rb_max = K <= 4096 ? 4 : (K <= 8192 ? 2 : 1);
     const uint32_t row_groups = ((M + 15) / 16 + rb_max - 1) / rb_max;
     const bool one_round = M > 16 && M <= 256 && (uint64_t)((N + 15) / 16) * row_groups <= 256 && (K > 2048 || M <= 64);
     const bool long_rows = M <= 16 && K > 8192;
-    if ((long_rows || one_round) && K <= 16384 && small_offsets) return kKernelRing;
+    if ((long_rows || one_round) && K <= 16384 && small_offsets) return kKernelLds;
     const uint32_t narrow_tiles = ((M + 63) / 64) * ((N + 127) / 128);
     const bool narrow_round = M > 64 && narrow_tiles >= 64 && narrow_tiles <= 256;
     auto tiles = [&](uint32_t bm, uint32_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -692,12 +692,19 @@ int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K)
     return kKernelTile;
 }
 
+int gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K)
+{
+    if (takes_wide_kernel(M, N, K)) return kKernelWide;
+    if (takes_lds_kernel(M, N, K)) return kKernelLds;
+    return select_gemm_kernel(M, N, K);
+}
+
 // batch > 1: `batch` problems of one shape, tensors contiguous over the batch, one launch (blockIdx.z is the
 // problem): the short-row, stream and prefill kernels only, the tile chosen on the whole batch.
 template <int EPI, bool BIAS>
 static void launch_epi(GemmParams &p, hipStream_t stream, uint32_t batch = 1)
 {
-    const int kernel = batch > 1 ? kKernelStream : select_gemm_kernel(p.M, p.N, p.K);
+    const int kernel = batch > 1 ? kKernelStream : gemm_kernel_for(p.M, p.N, p.K);
     // (EPI 5, the dual-uniform row-sum epilogue: of the kernels launched here, the stream and prefill kernels have it, and
     // only their shapes come here with it: gemm_fuses_dual_rowsum)
     if constexpr (EPI != 5) {
@@ -769,8 +776,8 @@ int launch_gemm_s4_batched(const uint8_t *A, const uint8_t *B, uint32_t M, uint3
 {
     if (M == 0 || N == 0 || batch == 0) return 0;
     if (batch == 1) {
-        const int kernel = select_gemm_kernel(M, N, K);
-        if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma || takes_wide_kernel(M, N, K) || takes_lds_kernel(M, N, K))
+        const int kernel = gemm_kernel_for(M, N, K);
+        if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma || kernel == kKernelWide || kernel == kKernelLds)
             return launch_decode_s4(A, B, M, N, K, out_acc, epi, y, stream);
     }
     GemmParams p{};

@@ -71,19 +71,22 @@ struct DualRowsumParams {
 };
 int launch_dual_rowsum_dequant(const DualRowsumParams &p, hipStream_t stream);
 
-// Kernel families of the int4 GEMM and the host-side rule that picks one (select_gemm_kernel: host arithmetic
-// only, exported as duq_gemm_kernel_for so that the rule can be tested without a GPU).  Buckets by size: a shape that
-// takes_wide_kernel or takes_lds_kernel takes runs those kernels of duq_decode.hip whatever its bucket.
+// Kernels of the int4 GEMM and the host-side rule that picks one (gemm_kernel_for: host arithmetic only, exported as
+// duq_gemm_kernel_for so that the rule can be tested without a GPU): takes_wide_kernel and takes_lds_kernel are asked first, what
+// they leave goes by size (select_gemm_kernel, whose answers for the shapes that they take only the question of who
+// asks for room for accumulators still goes by: gemm_fuses_dual_rowsum).
 enum GemmKernelId {
     kKernelDecodeRows = 1,  // duq_decode.hip, v_dot8_i32_i4, M <= 4
-    kKernelDecodeMfma = 2,  // duq_decode.hip, MFMA, 5 <= M <= 16 (K <= 12288), 17 <= M <= 64 (K <= 8192; 48 rows: 12288)
+    kKernelDecodeMfma = 2,  // duq_decode.hip, MFMA, 5 <= M <= 64, K <= 8192 (more than 32 rows: 4096)
     kKernelDot = 3,         // duq_gemm.hip, M <= 4 with rows longer than 16384 elements
-    kKernelRing = 4,        // 17 <= M <= 256 on narrow problems: all of them shapes of the LDS kernel
+    kKernelLds = 4,         // duq_decode.hip, both operands through LDS: 5 <= M <= 64 on up to 8192 columns, narrow problems
     kKernelSkinny = 5,      // duq_gemm.hip, 9 <= M <= 16 with 1536 or more column tiles, K <= 4096
     kKernelStream = 6,      // duq_prefill.hip (duq_gemm.hip for short rows), prefill
     kKernelTile = 7,        // the same kernels on problems of few tiles or rows too long for the others
+    kKernelWide = 8,        // duq_decode.hip, 5 <= M <= 64 on more than 8192 columns, weights through LDS
 };
 int select_gemm_kernel(uint32_t M, uint32_t N, uint32_t K);
+int gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
 // Tile of the LDS kernel in 16 x 16 units: the first of these, in the order of their time (64 x 4096 x 4096, one round of 256
 // workgroups: 4.0, 4.4, 4.5, 5.2, 5.4, 5.9, 6.1, 6.8 us), whose workgroups, a column range and a group of rows each, are one
 // round.  More row groups read the weights again, from their XCD's cache: 64 x 1024 x 8192 6.6 us with four row tiles each,
@@ -99,8 +102,8 @@ inline LdsShape lds_shape(uint32_t M, uint32_t N)
         if ((rows + t.rows - 1) / t.rows * ((cols + t.cols - 1) / t.cols) <= 256) return t;
     return rows <= 4 ? LdsShape{(uint32_t)rows, 2} : LdsShape{0, 0};
 }
-// Shapes of the LDS kernel (duq_decode.hip), asked next and before select_gemm_kernel's families (whose number such a shape keeps:
-// the buckets there are by size).  Measured against those on 900 shapes, us:
+// Shapes of the LDS kernel (duq_decode.hip), asked next and before select_gemm_kernel.  Measured against the kernels there on 900
+// shapes, us:
 //  - 5..64 rows: every length on up to 4096 columns (7 - 75 % less; 16 x 512 x 1024 3.2 -> 2.9, 64 x 1024 x 8192 7.9 -> 6.7, 16
 //    x 512 x 28672 25.6 -> 7.2).  Up to 8192 columns where the rows are many or long (64 x 5120 x 5120 9.6 -> 7.9, 16 x 8192 x
 //    8192 9.2 -> 8.5, but 16 x 8192 x 4096 5.1 -> 5.4 and 24 x 8192 x 4096 6.1 -> 6.3, and where rows begin inside a cache line, 19 x 5332 x 3648 5.0

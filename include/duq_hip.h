@@ -221,19 +221,18 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
                          float clip_a, int32_t qmax_a, float clip_b, int32_t qmax_b, duq_half *y, void *workspace,
                          uint64_t workspace_bytes, duq_stream_t stream);
 
-/* Which kernel family duq_matmul_host_4bit / duq_linear4bit_forward run for a shape (no GPU work; for tests
- * and tuning): 1 decode rows kernel (M <= 4), 2 decode MFMA kernel (M <= 16; up to 64 rows of at most 8192
- * elements, 48 of at most 12288, where family 6 is not ahead), 3 dot kernel (M <= 4, rows longer than 16384 elements),
- * 4 narrow problems, 5 skinny kernel (9 <= M <= 16, very wide problems), 6 prefill kernel (short rows: stream kernel),
- * 7 the same on problems of few tiles or long rows.  Families 1-5 address the weight tensor with 32-bit byte offsets and are
- * only picked while N * K / 2 < 2^32 - 256; larger tensors run families 6 and 7, whose bases are 64-bit per tile.  The
- * families are buckets by size: below that limit the decode kernels' LDS form (5..64 rows on up to 4096 columns, 8192 where the
- * rows are many or long, more rows while its tiles are one round of workgroups, very long rows) and wide form (some problems
- * of up to 64 rows and more than 8192 columns) come first, whatever the bucket.  No
- * counterpart in the reference (CUTLASS picks its own tile, src/kernels/gemm.cu:17-42). */
+/* Which kernel duq_matmul_host_4bit / duq_linear4bit_forward run for a shape (no GPU work; for tests and tuning): 1 decode
+ * rows kernel (M <= 4), 2 decode MFMA kernel (up to 64 rows on more than 4096 columns, where 4, 6 and 8 are not ahead), 3 dot
+ * kernel (M <= 4, rows longer than 16384 elements), 4 LDS kernel (5..64 rows on up to 4096 columns, 8192 where the rows
+ * are many or long, more rows while its tiles are one round of workgroups, very long rows), 5 skinny kernel (9 <= M <= 16,
+ * very wide problems), 6 prefill kernel (short rows: stream kernel), 7 the same on problems of few tiles or long rows, 8
+ * wide kernel (5..64 rows on more than 8192 columns).  Kernels 1-5 and 8 address the weight tensor with 32-bit byte offsets and
+ * are only picked while N * K / 2 < 2^32 - 256; larger tensors run 6 and 7, whose bases are 64-bit per tile.  No counterpart
+ * in the reference (CUTLASS picks its own tile, src/kernels/gemm.cu:17-42). */
 int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
-/* For a shape of family 6 (where the LDS and wide forms do not come first): its tile as rows * 1000 + columns (256256, 128256, 192128, 128128, 64128, 96064, 64064; the fused
- * entry points may cover the last columns of a problem in smaller tiles); 0 for the other families.  (The dual-uniform row-sum epilogue never runs the 256-row tile.) */
+/* For a shape of kernel 6: its tile as rows * 1000 + columns (256256, 128256, 192128, 128128, 64128, 96064, 64064; the fused
+ * entry points may cover the last columns of a problem in smaller tiles); 0 for the other kernels.  (The dual-uniform row-sum
+ * epilogue never runs the 256-row tile.) */
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
 
 /* Measurement aid, no counterpart in the reference: reads `bytes` (16-byte aligned, < 4 GiB) of device memory

@@ -51,9 +51,10 @@ def test_prefill_tiles(dev, M, N, K, n):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
-# tiles whose eight wavefronts split every stage: odd and even numbers of stages, a k that ends inside a piece, few rows and
-# columns (tile 0: a shape the query names no tile for)
-SPLIT = [(65, 4100, 2112, 64064), (200, 1101, 4160, 64064), (17, 8201, 16448, 0), (6, 66, 20032, 0), (64, 11008, 4096, 64064),
+# tiles whose eight wavefronts split every stage: odd and even numbers of stages, a k that ends inside a piece, few rows, columns
+# that end anywhere (tile 0: a shape the query names no tile for)
+SPLIT = [(65, 4100, 2112, 64064), (200, 2101, 4160, 64064), (17, 8201, 16448, 0), (6, 8193, 20032, 0), (64, 11008, 4096, 64064),
+         (250, 2049, 8256, 64064), (64, 11007, 4160, 64064),
          (256, 4096, 4096, 64064), (96, 8193, 4160, 96064), (77, 13824, 5120, 96064), (65, 12001, 16448, 96064)]
 
 

@@ -233,14 +233,14 @@ def test_libtorch_header_compiles_against_the_c_abi(tmp_path):
 
 
 def test_gemm_kernel_selection_keeps_32_bit_offsets_in_range():
-    """The dispatch rule (host arithmetic, exported as duq_gemm_kernel_for): every kernel family that addresses the
-    weight tensor with 32-bit byte offsets (decode rows 1, decode MFMA 2, dot 3, ring 4, skinny 5) is only picked
-    while the packed weights stay below 2^32 - 256 bytes; anything larger goes to the stream / tile kernels
-    (64-bit per-tile bases).  Also pins the shape buckets."""
+    """The dispatch rule (host arithmetic, exported as duq_gemm_kernel_for): every kernel that addresses the
+    weight tensor with 32-bit byte offsets (decode rows 1, decode MFMA 2, dot 3, LDS 4, skinny 5, wide 8) is only picked
+    while the packed weights stay below 2^32 - 256 bytes; anything larger goes to the prefill kernels
+    (64-bit per-tile bases).  Also pins which kernel runs at the lines between them."""
     from duqlinear4bitcuda_amd import _lib
 
     f = _lib.load().duq_gemm_kernel_for
-    small = {1, 2, 3, 4, 5}
+    small = {1, 2, 3, 4, 5, 8}
     limit = 0xFFFFFF00
     rng = np.random.default_rng(0)
     ks = [64, 128, 4096, 8192, 11008, 12288, 12352, 16384, 16448, 28672, 131008]
@@ -252,19 +252,23 @@ def test_gemm_kernel_selection_keeps_32_bit_offsets_in_range():
                 if N < 1 or N > (1 << 22):
                     continue
                 k = f(M, int(N), K)
-                assert k in (1, 2, 3, 4, 5, 6, 7)
+                assert k in (1, 2, 3, 4, 5, 6, 7, 8)
                 if int(N) * kb >= limit:
                     assert k not in small, (M, N, K, k)
-    # buckets at the benchmark shapes
-    assert [f(m, 4096, 4096) for m in (1, 4, 5, 16, 17, 64, 65, 2048)] == [1, 1, 2, 2, 2, 2, 6, 6]
+    # the benchmark's shapes and the lines: up to 4096 columns, 8192, more; rows of few and of many elements
+    assert [f(m, 4096, 4096) for m in (1, 4, 5, 16, 17, 64, 65, 128, 129, 2048)] == [1, 1, 4, 4, 4, 4, 4, 4, 6, 6]
     assert f(100, 1000, 4096) == 4 and f(200, 520, 8192) == 4 and f(128, 11008, 4096) == 6 and f(128, 28672, 8192) == 6
-    assert f(16, 11008, 4096) == 2 and f(16, 4096, 11008) == 2 and f(16, 28672, 8192) == 2
-    assert f(16, 28672, 4096) == 5 and f(8, 28672, 4096) == 2 and f(64, 28672, 4096) == 2
-    assert f(32, 4096, 8192) == 2 and f(33, 4096, 8192) == 2 and f(17, 4096, 11008) == 2 and f(48, 4096, 12288) == 2
-    assert f(33, 1024, 8192) == 4 and f(32, 1024, 8192) == 2 and f(49, 4096, 11008) != 2 and f(17, 2048, 11008) == 4
-    assert f(1, 28672, 8192) == 1 and f(1, 8192, 28672) == 3 and f(16, 8192, 28672) == 7
-    assert f(16, 64, 16384) == 4 and f(4, 64, 16384) == 1 and f(16, 4096, 12288) == 2
+    assert f(16, 4097, 4096) == 2 and f(16, 4097, 4160) == 4 and f(16, 8192, 4096) == 2 and f(16, 8193, 8256) == 4
+    assert f(24, 8192, 2048) == 4 and f(24, 8192, 2112) == 2 and f(24, 6144, 4096) == 4 and f(24, 6144, 4032) == 2
+    assert f(33, 8192, 4096) == 4 and f(33, 8193, 4096) == 2 and f(33, 8193, 2048) == 8 and f(49, 8193, 2048) == 6
+    assert f(24, 14336, 4096) == 8 and f(24, 14337, 4096) == 2 and f(24, 16385, 6208) == 8 and f(24, 8193, 4160) == 2
+    assert f(16, 11008, 4096) == 2 and f(16, 11008, 6208) == 8 and f(16, 4096, 11008) == 4 and f(16, 28672, 8192) == 8
+    assert f(16, 28672, 4096) == 5 and f(8, 28672, 4096) == 2 and f(64, 28672, 4096) == 2 and f(64, 28672, 2048) == 8
+    assert f(64, 11008, 4096) == 6 and f(64, 8200, 960) == 2 and f(40, 8192, 8192) == 4 and f(40, 8193, 8192) == 6
+    assert f(1, 28672, 8192) == 1 and f(1, 8192, 28672) == 3 and f(4, 8192, 28672) == 4 and f(16, 8192, 28672) == 4
+    assert f(16, 64, 16384) == 4 and f(4, 64, 16384) == 1 and f(4, 64, 16448) == 4 and f(1, 16385, 32000) == 7
     assert f(16, 1 << 22, 4096) == 7 and f(1, 1 << 22, 4096) == 7 and f(64, 1 << 22, 4096) in (6, 7)
+    assert f(65, 4096, 448) == 6 and f(65, 64, 448) == 7 and f(65, 64, 512) == 4 and f(1025, 64, 512) == 4
 
 
 def test_fp16_input_entry_point_validation_without_launch():
@@ -349,7 +353,7 @@ def test_stream_tile_rule():
     assert f(4000, 8200, 4160) == 128256          # three ragged rounds of 256-row tiles against five of 128-row ones
     assert f(2048, 11008, 4096) == 128256         # 344 tiles of 256 rows: two rounds, the second a third full
     assert f(512, 4096, 4096) == 64128 and f(1024, 4096, 4096) == 128128
-    assert f(16, 4096, 4096) == 0 and f(1, 4096, 4096) == 0   # decode kernels
+    assert f(16, 4096, 4096) == 0 and f(1, 4096, 4096) == 0 and f(200, 1101, 4160) == 0   # decode kernels
 
 
 def test_deferred_quantized_tensor_host_side():
