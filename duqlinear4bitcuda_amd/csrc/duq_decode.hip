@@ -1299,7 +1299,7 @@ int launch_decode_s4(const uint8_t *A, const uint8_t *B, uint32_t M, uint32_t N,
     p.y = y;
     if (epi) p.epi = *epi;
     const int mode = out_acc ? -1 : epi->mode;
-    if (!(takes_wide_kernel(M, N, K) ? launch_wide_any(p, mode, stream) : takes_lds_kernel(M, N, K) ? launch_lds_any(p, mode, stream) : launch_decode_any<false>(p, mode, stream))) return (int)hipErrorInvalidValue;
+    if (!(takes_wide_kernel(M, N, K) ? launch_wide_any(p, mode, stream) : takes_lds_kernel(M, N, K, mode == 5) ? launch_lds_any(p, mode, stream) : launch_decode_any<false>(p, mode, stream))) return (int)hipErrorInvalidValue;
     return (int)hipGetLastError();
 }
 

@@ -777,7 +777,8 @@ int launch_gemm_s4_batched(const uint8_t *A, const uint8_t *B, uint32_t M, uint3
     if (M == 0 || N == 0 || batch == 0) return 0;
     if (batch == 1) {
         const int kernel = gemm_kernel_for(M, N, K);
-        if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma || kernel == kKernelWide || kernel == kKernelLds)
+        if (kernel == kKernelDecodeRows || kernel == kKernelDecodeMfma || kernel == kKernelWide || kernel == kKernelLds ||
+            (epi && epi->mode == 5 && takes_lds_kernel(M, N, K, true)))
             return launch_decode_s4(A, B, M, N, K, out_acc, epi, y, stream);
     }
     GemmParams p{};

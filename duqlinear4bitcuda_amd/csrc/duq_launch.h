@@ -115,17 +115,19 @@ inline LdsShape lds_shape(uint32_t M, uint32_t N)
 //    1024 elements on and up to 1024 rows (128 x 1024 x 512 4.4 -> 3.6, x 28672 25.8 -> 11.3; 200 x 2048 x 1024 5.5 -> 5.0, but 128 x
 //    4000 x 512 4.6 -> 5.1 and 7787 x 58 x 6528 11.9 -> 12.5).
 //  - up to 4 rows longer than the rows kernel's 16384 (the dot kernel, one weight row per wavefront pair, or beyond 30720 a
-//    prefill tile): up to 4096 columns (4 x 2606 x 28672 13.4 -> 8.1, 1 x 1024 x 40000 34.2 -> 8.3), above for 3 and 4 rows (4 x
-//    8192 x 28672 28.9 -> 21.8, but 4 x 8192 x 16448 18.6 -> 20.1) and beyond 30720 (1 x 8192 x 40000 49.4 -> 31.1; 1 x 8192 x
-//    28672 21.5 against 22.0).
-inline bool takes_lds_kernel(uint32_t M, uint32_t N, uint32_t K)
+//    prefill tile): up to 4096 columns (4 x 2606 x 28672 13.4 -> 8.1, 1 x 1024 x 40000 34.2 -> 8.3; one row of up to 30720 from
+//    2048 columns on, weights out of the caches 1 x 2600 x 28672 10.6 -> 9.3, but 1 x 1024 x 28672 7.4 -> 8.0 and 1 x 512 x 24576 0.91 times
+//    as fast: the dot kernel has twice the workgroups; the dual-uniform row-sum epilogue, `mode5`, which that one does not have
+//    and which would be a launch more, stays here), above for 3 and 4 rows (4 x 8192 x 28672 28.9 -> 21.8, but 4 x 8192 x 16448 18.6 -> 20.1) and beyond 30720 (1 x 8192 x
+//    40000 49.4 -> 31.1; 1 x 8192 x 28672 21.5 against 22.0).
+inline bool takes_lds_kernel(uint32_t M, uint32_t N, uint32_t K, bool mode5 = false)
 {
     if (M == 0 || K == 0 || K > 65536 || (uint64_t)N * (K / 2) >= 0xFFFFFF00ull) return false;
     if (M > 64) {
         const LdsShape t = lds_shape(M, N);
         return t.rows > 0 && (t.rows * t.cols < 8 ? K >= 512 : K >= 1024 && M <= 1024);
     }
-    if (M <= 4) return K > 16384 && (N <= 4096 || (N <= 16384 && K > (M > 2 ? 18432 : 30720)));
+    if (M <= 4) return K > 16384 && (N <= 4096 ? M > 1 || N >= 2048 || K > 30720 || mode5 : N <= 16384 && K > (M > 2 ? 18432 : 30720));
     if (N <= 4096) return true;
     if (N <= 8192) return M > 32 || K > 4096 || (M > 16 && (K <= 2048 || (N <= 6144 && K % 256 == 0)));
     return K > 8192 && (M <= 16 ? K <= 16384 : M <= 32 && K <= 12288);
@@ -158,7 +160,7 @@ inline bool gemm_fuses_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 // themselves all the same)
 inline bool gemm_applies_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 {
-    return takes_wide_kernel(M, N, K) || takes_lds_kernel(M, N, K) || gemm_fuses_dual_rowsum(M, N, K);
+    return takes_wide_kernel(M, N, K) || takes_lds_kernel(M, N, K, true) || gemm_fuses_dual_rowsum(M, N, K);
 }
 // Tile for a problem select_gemm_kernel gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
 // 64 x 128 tiles (duq_gemm.hip).  Whole rounds of 256 workgroups (one per CU) cost about f + c * (K / 256) microseconds

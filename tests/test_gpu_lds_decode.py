@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 # one, less than a stage, stage boundaries, the longest rows; up to four rows beyond the rows kernel's.  32 columns (stages of
 # 1024 elements): the same, from 4097 columns on.
 SHAPES = [(5, 1, 64), (16, 17, 2048), (17, 15, 2112), (33, 4096, 960), (49, 31, 16448), (64, 48, 1984), (63, 2049, 4160),
-          (8, 16, 65536), (1, 20, 16448), (4, 33, 20480),
+          (8, 16, 65536), (1, 20, 16448), (1, 20, 30784), (1, 2050, 16448), (4, 33, 20480),
           (5, 4097, 4160), (20, 4100, 1088), (40, 4127, 64), (64, 8192, 1024), (16, 8180, 5184), (3, 4100, 18496), (2, 4112, 30784),
           (32, 8200, 8256), (16, 8193, 12352),
           # groups of rows in workgroups of their own: every tile, the most groups there can be, a last group with one row
@@ -30,7 +30,7 @@ def test_lds_kernel_against_the_oracle(hip, dev, M, N, K):  # noqa: F811
     _against_the_oracle(hip, dev, M, N, K)
 
 
-@pytest.mark.parametrize("M,N,K", [(7, 37, 16448), (33, 130, 2112), (24, 4110, 1088), (3, 50, 16448), (20, 8210, 2112), (130, 1000, 1088)])
+@pytest.mark.parametrize("M,N,K", [(1, 40, 16448), (7, 37, 16448), (33, 130, 2112), (24, 4110, 1088), (3, 50, 16448), (20, 8210, 2112), (130, 1000, 1088)])
 def test_lds_kernel_rowsum_epilogues(hip, dev, library_calls, M, N, K):  # noqa: F811
     x = cases.acts_uniform(M, K, seed=31 + M)
     w = (np.random.default_rng(M).standard_normal((N, K)) * 0.02).astype(np.float16)

@@ -267,6 +267,8 @@ def test_gemm_kernel_selection_keeps_32_bit_offsets_in_range():
     assert f(64, 11008, 4096) == 6 and f(64, 8200, 960) == 2 and f(40, 8192, 8192) == 4 and f(40, 8193, 8192) == 6
     assert f(1, 28672, 8192) == 1 and f(1, 8192, 28672) == 3 and f(4, 8192, 28672) == 4 and f(16, 8192, 28672) == 4
     assert f(16, 64, 16384) == 4 and f(4, 64, 16384) == 1 and f(4, 64, 16448) == 4 and f(1, 16385, 32000) == 7
+    # one row of 16385..30720 elements on fewer than 2048 columns stays with the dot kernel
+    assert f(1, 1024, 28672) == 3 and f(1, 2047, 16448) == 3 and f(1, 2048, 16448) == 4 and f(2, 1024, 28672) == 4 and f(1, 64, 30784) == 4
     assert f(16, 1 << 22, 4096) == 7 and f(1, 1 << 22, 4096) == 7 and f(64, 1 << 22, 4096) in (6, 7)
     assert f(65, 4096, 448) == 6 and f(65, 64, 448) == 7 and f(65, 64, 512) == 4 and f(1025, 64, 512) == 4
 
