@@ -23,8 +23,8 @@ def hip(dev):
     return _HIP
 
 
-# rows kernel (M <= 4: every K bucket, K and N tails), MFMA decode kernel (5..16 rows: K buckets of 4096 / 8192 /
-# 12288, tiles that end inside N, several tiles per workgroup), ring kernel for long rows
+# rows kernel (M <= 4: every K bucket, K and N tails); 5 and more rows: LDS kernel (any K, up to 4096 columns and some to 8192),
+# MFMA decode kernel and wide kernel (more columns); tiles that end inside N, several tiles per workgroup
 SHAPES = [(1, 64, 64), (1, 20, 128), (2, 37, 4096), (3, 100, 2048), (4, 4096, 4096), (1, 4096, 4096), (1, 515, 11008),
           (4, 130, 8192), (2, 64, 16384), (3, 33, 12352), (1, 11008, 4096),
           # three or four rows from binary16 on more than 256 column tiles: several tiles per workgroup
@@ -42,18 +42,23 @@ SHAPES = [(1, 64, 64), (1, 20, 128), (2, 37, 4096), (3, 100, 2048), (4, 4096, 40
           # up to eight rows on more than 16384 columns: one launch from binary16 (rows of at most 8192 elements at
           # two to four rows, of at most 4096 at five to eight)
           (4, 20000, 8192), (2, 17000, 4096), (3, 30000, 256), (8, 20000, 4096), (5, 40000, 1024), (7, 17000, 2112),
-          # MFMA decode kernel with two to four row tiles (17..64 rows of at most 4096 elements, 17..32 of at most
-          # 8192), one to several column tiles per workgroup, tiles that end inside M and N
+          # two to four row tiles (LDS kernel but for 64 x 11008 x 4096, tiles that split K, and 29 x 9000 x 4160, MFMA
+          # decode kernel), tiles that end inside M and N
           (17, 4096, 4096), (32, 300, 4096), (33, 4099, 2048), (48, 1000, 4096), (64, 11008, 4096), (50, 72, 64),
           (64, 40, 128), (20, 520, 8192), (32, 4100, 8192), (29, 9000, 4160), (64, 5000, 1024),
-          # the long-row forms (three and four row tiles of up to 8192 elements, two and three of up to 12288: from
-          # 192 column tiles on) and their neighbours on the ring kernel
+          # the same with long rows
           (33, 3072, 8192), (64, 3100, 4160), (48, 4096, 11008), (20, 3080, 12288), (40, 6200, 8256),
           (33, 300, 8192), (64, 130, 4160), (49, 3072, 11008),
           # 9..16 rows on 1536 or more column tiles: the skinny kernel
           (9, 24600, 64), (16, 28672, 256),
-          # rows longer than 16384 elements: the dot kernel
-          (1, 300, 20480), (1, 64, 28672), (1, 130, 16448), (2, 100, 20480), (4, 40, 28672)]
+          # rows longer than 16384 elements: the dot kernel for one row, the LDS kernel for more
+          (1, 300, 20480), (1, 64, 28672), (1, 130, 16448), (2, 100, 20480), (4, 40, 28672),
+          # the dot kernel on more than 4096 columns
+          (1, 4200, 16448), (2, 4112, 20480), (3, 4100, 16448), (4, 8210, 17408),
+          # MFMA decode kernel from packed codes: one to four row tiles of up to 4096 elements, one and two of up to 8192, one
+          # to several column tiles per workgroup
+          (16, 4200, 64), (9, 4100, 320), (7, 4100, 4096), (20, 8190, 2112), (30, 6150, 4032), (24, 14350, 1984), (40, 8200, 2112),
+          (64, 8210, 960), (56, 16390, 2112), (6, 8210, 6080), (12, 17000, 4160)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)

@@ -283,11 +283,11 @@ def test_asym_fp16_input_two_launch_shapes_and_errors(dev):
 
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (4, 11008, 4096), (8, 512, 2048), (3, 100, 8192), (16, 4096, 4096),
                                     (40, 1000, 1024), (100, 1000, 512), (16, 1000, 2048), (9, 200, 4096), (12, 4500, 2560),
-                                    (8, 17000, 512)])
+                                    (8, 17000, 512), (24, 6150, 2112), (16, 24600, 2112), (2, 4200, 16448)])
 def test_dual_uniform_rowsum_layer_decode(dev, library_calls, M, N, K):
     """LinearQuant4bitDUASQRowSum from binary16 rows: one library call up to 1024 rows (one launch up to eight, the
-    quantizer inside the rows kernel; quantizer + GEMM with the epilogue inside for the MFMA decode kernel's shapes;
-    three launches on the ring kernel's); the oracle's bits everywhere, and the op's codes / scales / zero points / row sums."""
+    quantizer inside the rows kernel; quantizer + GEMM with the epilogue inside for the MFMA decode and LDS kernels' shapes;
+    three launches on the skinny and dot kernels'); the oracle's bits everywhere, and the op's codes / scales / zero points / row sums."""
     from duqlinear4bitcuda_amd import _HIP as hip
     from duqlinear4bitcuda_amd.nn import LinearQuant4bitDUASQRowSum
     _say("dual row-sum decode", M, N, K)

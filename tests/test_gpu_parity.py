@@ -163,16 +163,16 @@ def _rand_packed(rng, rows, K):
     (17, 64, 64), (64, 64, 128), (65, 130, 192), (100, 257, 320), (128, 256, 4096), (300, 520, 1024),
     (2048, 4096, 256), (256, 4096, 11008), (130, 1000, 64), (16, 16, 8192), (2, 48, 28672), (7, 48, 28672),
     (9, 40000, 64), (16, 33000, 192), (12, 17000, 8192), (5, 100, 16384),
-    # one to four rows: dot kernel (one row; two rows with K > 4096; up to four with K > 16384), skinny otherwise
+    # one to four rows: rows kernel; of more than 16384 elements the dot kernel for one row, the LDS kernel for more
     (2, 512, 8192), (2, 300, 4096), (3, 300, 20480), (4, 64, 28672), (3, 1000, 2048), (4, 520, 8192), (1, 77, 20480),
-    # ring kernel: 17..64 rows (2, 3, 4 row blocks; several row groups when K is long) and long rows up to 16
+    # LDS kernel: 17..64 rows (2, 3, 4 row tiles; several row groups on narrow problems) and long rows up to 16
     (17, 4096, 4096), (33, 300, 8192), (64, 520, 11008), (48, 4099, 1024), (40, 64, 16384), (16, 300, 11008),
     (9, 4096, 16384), (64, 11008, 4096), (50, 1000, 4160),
-    # ring kernel with several row groups: 65..256 rows of a narrow or short problem
+    # LDS kernel with several row groups: 65..256 rows of a narrow problem
     (100, 1000, 4096), (200, 520, 8192), (90, 300, 11008), (256, 1024, 8192),
-    # stream kernel on 64 x 128 tiles (one round of 64..256 of them), tiles that end inside M, N and K
+    # more columns: LDS kernel's largest tile, 64 x 64, 96 x 64 and 64 x 128 tiles, ends inside M, N and K
     (128, 4096, 4096), (65, 4100, 320), (130, 8000, 4160), (200, 3000, 8192), (500, 4099, 448), (512, 4096, 1024),
-    # and on 128 x 128 tiles (one round where 64 x 128 tiles need two)
+    # 128 x 128 tiles (one round where 64 x 128 tiles need two)
     (700, 4000, 1024), (650, 4100, 1088),
 ])
 def test_matmul_bit_exact(hip, dev, M, N, K):
@@ -241,18 +241,17 @@ def test_dequant_kernels(hip, dev, M, N):
 
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (16, 4096, 4096), (16, 50, 128), (100, 257, 320), (512, 4096, 4096),
                                    (130, 1000, 64),
-                                   # the stream kernel at its three tile heights, aligned and ragged epilogues:
-                                   # 64 rows (1024 x 4096, 900 x 4100), 32 rows (200 x 2051), 128 rows (1100 x 8200)
+                                   # the stream kernel, aligned and ragged epilogues
                                    (1024, 4096, 512), (900, 4100, 128), (200, 2051, 192), (1100, 8200, 320),
-                                   # and on its 64 x 128 tiles
+                                   # 64 x 128 tiles
                                    (128, 4096, 512), (300, 3100, 320), (250, 8190, 384), (100, 4097, 1088),
-                                   # and on its 128 x 128 tiles
+                                   # 128 x 128 tiles
                                    (700, 4000, 1024), (650, 4100, 1088),
                                    # the short-row kernel (K <= 256): whole-line and ragged epilogues, every step count
                                    (300, 1024, 64), (520, 2048, 256), (1000, 520, 192), (65, 4096, 128),
-                                   # two to four rows on either decode kernel
+                                   # two to four rows: rows kernel, LDS kernel
                                    (2, 512, 8192), (3, 300, 20480), (4, 1000, 4096), (2, 300, 4096),
-                                   # ring kernel
+                                   # LDS kernel
                                    (33, 300, 8192), (64, 520, 11008), (48, 4099, 1024), (16, 300, 11008), (20, 4096, 4096),
                                    (100, 1000, 4096), (200, 520, 8192)])
 @pytest.mark.parametrize("with_bias", [False, True])
@@ -282,7 +281,7 @@ def test_fused_forward_equals_unfused_and_oracle(hip, dev, M, N, K, with_bias):
 
 @pytest.mark.parametrize("M,N,K,with_bias", [(4090, 4088, 4160, True), (4096, 4090, 4096, False)])
 def test_stream_kernel_256_row_tiles(hip, dev, M, N, K, with_bias):
-    """The stream kernel's 256 x 256 tiles (problems with at least one per CU): ragged last row tile, a last column
+    """The prefill kernel's 256 x 256 tiles (problems with at least one per CU): ragged last row tile, a last column
     tile that ends inside a 32-column fragment, an odd number of 64-element row segments, whole-line and
     per-element epilogues; int32 accumulators, the four reference epilogues and the row-sum one against the oracle
     over the whole output."""

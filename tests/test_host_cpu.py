@@ -273,6 +273,25 @@ def test_gemm_kernel_selection_keeps_32_bit_offsets_in_range():
     assert f(65, 4096, 448) == 6 and f(65, 64, 448) == 7 and f(65, 64, 512) == 4 and f(1025, 64, 512) == 4
 
 
+def test_gpu_shapes_reach_their_kernels():
+    """The shapes that the GPU tests of the 4-bit GEMM run are the shapes of the kernels that they are there for."""
+    from duqlinear4bitcuda_amd import _lib
+    from tests import test_gpu_decode as dec, test_gpu_lds_decode as lds, test_gpu_prefill_tiles as pre
+
+    f, tile = _lib.load().duq_gemm_kernel_for, _lib.load().duq_gemm_stream_tile_for
+    assert {f(*s) for s in dec.SHAPES} == {1, 2, 3, 4, 5, 6, 8}
+    assert {s[0] for s in dec.SHAPES if f(*s) == 3} == {1, 2, 3, 4}                       # dot kernel: rows
+    forms = {((s[0] + 15) // 16, s[2] > 4096) for s in dec.SHAPES if f(*s) == 2}          # MFMA decode kernel: row tiles, long rows
+    assert forms == {(1, False), (2, False), (3, False), (4, False), (1, True), (2, True)}
+    assert {f(*s) for s in lds.SHAPES} == {3, 4, 8}
+    assert {((s[0] + 15) // 16, -(-s[2] // 2048) if s[2] <= 4096 else 4) for s in lds.SHAPES if f(*s) == 8} == \
+        {(1, 4), (2, 1), (2, 2), (2, 4), (3, 1), (4, 1)}                                  # wide kernel: row tiles, kilobytes of a row
+    one = [s[:3] for s in pre.SHAPES if s[3] == 1] + [s[:3] for s in pre.SPLIT]
+    assert {f(*s) for s in one} == {6, 7}
+    assert {tile(*s) for s in one} == {0, 64064, 96064, 64128, 192128, 128128, 128256, 256256}
+    assert any(tile(*s) == 64064 and s[1] % 2 for s in one)
+
+
 def test_fp16_input_entry_point_validation_without_launch():
     from duqlinear4bitcuda_amd import _lib
 

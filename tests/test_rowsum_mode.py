@@ -344,7 +344,7 @@ def test_dual_rowsum_fused_shapes_and_validation():
     ws = lib.duq_linear4bit_dual_rowsum_workspace_bytes
     assert ws(512, 4096, 4096) == 0 and ws(128, 4096, 512) == 0 and ws(2048, 4096, 4096) == 0 and ws(700, 4000, 1024) == 0
     assert ws(16, 4096, 4096) == 0 and ws(1, 64, 64) == 0 and ws(64, 11008, 4096) == 0   # decode kernels apply it too
-    assert ws(100, 1000, 4096) == 100 * 1000 * 4    # ring kernel
+    assert ws(100, 1000, 4096) == 100 * 1000 * 4    # asked for, not written: the LDS kernel applies it
     assert ws(300, 1028, 320) == 300 * 1028 * 4     # N % 8 != 0
     assert ws(512, 4096, 256) == 512 * 4096 * 4     # short rows
     assert ws(0, 4096, 4096) == 0
