@@ -415,9 +415,9 @@ __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, G
 }
 
 // ---------------------------------------------------------------------------------
-// skinny kernel (5 <= M <= 16 on wide problems: 512 or more 16-column tiles, K <= 8192)
+// skinny kernel (9 <= M <= 16 on wide problems: 1536 or more 16-column tiles, K <= 4096)
 // ---------------------------------------------------------------------------------
-// Workgroup = WAVES wavefronts that split K; it walks `tiles_per_wg` consecutive 16-column
+// Workgroup = four wavefronts that split K; it walks `tiles_per_wg` consecutive 16-column
 // tiles.  Wavefront w owns 64-byte row segments [w*S, (w+1)*S), S <= 8: lane (l16, g) holds
 // bytes [g*16, +16) of each.  The activation fragments of that k range do not depend on the
 // column tile, so they are loaded and expanded ONCE per workgroup and stay in registers;
@@ -431,26 +431,26 @@ __global__ __launch_bounds__(256, 2) void gemm_s4_shortk_kernel(DUQ_HEAD_DECL, G
 // its 16-byte piece s ^ ((row / 2) % 8), which makes the 16 rows x 16 bytes of a fragment read cover every bank
 // once.  Measured 4-9 % faster than MFMA-layout loads from 512 column tiles on; smaller problems run the
 // decode kernels (duq_decode.hip), where the extra LDS hop is not hidden.
+constexpr int kSkinnyWaves = 4;
 constexpr int kSkinnySegs = 8;  // 64-byte segments per wavefront = 128-bit weight loads in flight per lane
 
-
-template <int WAVES, int EPI, bool BIAS>
-__global__ __launch_bounds__(WAVES * 64) void gemm_s4_skinny_kernel(DUQ_HEAD_DECL, GemmParams tail)
+template <int EPI, bool BIAS>
+__global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_s4_skinny_kernel(DUQ_HEAD_DECL, GemmParams tail)
 {
     GemmParams p = with_head(tail, DUQ_HEAD_USE);
     to_global(p.A);
     to_global(p.B);
     to_global(p.C);
     to_global(p.y);
-    __shared__ v4i part[2][WAVES][64];
-    __shared__ __attribute__((aligned(16))) uint8_t turn[WAVES * 8192];
+    __shared__ v4i part[2][kSkinnyWaves][64];
+    __shared__ __attribute__((aligned(16))) uint8_t turn[kSkinnyWaves * 8192];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     const uint32_t l16 = lane & 15u, g = lane >> 4;
     const uint32_t r8 = lane >> 3, j8 = lane & 7u;
     const uint32_t kbytes = p.K >> 1;
     const uint32_t segs = (kbytes + 63) / 64;
-    const uint32_t seg0 = wave * kSkinnySegs;  // the launcher guarantees WAVES * kSkinnySegs >= segs
+    const uint32_t seg0 = wave * kSkinnySegs;  // kSkinnyWaves * kSkinnySegs >= segs: rows of at most 4096 elements
     const uint32_t tiles_per_wg = p.tiles_m;   // (field reused: column tiles per workgroup)
     const uint32_t ntiles = (p.N + 15) / 16;
     const uint32_t tile0 = blockIdx.x * tiles_per_wg;
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_skinny_kernel(DUQ_HEAD_DEC
             const uint32_t src_lane = tid >> 2, r = tid & 3u;
             int sum = 0;
 #pragma unroll
-            for (int w2 = 0; w2 < WAVES; ++w2) sum += part[buf][w2][src_lane][r];
+            for (int w2 = 0; w2 < kSkinnyWaves; ++w2) sum += part[buf][w2][src_lane][r];
             sum >>= 8;
             const uint32_t m = src_lane & 15u, n = tile * 16 + (src_lane >> 4) * 4 + r;
             if (m < p.M && n < p.N) {
@@ -720,22 +720,11 @@ static void launch_epi(GemmParams &p, hipStream_t stream, uint32_t batch = 1)
         return;
     }
     if (kernel == kKernelSkinny) {
-        const uint32_t ntiles = (p.N + 15) / 16;
-        const uint32_t segs = (p.K / 2 + 63) / 64;
         // several column tiles per workgroup (activations are fetched and expanded once per workgroup); at least
-        // ~2 workgroups per CU stay.  Long rows (8 wavefronts per workgroup, one workgroup per CU): whole rounds
-        // of 256 workgroups, at most 8 tiles each.
-        uint32_t tpw = ntiles >= 6144 ? 8 : (ntiles >= 1536 ? 4 : (ntiles >= 640 ? 2 : 1));
-        if (segs > 4 * kSkinnySegs) {
-            const uint32_t rounds = (ntiles + 2047) / 2048;
-            tpw = (ntiles + 256 * rounds - 1) / (256 * rounds);
-        }
+        // ~2 workgroups per CU stay
+        const uint32_t ntiles = (p.N + 15) / 16, tpw = ntiles >= 6144 ? 8 : 4;
         p.tiles_m = tpw;
-        const dim3 grid((ntiles + tpw - 1) / tpw);
-        if (segs <= 4 * kSkinnySegs)
-            DUQ_LAUNCH_HEAD((gemm_s4_skinny_kernel<4, EPI, BIAS>), grid, dim3(256), 0, stream, p);
-        else
-            DUQ_LAUNCH_HEAD((gemm_s4_skinny_kernel<8, EPI, BIAS>), grid, dim3(512), 0, stream, p);
+        DUQ_LAUNCH_HEAD((gemm_s4_skinny_kernel<EPI, BIAS>), dim3((ntiles + tpw - 1) / tpw), dim3(kSkinnyWaves * 64), 0, stream, p);
         return;
     }
     }
