@@ -737,11 +737,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DEC
 // kilobyte of a row, and nothing waits for another wavefront until the sums meet.  32 columns: the
 // activations are a third less of what enters a CU, and the wavefronts share stages of 512 bytes a row, which 64 rows need
 // (8192 x 28672: 29 us against 42 with 64-byte pieces of their own, which are half lines).  Measured against what ran before
-// (N x K, us): 16 rows 4096 x 4096 4.1 -> 3.8, x 8192 6.9 -> 5.5, x 11008 8.5 -> 6.2, 2606 x 26944 31.9 -> 14.1, 8192 x 28672
-// 31.0 -> 21.3; 64 rows 7.4 -> 5.6, 11.2 -> 7.6, 15.2 -> 8.9, 40.6 -> 16.4, 39.2 -> 29.1.  Groups of rows in workgroups of their
-// own, where a column range leaves compute units without work: 64 x 1024 x 8192 7.9 -> 4.4, 128 x 1024 x 8192 8.2 -> 5.4, 256 x
-// 2048 x 4096 9.0 -> 7.4, 96 x 4096 x 11008 14.3 -> 10.4 (64 x 64 tiles of the prefill kernel: half the workgroups and twice the
-// operands each).
+// (N x K, weights out of the caches, us): 16 rows 4096 x 4096 4.25 -> 4.05, x 8192 7.4 -> 5.6, x 11008 9.2 -> 6.9, 2606 x 26944 32.3 ->
+// 14.7, 8192 x 28672 32.2 -> 22.8; 64 rows 7.2 -> 6.0, 13.9 -> 8.3, 17.9 -> 10.1, 40.8 -> 20.4, 40.6 -> 30.7.  Groups of rows in workgroups
+// of their own, where a column range leaves compute units without work: 64 x 1024 x 8192 8.1 -> 4.7, 128 x 1024 x 8192 8.2 -> 5.75,
+// 256 x 2048 x 4096 9.3 -> 7.3, 96 x 4096 x 11008 15.9 -> 11.4 (64 x 64 tiles of the prefill kernel: half the workgroups and twice
+// the operands each).
 template <int MT, int NT, int EPI>
 __global__ __launch_bounds__(512) void gemm_s4_lds_kernel(DUQ_HEAD_DECL, DecodeParams tail)
 {

@@ -77,7 +77,7 @@ int launch_dual_rowsum_dequant(const DualRowsumParams &p, hipStream_t stream);
 // asks for room for accumulators still goes by: gemm_fuses_dual_rowsum).
 enum GemmKernelId {
     kKernelDecodeRows = 1,  // duq_decode.hip, v_dot8_i32_i4, M <= 4
-    kKernelDecodeMfma = 2,  // duq_decode.hip, MFMA, 5 <= M <= 64, K <= 8192 (more than 32 rows: 4096)
+    kKernelDecodeMfma = 2,  // duq_decode.hip, MFMA, activations in registers: 5 <= M <= 64, K <= 8192 (more than 32 rows: 4096)
     kKernelDot = 3,         // duq_gemm.hip, M <= 4 with rows longer than 16384 elements
     kKernelLds = 4,         // duq_decode.hip, both operands through LDS: 5 <= M <= 64 on up to 8192 columns, narrow problems
     kKernelSkinny = 5,      // duq_gemm.hip, 9 <= M <= 16 with 1536 or more column tiles, K <= 4096
@@ -102,24 +102,24 @@ inline LdsShape lds_shape(uint32_t M, uint32_t N)
         if ((rows + t.rows - 1) / t.rows * ((cols + t.cols - 1) / t.cols) <= 256) return t;
     return rows <= 4 ? LdsShape{(uint32_t)rows, 2} : LdsShape{0, 0};
 }
-// Shapes of the LDS kernel (duq_decode.hip), asked next and before select_gemm_kernel.  Measured against the kernels there on 900
-// shapes, us:
-//  - 5..64 rows: every length on up to 4096 columns (7 - 75 % less; 16 x 512 x 1024 3.2 -> 2.9, 64 x 1024 x 8192 7.9 -> 6.7, 16
-//    x 512 x 28672 25.6 -> 7.2).  Up to 8192 columns where the rows are many or long (64 x 5120 x 5120 9.6 -> 7.9, 16 x 8192 x
-//    8192 9.2 -> 8.5, but 16 x 8192 x 4096 5.1 -> 5.4 and 24 x 8192 x 4096 6.1 -> 6.3, and where rows begin inside a cache line, 19 x 5332 x 3648 5.0
-//    -> 5.5: the MFMA kernel keeps its activations in
-//    registers over several column tiles, one fetch of them per CU).  More columns: the lengths that the MFMA kernel does not
-//    hold and for which the ring kernel streams the weights twice (16 x 12288 x 14336 26.8 -> 20.0, 32 x 16384 x 11008 26.9 ->
-//    23.0; 48 x 11008 x 11008 19.8 -> 22.6).
+// Shapes of the LDS kernel (duq_decode.hip), asked next and before select_gemm_kernel.  Measured against what would run otherwise (or
+// ran before it) on 2500 shapes, every weight out of the caches (a pool of 720 MB, 640 MB of other data read before each run), us:
+//  - 5..64 rows: up to 4096 columns (up to 60 % less; 16 x 512 x 1024 3.1 -> 2.9, 64 x 1024 x 8192 8.1 -> 4.7, 16 x 512 x 28672 26.4
+//    -> 10.3) but for up to 16 rows of 2049 to 4095 elements that begin inside a cache line, whose lines are fetched twice (5 x 1434 x
+//    3136 3.2 -> 3.4, 16 x 1024 x 2624 0.92 times as fast; 3072 and 3584 1.0 - 1.06 times, 2048 and 4096 1.1 and 1.05).  Up to 8192
+//    columns where the rows are many or long (64 x 5120 x 5120 11.1 -> 8.5, 16 x 8192 x 8192 10.8 -> 9.2, but 16 x 8192 x 4096 5.3 ->
+//    5.6 and 24 x 8192 x 4096 6.1 -> 6.3, and where rows begin inside a cache line, 19 x 5332 x 3648 5.55 -> 5.95: the MFMA kernel
+//    keeps its activations in registers over several column tiles, one fetch of them per CU).  More columns: lengths that the MFMA
+//    kernel does not hold (16 x 12288 x 14336 27.1 -> 20.8, 32 x 16384 x 11008 28.0 -> 23.1; 48 x 11008 x 11008 20.1 -> 22.8).
 //  - more rows while one round of its workgroups covers them (lds_shape), from 512 elements on, in its largest tile from
-//    1024 elements on and up to 1024 rows (128 x 1024 x 512 4.4 -> 3.6, x 28672 25.8 -> 11.3; 200 x 2048 x 1024 5.5 -> 5.0, but 128 x
-//    4000 x 512 4.6 -> 5.1 and 7787 x 58 x 6528 11.9 -> 12.5).
+//    1024 elements on and up to 1024 rows (128 x 1024 x 512 4.9 -> 3.5, x 28672 33.9 -> 13.5; 200 x 2048 x 1024 6.8 -> 5.0; 128 x 4000 x
+//    512 level).
 //  - up to 4 rows longer than the rows kernel's 16384 (the dot kernel, one weight row per wavefront pair, or beyond 30720 a
-//    prefill tile): up to 4096 columns (4 x 2606 x 28672 13.4 -> 8.1, 1 x 1024 x 40000 34.2 -> 8.3; one row of up to 30720 from
-//    2048 columns on, weights out of the caches 1 x 2600 x 28672 10.6 -> 9.3, but 1 x 1024 x 28672 7.4 -> 8.0 and 1 x 512 x 24576 0.91 times
-//    as fast: the dot kernel has twice the workgroups; the dual-uniform row-sum epilogue, `mode5`, which that one does not have
-//    and which would be a launch more, stays here), above for 3 and 4 rows (4 x 8192 x 28672 28.9 -> 21.8, but 4 x 8192 x 16448 18.6 -> 20.1) and beyond 30720 (1 x 8192 x
-//    40000 49.4 -> 31.1; 1 x 8192 x 28672 21.5 against 22.0).
+//    prefill tile): up to 4096 columns (4 x 2606 x 28672 13.2 -> 9.6, 1 x 1024 x 40000 37.6 -> 11.6; one row of up to 30720 from 2048
+//    columns on, 1 x 2600 x 28672 10.6 -> 9.3, but 1 x 1024 x 28672 7.4 -> 8.0: the dot kernel has twice the workgroups; the
+//    dual-uniform row-sum epilogue, `mode5`, which that one does not have and which would be a launch more, stays here), above
+//    for 3 and 4 rows (4 x 8192 x 28672 31.0 -> 22.9, but 4 x 8192 x 16448 18.4 -> 20.2) and beyond 30720 (1 x 8192 x 40000 46.6 ->
+//    32.0; 1 x 8192 x 28672 22.2 against 22.6).  Behind and left: one and two rows of 16448 on 4096 columns, 0.90 and 0.93.
 inline bool takes_lds_kernel(uint32_t M, uint32_t N, uint32_t K, bool mode5 = false)
 {
     if (M == 0 || K == 0 || K > 65536 || (uint64_t)N * (K / 2) >= 0xFFFFFF00ull) return false;
@@ -128,17 +128,19 @@ inline bool takes_lds_kernel(uint32_t M, uint32_t N, uint32_t K, bool mode5 = fa
         return t.rows > 0 && (t.rows * t.cols < 8 ? K >= 512 : K >= 1024 && M <= 1024);
     }
     if (M <= 4) return K > 16384 && (N <= 4096 ? M > 1 || N >= 2048 || K > 30720 || mode5 : N <= 16384 && K > (M > 2 ? 18432 : 30720));
-    if (N <= 4096) return true;
+    if (N <= 4096) return M > 16 || K <= 2048 || K >= 4096 || K % 256 == 0;
     if (N <= 8192) return M > 32 || K > 4096 || (M > 16 && (K <= 2048 || (N <= 6144 && K % 256 == 0)));
     return K > 8192 && (M <= 16 ? K <= 16384 : M <= 32 && K <= 12288);
 }
-// Shapes of the wide kernel (duq_decode.hip), asked first.  Measured against the MFMA kernel, us: up to 16 rows longer than 6144
-// elements, from 5120 on above 16384 columns (16 x 28672 x 5120 18.1 -> 16.3, 8 x 20000 x 8192 19.2 -> 17.1, but 8 x 16384 x 6144
-// 10.2 -> 10.8, and up to 4096 elements it is level or behind, 16 x 16384 x 4096 7.8 -> 8.3); 17..32 rows of up to 4096 elements
-// on up to 14336 columns (24 x 9000 x 4096 7.7 -> 6.8; 24 x 20000 x 3072 9.6 -> 10.0), of more than 6144 above 16384 (32 x
-// 28672 x 8192 31.1 -> 27.3, but 18 x 33087 x 4160 20.6 -> 22.3, half of whose steps are padding; of fewer columns, tiles of the prefill kernel, 32 x 11008 x 8192 12.3 against 12.9); 33 and more rows of up to
-// 2048 elements (48 x 28672 x 1024 10.7 -> 9.9, longer ones 48 x 13824 x 3072 9.5 -> 10.3), from 49 on above 16384 columns
-// (64 x 28672 x 2048 13.3 -> 12.6, 64 x 13824 x 2048 8.3 -> 8.8).
+// Shapes of the wide kernel (duq_decode.hip), asked first.  Measured against the MFMA kernel, us, (c) out of the caches as above, the
+// others with a few copies of the weight, which decided the lines: up to 16 rows longer than 6144 elements, from 5120 on above
+// 16384 columns ((c) 16 x 28672 x 5120 19.8 -> 17.5, 8 x 20000 x 8192 20.3 -> 17.7; 8 x 16384 x 6144 10.2 -> 10.8, (c) level, and up to
+// 4096 elements it is level or behind, 16 x 16384 x 4096 7.8 -> 8.3); 17..32 rows of up to 4096 elements on up to 14336 columns
+// ((c) 24 x 9000 x 4096 7.8 -> 7.1; 24 x 20000 x 3072 9.6 -> 10.0, (c) 10.6 -> 10.1), of more than 6144 above 16384 ((c) 32 x 28672 x 8192
+// 31.0 -> 27.7; 18 x 33087 x 4160 20.6 -> 22.3, half of whose steps are padding, (c) level; of fewer columns, tiles of the prefill
+// kernel, 32 x 11008 x 8192 12.3 against 12.9, (c) 15.0 against 14.0); 33 and more rows of up to 2048 elements ((c) 48 x 28672 x 1024
+// 11.1 -> 10.0; longer ones 48 x 13824 x 3072 9.5 -> 10.3), from 49 on above 16384 columns ((c) 64 x 28672 x 2048 14.8 -> 12.9, 64 x
+// 13824 x 2048 8.5 -> 8.6).
 inline bool takes_wide_kernel(uint32_t M, uint32_t N, uint32_t K)
 {
     if (M < 5 || M > 64 || N <= 8192 || K == 0 || K > 8192 || (uint64_t)N * (K / 2) >= 0xFFFFFF00ull) return false;

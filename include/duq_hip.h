@@ -222,7 +222,7 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
                          uint64_t workspace_bytes, duq_stream_t stream);
 
 /* Which kernel duq_matmul_host_4bit / duq_linear4bit_forward run for a shape (no GPU work; for tests and tuning): 1 decode
- * rows kernel (M <= 4), 2 decode MFMA kernel (up to 64 rows on more than 4096 columns, where 4, 6 and 8 are not ahead), 3 dot
+ * rows kernel (M <= 4), 2 decode MFMA kernel (5..64 rows, mostly on more than 4096 columns, where 4, 6 and 8 are not ahead), 3 dot
  * kernel (M <= 4, rows longer than 16384 elements), 4 LDS kernel (5..64 rows on up to 4096 columns, 8192 where the rows
  * are many or long, more rows while its tiles are one round of workgroups, very long rows), 5 skinny kernel (9 <= M <= 16,
  * very wide problems), 6 prefill kernel (short rows: stream kernel), 7 the same on problems of few tiles or long rows, 8

@@ -259,6 +259,8 @@ def test_gemm_kernel_selection_keeps_32_bit_offsets_in_range():
     assert [f(m, 4096, 4096) for m in (1, 4, 5, 16, 17, 64, 65, 128, 129, 2048)] == [1, 1, 4, 4, 4, 4, 4, 4, 6, 6]
     assert f(100, 1000, 4096) == 4 and f(200, 520, 8192) == 4 and f(128, 11008, 4096) == 6 and f(128, 28672, 8192) == 6
     assert f(16, 4097, 4096) == 2 and f(16, 4097, 4160) == 4 and f(16, 8192, 4096) == 2 and f(16, 8193, 8256) == 4
+    # up to 16 rows of 2049..4095 elements that begin inside a cache line: the MFMA kernel
+    assert f(16, 4096, 2048) == 4 and f(16, 4096, 2112) == 2 and f(5, 64, 4032) == 2 and f(17, 4096, 2112) == 4 and f(16, 4096, 2304) == 4
     assert f(24, 8192, 2048) == 4 and f(24, 8192, 2112) == 2 and f(24, 6144, 4096) == 4 and f(24, 6144, 4032) == 2
     assert f(33, 8192, 4096) == 4 and f(33, 8193, 4096) == 2 and f(33, 8193, 2048) == 8 and f(49, 8193, 2048) == 6
     assert f(24, 14336, 4096) == 8 and f(24, 14337, 4096) == 2 and f(24, 16385, 6208) == 8 and f(24, 8193, 4160) == 2
