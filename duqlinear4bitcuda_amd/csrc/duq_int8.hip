@@ -909,8 +909,8 @@ __global__ __launch_bounds__(512) void gemm_s8_lds_kernel(DUQ_HEAD_DECL, Gemm8Pa
 //    several groups 1.05 - 3.0, and with rows longer than 4096 elements, which the decode kernel does not hold, 1.0 - 3.5 (up
 //    to four rows of 16384 elements 0.9 - 1.15).
 //  - tiled, rows in one group of up to 4096 elements, whose decode kernel keeps the activations of up to 2048 or 4096 elements in
-//    registers: ahead or level where those are not full (16 x 4096 columns: K 512 / 1024 / 1536 / 2080 / 4096 1.04 / 1.07 / 1.02 /
-//    1.12 / 1.11, but 2048 0.93; 24 rows 1.0 / 1.0 / 0.98 / 1.10 / 1.08, 2048 0.91), with two column tiles a workgroup (more than 4096 columns) only for short
+//    registers: ahead or level where those are not full (16 x 4096 columns: K 512 / 1024 / 2080 / 4096 1.04 / 1.07 / 1.12 /
+//    1.11, but 1248 0.95 (most of a stage is padding) and 2048 0.93; 24 rows 1.0 / 1.0 / 0.98 / 1.10 / 1.08, 2048 0.91), with two column tiles a workgroup (more than 4096 columns) only for short
 //    rows, registers that are half empty, or many rows (8192 columns: 16 x 1024 1.03, x 2080 1.05, x 4096 0.95; 32 x 512 1.03, x 2560
 //    1.05, x 4096 0.93; 64 x 2560 1.24, x 4096 1.18; 40 x 3072 1.03, x 4096 0.96).
 //  - up to 16 rows in several rounds, the last of which may leave most compute units idle (9000 columns: 282 workgroups): the weight as
@@ -934,7 +934,7 @@ inline bool lds8_takes(uint32_t M, uint32_t N, uint32_t K, bool tiled)
     if (!tiled || groups > 1) return true;
     if (K > 4096) return M > 4 || K <= 12288;
     if (K > 2048) return t.cols == 1 || K <= 2560 || M > 40 || (M > 32 && K <= 3072);
-    return K <= (t.cols == 1 || M <= 16 || M > 48 ? 1024u : 512u) || (t.cols == 1 && M <= 16 && (K <= 1920 || M <= 12));
+    return K <= (t.cols == 1 || M <= 16 || M > 48 ? 1024u : 512u) || (t.cols == 1 && M <= 16 && K > 1536 && (K <= 1920 || M <= 12));
 }
 
 template <bool FUSED, bool BIAS, bool TILED>

@@ -289,7 +289,7 @@ def test_gemm8_kernel_rule():
     rows, decode, lds, skinny, split, tile = 1, 2, 3, 4, 5, 6
     # (tokens, columns, elements): tiled copy, weight as stored
     for shape, want in {(4, 4096, 4096): (decode, rows), (2, 4096, 8192): (lds, rows), (5, 4096, 4096): (lds, lds),
-                        (16, 4096, 4096): (lds, lds), (16, 4096, 2048): (decode, lds), (16, 4097, 4096): (decode, lds),
+                        (16, 4096, 4096): (lds, lds), (16, 4096, 2048): (decode, lds), (8, 4096, 1056): (decode, lds), (8, 4096, 2048): (lds, lds), (16, 4097, 4096): (decode, lds),
                         (16, 8192, 1024): (lds, lds), (16, 8193, 1024): (decode, lds), (16, 8193, 768): (lds, lds),
                         (8, 11008, 4096): (decode, lds), (16, 11008, 4096): (decode, lds), (16, 12288, 4096): (decode, lds),
                         (16, 11008, 6144): (lds, lds), (8, 8200, 8192): (skinny, lds), (8, 11008, 8192): (lds, lds), (16, 11008, 8192): (lds, lds), (8, 13824, 16384): (skinny, lds), (16, 13824, 4096): (decode, decode),
