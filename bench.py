@@ -803,7 +803,7 @@ def main():
                        "best_7b_frac": max(d["frac_hbm"] for d in rows_7b),
                        "read_floor_frac": round(worst["read_floor_GBps"] / PEAK_HBM_GBS, 4),
                        # the GEMM launch of that row (the quantizer launch of 16 rows before it moves 0.2 MB)
-                       "traffic": profile_shape_traffic_bytes("decode_kernels__bench_shapes.txt", "gemm_s4_decode_kernel<8, 4, 0, 1,", 256)
+                       "traffic": profile_shape_traffic_bytes("decode_kernels__bench_shapes.txt", "gemm_s4_lds_kernel<1, 1, 0>", 256)
                        if (worst["M"], worst["N"]) == (16, 4096) else None,
                        "traffic_source": "profiles/decode_kernels__bench_shapes.txt"}
 

@@ -908,10 +908,10 @@ __global__ __launch_bounds__(512) void gemm_s4_lds_kernel(DUQ_HEAD_DECL, DecodeP
 // The MFMA kernel's plan, several column tiles per workgroup against activations held in registers, with the LDS kernel's way
 // in: weights arrive in whole cache lines, without registers, and six to eight steps of 2 KB per wavefront are in flight
 // whatever tile they belong to, so that no tile begins with a wait.  The activations take the same way, as the first steps of
-// the sequence.  What bounds a launch is the reading of the weights, 4.9 TB/s at 16 x 28672 x 8192 (4.1 before).  A load whose
+// the sequence.  What bounds a launch is the reading of the weights, 4.7 TB/s at 16 x 28672 x 8192 (4.05 before).  A load whose
 // result the compiler waits for would empty that queue: eight wavefronts only load and multiply, and four others fetch the
-// parameters, add up the eight partial tiles and store, one tile behind.  Measured (us): 16 x 28672 x 8192 28.6 -> 24.1, x
-// 16384 x 8192 15.4 -> 14.1, 24 x 28672 x 8192 30.3 -> 26.6, 32 x 11008 x 4096 8.5 -> 7.4, 48 x 11008 x 2048 7.7 -> 6.6.
+// parameters, add up the eight partial tiles and store, one tile behind.  Measured (us, weights out of the caches): 16 x 28672 x
+// 8192 29.0 -> 24.9, x 16384 x 8192 17.5 -> 15.3, 24 x 28672 x 8192 30.3 -> 27.4, 32 x 11008 x 4096 8.6 -> 7.8, 48 x 11008 x 2048 7.6 -> 6.8.
 template <int MT, int KS>
 struct WideTile {
     static constexpr int kPart = MT * 8 * 1024;                              // one tile's partial sums

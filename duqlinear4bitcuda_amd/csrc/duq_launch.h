@@ -164,7 +164,7 @@ inline bool gemm_applies_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 {
     return takes_wide_kernel(M, N, K) || takes_lds_kernel(M, N, K, true) || gemm_fuses_dual_rowsum(M, N, K);
 }
-// Tile for a problem select_gemm_kernel gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
+// Tile for a problem gemm_kernel_for gives to the prefill kernel (duq_prefill.hip) or, `stream`, to the stream kernel's
 // 64 x 128 tiles (duq_gemm.hip).  Whole rounds of 256 workgroups (one per CU) cost about f + c * (K / 256) microseconds
 // each, measured per tile shape (N = 4096, one round, K = 1024 / 4096 / 16384): 64 x 128 6.6 / 11.9 / 33, 128 x 128 8.9 /
 // 17.5 / 55, 128 x 256 12.5 / 30 / 100, 256 x 256 21 / 52.7 / 178 (1.3 of it once per launch); the cheapest wins.  192 x 128

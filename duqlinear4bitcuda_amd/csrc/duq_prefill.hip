@@ -21,8 +21,8 @@
 // launch lasts as long as one workgroup's walk over K.  64 x 64 tiles (96 x 64 for 65..96 rows on wide layers) whose eight
 // wavefronts each take an eighth of every stage: twice the workgroups, half the walk (0.2 us per 256 k against 0.44),
 // for a longer end, since eight partial tiles have to meet (5.5 us with the start against 3.6).  128 x 4096 x 4096 10.5 ->
-// 8.7 us, 128 x 4096 x 11008 22.5 -> 16.9, 64 x 4096 x 16384 30.6 -> 22.7, 77 x 4096 x 28672 43.4 -> 32.5; 72 x 3072 x 4096,
-// on the ring kernel before, 13.8 -> 8.5; 96 x 64: 77 x 13824 x 5120 15.1 -> 14.4 (3.9 TB/s of weights).  A 128 x 64 tile
+// 8.7 us, 128 x 4096 x 11008 22.5 -> 16.9, 64 x 4096 x 16384 30.6 -> 22.7, 77 x 4096 x 28672 43.4 -> 32.5 (these narrow ones run
+// the LDS kernel of duq_decode.hip by now); 96 x 64: 77 x 13824 x 5120 15.1 -> 14.4 (3.9 TB/s of weights).  A 128 x 64 tile
 // measured behind 64 x 128 (512 x 4096 x 4096 13.4 against 12.4).
 #include "duq_gemm_common.h"
 #include <type_traits>
