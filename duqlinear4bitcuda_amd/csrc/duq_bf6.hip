@@ -24,9 +24,18 @@
 //
 // Kernel: tile 128 (M) x 256 (N) per workgroup, 4 wavefronts side by side along N (128 x 64
 // each: 8 x 4 MFMA tiles, 128 accumulator registers).  Weights go global -> registers (a ring
-// of four 128-k steps), activations global -> registers -> LDS (three buffers of 256 k, one
+// of four 128-k steps), activations into LDS (three buffers of 256 k, one
 // barrier per buffer) -> fragments read two MFMA groups ahead.  The weight operand is the
 // MFMA "A" side, so a lane ends up with four consecutive output columns of one row.
+// What bounds it is the bytes that a CU takes in: 72 KB per 256 k of a 128-row tile are 1152 cycles at 64 bytes a cycle,
+// against 1024 of MFMAs; the 256-row tile's 96 KB meet 2048.  Its activations used to be fetched 128 k at a time, half a
+// cache line of plane 0 and a quarter of plane 1 per row, and the L2 delivers whole lines: 80.7 million of them where 44
+// would do (4096 x 8192 x 28672), 176 KB per 256 k instead of 112.  Chunks of 256 k fit since they go to LDS without
+// registers: 51.4 million lines, 549 -> 462 us with the quantizer (first 5 ms of a load; 491 -> 416 later), 4096 x 4096 x
+// 4096 56.5 -> 50.2, 2048 x 8192 x 8192 93.5 -> 80.5; the 64-row tiles 1000 x 4096 x 11008 43.6 -> 39.4.  LDS holds the
+// pieces in swizzled order instead of padded rows: bank conflicts 44 -> 6 % of its cycles.  The 128-row tile is the one that
+// is faster with its activations loaded to registers first and stored a body later (2048 x 4096 x 4096 31.5 against 32.6):
+// they reach LDS a chunk earlier, and there the CU's intake is what is short.
 #include "duq_epilogue.h"
 #include "duq_launch.h"
 #include "duq_tiles.h"
@@ -139,7 +148,7 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 #define DUQ_BF6_COST64 0.68f
 #endif
 #ifndef DUQ_BF6_COST256
-#define DUQ_BF6_COST256 1.78f
+#define DUQ_BF6_COST256 1.6f
 #endif
 #ifndef DUQ_BF6_NARROW_MAX_TILES
 #define DUQ_BF6_NARROW_MAX_TILES 128
@@ -248,15 +257,12 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
     // 64-row tiles only: twice the workgroups for problems that leave CUs without a 64 x 256 tile)
     static_assert(TNI == 4 || (TNI == 2 && TMI == 4), "column tiles per wavefront");
     constexpr int BM = 16 * TMI, BN = 64 * TNI;
-    constexpr int CH = TMI == 16 ? 1 : 2;  // 128-k steps per activation chunk
-    constexpr int NPH = 4 / CH;            // chunk bodies per turn of the weight ring
-    // 16-byte activation pieces per thread and chunk: plane 0 (4*CH per row), plane 1 (2*CH per row)
-    constexpr int NX0 = BM * 4 * CH / 256, NX1 = BM * 2 * CH / 256, NXP = NX0 + NX1;
-    // LDS bytes per row: the 16-byte (8-byte) parts of the 4*CH blocks of a chunk + 16 bytes of padding, which
-    // makes the fragment reads of 16 rows conflict-free
-    constexpr uint32_t kP0Stride = 64 * CH + 16, kP1Stride = 32 * CH + 16;
-    constexpr uint32_t kP1Base = BM * kP0Stride;
-    constexpr uint32_t kBuf = BM * (kP0Stride + kP1Stride);
+    constexpr int CH = 2;                                   // 128-k steps per activation chunk
+    constexpr int NXA = TMI / 2, NXB = TMI / 4, NXP = NXA + NXB;  // activation loads per wavefront and chunk, a kilobyte each
+    constexpr uint32_t kP1Base = BM * 128;                  // a chunk: BM rows of 128 bytes (plane 0), then of 64 (plane 1)
+    constexpr uint32_t kBuf = BM * 192;
+    // The 128-row tile's activations go through registers, those of the others to LDS directly (see the kernel's head).
+    constexpr bool STAGED = TMI == 8;
     constexpr uint32_t kYStride = 32 * TNI + 16;  // bytes per staged output row: 16*TNI binary16 + pad
     constexpr uint32_t kLds = 3 * kBuf > 4 * BM * kYStride ? 3 * kBuf : 4 * BM * kYStride;
     constexpr bool LATE_PARAMS = TMI == 16;
@@ -321,8 +327,6 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
     const uint32_t wpairs = (min(p.N - n0, (uint32_t)BN) / 16 + 1) / 2;  // pairs of 16-row weight tiles in this tile
     const __amdgpu_buffer_rsrc_t rW =
         make_rsrc(p.W + (uint64_t)(n0 / 32) * ksteps * 3072, wpairs * ksteps * 3072);
-    const __amdgpu_buffer_rsrc_t rX =
-        make_rsrc(p.X + (uint64_t)m0 * row_bytes, min(p.M - m0, (uint32_t)BM) * row_bytes);
     const __amdgpu_buffer_rsrc_t rNone = make_rsrc(p.X, 0);  // every read returns zero
 
     // weight fragments (2*pi, 2*pi + 1) of step g: 3072 bytes at ((wave*NP + pi) * ksteps + g) * 3072, three 16-byte
@@ -342,33 +346,68 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
         dst[4 * part + 0] = a[0], dst[4 * part + 1] = a[1], dst[4 * part + 2] = a[2], dst[4 * part + 3] = a[3];
     };
 
-    // activation pieces of a chunk (256 k = 8 blocks): NX0 of plane 0 and NX1 of plane 1 per thread
-    uint32_t xoff[NXP], xlds[NXP];
+    // activations: load j of this wavefront brings eight whole lines of plane 0 (j < NXA) or sixteen half lines of plane 1
+    // into LDS; lane l's 16 bytes land 16 * l behind the load's base, so the lane's source swizzles: piece q of row r lies at
+    // position q ^ ((r / 2) % 8) of the row's 128 bytes, q ^ ((r / 4) % 4) of its 64.
+    auto desc = [](const uint8_t *base, uint32_t bytes) {
+        const uint64_t a = reinterpret_cast<uint64_t>(base);
+        return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
+                   (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+    };
+    const v4u dX = desc(p.X + (uint64_t)m0 * row_bytes, min(p.M - m0, (uint32_t)BM) * row_bytes);
+    const uint32_t uwave = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    uint32_t xoff[NXP];  // of the next chunk to be fetched, less what load_x adds first
 #pragma unroll
-    for (int j = 0; j < NX0; ++j) {
-        const uint32_t row = tid / (4 * CH) + j * (256 / (4 * CH)), piece = tid % (4 * CH);
-        xoff[j] = row * row_bytes + piece * 16;
-        xlds[j] = row * kP0Stride + piece * 16;
+    for (int j = 0; j < NXA; ++j) {
+        const uint32_t row = (wave * NXA + j) * 8 + (lane >> 3), piece = (lane & 7u) ^ ((row >> 1) & 7u);
+        xoff[j] = row * row_bytes + piece * 16 - 128;
     }
 #pragma unroll
-    for (int j = 0; j < NX1; ++j) {
-        const uint32_t row = tid / (2 * CH) + j * (256 / (2 * CH)), piece = tid % (2 * CH);
-        xoff[NX0 + j] = row * row_bytes + p1off + piece * 16;
-        xlds[NX0 + j] = kP1Base + row * kP1Stride + piece * 16;
+    for (int j = 0; j < NXB; ++j) {
+        const uint32_t row = (wave * NXB + j) * 16 + (lane >> 2), piece = (lane & 3u) ^ ((row >> 2) & 3u);
+        xoff[NXA + j] = row * row_bytes + p1off + piece * 16 - 64;
     }
-    // piece j of chunk c.  The chunk offset rides in the vector offset so that the range check sees it: when
-    // K is an odd number of steps the last chunk's second half reads the next row (unused) or, in the last
-    // row, past the descriptor (zero).
-    auto load_x = [&](v4u &dst, int j, uint32_t c, __amdgpu_buffer_rsrc_t r) {
-        dst = buf_load16(r, xoff[j] + (j < NX0 ? c * (64 * CH) : c * (32 * CH)), 0);
+    // Load j of the next chunk (d: of chunk c, chunk_desc) to buffer buf.  The chunk's offset is part of the vector offset, which
+    // the range check sees: with an odd number of steps the last chunk's second half reads on in its row's next plane or the next
+    // row, or past the descriptor (zeros), and meets weights of zero.
+    auto chunk_desc = [&](uint32_t c) {
+        v4u d = dX;
+        d[2] = c < nchunks ? d[2] : 0u;  // chunks past the end: every lane out of range, zeros
+        return d;
+    };
+    auto load_x = [&](int j, const v4u d, uint32_t buf) {
+        if (j < NXA)
+            asm volatile("s_add_u32 m0, %1, %2\n\tv_add_u32 %0, 0x80, %0\n\tbuffer_load_dwordx4 %0, %3, 0 offen lds"
+                         : "+v"(xoff[j])
+                         : "s"(lds0 + uwave * (NXA * 1024) + buf), "n"(j * 1024), "s"(d)
+                         : "memory", "m0", "scc");
+        else
+            asm volatile("s_add_u32 m0, %1, %2\n\tv_add_u32 %0, 64, %0\n\tbuffer_load_dwordx4 %0, %3, 0 offen lds"
+                         : "+v"(xoff[j])
+                         : "s"(lds0 + uwave * (NXB * 1024) + buf), "n"(kP1Base + (j - NXA) * 1024), "s"(d)
+                         : "memory", "m0", "scc");
+    };
+    // the same through registers: piece j of chunk c, and its way to buffer buf
+    v4u xreg[NXP];
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(p.X + (uint64_t)m0 * row_bytes, min(p.M - m0, (uint32_t)BM) * row_bytes);
+    auto fetch_x = [&](v4u &dst, int j, uint32_t c) {
+        dst = buf_load16(c < nchunks ? rX : rNone, xoff[j] + (j < NXA ? (c + 1) * 128 : (c + 1) * 64), 0);
+    };
+    auto store_x = [&](const v4u &src, int j, uint32_t buf) {
+        *reinterpret_cast<v4u *>(lds + buf + (j < NXA ? (wave * NXA + j) * 1024 : kP1Base + (wave * NXB + j - NXA) * 1024) + lane * 16) = src;
     };
 
-    // fragment of rows mi*16 + l16, k-step s of a chunk: plane 0 + mi*16*kP0Stride + s*64, plane 1 + ... + s*32
-    const uint32_t frag0 = l16 * kP0Stride + kb * 16, frag1 = kP1Base + l16 * kP1Stride + kb * 8;
+    // fragment of rows mi*16 + l16, k-step s of a chunk
+    uint32_t frag0[CH], frag1[CH];
+#pragma unroll
+    for (int s = 0; s < CH; ++s) {
+        frag0[s] = l16 * 128 + (((s * 4 + kb) ^ ((l16 >> 1) & 7u)) * 16);
+        frag1[s] = kP1Base + l16 * 64 + (((s * 2 + (kb >> 1)) ^ ((l16 >> 2) & 3u)) * 16) + (kb & 1u) * 8;
+    }
 
     v12i wf[4][NP];   // weight fragment pairs [ring slot][pair of column tiles], pinned to v[kRingBase + 12 * (slot * NP + pi) ..]
     v6i xf[4];        // activation fragments, ring over mi
-    v4u xreg[NXP];
     v4f acc[TMI][TNI];
 #pragma unroll
     for (int a = 0; a < TMI; ++a)
@@ -376,40 +415,52 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
         for (int b = 0; b < TNI; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
 
     auto read_x0 = [&](v6i &dst, uint32_t buf, int mi, int s) {
-        const v4i a = *reinterpret_cast<const v4i *>(lds + buf + frag0 + mi * 16 * kP0Stride + s * 64);
+        const v4i a = *reinterpret_cast<const v4i *>(lds + buf + frag0[s] + mi * 2048);
         dst[0] = a[0], dst[1] = a[1], dst[2] = a[2], dst[3] = a[3];
     };
     auto read_x1 = [&](v6i &dst, uint32_t buf, int mi, int s) {
-        const v2i b = *reinterpret_cast<const v2i *>(lds + buf + frag1 + mi * 16 * kP1Stride + s * 32);
+        const v2i b = *reinterpret_cast<const v2i *>(lds + buf + frag1[s] + mi * 1024);
         dst[4] = b[0], dst[5] = b[1];
     };
 
-    // ---- prologue: weights of steps 0..3, activations of chunks 0 and 1 -> LDS, chunk 2 -> registers.  Issued
-    // in the order of first use, so that the wait for the two activation chunks (vector memory waits are in
-    // order) leaves the weights of steps 1..3 in flight: all 256 workgroups start together and their first
-    // ~170 KB each are bound by the L2 -> CU rate, not by latency.
+    // ---- prologue: activations of chunks 0 and 1 -> LDS (chunk 2 -> registers), weights of steps 0..2 (0..3), in the order of
+    // first use, so that the wait for the activations leaves the weights of later steps in flight: all 256 workgroups start
+    // together and their first ~170 KB each are bound by the L2 -> CU rate, not by latency.  (Weights of step 3: the direct
+    // form's loop fetches them in its first step.)
     v4u x1[NXP];
 #pragma unroll
-    for (int j = 0; j < NXP; ++j) load_x(xreg[j], j, 0, rX);
+    for (int j = 0; j < NXP; ++j)
+        if constexpr (STAGED)
+            fetch_x(xreg[j], j, 0);
+        else
+            load_x(j, dX, 0);
 #pragma unroll
     for (int pi = 0; pi < NP; ++pi)
 #pragma unroll
         for (int part = 0; part < 3; ++part) load_w(wf[0][pi], pi, part, 0, rW);
 #pragma unroll
-    for (int j = 0; j < NXP; ++j) load_x(x1[j], j, 1, 1 < nchunks ? rX : rNone);
+    for (int j = 0; j < NXP; ++j)
+        if constexpr (STAGED)
+            fetch_x(x1[j], j, 1);
+        else
+            load_x(j, chunk_desc(1), kBuf);
 #pragma unroll
-    for (int g = 1; g < 4; ++g)
+    for (int g = 1; g < (STAGED ? 4 : 3); ++g)
 #pragma unroll
         for (int pi = 0; pi < NP; ++pi)
 #pragma unroll
             for (int part = 0; part < 3; ++part) load_w(wf[g][pi], pi, part, g, (uint32_t)g < ksteps ? rW : rNone);
+    if constexpr (STAGED) {
 #pragma unroll
-    for (int j = 0; j < NXP; ++j) *reinterpret_cast<v4u *>(lds + xlds[j]) = xreg[j];
+        for (int j = 0; j < NXP; ++j) store_x(xreg[j], j, 0);
 #pragma unroll
-    for (int j = 0; j < NXP; ++j) *reinterpret_cast<v4u *>(lds + kBuf + xlds[j]) = x1[j];
+        for (int j = 0; j < NXP; ++j) store_x(x1[j], j, kBuf);
 #pragma unroll
-    for (int j = 0; j < NXP; ++j) load_x(xreg[j], j, 2, 2 < nchunks ? rX : rNone);
-    lds_barrier();
+        for (int j = 0; j < NXP; ++j) fetch_x(xreg[j], j, 2);
+        lds_barrier();
+    } else {
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(9 * NP + NXP) : "memory");
+    }
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi) {
         read_x0(xf[mi], 0, mi, 0);
@@ -441,11 +492,15 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
 
     // One chunk = CH 128-k steps.  PH = position of the chunk in a turn of the weight ring: its steps use ring
     // slots CH*PH ..; a slot is refilled (with the step four ahead) during the step after its use.
-    auto chunk = [&](auto ph, uint32_t c, uint32_t cur, uint32_t nxt, uint32_t nx2) {
+    uint32_t cur = 0, nxt = kBuf, nx2 = 2 * kBuf;  // buffers of chunks c, c + 1, c + 2
+    auto chunk = [&](auto ph, auto last, uint32_t c) {
         constexpr int PH = decltype(ph)::value;
+        const v4u dXc = chunk_desc(c + 2);
+        // Vector memory instructions of this body up to its barrier, all of them behind the loads that the barrier waits for
+        // (direct form).  After the loop the compiler leaves out weight loads that nothing reads: only the activations count.
+        constexpr int kBehind = NXP + (decltype(last)::value ? 0 : TNI == 4 && TMI == 4 ? 10 : 6 * NP);
         // Side work is spread one instruction per MFMA: the loop is bound by the issue rate of its single
         // wavefront per SIMD, and a slot that holds more than about 12 cycles of other work stalls the matrix pipe.
-        const __amdgpu_buffer_rsrc_t rXc = c + 3 < nchunks ? rX : rNone;
 #pragma unroll
         for (int s = 0; s < CH; ++s) {
             const int slot = CH * PH + s;
@@ -461,6 +516,15 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
                     // cannot know of; the generated loop has none, and the bit-exact parity tests would show one.
                     mfma_pinned<kRingBase>(slot * NP + ni / 2, ni & 1, acc[mi][ni], wf[slot][ni / 2], xf[mi & 3]);
                     __builtin_amdgcn_sched_barrier(0);
+                    if (s == CH - 1 && mi == TMI - 2 && ni == 0) {
+                        // The next chunk is read from here on: it has to be there.  Every read of this chunk is done, so that
+                        // the next body may overwrite it.
+                        if constexpr (STAGED)
+                            lds_barrier();
+                        else
+                            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBehind) : "memory");
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                     // ---- side work in the shadow of this MFMA
                     if (ni < 2) {  // activation fragment two groups ahead
                         const int nm = (mi + 2) & (TMI - 1), ns = mi + 2 < TMI ? s : s + 1;
@@ -470,7 +534,7 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
                         else
                             read_x1(xf[nm & 3], buf, nm, ns % CH);
                     }
-                    // refill the previous step's slot: 3 * NP loads over the step (step 0 fetches step 3 again)
+                    // refill the previous step's slot: 3 * NP loads over the step
                     {
                         int widx = -1;  // which of the 3 * NP loads rides with this MFMA
                         if (TNI == 2) widx = mi < 2 ? mi * 2 + ni : -1;
@@ -479,19 +543,15 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
                         if (TNI == 4 && TMI == 16) widx = (ni == 2 && (mi & 1) == 0) ? mi / 2 : -1;
                         if (widx >= 0 && widx < 3 * NP) load_w(wf[prev][widx / 3], widx / 3, widx % 3, gprev, rG);
                     }
-                    if (TNI == 2 && s == 1 && mi >= 2) {  // three activation pieces per chunk: store, then refetch
-                        const int slot2 = (mi - 2) * 2 + ni;  // 0..3
-                        if (slot2 < NXP) *reinterpret_cast<v4u *>(lds + nx2 + xlds[slot2]) = xreg[slot2];
-                        if (slot2 >= 1 && slot2 <= NXP) load_x(xreg[slot2 - 1], slot2 - 1, c + 3, rXc);
-                    }
-                    // chunk c+2 -> its LDS buffer and, one group (one slot) later, chunk c+3 into the freed register
-                    if (TNI == 4 && TMI <= 8 && s == 1 && mi < NXP && ni == (TMI == 8 ? 3 : 0))
-                        *reinterpret_cast<v4u *>(lds + nx2 + xlds[mi]) = xreg[mi];
-                    if (TNI == 4 && TMI <= 8 && s == 1 && ni == 1 && mi >= 1 && mi <= NXP)
-                        load_x(xreg[mi - 1], mi - 1, c + 3, rXc);
-                    if (TMI == 16 && (mi & 1) == 1 && (mi >> 1) < NXP) {
-                        if (ni == 2) *reinterpret_cast<v4u *>(lds + nx2 + xlds[mi >> 1]) = xreg[mi >> 1];
-                        if (ni == 3) load_x(xreg[mi >> 1], mi >> 1, c + 3, rXc);
+                    if constexpr (STAGED) {  // chunk c + 2 -> its buffer and, one group later, chunk c + 3 into the freed register
+                        if (s == 1 && mi < NXP && ni == 3) store_x(xreg[mi], mi, nx2);
+                        if (s == 1 && ni == 1 && mi >= 1 && mi <= NXP) fetch_x(xreg[mi - 1], mi - 1, c + 3);
+                    } else {  // chunk c + 2 -> its buffer
+                        int xidx = -1;
+                        if (TNI == 2) xidx = s == 0 && mi >= 2 ? (mi - 2) * 2 + ni : -1;
+                        if (TNI == 4 && TMI == 4) xidx = s == 0 && ni == 0 ? mi : -1;
+                        if (TMI == 16) xidx = ni == 2 && (mi & 1) == 1 && mi < 12 ? s * 6 + mi / 2 : -1;
+                        if (xidx >= 0 && xidx < NXP) load_x(xidx, dXc, nx2);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -500,52 +560,24 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
         // the MFMAs are opaque to the compiler's hazard tracking: any accumulator copy it places
         // at a control-flow join must find them retired
         asm volatile("s_nop 15" ::: "memory");
-        lds_barrier();
-    };
-
-    uint32_t cur = 0, nxt = kBuf, nx2 = 2 * kBuf;
-    auto rotate = [&]() {
         const uint32_t t = cur;
         cur = nxt;
         nxt = nx2;
         nx2 = t;
     };
+
     using P0 = std::integral_constant<int, 0>;
     using P1 = std::integral_constant<int, 1>;
-    using P2 = std::integral_constant<int, 2>;
-    using P3 = std::integral_constant<int, 3>;
     uint32_t c = 0;
     // (no branch inside the loop: a path that skips a chunk would make the compiler count only that
     // path's loads when it waits for a fragment, and drain the prefetch ring every iteration)
-    if (NPH == 2) {
-        for (; c + 1 < nchunks; c += 2) {
-            chunk(P0{}, c, cur, nxt, nx2);
-            rotate();
-            chunk(P1{}, c + 1, cur, nxt, nx2);
-            rotate();
-        }
-        if (c < nchunks) chunk(P0{}, c, cur, nxt, nx2);
-    } else {
-        for (; c + 3 < nchunks; c += 4) {
-            chunk(P0{}, c, cur, nxt, nx2);
-            rotate();
-            chunk(P1{}, c + 1, cur, nxt, nx2);
-            rotate();
-            chunk(P2{}, c + 2, cur, nxt, nx2);
-            rotate();
-            chunk(P3{}, c + 3, cur, nxt, nx2);
-            rotate();
-        }
-        if (c < nchunks) {
-            chunk(P0{}, c, cur, nxt, nx2);
-            rotate();
-            if (c + 1 < nchunks) {
-                chunk(P1{}, c + 1, cur, nxt, nx2);
-                rotate();
-                if (c + 2 < nchunks) chunk(P2{}, c + 2, cur, nxt, nx2);
-            }
-        }
+    for (; c + 1 < nchunks; c += 2) {
+        chunk(P0{}, std::false_type{}, c);
+        chunk(P1{}, std::false_type{}, c + 1);
     }
+    if (c < nchunks) chunk(P0{}, std::true_type{}, c);
+    // (every wavefront's loads and reads are done: the epilogue stages its outputs over the buffers)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (LATE_PARAMS) load_params();
     // the MFMAs above are opaque to the compiler's hazard tracking: let the last ones retire
     asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");

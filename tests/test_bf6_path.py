@@ -245,6 +245,23 @@ def test_gpu_forward_bf6_equals_oracle(hip, dev, M, N, K, with_bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(4096 - 100, 4096, 640), (4096, 4096 - 16, 1152), (1000, 4096, 640), (1000, 4096, 1408), (500, 2048, 640),
+                                   (500, 2048 - 80, 1152), (2048 - 9, 4096, 640), (2048, 4096, 1152)])
+def test_gpu_forward_bf6_chunks(hip, dev, M, N, K):
+    """Three and more 256-k chunks, an odd number of them, the last one half full, on 256-, 64- and 128-row tiles: buffers that
+    come round again, loads that run past the row and past the last row."""
+    print("bf6 chunks", M, N, K, flush=True)
+    rng = np.random.default_rng(M + 3 * N + K)
+    a, b = _rand_packed(rng, M, K), _rand_packed(rng, N, K)
+    sr, _, sc1, _, _, _, bias = _epi_inputs(rng, M, N)
+    T = lambda v: cases.t(v, dev)
+    want = orc.add_bias(orc.sym_dequant(orc.matmul_s4(a, b), sr, sc1), bias)
+    got = hip.linear4bit_forward_bf6(hip.EPI_SYM, hip.activation_shadow_bf6(T(a)), T(sr), None, hip.weight_shadow_bf6(T(b)), T(sc1),
+                                     bias=T(bias)).cpu().numpy()
+    assert cases.bits_equal(got, want)
+
+
+@pytest.mark.gpu
 def test_gpu_forward_bf6_extreme_accumulation(hip, dev):
     """Every product 64 (or -64) over the longest row the library takes: |acc| = 64 * 130944, the largest
     magnitude the float32 accumulator has to hold exactly; plus rows that cancel to small odd sums."""
