@@ -182,28 +182,37 @@ inline bool gemm_applies_dual_rowsum(uint32_t M, uint32_t N, uint32_t K)
 struct StreamTile {
     uint32_t rows, cols;
     bool stream;
-    uint32_t main_cols = 0, rest_rows = 0;  // main_cols > 0: from that column on, tiles of rest_rows x 128
+    // main_cols > 0: fused, tiles of main_rows x 256 up to that column and of rest_rows x rest_cols from there on (rows x cols: int32 out)
+    uint32_t main_cols = 0, rest_rows = 0, main_rows = 0, rest_cols = 0;
 };
-// Rounds that do not come out even: tiles of 128 x 256 over as many columns as fill whole rounds, and the columns that are
-// left in one round of smaller tiles, 192 x 128, 128 x 128 or 64 x 128, in the same launch (a launch of their own would start
-// when the last large tile has ended).  Taken where the model above has it 4 % ahead of every uniform choice; measured, in
-// turn: 2048 x 6144 x 4096 50.9 -> 46.4 us, 4000 x 8200 x 4160 150 -> 137, 1999 x 11008 x 4096 81.3 -> 79.7.  (192 x 256 tiles are
-// ahead of it there, 77.9, but behind on 3000 x 5000 x 2048 and 2500 x 12000 x 5120, 46.7 against 34.5 and 134 against 119.)
+// Rounds that do not come out even: tiles of 128 x 256 or 256 x 256 over as many columns as fill whole rounds, and the columns
+// that are left in one round of smaller tiles, 192 x 128, 128 x 128, 64 x 128 or (behind 256 x 256) 128 x 256, in the same launch
+// (a launch of their own would start when the last large tile has ended).  Taken where the model above has it 4 % ahead of every uniform choice; measured, in
+// turn, against uniform tiles: 2048 x 6144 x 4096 50.9 -> 46.4 us, 4000 x 8200 x 4160 150 -> 137.  One round of 256 x 256 costs
+// 2.62 per 256 k where two of 128 x 256 cost 2.94 (a CU takes in a third less for the same outputs), and one end instead of two;
+// against whole rounds of 128 x 256, with the quantizer, in the first 5 ms of a load: 1999 x 11008 x 4096 96.5 -> 87.1, 1188 x
+// 14615 x 3136 73.5 -> 64.0, 2195 x 14547 x 4800 172 -> 149, 3806 x 4832 x 2048 52.9 -> 49.1; of 17 shapes the least 1.03, the mean 1.12.
 // Of 75 shapes drawn at random (128..4096 rows, 700..20000 columns) it and the 192 x 128 tiles alone change fifteen, by 1.02 to
 // 1.34 (147 x 24961 x 14464); rows of less than 2048 elements lose by it (1234 x 6658 x 832 0.87).
 inline StreamTile with_rest(StreamTile best, float best_cost, uint32_t M, uint32_t N, float nch)
 {
-    const uint32_t tm = (M + 127) / 128, rounds = (uint32_t)((uint64_t)tm * ((N + 255) / 256) / 256), cols = rounds * 256 / tm * 256;
-    if (rounds == 0 || cols >= N || nch < 8.0f) return best;
+    if (nch < 8.0f) return best;
     best_cost *= 0.96f;
-    const uint32_t rm[3] = {192, 128, 64};
-    const float c_us[3] = {1.146f, 0.76f, 0.44f}, f_us[3] = {7.1f, 4.3f, 3.6f};
-    for (int k = 0; k < 3; ++k) {
-        if ((uint64_t)((M + rm[k] - 1) / rm[k]) * ((N - cols + 127) / 128) > 256) continue;
-        const float cost = (float)rounds * (nch * 1.47f + 5.5f) + nch * c_us[k] + f_us[k];
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = StreamTile{128, 256, false, cols, rm[k]};
+    const uint32_t main_rows[2] = {128, 256};
+    const float main_c[2] = {1.47f, 2.62f}, main_f[2] = {5.5f, 9.5f};
+    const uint32_t rm[4] = {192, 128, 64, 128}, rn[4] = {128, 128, 128, 256};
+    const float c_us[4] = {1.146f, 0.76f, 0.44f, 1.47f}, f_us[4] = {7.1f, 4.3f, 3.6f, 5.5f};
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t tm = (M + main_rows[i] - 1) / main_rows[i], rounds = (uint32_t)((uint64_t)tm * ((N + 255) / 256) / 256);
+        const uint32_t cols = rounds * 256 / tm * 256;
+        if (rounds == 0 || cols >= N) continue;
+        for (int k = 0; k < 4; ++k) {
+            if ((i == 0 && k == 3) || (uint64_t)((M + rm[k] - 1) / rm[k]) * ((N - cols + rn[k] - 1) / rn[k]) > 256) continue;
+            const float cost = (float)rounds * (nch * main_c[i] + main_f[i]) + nch * c_us[k] + f_us[k];
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = StreamTile{128, 256, false, cols, rm[k], main_rows[i], rn[k]};
+            }
         }
     }
     return best;

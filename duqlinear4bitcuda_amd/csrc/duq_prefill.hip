@@ -380,13 +380,13 @@ using Tile64x128 = PrefillTile<2, 2, 1, 2, 4, 256>;
 using Tile128x128 = PrefillTile<2, 2, 2, 2, 2, 256>;
 using Tile192x128 = PrefillTile<3, 2, 2, 2, 2, 128>;
 using Tile128x256 = PrefillTile<2, 2, 2, 4, 1, 128>;
+using Tile256x256 = PrefillTile<4, 2, 2, 4, 1, 128>;
 
-// Rounds that do not come out even: p.tiles_m x p.tiles_n tiles of 128 x 256, as many as fill whole rounds of 256 workgroups,
-// and behind them the columns that are left in tiles of another kind.
-template <typename Rest, int EPI, bool BIAS>
+// Rounds that do not come out even: p.tiles_m x p.tiles_n tiles of 128 x 256 or 256 x 256, as many as fill whole rounds of 256
+// workgroups, and behind them the columns that are left in tiles of another kind.
+template <typename Tile, typename Rest, int EPI, bool BIAS>
 __global__ __launch_bounds__(512) void gemm_s4_prefill_mixed_kernel(DUQ_HEAD_DECL, GemmParams tail)
 {
-    using Tile = Tile128x256;
     GemmParams p = with_head(tail, DUQ_HEAD_USE);
     to_global(p.A);
     to_global(p.B);
@@ -405,15 +405,26 @@ __global__ __launch_bounds__(512) void gemm_s4_prefill_mixed_kernel(DUQ_HEAD_DEC
     }
 }
 
-// Whole rounds of 128 x 256 tiles over the first tile.main_cols columns, the rest in other tiles behind them.
-template <typename Rest, int EPI, bool BIAS>
+// Whole rounds of such tiles over the first tile.main_cols columns, the rest in other tiles behind them.
+template <typename Tile, typename Rest, int EPI, bool BIAS>
 static int launch_mixed(GemmParams &p, const StreamTile &tile, hipStream_t stream)
 {
-    p.tiles_m = (p.M + 127) / 128;
-    p.tiles_n = tile.main_cols / 256;
+    p.tiles_m = (p.M + Tile::BM - 1) / Tile::BM;
+    p.tiles_n = tile.main_cols / Tile::BN;
     const uint32_t rest = ((p.M + Rest::BM - 1) / Rest::BM) * ((p.N - tile.main_cols + Rest::BN - 1) / Rest::BN);
-    DUQ_LAUNCH_HEAD((gemm_s4_prefill_mixed_kernel<Rest, EPI, BIAS>), dim3(p.tiles_m * p.tiles_n + rest), dim3(512), 0, stream, p);
+    DUQ_LAUNCH_HEAD((gemm_s4_prefill_mixed_kernel<Tile, Rest, EPI, BIAS>), dim3(p.tiles_m * p.tiles_n + rest), dim3(512), 0, stream, p);
     return (int)hipGetLastError();
+}
+
+template <typename Tile, int EPI, bool BIAS>
+static int launch_mixed(GemmParams &p, const StreamTile &tile, hipStream_t stream)
+{
+    if constexpr (Tile::BM == 256) {
+        if (tile.rest_cols == 256) return launch_mixed<Tile, Tile128x256, EPI, BIAS>(p, tile, stream);
+    }
+    return tile.rest_rows == 192   ? launch_mixed<Tile, Tile192x128, EPI, BIAS>(p, tile, stream)
+           : tile.rest_rows == 128 ? launch_mixed<Tile, Tile128x128, EPI, BIAS>(p, tile, stream)
+                                   : launch_mixed<Tile, Tile64x128, EPI, BIAS>(p, tile, stream);
 }
 
 template <int EPI, bool BIAS>
@@ -422,9 +433,8 @@ static int launch_prefill_epi(GemmParams &p, StreamTile tile, hipStream_t stream
     const uint32_t bm = tile.rows, bn = tile.cols;
     if constexpr (EPI >= 0 && EPI != 5) {
         if (tile.main_cols)
-            return tile.rest_rows == 192   ? launch_mixed<Tile192x128, EPI, BIAS>(p, tile, stream)
-                   : tile.rest_rows == 128 ? launch_mixed<Tile128x128, EPI, BIAS>(p, tile, stream)
-                                           : launch_mixed<Tile64x128, EPI, BIAS>(p, tile, stream);
+            return tile.main_rows == 256 ? launch_mixed<Tile256x256, EPI, BIAS>(p, tile, stream)
+                                         : launch_mixed<Tile128x256, EPI, BIAS>(p, tile, stream);
     }
     p.tiles_m = (p.M + bm - 1) / bm;
     p.tiles_n = (p.N + bn - 1) / bn;

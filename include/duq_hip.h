@@ -230,8 +230,8 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
  * are only picked while N * K / 2 < 2^32 - 256; larger tensors run 6 and 7, whose bases are 64-bit per tile.  No counterpart
  * in the reference (CUTLASS picks its own tile, src/kernels/gemm.cu:17-42). */
 int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
-/* For a shape of kernel 6: its tile as rows * 1000 + columns (256256, 128256, 192128, 128128, 64128, 96064, 64064; the fused
- * entry points may cover the last columns of a problem in smaller tiles); 0 for the other kernels.  (The dual-uniform row-sum
+/* For a shape of kernel 6: its tile as rows * 1000 + columns (256256, 128256, 192128, 128128, 64128, 96064, 64064; 128256 also
+ * where the fused entry points cover the last columns of a problem in smaller tiles, behind tiles of 128 x 256 or 256 x 256); 0 for the other kernels.  (The dual-uniform row-sum
  * epilogue never runs the 256-row tile.) */
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
 

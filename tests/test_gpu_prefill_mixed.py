@@ -19,6 +19,18 @@ def test_mixed(dev, M, N, K):
     check(dev, M, N, K, 1)
 
 
+# (the query names one tile for both kinds of first part)
+@pytest.mark.parametrize("M,N,K", [(690, 13001, 2112), (1999, 5003, 2112),    # 64 x 128 behind one round of 128 x 256
+                                   (520, 21912, 2560),                       # 192 x 128 behind 1
+                                   (935, 20001, 2112), (1203, 15441, 2176),    # 128 x 128 behind one round of 256 x 256
+                                   (1801, 12518, 2112)])                      # 128 x 256 behind one
+def test_mixed_of_either_kind(dev, M, N, K):
+    from duqlinear4bitcuda_amd import _HIP as hip
+    print("mixed", M, N, K, flush=True)
+    assert hip.gemm_stream_tile_for(M, N, K) == 128256
+    check(dev, M, N, K, 1)
+
+
 @pytest.mark.parametrize("M,N,K,n", [(1536, 4096, 2048, 1), (1501, 4001, 4160, 1), (700, 8190, 2112, 1), (190, 1000, 4096, 17)])
 def test_192_row_tiles(dev, M, N, K, n):
     from duqlinear4bitcuda_amd import _HIP as hip
