@@ -32,10 +32,10 @@
 // cache line of plane 0 and a quarter of plane 1 per row, and the L2 delivers whole lines: 80.7 million of them where 44
 // would do (4096 x 8192 x 28672), 176 KB per 256 k instead of 112.  Chunks of 256 k fit since they go to LDS without
 // registers: 51.4 million lines, 549 -> 462 us with the quantizer (first 5 ms of a load; 491 -> 416 later), 4096 x 4096 x
-// 4096 56.5 -> 50.2, 2048 x 8192 x 8192 93.5 -> 80.5; the 64-row tiles 1000 x 4096 x 11008 43.6 -> 39.4.  LDS holds the
-// pieces in swizzled order instead of padded rows: bank conflicts 44 -> 6 % of its cycles.  The 128-row tile is the one that
-// is faster with its activations loaded to registers first and stored a body later (2048 x 4096 x 4096 31.5 against 32.6):
-// they reach LDS a chunk earlier, and there the CU's intake is what is short.
+// 4096 56.5 -> 50.2, 2048 x 8192 x 8192 93.5 -> 80.5.  LDS holds the pieces in swizzled order instead of padded rows: bank
+// conflicts 44 -> 6 % of its cycles.  The smaller tiles are faster with their activations loaded to registers first and stored
+// a body later (2048 x 4096 x 4096 31.5 against 32.6, 505 x 8960 x 4560 36.9 / 38.8): they are asked for a chunk earlier, and
+// there the CU's intake is what is short.
 #include "duq_epilogue.h"
 #include "duq_launch.h"
 #include "duq_tiles.h"
@@ -144,12 +144,6 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 #define DUQ_BF6_STORE_AUX 2
 #endif
 
-#ifndef DUQ_BF6_COST64
-#define DUQ_BF6_COST64 0.68f
-#endif
-#ifndef DUQ_BF6_COST256
-#define DUQ_BF6_COST256 1.6f
-#endif
 #ifndef DUQ_BF6_NARROW_MAX_TILES
 #define DUQ_BF6_NARROW_MAX_TILES 128
 #endif
@@ -245,41 +239,38 @@ static_assert(offsetof(Bf6Params, epi) + 8 == kHeadBytes, "the fields delivered 
 // with at least one such tile per CU: the same weight traffic feeds twice the MFMAs, which takes the kernel off
 // the L2 -> CU limit that bounds the smaller tiles; all 256 AGPRs hold accumulators, an activation chunk is one
 // 128-k step (three buffers of two steps would not fit in LDS) and the epilogue parameters are fetched after the loop.
+template <int TMI, int TNI, int EPI>
+struct Bf6Tile {
+    static constexpr int BM = 16 * TMI, BN = 64 * TNI;
+    static constexpr uint32_t kBuf = BM * 192;             // a chunk of 256 k: BM rows of 128 bytes (plane 0), then of 64 (plane 1)
+    static constexpr uint32_t kYStride = 32 * TNI + 16;    // bytes per staged output row: 16*TNI binary16 + pad
+    static constexpr uint32_t kLds = 3 * kBuf > 4 * BM * kYStride ? 3 * kBuf : 4 * BM * kYStride;
+};
+
+// The tile of rows m0 .. and columns n0 ...  lds: Bf6Tile::kLds bytes; dpar, dwide: staged parameters of EPI 5.
 template <int TMI, int TNI, int EPI, bool BIAS>
-__global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params tail)
+__device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint32_t *dpar, uint32_t &dwide, const uint32_t m0, const uint32_t n0)
 {
-    Bf6Params p = with_head(tail, DUQ_HEAD_USE);
-    to_global(p.X);
-    to_global(p.W);
-    to_global(p.y);
     static_assert(TMI == 16 || TMI == 8 || TMI == 4, "16-row MFMA tiles per wavefront along M");
     // TNI = 16 x 16 MFMA tiles per wavefront along N: BM rows x 64 columns (TNI = 4), or BM x 32 (TNI = 2, with
     // 64-row tiles only: twice the workgroups for problems that leave CUs without a 64 x 256 tile)
     static_assert(TNI == 4 || (TNI == 2 && TMI == 4), "column tiles per wavefront");
-    constexpr int BM = 16 * TMI, BN = 64 * TNI;
+    using Tile = Bf6Tile<TMI, TNI, EPI>;
+    constexpr int BM = Tile::BM, BN = Tile::BN;
     constexpr int CH = 2;                                   // 128-k steps per activation chunk
     constexpr int NXA = TMI / 2, NXB = TMI / 4, NXP = NXA + NXB;  // activation loads per wavefront and chunk, a kilobyte each
-    constexpr uint32_t kP1Base = BM * 128;                  // a chunk: BM rows of 128 bytes (plane 0), then of 64 (plane 1)
-    constexpr uint32_t kBuf = BM * 192;
-    // The 128-row tile's activations go through registers, those of the others to LDS directly (see the kernel's head).
-    constexpr bool STAGED = TMI == 8;
-    constexpr uint32_t kYStride = 32 * TNI + 16;  // bytes per staged output row: 16*TNI binary16 + pad
-    constexpr uint32_t kLds = 3 * kBuf > 4 * BM * kYStride ? 3 * kBuf : 4 * BM * kYStride;
+    constexpr uint32_t kP1Base = BM * 128, kBuf = Tile::kBuf, kYStride = Tile::kYStride;
+    // The 256-row tile's activations go to LDS directly, those of the others through registers (see the kernel's head).
+    constexpr bool STAGED = TMI != 16;
     constexpr bool LATE_PARAMS = TMI == 16;
     constexpr int MODE = EPI;
 
-    __shared__ __attribute__((aligned(16))) uint8_t lds[kLds];
-    // dual-uniform row-sum epilogue (EPI 5): its parameters, eight words per column of the tile and per row, fetched
+    // dual-uniform row-sum epilogue (EPI 5): its parameters in dpar, eight words per column of the tile and per row, fetched
     // by the first BN / BM threads before the loop and read back from here after it (the records of the integer
     // kernel's epilogue, gemm_s4_stream_kernel)
     //   column: wlo, whi (first eight bytes of the packed weight row), s1 | s2 << 16, z1, z2, adj1, adj2, bias
     //   row   : xlo, xhi & 0xFF (first ten codes of the packed activation row), float(s), z, rx - rxl, rxl
-    __shared__ __attribute__((aligned(16))) uint32_t dpar[EPI == 5 ? (BN + BM) * 8 : 4];
-    __shared__ uint32_t dwide;  // EPI 5: non-zero when a factor of the corrections leaves the signed 24-bit range
-
-    uint32_t tile_m, tile_n;
-    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-    const uint32_t m0 = tile_m * BM, n0 = tile_n * BN;
+    // dwide: non-zero when a factor of the corrections leaves the signed 24-bit range
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     const uint32_t l16 = lane & 15u, kb = lane >> 4;
@@ -346,57 +337,41 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
         dst[4 * part + 0] = a[0], dst[4 * part + 1] = a[1], dst[4 * part + 2] = a[2], dst[4 * part + 3] = a[3];
     };
 
-    // activations: load j of this wavefront brings eight whole lines of plane 0 (j < NXA) or sixteen half lines of plane 1
-    // into LDS; lane l's 16 bytes land 16 * l behind the load's base, so the lane's source swizzles: piece q of row r lies at
-    // position q ^ ((r / 2) % 8) of the row's 128 bytes, q ^ ((r / 4) % 4) of its 64.
+    // activations: load j of this wavefront brings eight whole lines of plane 0 (j < NXA; rows 32 * j + 8 * wave ..) or sixteen
+    // half lines of plane 1 (rows 64 * (j - NXA) + 16 * wave ..).  Lane l's 16 bytes go to 16 * l behind the load's base in LDS, so the
+    // lane's source swizzles: piece q of row r lies at position q ^ ((r / 2) % 8) of the row's 128 bytes, q ^ ((r / 4) % 4) of its 64.
+    const uint32_t uwave = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
+    const uint32_t xrow0 = wave * 8 + (lane >> 3), xrow1 = wave * 16 + (lane >> 2);
+    const uint32_t xoff0 = xrow0 * row_bytes + ((lane & 7u) ^ ((xrow0 >> 1) & 7u)) * 16,
+                   xoff1 = xrow1 * row_bytes + p1off + ((lane & 3u) ^ ((xrow1 >> 2) & 3u)) * 16;
+    // (the chunk's offset is part of the vector offset, which the range check sees: with an odd number of steps the last chunk's
+    // second half reads on in its row's next plane or the next row, or past the descriptor (zeros), and meets weights of zero)
+    auto x_off = [&](int j, uint32_t c) {
+        return j < NXA ? xoff0 + (j * 32 * row_bytes + c * 128) : xoff1 + ((j - NXA) * 64 * row_bytes + c * 64);
+    };
+    auto x_lds = [&](int j) { return j < NXA ? j * 4096 : kP1Base + (j - NXA) * 4096; };  // + 1024 * wave
     auto desc = [](const uint8_t *base, uint32_t bytes) {
         const uint64_t a = reinterpret_cast<uint64_t>(base);
         return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
     };
     const v4u dX = desc(p.X + (uint64_t)m0 * row_bytes, min(p.M - m0, (uint32_t)BM) * row_bytes);
-    const uint32_t uwave = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
-    uint32_t xoff[NXP];  // of the next chunk to be fetched, less what load_x adds first
-#pragma unroll
-    for (int j = 0; j < NXA; ++j) {
-        const uint32_t row = (wave * NXA + j) * 8 + (lane >> 3), piece = (lane & 7u) ^ ((row >> 1) & 7u);
-        xoff[j] = row * row_bytes + piece * 16 - 128;
-    }
-#pragma unroll
-    for (int j = 0; j < NXB; ++j) {
-        const uint32_t row = (wave * NXB + j) * 16 + (lane >> 2), piece = (lane & 3u) ^ ((row >> 2) & 3u);
-        xoff[NXA + j] = row * row_bytes + p1off + piece * 16 - 64;
-    }
-    // Load j of the next chunk (d: of chunk c, chunk_desc) to buffer buf.  The chunk's offset is part of the vector offset, which
-    // the range check sees: with an odd number of steps the last chunk's second half reads on in its row's next plane or the next
-    // row, or past the descriptor (zeros), and meets weights of zero.
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds + uwave * 1024;
     auto chunk_desc = [&](uint32_t c) {
         v4u d = dX;
         d[2] = c < nchunks ? d[2] : 0u;  // chunks past the end: every lane out of range, zeros
         return d;
     };
-    auto load_x = [&](int j, const v4u d, uint32_t buf) {
-        if (j < NXA)
-            asm volatile("s_add_u32 m0, %1, %2\n\tv_add_u32 %0, 0x80, %0\n\tbuffer_load_dwordx4 %0, %3, 0 offen lds"
-                         : "+v"(xoff[j])
-                         : "s"(lds0 + uwave * (NXA * 1024) + buf), "n"(j * 1024), "s"(d)
-                         : "memory", "m0", "scc");
-        else
-            asm volatile("s_add_u32 m0, %1, %2\n\tv_add_u32 %0, 64, %0\n\tbuffer_load_dwordx4 %0, %3, 0 offen lds"
-                         : "+v"(xoff[j])
-                         : "s"(lds0 + uwave * (NXB * 1024) + buf), "n"(kP1Base + (j - NXA) * 1024), "s"(d)
-                         : "memory", "m0", "scc");
+    // load j of chunk c (d: chunk_desc(c)) to buffer buf
+    auto load_x = [&](int j, uint32_t c, const v4u d, uint32_t buf) {
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds" ::"s"(lds0 + buf), "n"(x_lds(j)), "v"(x_off(j, c)), "s"(d)
+                     : "memory", "m0", "scc");
     };
-    // the same through registers: piece j of chunk c, and its way to buffer buf
+    // the same through registers: load j of chunk c, and its way to buffer buf
     v4u xreg[NXP];
     const __amdgpu_buffer_rsrc_t rX = make_rsrc(p.X + (uint64_t)m0 * row_bytes, min(p.M - m0, (uint32_t)BM) * row_bytes);
-    auto fetch_x = [&](v4u &dst, int j, uint32_t c) {
-        dst = buf_load16(c < nchunks ? rX : rNone, xoff[j] + (j < NXA ? (c + 1) * 128 : (c + 1) * 64), 0);
-    };
-    auto store_x = [&](const v4u &src, int j, uint32_t buf) {
-        *reinterpret_cast<v4u *>(lds + buf + (j < NXA ? (wave * NXA + j) * 1024 : kP1Base + (wave * NXB + j - NXA) * 1024) + lane * 16) = src;
-    };
+    auto fetch_x = [&](v4u &dst, int j, uint32_t c) { dst = buf_load16(c < nchunks ? rX : rNone, x_off(j, c), 0); };
+    auto store_x = [&](const v4u &src, int j, uint32_t buf) { *reinterpret_cast<v4u *>(lds + buf + tid * 16 + x_lds(j)) = src; };
 
     // fragment of rows mi*16 + l16, k-step s of a chunk
     uint32_t frag0[CH], frag1[CH];
@@ -433,7 +408,7 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
         if constexpr (STAGED)
             fetch_x(xreg[j], j, 0);
         else
-            load_x(j, dX, 0);
+            load_x(j, 0, dX, 0);
 #pragma unroll
     for (int pi = 0; pi < NP; ++pi)
 #pragma unroll
@@ -443,7 +418,7 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
         if constexpr (STAGED)
             fetch_x(x1[j], j, 1);
         else
-            load_x(j, chunk_desc(1), kBuf);
+            load_x(j, 1, chunk_desc(1), kBuf);
 #pragma unroll
     for (int g = 1; g < (STAGED ? 4 : 3); ++g)
 #pragma unroll
@@ -498,7 +473,7 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
         const v4u dXc = chunk_desc(c + 2);
         // Vector memory instructions of this body up to its barrier, all of them behind the loads that the barrier waits for
         // (direct form).  After the loop the compiler leaves out weight loads that nothing reads: only the activations count.
-        constexpr int kBehind = NXP + (decltype(last)::value ? 0 : TNI == 4 && TMI == 4 ? 10 : 6 * NP);
+        constexpr int kBehind = NXP + (decltype(last)::value ? 0 : 6 * NP);
         // Side work is spread one instruction per MFMA: the loop is bound by the issue rate of its single
         // wavefront per SIMD, and a slot that holds more than about 12 cycles of other work stalls the matrix pipe.
 #pragma unroll
@@ -516,13 +491,10 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
                     // cannot know of; the generated loop has none, and the bit-exact parity tests would show one.
                     mfma_pinned<kRingBase>(slot * NP + ni / 2, ni & 1, acc[mi][ni], wf[slot][ni / 2], xf[mi & 3]);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (s == CH - 1 && mi == TMI - 2 && ni == 0) {
-                        // The next chunk is read from here on: it has to be there.  Every read of this chunk is done, so that
-                        // the next body may overwrite it.
-                        if constexpr (STAGED)
-                            lds_barrier();
-                        else
-                            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBehind) : "memory");
+                    if (!STAGED && s == CH - 1 && mi == TMI - 2 && ni == 0) {
+                        // The next chunk is read from here on: its loads, issued before those of this body, have to be there.
+                        // Every read of this chunk is done, so that the next body's loads may overwrite it.
+                        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBehind) : "memory");
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     // ---- side work in the shadow of this MFMA
@@ -544,14 +516,11 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
                         if (widx >= 0 && widx < 3 * NP) load_w(wf[prev][widx / 3], widx / 3, widx % 3, gprev, rG);
                     }
                     if constexpr (STAGED) {  // chunk c + 2 -> its buffer and, one group later, chunk c + 3 into the freed register
-                        if (s == 1 && mi < NXP && ni == 3) store_x(xreg[mi], mi, nx2);
-                        if (s == 1 && ni == 1 && mi >= 1 && mi <= NXP) fetch_x(xreg[mi - 1], mi - 1, c + 3);
+                        const int slot2 = TNI == 2 ? (mi - 2) * 2 + ni : ni == (TMI == 8 ? 3 : 0) ? mi : -1, next2 = TNI == 2 ? slot2 : ni == 1 ? mi : 0;
+                        if (s == 1 && slot2 >= 0 && slot2 < NXP) store_x(xreg[slot2], slot2, nx2);
+                        if (s == 1 && next2 >= 1 && next2 <= NXP) fetch_x(xreg[next2 - 1], next2 - 1, c + 3);
                     } else {  // chunk c + 2 -> its buffer
-                        int xidx = -1;
-                        if (TNI == 2) xidx = s == 0 && mi >= 2 ? (mi - 2) * 2 + ni : -1;
-                        if (TNI == 4 && TMI == 4) xidx = s == 0 && ni == 0 ? mi : -1;
-                        if (TMI == 16) xidx = ni == 2 && (mi & 1) == 1 && mi < 12 ? s * 6 + mi / 2 : -1;
-                        if (xidx >= 0 && xidx < NXP) load_x(xidx, dXc, nx2);
+                        if (ni == 2 && (mi & 1) == 1 && mi < 12) load_x(s * 6 + mi / 2, c + 2, dXc, nx2);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -560,6 +529,7 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
         // the MFMAs are opaque to the compiler's hazard tracking: any accumulator copy it places
         // at a control-flow join must find them retired
         asm volatile("s_nop 15" ::: "memory");
+        if (STAGED) lds_barrier();  // (a body's stores are for the next body but one, which begins to read them in the next)
         const uint32_t t = cur;
         cur = nxt;
         nxt = nx2;
@@ -654,6 +624,46 @@ __global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params 
     }
 }
 
+template <int TMI, int TNI, int EPI, bool BIAS>
+__global__ __launch_bounds__(256) void gemm_bf6_kernel(DUQ_HEAD_DECL, Bf6Params tail)
+{
+    using Tile = Bf6Tile<TMI, TNI, EPI>;
+    Bf6Params p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.X);
+    to_global(p.W);
+    to_global(p.y);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[Tile::kLds];
+    __shared__ __attribute__((aligned(16))) uint32_t dpar[EPI == 5 ? (Tile::BN + Tile::BM) * 8 : 4];
+    __shared__ uint32_t dwide;
+    uint32_t tile_m, tile_n;
+    tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    bf6_tile<TMI, TNI, EPI, BIAS>(p, lds, dpar, dwide, tile_m * Tile::BM, tile_n * Tile::BN);
+}
+
+// Rounds that do not come out even: p.tiles_m x p.tiles_n tiles of 256 rows, as many as fill whole rounds of 256 workgroups, and
+// behind them the columns that are left in tiles of REST * 16 rows (256 columns either way).
+template <int REST, int EPI, bool BIAS>
+__global__ __launch_bounds__(256) void gemm_bf6_mixed_kernel(DUQ_HEAD_DECL, Bf6Params tail)
+{
+    using Tile = Bf6Tile<16, 4, EPI>;
+    using Rest = Bf6Tile<REST, 4, EPI>;
+    Bf6Params p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.X);
+    to_global(p.W);
+    to_global(p.y);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[Tile::kLds];
+    uint32_t none = 0, tile_m, tile_n;
+    const uint32_t whole = p.tiles_m * p.tiles_n;
+    if (blockIdx.x < whole) {
+        tile_of_block(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+        bf6_tile<16, 4, EPI, BIAS>(p, lds, &none, none, tile_m * Tile::BM, tile_n * 256);
+    } else {
+        const uint32_t n1 = p.tiles_n * 256;
+        tile_of_block(blockIdx.x - whole, (p.M + Rest::BM - 1) / Rest::BM, (p.N - n1 + 255) / 256, tile_m, tile_n);
+        bf6_tile<REST, 4, EPI, BIAS>(p, lds, &none, none, tile_m * Rest::BM, n1 + tile_n * 256);
+    }
+}
+
 template <int TMI, int TNI, int EPI>
 static void launch_tile(const Bf6Params &p, hipStream_t stream)
 {
@@ -664,33 +674,69 @@ static void launch_tile(const Bf6Params &p, hipStream_t stream)
         DUQ_LAUNCH_HEAD((gemm_bf6_kernel<TMI, TNI, EPI, false>), grid, dim3(256), 0, stream, p);
 }
 
+template <int REST, int EPI>
+static void launch_mixed(const Bf6Params &p, hipStream_t stream)
+{
+    const dim3 grid(p.tiles_m * p.tiles_n + ((p.M + 16 * REST - 1) / (16 * REST)) * ((p.N + 255) / 256 - p.tiles_n));
+    if (p.epi.bias)
+        DUQ_LAUNCH_HEAD((gemm_bf6_mixed_kernel<REST, EPI, true>), grid, dim3(256), 0, stream, p);
+    else
+        DUQ_LAUNCH_HEAD((gemm_bf6_mixed_kernel<REST, EPI, false>), grid, dim3(256), 0, stream, p);
+}
+
+// Tile height: a round of 256 workgroups lasts about f + c * (K / 256) microseconds, measured (one round, K = 1024 / 4096 / 8192):
+// 64 x 256 8.0 / 17.5 / 30.5, 128 x 256 10.9 / 24 / 40.6, 256 x 256 18 / 38 / 65.5 (1.4 of it once per launch); the cheapest of uniform
+// tiles and, where the model has them 4 % ahead, whole rounds of 256 rows with the columns that are left in one round of smaller
+// tiles behind them, in the same launch (with the quantizer, first 5 ms of a load: 2048 x 11008 x 4096 70.7 -> 66.5 us, 1743 x
+// 9520 x 6528 104 -> 91.6, 1000 x 22016 x 4096 68.3 -> 62.6, 1500 x 13824 x 4096 68.2 -> 62.2).
+struct Bf6Plan {
+    uint32_t rows, cols = 0, rest = 0;  // cols > 0: columns of 256-row tiles, the others in tiles of `rest` rows
+};
+static Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
+{
+    const float n = (float)((K + 255) / 256);
+    const uint32_t rows[3] = {64, 128, 256}, tn = (N + 255) / 256;
+    const float cost[3] = {n * 0.79f + 3.6f, n * 1.06f + 5.1f, n * 1.69f + 9.5f};
+    auto tiles = [&](int k, uint32_t cols) { return (uint64_t)((M + rows[k] - 1) / rows[k]) * cols; };
+    auto rounds = [](uint64_t t) { return (float)((t + 255) / 256); };
+    Bf6Plan best{128};
+    float least = rounds(tiles(1, tn)) * cost[1];
+    if (rounds(tiles(0, tn)) * cost[0] < least) best.rows = 64, least = rounds(tiles(0, tn)) * cost[0];
+    if (mode5) return best;  // (the 256-row tile leaves no LDS for the staged parameters of epilogue 5)
+    if (rounds(tiles(2, tn)) * cost[2] < least) best.rows = 256, least = rounds(tiles(2, tn)) * cost[2];
+    least *= 0.96f;
+    // (whole rounds of 256 rows only: a round of 128-row tiles and one of 64-row tiles take longer than a round of 256-row ones;
+    // not for rows so short that the outputs are most of a tile's time: 2242 x 9872 x 640 31.9 -> 33.4 us)
+    const uint32_t whole = (uint32_t)(tiles(2, tn) / 256), cols = whole * 256 / ((M + 255) / 256);
+    if (whole == 0 || cols >= tn || n < 6.0f) return best;
+    for (int r = 0; r < 2; ++r) {
+        const float c = (float)whole * cost[2] + cost[r];
+        if (tiles(r, tn - cols) <= 256 && c < least) least = c, best = Bf6Plan{256, cols, rows[r]};
+    }
+    return best;
+}
+
 template <int EPI>
 static void launch_mode(Bf6Params &p, hipStream_t stream)
 {
-    // Tile height: whole rounds of 256 workgroups, with a 64-row / 256-row tile priced relative to a 128-row one
-    // (the weight traffic per tile is the same, the MFMAs are half / twice; measured on an MI355X).
-    constexpr float kCost64 = DUQ_BF6_COST64, kCost256 = DUQ_BF6_COST256;
-    const uint32_t t256 = ((p.M + 255) / 256) * p.tiles_n, t128 = ((p.M + 127) / 128) * p.tiles_n,
-                   t64 = ((p.M + 63) / 64) * p.tiles_n;
-    const float c256 = kCost256 * (float)((t256 + 255) / 256), c128 = (float)((t128 + 255) / 256),
-                c64 = kCost64 * (float)((t64 + 255) / 256);
-    // (the 256-row tile leaves no LDS for the staged parameters of epilogue 5)
-    if (EPI != 5 && c256 < c128 && c256 <= c64) {
-        p.tiles_m = (p.M + 255) / 256;
-        if constexpr (EPI != 5) launch_tile<16, 4, EPI>(p, stream);
-    } else if (c64 < c128) {
-        p.tiles_m = (p.M + 63) / 64;
-        // CUs left without a 64 x 256 tile: 64 x 128 tiles, twice as many, as long as they still run in one round
-        // (measured: 23-35 % faster up to 128 tiles of 64 x 256, slower from 160 on)
-        if (t64 <= DUQ_BF6_NARROW_MAX_TILES) {
-            p.tiles_n = (p.N + 127) / 128;
-            launch_tile<4, 2, EPI>(p, stream);
-        } else {
-            launch_tile<4, 4, EPI>(p, stream);
+    const Bf6Plan plan = plan_bf6(p.M, p.N, p.K, EPI == 5);
+    p.tiles_m = (p.M + plan.rows - 1) / plan.rows;
+    if constexpr (EPI != 5) {
+        if (plan.cols) {
+            p.tiles_n = plan.cols;
+            if (plan.rest == 128) return launch_mixed<8, EPI>(p, stream);
+            return launch_mixed<4, EPI>(p, stream);
         }
+        if (plan.rows == 256) return launch_tile<16, 4, EPI>(p, stream);
+    }
+    if (plan.rows == 128) return launch_tile<8, 4, EPI>(p, stream);
+    // CUs left without a 64 x 256 tile: 64 x 128 tiles, twice as many, as long as they still run in one round
+    // (measured: 23-35 % faster up to 128 tiles of 64 x 256, slower from 160 on)
+    if (p.tiles_m * p.tiles_n <= DUQ_BF6_NARROW_MAX_TILES) {
+        p.tiles_n = (p.N + 127) / 128;
+        launch_tile<4, 2, EPI>(p, stream);
     } else {
-        p.tiles_m = (p.M + 127) / 128;
-        launch_tile<8, 4, EPI>(p, stream);
+        launch_tile<4, 4, EPI>(p, stream);
     }
 }
 

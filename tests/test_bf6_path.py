@@ -245,6 +245,31 @@ def test_gpu_forward_bf6_equals_oracle(hip, dev, M, N, K, with_bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2048 - 30, 11008, 1408), (1000, 22016 - 16, 1408),     # 128-row tiles behind a round of 256-row ones
+                                   (1743, 9520, 1408), (4096 - 9, 4096 + 48, 1536)])        # 64-row tiles behind them
+def test_gpu_forward_bf6_uneven_rounds(hip, dev, M, N, K):
+    """Whole rounds of one kind of tile and the columns that are left in another; rows and columns that end inside either;
+    every epilogue that such a launch has."""
+    print("bf6 uneven rounds", M, N, K, flush=True)
+    rng = np.random.default_rng(M + 5 * N + K)
+    a, b = _rand_packed(rng, M, K), _rand_packed(rng, N, K)
+    sr, zr, sc1, zc1, sc2, zc2, bias = _epi_inputs(rng, M, N)
+    T = lambda v: cases.t(v, dev)
+    acc, xs, ws = orc.matmul_s4(a, b), hip.activation_shadow_bf6(T(a)), hip.weight_shadow_bf6(T(b))
+    got = hip.linear4bit_forward_bf6(hip.EPI_SYM, xs, T(sr), None, ws, T(sc1), bias=T(bias)).cpu().numpy()
+    assert cases.bits_equal(got, orc.add_bias(orc.sym_dequant(acc, sr, sc1), bias))
+    got = hip.linear4bit_forward_bf6(hip.EPI_SYM_DUAL, xs, T(sr), None, ws, T(sc1), None, T(sc2)).cpu().numpy()
+    assert cases.bits_equal(got, orc.sym_dual_dequant(acc, sr, sc1, sc2))
+    got = hip.linear4bit_forward_bf6(hip.EPI_ASYM, xs, T(sr), T(zr), ws, T(sc1), T(zc1)).cpu().numpy()
+    assert cases.bits_equal(got, orc.asym_dequant(acc, sr, zr, sc1, zc1))
+    got = hip.linear4bit_forward_bf6(hip.EPI_ASYM_DUAL, xs, T(sr), T(zr), ws, T(sc1), T(zc1), T(sc2), T(zc2), bias=T(bias)).cpu().numpy()
+    assert cases.bits_equal(got, orc.add_bias(orc.asym_dual_dequant(acc, sr, zr, sc1, zc1, sc2, zc2), bias))
+    rr, rc = rng.integers(-8 * K, 8 * K, M).astype(np.int32), rng.integers(-8 * K, 8 * K, N).astype(np.int32)
+    got = hip.linear4bit_forward_bf6(hip.EPI_ASYM_ROWSUM, xs, T(sr), T(zr), ws, T(sc1), T(zc1), rowsum_x=T(rr), w_rowsum_adj=T(rc)).cpu().numpy()
+    assert cases.bits_equal(got, orc.asym_rowsum_dequant(acc, sr, zr, rr, sc1, zc1, rc, None))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(4096 - 100, 4096, 640), (4096, 4096 - 16, 1152), (1000, 4096, 640), (1000, 4096, 1408), (500, 2048, 640),
                                    (500, 2048 - 80, 1152), (2048 - 9, 4096, 640), (2048, 4096, 1152)])
 def test_gpu_forward_bf6_chunks(hip, dev, M, N, K):
