@@ -32,8 +32,8 @@ using at::Tensor;
 PyObject *g_packed = nullptr;  // class PackedQuantizedTensor
 PyObject *g_check = nullptr;   // _lib.check(status, name): raises for a status other than 0
 // byte offsets of PackedQuantizedTensor's __slots__ in its instances
-enum Slot { kQ, kS, kZeros, kRowsum, kShadow, kSrc, kVersion, kClip, kQmax, kSlots };
-const char *const kSlotNames[kSlots] = {"_q", "_s", "zeros_x", "rowsum_x", "shadow_x", "_src", "_src_version", "_clip", "_qmax"};
+enum Slot { kQ, kS, kZeros, kRowsum, kShadow, kSrc, kVersion, kClip, kQmax, kStaged, kSlots };
+const char *const kSlotNames[kSlots] = {"_q", "_s", "zeros_x", "rowsum_x", "shadow_x", "_src", "_src_version", "_clip", "_qmax", "_staged"};
 Py_ssize_t g_offset[kSlots];
 
 inline PyObject *&slot(PyObject *packed, Slot s) { return *reinterpret_cast<PyObject **>(reinterpret_cast<char *>(packed) + g_offset[s]); }
@@ -213,8 +213,61 @@ bool still_current(FusedCall *c, PyObject *buffers)
     return true;
 }
 
-// min_tiles: the module's fp6_min_tiles, negative where the caller does not know it
-PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip, int qmax, int64_t min_tiles = -1)
+// What the first of several layers that take one deferred PackedQuantizedTensor leaves in it where it runs quantizer and GEMM as two
+// launches: the codes [M, K/2] and behind them the scales [M], in memory of the stream they were written on.  The next layers on
+// that stream run their GEMM alone (77 rows of 5120, two layers of 13824 columns: 29.6 -> 27.3 us, a third one 2.3 less again); on
+// another stream, or in another recording than the launch that writes them, a layer quantizes for itself.
+struct Staged {
+    PyObject_HEAD
+    c10::DataPtr *data;
+    int64_t rows, cols;
+    hipStream_t stream;
+    unsigned long long recording;  // id of the stream's recording, 0: none
+};
+PyTypeObject g_staged_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+int64_t staged_codes(int64_t M, int64_t K) { return (M * (K / 2) + 255) / 256 * 256; }
+
+// The recording that the stream is in, or false where it cannot be told.
+bool recording_of(hipStream_t stream, unsigned long long *id)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    *id = 0;
+    if (hipStreamGetCaptureInfo(stream, &status, id) != hipSuccess) {
+        (void)hipGetLastError();  // (not the launch's that follows)
+        return false;
+    }
+    if (status == hipStreamCaptureStatusInvalidated) return false;
+    if (status == hipStreamCaptureStatusNone) *id = 0;
+    return true;
+}
+
+PyObject *new_staged(c10::DataPtr &&data, int64_t M, int64_t K, hipStream_t stream, unsigned long long recording)
+{
+    Staged *o = reinterpret_cast<Staged *>(g_staged_type.tp_alloc(&g_staged_type, 0));
+    if (!o) return nullptr;
+    o->data = new c10::DataPtr(std::move(data));
+    o->rows = M;
+    o->cols = K;
+    o->stream = stream;
+    o->recording = recording;
+    return reinterpret_cast<PyObject *>(o);
+}
+
+void staged_dealloc(PyObject *self)
+{
+    delete reinterpret_cast<Staged *>(self)->data;
+    Py_TYPE(self)->tp_free(self);
+}
+
+// A copy or a saved file of the packed tensor goes without it.
+PyObject *staged_reduce(PyObject *, PyObject *) { return Py_BuildValue("(O())", reinterpret_cast<PyObject *>(Py_TYPE(Py_None))); }
+
+PyMethodDef g_staged_methods[] = {{"__reduce__", staged_reduce, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+
+// min_tiles: the module's fp6_min_tiles, negative where the caller does not know it.  packed: the deferred tensor that x is the rows
+// of, or null
+PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip, int qmax, int64_t min_tiles = -1, PyObject *packed = nullptr)
 {
     duq_fused_layer l = c->layer;
     if (x.dim() == 0 || x.size(-1) != static_cast<int64_t>(l.K) || x.get_device() != c->dev || l.K % 64) return none();
@@ -231,14 +284,53 @@ PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip,
     const int64_t bytes = staging_of(c, M);
     l.clip = clip;
     l.qmax = qmax;
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(c->dev)).stream();
+    const bool shares = packed && bytes > 0 && (l.mode == DUQ_EPI_SYM || l.mode == DUQ_EPI_SYM_DUAL);
+    unsigned long long recording = 0;
+    if (shares && recording_of(stream, &recording)) {
+        const int64_t at = staged_codes(M, l.K);
+        PyObject *s = slot(packed, kStaged);
+        if (s && Py_TYPE(s) == &g_staged_type) {
+            Staged *staged = reinterpret_cast<Staged *>(s);
+            if (staged->stream == stream && staged->recording == recording && staged->rows == M && staged->cols == static_cast<int64_t>(l.K)) {
+                const Held<1> h({s});  // (another thread may put something else there)
+                Tensor y = output(x, l.N, ScalarType::Half);
+                const uint8_t *q = static_cast<const uint8_t *>(staged->data->get());
+                int st;
+                {
+                    Unlocked u;
+                    st = duq_linear4bit_forward(l.mode, q, half(q + at), nullptr, l.w, l.w_scale_1, nullptr, l.w_scale_2, nullptr, l.bias,
+                                                static_cast<uint32_t>(M), l.N, l.K, out<duq_half>(y), stream);
+                }
+                if (st) return finish(st, "linear4bit_forward", nullptr);
+                return wrap(std::move(y));
+            }
+        }
+        Tensor y = output(x, l.N, ScalarType::Half);
+        Scratch ws(static_cast<uint64_t>(at + 2 * M));
+        uint8_t *q = static_cast<uint8_t *>(ws.get());
+        int st;
+        {
+            Unlocked u;
+            st = duq_quantize_linear4bit_forward(l.mode, half(x.const_data_ptr()), clip, qmax, l.w, l.w_scale_1, l.w_scale_2, l.bias,
+                                                 static_cast<uint32_t>(M), l.N, l.K, out<duq_half>(y), q, reinterpret_cast<duq_half *>(q + at),
+                                                 nullptr, 0, stream);
+        }
+        if (st) return finish(st, "quantize_linear4bit_forward", nullptr);
+        PyObject *left = new_staged(std::move(ws.data), M, l.K, stream, recording);
+        if (!left) return nullptr;
+        PyObject *before = slot(packed, kStaged);
+        slot(packed, kStaged) = left;
+        Py_XDECREF(before);
+        return wrap(std::move(y));
+    }
     Tensor y = output(x, l.N, ScalarType::Half);
     Scratch ws(static_cast<uint64_t>(bytes));
     int st;
     {
         Unlocked u;
         st = duq_quantize_linear4bit_forward_layer(&l, half(x.const_data_ptr()), static_cast<uint32_t>(M), out<duq_half>(y),
-                                                   ws.get(), static_cast<uint64_t>(bytes),
-                                                   c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(c->dev)).stream());
+                                                   ws.get(), static_cast<uint64_t>(bytes), stream);
     }
     if (st) return finish(st, "quantize_linear4bit_forward", nullptr);
     return wrap(std::move(y));
@@ -260,7 +352,7 @@ PyObject *fused_take(PyObject *self, PyObject *const *a, Py_ssize_t n)
     if (!x || x->is_inference() || x->_version() != whole(version) || !still_current(c, a[0])) return none();
     const Tensor held = *x;  // (another thread may quantize the packed tensor, which drops its rows)
     return guarded([&] { return run_rows(c, a[0], held, static_cast<float>(PyFloat_AS_DOUBLE(clip)), static_cast<int>(whole(qmax)),
-                                         tiles_argument(a, n)); });
+                                         tiles_argument(a, n), a[1]); });
 }
 
 // take_rows(buffers, x[, fp6_min_tiles]): the same for a layer with its own quantizer
@@ -351,7 +443,7 @@ PyObject *m_defer(PyObject *, PyObject *const *a, Py_ssize_t n)
     const Held<3> h({a[0], a[4], a[5]});   // (the allocation may run the garbage collector)
     PyObject *p = type->tp_alloc(type, 0);
     if (!p) return nullptr;
-    for (Slot s : {kQ, kS, kZeros, kRowsum, kShadow}) slot(p, s) = none();
+    for (Slot s : {kQ, kS, kZeros, kRowsum, kShadow, kStaged}) slot(p, s) = none();
     auto put = [&](Slot s, PyObject *v) {
         Py_INCREF(v);
         slot(p, s) = v;
@@ -1027,6 +1119,12 @@ PyMODINIT_FUNC PyInit__duq_host(void)
     g_fused_type.tp_dealloc = fused_dealloc;
     g_fused_type.tp_methods = g_fused_methods;
     if (PyType_Ready(&g_fused_type) < 0) return nullptr;
+    g_staged_type.tp_name = "_duq_host.Staged";
+    g_staged_type.tp_basicsize = sizeof(Staged);
+    g_staged_type.tp_flags = Py_TPFLAGS_DEFAULT;
+    g_staged_type.tp_dealloc = staged_dealloc;
+    g_staged_type.tp_methods = g_staged_methods;
+    if (PyType_Ready(&g_staged_type) < 0) return nullptr;
     g_module_call_type.tp_name = "_duq_host.ModuleCall";
     g_module_call_type.tp_basicsize = sizeof(ModuleCall);
     g_module_call_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL | Py_TPFLAGS_METHOD_DESCRIPTOR;

@@ -20,7 +20,8 @@ class PackedQuantizedTensor:
     launch consumes those directly, and ``quantized_x`` / ``scales_x`` are computed (one quantizer launch, the same
     bits) the first time anything reads them."""
 
-    __slots__ = ("_q", "_s", "zeros_x", "rowsum_x", "shadow_x", "_src", "_src_version", "_clip", "_qmax")
+    # (_staged: codes and scales that the first of several layers left for the others, csrc/duq_host.cpp)
+    __slots__ = ("_q", "_s", "zeros_x", "rowsum_x", "shadow_x", "_src", "_src_version", "_clip", "_qmax", "_staged")
 
     def __init__(self, quantized_x: torch.Tensor, scales_x: torch.Tensor, zeros_x: torch.Tensor = None,
                  rowsum_x: torch.Tensor = None, shadow_x: torch.Tensor = None):
@@ -32,14 +33,14 @@ class PackedQuantizedTensor:
         # set by a quantizer with shadow=True / "only": the same codes as 6-bit floats [..., 3K/4] for the
         # 6-bit float matrix path; with "only", quantized_x is None
         self.shadow_x = shadow_x
-        self._src = None
+        self._src = self._staged = None
 
     @classmethod
     def deferred(cls, x: torch.Tensor, clip: float, qmax: int):
         """The symmetric quantization of ``x`` (contiguous binary16 [..., K], K % 32 == 0, 16-byte aligned, no inference
         tensor), not yet computed."""
         self = cls.__new__(cls)
-        self._q = self._s = self.zeros_x = self.rowsum_x = self.shadow_x = None
+        self._q = self._s = self.zeros_x = self.rowsum_x = self.shadow_x = self._staged = None
         self._src = x
         self._src_version = x._version
         self._clip = clip
@@ -61,7 +62,7 @@ class PackedQuantizedTensor:
             self._q, self.shadow_x, self._s = quantize_sym_shadow(x, self._clip, self._qmax, shadow != "only")
         else:
             self._q, self._s = _ops.quantize_rows_sym(x, self._clip, self._qmax)
-        self._src = None
+        self._src = self._staged = None
 
     def materialize(self, shadow=False):
         """Quantize a deferred tensor now (no effect on one that is quantized already).  ``shadow``: True also
