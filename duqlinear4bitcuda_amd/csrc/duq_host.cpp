@@ -274,12 +274,16 @@ PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip,
     const int64_t M = x.numel() / l.K;
     if (M < 1 || M > c->max_rows || current_device() != c->dev) return none();
     // more than 64 rows of a layer with a 6-bit float shadow: those of the 6-bit float path are not run here (the rule
-    // of the layer's _fp6_wanted)
+    // of the layer's _fp6_pays)
     static PyObject *const shadow_name = PyUnicode_InternFromString("weight_shadow");
     if (M > 64) {
         PyObject *s = PyDict_GetItemWithError(buffers, shadow_name);
         const int64_t tiles = (M + 63) / 64 * ((l.N + 255) / 256);
-        if (s && s != Py_None && (min_tiles < 0 || tiles >= min_tiles || (M > 256 && 8 * tiles >= 5 * min_tiles))) return none();
+        const int64_t per = l.K >= 8192 ? 8 : l.K >= 2048 ? 10 : 20;
+        if (s && s != Py_None &&
+            (min_tiles < 0 || ((M > 1024 || l.K < 1024 || tiles / per >= min_tiles) &&
+                               (tiles >= min_tiles || (M > 256 && 8 * tiles >= 5 * min_tiles)))))
+            return none();
     }
     const int64_t bytes = staging_of(c, M);
     l.clip = clip;

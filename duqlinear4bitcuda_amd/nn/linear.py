@@ -220,8 +220,11 @@ class _Linear4bitBase(_MovesTogether):
     # 6-bit float matrix path (not in the reference): taken when the layer holds a weight shadow
     # (enable_fp6) and the input brings one, for more rows than the integer decode kernel takes (64 of up to 8192
     # elements, 48 of up to 12288, 32 beyond) and at least fp6_min_tiles output tiles of 64 x 256, or more than 256
-    # rows and 5/8 of that (below, the integer kernels' smaller tiles and the decode kernels do better; measured
-    # crossover on an MI355X)
+    # rows and 5/8 of that (below, the integer kernels' smaller tiles and the decode kernels do better).  Rows that the layer
+    # gets unquantized, up to 1024 of 1024 elements and more, which the integer kernels take in one library call: ten times as
+    # many tiles, twenty below 2048 elements, eight from 8192 on (_fp6_pays).  Eager steps of Linear4bitASQ, 6-bit float against integer, us: 160 x 4096 x 4096 25.4 / 11.8, 512 x 4096 x 8192
+    # 25.0 / 21.6, 768 x 4096 x 8192 26.9 / 29.2, 384 x 8192 x 8192 32.7 / 32.0, 512 x 8192 x 8192 33.9 / 35.0, 248 x 19968 x 17264 106 / 114, 1024 x 16384 x 4096 64.9 /
+    # 63.2, 512 x 1536 x 16384 25.3 / 19.0, 768 x 1536 x 16384 25.0 / 27.4
     fp6_min_tiles = 32
     _shadow_key = None
 
@@ -272,7 +275,7 @@ class _Linear4bitBase(_MovesTogether):
         M = x.numel() // K
         if d._one.get(M, -1) < 0 and not d.admits(M):
             return None
-        if M > 64 and self._fp6_wanted(M):  # large enough for the 6-bit float path, and the layer holds a shadow
+        if M > 64 and self._fp6_pays(M):  # large enough for the 6-bit float path, and the layer holds a shadow
             return None
         return d.run(x, M, clip, qmax, checked)
 
@@ -288,7 +291,7 @@ class _Linear4bitBase(_MovesTogether):
         if y is None:
             src = x._src
             rows = src.numel() // src.shape[-1]
-            x.materialize(shadow=bool(self.fused and src.shape[-1] % 128 == 0 and self._fp6_wanted(rows)))
+            x.materialize(shadow=bool(self.fused and src.shape[-1] % 128 == 0 and self._fp6_pays(rows)))
         return y
 
     def enable_fp6(self):
@@ -324,6 +327,13 @@ class _Linear4bitBase(_MovesTogether):
         return self._fp6_ready() and rows > decode_rows and \
             (tiles >= self.fp6_min_tiles or (rows > 256 and 8 * tiles >= 5 * self.fp6_min_tiles))
 
+    def _fp6_pays(self, rows):
+        """The same for rows that are not quantized yet."""
+        K = self.in_features
+        if rows <= 1024 <= K and -(-rows // 64) * -(-self.out_features // 256) < (8 if K >= 8192 else 10 if K >= 2048 else 20) * self.fp6_min_tiles:
+            return False
+        return self._fp6_wanted(rows)
+
     def _use_shadow(self, x):
         """The input's shadow is used when the layer is ready for it and the problem is large enough, or
         when the input brings nothing else."""
@@ -350,7 +360,7 @@ class _Linear4bitBase(_MovesTogether):
     def _quantize(self, x):
         """Own quantizer of the asymmetric layers: shadow only when this call will take the 6-bit float path."""
         rows = x.numel() // x.shape[-1]
-        return self.quantizer(x, shadow="only" if self._fp6_wanted(rows) else False)
+        return self.quantizer(x, shadow="only" if self._fp6_pays(rows) else False)
 
 
 @native_call("sym_layer")
@@ -564,7 +574,7 @@ class LinearQuant4bitDUASQRowSum(_Linear4bitBase):
                 return y
             # (the 6-bit float path of this layer reads the packed codes too: shadow and codes)
             rows = x.numel() // x.shape[-1]
-            x = self.quantizer(x, shadow=True if self.fused and self._fp6_wanted(rows) else False)
+            x = self.quantizer(x, shadow=True if self.fused and self._fp6_pays(rows) else False)
         assert type(x) == tensor_utils.PackedQuantizedTensor and x.rowsum_x is not None, \
             "Input should come from AsymQuantizer(shifted=True), or require_quantizer should be set"
         xq = x.quantized_x
