@@ -15,6 +15,7 @@
 //   scale: qlinear4bit/nn/quantizer.py:13, 27-31
 #include "duq_device.h"
 #include "duq_launch.h"
+#include "duq_epilogue.h"
 #include "duq_rowquant.h"
 #include "duq_tiles.h"
 
@@ -429,6 +430,38 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
     }
 }
 
+// LANES lanes hold a row, lane u0 of them its units u0, u0 + LANES, ...: the row's parameters and the codes of those units
+// (of units past its end: anything).
+template <int LANES, bool ASYM, bool UNIFORM, int NU>
+__device__ __forceinline__ void quantize_in_group(const v4u (&regs)[NU], uint32_t u0, uint32_t nunits, float clip, int qmax,
+                                                  RowQuant<ASYM, UNIFORM> &rq, uint32_t (&w)[NU])
+{
+    PkMinMax st;
+#pragma unroll
+    for (int j = 0; j < NU; ++j)
+        if (u0 + j * LANES < nunits) st.add8(regs[j]);
+    float a = 0.f, b = 0.f;
+    uint32_t m16;
+    if (!ASYM) {
+        m16 = group_reduce<LANES>(st.absmax_bits(), [](uint32_t x, uint32_t y) { return max(x, y); });
+    } else {
+        st.mx = group_reduce<LANES>(st.mx, [](uint32_t x, uint32_t y) {
+            asm("v_pk_maximum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
+            return x;
+        });
+        st.mn = group_reduce<LANES>(st.mn, [](uint32_t x, uint32_t y) {
+            asm("v_pk_minimum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
+            return x;
+        });
+        m16 = st.absmax_bits();
+        a = st.min_f32();
+        b = st.max_f32();
+        if (m16 > 0x7C00u) a = b = __builtin_nanf("");  // torch's min / max return NaN for a row that holds one
+    }
+    rq.init(m16, a, b, clip, qmax);
+    rq.quant_units(regs, w);
+}
+
 // Short rows (at most 512 elements, no shadow: the operands of quantized attention).  With a workgroup per row such a
 // launch is bound by how fast workgroups start (65536 rows of 128 elements, asymmetric: 21.4 us for 21 MB, a quarter of a workgroup's
 // lanes at work).  Here LANES lanes hold a row, two units each, and a workgroup takes 256 / LANES rows; the same launch takes
@@ -457,32 +490,9 @@ __global__ __launch_bounds__(256) void quantize_short_rows_kernel(DUQ_HEAD_DECL,
         const uint32_t u = u0 + j * LANES;
         regs[j] = row < p.rows && u < nunits ? __builtin_nontemporal_load(row_units<FORM>(p, row) + u) : v4u{0u, 0u, 0u, 0u};
     }
-    PkMinMax st;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-        if (u0 + j * LANES < nunits) st.add8(regs[j]);
-    float a = 0.f, b = 0.f;
-    uint32_t m16;
-    if (!ASYM) {
-        m16 = group_reduce<LANES>(st.absmax_bits(), [](uint32_t x, uint32_t y) { return max(x, y); });
-    } else {
-        st.mx = group_reduce<LANES>(st.mx, [](uint32_t x, uint32_t y) {
-            asm("v_pk_maximum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
-            return x;
-        });
-        st.mn = group_reduce<LANES>(st.mn, [](uint32_t x, uint32_t y) {
-            asm("v_pk_minimum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
-            return x;
-        });
-        m16 = st.absmax_bits();
-        a = st.min_f32();
-        b = st.max_f32();
-        if (m16 > 0x7C00u) a = b = __builtin_nanf("");  // torch's min / max return NaN for a row that holds one
-    }
     RowQuant<ASYM, false> rq;
-    rq.init(m16, a, b, p.clip, p.qmax);
     uint32_t w[2];
-    rq.quant_units(regs, w);
+    quantize_in_group<LANES>(regs, u0, nunits, p.clip, p.qmax, rq, w);
     if (shifted) {  // uniform branch: see quantize_rows_kernel
         uint32_t sum = 0;
 #pragma unroll
@@ -524,6 +534,111 @@ static int launch_short_rows(const RowParams &p, hipStream_t stream)
         DUQ_SHORT(32);
 #undef DUQ_SHORT
     return (int)hipGetLastError();
+}
+
+// Products with one row of A (one query per head), both operands in binary16: a row of B goes into a single output, so its codes
+// are multiplied where they are made.  LANES lanes hold a row of B, NU units each, and the codes of the same units of A's row,
+// which every workgroup quantizes for itself; a group of lanes takes `per` rows of B, the next one's units on their way while it
+// finishes one.  Instead of a launch that quantizes both operands and one that multiplies: 32 products of 1 x 2048 x 128 10.2 ->
+// 5.9 us, 32 of 1 x 128 x 2048 12.5 -> 5.9, 40 of 1 x 4096 x 128 16.0 -> 11.5 (3.7 TB/s), 8 of 1 x 192 x 64 8.7 -> 4.2, of which a launch
+// alone takes 4.  With four rows of A in the same way, 40 products of 4 x 4096 x 256 27.6 -> 30.5: one row only.
+struct ProductParams {
+    const uint16_t *a, *b;  // [batch, K], [batch, N, K]
+    uint16_t *y;            // [batch, N]
+    uint32_t N, K, per;
+    float clip_a;
+    int qmax_a;
+    float clip_b;
+    int qmax_b;
+    uint32_t reserved;
+};
+static_assert(sizeof(ProductParams) == kHeadBytes, "all fields delivered in registers");
+
+template <int LANES, int NU, bool ASYM>
+__global__ __launch_bounds__(256) void product_row_kernel(DUQ_HEAD_DECL, ProductParams tail)
+{
+    ProductParams p = with_head(tail, DUQ_HEAD_USE);
+    to_global(p.a);
+    to_global(p.b);
+    to_global(p.y);
+    constexpr uint32_t G = 256 / LANES;
+    const uint32_t nunits = p.K >> 3;  // <= NU * LANES
+    const uint32_t u0 = threadIdx.x % LANES;
+    const uint32_t first = blockIdx.x * (G * p.per), n0 = first + threadIdx.x / LANES;
+    const v4u *const a = reinterpret_cast<const v4u *>(p.a) + (uint64_t)blockIdx.y * nunits;
+    const v4u *const b = reinterpret_cast<const v4u *>(p.b) + (uint64_t)blockIdx.y * p.N * nunits;
+    uint16_t *const y = p.y + (uint64_t)blockIdx.y * p.N;
+    // (rows past N: the last one again, stored by nobody)
+    auto fetch = [&](uint32_t n, v4u(&r)[NU]) {
+        const v4u *const row = b + (uint64_t)min(n, p.N - 1) * nunits;
+#pragma unroll
+        for (int j = 0; j < NU; ++j)
+            r[j] = u0 + j * LANES < nunits ? __builtin_nontemporal_load(row + u0 + j * LANES) : v4u{0u, 0u, 0u, 0u};
+    };
+    v4u cur[NU];
+#pragma unroll
+    for (int j = 0; j < NU; ++j) cur[j] = u0 + j * LANES < nunits ? a[u0 + j * LANES] : v4u{0u, 0u, 0u, 0u};
+    v4u next[NU];
+    fetch(n0, next);
+    uint32_t wa[NU], wb[NU];
+    RowQuant<ASYM, LANES == 64> rq;
+    quantize_in_group<LANES>(cur, u0, nunits, p.clip_a, p.qmax_a, rq, wa);
+#pragma unroll
+    for (int j = 0; j < NU; ++j)
+        if (u0 + j * LANES >= nunits) wa[j] = 0;
+    const RowEpi ra{rq.s, rq.z, 0};
+    for (uint32_t i = 0; i < p.per && first + i * G < p.N; ++i) {
+        const uint32_t n = n0 + i * G;
+#pragma unroll
+        for (int j = 0; j < NU; ++j) cur[j] = next[j];
+        if (i + 1 < p.per) fetch(n + G, next);
+        quantize_in_group<LANES>(cur, u0, nunits, p.clip_b, p.qmax_b, rq, wb);
+        int acc = 0;
+#pragma unroll
+        for (int j = 0; j < NU; ++j) acc = __builtin_amdgcn_sdot8((int)wa[j], (int)wb[j], acc, false);
+        acc = (int)group_reduce<LANES>((uint32_t)acc, [](uint32_t x, uint32_t z) { return x + z; });
+        const uint16_t out = dequant_one<ASYM ? 1 : 0, false>(acc, ra, ColParams{rq.s, rq.z, (f16)0, 0});
+        if (u0 == 0 && n < p.N) y[n] = out;
+    }
+}
+
+// (rows of up to 4096 elements: a wavefront's registers)
+bool product_row_takes(uint32_t M, uint32_t K) { return M == 1 && K <= 4096; }
+
+template <bool ASYM>
+static void launch_product(ProductParams &p, uint32_t batch, hipStream_t stream)
+{
+    // Two rows of B per group of lanes where that leaves four workgroups a CU: A's row costs as much as one of B's (40 x 256 x 3392
+    // 19.2 -> 16.4 us, 40 x 4096 x 128 12.8 -> 11.5, 40 x 3392 x 256 18.1 -> 14.8; more than two: level, or 1 us behind)
+#define DUQ_PRODUCT(L, U)                                                                                                \
+    do {                                                                                                                 \
+        const uint64_t groups = ((uint64_t)p.N + 256 / L - 1) / (256 / L);                                               \
+        p.per = groups * batch >= 2048 ? 2 : 1;                                                                          \
+        DUQ_LAUNCH_HEAD((product_row_kernel<L, U, ASYM>), dim3((uint32_t)((groups + p.per - 1) / p.per), batch),         \
+                        dim3(256), 0, stream, p);                                                                        \
+    } while (0)
+    if (p.K <= 64) DUQ_PRODUCT(4, 2);
+    else if (p.K <= 128) DUQ_PRODUCT(8, 2);
+    else if (p.K <= 256) DUQ_PRODUCT(16, 2);
+    else if (p.K <= 512) DUQ_PRODUCT(32, 2);
+    else if (p.K <= 1024) DUQ_PRODUCT(64, 2);
+    else if (p.K <= 2048) DUQ_PRODUCT(64, 4);
+    else DUQ_PRODUCT(64, 8);
+#undef DUQ_PRODUCT
+}
+
+int launch_product_row(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t N, uint32_t K, float clip_a,
+                       int qmax_a, float clip_b, int qmax_b, uint16_t *y, hipStream_t stream)
+{
+    constexpr uint32_t kSlice = 65535;  // problems per launch: the grid's y
+    for (uint32_t b0 = 0; b0 < batch; b0 += kSlice) {
+        const uint32_t nb = std::min(batch - b0, kSlice);
+        ProductParams p{a + (uint64_t)b0 * K, b + (uint64_t)b0 * N * K, y + (uint64_t)b0 * N, N, K, 1, clip_a, qmax_a, clip_b, qmax_b, 0};
+        if (asym) launch_product<true>(p, nb, stream);
+        else launch_product<false>(p, nb, stream);
+        if (int e = (int)hipGetLastError()) return e;
+    }
+    return 0;
 }
 
 template <bool ASYM, int FORM>
