@@ -137,13 +137,6 @@ int launch_activation_shadow_bf6(const uint8_t *q, uint32_t M, uint32_t K, uint8
 // prefetches issued just before it (a full memory latency per chunk).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Cache policy of the output stores: 2 = non-temporal.  The output is written once and read by nobody in this
-// launch; streamed past the L2 it leaves the operand panels there and the launch ends sooner (measured at
-// M = 2048, N = K = 4096: 21.8 against 23.0 us; same bits).
-#ifndef DUQ_BF6_STORE_AUX
-#define DUQ_BF6_STORE_AUX 2
-#endif
-
 #ifndef DUQ_BF6_NARROW_MAX_TILES
 #define DUQ_BF6_NARROW_MAX_TILES 128
 #endif
@@ -615,13 +608,17 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
     constexpr uint32_t PPR = 2 * TNI, RPI = 64 / PPR;  // 16-byte pieces per staged row, rows per store instruction
     const uint32_t piece = lane % PPR, rsub = lane / PPR;
     const uint32_t ncol0 = n0 + wave * (16 * TNI) + piece * 8;
+    auto store_rows = [&](auto streamed) {
 #pragma unroll
-    for (int it = 0; it < BM / (int)RPI; ++it) {
-        const uint32_t row = it * RPI + rsub;
-        const v4u v = *reinterpret_cast<const v4u *>(stage + row * kYStride + piece * 16);
-        const uint32_t off = (row < rows_here && ncol0 < p.N) ? (row * p.N + ncol0) * 2 : kOobOffset;
-        __builtin_amdgcn_raw_buffer_store_b128(v, rY, (int)off, 0, DUQ_BF6_STORE_AUX);
-    }
+        for (int it = 0; it < BM / (int)RPI; ++it) {
+            const uint32_t row = it * RPI + rsub;
+            const v4u v = *reinterpret_cast<const v4u *>(stage + row * kYStride + piece * 16);
+            const uint32_t off = (row < rows_here && ncol0 < p.N) ? (row * p.N + ncol0) * 2 : kOobOffset;
+            __builtin_amdgcn_raw_buffer_store_b128(v, rY, (int)off, 0, decltype(streamed)::value ? 2 : 0);
+        }
+    };
+    if (streams_outputs(p.M, p.N)) store_rows(std::true_type{});
+    else store_rows(std::false_type{});
 }
 
 template <int TMI, int TNI, int EPI, bool BIAS>

@@ -5,13 +5,6 @@
 #include "duq_launch.h"
 #include "duq_tiles.h"
 
-// Cache policy of the output stores of the kernels that include duq_stream_epilogue_store.inc: 2 = non-temporal (the
-// output is written once and read by nobody in the launch; measured at M = 2048, N = K = 4096: 30.2 against 31.5 us,
-// M = 4096: 58.8 against 61.1)
-#ifndef DUQ_STREAM_STORE_AUX
-#define DUQ_STREAM_STORE_AUX 2
-#endif
-
 namespace duq {
 
 constexpr uint32_t kNibbleMask = 0xF0F0F0F0u;

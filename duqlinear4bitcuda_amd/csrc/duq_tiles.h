@@ -43,6 +43,14 @@ __device__ __forceinline__ v4u buf_load16_aux(__amdgpu_buffer_rsrc_t r, uint32_t
     return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, AUX));
 }
 
+// Binary16 outputs of prefill-sized launches (rows of y 16-byte aligned): stored past the L2 (non-temporal) or into it.  What fits
+// in the eight L2s, 32 MB, is still there when the last workgroup ends and would be written back only then, and rows that are whole
+// cache lines leave as whole lines either way: streamed (integer kernel 2048 x 4096 x 4096 30.5 us against 31.5, 2048 x 4096 x 1024
+// 12.6 / 14.0, 2461 x 28288 x 768 75.6 / 77.2; 6-bit floats 23.8 / 25.6, 10.3 / 12.0, 62.6 / 66.2).  Larger outputs of other widths:
+// the pieces of a line that come from different workgroups meet in the L2, if they stop there (integer kernel 2461 x 28336 x 768 92.2
+// -> 78.4, 4078 x 13360 x 832 91.7 -> 82.2, 1999 x 11024 x 4096 80.0 -> 74.0; 6-bit floats 80.3 -> 67.8, 61.6 -> 53.9, 59.2 -> 56.2).
+__device__ __forceinline__ bool streams_outputs(uint32_t M, uint32_t N) { return N % 64 == 0 || (uint64_t)M * N <= (16u << 20); }
+
 // Stages of the LDS kernels (duq_decode.hip, duq_int8.hip): MT row tiles and NT column tiles of 16 per workgroup of eight
 // wavefronts.
 template <int MT, int NT>
