@@ -227,7 +227,7 @@ struct Bf6Params {
 };
 static_assert(offsetof(Bf6Params, epi) + 8 == kHeadBytes, "the fields delivered in registers");
 
-// TMI = 8: 128-row tiles.  TMI = 4: 64-row tiles for problems that would leave most CUs without a 128-row tile
+// TMI = 8: 128-row tiles (6: 96).  TMI = 4: 64-row tiles for problems that would leave most CUs without a 128-row tile
 // (half the MFMAs for the same weight traffic, but twice the workgroups).  TMI = 16: 256-row tiles for problems
 // with at least one such tile per CU: the same weight traffic feeds twice the MFMAs, which takes the kernel off
 // the L2 -> CU limit that bounds the smaller tiles; all 256 AGPRs hold accumulators, an activation chunk is one
@@ -235,7 +235,7 @@ static_assert(offsetof(Bf6Params, epi) + 8 == kHeadBytes, "the fields delivered 
 template <int TMI, int TNI, int EPI>
 struct Bf6Tile {
     static constexpr int BM = 16 * TMI, BN = 64 * TNI;
-    static constexpr uint32_t kBuf = BM * 192;             // a chunk of 256 k: BM rows of 128 bytes (plane 0), then of 64 (plane 1)
+    static constexpr uint32_t kBuf = BM * 128 + (BM + 63) / 64 * 4096;  // a chunk of 256 k: BM rows of 128 bytes (plane 0), then of 64 (plane 1), in loads of 64 rows
     static constexpr uint32_t kYStride = 32 * TNI + 16;    // bytes per staged output row: 16*TNI binary16 + pad
     static constexpr uint32_t kLds = 3 * kBuf > 4 * BM * kYStride ? 3 * kBuf : 4 * BM * kYStride;
 };
@@ -244,14 +244,14 @@ struct Bf6Tile {
 template <int TMI, int TNI, int EPI, bool BIAS>
 __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint32_t *dpar, uint32_t &dwide, const uint32_t m0, const uint32_t n0)
 {
-    static_assert(TMI == 16 || TMI == 8 || TMI == 4, "16-row MFMA tiles per wavefront along M");
+    static_assert(TMI == 16 || TMI == 8 || TMI == 6 || TMI == 4, "16-row MFMA tiles per wavefront along M");
     // TNI = 16 x 16 MFMA tiles per wavefront along N: BM rows x 64 columns (TNI = 4), or BM x 32 (TNI = 2, with
     // 64-row tiles only: twice the workgroups for problems that leave CUs without a 64 x 256 tile)
     static_assert(TNI == 4 || (TNI == 2 && TMI == 4), "column tiles per wavefront");
     using Tile = Bf6Tile<TMI, TNI, EPI>;
     constexpr int BM = Tile::BM, BN = Tile::BN;
     constexpr int CH = 2;                                   // 128-k steps per activation chunk
-    constexpr int NXA = TMI / 2, NXB = TMI / 4, NXP = NXA + NXB;  // activation loads per wavefront and chunk, a kilobyte each
+    constexpr int NXA = TMI / 2, NXB = (TMI + 3) / 4, NXP = NXA + NXB;  // activation loads per wavefront and chunk, a kilobyte each
     constexpr uint32_t kP1Base = BM * 128, kBuf = Tile::kBuf, kYStride = Tile::kYStride;
     // The 256-row tile's activations go to LDS directly, those of the others through registers (see the kernel's head).
     constexpr bool STAGED = TMI != 16;
@@ -482,7 +482,7 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
                     // The operands are written by loads only (the compiler waits for those).  A register move
                     // placed right in front of this opaque statement would need wait states the compiler
                     // cannot know of; the generated loop has none, and the bit-exact parity tests would show one.
-                    mfma_pinned<kRingBase>(slot * NP + ni / 2, ni & 1, acc[mi][ni], wf[slot][ni / 2], xf[mi & 3]);
+                    mfma_pinned<kRingBase>(slot * NP + ni / 2, ni & 1, acc[mi][ni], wf[slot][ni / 2], xf[(s * TMI + mi) & 3]);
                     __builtin_amdgcn_sched_barrier(0);
                     if (!STAGED && s == CH - 1 && mi == TMI - 2 && ni == 0) {
                         // The next chunk is read from here on: its loads, issued before those of this body, have to be there.
@@ -492,24 +492,24 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
                     }
                     // ---- side work in the shadow of this MFMA
                     if (ni < 2) {  // activation fragment two groups ahead
-                        const int nm = (mi + 2) & (TMI - 1), ns = mi + 2 < TMI ? s : s + 1;
+                        const int nm = (mi + 2) % TMI, ns = mi + 2 < TMI ? s : s + 1, nf = (s * TMI + mi + 2) & 3;  // (CH * TMI is a multiple of 4)
                         const uint32_t buf = ns < CH ? cur : nxt;
                         if (ni == 0)
-                            read_x0(xf[nm & 3], buf, nm, ns % CH);
+                            read_x0(xf[nf], buf, nm, ns % CH);
                         else
-                            read_x1(xf[nm & 3], buf, nm, ns % CH);
+                            read_x1(xf[nf], buf, nm, ns % CH);
                     }
                     // refill the previous step's slot: 3 * NP loads over the step
                     {
                         int widx = -1;  // which of the 3 * NP loads rides with this MFMA
                         if (TNI == 2) widx = mi < 2 ? mi * 2 + ni : -1;
-                        if (TNI == 4 && TMI == 8) widx = ni == 2 ? mi : -1;
+                        if (TNI == 4 && (TMI == 8 || TMI == 6)) widx = ni == 2 ? mi : -1;
                         if (TNI == 4 && TMI == 4) widx = ni >= 2 ? mi * 2 + (ni - 2) : -1;
                         if (TNI == 4 && TMI == 16) widx = (ni == 2 && (mi & 1) == 0) ? mi / 2 : -1;
                         if (widx >= 0 && widx < 3 * NP) load_w(wf[prev][widx / 3], widx / 3, widx % 3, gprev, rG);
                     }
                     if constexpr (STAGED) {  // chunk c + 2 -> its buffer and, one group later, chunk c + 3 into the freed register
-                        const int slot2 = TNI == 2 ? (mi - 2) * 2 + ni : ni == (TMI == 8 ? 3 : 0) ? mi : -1, next2 = TNI == 2 ? slot2 : ni == 1 ? mi : 0;
+                        const int slot2 = TNI == 2 ? (mi - 2) * 2 + ni : ni == (TMI >= 6 ? 3 : 0) ? mi : -1, next2 = TNI == 2 ? slot2 : ni == 1 ? mi : 0;
                         if (s == 1 && slot2 >= 0 && slot2 < NXP) store_x(xreg[slot2], slot2, nx2);
                         if (s == 1 && next2 >= 1 && next2 <= NXP) fetch_x(xreg[next2 - 1], next2 - 1, c + 3);
                     } else {  // chunk c + 2 -> its buffer
@@ -682,32 +682,41 @@ static void launch_mixed(const Bf6Params &p, hipStream_t stream)
 }
 
 // Tile height: a round of 256 workgroups lasts about f + c * (K / 256) microseconds, measured (one round, K = 1024 / 4096 / 8192):
-// 64 x 256 8.0 / 17.5 / 30.5, 128 x 256 10.9 / 24 / 40.6, 256 x 256 18 / 38 / 65.5 (1.4 of it once per launch); the cheapest of uniform
+// 64 x 256 8.0 / 17.5 / 30.5, 96 x 256 9.7 / 20.2 / 35.7, 128 x 256 10.9 / 24 / 40.6, 256 x 256 18 / 38 / 65.5 (1.4 of it once per launch); the cheapest of uniform
 // tiles and, where the model has them 4 % ahead, whole rounds of 256 rows with the columns that are left in one round of smaller
 // tiles behind them, in the same launch (with the quantizer, first 5 ms of a load: 2048 x 11008 x 4096 70.7 -> 66.5 us, 1743 x
-// 9520 x 6528 104 -> 91.6, 1000 x 22016 x 4096 68.3 -> 62.6, 1500 x 13824 x 4096 68.2 -> 62.2).
+// 9520 x 6528 104 -> 91.6, 1000 x 22016 x 4096 68.3 -> 62.6, 1500 x 13824 x 4096 68.2 -> 62.2).  The 96-row tile is for what needs a
+// round and a bit of 64-row tiles and leaves half the CUs without a 128-row one (GEMM alone: 2894 x 1536 x 3840 22.8 -> 20.1, 1957 x
+// 2256 x 19968 87.5 -> 78.9, 3000 x 2048 x 2048 14.0 -> 12.4; with epilogue 5 1536 x 4096 x 4096 32.1 -> 27.8).
 struct Bf6Plan {
     uint32_t rows, cols = 0, rest = 0;  // cols > 0: columns of 256-row tiles, the others in tiles of `rest` rows
 };
 static Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
 {
     const float n = (float)((K + 255) / 256);
-    const uint32_t rows[3] = {64, 128, 256}, tn = (N + 255) / 256;
-    const float cost[3] = {n * 0.79f + 3.6f, n * 1.06f + 5.1f, n * 1.69f + 9.5f};
+    const uint32_t rows[4] = {64, 96, 128, 256}, tn = (N + 255) / 256;
+    const float cost[4] = {n * 0.79f + 3.6f, n * 0.93f + 4.4f, n * 1.06f + 5.1f, n * 1.69f + 9.5f};
     auto tiles = [&](int k, uint32_t cols) { return (uint64_t)((M + rows[k] - 1) / rows[k]) * cols; };
     auto rounds = [](uint64_t t) { return (float)((t + 255) / 256); };
     Bf6Plan best{128};
-    float least = rounds(tiles(1, tn)) * cost[1];
-    if (rounds(tiles(0, tn)) * cost[0] < least) best.rows = 64, least = rounds(tiles(0, tn)) * cost[0];
-    if (mode5) return best;  // (the 256-row tile leaves no LDS for the staged parameters of epilogue 5)
-    if (rounds(tiles(2, tn)) * cost[2] < least) best.rows = 256, least = rounds(tiles(2, tn)) * cost[2];
+    float least = rounds(tiles(2, tn)) * cost[2];
+    const int order[3] = {0, 1, 3};
+    for (int k : order) {
+        if (k == 3 && mode5) continue;  // (the 256-row tile leaves no LDS for the staged parameters of epilogue 5)
+        // (as many tiles of 96 rows as of 128, and weights beyond the last-level cache, whose rate decides: 185 x 24464 x 26496 147
+        // us with 128 rows, 157 with 96, 180 x 28672 x 20480 110 / 115; but 185 x 24464 x 12800 63.8 / 49.0)
+        if (k == 1 && tiles(1, tn) == tiles(2, tn) && (uint64_t)N * K * 3 / 4 > (256u << 20)) continue;
+        const float c = rounds(tiles(k, tn)) * cost[k];
+        if (c < least) best.rows = rows[k], least = c;
+    }
+    if (mode5) return best;
     least *= 0.96f;
     // (whole rounds of 256 rows only: a round of 128-row tiles and one of 64-row tiles take longer than a round of 256-row ones;
     // not for rows so short that the outputs are most of a tile's time: 2242 x 9872 x 640 31.9 -> 33.4 us)
-    const uint32_t whole = (uint32_t)(tiles(2, tn) / 256), cols = whole * 256 / ((M + 255) / 256);
+    const uint32_t whole = (uint32_t)(tiles(3, tn) / 256), cols = whole * 256 / ((M + 255) / 256);
     if (whole == 0 || cols >= tn || n < 6.0f) return best;
-    for (int r = 0; r < 2; ++r) {
-        const float c = (float)whole * cost[2] + cost[r];
+    for (int r = 0; r < 3; ++r) {
+        const float c = (float)whole * cost[3] + cost[r];
         if (tiles(r, tn - cols) <= 256 && c < least) least = c, best = Bf6Plan{256, cols, rows[r]};
     }
     return best;
@@ -722,11 +731,13 @@ static void launch_mode(Bf6Params &p, hipStream_t stream)
         if (plan.cols) {
             p.tiles_n = plan.cols;
             if (plan.rest == 128) return launch_mixed<8, EPI>(p, stream);
+            if (plan.rest == 96) return launch_mixed<6, EPI>(p, stream);
             return launch_mixed<4, EPI>(p, stream);
         }
         if (plan.rows == 256) return launch_tile<16, 4, EPI>(p, stream);
     }
     if (plan.rows == 128) return launch_tile<8, 4, EPI>(p, stream);
+    if (plan.rows == 96) return launch_tile<6, 4, EPI>(p, stream);
     // CUs left without a 64 x 256 tile: 64 x 128 tiles, twice as many, as long as they still run in one round
     // (measured: 23-35 % faster up to 128 tiles of 64 x 256, slower from 160 on)
     if (p.tiles_m * p.tiles_n <= DUQ_BF6_NARROW_MAX_TILES) {

@@ -270,6 +270,28 @@ def test_gpu_forward_bf6_uneven_rounds(hip, dev, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1500, 4096, 640), (1441, 4096 - 16, 1152), (1536, 4096, 128),  # 96-row tiles
+                                   (2048, 11520, 1408)])   # the other tests' rests are in 64- and 96-row tiles: 128 rows behind 256
+def test_gpu_forward_bf6_96_rows(hip, dev, M, N, K):
+    test_gpu_forward_bf6_uneven_rounds(hip, dev, M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1441, 1536])
+def test_gpu_96_rows_dual_rowsum(dev, M):
+    """The dual-uniform row-sum epilogue on 96-row tiles, against the integer kernels."""
+    import torch
+    from duqlinear4bitcuda_amd import nn as qnn
+    print("bf6 96 rows, dual row sums", M, flush=True)
+    K, N = 640, 4096 - 16
+    g = torch.Generator(device=dev).manual_seed(M)
+    lin = torch.nn.Linear(K, N, device=dev, dtype=torch.float16).requires_grad_(False)
+    x = torch.rand(M, K, generator=g, device=dev).half() * 6
+    plain, fp6 = (qnn.LinearQuant4bitDUASQRowSum.from_linear(lin).to(dev) for _ in range(2))
+    assert torch.equal(fp6.enable_fp6()(x), plain(x))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(4096 - 100, 4096, 640), (4096, 4096 - 16, 1152), (1000, 4096, 640), (1000, 4096, 1408), (500, 2048, 640),
                                    (500, 2048 - 80, 1152), (2048 - 9, 4096, 640), (2048, 4096, 1152)])
 def test_gpu_forward_bf6_chunks(hip, dev, M, N, K):
