@@ -708,13 +708,20 @@ struct Names {
     NAME(transpose_B);
     NAME(weight);
     NAME(weight_tiled);
+    NAME(weight_shadow);
     NAME(weight_scales);
+    NAME(weight_scales_1);
+    NAME(weight_scales_2);
     NAME(weight_zeros);
     NAME(bias);
     NAME(_tiled_key);
+    NAME(_shadow_key);
+    NAME(only);
     NAME(_launch);
     NAME(duq_quantize_linear8bit_forward);
     NAME(duq_quantize_product);
+    NAME(duq_quantize_rows_sym_bf6);
+    NAME(duq_linear4bit_forward_bf6);
     NAME(__call__);
 #undef NAME
 };
@@ -788,12 +795,80 @@ PyObject *call_sym_quantizer(PyObject *self, PyObject *dict, PyObject *x)
                       get(dict, n.qmax)};
     for (PyObject *v : a)
         if (!v) return none();
-    return m_defer(nullptr, a, 6);
+    PyObject *p = m_defer(nullptr, a, 6);
+    if (p != Py_None || a[2] == Py_False) return p;
+    // a quantizer set to write the 6-bit float shadow (True: beside the codes, "only": alone), rows enough for it
+    const bool codes = a[2] == Py_True;
+    const Tensor *t = plain(x, ScalarType::Half, -1);
+    if (!t || t->dim() == 0 || !(codes || (PyUnicode_CheckExact(a[2]) && PyUnicode_Compare(a[2], n.only) == 0)) || !PyLong_Check(a[3]) ||
+        !PyFloat_Check(a[4]) || !PyLong_Check(a[5]) || get(g_ops_dict, n._launch) != g_launch || !library_function(n.duq_quantize_rows_sym_bf6))
+        return p;
+    const int64_t K = t->size(-1), numel = t->numel();
+    if (K % 128 || numel <= 0 || numel / K < whole(a[3]) || numel / K > UINT32_MAX || K > UINT32_MAX ||
+        reinterpret_cast<uintptr_t>(t->const_data_ptr()) % 16 || t->get_device() != current_device())
+        return p;
+    Py_DECREF(p);
+    return guarded([&]() -> PyObject * {
+        const Held<1> h({x});
+        const float clip = static_cast<float>(PyFloat_AS_DOUBLE(a[4]));
+        const int qmax = static_cast<int>(whole(a[5]));
+        Tensor q, b = output(*t, K * 3 / 4, ScalarType::Byte), s = output(*t, 1, ScalarType::Half);
+        if (codes) q = output(*t, K / 2, ScalarType::Byte);
+        const hipStream_t st = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(t->get_device())).stream();
+        int e;
+        {
+            Unlocked u;
+            e = duq_quantize_rows_sym_bf6(half(t->const_data_ptr()), static_cast<uint32_t>(numel / K), static_cast<uint32_t>(K), clip, qmax,
+                                          out<uint8_t>(q), out<uint8_t>(b), out<duq_half>(s), st);
+        }
+        if (e) return finish(e, "quantize_rows_sym_bf6", nullptr);
+        PyTypeObject *type = reinterpret_cast<PyTypeObject *>(g_packed);
+        PyObject *packed = type->tp_alloc(type, 0);
+        if (!packed) return nullptr;
+        for (Slot i : {kZeros, kRowsum, kSrc, kStaged}) slot(packed, i) = none();
+        slot(packed, kQ) = codes ? wrap(std::move(q)) : none();
+        slot(packed, kS) = wrap(std::move(s));
+        slot(packed, kShadow) = wrap(std::move(b));
+        return packed;
+    });
+}
+
+// A symmetric layer whose input is a 6-bit float shadow alone (the rule for one that comes with codes: the layer's _use_shadow).
+PyObject *call_layer_on_shadow(PyObject *self, PyObject *dict, PyObject *packed)
+{
+    const Names &n = *g_names;
+    PyObject *q = slot(packed, kQ), *src = slot(packed, kSrc), *shadow = slot(packed, kShadow), *scales = slot(packed, kS);
+    PyObject *buffers = get(dict, n._buffers), *key = get(dict, n._shadow_key);
+    if (q != Py_None || src != Py_None || !shadow || !scales || !buffers || !key || !PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 ||
+        attr(self, dict, n.fused) != Py_True || get(g_ops_dict, n._launch) != g_launch || !library_function(n.duq_linear4bit_forward_bf6))
+        return none();
+    PyObject *w = get(buffers, n.weight), *ws = get(buffers, n.weight_shadow), *s1 = get(buffers, n.weight_scales), *s2 = Py_None;
+    const bool dual = !s1;
+    if (dual) s1 = get(buffers, n.weight_scales_1), s2 = get(buffers, n.weight_scales_2);
+    PyObject *bias = get(buffers, n.bias);
+    if (!bias) bias = get(dict, n.bias) == Py_None ? Py_None : nullptr;
+    if (!w || !ws || !s1 || !s2 || !bias) return none();
+    const Tensor *pw = plain(w, ScalarType::Byte, -1), *px = plain(shadow, ScalarType::Byte, -1);
+    // the shadow is the weight's as it is now: version, address, device (the layer's _fp6_ready)
+    if (!pw || !px || pw->is_inference() || !THPVariable_CheckExact(ws) || THPVariable_Unpack(ws).get_device() != pw->get_device() ||
+        whole(PyTuple_GET_ITEM(key, 0)) != pw->_version() || PyLong_AsVoidPtr(PyTuple_GET_ITEM(key, 1)) != pw->const_data_ptr() ||
+        px->get_device() != current_device()) {
+        PyErr_Clear();
+        return none();
+    }
+    static PyObject *const modes[2] = {PyLong_FromLong(DUQ_EPI_SYM), PyLong_FromLong(DUQ_EPI_SYM_DUAL)};
+    PyObject *st = PyLong_FromVoidPtr(c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(px->get_device())).stream());
+    if (!st) return nullptr;
+    const Held<14> a({modes[dual], shadow, scales, Py_None, ws, s1, Py_None, s2, Py_None, bias, Py_None, Py_None, Py_True, st});
+    Py_DECREF(st);
+    return m_linear4(nullptr, a.o, 14);
 }
 
 PyObject *call_layer(PyObject *self, PyObject *dict, PyObject *x, bool own_quantizer)
 {
     const Names &n = *g_names;
+    if (!own_quantizer && reinterpret_cast<PyObject *>(Py_TYPE(x)) == g_packed && slot(x, kQ) == Py_None && slot(x, kSrc) == Py_None)
+        return call_layer_on_shadow(self, dict, x);
     PyObject *decode = get(dict, n._decode), *buffers = get(dict, n._buffers);
     if (!decode || decode == Py_None || !buffers || attr(self, dict, n.fused) != Py_True) return none();
     if (own_quantizer && get(dict, n.require_quantizer) != Py_True) return none();
