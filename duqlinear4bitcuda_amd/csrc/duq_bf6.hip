@@ -695,7 +695,7 @@ static Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
 {
     const float n = (float)((K + 255) / 256);
     const uint32_t rows[4] = {64, 96, 128, 256}, tn = (N + 255) / 256;
-    const float cost[4] = {n * 0.79f + 3.6f, n * 0.93f + 4.4f, n * 1.06f + 5.1f, n * 1.69f + 9.5f};
+    const float cost[4] = {n * 0.79f + 3.6f, n * 0.93f + 4.4f, n * 1.06f + 5.1f, n * 1.69f + 9.9f};
     auto tiles = [&](int k, uint32_t cols) { return (uint64_t)((M + rows[k] - 1) / rows[k]) * cols; };
     auto rounds = [](uint64_t t) { return (float)((t + 255) / 256); };
     Bf6Plan best{128};
@@ -703,6 +703,9 @@ static Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
     const int order[3] = {0, 1, 3};
     for (int k : order) {
         if (k == 3 && mode5) continue;  // (the 256-row tile leaves no LDS for the staged parameters of epilogue 5)
+        // (several rounds of short rows are their outputs, and the model's differences are small: 1410 x 10928 x 768 18.8 us with
+        // 64 rows, 21.1 with 96)
+        if (k == 1 && n < 6.0f && tiles(1, tn) > 256) continue;
         // (as many tiles of 96 rows as of 128, and weights beyond the last-level cache, whose rate decides: 185 x 24464 x 26496 147
         // us with 128 rows, 157 with 96, 180 x 28672 x 20480 110 / 115; but 185 x 24464 x 12800 63.8 / 49.0)
         if (k == 1 && tiles(1, tn) == tiles(2, tn) && (uint64_t)N * K * 3 / 4 > (256u << 20)) continue;
