@@ -431,7 +431,7 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
     if (!aligned(workspace, 16)) return DUQ_E_ALIGN;
     if (workspace_bytes < duq_quantize_product_workspace_bytes(mode, batch_count, M, N, K)) return DUQ_E_SHAPE;
     const bool asym = mode == DUQ_EPI_ASYM;
-    if (duq::product_row_takes(M, K))
+    if (duq::product_row_takes(M, N, K))
         return duq::launch_product_row(asym, a, b, batch_count, N, K, clip_a, qmax_a, clip_b, qmax_b, y, as_stream(stream));
     uint8_t *q = static_cast<uint8_t *>(workspace);
     duq_half *s = reinterpret_cast<duq_half *>(q + up16(rows * (K / 2)));

@@ -28,7 +28,7 @@ int launch_quantize_rows_asym(const uint16_t *x, uint32_t rows, uint32_t cols, u
 int launch_quantize_two(const uint16_t *x, uint32_t rows, const uint16_t *x2, uint32_t rows2, uint32_t cols, bool asym, float clip,
                         int qmax, uint8_t *q, uint16_t *scale, uint16_t *zeros, hipStream_t stream);
 // A product with one row of A per problem in one launch, without packed operands: the shapes of product_row_takes.  N > 0, K > 0.
-bool product_row_takes(uint32_t M, uint32_t K);
+bool product_row_takes(uint32_t M, uint32_t N, uint32_t K);
 int launch_product_row(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t N, uint32_t K, float clip_a,
                        int qmax_a, float clip_b, int qmax_b, uint16_t *y, hipStream_t stream);
 

@@ -602,8 +602,8 @@ __global__ __launch_bounds__(256) void product_row_kernel(DUQ_HEAD_DECL, Product
     }
 }
 
-// (rows of up to 4096 elements: a wavefront's registers)
-bool product_row_takes(uint32_t M, uint32_t K) { return M == 1 && K <= 4096; }
+// (rows of up to 4096 elements: a wavefront's registers; a launch has less than 2^32 threads in a dimension)
+bool product_row_takes(uint32_t M, uint32_t N, uint32_t K) { return M == 1 && N <= 1u << 24 && K <= 4096; }
 
 template <bool ASYM>
 static void launch_product(ProductParams &p, uint32_t batch, hipStream_t stream)
