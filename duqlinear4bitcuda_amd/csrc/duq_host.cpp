@@ -216,10 +216,13 @@ bool still_current(FusedCall *c, PyObject *buffers)
 // What the first of several layers that take one deferred PackedQuantizedTensor leaves in it where it runs quantizer and GEMM as two
 // launches: the codes [M, K/2] and behind them the scales [M], in memory of the stream they were written on.  The next layers on
 // that stream run their GEMM alone (77 rows of 5120, two layers of 13824 columns: 29.6 -> 27.3 us, a third one 2.3 less again); on
-// another stream, or in another recording than the launch that writes them, a layer quantizes for itself.
+// another stream, in another recording than the launch that writes them, or where the tensor of rows was given other memory since (an
+// assignment to its .data), a layer quantizes for itself.  The rows' storage is kept, so that no other rows can come to lie at its address.
 struct Staged {
     PyObject_HEAD
-    c10::DataPtr *data;
+    c10::DataPtr data;
+    c10::Storage storage;  // of the rows
+    const void *at;        // the first row
     int64_t rows, cols;
     hipStream_t stream;
     unsigned long long recording;  // id of the stream's recording, 0: none
@@ -242,11 +245,13 @@ bool recording_of(hipStream_t stream, unsigned long long *id)
     return true;
 }
 
-PyObject *new_staged(c10::DataPtr &&data, int64_t M, int64_t K, hipStream_t stream, unsigned long long recording)
+PyObject *new_staged(c10::DataPtr &&data, const Tensor &x, int64_t M, int64_t K, hipStream_t stream, unsigned long long recording)
 {
     Staged *o = reinterpret_cast<Staged *>(g_staged_type.tp_alloc(&g_staged_type, 0));
     if (!o) return nullptr;
-    o->data = new c10::DataPtr(std::move(data));
+    new (&o->data) c10::DataPtr(std::move(data));
+    new (&o->storage) c10::Storage(x.storage());
+    o->at = x.const_data_ptr();
     o->rows = M;
     o->cols = K;
     o->stream = stream;
@@ -254,9 +259,18 @@ PyObject *new_staged(c10::DataPtr &&data, int64_t M, int64_t K, hipStream_t stre
     return reinterpret_cast<PyObject *>(o);
 }
 
+// Whether the codes are those of x as [M, K] rows, on this stream and in this recording of it.
+bool staged_for(const Staged *s, const Tensor &x, int64_t M, int64_t K, hipStream_t stream, unsigned long long recording)
+{
+    return s->stream == stream && s->recording == recording && s->rows == M && s->cols == K &&
+           s->storage.unsafeGetStorageImpl() == x.storage().unsafeGetStorageImpl() && s->at == x.const_data_ptr();
+}
+
 void staged_dealloc(PyObject *self)
 {
-    delete reinterpret_cast<Staged *>(self)->data;
+    Staged *s = reinterpret_cast<Staged *>(self);
+    s->data.~DataPtr();
+    s->storage.~Storage();
     Py_TYPE(self)->tp_free(self);
 }
 
@@ -296,10 +310,10 @@ PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip,
         PyObject *s = slot(packed, kStaged);
         if (s && Py_TYPE(s) == &g_staged_type) {
             Staged *staged = reinterpret_cast<Staged *>(s);
-            if (staged->stream == stream && staged->recording == recording && staged->rows == M && staged->cols == static_cast<int64_t>(l.K)) {
+            if (staged_for(staged, x, M, l.K, stream, recording)) {
                 const Held<1> h({s});  // (another thread may put something else there)
                 Tensor y = output(x, l.N, ScalarType::Half);
-                const uint8_t *q = static_cast<const uint8_t *>(staged->data->get());
+                const uint8_t *q = static_cast<const uint8_t *>(staged->data.get());
                 int st;
                 {
                     Unlocked u;
@@ -321,7 +335,7 @@ PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip,
                                                  nullptr, 0, stream);
         }
         if (st) return finish(st, "quantize_linear4bit_forward", nullptr);
-        PyObject *left = new_staged(std::move(ws.data), M, l.K, stream, recording);
+        PyObject *left = new_staged(std::move(ws.data), x, M, l.K, stream, recording);
         if (!left) return nullptr;
         PyObject *before = slot(packed, kStaged);
         slot(packed, kStaged) = left;

@@ -102,3 +102,22 @@ def test_rows_that_change_are_refused_and_copies_go_without(dev):
     x.add_(1)
     with pytest.raises(RuntimeError, match="modified in place"):
         layers[1](p)
+
+
+@pytest.mark.parametrize("rounds", [1, 2])   # (2: the second rows may come to lie where the first ones were)
+def test_rows_given_other_memory_are_quantized(dev, rounds):
+    """An assignment to .data between two layers keeps the tensor's version: the second layer takes the rows that are there now."""
+    from duqlinear4bitcuda_amd import nn as qnn
+    layers, q = _layers(dev, 512, (128, 256)), qnn.SymQuantizer()
+    x = torch.randn(33, 512, device=dev, dtype=torch.float16)
+    _alone(layers, q, x)
+    p = q(x)
+    layers[0](p)
+    for _ in range(rounds):
+        x.data = torch.randn(33, 512, device=dev, dtype=torch.float16)
+    want = _alone(layers, q, x.clone())
+    _equal([layers[1](p)], want[1:])
+    _equal([m(p) for m in layers], want)
+    codes, scales = tuple(t.clone() for t in (p.quantized_x, p.scales_x))
+    other = q(x.clone())
+    assert torch.equal(codes, other.quantized_x) and torch.equal(scales, other.scales_x)
