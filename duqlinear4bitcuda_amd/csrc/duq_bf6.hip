@@ -230,8 +230,8 @@ static_assert(offsetof(Bf6Params, epi) + 8 == kHeadBytes, "the fields delivered 
 // TMI = 8: 128-row tiles (6: 96).  TMI = 4: 64-row tiles for problems that would leave most CUs without a 128-row tile
 // (half the MFMAs for the same weight traffic, but twice the workgroups).  TMI = 16: 256-row tiles for problems
 // with at least one such tile per CU: the same weight traffic feeds twice the MFMAs, which takes the kernel off
-// the L2 -> CU limit that bounds the smaller tiles; all 256 AGPRs hold accumulators, an activation chunk is one
-// 128-k step (three buffers of two steps would not fit in LDS) and the epilogue parameters are fetched after the loop.
+// the L2 -> CU limit that bounds the smaller tiles; all 256 AGPRs hold accumulators, its three buffers of 256 k take 144 KB
+// of LDS, and the epilogue parameters are fetched after the loop.
 template <int TMI, int TNI, int EPI>
 struct Bf6Tile {
     static constexpr int BM = 16 * TMI, BN = 64 * TNI;
@@ -427,7 +427,8 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
         for (int j = 0; j < NXP; ++j) fetch_x(xreg[j], j, 2);
         lds_barrier();
     } else {
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(9 * NP + NXP) : "memory");
+        // (counts what is certain to be issued behind chunk 0, see kBehind)
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NXP) : "memory");
     }
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi) {
@@ -461,12 +462,15 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
     // One chunk = CH 128-k steps.  PH = position of the chunk in a turn of the weight ring: its steps use ring
     // slots CH*PH ..; a slot is refilled (with the step four ahead) during the step after its use.
     uint32_t cur = 0, nxt = kBuf, nx2 = 2 * kBuf;  // buffers of chunks c, c + 1, c + 2
-    auto chunk = [&](auto ph, auto last, uint32_t c) {
+    auto chunk = [&](auto ph, uint32_t c) {
         constexpr int PH = decltype(ph)::value;
         const v4u dXc = chunk_desc(c + 2);
-        // Vector memory instructions of this body up to its barrier, all of them behind the loads that the barrier waits for
-        // (direct form).  After the loop the compiler leaves out weight loads that nothing reads: only the activations count.
-        constexpr int kBehind = NXP + (decltype(last)::value ? 0 : 6 * NP);
+        // Direct form: the loads that the body's barrier waits for have at least this many vector memory instructions behind them,
+        // its own activation loads.  The weight loads between those are ordinary ones, which a compiler may leave out where nothing
+        // reads them (after the loop it does): a wait that counted them would be too weak then.  Counting them, as the generated code
+        // would allow, gains nothing: 4096 x 4096 x 1152 19.4 us either way, 4096 x 28672 x 8192 421 / 422.
+        constexpr int kBehind = NXP;
+        static_assert(STAGED || NXP == 6 * CH, "six activation loads in every step of a body, all in front of its barrier");
         // Side work is spread one instruction per MFMA: the loop is bound by the issue rate of its single
         // wavefront per SIMD, and a slot that holds more than about 12 cycles of other work stalls the matrix pipe.
 #pragma unroll
@@ -535,10 +539,10 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
     // (no branch inside the loop: a path that skips a chunk would make the compiler count only that
     // path's loads when it waits for a fragment, and drain the prefetch ring every iteration)
     for (; c + 1 < nchunks; c += 2) {
-        chunk(P0{}, std::false_type{}, c);
-        chunk(P1{}, std::false_type{}, c + 1);
+        chunk(P0{}, c);
+        chunk(P1{}, c + 1);
     }
-    if (c < nchunks) chunk(P0{}, std::true_type{}, c);
+    if (c < nchunks) chunk(P0{}, c);
     // (every wavefront's loads and reads are done: the epilogue stages its outputs over the buffers)
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (LATE_PARAMS) load_params();
