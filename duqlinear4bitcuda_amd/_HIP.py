@@ -471,6 +471,14 @@ def gemm_stream_tile_for(M: int, N: int, K: int) -> int:
     return _lib.load().duq_gemm_stream_tile_for(M, N, K)
 
 
+def gemm_plan_for(M: int, N: int, K: int, mode: int = EPI_SYM):
+    """Tiles of the prefill kernel for a shape, (rows, columns, column up to which, rows behind it, columns behind it);
+    ``mode`` -1: int32 outputs.  See ``duq_gemm_plan_for`` in include/duq_hip.h."""
+    plan = (ctypes.c_uint32 * 5)()
+    _lib.check(_lib.load().duq_gemm_plan_for(mode, M, N, K, ctypes.addressof(plan)), "gemm_plan_for")
+    return tuple(plan)
+
+
 def gemm_kernel_for(M: int, N: int, K: int) -> int:
     """Which kernel the int4 GEMM runs for a shape (host arithmetic, no GPU work): see
     ``duq_gemm_kernel_for`` in include/duq_hip.h."""

@@ -465,7 +465,28 @@ int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K)
 {
     if (duq::gemm_kernel_for(M, N, K) != duq::kKernelStream) return 0;
     const duq::StreamTile t = duq::select_stream_tile(M, N, K, 1, false);
-    return (int)(t.rows * 1000 + t.cols);
+    return t.main_cols ? 128256 : (int)(t.rows * 1000 + t.cols);
+}
+
+int duq_gemm_plan_for(int32_t mode, uint32_t M, uint32_t N, uint32_t K, uint32_t plan[5])
+{
+    if (!plan) return DUQ_E_NULL;
+    if (mode < -1 || mode > DUQ_EPI_ASYM_DUAL_ROWSUM) return DUQ_E_MODE;
+    for (int i = 0; i < 5; ++i) plan[i] = 0;
+    const bool mode5 = mode == DUQ_EPI_ASYM_DUAL_ROWSUM;
+    const int kernel = mode5 && duq::takes_lds_kernel(M, N, K, true) ? duq::kKernelLds : duq::gemm_kernel_for(M, N, K);
+    if ((kernel != duq::kKernelStream && kernel != duq::kKernelTile) || (K <= 256 && !mode5) ||
+        (mode5 && !duq::gemm_fuses_dual_rowsum(M, N, K)))
+        return DUQ_OK;
+    const duq::StreamTile t = duq::select_stream_tile(M, N, K, 1, mode5);
+    if (mode >= 0 && t.main_cols) {
+        const uint32_t mixed[5] = {t.main_rows, 256, t.main_cols, t.rest_rows, t.rest_cols};
+        for (int i = 0; i < 5; ++i) plan[i] = mixed[i];
+    } else if (!t.stream) {
+        plan[0] = t.rows;
+        plan[1] = t.cols;
+    }
+    return DUQ_OK;
 }
 
 uint64_t duq_quantize_linear4bit_workspace_bytes(uint32_t M, uint32_t N, uint32_t K)

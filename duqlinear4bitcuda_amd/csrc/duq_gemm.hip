@@ -745,7 +745,7 @@ static void launch_epi(GemmParams &p, hipStream_t stream, uint32_t batch = 1)
         }
     }
     const StreamTile tile = select_stream_tile(p.M, p.N, p.K, batch, EPI == 5);
-    if (tile.stream) {
+    if (tile.stream && (EPI < 0 || !tile.main_cols)) {
         p.tiles_m = (p.M + 63) / 64;
         p.tiles_n = (p.N + 127) / 128;
         DUQ_LAUNCH_HEAD((gemm_s4_stream_kernel<EPI, BIAS>), dim3(p.tiles_m * p.tiles_n, 1, batch), dim3(256), 0, stream, p);

@@ -234,6 +234,10 @@ int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
  * where the fused entry points cover the last columns of a problem in smaller tiles, behind tiles of 128 x 256 or 256 x 256); 0 for the other kernels.  (The dual-uniform row-sum
  * epilogue never runs the 256-row tile.) */
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
+/* The tiles of a launch of the prefill kernel: mode DUQ_EPI_* (binary16 outputs) or -1 (int32 outputs, duq_matmul_host_4bit);
+ * plan = rows and columns of a tile, and where plan[2] > 0 the column up to which these reach, with the rows and columns of the
+ * tiles behind it.  All zero for shapes that other kernels run.  (No GPU work; for tests and tuning.) */
+int duq_gemm_plan_for(int32_t mode, uint32_t M, uint32_t N, uint32_t K, uint32_t plan[5]);
 
 /* Measurement aid, no counterpart in the reference: reads `bytes` (16-byte aligned, < 4 GiB) of device memory
  * with the access pattern of the decode kernels (every load of a workgroup requested up front, 32 KB per

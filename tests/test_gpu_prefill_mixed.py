@@ -23,7 +23,8 @@ def test_mixed(dev, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(690, 13001, 2112), (1999, 5003, 2112),    # 64 x 128 behind one round of 128 x 256
                                    (520, 21912, 2560),                       # 192 x 128 behind 1
                                    (935, 20001, 2112), (1203, 15441, 2176),    # 128 x 128 behind one round of 256 x 256
-                                   (1801, 12518, 2112)])                      # 128 x 256 behind one
+                                   (1801, 12518, 2112),                       # 128 x 256 behind one
+                                   (2355, 3344, 2496), (4160, 3924, 5888)])   # int32 outputs: stream kernel, 128 x 128
 def test_mixed_of_either_kind(dev, M, N, K):
     from duqlinear4bitcuda_amd import _HIP as hip
     print("mixed", M, N, K, flush=True)

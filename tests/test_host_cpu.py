@@ -379,6 +379,35 @@ def test_stream_tile_rule():
     assert f(16, 4096, 4096) == 0 and f(1, 4096, 4096) == 0 and f(200, 1101, 4160) == 0   # decode kernels
 
 
+def test_tile_of_int32_outputs():
+    """Uneven rounds in tiles of two kinds are for binary16 outputs; int32 outputs keep the cheapest uniform tile, which is what the
+    dual-uniform row-sum epilogue, that has no uneven rounds either, names (it has no 256-row tile)."""
+    from duqlinear4bitcuda_amd import _HIP as hip
+    assert hip.gemm_plan_for(4160, 3924, 5888) == (256, 256, 3840, 64, 128)
+    assert hip.gemm_plan_for(4160, 3924, 5888, -1) == (128, 128, 0, 0, 0)
+    assert hip.gemm_plan_for(897, 8688, 4544)[2] and hip.gemm_plan_for(897, 8688, 4544, -1) == (64, 128, 0, 0, 0)
+    # (the stream kernel's tile: none of the prefill kernel's)
+    assert hip.gemm_plan_for(2355, 3344, 2496) == (128, 256, 3328, 64, 128) and hip.gemm_plan_for(2355, 3344, 2496, -1) == (0,) * 5
+    assert hip.gemm_plan_for(2048, 4096, 4096) == hip.gemm_plan_for(2048, 4096, 4096, -1) == (128, 256, 0, 0, 0)
+    assert hip.gemm_plan_for(8, 4096, 4096) == hip.gemm_plan_for(2048, 4096, 256) == (0,) * 5
+    rng, uneven = np.random.default_rng(9), 0
+    for _ in range(4000):
+        M, N, K = (int(np.exp(rng.uniform(np.log(a), np.log(b)))) for a, b in ((128, 4096), (256, 28672), (512, 28672)))
+        K = K // 64 * 64
+        plan, whole = hip.gemm_plan_for(M, N, K), hip.gemm_plan_for(M, N, K, -1)
+        assert whole[2:] == (0, 0, 0)
+        uneven += plan[2] > 0
+        if plan[2] == 0:
+            assert whole == plan
+        else:
+            assert plan[1] == 256 and 0 < plan[2] < N and plan[2] % 256 == 0 and plan[0] in (128, 256)
+            assert -(-M // plan[0]) * plan[2] // 256 <= 256 * max(1, -(-M // plan[0]) * -(-N // 256) // 256)
+            assert -(-M // plan[3]) * -(-(N - plan[2]) // plan[4]) <= 256
+        if whole[:2] != (256, 256):
+            assert whole == hip.gemm_plan_for(M, N, K, hip.EPI_ASYM_DUAL_ROWSUM), (M, N, K)
+    assert uneven > 200
+
+
 def test_deferred_quantized_tensor_host_side():
     """What SymQuantizer hands over for a few rows: shape, device and the check that the rows were not written to,
     without anything being computed (quantizing needs the GPU)."""
