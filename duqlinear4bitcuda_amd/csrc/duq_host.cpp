@@ -279,6 +279,8 @@ PyObject *staged_reduce(PyObject *, PyObject *) { return Py_BuildValue("(O())", 
 
 PyMethodDef g_staged_methods[] = {{"__reduce__", staged_reduce, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 
+constexpr int64_t kFp6MinTiles = 32;  // _FP6_MIN_TILES of nn/linear.py: smaller settings are taken as they are (_fp6_pays)
+
 // min_tiles: the module's fp6_min_tiles, negative where the caller does not know it.  packed: the deferred tensor that x is the rows
 // of, or null
 PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip, int qmax, int64_t min_tiles = -1, PyObject *packed = nullptr)
@@ -295,7 +297,7 @@ PyObject *run_rows(FusedCall *c, PyObject *buffers, const Tensor &x, float clip,
         const int64_t tiles = (M + 63) / 64 * ((l.N + 255) / 256);
         const int64_t per = l.K >= 8192 ? 8 : l.K >= 2048 ? 10 : 20;
         if (s && s != Py_None &&
-            (min_tiles < 0 || ((M > 1024 || l.K < 1024 || tiles / per >= min_tiles) &&
+            (min_tiles < 0 || ((M > 1024 || l.K < 1024 || min_tiles < kFp6MinTiles || tiles / per >= min_tiles) &&
                                (tiles >= min_tiles || (M > 256 && 8 * tiles >= 5 * min_tiles)))))
             return none();
     }

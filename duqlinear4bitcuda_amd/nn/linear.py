@@ -215,6 +215,9 @@ def _asym_params(w: torch.Tensor):
     return scale, zeros, codes
 
 
+_FP6_MIN_TILES = 32  # the rule for smaller settings is written in csrc/duq_host.cpp too
+
+
 class _Linear4bitBase(_MovesTogether):
     fused = True
     # 6-bit float matrix path (not in the reference): taken when the layer holds a weight shadow
@@ -222,10 +225,12 @@ class _Linear4bitBase(_MovesTogether):
     # elements, 48 of up to 12288, 32 beyond) and at least fp6_min_tiles output tiles of 64 x 256, or more than 256
     # rows and 5/8 of that (below, the integer kernels' smaller tiles and the decode kernels do better).  Rows that the layer
     # gets unquantized, up to 1024 of 1024 elements and more, which the integer kernels take in one library call: ten times as
-    # many tiles, twenty below 2048 elements, eight from 8192 on (_fp6_pays).  Eager steps of Linear4bitASQ, 6-bit float against integer, us: 160 x 4096 x 4096 25.4 / 11.8, 512 x 4096 x 8192
+    # many tiles, twenty below 2048 elements, eight from 8192 on (_fp6_pays).  A setting below the default asks for the 6-bit
+    # float path where these rules have the integer kernels ahead, and is taken as it is in either case.
+    # Eager steps of Linear4bitASQ, 6-bit float against integer, us: 160 x 4096 x 4096 25.4 / 11.8, 512 x 4096 x 8192
     # 25.0 / 21.6, 768 x 4096 x 8192 26.9 / 29.2, 384 x 8192 x 8192 32.7 / 32.0, 512 x 8192 x 8192 33.9 / 35.0, 248 x 19968 x 17264 106 / 114, 1024 x 16384 x 4096 64.9 /
     # 63.2, 512 x 1536 x 16384 25.3 / 19.0, 768 x 1536 x 16384 25.0 / 27.4
-    fp6_min_tiles = 32
+    fp6_min_tiles = _FP6_MIN_TILES
     _shadow_key = None
 
     def _finish(self, y):
@@ -329,8 +334,9 @@ class _Linear4bitBase(_MovesTogether):
 
     def _fp6_pays(self, rows):
         """The same for rows that are not quantized yet."""
-        K = self.in_features
-        if rows <= 1024 <= K and -(-rows // 64) * -(-self.out_features // 256) < (8 if K >= 8192 else 10 if K >= 2048 else 20) * self.fp6_min_tiles:
+        K, least = self.in_features, self.fp6_min_tiles
+        if rows <= 1024 <= K and least >= _FP6_MIN_TILES and \
+                -(-rows // 64) * -(-self.out_features // 256) < (8 if K >= 8192 else 10 if K >= 2048 else 20) * least:
             return False
         return self._fp6_wanted(rows)
 

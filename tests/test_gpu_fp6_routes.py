@@ -20,9 +20,25 @@ def test_rule(monkeypatch, rows, K, N, wanted):
     assert layer._fp6_pays(rows) == wanted
 
 
+@pytest.mark.parametrize("rows,K,N,least,wanted", [(65, 4096, 256, 1, True), (65, 4096, 256, 2, True), (65, 4096, 256, 3, False),
+                                                   (64, 4096, 4096, 1, False), (65, 1024, 31 * 128, 31, True), (65, 1024, 30 * 128, 31, False),
+                                                   (257, 4096, 1024, 31, True), (257, 4096, 768, 31, False),     # 5/8 of it above 256 rows
+                                                   (65, 4096, 16 * 256, 32, False), (65, 4096, 16 * 256, 31, True),
+                                                   (65, 4096, 176 * 256, 33, True), (65, 4096, 164 * 256, 33, False)])
+def test_setting_below_the_default(monkeypatch, rows, K, N, least, wanted):
+    """A caller who asks for the 6-bit float path from fewer tiles on than the default gets it there for rows of any origin."""
+    from duqlinear4bitcuda_amd.nn import Linear4bitASQ
+    layer = Linear4bitASQ.__new__(Linear4bitASQ)
+    torch.nn.Module.__init__(layer)
+    layer.in_features, layer.out_features, layer.fp6_min_tiles = K, N, least
+    monkeypatch.setattr(Linear4bitASQ, "_fp6_ready", lambda self: True)
+    assert layer._fp6_pays(rows) == wanted
+    assert least > 31 or layer._fp6_wanted(rows) == wanted
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,N", [(70, 1024, 512), (300, 512, 1024), (1000, 1152, 4096), (1024, 2048, 5120), (1024, 2048, 4864), (1024, 1024, 10240),
-                                   (1030, 1024, 512)])
+                                   (1030, 1024, 512), (300, 2048, 1024)])
 def test_native_code_agrees(dev, M, K, N):
     from duqlinear4bitcuda_amd import nn as qnn
     print("fp6 routes", M, K, N, flush=True)
@@ -32,7 +48,7 @@ def test_native_code_agrees(dev, M, K, N):
     for layer in (qnn.Linear4bitASQ.from_linear(lin).to(dev), qnn.LinearQuant4bitDUASQRowSum.from_linear(lin)):
         want = layer(x)
         layer.enable_fp6()
-        for tiles in (32, 1, 10 ** 6):
+        for tiles in (32, 31, 1, 10 ** 6):
             layer.fp6_min_tiles = tiles
             got = layer(x)
             assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (type(layer).__name__, tiles)
