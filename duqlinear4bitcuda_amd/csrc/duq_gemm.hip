@@ -776,6 +776,7 @@ int launch_gemm_s4_batched(const uint8_t *A, const uint8_t *B, uint32_t M, uint3
     p.M = M;
     p.N = N;
     p.K = K;
+    p.problems = batch;
     p.C = out_acc;
     p.y = y;
     if (epi) p.epi = *epi;

@@ -18,6 +18,7 @@ struct GemmParams {
     int32_t *C;        // int32 out (EPI < 0)
     uint16_t *y;       // fp16 out  (EPI >= 0)
     uint32_t tiles_n;
+    uint32_t problems; // in the launch, see batch_shift
     Epilogue epi;
 };
 static_assert(offsetof(GemmParams, epi) == kHeadBytes, "the fields delivered in registers");

@@ -48,8 +48,13 @@ __device__ __forceinline__ v4u buf_load16_aux(__amdgpu_buffer_rsrc_t r, uint32_t
 // cache lines leave as whole lines either way: streamed (integer kernel 2048 x 4096 x 4096 30.5 us against 31.5, 2048 x 4096 x 1024
 // 12.6 / 14.0, 2461 x 28288 x 768 75.6 / 77.2; 6-bit floats 23.8 / 25.6, 10.3 / 12.0, 62.6 / 66.2).  Larger outputs of other widths:
 // the pieces of a line that come from different workgroups meet in the L2, if they stop there (integer kernel 2461 x 28336 x 768 92.2
-// -> 78.4, 4078 x 13360 x 832 91.7 -> 82.2, 1999 x 11024 x 4096 80.0 -> 74.0; 6-bit floats 80.3 -> 67.8, 61.6 -> 53.9, 59.2 -> 56.2).
-__device__ __forceinline__ bool streams_outputs(uint32_t M, uint32_t N) { return N % 64 == 0 || (uint64_t)M * N <= (16u << 20); }
+// -> 78.4, 4078 x 13360 x 832 91.7 -> 82.2, 1999 x 11024 x 4096 80.0 -> 74.0; 6-bit floats 80.3 -> 67.8, 61.6 -> 53.9, 59.2 -> 56.2).  The output
+// is that of all problems of a launch (8 of 2000 x 2008 x 512 43.3 -> 35.1, 16 of 1000 x 1992 x 640 48.2 -> 39.6, 32 of 1000 x 1000 x 1024 51.6
+// -> 43.9, 8 of 2048 x 2056 x 2048 83.1 -> 80.9; the least 5 of 2000 x 2008 x 512 23.0 -> 23.4).
+__device__ __forceinline__ bool streams_outputs(uint32_t M, uint32_t N, uint32_t problems = 1)
+{
+    return N % 64 == 0 || (uint64_t)M * N * problems <= (16u << 20);
+}
 
 // Stages of the LDS kernels (duq_decode.hip, duq_int8.hip): MT row tiles and NT column tiles of 16 per workgroup of eight
 // wavefronts.

@@ -24,3 +24,24 @@ def test_either_side_of_the_line(dev, N, K, fp6):
     for part in (slice(0, 64), slice(most - 130, most), slice(most + 170, most + 300)):
         assert torch.equal(layer(quantizer(x[part])), large[part])
     assert torch.equal(layer(quantizer(x[:most])), large[:most])
+
+
+# every kernel that takes batches (rows of up to 256 elements in tiles of 64 and 32 rows, of 640: 64 x 128, of 2048: prefill tiles), rows of
+# whole and half lines, of 16-byte pieces and others, on either side of 16 Mi outputs in all problems together
+@pytest.mark.parametrize("b,M", [(9, 1000), (7, 1000), (300, 30)])
+@pytest.mark.parametrize("N", [2048, 2016, 2008, 1998])
+@pytest.mark.parametrize("K", [128, 192, 256, 640, 2048])
+def test_batches(dev, b, M, N, K):
+    from duqlinear4bitcuda_amd import _HIP as hip
+    print("output stores of a batch", b, M, N, K, flush=True)
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    codes = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
+    q, w = codes(b, M, K // 2), codes(b, N, K // 2)
+    sx, sw = (torch.rand(b, r, generator=g, device=dev).half() / 64 for r in (M, N))
+    zx, zw = (torch.randint(0, 15, (b, r), generator=g, device=dev).half() for r in (M, N))
+    for mode, z in ((hip.EPI_SYM, (None, None)), (hip.EPI_ASYM, (zx, zw))):
+        got = hip.batch_linear4bit_forward(mode, q, sx, z[0], w, sw, z[1])
+        for i in sorted({0, 1, b // 2, b - 1}):
+            zi = [None if t is None else t[i] for t in z]
+            want = hip.linear4bit_forward(mode, q[i], sx[i], zi[0], w[i], sw[i], zi[1])
+            assert torch.equal(got[i].view(torch.int16), want.view(torch.int16)), (mode, i)
