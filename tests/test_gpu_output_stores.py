@@ -45,3 +45,19 @@ def test_batches(dev, b, M, N, K):
             zi = [None if t is None else t[i] for t in z]
             want = hip.linear4bit_forward(mode, q[i], sx[i], zi[0], w[i], sw[i], zi[1])
             assert torch.equal(got[i].view(torch.int16), want.view(torch.int16)), (mode, i)
+
+
+# one problem of short rows: either side of 16 Mi and of 128 Mi outputs, of 128 and 192 elements
+@pytest.mark.parametrize("N,K,M", [(2016, 128, 9000), (2016, 192, 9000), (2008, 192, 9000), (2008, 256, 9000), (2008, 256, 8000), (8200, 256, 16400), (8200, 192, 16400)])
+def test_short_rows(dev, N, K, M):
+    from duqlinear4bitcuda_amd import _HIP as hip
+    print("output stores, short rows", M, N, K, flush=True)
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    codes = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
+    q, w = codes(M, K // 2), codes(N, K // 2)
+    sx, sw = (torch.rand(r, generator=g, device=dev).half() / 64 for r in (M, N))
+    got = hip.linear4bit_forward(hip.EPI_SYM, q, sx, None, w, sw)
+    for lo in (0, M // 2 - 65, M - 130):   # (as many rows: outputs that are always streamed)
+        part = slice(lo, lo + 130)
+        want = hip.linear4bit_forward(hip.EPI_SYM, q[part], sx[part], None, w, sw)
+        assert torch.equal(got[part].view(torch.int16), want.view(torch.int16)), lo
