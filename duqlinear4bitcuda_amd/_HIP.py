@@ -479,6 +479,13 @@ def gemm_plan_for(M: int, N: int, K: int, mode: int = EPI_SYM):
     return tuple(plan)
 
 
+def gemm_bf6_plan_for(M: int, N: int, K: int, mode: int = EPI_SYM):
+    """``gemm_plan_for`` for the 6-bit float matrix path."""
+    plan = (ctypes.c_uint32 * 5)()
+    _lib.check(_lib.load().duq_gemm_bf6_plan_for(mode, M, N, K, ctypes.addressof(plan)), "gemm_bf6_plan_for")
+    return tuple(plan)
+
+
 def gemm_kernel_for(M: int, N: int, K: int) -> int:
     """Which kernel the int4 GEMM runs for a shape (host arithmetic, no GPU work): see
     ``duq_gemm_kernel_for`` in include/duq_hip.h."""

@@ -489,6 +489,19 @@ int duq_gemm_plan_for(int32_t mode, uint32_t M, uint32_t N, uint32_t K, uint32_t
     return DUQ_OK;
 }
 
+int duq_gemm_bf6_plan_for(int32_t mode, uint32_t M, uint32_t N, uint32_t K, uint32_t plan[5])
+{
+    if (!plan) return DUQ_E_NULL;
+    if (mode < 0 || mode > DUQ_EPI_ASYM_DUAL_ROWSUM) return DUQ_E_MODE;
+    for (int i = 0; i < 5; ++i) plan[i] = 0;
+    if (M == 0 || N == 0) return DUQ_OK;
+    const duq::Bf6Plan t = duq::plan_bf6(M, N, K, mode == DUQ_EPI_ASYM_DUAL_ROWSUM);
+    plan[0] = t.rows;
+    plan[1] = t.width;
+    if (t.cols) plan[2] = t.cols * 256, plan[3] = t.rest, plan[4] = 256;
+    return DUQ_OK;
+}
+
 uint64_t duq_quantize_linear4bit_workspace_bytes(uint32_t M, uint32_t N, uint32_t K)
 {
     if (M == 0 || N == 0 || K == 0) return 0;

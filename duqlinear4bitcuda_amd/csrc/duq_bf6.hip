@@ -137,10 +137,6 @@ int launch_activation_shadow_bf6(const uint8_t *q, uint32_t M, uint32_t K, uint8
 // prefetches issued just before it (a full memory latency per chunk).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-#ifndef DUQ_BF6_NARROW_MAX_TILES
-#define DUQ_BF6_NARROW_MAX_TILES 128
-#endif
-
 // One MFMA on half h (0: registers 0..5, 1: registers 6..11) of weight pair tuple t, which lives in the twelve
 // registers v[128 + 12*t .. 139 + 12*t].  Naming the registers pins the tuple, so that the three 128-bit loads that
 // fill it write them in place and the two operands are its halves: no register moves, which an opaque MFMA would
@@ -692,10 +688,7 @@ static void launch_mixed(const Bf6Params &p, hipStream_t stream)
 // 9520 x 6528 104 -> 91.6, 1000 x 22016 x 4096 68.3 -> 62.6, 1500 x 13824 x 4096 68.2 -> 62.2).  The 96-row tile is for what needs a
 // round and a bit of 64-row tiles and leaves half the CUs without a 128-row one (GEMM alone: 2894 x 1536 x 3840 22.8 -> 20.1, 1957 x
 // 2256 x 19968 87.5 -> 78.9, 3000 x 2048 x 2048 14.0 -> 12.4; with epilogue 5 1536 x 4096 x 4096 32.1 -> 27.8).
-struct Bf6Plan {
-    uint32_t rows, cols = 0, rest = 0;  // cols > 0: columns of 256-row tiles, the others in tiles of `rest` rows
-};
-static Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
+Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
 {
     const float n = (float)((K + 255) / 256);
     const uint32_t rows[4] = {64, 96, 128, 256}, tn = (N + 255) / 256;
@@ -716,6 +709,9 @@ static Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
         const float c = rounds(tiles(k, tn)) * cost[k];
         if (c < least) best.rows = rows[k], least = c;
     }
+    // CUs left without a 64 x 256 tile: 64 x 128 tiles, twice as many, as long as they still run in one round
+    // (measured: 23-35 % faster up to 128 tiles of 64 x 256, slower from 160 on)
+    if (best.rows == 64 && tiles(0, tn) <= 128) best.width = 128;
     if (mode5) return best;
     least *= 0.96f;
     // (whole rounds of 256 rows only: a round of 128-row tiles and one of 64-row tiles take longer than a round of 256-row ones;
@@ -724,7 +720,7 @@ static Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
     if (whole == 0 || cols >= tn || n < 6.0f) return best;
     for (int r = 0; r < 3; ++r) {
         const float c = (float)whole * cost[3] + cost[r];
-        if (tiles(r, tn - cols) <= 256 && c < least) least = c, best = Bf6Plan{256, cols, rows[r]};
+        if (tiles(r, tn - cols) <= 256 && c < least) least = c, best = Bf6Plan{256, 256, cols, rows[r]};
     }
     return best;
 }
@@ -745,14 +741,9 @@ static void launch_mode(Bf6Params &p, hipStream_t stream)
     }
     if (plan.rows == 128) return launch_tile<8, 4, EPI>(p, stream);
     if (plan.rows == 96) return launch_tile<6, 4, EPI>(p, stream);
-    // CUs left without a 64 x 256 tile: 64 x 128 tiles, twice as many, as long as they still run in one round
-    // (measured: 23-35 % faster up to 128 tiles of 64 x 256, slower from 160 on)
-    if (p.tiles_m * p.tiles_n <= DUQ_BF6_NARROW_MAX_TILES) {
-        p.tiles_n = (p.N + 127) / 128;
-        launch_tile<4, 2, EPI>(p, stream);
-    } else {
-        launch_tile<4, 4, EPI>(p, stream);
-    }
+    if (plan.width == 256) return launch_tile<4, 4, EPI>(p, stream);
+    p.tiles_n = (p.N + 127) / 128;
+    launch_tile<4, 2, EPI>(p, stream);
 }
 
 int launch_gemm_bf6(const uint8_t *X, const uint8_t *W, uint32_t M, uint32_t N, uint32_t K, const Epilogue &epi,

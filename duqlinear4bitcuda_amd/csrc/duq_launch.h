@@ -305,6 +305,11 @@ int launch_gemm_s4_batched(const uint8_t *A, const uint8_t *B, uint32_t M, uint3
 // (duq_bf6.hip).  K % 128 == 0, N % 16 == 0.
 int launch_weight_shadow_bf6(const uint8_t *w, uint32_t N, uint32_t K, uint8_t *out, hipStream_t stream);
 int launch_activation_shadow_bf6(const uint8_t *q, uint32_t M, uint32_t K, uint8_t *out, hipStream_t stream);
+// Tiles of a launch: rows x width; cols > 0: that many columns of them, the others in tiles of `rest` rows.
+struct Bf6Plan {
+    uint32_t rows, width = 256, cols = 0, rest = 0;
+};
+Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5);
 // epi.mode 5 (row-sum epilogue of the dual-uniform layer) also needs the packed-int4 operands the shadows were made
 // from, xq [M, K/2] and wq [N, K/2]: the first eight bytes of every row are read.
 int launch_gemm_bf6(const uint8_t *X, const uint8_t *W, uint32_t M, uint32_t N, uint32_t K, const Epilogue &epi,

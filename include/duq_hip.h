@@ -238,6 +238,8 @@ int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
  * plan = rows and columns of a tile, and where plan[2] > 0 the column up to which these reach, with the rows and columns of the
  * tiles behind it.  All zero for shapes that other kernels run.  (No GPU work; for tests and tuning.) */
 int duq_gemm_plan_for(int32_t mode, uint32_t M, uint32_t N, uint32_t K, uint32_t plan[5]);
+/* The same for duq_linear4bit_forward_bf6 and, mode DUQ_EPI_ASYM_DUAL_ROWSUM, duq_linear4bit_forward_dual_rowsum_bf6. */
+int duq_gemm_bf6_plan_for(int32_t mode, uint32_t M, uint32_t N, uint32_t K, uint32_t plan[5]);
 
 /* Measurement aid, no counterpart in the reference: reads `bytes` (16-byte aligned, < 4 GiB) of device memory
  * with the access pattern of the decode kernels (every load of a workgroup requested up front, 32 KB per

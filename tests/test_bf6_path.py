@@ -211,9 +211,10 @@ def _epi_inputs(rng, M, N):
                                    # more than 160 tiles of 64 x 256 (the ones above run 64 x 128 tiles): 64 x 256 tiles
                                    (704, 4096, 512), (1000, 4096, 256), (900, 3000 - 8, 384),
                                    # enough tiles for the 128-row variant of the kernel
-                                   (2048 + 70, 4096 - 48, 384), (2048, 4096, 128),
-                                   # ... and for the 256-row variant: one to seven steps (its loop turns every four), ragged edges
-                                   (4096, 4096, 128), (4096 - 37, 4096 - 48, 384), (4096, 4096, 512), (4096, 4096 - 16, 896)])
+                                   (2048 - 30, 4096 - 48, 384), (2048, 4096, 128),
+                                   # ... and for the 256-row variant: one to seven steps of 128 k, ragged edges
+                                   (2048 + 70, 4096 - 48, 384), (4096, 4096, 128), (4096 - 37, 4096 - 48, 384), (4096, 4096, 512),
+                                   (4096, 4096 - 16, 896)])
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_gpu_forward_bf6_equals_oracle(hip, dev, M, N, K, with_bias):
     """One and several chunks, odd and even numbers of 128-k steps, ragged M, N that ends inside a
@@ -245,11 +246,13 @@ def test_gpu_forward_bf6_equals_oracle(hip, dev, M, N, K, with_bias):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(2048 - 30, 11008, 1408), (1000, 22016 - 16, 1408),     # 128-row tiles behind a round of 256-row ones
-                                   (1743, 9520, 1408), (4096 - 9, 4096 + 48, 1536)])        # 64-row tiles behind them
-def test_gpu_forward_bf6_uneven_rounds(hip, dev, M, N, K):
+@pytest.mark.parametrize("M,N,K,plan", [(2048 - 30, 11008, 1408, (256, 256, 8192, 96, 256)), (1000, 22016 - 16, 1408, (256, 256, 16384, 96, 256)),
+                                        (1743, 9520, 1408, (256, 256, 9216, 64, 256)), (4096 - 9, 4096 + 48, 1536, (256, 256, 4096, 64, 256)),
+                                        (2048, 11520, 1408, (256, 256, 8192, 128, 256))])
+def test_gpu_forward_bf6_uneven_rounds(hip, dev, M, N, K, plan):
     """Whole rounds of one kind of tile and the columns that are left in another; rows and columns that end inside either;
     every epilogue that such a launch has."""
+    assert all(hip.gemm_bf6_plan_for(M, N, K, mode) == plan for mode in range(hip.EPI_ASYM_DUAL_ROWSUM))
     print("bf6 uneven rounds", M, N, K, flush=True)
     rng = np.random.default_rng(M + 5 * N + K)
     a, b = _rand_packed(rng, M, K), _rand_packed(rng, N, K)
@@ -270,10 +273,9 @@ def test_gpu_forward_bf6_uneven_rounds(hip, dev, M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(1500, 4096, 640), (1441, 4096 - 16, 1152), (1536, 4096, 128),  # 96-row tiles
-                                   (2048, 11520, 1408)])   # the other tests' rests are in 64- and 96-row tiles: 128 rows behind 256
+@pytest.mark.parametrize("M,N,K", [(1500, 4096, 640), (1441, 4096 - 16, 1152), (1536, 4096, 128)])
 def test_gpu_forward_bf6_96_rows(hip, dev, M, N, K):
-    test_gpu_forward_bf6_uneven_rounds(hip, dev, M, N, K)
+    test_gpu_forward_bf6_uneven_rounds(hip, dev, M, N, K, (96, 256, 0, 0, 0))
 
 
 @pytest.mark.gpu
@@ -284,6 +286,8 @@ def test_gpu_96_rows_dual_rowsum(dev, M):
     from duqlinear4bitcuda_amd import nn as qnn
     print("bf6 96 rows, dual row sums", M, flush=True)
     K, N = 640, 4096 - 16
+    from duqlinear4bitcuda_amd import _HIP as hip
+    assert hip.gemm_bf6_plan_for(M, N, K, hip.EPI_ASYM_DUAL_ROWSUM) == (96, 256, 0, 0, 0)
     g = torch.Generator(device=dev).manual_seed(M)
     lin = torch.nn.Linear(K, N, device=dev, dtype=torch.float16).requires_grad_(False)
     x = torch.rand(M, K, generator=g, device=dev).half() * 6

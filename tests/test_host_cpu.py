@@ -408,6 +408,30 @@ def test_tile_of_int32_outputs():
     assert uneven > 200
 
 
+def test_tiles_of_the_6bit_float_path():
+    """Every tile of a launch covers its part of the outputs, uneven rounds are whole ones with one of smaller tiles behind, and the
+    dual-uniform row-sum epilogue runs tiles of one kind of up to 128 rows."""
+    from duqlinear4bitcuda_amd import _HIP as hip
+    assert hip.gemm_bf6_plan_for(512, 4096, 4096) == (64, 128, 0, 0, 0) and hip.gemm_bf6_plan_for(1000, 4096, 4096) == (64, 256, 0, 0, 0)
+    assert hip.gemm_bf6_plan_for(2048, 4096, 4096) == (128, 256, 0, 0, 0)
+    assert hip.gemm_bf6_plan_for(4096, 28672, 8192) == (256, 256, 0, 0, 0)
+    assert hip.gemm_bf6_plan_for(0, 16, 128) == (0,) * 5
+    rng, uneven = np.random.default_rng(10), 0
+    for _ in range(4000):
+        M, N, K = (int(np.exp(rng.uniform(np.log(a), np.log(b)))) for a, b in ((1, 8192), (16, 28672), (128, 28672)))
+        N, K = -(-N // 16) * 16, -(-K // 128) * 128
+        rows, width, cols, rest, rest_width = hip.gemm_bf6_plan_for(M, N, K)
+        assert rows in (64, 96, 128, 256) and width == (128 if rows == 64 and -(-M // 64) * -(-N // 256) <= 128 else 256)
+        uneven += cols > 0
+        if cols:
+            assert rows == 256 and cols % 256 == 0 and cols < N and rest in (64, 96, 128) and rest_width == 256
+            assert -(-M // 256) * cols // 256 <= -(-M // 256) * -(-N // 256) // 256 * 256
+            assert -(-M // rest) * -(-(N - cols) // 256) <= 256
+        dual = hip.gemm_bf6_plan_for(M, N, K, hip.EPI_ASYM_DUAL_ROWSUM)
+        assert dual[0] <= 128 and dual[2:] == (0, 0, 0) and (rows == 256 or dual == (rows, width, 0, 0, 0))
+    assert uneven > 50
+
+
 def test_deferred_quantized_tensor_host_side():
     """What SymQuantizer hands over for a few rows: shape, device and the check that the rows were not written to,
     without anything being computed (quantizing needs the GPU)."""
