@@ -400,6 +400,6 @@ def test_gpu_dual_rowsum_module_config4(dev):
     other.load_state_dict(mod.state_dict())
     assert torch.equal(other(cases.t(x, dev)).view(torch.int16), y.view(M, N).view(torch.int16))
     # the same layer on the 6-bit float matrix path: same bits
-    other.enable_fp6()
-    assert other._fp6_wanted(M)
+    other.enable_fp6().fp6_min_tiles = 1
+    assert other._fp6_pays(M)
     assert torch.equal(other(cases.t(x, dev)).view(torch.int16), y.view(M, N).view(torch.int16))
