@@ -6,7 +6,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# N: whole lines, 16-byte rows, others; M: 16 Mi outputs at most, and more, in every kind of tile
+# N: whole lines, 16-byte rows, others; M: 16 Mi outputs at most, and more (integer path: short rows, the stream kernel and, whole
+# lines only, 256 x 256 tiles; 6-bit floats: 128 x 256 and 256 x 256)
 @pytest.mark.parametrize("N,fp6", [(8192, False), (8208, False), (8200, False), (8196, False), (2049, False), (8192, True), (8208, True)])
 @pytest.mark.parametrize("K", [128, 640])
 def test_either_side_of_the_line(dev, N, K, fp6):
@@ -24,6 +25,29 @@ def test_either_side_of_the_line(dev, N, K, fp6):
     for part in (slice(0, 64), slice(most - 130, most), slice(most + 170, most + 300)):
         assert torch.equal(layer(quantizer(x[part])), large[part])
     assert torch.equal(layer(quantizer(x[:most])), large[:most])
+
+
+# more than 16 Mi outputs of 16-byte rows that are no whole lines in every kind of the prefill kernel's tiles; `part` rows, which are
+# compared with them, run smaller ones
+@pytest.mark.parametrize("M,N,plan", [(16390, 1032, (128, 128, 0, 0, 0)), (772, 25656, (128, 256, 0, 0, 0)), (1062, 22008, (256, 256, 0, 0, 0)),
+                                      (798, 21272, (128, 256, 18688, 128, 128)), (810, 21016, (128, 256, 18688, 64, 128)),
+                                      (1323, 16400, (256, 256, 10752, 128, 256)), (1825, 11000, (256, 256, 8192, 192, 128)),
+                                      (3027, 6152, (256, 256, 5376, 128, 128)), (11993, 1400, (256, 256, 1280, 64, 128))])
+def test_prefill_tiles_past_the_line(dev, M, N, plan):
+    from duqlinear4bitcuda_amd import _HIP as hip
+    K, part = 2112, 130
+    print("output stores, prefill tiles", M, N, plan, flush=True)
+    assert hip.gemm_plan_for(M, N, K) == plan and M * N > 16 << 20 and hip.gemm_plan_for(part, N, K) != plan
+    g = torch.Generator(device=dev).manual_seed(N)
+    codes = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
+    q, w = codes(M, K // 2), codes(N, K // 2)
+    sx, sw = (torch.rand(r, generator=g, device=dev).half() / 64 for r in (M, N))
+    zx, zw = (torch.randint(0, 15, (r,), generator=g, device=dev).half() for r in (M, N))
+    got = hip.linear4bit_forward(hip.EPI_ASYM, q, sx, zx, w, sw, zw)
+    for lo in (*range(0, M - part, 4 * part), M - part):
+        rows = slice(lo, lo + part)
+        want = hip.linear4bit_forward(hip.EPI_ASYM, q[rows], sx[rows], zx[rows], w, sw, zw)
+        assert torch.equal(got[rows].view(torch.int16), want.view(torch.int16)), lo
 
 
 # every kernel that takes batches (rows of up to 256 elements in tiles of 64 and 32 rows, of 640: 64 x 128, of 2048: prefill tiles), rows of
