@@ -617,7 +617,9 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
             __builtin_amdgcn_raw_buffer_store_b128(v, rY, (int)off, 0, decltype(streamed)::value ? 2 : 0);
         }
     };
-    if (streams_outputs(p.M, p.N)) store_rows(std::true_type{});
+    // (rows that begin at half lines are streamed too: us, past the L2 / into it, 1963 x 25056 x 896 58.9 / 60.2, 4096 x 16416 x 1024 82.2 /
+    // 86.2, 4096 x 28640 x 4096 267 / 288, 2048 x 20512 x 2048 69.2 / 70.1; but 4000 x 12064 x 4096 117.6 / 113.5)
+    if (p.N % 32 == 0 || streams_outputs(p.M, p.N, 1, 100u << 20)) store_rows(std::true_type{});
     else store_rows(std::false_type{});
 }
 

@@ -51,9 +51,20 @@ __device__ __forceinline__ v4u buf_load16_aux(__amdgpu_buffer_rsrc_t r, uint32_t
 // -> 78.4, 4078 x 13360 x 832 91.7 -> 82.2, 1999 x 11024 x 4096 80.0 -> 74.0; 6-bit floats 80.3 -> 67.8, 61.6 -> 53.9, 59.2 -> 56.2).  The output
 // is that of all problems of a launch (8 of 2000 x 2008 x 512 43.3 -> 35.1, 16 of 1000 x 1992 x 640 48.2 -> 39.6, 32 of 1000 x 1000 x 1024 51.6
 // -> 43.9, 8 of 2048 x 2056 x 2048 83.1 -> 80.9; the least 5 of 2000 x 2008 x 512 23.0 -> 23.4).
-__device__ __forceinline__ bool streams_outputs(uint32_t M, uint32_t N, uint32_t problems = 1)
+__device__ __forceinline__ bool few_or_whole_lines(uint32_t M, uint32_t N, uint32_t problems = 1)
 {
     return N % 64 == 0 || (uint64_t)M * N * problems <= (16u << 20);
+}
+// And streamed again above `most` outputs, where the last-level cache (256 MB) does not hold them beside what else is in it.  Past the L2 /
+// into it, us, into one output and into four in turn.  One problem, integer kernel: 4608 x 25072 x 1024 145 / 128 and 144 / 139, 8192 x
+// 16400 x 1024 172 / 170 and 169 / 194, 8192 x 28688 x 1024 284 / 328 and 280 / 328.  6-bit floats: 3600 x 28656 x 1024 123 / 113 and 121 / 120,
+// 4608 x 25072 x 1024 130 / 131 and 129 / 133, 8192 x 28688 x 1024 256 / 308 and 253 / 309.  Batches of small problems: 16 of 2000 x 2008 x 512
+// 70 / 59 and 69 / 70, 24 of them 96 / 84 and 97 / 110, 32 128 / 148 and 124 / 147; 64 of 1000 x 1000 x 1024 97 / 87 and 99 / 98, 96 136 / 138
+// and 136 / 141 (the most lost below the line: 200 of 500 x 504 x 640 83 / 84 and 82 / 90); of large ones 4 of 4090 x 4104 x 2048 158 / 142 and
+// 156 / 147, 6 of 4090 x 4104 x 512 107 / 91 and 107 / 110.
+__device__ __forceinline__ bool streams_outputs(uint32_t M, uint32_t N, uint32_t problems, uint32_t most)
+{
+    return few_or_whole_lines(M, N, problems) || (uint64_t)M * N * problems > most;
 }
 
 // Stages of the LDS kernels (duq_decode.hip, duq_int8.hip): MT row tiles and NT column tiles of 16 per workgroup of eight

@@ -32,7 +32,8 @@ def test_either_side_of_the_line(dev, N, K, fp6):
 @pytest.mark.parametrize("M,N,plan", [(16390, 1032, (128, 128, 0, 0, 0)), (772, 25656, (128, 256, 0, 0, 0)), (1062, 22008, (256, 256, 0, 0, 0)),
                                       (798, 21272, (128, 256, 18688, 128, 128)), (810, 21016, (128, 256, 18688, 64, 128)),
                                       (1323, 16400, (256, 256, 10752, 128, 256)), (1825, 11000, (256, 256, 8192, 192, 128)),
-                                      (3027, 6152, (256, 256, 5376, 128, 128)), (11993, 1400, (256, 256, 1280, 64, 128))])
+                                      (3027, 6152, (256, 256, 5376, 128, 128)), (11993, 1400, (256, 256, 1280, 64, 128)),
+                                      (8200, 16408, (256, 256, 15872, 192, 128))])   # (more than 128 Mi)
 def test_prefill_tiles_past_the_line(dev, M, N, plan):
     from duqlinear4bitcuda_amd import _HIP as hip
     K, part = 2112, 130
@@ -50,9 +51,26 @@ def test_prefill_tiles_past_the_line(dev, M, N, plan):
         assert torch.equal(got[rows].view(torch.int16), want.view(torch.int16)), lo
 
 
+# the same of the 6-bit float path: up to and above 100 Mi outputs, rows that begin at half lines
+@pytest.mark.parametrize("M,N", [(2000, 10576), (5300, 20016), (2000, 10592), (900, 20000)])
+def test_fp6_past_the_line(dev, M, N):
+    from duqlinear4bitcuda_amd import _HIP as hip
+    K, part = 640, 130
+    print("output stores, 6-bit floats", M, N, flush=True)
+    g = torch.Generator(device=dev).manual_seed(N)
+    codes = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
+    q, w = hip.activation_shadow_bf6(codes(M, K // 2)), hip.weight_shadow_bf6(codes(N, K // 2))
+    sx, sw = (torch.rand(r, generator=g, device=dev).half() / 64 for r in (M, N))
+    got = hip.linear4bit_forward_bf6(hip.EPI_SYM, q, sx, None, w, sw)
+    for lo in (*range(0, M - part, 4 * part), M - part):
+        rows = slice(lo, lo + part)
+        want = hip.linear4bit_forward_bf6(hip.EPI_SYM, q[rows], sx[rows], None, w, sw)
+        assert torch.equal(got[rows].view(torch.int16), want.view(torch.int16)), lo
+
+
 # every kernel that takes batches (rows of up to 256 elements in tiles of 64 and 32 rows, of 640: 64 x 128, of 2048: prefill tiles), rows of
-# whole and half lines, of 16-byte pieces and others, on either side of 16 Mi outputs in all problems together
-@pytest.mark.parametrize("b,M", [(9, 1000), (7, 1000), (300, 30)])
+# whole and half lines, of 16-byte pieces and others, on either side of 16 Mi and of 64 Mi outputs in all problems together
+@pytest.mark.parametrize("b,M", [(9, 1000), (7, 1000), (300, 30), (35, 1000)])
 @pytest.mark.parametrize("N", [2048, 2016, 2008, 1998])
 @pytest.mark.parametrize("K", [128, 192, 256, 640, 2048])
 def test_batches(dev, b, M, N, K):
