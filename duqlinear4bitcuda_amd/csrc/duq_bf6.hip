@@ -27,8 +27,10 @@
 // of four 128-k steps), activations into LDS (three buffers of 256 k, one
 // barrier per buffer) -> fragments read two MFMA groups ahead.  The weight operand is the
 // MFMA "A" side, so a lane ends up with four consecutive output columns of one row.
-// What bounds it is the bytes that a CU takes in: 72 KB per 256 k of a 128-row tile are 1152 cycles at 64 bytes a cycle,
-// against 1024 of MFMAs; the 256-row tile's 96 KB meet 2048.  Its activations used to be fetched 128 k at a time, half a
+// What bounds it is the bytes that a CU takes in, beside the MFMAs.  Loops of loads alone get 57 to 59 bytes a cycle from the L2
+// in whole lines, 29 where the other half of a line is asked for later: the 80 KB of lines per 256 k of a 128-row tile (72 of
+// operands; plane 1 comes in half lines) are 1410 cycles against 1024 of MFMAs, the 112 KB of a 256-row tile (96) 1980 against
+// 2048.  The latter's activations used to be fetched 128 k at a time, half a
 // cache line of plane 0 and a quarter of plane 1 per row, and the L2 delivers whole lines: 80.7 million of them where 44
 // would do (4096 x 8192 x 28672), 176 KB per 256 k instead of 112.  Chunks of 256 k fit since they go to LDS without
 // registers: 51.4 million lines, 549 -> 462 us with the quantizer (first 5 ms of a load; 491 -> 416 later), 4096 x 4096 x
@@ -617,8 +619,9 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
             __builtin_amdgcn_raw_buffer_store_b128(v, rY, (int)off, 0, decltype(streamed)::value ? 2 : 0);
         }
     };
-    // (rows that begin at half lines are streamed too: us, past the L2 / into it, 1963 x 25056 x 896 58.9 / 60.2, 4096 x 16416 x 1024 82.2 /
-    // 86.2, 4096 x 28640 x 4096 267 / 288, 2048 x 20512 x 2048 69.2 / 70.1; but 4000 x 12064 x 4096 117.6 / 113.5)
+    // (rows that begin at half lines are streamed too.  75 shapes of 17 to 110 Mi outputs, 640 to 4096 elements: 1 % ahead in the
+    // geometric mean with one weight and one output, 2 % with three weights, 7 % with three of both in turn; 4096 x 28640 x 4096 267
+    // against 288 us, 2000 x 28320 x 1280 27 % with three of both; the most lost 6 %, 1000 x 28320 x 640 and 3000 x 9056 x 1280)
     if (p.N % 32 == 0 || streams_outputs(p.M, p.N, 1, 100u << 20)) store_rows(std::true_type{});
     else store_rows(std::false_type{});
 }

@@ -199,8 +199,8 @@ struct StreamTile {
 // 2.62 per 256 k where two of 128 x 256 cost 2.94 (a CU takes in a third less for the same outputs), and one end instead of two;
 // against whole rounds of 128 x 256, with the quantizer, in the first 5 ms of a load: 1999 x 11008 x 4096 96.5 -> 87.1, 1188 x
 // 14615 x 3136 73.5 -> 64.0, 2195 x 14547 x 4800 172 -> 149, 3806 x 4832 x 2048 52.9 -> 49.1; of 17 shapes the least 1.03, the mean 1.12.
-// Of 75 shapes drawn at random (128..4096 rows, 700..20000 columns) it and the 192 x 128 tiles alone change fifteen, by 1.02 to
-// 1.34 (147 x 24961 x 14464); rows of less than 2048 elements lose by it (1234 x 6658 x 832 0.87).
+// Rows of less than 2048 elements lose by it (1234 x 6658 x 832 0.87).  Before the rounds of 256 x 256 it and the 192 x 128 tiles
+// changed fifteen of 75 shapes drawn at random (128..4096 rows, 700..20000 columns), by 1.02 to 1.34 (147 x 24961 x 14464).
 inline StreamTile with_rest(StreamTile best, float best_cost, uint32_t M, uint32_t N, float nch)
 {
     if (nch < 8.0f) return best;
