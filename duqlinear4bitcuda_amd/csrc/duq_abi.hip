@@ -49,6 +49,15 @@ int static_scratch(hipStream_t stream, unsigned char **out)
 }
 
 inline hipStream_t as_stream(duq_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
+// Whether launches on the stream are being recorded into a graph (yes where it cannot be told).
+bool recording(hipStream_t stream)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // (not the launch's that follows)
+    return true;
+}
+
 inline bool aligned(const void *p, uintptr_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; }
 
 int check_quant_shape(uint32_t rows, uint32_t colsSrc, uint32_t colsDst)
@@ -73,7 +82,8 @@ int check_gemm(const void *A, const void *B, uint32_t M, uint32_t N, uint32_t K)
 }
 
 // quantize + GEMM + dequant from binary16 activations: one launch for decode shapes, otherwise the quantizer
-// into `workspace` (codes, scales, then zero points and row sums for the asymmetric modes) followed by the GEMM.
+// into `workspace` (codes, scales, then zero points and row sums for the asymmetric modes) followed by the GEMM, or one kernel that
+// leaves the same there (quant_gemm_shape).
 // The epilogue mode decides the quantizer: symmetric for DUQ_EPI_SYM / SYM_DUAL, asymmetric for DUQ_EPI_ASYM /
 // ASYM_DUAL, its signed-shifted form for DUQ_EPI_ASYM_ROWSUM.
 struct FusedOut {
@@ -115,10 +125,17 @@ int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t
     if (rowsum && !e.rs_col) return DUQ_E_NULL;
     if (mode == DUQ_EPI_ASYM_DUAL_ROWSUM && !e.rs_col_2) return DUQ_E_NULL;
     if ((out.q && !aligned(out.q, 16))) return DUQ_E_ALIGN;
-    if (duq::decode_fp16in_one_launch(M, N, K))
-        return duq::launch_decode_fp16in(x, clip, qmax, w, M, N, K, e, y, out.q, out.scale, asym ? out.zeros : nullptr,
-                                         rowsum ? out.rowsum : nullptr, as_stream(stream));
-    // two launches: codes and per-token parameters go to the caller's outputs where given, else to the workspace
+    const duq::QuantGemmShape tile = duq::quant_gemm_shape(M, N, K);
+    const bool no_room = duq::decode_fp16in_one_launch(M, N, K);  // (the caller was asked for none)
+    const bool one_kernel = tile.rows != 0 && (no_room || !tile.eager_only || !recording(as_stream(stream)));
+    auto launch_one = [&] {
+        return one_kernel ? duq::launch_quant_gemm(tile, x, clip, qmax, w, M, N, K, e, y, out.q, out.scale, asym ? out.zeros : nullptr,
+                                                   rowsum ? out.rowsum : nullptr, as_stream(stream))
+                          : duq::launch_decode_fp16in(x, clip, qmax, w, M, N, K, e, y, out.q, out.scale, asym ? out.zeros : nullptr,
+                                                      rowsum ? out.rowsum : nullptr, as_stream(stream));
+    };
+    if (no_room) return launch_one();
+    // codes and per-token parameters go to the caller's outputs where given, else to the workspace
     const bool acc_ws = mode == DUQ_EPI_ASYM_DUAL_ROWSUM && !duq::gemm_fuses_dual_rowsum(M, N, K);
     const bool need_ws = !out.q || !out.scale || (asym && !out.zeros) || (rowsum && !out.rowsum) || acc_ws;
     int32_t *acc = nullptr;
@@ -137,6 +154,7 @@ int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t
         at += up16((uint64_t)M * 4);
         if (acc_ws) acc = reinterpret_cast<int32_t *>(at);
     }
+    if (one_kernel) return launch_one();
     int st;
     if (!asym)
         st = duq::launch_quantize_rows_sym(x, M, K, clip, qmax, out.q, out.scale, nullptr, as_stream(stream));
@@ -466,6 +484,12 @@ int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K)
     if (duq::gemm_kernel_for(M, N, K) != duq::kKernelStream) return 0;
     const duq::StreamTile t = duq::select_stream_tile(M, N, K, 1, false);
     return t.main_cols ? 128256 : (int)(t.rows * 1000 + t.cols);
+}
+
+int duq_quant_gemm_tile_for(uint32_t M, uint32_t N, uint32_t K)
+{
+    const duq::QuantGemmShape t = duq::quant_gemm_shape(M, N, K);
+    return (int)(t.rows + 256 * t.cols + 65536 * t.chunks + ((uint32_t)t.eager_only << 24));
 }
 
 int duq_gemm_plan_for(int32_t mode, uint32_t M, uint32_t N, uint32_t K, uint32_t plan[5])

@@ -26,20 +26,14 @@
 //  wide kernel (5 <= M <= 64, many column tiles per CU, K <= 8192): the MFMA kernel's plan with the weights through LDS.
 //  LDS kernel (one or two column tiles and up to four row tiles per workgroup, any K): the same MFMAs, both operands through LDS in whole
 //    cache lines, K in a loop.
-#include <cstddef>
-
-#include "duq_epilogue.h"
-#include "duq_launch.h"
-#include "duq_rowquant.h"
-#include "duq_tiles.h"
+#include "duq_decode_common.h"
 
 // Wavefronts per workgroup of the rows kernel when it quantizes its rows itself (binary16 in).  The quantize phase is
 // vector arithmetic (about 27 instructions per eight elements), the same for every workgroup, and sits between the
 // arrival of the activations and the dot products: a wavefront alone on its SIMD issues it at half the rate that
 // two reach together.  Measured (us, N = K = 4096 unless said): two rows 3.25 with four wavefronts, 3.21 with eight;
 // three / four rows 4.11 / 4.17 with four, 3.67 / 3.68 with eight (and with sixteen); four rows of 8192 / 11008
-// elements 7.5 / 8.9 with four, 6.5 / 7.1 with sixteen; eight rows 5.0 with eight, 5.1 with sixteen, of 8192
-// elements 9.1 with eight, 8.7 with sixteen.
+// elements 7.5 / 8.9 with four, 6.5 / 7.1 with sixteen; eight rows 5.0 with eight, 5.1 with sixteen.
 #ifndef DUQ_DEC_FUSEQ_WAVES
 #define DUQ_DEC_FUSEQ_WAVES 8     // eight rows; and several tiles per workgroup
 #endif
@@ -48,9 +42,6 @@
 #endif
 #ifndef DUQ_DEC_FUSEQ_WAVES_M4L
 #define DUQ_DEC_FUSEQ_WAVES_M4L 16  // of more
-#endif
-#ifndef DUQ_DEC_FUSEQ_WAVES_M8L
-#define DUQ_DEC_FUSEQ_WAVES_M8L 16  // eight rows of more than 4096 elements
 #endif
 #ifndef DUQ_DEC_FUSEQ_WAVES_M2
 #define DUQ_DEC_FUSEQ_WAVES_M2 4
@@ -72,115 +63,9 @@
 #ifndef DUQ_DEC_QUANT_GROUP
 #define DUQ_DEC_QUANT_GROUP 8
 #endif
-// wavefronts per workgroup of the MFMA kernel when it quantizes its 16 rows itself
-// (16 rows, N = 4096: sixteen against eight wavefronts K = 4096 7.2 against 7.9 us, K = 2048 4.9 against 5.4)
-#ifndef DUQ_DEC_MFMA_FUSEQ_WAVES
-#define DUQ_DEC_MFMA_FUSEQ_WAVES 16
-#endif
-
 namespace duq {
 
 namespace {
-
-constexpr uint32_t kNibbleMaskD = 0xF0F0F0F0u;
-
-// The first 56 bytes (through `y`) reach the kernels in registers (DUQ_HEAD_DECL / with_head).
-struct DecodeParams {
-    const uint8_t *A;    // packed activations [M, K/2] (pre-quantized input)
-    const uint16_t *X;   // binary16 activations [M, K] (FUSEQ)
-    const uint8_t *B;    // packed weights [N, K/2]
-    uint32_t M, N, K;
-    uint32_t tiles_per_wg;
-    int32_t *C;          // int32 out (EPI < 0)
-    uint16_t *y;         // binary16 out (EPI >= 0)
-    Epilogue epi;        // FUSEQ: s_row is not read, the kernel computes it
-    float clip;          // FUSEQ
-    int qmax;            // FUSEQ
-    uint8_t *q_out;      // FUSEQ, optional: the packed codes [M, K/2] (written by workgroup 0)
-    uint16_t *s_out;     // FUSEQ, optional: the per-token scales [M]
-    uint16_t *z_out;     // FUSEQ with an asymmetric epilogue, optional: the per-token zero points [M]
-    int32_t *rs_out;     // FUSEQ with the row-sum epilogue, optional: the per-token sums of the shifted codes [M]
-};
-static_assert(offsetof(DecodeParams, y) + sizeof(uint16_t *) == kHeadBytes, "the fields delivered in registers");
-
-// The quantization step over N units, G at a time (RowQuant::quant_units: the path is chosen once per group and the
-// group's chains interleave; a group holds 4 G more registers than a single unit).
-template <int G, int S = 0, bool ASYM, int N>
-__device__ __forceinline__ void quant_in_groups(const RowQuant<ASYM> &rq, const v4u (&raw)[N], uint32_t (&out)[N])
-{
-    if constexpr (S < N) {
-        constexpr int L = N - S < G ? N - S : G;
-        v4u in[L];
-        uint32_t w[L];
-#pragma unroll
-        for (int j = 0; j < L; ++j) in[j] = raw[S + j];
-        rq.quant_units(in, w);
-#pragma unroll
-        for (int j = 0; j < L; ++j) out[S + j] = w[j];
-        quant_in_groups<G, S + L>(rq, raw, out);
-    }
-}
-
-template <int CTRL>
-__device__ __forceinline__ int dpp_add(int v)
-{
-    return v + __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
-}
-// Sum over groups of G consecutive lanes (G = 2, 4, 8 or 16, inside one DPP row): every lane of a group
-// ends with the group's total.
-template <int G>
-__device__ __forceinline__ int group_sum(int v)
-{
-    v = dpp_add<0xB1>(v);               // quad_perm [1,0,3,2]
-    if (G >= 4) v = dpp_add<0x4E>(v);   // quad_perm [2,3,0,1]
-    if (G >= 8) v = dpp_add<0x141>(v);  // row_half_mirror: lane i <- lane 7 - i
-    if (G >= 16) v = dpp_add<0x140>(v); // row_mirror: lane i <- lane 15 - i
-    return v;
-}
-
-__device__ __forceinline__ v4u load16(const void *p) { return *reinterpret_cast<const v4u *>(p); }
-
-// Epilogue records of one output row / one output column, by mode: modes 0..4 the shared ColParams / RowEpi,
-// mode 5 (row-sum epilogue of the dual-uniform layer) the records that also carry the codes of input columns 0..9.
-template <int MODE>
-struct EpiRec {
-    using Col = ColParams;
-    using Row = RowEpi;
-};
-template <>
-struct EpiRec<5> {
-    using Col = DualCol;
-    using Row = DualRow;
-};
-
-// B / A: the packed operands (mode 5 reads the first eight bytes of the row)
-template <int MODE>
-__device__ __forceinline__ typename EpiRec<MODE>::Col load_col_rt(const Epilogue &e, uint32_t col, bool bias, const uint8_t *B,
-                                                                  uint32_t kbytes)
-{
-    if constexpr (MODE == 5)
-        return load_dual_col(e, B, kbytes, col, bias);
-    else
-        return bias ? load_col<MODE, true>(e.s_col_1, e.z_col_1, e.s_col_2, e.z_col_2, e.bias, col, e.rs_col)
-                    : load_col<MODE, false>(e.s_col_1, e.z_col_1, e.s_col_2, e.z_col_2, e.bias, col, e.rs_col);
-}
-template <int MODE>
-__device__ __forceinline__ typename EpiRec<MODE>::Row load_row_rt(const Epilogue &e, uint32_t row, const uint8_t *A, uint32_t kbytes)
-{
-    if constexpr (MODE == 5)
-        return load_dual_row(e, A, kbytes, row);
-    else
-        return load_row<MODE>(e, row);
-}
-template <int MODE>
-__device__ __forceinline__ uint16_t dequant_rt(int acc, const typename EpiRec<MODE>::Row &r, const typename EpiRec<MODE>::Col &c,
-                                               bool bias)
-{
-    if constexpr (MODE == 5)
-        return dual_finish(acc, r, c, bias);
-    else
-        return bias ? dequant_one<MODE, true>(acc, r, c) : dequant_one<MODE, false>(acc, r, c);
-}
 
 // ---------------------------------------------------------------------------------
 // rows kernel: M <= MR <= 4 (8 with binary16 activations quantized inside), K <= XS * 2048
@@ -475,32 +360,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_s4_rows_kernel(DUQ_HEAD_DECL,
 // and registers (MT * SEGS * 4 for the packed activations), not weight traffic.  Nibble -> byte as in the
 // GEMM kernels: (w & 0xF0F0F0F0) is the four odd-k nibbles times 16, ((w << 4) & 0xF0F0F0F0) the even ones;
 // every product is 256 * a * b and one arithmetic shift recovers the sum.
-//
-// FUSEQ (one row tile, EPI >= 0): the activations arrive as binary16 and the workgroup quantizes its 16 rows itself,
-// 16 / WAVES whole rows per wavefront (so a row's statistics never leave its wavefront), into LDS; the fragments
-// then come from there.  Every workgroup repeats that work: it pays while the quantizer's own launch (about 2.6 us
-// with the wait between the two) costs more than sixteen rows on a CU's vector units.
-template <int WAVES, int SEGS, int EPI, int MT = 1, bool FUSEQ = false>
+template <int WAVES, int SEGS, int EPI, int MT = 1>
 __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DECL, DecodeParams tail)
 {
     const DecodeParams p = with_head(tail, DUQ_HEAD_USE);
     constexpr int MODE = EPI < 0 ? 0 : EPI;
-    static_assert(WAVES == 4 || WAVES == 8 || (WAVES == 16 && FUSEQ), "wavefronts per workgroup");
+    static_assert(WAVES == 4 || WAVES == 8, "wavefronts per workgroup");
     static_assert(MT >= 1 && MT <= 4, "16-row activation tiles");
-    static_assert(!FUSEQ || (MT == 1 && EPI >= 0 && WAVES >= 8 && (WAVES * SEGS) % 4 == 0), "rows quantized in the kernel");
     constexpr int NG = WAVES / 4;             // groups of 256 finishing threads
     constexpr int FT = (MT + NG - 1) / NG;    // row tiles a finishing thread completes
     __shared__ v4i part[2][MT][WAVES][64];
-    // FUSEQ: the codes of the 16 rows (a row every XSTRIDE bytes: 16 bytes more than the longest row, so that the 16
-    // rows a fragment read touches fall on different banks) and their per-token parameters
-    constexpr int RPW = FUSEQ ? 16 / WAVES : 1;        // rows a wavefront quantizes
-    constexpr int UPR = FUSEQ ? WAVES * SEGS / 4 : 1;  // 8-element units per lane and row
-    constexpr uint32_t XSTRIDE = WAVES * SEGS * 64 + 16;
-    __shared__ __attribute__((aligned(16))) uint8_t xs[FUSEQ ? 16 * XSTRIDE : 16];
-    __shared__ uint16_t srow[16], zrow[16];
-    __shared__ int rsrow[16];
-    constexpr bool ASYMQ = FUSEQ && (MODE == 1 || MODE == 3 || MODE == 4 || MODE == 5);
-    constexpr bool SHIFTQ = FUSEQ && (MODE == 4 || MODE == 5);
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t l16 = lane & 15u, g = lane >> 4;
@@ -529,28 +398,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DEC
     // wavefront's k range (packed; expanded when used), the first tile's weights, the parameters of the outputs
     // this thread will finish
     v4u xp[MT][SEGS];
-    v4u raw[RPW][UPR];
-    const uint32_t nunits = p.K >> 3;
-    if constexpr (!FUSEQ) {
-        const __amdgpu_buffer_rsrc_t rX = make_rsrc(p.A, p.M * kbytes);  // rows past M read as zero
+    const __amdgpu_buffer_rsrc_t rX = make_rsrc(p.A, p.M * kbytes);  // rows past M read as zero
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int u = 0; u < SEGS; ++u)
-                xp[t][u] = buf_load16(rX, koff[u] != kOobOffset ? (t * 16 + l16) * kbytes + koff[u] : kOobOffset, 0);
-    } else {
-        // wavefront v quantizes rows v * RPW ..; lane l owns the 8-element units l, l + 64, ... of each
-        const __amdgpu_buffer_rsrc_t rX = make_rsrc(p.X, p.M * p.K * 2);  // rows past M read as zero
-#pragma unroll
-        for (int r = 0; r < RPW; ++r)
-#pragma unroll
-            for (int j = 0; j < UPR; ++j) {
-                const uint32_t c = lane + j * 64;
-                raw[r][j] = buf_load16(rX, c < nunits ? ((wave * RPW + r) * p.K + c * 8) * 2 : kOobOffset, 0);
-            }
-        // every wavefront requests its activations before any requests weights (requests are served in order)
-        __builtin_amdgcn_s_barrier();
-    }
+        for (int u = 0; u < SEGS; ++u)
+            xp[t][u] = buf_load16(rX, koff[u] != kOobOffset ? (t * 16 + l16) * kbytes + koff[u] : kOobOffset, 0);
     v4u w0[SEGS], w1[SEGS];
     load_tile(tile0, w0);
 
@@ -576,92 +429,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_s4_decode_kernel(DUQ_HEAD_DEC
 #pragma unroll
     for (int f = 0; f < FT; ++f) {
         rp[f] = RowRec{};
-        if (EPI >= 0 && finisher && !FUSEQ)
+        if (EPI >= 0 && finisher)
             rp[f] = load_row_rt<MODE>(p.epi, min((fg + f * NG) * 16 + my_m, p.M - 1), p.A, kbytes);
-    }
-
-    if constexpr (FUSEQ) {
-        // the quantizer's arguments, fetched under the vector loads above (a scalar load issued where its value is
-        // first used is waited for on its own)
-        const float q_clip = p.clip;
-        const int q_qmax = p.qmax;
-        uint8_t *const q_out = p.q_out;
-        uint16_t *const s_out = p.s_out, *const z_out = p.z_out;
-        int32_t *const rs_out = p.rs_out;
-        asm volatile("" ::"s"(q_clip), "s"(q_qmax), "s"(q_out), "s"(s_out), "s"(z_out), "s"(rs_out));
-        const bool copy_out = blockIdx.x == 0;
-#pragma unroll
-        for (int r = 0; r < RPW; ++r) {
-            const uint32_t qrow = wave * RPW + r;
-            // units past the row end read as zero: no maximum of |x| changes, a minimum or maximum would
-            PkMinMax st;
-#pragma unroll
-            for (int j = 0; j < UPR; ++j)
-                if (!ASYMQ || lane + j * 64 < nunits) st.add8(raw[r][j]);
-            uint32_t m16;
-            float lo = 0.f, hi = 0.f;
-            if (!ASYMQ) {
-                m16 = wave_max_u32(st.absmax_bits());
-            } else {
-                st.wave_reduce();
-                m16 = st.absmax_bits();
-                lo = st.min_f32();
-                hi = st.max_f32();
-                if (m16 > 0x7C00u) lo = hi = __builtin_nanf("");  // torch's min / max of a row that holds a NaN
-            }
-            if (qrow < p.M) {  // rows past M are neither quantized nor used
-                RowQuant<ASYMQ> rq;
-                rq.init(m16, lo, hi, q_clip, q_qmax);
-                int code_sum = 0;
-                uint32_t words[UPR];
-                quant_in_groups<DUQ_DEC_QUANT_GROUP>(rq, raw[r], words);
-#pragma unroll
-                for (int j = 0; j < UPR; ++j) {
-                    const uint32_t c = lane + j * 64;
-                    if (c < nunits) {
-                        uint32_t word = words[j];
-                        if (SHIFTQ) {
-                            const uint32_t pairs = (word & 0x0F0F0F0Fu) + ((word >> 4) & 0x0F0F0F0Fu);
-                            code_sum = (int)__builtin_amdgcn_udot4(pairs, 0x01010101u, (uint32_t)code_sum, false);
-                            word ^= 0x88888888u;  // u - 8 as a signed nibble
-                        }
-                        *reinterpret_cast<uint32_t *>(xs + qrow * XSTRIDE + c * 4) = word;
-                        if (copy_out && q_out) reinterpret_cast<uint32_t *>(q_out + (uint64_t)qrow * kbytes)[c] = word;
-                    }
-                }
-                if (SHIFTQ) code_sum = wave_sum_i32(code_sum) - 8 * (int)p.K;
-                if (lane == 0) {
-                    const f16 z = SHIFTQ ? rq.z - (f16)8.0f : rq.z;
-                    srow[qrow] = f16_to_bits(rq.s);
-                    if (ASYMQ) zrow[qrow] = f16_to_bits(z);
-                    if (SHIFTQ) rsrow[qrow] = code_sum;
-                    if (copy_out && s_out) s_out[qrow] = f16_to_bits(rq.s);
-                    if (ASYMQ && copy_out && z_out) z_out[qrow] = f16_to_bits(z);
-                    if (SHIFTQ && copy_out && rs_out) rs_out[qrow] = code_sum;
-                }
-            }
-        }
-        __syncthreads();
-        // (bytes past the row end, and rows past M, are never written: the weights read as zero there, and a row's
-        // codes only reach that row's outputs)
-#pragma unroll
-        for (int u = 0; u < SEGS; ++u)
-            xp[0][u] = koff[u] != kOobOffset ? load16(xs + l16 * XSTRIDE + koff[u]) : v4u{0, 0, 0, 0};
-        if (finisher) {
-            if constexpr (MODE == 5) {
-                const v2u head = *reinterpret_cast<const v2u *>(xs + my_m * XSTRIDE);
-                rp[0].xlo = head[0];
-                rp[0].xhi = head[1] & 0xFFu;
-                rp[0].zx = (uint32_t)rint_i32((float)bits_to_f16(zrow[my_m]));
-                rp[0].sx = (float)bits_to_f16(srow[my_m]);
-                rp[0].rxl = dual_head_sum(rp[0].xlo, rp[0].xhi);
-                rp[0].rxr = (uint32_t)rsrow[my_m] - rp[0].rxl;
-            } else {
-                rp[0].s = bits_to_f16(srow[my_m]);
-                if (ASYMQ) rp[0].z = bits_to_f16(zrow[my_m]);
-                if (SHIFTQ) rp[0].rs = rsrow[my_m];
-            }
-        }
     }
 
     auto compute_tile = [&](uint32_t tile, const v4u(&w)[SEGS], uint32_t buf) {
@@ -1078,7 +847,7 @@ bool launch_rows_mode(DecodeParams &p, int epi, hipStream_t stream)
     // wavefronts per workgroup: four, or with three or more rows to quantize WQ (DUQ_DEC_FUSEQ_WAVES above)
     constexpr int WQ = !FUSEQ || MR == 1 ? 4
                        : MR == 2         ? DUQ_DEC_FUSEQ_WAVES_M2
-                       : MR == 8         ? (XS >= 4 ? DUQ_DEC_FUSEQ_WAVES_M8L : DUQ_DEC_FUSEQ_WAVES)
+                       : MR == 8         ? DUQ_DEC_FUSEQ_WAVES
                                          : (XS >= 4 ? DUQ_DEC_FUSEQ_WAVES_M4L : DUQ_DEC_FUSEQ_WAVES_M4);
     constexpr int WMULTI = DUQ_DEC_FUSEQ_WAVES;
     bool launched = false;
@@ -1113,26 +882,23 @@ bool launch_rows_xs(DecodeParams &p, int epi, hipStream_t stream)
 {
     const uint32_t kbytes = p.K / 2;
     if (kbytes <= 2048) return launch_rows_mode<MR, 2, FUSEQ>(p, epi, stream);
-    if (kbytes <= 4096) return launch_rows_mode<MR, 4, FUSEQ>(p, epi, stream);
-    if constexpr (MR <= 4) {  // (eight rows: up to 8192 elements, decode_fp16in_one_launch)
+    if constexpr (MR <= 4) {  // (eight longer rows: quant_gemm_shape)
+        if (kbytes <= 4096) return launch_rows_mode<MR, 4, FUSEQ>(p, epi, stream);
         if (kbytes <= 6144) return launch_rows_mode<MR, 6, FUSEQ>(p, epi, stream);
         if (kbytes <= 8192) return launch_rows_mode<MR, 8, FUSEQ>(p, epi, stream);
     }
     return false;
 }
 
-template <int WAVES, int SEGS, int MT = 1, bool FUSEQ = false>
+template <int WAVES, int SEGS, int MT = 1>
 bool launch_mfma_mode(const DecodeParams &p, int epi, hipStream_t stream)
 {
     const uint32_t ntiles = (p.N + 15) / 16;
     const dim3 grid((ntiles + p.tiles_per_wg - 1) / p.tiles_per_wg);
 #define DUQ_DEC(E) \
-    DUQ_LAUNCH_HEAD((gemm_s4_decode_kernel<WAVES, SEGS, E, MT, FUSEQ>), grid, dim3(WAVES * 64), 0, stream, p)
+    DUQ_LAUNCH_HEAD((gemm_s4_decode_kernel<WAVES, SEGS, E, MT>), grid, dim3(WAVES * 64), 0, stream, p)
     switch (epi) {
-    case -1:
-        if constexpr (FUSEQ) return false;
-        else DUQ_DEC(-1);
-        break;
+    case -1: DUQ_DEC(-1); break;
     case 0: DUQ_DEC(0); break;
     case 1: DUQ_DEC(1); break;
     case 2: DUQ_DEC(2); break;
@@ -1155,15 +921,7 @@ bool launch_decode_any(DecodeParams &p, int epi, hipStream_t stream)
         return launch_rows_xs<4, FUSEQ>(p, epi, stream);
     }
     if constexpr (FUSEQ) {
-#ifndef DUQ_DEC_M8_MFMA
-        if (p.M <= 8) return launch_rows_xs<8, true>(p, epi, stream);  // 5..8 rows
-#endif
-        if (p.M > 16 || kbytes > 2048) return false;
-        // 9..16 rows: the MFMA kernel, rows quantized by every workgroup
-        constexpr int W = DUQ_DEC_MFMA_FUSEQ_WAVES;
-        p.tiles_per_wg = decode_tiles_per_workgroup((p.N + 15) / 16);
-        if (kbytes <= 1024) return launch_mfma_mode<W, 16 / W, 1, true>(p, epi, stream);
-        return launch_mfma_mode<W, 32 / W, 1, true>(p, epi, stream);
+        return p.M <= 8 && launch_rows_xs<8, true>(p, epi, stream);  // 5..8 rows on more columns than quant_gemm_shape has
     } else {
         const uint32_t ntiles = (p.N + 15) / 16;
         p.tiles_per_wg = decode_tiles_per_workgroup(ntiles);

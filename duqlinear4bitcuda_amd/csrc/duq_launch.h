@@ -257,23 +257,14 @@ inline uint32_t decode_tiles_per_workgroup(uint32_t ntiles) { return (ntiles + 2
 // output columns: every workgroup quantizes the rows again (4 rows: N = 28672 K = 8192 20.5 - 21.9 against 23.4 us,
 // N = 32000 K = 4096 12.6 against 14.1, N = 128256 K = 4096 41.3 against 42.4, but N = 20000 K = 16384 45.2 against
 // 36.3).
-// 9..16 rows: the MFMA kernel with sixteen wavefronts, one quantizing each row, while the rows together hold at most
-// 32768 elements, 40960 on at most 4096 columns (measured against two launches, N = 4096: 16 rows of 2048 4.9 against
-// 6.0 us, of 1024 4.1 against 5.3, 10 of 3072 5.9 against 6.3, 9 of 4096 6.2 against 6.5; 16 of 3072 6.45 either way,
-// 16 of 4096 7.2 against 6.55: each CU then spends 2 us of vector work and 0.85 us of fetching on the rows.  16 rows
-// of 2048: N = 8192 5.9 against 6.6, N = 16384 8.4 against 8.9; 10 of 4096 on N = 11008 9.3 either way, 13 of 3072
-// on N = 11008 9.0 against 8.6).
+// 9..16 rows: while the rows together hold at most 32768 elements, 40960 on at most 4096 columns (quant_gemm_shape).
+// This is the rule of the entry points that ask for no room for codes; quant_gemm_shape makes more shapes one launch, and takes
+// most of these from the rows kernel.
 inline bool decode_fp16in_one_launch(uint32_t M, uint32_t N, uint32_t K)
 {
     const int kernel = select_gemm_kernel(M, N, K);
     if (kernel == kKernelDecodeRows) return M == 1 || N <= 16384 || K <= 8192;
-#ifndef DUQ_DEC_FUSEQ16_ELEMS
-#define DUQ_DEC_FUSEQ16_ELEMS 32768u
-#define DUQ_DEC_FUSEQ16_ELEMS_NARROW 40960u
-#endif
-    if (M > 8)
-        return M <= 16 && K <= 4096 && M * K <= (N <= 4096 ? DUQ_DEC_FUSEQ16_ELEMS_NARROW : DUQ_DEC_FUSEQ16_ELEMS) && N <= 16384 &&
-               kernel == kKernelDecodeMfma;
+    if (M > 8) return M <= 16 && K <= 4096 && M * K <= (N <= 4096 ? 40960u : 32768u) && N <= 16384 && kernel == kKernelDecodeMfma;
     return M <= 8 && (K <= 4096 || (K <= 8192 && N <= 4096)) && kernel == kKernelDecodeMfma;
 }
 // decode kernels (duq_decode.hip); the shape must be one select_gemm_kernel gives to them
@@ -288,6 +279,56 @@ int launch_decode_s4(const uint8_t *A, const uint8_t *B, uint32_t M, uint32_t N,
 int launch_decode_fp16in(const uint16_t *x, float clip, int qmax, const uint8_t *B, uint32_t M, uint32_t N, uint32_t K,
                          const Epilogue &epi, uint16_t *y, uint8_t *q_out, uint16_t *s_out, uint16_t *z_out,
                          int32_t *rs_out, hipStream_t stream);
+
+// The same in workgroups that quantize the rows of their tile (duq_quant_gemm.hip): `rows` rows (8 of up to 8192 elements, 16 of 4096 or
+// 32 of 1024) and `chunks` times `cols` tiles of 16 columns.  rows = 0: not a shape of that kernel.
+struct QuantGemmShape {
+    uint32_t rows, cols, chunks;
+    bool eager_only = false;  // in a recording, where a launch costs the host nothing, two launches are level or ahead
+};
+// The cheapest of the tiles whose workgroups are one round of 256, by time fitted to one launch of each in a graph (base + per
+// 1024 elements of a row, us; mode 0, three tiles of columns 0.5 more than one), against quantizer launch and GEMM launch: a step of
+// two launches takes 8.2 us of host time and 4.7 of a graph's at least, and this kernel is 3.0 to 6.8.  Measured (N x K, graph, us):
+// 128 rows 1024 x 1024 5.5 -> 3.7, 512 x 1024 x 512 6.9 -> 4.0, 1000 x 1000 x 1024 9.8 -> 6.7, 32 x 4096 x 2048 5.8 -> 4.6, 16 x 28672 x
+// 2048 11.7 -> 8.0, 100 x 300 x 4096 5.5 -> 4.6, 128 x 4096 x 2048 8.0 -> 6.2.  Against the decode kernels' own quantizers: 8 x 4096 x
+// 4096 5.9 -> 4.8, 8 x 12000 x 1024 7.1 -> 4.5, 4 x 8192 x 2048 5.1 -> 4.1, 3 x 4096 x 4096 4.6 -> 4.1, but 2 x 4096 x 4096 3.7 against 4.1.
+// Sixteen rows of more than 2048 elements take two sets of registers one after the other, and groups of eight rows of more than 4096
+// twice as many registers: level in a graph, or behind (28 x 3136 x 3136 6.65 / 6.6, 75 x 1270 x 2560 6.1 / 6.6, 36 x 604 x 7680 7.7 / 7.9), so
+// that only the launch less decides (`eager_only`).  More than four chunks are behind (300 x 8000 x 512 8.7 against
+// 9.4 with five, 64 x 28672 x 512 12.7 against 8.2 with four).
+inline QuantGemmShape quant_gemm_shape(uint32_t M, uint32_t N, uint32_t K)
+{
+    QuantGemmShape best{0, 0, 0};
+    if (M < 3 || M > 2048 || N == 0 || N > 65536 || K == 0 || K > 8192) return best;
+    float best_us = 1e9f;
+    const float k = (float)K / 1024.0f;
+    auto offer = [&](uint32_t rows, uint32_t cols, uint32_t most_chunks, float us, float more_us) {
+        const uint32_t groups = (M + rows - 1) / rows, tiles = (N + 16 * cols - 1) / (16 * cols);
+        if (groups > 64 || groups * ((tiles + most_chunks - 1) / most_chunks) > 256) return;
+        const uint32_t per = 256 / groups, chunks = (tiles + per - 1) / per;  // (at most that many workgroups a group of rows)
+        if (chunks > most_chunks) return;
+        us += more_us * (float)(chunks - 1);
+        if (us < best_us) {
+            best_us = us;
+            best = QuantGemmShape{rows, cols, chunks, (rows == 16 && K > 2048) || (K > 4096 && M > 8)};
+        }
+    };
+    const float three[3] = {0.f, 0.12f, 0.6f};
+    for (uint32_t c = 1; c <= 3; ++c) {
+        if (K <= 4096) offer(8, c, 1, 3.0f + 0.45f * k + three[c - 1], 0.f);
+        if (K <= 2048) offer(16, c, 1, 3.0f + 0.6f * k + three[c - 1], 0.f);
+        else if (K <= 4096 && c > 1) offer(16, c, 1, 4.0f + 0.62f * k + three[c - 1], 0.f);
+    }
+    if (K > 4096) offer(8, 1, 1, 0.f, 0.f);
+    if (K <= 2048) offer(16, 8, 1, 3.4f + 1.25f * k, 0.f);
+    if (K <= 1024) offer(32, 4, 4, 3.2f + 1.6f * k, 0.9f + 1.1f * k);
+    if (K > 2048 && K <= 4096) offer(16, 1, 4, 4.0f + 0.62f * k, 1.0f);
+    return best;
+}
+// q_out / s_out / z_out / rs_out as above.
+int launch_quant_gemm(QuantGemmShape s, const uint16_t *x, float clip, int qmax, const uint8_t *B, uint32_t M, uint32_t N, uint32_t K,
+                      const Epilogue &epi, uint16_t *y, uint8_t *q_out, uint16_t *s_out, uint16_t *z_out, int32_t *rs_out,
+                      hipStream_t stream);
 
 // measurement aid: read `bytes` (< 4 GiB) with the decode kernels' access pattern and discard them
 int launch_probe_read(const void *src, uint64_t bytes, uint32_t *sink, hipStream_t stream);

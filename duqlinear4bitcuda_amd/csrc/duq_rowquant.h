@@ -90,7 +90,8 @@ struct RowQuant {
     int zi, qmax;
     bool fast, clamp_lo, clamp_hi;
     v2h lo2, hi2;
-    uint32_t zadd;
+    v2h base;       // what the packed path adds so that the sum is an integer: 1536, or (asym) 1552 and the even part of the zero point
+    uint32_t zodd;  // and what is then missing in every byte
 
     // sym: amax_bits = largest |x| bit pattern of the row (above 0x7C00: a NaN).
     // asym: mn / mx = the row's minimum / maximum as float (NaN when the row holds one).
@@ -183,24 +184,31 @@ struct RowQuant {
         }
         lo2 = ASYM ? v2h{(f16)(float)(-zi), (f16)(float)(-zi)} : v2h{(f16)-8.0f, (f16)-8.0f};
         hi2 = ASYM ? v2h{(f16)(float)(15 - zi), (f16)(float)(15 - zi)} : v2h{(f16)(float)qmax, (f16)(float)qmax};
-        zadd = ASYM ? (((uint32_t)zi & 0xFFFFu) * 0x00010001u) : 0u;
+        // (an odd number added before the rounding would turn ties the other way; 16 more keep a byte that is one short of its
+        // code from borrowing of the next one)
+        const f16 b16 = (f16)(float)(ASYM ? 1552 + (zi & ~1) : 1536);
+        base = v2h{b16, b16};
+        zodd = ASYM ? (uint32_t)(zi & 1) * 0x01010101u : 0u;
     }
 
     // 8 elements -> one packed word on the packed path (finite rows).  Per pair of binary16 values:
-    // h(float(x) * rcp) for both halves is one mixed-precision instruction each (binary16 source, float32
-    // arithmetic, binary16 result); clamp; add 1536, which leaves the codes in the low nibbles of bytes 0 and 2
-    // (the high nibbles of those bytes hold the sign extension); asym adds the zero point.  The four pairs go
+    // float(x) * rcp for either half is one mixed-precision instruction (binary16 source, float32 result), h of both a third
+    // (the forms with a binary16 result issue at half their rate: 16 x 11008 x 4096 quantized in the GEMM 7.5 -> 7.4 us, asymmetric
+    // 8.9 -> 8.5); clamp; add 1536, which leaves the codes in the low nibbles of bytes 0 and 2
+    // (the high nibbles of those bytes hold the sign extension); asym adds the zero point there too.  The four pairs go
     // through each stage together so that no instruction waits for the one before it.
     template <bool LO, bool HI>
     __device__ __forceinline__ uint32_t quant8_packed(const v4u raw) const
     {
         uint32_t d[4];
+        float lo[4], hi[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(d[i]) : "v"(rcp_fast), "v"(raw[i]));
+        for (int i = 0; i < 4; ++i) {
+            asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(lo[i]) : "v"(rcp_fast), "v"(raw[i]));
+            asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(hi[i]) : "v"(rcp_fast), "v"(raw[i]));
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            asm("v_fma_mixhi_f16 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "+v"(d[i]) : "v"(rcp_fast), "v"(raw[i]));
+        for (int i = 0; i < 4; ++i) asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(d[i]) : "v"(lo[i]), "v"(hi[i]));
         // written out: the generic minimum / maximum would first canonicalize the opaque results above, one
         // more instruction per pair that a finite row has no use for
         if (LO)
@@ -212,17 +220,17 @@ struct RowQuant {
         uint32_t b[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const v2h q = __builtin_bit_cast(v2h, d[i]) + v2h{(f16)1536.0f, (f16)1536.0f};
+            const v2h q = __builtin_bit_cast(v2h, d[i]) + base;
             b[i] = __builtin_bit_cast(uint32_t, q);
-            if (ASYM) {
-                const v2us sum = __builtin_bit_cast(v2us, b[i]) + __builtin_bit_cast(v2us, zadd);
-                b[i] = __builtin_bit_cast(uint32_t, sum);
-            }
         }
         // gather the code bytes (bytes 0 and 2 of every pair), then merge the low nibbles of neighbours into one
         // byte (a bit-field insert: low nibbles from p, high nibbles from p >> 4)
-        const uint32_t p0 = __builtin_amdgcn_perm(b[1], b[0], 0x06040200u);
-        const uint32_t p1 = __builtin_amdgcn_perm(b[3], b[2], 0x06040200u);
+        uint32_t p0 = __builtin_amdgcn_perm(b[1], b[0], 0x06040200u);
+        uint32_t p1 = __builtin_amdgcn_perm(b[3], b[2], 0x06040200u);
+        if (ASYM) {
+            p0 += zodd;
+            p1 += zodd;
+        }
         uint32_t t0, t1;
         const uint32_t low = 0x0F0F0F0Fu;
         asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(t0) : "s"(low), "v"(p0), "v"(p0 >> 4));
@@ -247,7 +255,15 @@ struct RowQuant {
         if (!fast) {
 #pragma unroll
             for (int j = 0; j < N; ++j) out[j] = quant8_exact<ASYM>(raw[j], rcp, qmax, zi);
-        } else if (!ASYM && clamp_lo) {
+        } else {
+            quant_units_packed(raw, out);
+        }
+    }
+    // (for rows with `fast`)
+    template <int N>
+    __device__ __forceinline__ void quant_units_packed(const v4u (&raw)[N], uint32_t (&out)[N]) const
+    {
+        if (!ASYM && clamp_lo) {
 #pragma unroll
             for (int j = 0; j < N; ++j) out[j] = quant8_packed<true, true>(raw[j]);
         } else if (clamp_hi) {

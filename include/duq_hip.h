@@ -234,6 +234,10 @@ int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
  * where the fused entry points cover the last columns of a problem in smaller tiles, behind tiles of 128 x 256 or 256 x 256); 0 for the other kernels.  (The dual-uniform row-sum
  * epilogue never runs the 256-row tile.) */
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
+/* The tile of the one kernel that runs duq_quantize_linear4bit_forward (and its relatives) for a shape: rows of a workgroup + 256 * tiles
+ * of 16 columns + 65536 * chunks of those, + 2^24 where a call that is being recorded into a graph runs two launches instead.  0:
+ * the rows kernel that quantizes for itself (up to eight rows), or two launches. */
+int duq_quant_gemm_tile_for(uint32_t M, uint32_t N, uint32_t K);
 /* The tiles of a launch of the prefill kernel: mode DUQ_EPI_* (binary16 outputs) or -1 (int32 outputs, duq_matmul_host_4bit);
  * plan = rows and columns of a tile, and where plan[2] > 0 the column up to which these reach, with the rows and columns of the
  * tiles behind it.  All zero for shapes that other kernels run.  (No GPU work; for tests and tuning.) */

@@ -1,0 +1,134 @@
+"""The kernel that quantizes its rows, multiplies and dequantizes (``csrc/duq_quant_gemm.hip``): the oracle's bits at the edges of
+its tiles, what it hands out of its quantizer, and the rule that picks its tile."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import duq_oracle as orc
+from tests import cases
+from tests.test_gpu_random_shapes import hip, test_random_shapes_fp16_input as _against_the_oracle  # noqa: F401 (fixture)
+
+
+def _tile(M, N, K):
+    from duqlinear4bitcuda_amd import _lib
+
+    t = _lib.load().duq_quant_gemm_tile_for(M, N, K)
+    return t & 255, t >> 8 & 255, t >> 16 & 255
+
+
+# tile (rows, column tiles, chunks), then shapes at its edges: one row in the last group, one column in the last tile, short rows,
+# rows that end inside a slice, the longest rows
+EDGES = {
+    (8, 1, 1): [(3, 1, 64), (8, 4096, 4096), (9, 17, 2112), (17, 1024, 3136), (5, 4096, 8192), (6, 33, 4160), (250, 100, 4032)],
+    (8, 2, 1): [(8, 8190, 3072), (65, 700, 4096), (120, 500, 2560)],
+    (8, 3, 1): [(8, 12288, 4096), (3, 9000, 2112), (24, 4000, 3072)],
+    (16, 1, 1): [(500, 100, 64), (513, 110, 1088), (1000, 50, 1984)],
+    (16, 2, 1): [(16, 8192, 64), (130, 777, 960), (33, 2700, 2048)],
+    (16, 3, 1): [(40, 4000, 2048), (33, 4000, 1984)],
+    (16, 8, 1): [(16, 30000, 2048), (64, 8100, 2048), (100, 4200, 1984)],
+    (32, 4, 1): [(512, 1024, 512), (500, 1023, 576), (60, 8190, 512), (2000, 17, 576)],
+    (32, 4, 2): [(500, 2001, 960), (1000, 1000, 1024), (40, 16001, 64)],
+    (32, 4, 3): [(200, 6002, 512)],
+    (32, 4, 4): [(64, 30003, 512)],
+}
+LONG = {  # two sets of registers one after the other
+    (16, 2, 1): [(32, 4000, 4032)],
+    (16, 3, 1): [(13, 12287, 3072)],
+    (16, 1, 4): [(9, 16383, 4096)],
+}
+SHAPES = [(t, s) for edges in (EDGES, LONG) for t, shapes in edges.items() for s in shapes]
+
+
+@pytest.mark.parametrize("tile,shape", SHAPES)
+def test_shapes_reach_their_tile(tile, shape):
+    assert _tile(*shape) == tile
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("i", range(len(SHAPES)))
+def test_tiles_against_the_oracle(hip, dev, i):  # noqa: F811
+    M, N, K = SHAPES[i][1]
+    for mode in (i % 6, (i + 3) % 6):   # a symmetric and an asymmetric epilogue
+        _against_the_oracle(hip, dev, M, N, K, mode)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(20, 40, 2112), (33, 2700, 2048), (500, 2001, 960), (40, 4000, 4096)])
+def test_rows_that_are_not_finite_beside_rows_that_are(hip, dev, M, N, K):  # noqa: F811
+    """A wavefront holds several rows: a zero row, an infinity and a NaN among them, and a scale that underflows."""
+    x = cases.acts_outliers(M, K, seed=M)
+    x[1], x[4, 3], x[6, K - 1], x[9] = 0, np.inf, np.nan, np.float16(6e-8)
+    x[11] = -x[11]
+    wq, sw = cases.weights_random_nibbles(N, K, seed=3)
+    with np.errstate(all="ignore"):
+        want = orc.linear4bit_sq_forward(x, wq, sw)[0]
+    got = hip.quantize_linear4bit_forward(cases.t(x, dev), cases.t(wq, dev), cases.t(sw, dev))
+    assert cases.bits_equal(got.cpu().numpy(), want)
+    u = cases.acts_uniform(M, K, seed=M + 1)
+    u[1], u[4, 3], u[6, K - 1], u[9], u[11] = 0, np.inf, np.nan, 3, -u[11]
+    w = (np.random.default_rng(M).standard_normal((N, K)) * 0.02).astype(np.float16)
+    wq, sw, zw, adj = orc.weight_asym_shifted_from_linear(w)
+    with np.errstate(all="ignore"):
+        want = orc.linear4bit_asq_rowsum_forward(u, wq, sw, zw, adj)[0]
+    got = hip.quantize_linear4bit_forward_asym(hip.EPI_ASYM_ROWSUM, cases.t(u, dev), cases.t(wq, dev), cases.t(sw, dev),
+                                               cases.t(zw, dev), None, None, cases.t(adj, dev))
+    assert cases.bits_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(13, 3000, 2048), (37, 500, 960), (100, 5000, 768), (9, 16384, 2560), (21, 600, 4096), (7, 4096, 6208)])
+def test_codes_and_parameters_of_the_rows(hip, dev, M, N, K):  # noqa: F811
+    """What the caller may ask for of the quantizer: the stand-alone quantizer's bits, whatever the launch."""
+    T = lambda v: cases.t(v, dev)
+    wq, sw = cases.weights_random_nibbles(N, K, seed=5)
+    x = T(cases.acts_outliers(M, K, seed=M))
+    y, q, s = hip.quantize_linear4bit_forward(x, T(wq), T(sw), return_quantized=True)
+    q0, s0 = hip.quantize_rows_sym(x)[:2]
+    assert torch.equal(q, q0) and torch.equal(s, s0)
+    assert torch.equal(y, hip.linear4bit_forward(hip.EPI_SYM, q0, s0, None, T(wq), T(sw)))
+    x, adj = T(cases.acts_uniform(M, K, seed=M)), torch.zeros(N, dtype=torch.int32, device=dev)
+    y, q, s, z, r = hip.quantize_linear4bit_forward_asym(hip.EPI_ASYM_ROWSUM, x, T(wq), T(sw), T(sw), None, None, adj, return_quantized=True)
+    for got, want in zip((q, s, z, r), hip.quantize_rows_asym_shifted(x)):
+        assert torch.equal(got.flatten(), want.flatten())
+
+
+def test_every_shape_without_room_for_codes_has_its_kernel():
+    """Callers bring no workspace for these, so there are no two launches to fall back to: up to eight rows of up to 4096
+    elements the rows kernel, everything else a tile of this one."""
+    from duqlinear4bitcuda_amd import _lib
+
+    lib = _lib.load()
+    rng = np.random.default_rng(8)
+    seen = 0
+    for M in range(3, 17):
+        for K in [64, 1024, 1088, 2048, 2112, 2496, 2560, 3072, 3136, 3584, 4096, 4160, 8192] + list(64 * rng.integers(1, 129, 12)):
+            for N in [1, 16, 4096, 4097, 8192, 12288, 12289, 16384, 16385] + list(rng.integers(1, 40000, 12)):
+                M, N, K = int(M), int(N), int(K)
+                if lib.duq_quantize_linear4bit_workspace_bytes(M, N, K) or (M <= 4 or (M <= 8 and K <= 4096)):
+                    continue
+                seen += 1
+                assert _tile(M, N, K)[0], (M, N, K)
+    assert seen > 500
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,launches", [(32, 4000, 4032, 2), (40, 600, 3008, 1), (36, 604, 7680, 2), (48, 1024, 1024, 1)])
+def test_recorded_calls(hip, dev, M, N, K, launches):  # noqa: F811
+    """Replays of a recording, where a launch less counts for less, give the eager call's bits."""
+    from duqlinear4bitcuda_amd import _lib
+
+    assert 1 + (_lib.load().duq_quant_gemm_tile_for(M, N, K) >> 24) == launches
+    T = lambda v: cases.t(v, dev)
+    wq, sw = cases.weights_random_nibbles(N, K, seed=7)
+    wq, sw = T(wq), T(sw)
+    x = T(cases.acts_outliers(M, K, seed=M))
+    want = hip.quantize_linear4bit_forward(x, wq, sw)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = hip.quantize_linear4bit_forward(x, wq, sw)
+    for _ in range(3):
+        got.fill_(0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
