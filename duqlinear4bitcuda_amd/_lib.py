@@ -53,6 +53,7 @@ PROTOTYPES = {
     "duq_quant_gemm_tile_for": [_c_u32, _c_u32, _c_u32],
     "duq_gemm_plan_for": [_c_i32, _c_u32, _c_u32, _c_u32, _c_p],
     "duq_gemm_bf6_plan_for": [_c_i32, _c_u32, _c_u32, _c_u32, _c_p],
+    "duq_quant_gemm8_tile_for": [_c_u32, _c_u32, _c_u32],
     "duq_gemm8_kernel_for": [_c_u32, _c_u32, _c_u32, _c_i32],
     "duq_probe_read": [_c_p, ctypes.c_uint64, _c_p, _c_p],
     "duq_quantize_linear4bit_workspace_bytes": [_c_u32, _c_u32, _c_u32],  # returns uint64_t (restype set in load())

@@ -874,6 +874,12 @@ int duq_linear8bit_forward_tiled(const int8_t *xq, const float *scale_x, const f
                                as_stream(stream));
 }
 
+int duq_quant_gemm8_tile_for(uint32_t M, uint32_t N, uint32_t K)
+{
+    const duq::QuantGemmShape t = duq::quant_gemm8_shape(M, N, K);
+    return (int)(t.rows + 256 * t.cols + 65536 * t.chunks);
+}
+
 int duq_gemm8_kernel_for(uint32_t M, uint32_t N, uint32_t K, int32_t tiled)
 {
     if (M == 0 || N == 0 || K == 0) return 0;
@@ -904,11 +910,12 @@ int duq_quantize_linear8bit_forward(const float *x, const int8_t *w, const int8_
     if (int e = check_gemm8(q, weight, M, N, K)) return e;
     if (!w_scale || !w_zeros || !y) return DUQ_E_NULL;
     if (!aligned(y, 4)) return DUQ_E_ALIGN;
-    if (duq::quantize_gemm8_fuses(M, N, K)) {
-        // (up to four rows, where `weight` is w: a copy that is not aligned is no reason to refuse the call, only not to read it)
-        const bool copy = w_tiled && aligned(w_tiled, 16);
+    // (up to four rows, where `weight` is w: a copy that is not aligned is no reason to refuse the call, only not to read it)
+    const bool copy = w_tiled && aligned(w_tiled, 16);
+    if (const duq::QuantGemmShape t = duq::quant_gemm8_shape(M, N, K); t.rows)
+        return duq::launch_quant_gemm8(t, x, copy ? w_tiled : w, copy, M, N, K, w_scale, w_zeros, bias, y, as_stream(stream));
+    if (duq::quantize_gemm8_fuses(M, N, K))
         return duq::launch_quantize_gemm_s8(x, copy ? w_tiled : w, copy, M, N, K, w_scale, w_zeros, bias, y, as_stream(stream));
-    }
     if (int e = duq::launch_quantize_rows_asym8(x, M, K, q, sx, zx, as_stream(stream))) return e;
     return duq::launch_gemm_s8(q, weight, tiled, M, N, K, nullptr, sx, zx, w_scale, w_zeros, bias, y, as_stream(stream));
 }

@@ -133,6 +133,21 @@ __device__ __forceinline__ uint32_t group_reduce(uint32_t v, OP op)
     if (N >= 64) v = op(v, (uint32_t)__shfl_xor((int)v, 32, kWave));
     return v;
 }
+// The same without a trip through the LDS crossbar, N = 8 to 64.
+template <int N, typename OP>
+__device__ __forceinline__ uint32_t lanes_reduce(uint32_t v, OP op)
+{
+    v = group_reduce<(N < 16 ? N : 16)>(v, op);
+    if (N >= 32) {  // rows of sixteen lanes change places: 0 1 2 3 -> 0 0 2 2 and 1 1 3 3
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        v = op(r[0], r[1]);
+    }
+    if (N >= 64) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        v = op(r[0], r[1]);
+    }
+    return v;
+}
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
 {
     return wave_reduce_dpp(v, [](uint32_t x, uint32_t y) { return max(x, y); });

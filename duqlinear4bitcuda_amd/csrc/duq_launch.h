@@ -365,6 +365,45 @@ int launch_quantize_rows_asym8(const float *x, uint32_t rows, uint32_t cols, int
 bool quantize_gemm8_fuses(uint32_t M, uint32_t N, uint32_t K);
 int launch_quantize_gemm_s8(const float *x, const int8_t *B, bool b_tiled, uint32_t M, uint32_t N, uint32_t K, const float *s_col,
                             const float *z_col, const float *bias, float *y, hipStream_t stream);
+// the same in workgroups that quantize the rows of their tile (duq_quant_gemm8.hip): `rows` rows (8 of up to 4096 elements, 16 of 2048, 32
+// of 1024) and `chunks` times `cols` tiles of 16 columns.  The cheapest tile whose workgroups are one round, by times fitted to
+// launches of each in a graph, as quant_gemm_shape; against two launches (5.0 us of a graph at least, 8.2 of host time) or, up to
+// eight rows, the decode kernel's own quantizer (N x K, tiled copy, us): 64 rows 1024 x 1024 5.1 -> 3.7, 512 x 1024 x 512 7.1 -> 4.3, 73 x
+// 4359 x 896 10.0 -> 5.6, 16 x 11008 x 1024 7.9 -> 4.7, 32 x 4096 x 2048 7.2 -> 5.5, 78 x 310 x 3296 6.3 -> 5.2, 256 x 2048 x 1024 7.6 -> 5.9, 1000 x
+// 1000 x 512 8.7 -> 6.4; 8 x 4096 x 4096 6.8 -> 5.6, 4 rows 6.2 -> 5.7, but two 5.67 against 5.80.
+inline QuantGemmShape quant_gemm8_shape(uint32_t M, uint32_t N, uint32_t K)
+{
+    QuantGemmShape best{0, 0, 0};
+    if (M < 3 || M > 2048 || N == 0 || N > 65536 || K == 0 || K > 4096) return best;
+    float best_us = 1e9f;
+    const float k = (float)K / 1024.0f;
+    auto offer = [&](uint32_t rows, uint32_t cols, uint32_t most_chunks, float us) {
+        const uint32_t groups = (M + rows - 1) / rows, tiles = (N + 16 * cols - 1) / (16 * cols);
+        if (groups > 64 || groups * ((tiles + most_chunks - 1) / most_chunks) > 256) return;
+        const uint32_t per = 256 / groups, chunks = (tiles + per - 1) / per;  // (at most that many workgroups a group of rows)
+        if (chunks > most_chunks) return;
+        us += 2.1f * (float)(chunks - 1);
+        if (us < best_us) {
+            best_us = us;
+            best = QuantGemmShape{rows, cols, chunks};
+        }
+    };
+    offer(8, 1, 1, 2.8f + 0.7f * k);
+    if (K <= 2048) {
+        offer(8, 2, 1, 3.4f + 0.7f * k);
+        offer(8, 3, 1, 4.3f + 0.7f * k);
+        offer(16, 1, 1, 2.5f + 1.2f * k);
+        offer(16, 2, 1, 2.6f + 1.2f * k);
+        offer(16, 3, 1, 2.7f + 1.7f * k);
+    }
+    if (K <= 1024) {
+        offer(16, 8, 1, 3.3f + 3.4f * k);
+        offer(32, 4, K <= 512 ? 2 : 1, 3.2f + 2.7f * k);
+    }
+    return best;
+}
+int launch_quant_gemm8(QuantGemmShape s, const float *x, const int8_t *B, bool b_tiled, uint32_t M, uint32_t N, uint32_t K, const float *s_col,
+                       const float *z_col, const float *bias, float *y, hipStream_t stream);
 int launch_dequant_hprec(const int32_t *acc, const float *s_row, const float *z_row, const float *s_col,
                          const float *z_col, const float *bias, uint32_t rows, uint32_t cols, float *x,
                          hipStream_t stream);

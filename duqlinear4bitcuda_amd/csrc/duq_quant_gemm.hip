@@ -47,22 +47,6 @@ struct QuantTile {
     static_assert(kX + BUFS * kW + kPart <= 159 * 1024, "LDS");
 };
 
-// The same value in the lanes of a group of N, N = 8 to 64.
-template <int N, typename OP>
-__device__ __forceinline__ uint32_t lanes_reduce(uint32_t v, OP op)
-{
-    v = group_reduce<(N < 16 ? N : 16)>(v, op);
-    if (N >= 32) {  // rows of sixteen lanes change places: 0 1 2 3 -> 0 0 2 2 and 1 1 3 3
-        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-        v = op(r[0], r[1]);
-    }
-    if (N >= 64) {
-        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-        v = op(r[0], r[1]);
-    }
-    return v;
-}
-
 // Eight wavefronts quantize and then multiply, four others only fetch the weights (a wavefront's wait for its activations would
 // otherwise be a wait for the weights it requested too).  Sums as in the other decode kernels: the wavefronts split K, eight
 // partial tiles meet in LDS.  A workgroup takes p.chunks times NT column tiles, with BUFS = 2 the next ones' weights on their way

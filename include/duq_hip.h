@@ -505,6 +505,8 @@ int duq_linear8bit_forward_tiled(const int8_t *xq, const float *scale_x, const f
  * shape (no GPU work; for tests and tuning): 1 rows kernel, 2 decode kernel, 3 LDS kernel, 4 skinny kernel, 5 split kernel, 6
  * prefill tiles; 0 for an empty problem.  No counterpart in the reference. */
 int duq_gemm8_kernel_for(uint32_t M, uint32_t N, uint32_t K, int32_t tiled);
+/* The tile of the one kernel that runs duq_quantize_linear8bit_forward for a shape, as duq_quant_gemm_tile_for; 0: another one. */
+int duq_quant_gemm8_tile_for(uint32_t M, uint32_t N, uint32_t K);
 
 /* No counterpart in the reference: LinearQuant8bitASQ.forward with its own quantizer (qlinear4bit/nn/linear.py:323-335)
  * in one call: duq_quantize_rows_asym_8bit into `workspace`, then duq_linear8bit_forward(_tiled) on it; the same
