@@ -349,6 +349,37 @@ int duq_linear4bit_forward(int32_t mode, const uint8_t *xq, const duq_half *scal
     return duq::launch_gemm_s4(xq, w, M, N, K, nullptr, &e, y, as_stream(stream));
 }
 
+uint64_t duq_linear4bit_room_bytes(int32_t mode, uint32_t M, uint32_t N, uint32_t K)
+{
+    if (mode < DUQ_EPI_SYM || mode > DUQ_EPI_ASYM_ROWSUM || M > (1u << 24) || N > (1u << 22) || K > 131008u || K % 64 != 0 ||
+        !duq::pays_shadows(M, N, K))
+        return 0;
+    const uint64_t bytes = duq::shadows_bytes(M, N, K);
+    return bytes <= 0x80000000ull ? bytes : 0;
+}
+
+int duq_linear4bit_forward_room(int32_t mode, const uint8_t *xq, const duq_half *scale_x, const duq_half *zeros_x,
+                                const int32_t *rowsum_x, const uint8_t *w, const duq_half *w_scale_1, const duq_half *w_zeros_1,
+                                const duq_half *w_scale_2, const duq_half *w_zeros_2, const int32_t *w_rowsum_adj,
+                                const duq_half *bias, uint32_t M, uint32_t N, uint32_t K, duq_half *y, void *room,
+                                uint64_t room_bytes, duq_stream_t stream)
+{
+    if (mode < DUQ_EPI_SYM || mode > DUQ_EPI_ASYM_ROWSUM) return DUQ_E_MODE;
+    if (int e = check_gemm(xq, w, M, N, K)) return e;
+    if (M == 0 || N == 0) return DUQ_OK;
+    const bool asym = mode == DUQ_EPI_ASYM || mode == DUQ_EPI_ASYM_DUAL || mode == DUQ_EPI_ASYM_ROWSUM;
+    const bool dual = mode == DUQ_EPI_SYM_DUAL || mode == DUQ_EPI_ASYM_DUAL;
+    if (!scale_x || !w_scale_1 || !y || (asym && (!zeros_x || !w_zeros_1)) || (dual && (!w_scale_2 || (asym && !w_zeros_2))) ||
+        (mode == DUQ_EPI_ASYM_ROWSUM && (!rowsum_x || !w_rowsum_adj)))
+        return DUQ_E_NULL;
+    duq::Epilogue e{mode, scale_x, zeros_x, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias, rowsum_x, w_rowsum_adj};
+    const uint64_t need = duq_linear4bit_room_bytes(mode, M, N, K);
+    if (need == 0 || !room) return duq::launch_gemm_s4(xq, w, M, N, K, nullptr, &e, y, as_stream(stream));
+    if (room_bytes < need) return DUQ_E_SHAPE;
+    if (!aligned(room, 16)) return DUQ_E_ALIGN;
+    return duq::launch_gemm_via_shadows(xq, w, M, N, K, e, y, static_cast<uint8_t *>(room), as_stream(stream));
+}
+
 // One launch holds at most 65535 batch entries (grid limit of the second and third dimension): longer batches
 // run in slices, every tensor moved on by whole entries.
 constexpr uint32_t kBatchSlice = 65535;

@@ -20,7 +20,7 @@
 //                      kernel pins (mfma_pinned) so that the loads write them in place: three memory
 //                      instructions per two fragments instead of four (a 128-bit and a 64-bit load per
 //                      fragment), without a register move.  An odd last tile is paired with zeros.
-// K % 128 == 0 and N % 16 == 0.
+// K % 128 == 0; parameter arrays as long as whole quads of columns, N % 16 == 0 where epilogue 5 reads its heads.
 //
 // Kernel: tile 128 (M) x 256 (N) per workgroup, 4 wavefronts side by side along N (128 x 64
 // each: 8 x 4 MFMA tiles, 128 accumulator registers).  Weights go global -> registers (a ring
@@ -57,16 +57,20 @@ typedef _Float16 v32h __attribute__((ext_vector_type(32)));
 // 32 signed nibbles (16 bytes, element 2j in the low nibble of byte j) -> one bf6 block.
 // Position 8d + 2i + h of the block holds nibble i + 4h of word d (the order the quantizer
 // kernels produce cheaply); both operands use it, and the sum over k does not care.
+// A pair of positions (2i, 2i + 1) is one shift and one mask of the word: the nibbles' upper bits turned, they are the
+// binary16 numbers 1024 + 8 + code, and a packed subtraction leaves the code.
 __device__ __forceinline__ v6i bf6_block_from_nibbles(const v4u w)
 {
-    v32h f;
+    typedef uint32_t v16u __attribute__((ext_vector_type(16)));
+    v16u f;
 #pragma unroll
-    for (int pos = 0; pos < 32; ++pos) {
-        const int d = pos >> 3, e = ((pos & 7) >> 1) + 4 * (pos & 1);
-        const int v = ((int)(w[d] << (28 - 4 * e))) >> 28;
-        f[pos] = (f16)(float)v;
+    for (int d = 0; d < 4; ++d) {
+        const uint32_t u = w[d] ^ 0x88888888u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            f[4 * d + i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, ((u >> (4 * i)) & 0x000F000Fu) | 0x64006400u) - v2h{(f16)1032.0f, (f16)1032.0f});
     }
-    return __builtin_bit_cast(v6i, __builtin_amdgcn_cvt_scalef32_pk32_bf6_f16(f, 1.0f));
+    return __builtin_bit_cast(v6i, __builtin_amdgcn_cvt_scalef32_pk32_bf6_f16(__builtin_bit_cast(v32h, f), 1.0f));
 }
 
 // Layout: for every pair of 16-row tiles and every 128-k step, 3072 bytes.  Lane l = (row l % 16, k-block l / 16) owns
@@ -129,6 +133,57 @@ int launch_activation_shadow_bf6(const uint8_t *q, uint32_t M, uint32_t K, uint8
     const uint32_t blocks = (uint32_t)std::min<uint64_t>((total + 255) / 256, 1u << 16);
     hipLaunchKernelGGL(activation_shadow_kernel, dim3(blocks), dim3(256), 0, stream, q, M, K, out);
     return (int)hipGetLastError();
+}
+
+// Shadows of both operands of one product in one launch, for a call that comes without any (launch_gemm_via_shadows): a thread a
+// block of 32 codes of an activation row, or the two blocks of a lane of the weight shadow.  Columns past K (up to a multiple of 128)
+// and weight rows past N are zeros.  Behind them the column parameters, padded to a multiple of 16, where the GEMM cannot read them
+// in place.  Bound by memory, half a byte in and three quarters out per code: 4096 x 28672 x 8192 some 50 us at 6.7 TB/s of both.
+struct ShadowsParams {
+    const uint8_t *x, *w;
+    uint8_t *X, *W;
+    uint32_t M, N, K;
+    uint32_t blocks_w, blocks_x;    // workgroups of either part; the rest copies parameters
+    const uint16_t *par[5];         // s1, z1, s2, z2, bias (nullptr: not used), and the sums of epilogue 4
+    const int32_t *sums;
+    uint16_t *par_out;              // [5][N up to a multiple of 16], sums behind them
+};
+
+__global__ __launch_bounds__(256) void shadows_kernel(ShadowsParams p)
+{
+    const uint32_t ksteps = (p.K + 127) / 128, kblocks = p.K / 32, kbytes = p.K / 2;
+    const v4u none = v4u{0u, 0u, 0u, 0u};
+    if (blockIdx.x < p.blocks_w) {
+        const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x, ps = i >> 6;  // pair * ksteps + step
+        const uint32_t lane = (uint32_t)(i & 63u), step = (uint32_t)(ps % ksteps), pair = (uint32_t)(ps / ksteps);
+        const uint32_t kb = step * 4 + (lane >> 4), n = pair * 32 + (lane & 15u);
+        if (pair * 32 >= p.N) return;
+        v4u raw[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            raw[h] = n + 16 * h < p.N && kb < kblocks ? *reinterpret_cast<const v4u *>(p.w + (uint64_t)(n + 16 * h) * kbytes + kb * 16) : none;
+        const v6i f0 = bf6_block_from_nibbles(raw[0]), f1 = bf6_block_from_nibbles(raw[1]);
+        uint8_t *dst = p.W + ps * 3072 + lane * 16;
+        *reinterpret_cast<v4i *>(dst) = v4i{f0[0], f0[1], f0[2], f0[3]};
+        *reinterpret_cast<v4i *>(dst + 1024) = v4i{f0[4], f0[5], f1[0], f1[1]};
+        *reinterpret_cast<v4i *>(dst + 2048) = v4i{f1[2], f1[3], f1[4], f1[5]};
+    } else if (blockIdx.x < p.blocks_w + p.blocks_x) {
+        const uint64_t i = (uint64_t)(blockIdx.x - p.blocks_w) * 256 + threadIdx.x;
+        const uint32_t nblk = ksteps * 4, kb = (uint32_t)(i % nblk);
+        const uint64_t m = i / nblk;
+        if (m >= p.M) return;
+        const v6i f = bf6_block_from_nibbles(kb < kblocks ? *reinterpret_cast<const v4u *>(p.x + m * kbytes + kb * 16) : none);
+        uint8_t *row = p.X + m * nblk * 24;
+        *reinterpret_cast<v4i *>(row + kb * 16) = v4i{f[0], f[1], f[2], f[3]};
+        *reinterpret_cast<v2i *>(row + (uint64_t)nblk * 16 + kb * 8) = v2i{f[4], f[5]};
+    } else {
+        const uint32_t n = (blockIdx.x - p.blocks_w - p.blocks_x) * 256 + threadIdx.x, padded = (p.N + 15) & ~15u;
+        if (n >= padded) return;
+#pragma unroll
+        for (int k = 0; k < 5; ++k)
+            if (p.par[k]) p.par_out[k * (uint64_t)padded + n] = n < p.N ? p.par[k][n] : (uint16_t)0;
+        if (p.sums) reinterpret_cast<int32_t *>(p.par_out + 5 * (uint64_t)padded)[n] = n < p.N ? p.sums[n] : 0;
+    }
 }
 
 // ---------------------------------------------------------------------------------
@@ -306,7 +361,8 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
     const uint32_t ksteps = p.K / 128;
     const uint32_t nchunks = (ksteps + CH - 1) / CH;
 
-    const uint32_t wpairs = (min(p.N - n0, (uint32_t)BN) / 16 + 1) / 2;  // pairs of 16-row weight tiles in this tile
+    const uint32_t last_quad = ((p.N + 3) & ~3u) - 4;  // (parameter arrays are as long as whole quads of columns)
+    const uint32_t wpairs = (min(p.N - n0, (uint32_t)BN) + 31) / 32;  // pairs of 16-row weight tiles in this tile
     const __amdgpu_buffer_rsrc_t rW =
         make_rsrc(p.W + (uint64_t)(n0 / 32) * ksteps * 3072, wpairs * ksteps * 3072);
     const __amdgpu_buffer_rsrc_t rNone = make_rsrc(p.X, 0);  // every read returns zero
@@ -446,7 +502,7 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
         for (int mi = 0; mi < TMI; ++mi) rowp[mi] = load_row<MODE == 5 ? 0 : MODE>(e, min(m0 + mi * 16 + l16, p.M - 1));
 #pragma unroll
         for (int ni = 0; ni < TNI; ++ni) {
-            const uint32_t nq = min(n0 + wave * (16 * TNI) + ni * 16 + kb * 4, p.N - 4);
+            const uint32_t nq = min(n0 + wave * (16 * TNI) + ni * 16 + kb * 4, last_quad);
             raw_s1[ni] = *reinterpret_cast<const v2u *>(e.s_col_1 + nq);
             if (MODE == 1 || MODE == 3 || MODE == 4) raw_z1[ni] = *reinterpret_cast<const v2u *>(e.z_col_1 + nq);
             if (MODE == 4) raw_rs[ni] = *reinterpret_cast<const v4i *>(e.rs_col + nq);
@@ -592,7 +648,7 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
 #pragma unroll
     for (int ni = 0; ni < TNI; ++ni) {
         const uint32_t ncol = ni * 16 + kb * 4;
-        const uint32_t nq = min(n0 + wave * (16 * TNI) + ncol, p.N - 4);
+        const uint32_t nq = min(n0 + wave * (16 * TNI) + ncol, last_quad);
         PairCols<MODE, BIAS> cols[2];
 #pragma unroll
         for (int k = 0; k < 2; ++k)
@@ -619,6 +675,14 @@ __device__ __forceinline__ void bf6_tile(const Bf6Params &p, uint8_t *lds, uint3
             __builtin_amdgcn_raw_buffer_store_b128(v, rY, (int)off, 0, decltype(streamed)::value ? 2 : 0);
         }
     };
+    // (rows that are not 16-byte aligned: the same pieces at whatever alignment they have, the last one element by element)
+    if (p.N % 8 != 0 || reinterpret_cast<uintptr_t>(p.y) % 16 != 0) {
+        for (uint32_t row = rsub; row < rows_here; row += RPI) {
+            const v4u v = *reinterpret_cast<const v4u *>(stage + row * kYStride + piece * 16);
+            store_row_piece(p.y + (uint64_t)(m0 + row) * p.N + ncol0, v, p.N - min(ncol0, p.N));
+        }
+        return;
+    }
     // (rows that begin at half lines are streamed too.  75 shapes of 17 to 110 Mi outputs, 640 to 4096 elements: 1 % ahead in the
     // geometric mean with one weight and one output, 2 % with three weights, 7 % with three of both in turn; 4096 x 28640 x 4096 267
     // against 288 us, 2000 x 28320 x 1280 27 % with three of both; the most lost 6 %, 1000 x 28320 x 640 and 3000 x 9056 x 1280)
@@ -717,6 +781,7 @@ Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
     // CUs left without a 64 x 256 tile: 64 x 128 tiles, twice as many, as long as they still run in one round
     // (measured: 23-35 % faster up to 128 tiles of 64 x 256, slower from 160 on)
     if (best.rows == 64 && tiles(0, tn) <= 128) best.width = 128;
+    best.us = least;
     if (mode5) return best;
     least *= 0.96f;
     // (whole rounds of 256 rows only: a round of 128-row tiles and one of 64-row tiles take longer than a round of 256-row ones;
@@ -725,7 +790,7 @@ Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5)
     if (whole == 0 || cols >= tn || n < 6.0f) return best;
     for (int r = 0; r < 3; ++r) {
         const float c = (float)whole * cost[3] + cost[r];
-        if (tiles(r, tn - cols) <= 256 && c < least) least = c, best = Bf6Plan{256, 256, cols, rows[r]};
+        if (tiles(r, tn - cols) <= 256 && c < least) least = c, best = Bf6Plan{256, 256, cols, rows[r], c};
     }
     return best;
 }
@@ -769,6 +834,67 @@ int launch_gemm_bf6(const uint8_t *X, const uint8_t *W, uint32_t M, uint32_t N, 
     default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();
+}
+
+static uint64_t up256(uint64_t bytes) { return (bytes + 255) & ~(uint64_t)255; }
+static uint32_t padded_k(uint32_t K) { return (K + 127) & ~127u; }
+
+// [activation shadow | weight shadow | parameters], each from a multiple of 256 bytes on
+uint64_t shadows_bytes(uint32_t M, uint32_t N, uint32_t K)
+{
+    const uint64_t row = padded_k(K) / 4 * 3;
+    return up256(M * row) + up256((N + 31ull) / 32 * 32 * row) + (N + 15ull) / 16 * 16 * 14;
+}
+
+// Whether a product that comes without shadows is faster by the 6-bit float kernel with the time to make them, by the two kernels'
+// models.  Up to 1024 rows the pass takes what the kernel gains (1024 x 11008 x 4096 42.1 us integer, 28.6 and 11 of the pass).  Integer / by
+// shadows, us: 4096 x 28672 x 8192 662 / 493, 1999 x 11008 x 4096 76 / 68, 3072 x 4096 x 4096 49.6 / 40.4, 3679 x 3712 x 10240 110.7 / 87.0, 1827 x
+// 7352 x 13824 142 / 119; of 70 shapes (700..4096 rows, 256..28672 columns, 512..28672 elements) the 18 that it takes are 1.16 times as
+// fast in the geometric mean and 1.03 at least, of those that it leaves five would be 1.05 to 1.13 times as fast (3181 x 2959 x 23872
+// 198 / 176), 2048 x 4096 x 4096 31.6 / 32.9.
+bool pays_shadows(uint32_t M, uint32_t N, uint32_t K)
+{
+    if (M <= 1024 || K < 512 || (uint64_t)M * N < (1u << 22)) return false;
+    const float pass = 2.0f + 1.25f * (float)(((double)M + N) * K * 1.7e-7);
+    return plan_bf6(M, N, K, false).us + pass < 0.96f * select_stream_tile(M, N, K, 1, false).us;
+}
+
+int launch_gemm_via_shadows(const uint8_t *xq, const uint8_t *w, uint32_t M, uint32_t N, uint32_t K, const Epilogue &epi, uint16_t *y,
+                            uint8_t *room, hipStream_t stream)
+{
+    if (M == 0 || N == 0 || K == 0) return (int)hipErrorInvalidValue;
+    const uint32_t kpad = padded_k(K), npad = (N + 15) & ~15u;
+    ShadowsParams s{};
+    s.x = xq;
+    s.w = w;
+    s.X = room;
+    s.W = room + up256((uint64_t)M * (kpad / 4 * 3));
+    s.M = M;
+    s.N = N;
+    s.K = K;
+    s.par_out = reinterpret_cast<uint16_t *>(s.W + up256((N + 31ull) / 32 * 32 * (kpad / 4 * 3)));
+    const uint64_t bw = ((N + 31ull) / 32 * (kpad / 128) * 64 + 255) / 256, bx = ((uint64_t)M * (kpad / 32) + 255) / 256;
+    s.blocks_w = (uint32_t)bw;
+    s.blocks_x = (uint32_t)bx;
+    Epilogue e = epi;
+    // (the GEMM reads four columns' parameters at a time)
+    auto in_place = [](const void *p, uintptr_t to) { return reinterpret_cast<uintptr_t>(p) % to == 0; };
+    uint32_t bp = 0;
+    if (N % 16 != 0 || !in_place(e.s_col_1, 8) || !in_place(e.z_col_1, 8) || !in_place(e.s_col_2, 8) || !in_place(e.z_col_2, 8) ||
+        !in_place(e.bias, 8) || !in_place(e.rs_col, 16)) {
+        const uint16_t **const at[5] = {&e.s_col_1, &e.z_col_1, &e.s_col_2, &e.z_col_2, &e.bias};
+        for (int k = 0; k < 5; ++k) {
+            s.par[k] = *at[k];
+            if (*at[k]) *at[k] = s.par_out + (uint64_t)k * npad;
+        }
+        s.sums = e.rs_col;
+        if (e.rs_col) e.rs_col = reinterpret_cast<int32_t *>(s.par_out + 5ull * npad);
+        bp = (npad + 255) / 256;
+    }
+    if (bw + bx + bp > 0x7FFFFFFFull) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(shadows_kernel, dim3((uint32_t)(bw + bx) + bp), dim3(256), 0, stream, s);
+    if (const int st = (int)hipGetLastError()) return st;
+    return launch_gemm_bf6(s.X, s.W, M, N, kpad, e, y, stream);
 }
 
 }  // namespace duq

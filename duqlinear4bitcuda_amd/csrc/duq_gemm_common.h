@@ -81,19 +81,6 @@ __device__ __forceinline__ void store_quad(const GemmParams &p, uint32_t m, uint
     }
 }
 
-// Eight neighbouring outputs (`left` of them inside the row) to a place of any alignment.
-__device__ __forceinline__ void store_row_piece(uint16_t *dst, const v4u v, uint32_t left)
-{
-    typedef v4u v4u_any __attribute__((aligned(2)));
-    if (left >= 8) {
-        *reinterpret_cast<v4u_any *>(dst) = v;
-    } else {
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-            if ((uint32_t)r < left) dst[r] = (uint16_t)((r & 1) ? (v[r >> 1] >> 16) : (v[r >> 1] & 0xFFFFu));
-    }
-}
-
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 // Prefill kernel (duq_prefill.hip) on a tile that select_stream_tile picked; `fused`: p.epi into p.y, else int32 into p.C.

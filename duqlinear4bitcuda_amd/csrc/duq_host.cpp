@@ -151,6 +151,15 @@ struct Scratch {  // device memory of the current stream for the length of one c
     {
         if (bytes) data = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
     }
+    // none where the device's memory does not hold it
+    static Scratch if_there_is(uint64_t bytes)
+    {
+        try {
+            return Scratch(bytes);
+        } catch (const c10::OutOfMemoryError &) {
+            return Scratch(0);
+        }
+    }
     void *get() const { return data.get(); }
 };
 
@@ -570,10 +579,15 @@ PyObject *m_linear4(PyObject *, PyObject *const *a, Py_ssize_t n)
         Tensor y = output(*x, N, ScalarType::Half);
         const uint8_t *px = static_cast<const uint8_t *>(x->const_data_ptr()), *pw = static_cast<const uint8_t *>(w->const_data_ptr());
         const uint32_t m = static_cast<uint32_t>(M), nn = static_cast<uint32_t>(N), k = static_cast<uint32_t>(K);
+        const uint64_t bytes = shadows ? 0 : duq_linear4bit_room_bytes(mode, m, nn, k);
+        const Scratch room = bytes ? Scratch::if_there_is(bytes) : Scratch(0);
         int e;
         {
             Unlocked u;
-            if (shadows)
+            if (room.get())
+                e = duq_linear4bit_forward_room(mode, px, half(p[2]), half(p[3]), i32(p[10]), pw, half(p[5]), half(p[6]), half(p[7]),
+                                                half(p[8]), i32(p[11]), half(p[9]), m, nn, k, out<duq_half>(y), room.get(), bytes, st);
+            else if (shadows)
                 e = duq_linear4bit_forward_bf6(mode, px, half(p[2]), half(p[3]), i32(p[10]), pw, half(p[5]), half(p[6]), half(p[7]),
                                                half(p[8]), i32(p[11]), half(p[9]), m, nn, k, out<duq_half>(y), st);
             else if (rowsum)

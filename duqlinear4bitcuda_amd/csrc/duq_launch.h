@@ -191,6 +191,7 @@ struct StreamTile {
     // against it, us: 4160 x 3924 x 5888 114 -> 104, 897 x 8688 x 4544 60.3 -> 49.3, 2355 x 3344 x 2496 40.7 -> 32.0, 2614 x 3424 x 15360
     // 168 -> 145; of 26 shapes two behind by more than 2 %, 2048 x 6100 x 4096 56.9 -> 59.6 and 1203 x 15441 x 2176 103 -> 107)
     uint32_t main_cols = 0, rest_rows = 0, main_rows = 0, rest_cols = 0;
+    float us = 0.f;  // what the model gives it
 };
 // Rounds that do not come out even: tiles of 128 x 256 or 256 x 256 over as many columns as fill whole rounds, and the columns
 // that are left in one round of smaller tiles, 192 x 128, 128 x 128, 64 x 128 or (behind 256 x 256) 128 x 256, in the same launch
@@ -203,6 +204,7 @@ struct StreamTile {
 // changed fifteen of 75 shapes drawn at random (128..4096 rows, 700..20000 columns), by 1.02 to 1.34 (147 x 24961 x 14464).
 inline StreamTile with_rest(StreamTile best, float best_cost, uint32_t M, uint32_t N, float nch)
 {
+    best.us = best_cost;
     if (nch < 8.0f) return best;
     best_cost *= 0.96f;
     const uint32_t main_rows[2] = {128, 256};
@@ -218,7 +220,7 @@ inline StreamTile with_rest(StreamTile best, float best_cost, uint32_t M, uint32
             const float cost = (float)rounds * (nch * main_c[i] + main_f[i]) + nch * c_us[k] + f_us[k];
             if (cost < best_cost) {
                 best_cost = cost;
-                best = StreamTile{best.rows, best.cols, best.stream, cols, rm[k], main_rows[i], rn[k]};
+                best = StreamTile{best.rows, best.cols, best.stream, cols, rm[k], main_rows[i], rn[k], cost};
             }
         }
     }
@@ -349,12 +351,19 @@ int launch_activation_shadow_bf6(const uint8_t *q, uint32_t M, uint32_t K, uint8
 // Tiles of a launch: rows x width; cols > 0: that many columns of them, the others in tiles of `rest` rows.
 struct Bf6Plan {
     uint32_t rows, width = 256, cols = 0, rest = 0;
+    float us = 0.f;  // what the model gives it
 };
 Bf6Plan plan_bf6(uint32_t M, uint32_t N, uint32_t K, bool mode5);
 // epi.mode 5 (row-sum epilogue of the dual-uniform layer) also needs the packed-int4 operands the shadows were made
 // from, xq [M, K/2] and wq [N, K/2]: the first eight bytes of every row are read.
 int launch_gemm_bf6(const uint8_t *X, const uint8_t *W, uint32_t M, uint32_t N, uint32_t K, const Epilogue &epi,
                     uint16_t *y, hipStream_t stream, const uint8_t *xq = nullptr, const uint8_t *wq = nullptr);
+// The same product from packed operands that come without shadows (epilogue modes 0 - 4): both are made first, in `room` of
+// shadows_bytes(M, N, K) bytes, 16-byte aligned.  Any N, K % 64 == 0, y at any address.
+uint64_t shadows_bytes(uint32_t M, uint32_t N, uint32_t K);
+bool pays_shadows(uint32_t M, uint32_t N, uint32_t K);
+int launch_gemm_via_shadows(const uint8_t *xq, const uint8_t *w, uint32_t M, uint32_t N, uint32_t K, const Epilogue &epi, uint16_t *y,
+                            uint8_t *room, hipStream_t stream);
 
 // 8-bit asymmetric layer (duq_int8.hip): float32 activations, int8 codes, int32 accumulators, float32 results.
 int launch_asym_quant8(const float *x, const float *scale, const float *zeros, uint32_t rows, uint32_t cols, int8_t *q,

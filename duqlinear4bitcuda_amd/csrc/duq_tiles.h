@@ -43,6 +43,19 @@ __device__ __forceinline__ v4u buf_load16_aux(__amdgpu_buffer_rsrc_t r, uint32_t
     return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, AUX));
 }
 
+// Eight neighbouring outputs (`left` of them inside the row) to a place of any alignment.
+__device__ __forceinline__ void store_row_piece(uint16_t *dst, const v4u v, uint32_t left)
+{
+    typedef v4u v4u_any __attribute__((aligned(2)));
+    if (left >= 8) {
+        *reinterpret_cast<v4u_any *>(dst) = v;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+            if ((uint32_t)r < left) dst[r] = (uint16_t)((r & 1) ? (v[r >> 1] >> 16) : (v[r >> 1] & 0xFFFFu));
+    }
+}
+
 // Binary16 outputs of prefill-sized launches (rows of y 16-byte aligned): stored past the L2 (non-temporal) or into it.  What fits
 // in the eight L2s, 32 MB, is still there when the last workgroup ends and would be written back only then, and rows that are whole
 // cache lines leave as whole lines either way: streamed (integer kernel 2048 x 4096 x 4096 30.5 us against 31.5, 2048 x 4096 x 1024

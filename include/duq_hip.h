@@ -198,6 +198,18 @@ int duq_linear4bit_forward(int32_t mode, const uint8_t *xq, const duq_half *scal
                            const duq_half *w_scale_2, const duq_half *w_zeros_2, const duq_half *bias,
                            uint32_t M, uint32_t N, uint32_t K, duq_half *y, duq_stream_t stream);
 
+/* No counterpart in the reference.  duq_linear4bit_forward (modes 0 - 3; rowsum_x and w_rowsum_adj NULL) and
+ * duq_linear4bit_forward_rowsum (DUQ_EPI_ASYM_ROWSUM), the same bits, with room for 6-bit float shadows of both operands: where
+ * duq_linear4bit_room_bytes is not 0, making these and multiplying them is the faster way (prefill of some thousand rows), and
+ * `room` is that many bytes of device memory, 16-byte aligned, that the caller provides and may reuse once the call's work
+ * has completed on the stream.  room NULL: as without. */
+uint64_t duq_linear4bit_room_bytes(int32_t mode, uint32_t M, uint32_t N, uint32_t K);
+int duq_linear4bit_forward_room(int32_t mode, const uint8_t *xq, const duq_half *scale_x, const duq_half *zeros_x,
+                                const int32_t *rowsum_x, const uint8_t *w, const duq_half *w_scale_1, const duq_half *w_zeros_1,
+                                const duq_half *w_scale_2, const duq_half *w_zeros_2, const int32_t *w_rowsum_adj,
+                                const duq_half *bias, uint32_t M, uint32_t N, uint32_t K, duq_half *y, void *room,
+                                uint64_t room_bytes, duq_stream_t stream);
+
 /* duq_linear4bit_forward over batch_count problems of one shape in ONE launch: what the loop of
  * AsymQuantMatMul.forward (qlinear4bit/nn/matmul.py:55-63: a GEMM per batch entry into an int32 tensor, then
  * asym_batch_dequant) and a batched SymQuantMatMul compute, without the int32 tensor.  Every tensor is

@@ -1,0 +1,91 @@
+"""Prefill of packed codes without shadows, where both are made in the call (csrc/duq_bf6.hip, shadows_kernel): rows, columns and k that
+end inside a tile, a pair of weight tiles and a step, output rows and parameters at any alignment, every epilogue; against the oracle on
+some of the rows and the integer kernels (which a call as a batch of one runs) on all."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import duq_oracle as orc
+
+
+def _room(mode, M, N, K):
+    from duqlinear4bitcuda_amd import _lib
+    return _lib.load().duq_linear4bit_room_bytes(mode, M, N, K)
+
+
+def test_rule():
+    assert _room(0, 4096, 28672, 8192) and _room(4, 1999, 11008, 4096) and _room(1, 1999, 11003, 4160)
+    # up to 1024 rows, short rows, few columns, the epilogue with packed heads, what the GEMM refuses
+    for mode, M, N, K in ((0, 1024, 28672, 8192), (0, 4096, 4096, 448), (0, 4096, 256, 4096), (5, 4096, 28672, 8192),
+                          (0, 4096, 28672, 8200), (0, (1 << 24) + 1, 28672, 8192), (0, 0, 4096, 4096), (0, 4096, 0, 4096),
+                          (0, 4096, 4096, 0), (0, 4096, (1 << 22) + 1, 8192)):
+        assert _room(mode, M, N, K) == 0, (mode, M, N, K)
+
+
+def test_errors():
+    from duqlinear4bitcuda_amd import _lib
+    call, P = _lib.load().duq_linear4bit_forward_room, 4096
+    args = lambda mode=0, xq=P, zeros=None, K=8192, room=P, n=1 << 31: (mode, xq, P, zeros, None, P, P, None, None, None, None, None,
+                                                                        4096, 28672, K, P, room, n, None)
+    assert call(*args(mode=5)) == -4 and call(*args(xq=None)) == -1 and call(*args(mode=1)) == -1 and call(*args(mode=4, zeros=P)) == -1
+    assert call(*args(K=8200)) == -3 and call(*args(xq=P + 8)) == call(*args(room=P + 8)) != 0 and call(*args(n=1 << 20)) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1999, 11003, 4096), (2049, 11015, 4160), (1553, 8561, 7936), (3073, 4097, 4032), (1712, 25720, 2880),
+                                   (2100, 12000, 1088), (2401, 8208, 8256), (1025, 30000, 8192), (1323, 16400, 2112)])
+def test_against_integer_kernels(dev, M, N, K):
+    from duqlinear4bitcuda_amd import _HIP as hip
+    print("prefill with shadows made in the call", M, N, K, flush=True)
+    assert _room(0, M, N, K)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    a, b = (torch.randint(0, 256, (n, K // 2), dtype=torch.uint8, device=dev, generator=g) for n in (M, N))
+    a[0], b[-1] = 0x88, 0x88   # the largest products there are
+    h = lambda n: (torch.rand(n, device=dev, generator=g) * 4 - 1).half() / 64
+    i = lambda n: torch.randint(-5000, 5000, (n,), device=dev, generator=g).int()
+    sr, zr, rr, s1, s2, bias, r1 = h(M), (h(M) * 64).round(), i(M), h(N), h(N), h(N), i(N)
+    z1, z2 = (h(N) * 64).round(), (h(N) * 64).round()
+    place = lambda t: torch.cat([t.flatten()[:1], t.flatten()])[1:]   # parameters at an odd address
+    rows = [0, 1, 31, 128, M // 2, M - 2, M - 1]
+    acc = orc.matmul_s4(a[rows].cpu().numpy(), b.cpu().numpy())
+    n = lambda t, r=None: (t if r is None else t[r]).cpu().numpy().reshape(-1, 1)
+    for mode, r, c, want in (
+            (hip.EPI_SYM, (sr, None), (s1, None, None, None), lambda: orc.sym_dequant(acc, n(sr, rows), n(s1))),
+            (hip.EPI_ASYM, (sr, zr), (s1, z1, None, None), lambda: orc.asym_dequant(acc, n(sr, rows), n(zr, rows), n(s1), n(z1))),
+            (hip.EPI_SYM_DUAL, (sr, None), (s1, None, s2, None), lambda: orc.sym_dual_dequant(acc, n(sr, rows), n(s1), n(s2))),
+            (hip.EPI_ASYM_DUAL, (sr, zr), (s1, z1, s2, z2),
+             lambda: orc.asym_dual_dequant(acc, n(sr, rows), n(zr, rows), n(s1), n(z1), n(s2), n(z2)))):
+        for off in (lambda t: t, place):
+            got = hip.linear4bit_forward(mode, a, *r, b, *(t if t is None else off(t) for t in c))
+            assert np.array_equal(got[rows].cpu().numpy().view(np.uint16), np.asarray(want()).view(np.uint16)), mode
+            with_bias = hip.linear4bit_forward(mode, a, *r, b, *(t if t is None else off(t) for t in c), bias=off(bias))
+            integer = hip.batch_linear4bit_forward(mode, a[None], *(t if t is None else t[None] for t in r), b[None],
+                                                   *(t if t is None else t[None] for t in c))[0]
+            assert torch.equal(got.view(torch.int16), integer.view(torch.int16)), mode
+            assert torch.equal(with_bias.view(torch.int16), (integer + bias).view(torch.int16)), mode
+    got = hip.linear4bit_forward_rowsum(a, sr, zr, rr, b, s1, z1, r1, bias)
+    want = hip.asym_rowsum_dequant(hip.matmul(a, b), sr, zr, rr, s1, z1, r1, bias)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.gpu
+def test_in_a_recording(dev):
+    """Room and shadows of several layers in one graph, replayed with eager work in between."""
+    from duqlinear4bitcuda_amd import nn as qnn
+    from duqlinear4bitcuda_amd.tools.graphs import GraphedForward
+    M, K = 3072, 4096
+    assert _room(0, M, K, K)
+    g = torch.Generator(device=dev).manual_seed(5)
+    mods = []
+    for _ in range(3):
+        lin = torch.nn.Linear(K, K, device=dev, dtype=torch.float16).requires_grad_(False)
+        mods += [qnn.SymQuantizer(), qnn.Linear4bitSQ.from_float(lin, lin.weight.abs().amax(1, keepdim=True) / 7).to(dev)]
+    model = torch.nn.Sequential(*mods)
+    x = torch.randn(M, K, device=dev, generator=g).half()
+    graphed = GraphedForward(model, x)
+    for k in range(4):
+        x = torch.randn(M, K, device=dev, generator=g).half()
+        want = model(x)
+        assert torch.equal(graphed(x), want), k
+        del want
+        torch.cuda.synchronize()
