@@ -482,6 +482,10 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
     const bool asym = mode == DUQ_EPI_ASYM;
     if (duq::product_row_takes(M, N, K))
         return duq::launch_product_row(asym, a, b, batch_count, N, K, clip_a, qmax_a, clip_b, qmax_b, y, as_stream(stream));
+    if (duq::product_tiles_takes(asym, batch_count, M, N, K) &&
+        !(duq::product_tiles_eager_only(batch_count, M, N, K) && recording(as_stream(stream))))
+        return duq::launch_product_tiles(asym, a, b, batch_count, M, N, K, asym ? 1.0f : clip_a, asym ? 15 : qmax_a, asym ? 1.0f : clip_b,
+                                         asym ? 15 : qmax_b, y, as_stream(stream));
     uint8_t *q = static_cast<uint8_t *>(workspace);
     duq_half *s = reinterpret_cast<duq_half *>(q + up16(rows * (K / 2)));
     duq_half *z = asym ? s + up16(rows * 2) / 2 : nullptr;

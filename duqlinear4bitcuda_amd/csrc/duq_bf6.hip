@@ -189,10 +189,6 @@ __global__ __launch_bounds__(256) void shadows_kernel(ShadowsParams p)
 // ---------------------------------------------------------------------------------
 // GEMM
 // ---------------------------------------------------------------------------------
-// Workgroup barrier that waits for this wavefront's LDS traffic only.  __syncthreads() also
-// drains the vector memory counter, which here would wait for the weight and activation
-// prefetches issued just before it (a full memory latency per chunk).
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // One MFMA on half h (0: registers 0..5, 1: registers 6..11) of weight pair tuple t, which lives in the twelve
 // registers v[128 + 12*t .. 139 + 12*t].  Naming the registers pins the tuple, so that the three 128-bit loads that

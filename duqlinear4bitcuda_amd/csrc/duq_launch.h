@@ -31,6 +31,11 @@ int launch_quantize_two(const uint16_t *x, uint32_t rows, const uint16_t *x2, ui
 bool product_row_takes(uint32_t M, uint32_t N, uint32_t K);
 int launch_product_row(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t N, uint32_t K, float clip_a,
                        int qmax_a, float clip_b, int qmax_b, uint16_t *y, hipStream_t stream);
+// Products of short rows, K = 64, 128, 192 or 256, in the same form (duq_product.hip); eager_only: not in a recording.
+bool product_tiles_takes(bool asym, uint32_t batch, uint32_t M, uint32_t N, uint32_t K);
+bool product_tiles_eager_only(uint32_t batch, uint32_t M, uint32_t N, uint32_t K);
+int launch_product_tiles(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t M, uint32_t N, uint32_t K, float clip_a,
+                         int qmax_a, float clip_b, int qmax_b, uint16_t *y, hipStream_t stream);
 
 // Epilogue description shared by the stand-alone dequant kernels and the fused GEMM.
 // mode: 0 sym, 1 asym, 2 sym-dual, 3 asym-dual, 4 asym with row-sum zero-point correction, 5 the same for the

@@ -430,38 +430,6 @@ __global__ __launch_bounds__(WAVES * 64) void quantize_rows_kernel(DUQ_HEAD_DECL
     }
 }
 
-// LANES lanes hold a row, lane u0 of them its units u0, u0 + LANES, ...: the row's parameters and the codes of those units
-// (of units past its end: anything).
-template <int LANES, bool ASYM, bool UNIFORM, int NU>
-__device__ __forceinline__ void quantize_in_group(const v4u (&regs)[NU], uint32_t u0, uint32_t nunits, float clip, int qmax,
-                                                  RowQuant<ASYM, UNIFORM> &rq, uint32_t (&w)[NU])
-{
-    PkMinMax st;
-#pragma unroll
-    for (int j = 0; j < NU; ++j)
-        if (u0 + j * LANES < nunits) st.add8(regs[j]);
-    float a = 0.f, b = 0.f;
-    uint32_t m16;
-    if (!ASYM) {
-        m16 = group_reduce<LANES>(st.absmax_bits(), [](uint32_t x, uint32_t y) { return max(x, y); });
-    } else {
-        st.mx = group_reduce<LANES>(st.mx, [](uint32_t x, uint32_t y) {
-            asm("v_pk_maximum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
-            return x;
-        });
-        st.mn = group_reduce<LANES>(st.mn, [](uint32_t x, uint32_t y) {
-            asm("v_pk_minimum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
-            return x;
-        });
-        m16 = st.absmax_bits();
-        a = st.min_f32();
-        b = st.max_f32();
-        if (m16 > 0x7C00u) a = b = __builtin_nanf("");  // torch's min / max return NaN for a row that holds one
-    }
-    rq.init(m16, a, b, clip, qmax);
-    rq.quant_units(regs, w);
-}
-
 // Short rows (at most 512 elements, no shadow: the operands of quantized attention).  With a workgroup per row such a
 // launch is bound by how fast workgroups start (65536 rows of 128 elements, asymmetric: 21.4 us for 21 MB, a quarter of a workgroup's
 // lanes at work).  Here LANES lanes hold a row, two units each, and a workgroup takes 256 / LANES rows; the same launch takes

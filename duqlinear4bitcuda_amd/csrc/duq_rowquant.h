@@ -198,7 +198,7 @@ struct RowQuant {
     // (the high nibbles of those bytes hold the sign extension); asym adds the zero point there too.  The four pairs go
     // through each stage together so that no instruction waits for the one before it.
     template <bool LO, bool HI>
-    __device__ __forceinline__ uint32_t quant8_packed(const v4u raw) const
+    __device__ __forceinline__ v2u code_bytes(const v4u raw) const
     {
         uint32_t d[4];
         float lo[4], hi[4];
@@ -223,19 +223,65 @@ struct RowQuant {
             const v2h q = __builtin_bit_cast(v2h, d[i]) + base;
             b[i] = __builtin_bit_cast(uint32_t, q);
         }
-        // gather the code bytes (bytes 0 and 2 of every pair), then merge the low nibbles of neighbours into one
-        // byte (a bit-field insert: low nibbles from p, high nibbles from p >> 4)
+        // gather the code bytes (bytes 0 and 2 of every pair)
         uint32_t p0 = __builtin_amdgcn_perm(b[1], b[0], 0x06040200u);
         uint32_t p1 = __builtin_amdgcn_perm(b[3], b[2], 0x06040200u);
         if (ASYM) {
             p0 += zodd;
             p1 += zodd;
         }
+        return v2u{p0, p1};
+    }
+    // merge the low nibbles of neighbouring bytes into one (a bit-field insert: low nibbles from p, high nibbles from p >> 4)
+    static __device__ __forceinline__ uint32_t merge_nibbles(const v2u p)
+    {
         uint32_t t0, t1;
         const uint32_t low = 0x0F0F0F0Fu;
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(t0) : "s"(low), "v"(p0), "v"(p0 >> 4));
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(t1) : "s"(low), "v"(p1), "v"(p1 >> 4));
+        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(t0) : "s"(low), "v"(p[0]), "v"(p[0] >> 4));
+        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(t1) : "s"(low), "v"(p[1]), "v"(p[1] >> 4));
         return __builtin_amdgcn_perm(t1, t0, 0x06040200u);
+    }
+    template <bool LO, bool HI>
+    __device__ __forceinline__ uint32_t quant8_packed(const v4u raw) const
+    {
+        return merge_nibbles(code_bytes<LO, HI>(raw));
+    }
+
+    // 8 elements -> a byte each in two words, in their order: the sign-extended code (sym), or 16 times the code's nibble read as a
+    // signed one (asym), as an MFMA on bytes takes them.
+    template <int N>
+    __device__ __forceinline__ void quant_units_bytes(const v4u (&raw)[N], v2u (&out)[N]) const
+    {
+        if (!fast) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const uint32_t w = quant8_exact<ASYM>(raw[j], rcp, qmax, zi);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    uint32_t v = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t nibble = (w >> (16 * k + 4 * e)) & 0xFu;
+                        v |= (ASYM ? nibble << 4 : (uint32_t)((int)(nibble << 28) >> 28) & 0xFFu) << (8 * e);
+                    }
+                    out[j][k] = v;
+                }
+            }
+            return;
+        }
+        if (!ASYM && clamp_lo) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) out[j] = code_bytes<true, true>(raw[j]);
+        } else if (clamp_hi) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) out[j] = code_bytes<false, true>(raw[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) out[j] = code_bytes<false, false>(raw[j]);
+        }
+        if (ASYM)
+#pragma unroll
+            for (int j = 0; j < N; ++j) out[j] = v2u{(out[j][0] << 4) & 0xF0F0F0F0u, (out[j][1] << 4) & 0xF0F0F0F0u};
     }
 
     // 8 elements (one 128-bit load) -> one packed word, element 0 in the low nibble
@@ -275,5 +321,44 @@ struct RowQuant {
         }
     }
 };
+
+// LANES lanes hold a row, lane u0 of them its units u0, u0 + LANES, ...: the row's parameters.
+template <int LANES, bool ASYM, bool UNIFORM, int NU>
+__device__ __forceinline__ void row_in_group(const v4u (&regs)[NU], uint32_t u0, uint32_t nunits, float clip, int qmax,
+                                             RowQuant<ASYM, UNIFORM> &rq)
+{
+    PkMinMax st;
+#pragma unroll
+    for (int j = 0; j < NU; ++j)
+        if (u0 + j * LANES < nunits) st.add8(regs[j]);
+    float a = 0.f, b = 0.f;
+    uint32_t m16;
+    if (!ASYM) {
+        m16 = group_reduce<LANES>(st.absmax_bits(), [](uint32_t x, uint32_t y) { return max(x, y); });
+    } else {
+        st.mx = group_reduce<LANES>(st.mx, [](uint32_t x, uint32_t y) {
+            asm("v_pk_maximum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
+            return x;
+        });
+        st.mn = group_reduce<LANES>(st.mn, [](uint32_t x, uint32_t y) {
+            asm("v_pk_minimum3_f16 %0, %0, %1, %1" : "+v"(x) : "v"(y));
+            return x;
+        });
+        m16 = st.absmax_bits();
+        a = st.min_f32();
+        b = st.max_f32();
+        if (m16 > 0x7C00u) a = b = __builtin_nanf("");  // torch's min / max return NaN for a row that holds one
+    }
+    rq.init(m16, a, b, clip, qmax);
+}
+
+// The same, and the codes of those units (of units past the row's end: anything).
+template <int LANES, bool ASYM, bool UNIFORM, int NU>
+__device__ __forceinline__ void quantize_in_group(const v4u (&regs)[NU], uint32_t u0, uint32_t nunits, float clip, int qmax,
+                                                  RowQuant<ASYM, UNIFORM> &rq, uint32_t (&w)[NU])
+{
+    row_in_group<LANES>(regs, u0, nunits, clip, qmax, rq);
+    rq.quant_units(regs, w);
+}
 
 }  // namespace duq

@@ -56,6 +56,11 @@ __device__ __forceinline__ void store_row_piece(uint16_t *dst, const v4u v, uint
     }
 }
 
+// Workgroup barrier that waits for this wavefront's LDS traffic only.  __syncthreads() also
+// drains the vector memory counter, which would wait for loads requested ahead
+// (a full memory latency) and for stores on their way.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // Binary16 outputs of prefill-sized launches (rows of y 16-byte aligned): stored past the L2 (non-temporal) or into it.  What fits
 // in the eight L2s, 32 MB, is still there when the last workgroup ends and would be written back only then, and rows that are whole
 // cache lines leave as whole lines either way: streamed (integer kernel 2048 x 4096 x 4096 30.5 us against 31.5, 2048 x 4096 x 1024
