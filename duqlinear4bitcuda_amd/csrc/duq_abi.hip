@@ -489,6 +489,10 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
     uint8_t *q = static_cast<uint8_t *>(workspace);
     duq_half *s = reinterpret_cast<duq_half *>(q + up16(rows * (K / 2)));
     duq_half *z = asym ? s + up16(rows * 2) / 2 : nullptr;
+    // (M >= 32: the workspace has the room of whole tiles of B)
+    if (duq::product_long_takes(batch_count, M, N, K))
+        return duq::launch_product_long(asym, a, b, batch_count, M, N, K, asym ? 1.0f : clip_a, asym ? 15 : qmax_a, asym ? 1.0f : clip_b,
+                                        asym ? 15 : qmax_b, y, q, s, z, as_stream(stream));
     if (asym || (clip_a == clip_b && qmax_a == qmax_b)) {
         if (int e = duq::launch_quantize_two(a, (uint32_t)rows_a, b, (uint32_t)rows_b, K, asym, asym ? 1.0f : clip_a,
                                              asym ? 15 : qmax_a, q, s, z, as_stream(stream)))

@@ -37,6 +37,11 @@ bool product_tiles_eager_only(uint32_t batch, uint32_t M, uint32_t N, uint32_t K
 int launch_product_tiles(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t M, uint32_t N, uint32_t K, float clip_a,
                          int qmax_a, float clip_b, int qmax_b, uint16_t *y, hipStream_t stream);
 
+// Products of long rows with few columns (duq_product_long.hip); q: room for the codes of B, whole tiles of 32 rows; s, z [batch, N].
+bool product_long_takes(uint32_t batch, uint32_t M, uint32_t N, uint32_t K);
+int launch_product_long(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t M, uint32_t N, uint32_t K, float clip_a,
+                        int qmax_a, float clip_b, int qmax_b, uint16_t *y, uint8_t *q, uint16_t *s, uint16_t *z, hipStream_t stream);
+
 // Epilogue description shared by the stand-alone dequant kernels and the fused GEMM.
 // mode: 0 sym, 1 asym, 2 sym-dual, 3 asym-dual, 4 asym with row-sum zero-point correction, 5 the same for the
 // dual-uniform layer (fused GEMM only, shapes of gemm_fuses_dual_rowsum) (DUQ_EPI_* of the public header).

@@ -224,7 +224,8 @@ int duq_batch_linear4bit_forward(int32_t mode, const uint8_t *xq, const duq_half
 
 /* The whole forward of AsymQuantMatMul (mode DUQ_EPI_ASYM) and SymQuantMatMul (DUQ_EPI_SYM): both operands quantized per
  * row, in one launch unless the symmetric settings of the two differ, then duq_batch_linear4bit_forward (M = 1, N <= 2^24, K <= 4096,
- * and most shapes of K <= 256: all of it in one launch that leaves the workspace alone); the same bits as those steps (qlinear4bit/nn/matmul.py:38-63, 78-84).
+ * and most shapes of K <= 256: all of it in one launch that leaves the workspace alone; a launch for
+ * b and one for the rest where N <= 256 and b is the smaller part); the same bits as those steps (qlinear4bit/nn/matmul.py:38-63, 78-84).
  *   a [batch_count, M, K], b [batch_count, N, K] fp16, 16-byte aligned, K % 64 == 0;  y [batch_count, M, N] fp16
  *   clip, qmax   settings of the symmetric quantizers (not read by DUQ_EPI_ASYM, qmax has to be valid)
  *   workspace    duq_quantize_product_workspace_bytes(...) bytes, 16-byte aligned */
