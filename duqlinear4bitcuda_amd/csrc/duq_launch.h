@@ -318,7 +318,7 @@ inline QuantGemmShape quant_gemm_shape(uint32_t M, uint32_t N, uint32_t K)
         const uint32_t groups = (M + rows - 1) / rows, tiles = (N + 16 * cols - 1) / (16 * cols);
         if (groups > 64 || groups * ((tiles + most_chunks - 1) / most_chunks) > 256) return;
         const uint32_t per = 256 / groups, chunks = (tiles + per - 1) / per;  // (at most that many workgroups a group of rows)
-        if (chunks > most_chunks) return;
+        if (chunks > most_chunks || (rows == 16 && cols == 1 && K > 2048 && chunks == 1)) return;  // (that tile has two buffers of weights)
         us += more_us * (float)(chunks - 1);
         if (us < best_us) {
             best_us = us;

@@ -32,7 +32,7 @@ EDGES = {
     (32, 4, 4): [(64, 30003, 512)],
 }
 LONG = {  # two sets of registers one after the other
-    (16, 2, 1): [(32, 4000, 4032)],
+    (16, 2, 1): [(32, 4000, 4032), (513, 1, 2112), (1024, 64, 4096)],   # (the last two: as many groups of rows as there may be)
     (16, 3, 1): [(13, 12287, 3072)],
     (16, 1, 4): [(9, 16383, 4096)],
 }
@@ -42,6 +42,18 @@ SHAPES = [(t, s) for edges in (EDGES, LONG) for t, shapes in edges.items() for s
 @pytest.mark.parametrize("tile,shape", SHAPES)
 def test_shapes_reach_their_tile(tile, shape):
     assert _tile(*shape) == tile
+
+
+def test_the_rule_gives_no_other_tile():
+    """The tiles above are the ones there are kernels for (several chunks of columns are one kernel, whatever their number)."""
+    kind = lambda rows, cols, chunks, K: (rows, cols, chunks > 1, rows == 16 and K > 2048)
+    there = {kind(*t, s[2]) for t, s in SHAPES}
+    rows = [*range(3, 34), 40, 64, 65, 100, 128, 129, 200, 256, 257, 500, 512, 513, 700, 1000, 1024, 1025, 2000, 2048]
+    for M in rows:
+        for N in (1, 16, 17, 48, 64, 65, 128, 200, 300, 512, 1000, 2048, 4096, 8192, 16384, 28672, 65536):
+            for K in (64, 512, 576, 1024, 1088, 2048, 2112, 3072, 4096, 4160, 8192):
+                tile = _tile(M, N, K)
+                assert tile[0] == 0 or kind(*tile, K) in there, (M, N, K, tile)
 
 
 @pytest.mark.gpu
