@@ -200,7 +200,7 @@ __global__ __launch_bounds__(512, 4) void product_tiles_kernel(DUQ_HEAD_DECL, Pr
 // 7.5 / 7.0, 7.4 / 5.4).
 bool product_tiles_takes(bool asym, uint32_t batch, uint32_t M, uint32_t N, uint32_t K)
 {
-    if (K == 0 || K > 256 || K % 64 != 0 || M < 2) return false;
+    if (K == 0 || K > 256 || K % 64 != 0 || M < 2 || N > (1u << 24)) return false;  // (a tile of outputs: 32-bit offsets)
     const uint64_t blocks = (uint64_t)batch * ((N + 255) / 256);
     if (blocks * ((M + 63) / 64) >= (1u << 30)) return false;
     if (K > 192 && N % 32 != 0 && (uint64_t)M * N * batch > (16u << 20)) return false;
