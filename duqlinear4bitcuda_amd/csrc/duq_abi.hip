@@ -127,7 +127,8 @@ int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t
     if ((out.q && !aligned(out.q, 16))) return DUQ_E_ALIGN;
     const duq::QuantGemmShape tile = duq::quant_gemm_shape(M, N, K);
     const bool no_room = duq::decode_fp16in_one_launch(M, N, K);  // (the caller was asked for none)
-    const bool one_kernel = tile.rows != 0 && (no_room || !tile.eager_only || !recording(as_stream(stream)));
+    const bool one_kernel = tile.rows != 0 && !duq::leaves_few_rows(M, N, K, asym, rowsum) &&
+                            (no_room || !tile.eager_only || !recording(as_stream(stream)));
     auto launch_one = [&] {
         return one_kernel ? duq::launch_quant_gemm(tile, x, clip, qmax, w, M, N, K, e, y, out.q, out.scale, asym ? out.zeros : nullptr,
                                                    rowsum ? out.rowsum : nullptr, as_stream(stream))

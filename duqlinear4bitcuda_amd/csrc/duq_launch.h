@@ -337,6 +337,16 @@ inline QuantGemmShape quant_gemm_shape(uint32_t M, uint32_t N, uint32_t K)
     if (K > 2048 && K <= 4096) offer(16, 1, 4, 4.0f + 0.62f * k, 1.0f);
     return best;
 }
+// Three and four rows of more than 2048 elements whose quantizer delivers no row sums: the rows kernel, which splits a row's quantization over
+// all its wavefronts, is ahead up to 4096 elements, and beyond on narrow layers (graph, us, rows kernel / this one; 3 rows symmetric, 4
+// symmetric, 4 asymmetric, 4 with row sums: N x K 4096 x 2048 3.88 / 3.70, 3.89 / 3.72, 4.11 / 3.89, 4.45 / 4.09; 4096 x 3072 3.88 / 4.12, 3.90 / 4.16, 4.13
+// / 4.34, 4.50 / 4.51; 4096 x 4096 3.96 / 4.37, 3.98 / 4.41, 4.37 / 4.49, 4.95 / 4.62; 1024 x 4160 4.73 / 4.93, 5.17 / 4.94, 5.60 / 5.27, 6.03 / 5.39; 1024 x
+// 8192 4.79 / 5.63, 5.32 / 5.68, 5.89 / 6.16, 6.43 / 6.19; 4096 x 8192 5.91 / 6.14, 6.19 / 6.13, 6.81 / 6.34, 7.43 / 6.39).
+inline bool leaves_few_rows(uint32_t M, uint32_t N, uint32_t K, bool asym, bool rowsum)
+{
+    if (M > 4 || K <= 2048 || rowsum || !decode_fp16in_one_launch(M, N, K)) return false;
+    return K <= 4096 || (K > 6144 && (N <= 2048 || !asym)) || (M <= 3 && N <= 2048 && !asym);
+}
 // q_out / s_out / z_out / rs_out as above.
 int launch_quant_gemm(QuantGemmShape s, const uint16_t *x, float clip, int qmax, const uint8_t *B, uint32_t M, uint32_t N, uint32_t K,
                       const Epilogue &epi, uint16_t *y, uint8_t *q_out, uint16_t *s_out, uint16_t *z_out, int32_t *rs_out,

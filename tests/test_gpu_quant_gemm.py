@@ -64,6 +64,14 @@ def test_tiles_against_the_oracle(hip, dev, i):  # noqa: F811
         _against_the_oracle(hip, dev, M, N, K, mode)
 
 
+# three and four rows, which go to one kernel or the other by their length, the columns and the quantizer
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(3, 1030, 2112), (4, 1001, 4096), (3, 2048, 4160), (4, 2050, 4160), (4, 2048, 6208), (3, 4096, 8192), (4, 16390, 3008)])
+def test_few_long_rows(hip, dev, M, N, K):  # noqa: F811
+    for mode in range(6):
+        _against_the_oracle(hip, dev, M, N, K, mode)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(20, 40, 2112), (33, 2700, 2048), (500, 2001, 960), (40, 4000, 4096)])
 def test_rows_that_are_not_finite_beside_rows_that_are(hip, dev, M, N, K):  # noqa: F811
