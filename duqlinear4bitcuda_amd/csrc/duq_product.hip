@@ -196,8 +196,8 @@ __global__ __launch_bounds__(512, 4) void product_tiles_kernel(DUQ_HEAD_DECL, Pr
 // All rows of up to 256 elements but for a few where the quantizer launch and the short-row kernel are ahead, asymmetric, us: rows of 256
 // on few blocks of columns, where many workgroups quantize the same rows of B (1 x 4090 x 4096 15.7 / 16.9, 8 x 1215 x 1216 15.4 / 15.8, but 12 x
 // 2046 x 2048 42.1 / 39.0), or with large outputs whose rows do not begin at half lines (32 x 2000 x 1992 94.5 / 97.7); in a recording, where a
-// launch costs the host nothing, a few tiles (1 x 64 x 64 x 256 4.9 / 7.0, 8 x 60 x 64 x 256 6.8 / 7.2, 1 x 64 x 64 x 128 4.9 / 5.6; eager 7.5 / 6.8,
-// 7.5 / 7.0, 7.4 / 5.4).
+// launch costs the host nothing, a few tiles (1 x 64 x 64 x 256 4.9 / 7.0, 8 x 60 x 64 x 256 6.8 / 7.2, 16 x 60 x 64 x 256 7.2 / 7.4, 1 x 64 x 64 x 128 4.9 /
+// 5.6, 1 x 2 x 4096 x 128 5.1 / 5.8, 1 x 16 x 4096 x 128 5.4 / 5.8; eager the first two and the fourth 7.5 / 6.8, 7.5 / 7.0, 7.4 / 5.4).
 bool product_tiles_takes(bool asym, uint32_t batch, uint32_t M, uint32_t N, uint32_t K)
 {
     if (K == 0 || K > 256 || K % 64 != 0 || M < 2 || N > (1u << 24)) return false;  // (a tile of outputs: 32-bit offsets)
@@ -209,7 +209,7 @@ bool product_tiles_takes(bool asym, uint32_t batch, uint32_t M, uint32_t N, uint
 
 bool product_tiles_eager_only(uint32_t batch, uint32_t M, uint32_t N, uint32_t K)
 {
-    return K > 64 && (uint64_t)batch * ((N + 255) / 256) * ((M + 63) / 64) < (K > 128 ? 12u : 2u);
+    return K > 64 && (uint64_t)batch * ((N + 255) / 256) * ((M + 63) / 64) < (M <= 16 || K > 128 ? 32u : 2u);
 }
 
 int launch_product_tiles(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t M, uint32_t N, uint32_t K, float clip_a,

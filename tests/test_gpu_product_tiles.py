@@ -66,7 +66,7 @@ def test_against_separate_launches(dev, n, M, N, K):
 
 
 # one tile and a few, which a recording runs as two launches, and more
-@pytest.mark.parametrize("n,M,N,K", [(1, 64, 64, 256), (1, 50, 200, 128), (11, 60, 64, 192), (12, 64, 64, 256), (8, 300, 300, 128)])
+@pytest.mark.parametrize("n,M,N,K", [(1, 64, 64, 256), (1, 50, 200, 128), (11, 60, 64, 192), (15, 64, 64, 256), (31, 60, 64, 256), (32, 64, 64, 256), (1, 16, 4096, 128), (8, 300, 300, 128)])
 def test_in_a_recording(dev, n, M, N, K):
     from duqlinear4bitcuda_amd.nn import AsymQuantMatMul
     print("product tiles, recorded", n, M, N, K, flush=True)
