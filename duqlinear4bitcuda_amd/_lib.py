@@ -50,6 +50,7 @@ PROTOTYPES = {
                                _c_u32, _c_p, _c_p],
     "duq_linear4bit_room_bytes": [_c_i32, _c_u32, _c_u32, _c_u32],  # returns uint64_t
     "duq_linear4bit_forward_room": [_c_i32] + [_c_p] * 11 + [_c_u32, _c_u32, _c_u32, _c_p, _c_p, ctypes.c_uint64, _c_p],
+    "duq_product_long_reads_for": [_c_u32, _c_u32],  # returns uint32_t
     "duq_gemm_kernel_for": [_c_u32, _c_u32, _c_u32],
     "duq_gemm_stream_tile_for": [_c_u32, _c_u32, _c_u32],
     "duq_quant_gemm_tile_for": [_c_u32, _c_u32, _c_u32],
@@ -143,6 +144,7 @@ def _load():
     lib.duq_quantize_linear8bit_workspace_bytes.restype = ctypes.c_uint64
     lib.duq_quantize_product_workspace_bytes.restype = ctypes.c_uint64
     lib.duq_linear4bit_room_bytes.restype = ctypes.c_uint64
+    lib.duq_product_long_reads_for.restype = ctypes.c_uint32
     lib.duq_status_string.argtypes = [ctypes.c_int]
     lib.duq_status_string.restype = ctypes.c_char_p
     _lib = lib

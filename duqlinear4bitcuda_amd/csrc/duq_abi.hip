@@ -508,6 +508,11 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
                                         nullptr, batch_count, M, N, K, y, stream);
 }
 
+uint32_t duq_product_long_reads_for(uint32_t N, uint32_t K)
+{
+    return N == 0 || N > 256 || K == 0 || K > 4096 || K % 64 != 0 ? 0 : duq::product_long_reads(N, K);
+}
+
 int duq_probe_read(const void *src, uint64_t bytes, uint32_t *sink, duq_stream_t stream)
 {
     if (bytes == 0) return DUQ_OK;

@@ -39,6 +39,7 @@ int launch_product_tiles(bool asym, const uint16_t *a, const uint16_t *b, uint32
 
 // Products of long rows with few columns (duq_product_long.hip); q: room for the codes of B, whole tiles of 32 rows; s, z [batch, N].
 bool product_long_takes(uint32_t batch, uint32_t M, uint32_t N, uint32_t K);
+uint32_t product_long_reads(uint32_t N, uint32_t K);
 int launch_product_long(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t M, uint32_t N, uint32_t K, float clip_a,
                         int qmax_a, float clip_b, int qmax_b, uint16_t *y, uint8_t *q, uint16_t *s, uint16_t *z, hipStream_t stream);
 

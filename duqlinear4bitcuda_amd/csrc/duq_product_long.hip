@@ -11,6 +11,8 @@
 // Tiles of 64 rows, two workgroups a CU: the first three 57.7, 72.3, 46.1, 8 x 1021 x 64 x 1024 13.1 (half the workgroups).  Two groups of
 // rows requested ahead at two workgroups a CU: 58.2, 75.4, 51.4.  Workgroups that stay for several tiles and request the next tile's rows
 // behind the last codes of B: 103, 114, 73, since loads return in their order and the multiplications come to wait for those rows.
+#include <algorithm>
+
 #include "duq_epilogue.h"
 #include "duq_launch.h"
 #include "duq_rowquant.h"
@@ -59,6 +61,23 @@ __global__ __launch_bounds__(256) void quantize_tiles_kernel(TileQuantParams p)
         p.s[row] = f16_to_bits(rq.s);
         if (ASYM) p.z[row] = f16_to_bits(rq.z);
     }
+}
+
+// Tiles of 32 columns that a workgroup has wavefronts for.
+constexpr uint32_t long_column_tiles(uint32_t N) { return N <= 32 ? 1 : N <= 64 ? 2 : N <= 128 ? 4 : 8; }
+
+// What a wavefront with column tile ct may read of its problem's codes: for tiles past the last (of four or eight, 65 to 96 and 129 to
+// 224 columns have fewer) nothing, and every load gives zeros.
+__host__ __device__ __forceinline__ uint32_t long_codes(uint32_t ct, uint32_t tiles, uint32_t steps) { return ct < tiles ? tiles * steps * 1024 : 0; }
+
+// Where a lane finds its 16 bytes of step i.  Only the lane's offset is sure to be compared with the end of the codes, so it is what sends
+// steps past the last out of range.
+struct LongPiece {
+    uint32_t lane_offset, offset;
+};
+__host__ __device__ __forceinline__ LongPiece long_piece(uint32_t lane, uint32_t ct, uint32_t i, uint32_t steps)
+{
+    return {i < steps ? lane * 16 : kOobOffset, i < steps ? (ct * steps + i) * 1024 : 0};
 }
 
 // The first 56 bytes (through reserved) reach the kernel in registers (DUQ_HEAD_DECL / with_head).
@@ -114,15 +133,15 @@ __global__ __launch_bounds__(512, LANES * UNITS > 384 ? 4 : 6) void product_long
         if (ASYM) col_z[tid] = p.z[n];
     }
 
-    // ---- codes of B: this wavefront's columns, steps ks, ks + KS, ..., four at a time (past the end: zeros)
+    // ---- codes of B: this wavefront's columns, steps ks, ks + KS, ..., four at a time (steps and whole tiles of columns past the end: zeros)
     const uint32_t ct = wave % CT, ks = wave / CT, tiles = (p.N + 31) / 32;
-    const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.q + (uint64_t)problem * tiles * steps * 1024, tiles * steps * 1024);
+    const __amdgpu_buffer_rsrc_t rB = make_rsrc(p.q + (uint64_t)problem * tiles * steps * 1024, long_codes(ct, tiles, steps));
     v4u w[2][4];
     auto fetch_b = [&](v4u(&to)[4], uint32_t at) {
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-            const uint32_t i = ks + (at + k) * KS;
-            to[k] = buf_load16(rB, i < steps ? lane * 16 : kOobOffset, i < steps ? (ct * steps + i) * 1024 : 0u);
+            const LongPiece piece = long_piece(lane, ct, ks + (at + k) * KS, steps);
+            to[k] = buf_load16(rB, piece.lane_offset, piece.offset);
         }
     };
 #pragma unroll
@@ -217,6 +236,19 @@ bool product_long_takes(uint32_t batch, uint32_t M, uint32_t N, uint32_t K)
     return tiles >= (N <= 128 ? (K <= 2048 ? 64u : 128u) : K <= 1536 ? 64u : K <= 2048 ? 256u : 1024u);
 }
 
+// The end of what a workgroup reads of its problem's codes of B.
+uint32_t product_long_reads(uint32_t N, uint32_t K)
+{
+    uint32_t end = 0;
+    const uint32_t tiles = (N + 31) / 32, steps = K / 64, ct = long_column_tiles(N), ks = 8 / ct;
+    for (uint32_t wave = 0; wave < 8; ++wave)
+        for (uint32_t at = 0; at < (steps + ks - 1) / ks + 16; ++at) {  // (the ring requests up to sixteen steps past the last)
+            const LongPiece piece = long_piece(63, wave % ct, wave / ct + at * ks, steps);
+            if (piece.lane_offset < long_codes(wave % ct, tiles, steps)) end = std::max(end, piece.offset + piece.lane_offset + 16);
+        }
+    return end;
+}
+
 // q: codes of B, batch * ((N + 31) / 32 * 32) * (K / 2) bytes; s, z [batch, N].
 int launch_product_long(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t M, uint32_t N, uint32_t K, float clip_a,
                         int qmax_a, float clip_b, int qmax_b, uint16_t *y, uint8_t *q, uint16_t *s, uint16_t *z, hipStream_t stream)
@@ -231,9 +263,10 @@ int launch_product_long(bool asym, const uint16_t *a, const uint16_t *b, uint32_
     auto launch = [&](auto l, auto u, auto zero_points) {
         hipLaunchKernelGGL((quantize_tiles_kernel<decltype(l)::value, decltype(u)::value, decltype(zero_points)::value>), quantizers, dim3(256), 0, stream, t);
         if (const int e = (int)hipGetLastError()) return e;
-        if (N <= 32) DUQ_LONG_CT(1);
-        else if (N <= 64) DUQ_LONG_CT(2);
-        else if (N <= 128) DUQ_LONG_CT(4);
+        const uint32_t ct = long_column_tiles(N);
+        if (ct == 1) DUQ_LONG_CT(1);
+        else if (ct == 2) DUQ_LONG_CT(2);
+        else if (ct == 4) DUQ_LONG_CT(4);
         else DUQ_LONG_CT(8);
         return (int)hipGetLastError();
     };

@@ -234,6 +234,10 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
                          float clip_a, int32_t qmax_a, float clip_b, int32_t qmax_b, duq_half *y, void *workspace,
                          uint64_t workspace_bytes, duq_stream_t stream);
 
+/* How many bytes of a problem's codes of b, whole tiles of 32 rows of K / 2 bytes, a workgroup of the launch for long rows reaches
+ * (N <= 256, K <= 4096, else 0; no GPU work; for tests). */
+uint32_t duq_product_long_reads_for(uint32_t N, uint32_t K);
+
 /* Which kernel duq_matmul_host_4bit / duq_linear4bit_forward run for a shape (no GPU work; for tests and tuning): 1 decode
  * rows kernel (M <= 4), 2 decode MFMA kernel (5..64 rows, mostly on more than 4096 columns, where 4, 6 and 8 are not ahead), 3 dot
  * kernel (M <= 4, rows longer than 16384 elements), 4 LDS kernel (5..64 rows on up to 4096 columns, 8192 where the rows
