@@ -18,6 +18,9 @@
 #include <structmember.h>
 #include <torch/version.h>
 
+#include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <vector>
@@ -151,17 +154,43 @@ struct Scratch {  // device memory of the current stream for the length of one c
     {
         if (bytes) data = c10::hip::HIPCachingAllocator::get()->allocate(bytes);
     }
-    // none where the device's memory does not hold it
-    static Scratch if_there_is(uint64_t bytes)
+    void *get() const { return data.get(); }
+};
+
+// Memory that a call is faster with and does without where the device has none left.  To find that out, torch's allocator waits for the
+// device and gives every cached block back, which the program around the call then has to allocate anew (asked on every call, 4096 x 4096 x
+// 28672 beside four blocks of 16 MB in a process at its limit: 349 us instead of 344, and the host behind the device each time), so that
+// one answer stands for a minute: until then nobody on the device asks for as much.
+class Rooms {
+    static constexpr int kDevices = 64;
+    struct Refused {
+        std::atomic<uint64_t> bytes{0};  // the least that there was no memory for (0: no answer)
+        std::atomic<int64_t> until{0};
+    };
+    Refused refused_[kDevices];
+    static int64_t seconds() { return std::chrono::duration_cast<std::chrono::seconds>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
+
+public:
+    Scratch take(int dev, uint64_t bytes)
     {
+        if (!bytes || dev < 0 || dev >= kDevices) return Scratch(0);
+        Refused &r = refused_[dev];
+        uint64_t least = r.bytes.load();
+        if (least && seconds() >= r.until.load()) r.bytes.store(least = 0);
+        if (least && bytes >= least) return Scratch(0);
         try {
             return Scratch(bytes);
         } catch (const c10::OutOfMemoryError &) {
+            r.until.store(seconds() + 60);
+            r.bytes.store(bytes);  // (less than what was refused before)
             return Scratch(0);
         }
     }
-    void *get() const { return data.get(); }
-};
+    void forget()
+    {
+        for (Refused &r : refused_) r.bytes.store(0);
+    }
+} g_rooms;
 
 PyObject *wrap(Tensor &&t) { return THPVariable_Wrap(std::move(t)); }
 
@@ -580,7 +609,7 @@ PyObject *m_linear4(PyObject *, PyObject *const *a, Py_ssize_t n)
         const uint8_t *px = static_cast<const uint8_t *>(x->const_data_ptr()), *pw = static_cast<const uint8_t *>(w->const_data_ptr());
         const uint32_t m = static_cast<uint32_t>(M), nn = static_cast<uint32_t>(N), k = static_cast<uint32_t>(K);
         const uint64_t bytes = shadows ? 0 : duq_linear4bit_room_bytes(mode, m, nn, k);
-        const Scratch room = bytes ? Scratch::if_there_is(bytes) : Scratch(0);
+        const Scratch room = g_rooms.take(dev, bytes);
         int e;
         {
             Unlocked u;
@@ -600,6 +629,13 @@ PyObject *m_linear4(PyObject *, PyObject *const *a, Py_ssize_t n)
         if (e) return finish(e, shadows ? "linear4bit_forward_bf6" : rowsum ? "linear4bit_forward_rowsum" : "linear4bit_forward", nullptr);
         return wrap(std::move(y));
     });
+}
+
+// forget_refused_rooms(): calls ask for memory again, whatever the answer was
+PyObject *m_forget_refused_rooms(PyObject *, PyObject *)
+{
+    g_rooms.forget();
+    return none();
 }
 
 // linear4_batched(mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias, stream)
@@ -1192,6 +1228,7 @@ PyMethodDef g_methods[] = {FAST("defer", m_defer),
                            FAST("linear4_batched", m_linear4_batched),
                            FAST("linear8", m_linear8),
                            {"setup", m_setup, METH_VARARGS, nullptr},
+                           {"forget_refused_rooms", m_forget_refused_rooms, METH_NOARGS, nullptr},
                            {"install", m_install, METH_VARARGS, nullptr},
                            {"plain_call", m_plain_call, METH_O, nullptr},
                            {nullptr, nullptr, 0, nullptr}};

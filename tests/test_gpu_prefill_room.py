@@ -89,3 +89,59 @@ def test_in_a_recording(dev):
         assert torch.equal(graphed(x), want), k
         del want
         torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_short_of_memory(dev):
+    """Where the device has no room left the integer kernel runs, and torch's allocator, which gives all of its cached blocks back
+    before it says so, is asked once and not on every call."""
+    import gc
+
+    from duqlinear4bitcuda_amd import _HIP as hip
+    from duqlinear4bitcuda_amd import _lib
+    M, N, K = 4096, 4096, 28672
+    need, out = _room(0, M, N, K), 2 * M * N
+    assert need > 3 * out
+    g = torch.Generator(device=dev).manual_seed(1)
+    a, b = (torch.randint(0, 256, (n, K // 2), dtype=torch.uint8, device=dev, generator=g) for n in (M, N))
+    s, t = (torch.rand(n, device=dev, generator=g).half() / 64 for n in (M, N))
+    run = lambda m=M: hip.linear4bit_forward(hip.EPI_SYM, a[:m], s[:m], None, b, t)
+
+    def took():
+        """Bytes beyond what is in use that a call took, its output aside."""
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        del_me = run()
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - before - del_me.nbytes
+
+    _lib.host().forget_refused_rooms()
+    want = run()
+    assert took() >= need
+    torch.cuda.synchronize()
+    gc.collect()
+    torch.cuda.empty_cache()
+    free = out + need // 2   # an output, and half a room
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + free) / torch.cuda.get_device_properties(dev).total_memory)
+        before = torch.cuda.memory_stats()
+        for _ in range(5):
+            got = None
+            got = run()
+            torch.cuda.synchronize()
+        after = torch.cuda.memory_stats()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for counter in ("num_ooms", "num_alloc_retries"):
+        assert after[counter] - before[counter] == 1, counter
+    assert took() < need // 2            # (still the answer)
+    small = _room(0, 2048, N, K)         # less than what was refused is asked for
+    assert 0 < small < need
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    y = run(2048)
+    assert torch.cuda.max_memory_allocated() - before >= small + y.nbytes
+    _lib.host().forget_refused_rooms()
+    assert took() >= need
