@@ -362,24 +362,29 @@ EPI_ASYM_ROWSUM = 4        # exact zero-point correction with row sums; not in t
 EPI_ASYM_DUAL_ROWSUM = 5   # the same for the dual-uniform layer (one-launch decode entry point only)
 
 
+ROOM_BYTES = 2 << 30   # what a forward on packed codes may take for shadows made in the call
+
+
 def _linear4_native(entry, mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias, rowsum_x=None,
-                    w_rowsum_adj=None, shadows=False):
+                    w_rowsum_adj=None, shadows=False, room_bytes=ROOM_BYTES):
     """GEMM + dequant through the native host module; None for what it does not take."""
     if type(xq) is not torch.Tensor or not xq.is_cuda:
         return None
     host = _host_for(entry)
     return None if host is None else _launch(xq.device, host.linear4, mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2,
-                                             w_zeros_2, bias, rowsum_x, w_rowsum_adj, shadows)
+                                             w_zeros_2, bias, rowsum_x, w_rowsum_adj, shadows, room_bytes)
 
 
 def linear4bit_forward(mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1=None, w_scale_2=None, w_zeros_2=None,
-                       bias=None):
-    """matmul + dequant (+ bias) in one launch; bit-identical to the separate ops.
+                       bias=None, room_bytes=ROOM_BYTES):
+    """matmul + dequant (+ bias); bit-identical to the separate ops.  One launch, or for prefill of some thousand rows, where that
+    is faster, two: 6-bit float shadows of both operands into memory of the call, of at most ``room_bytes``, and their product.
     ``xq`` is uint8 [..., K/2] (leading dimensions are flattened to M rows), ``w`` uint8
     [N, K/2]; per-row tensors hold M, per-column tensors N fp16 values in any contiguous
     shape.  Returns fp16 [..., N]."""
     name = "linear4bit_forward"
-    y = _linear4_native("duq_linear4bit_forward", mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias)
+    y = _linear4_native("duq_linear4bit_forward", mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias,
+                        room_bytes=room_bytes)
     if y is not None:
         return y
     if not isinstance(xq, torch.Tensor) or not isinstance(w, torch.Tensor):
@@ -812,13 +817,13 @@ def _rowsum_args(name, M, N, dev, scale_x, zeros_x, rowsum_x, w_scale, w_zeros, 
     return pb
 
 
-def linear4bit_forward_rowsum(xq, scale_x, zeros_x, rowsum_x, w, w_scale, w_zeros, w_rowsum_adj, bias=None):
-    """GEMM + exact asymmetric dequant (+ bias) in one launch on signed-shifted operands:
+def linear4bit_forward_rowsum(xq, scale_x, zeros_x, rowsum_x, w, w_scale, w_zeros, w_rowsum_adj, bias=None, room_bytes=ROOM_BYTES):
+    """GEMM + exact asymmetric dequant (+ bias) on signed-shifted operands (launches and ``room_bytes`` as ``linear4bit_forward``):
     y = s_x*s_w * (acc - z_x*w_rowsum_adj - z_w*rowsum_x), w_rowsum_adj = sum_k c_w - K*z_w.
     ``xq`` uint8 [..., K/2]; returns fp16 [..., N]."""
     name = "linear4bit_forward_rowsum"
     y = _linear4_native("duq_linear4bit_forward_rowsum", EPI_ASYM_ROWSUM, xq, scale_x, zeros_x, w, w_scale, w_zeros, None, None, bias,
-                        rowsum_x, w_rowsum_adj)
+                        rowsum_x, w_rowsum_adj, room_bytes=room_bytes)
     if y is not None:
         return y
     if not isinstance(xq, torch.Tensor) or not isinstance(w, torch.Tensor):

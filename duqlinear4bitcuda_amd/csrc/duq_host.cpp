@@ -580,10 +580,11 @@ PyObject *m_quantize_rows_8bit(PyObject *, PyObject *const *a, Py_ssize_t n)
 // ---- GEMM + dequant ----------------------------------------------------------------------------------------
 
 // linear4(mode, xq, scale_x, zeros_x, w, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias, rowsum_x, w_rowsum_adj,
-//         shadows, stream): modes 0 - 4 on packed codes, or with `shadows` on the 6-bit float shadows of both operands
+//         shadows[, room_bytes], stream): modes 0 - 4 on packed codes, with at most so many bytes of room for shadows made in the call, or with
+// `shadows` on the 6-bit float shadows of both operands
 PyObject *m_linear4(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
-    if (n != 14 || !PyLong_Check(a[0])) return none();
+    if ((n != 14 && n != 15) || !PyLong_Check(a[0]) || (n == 15 && !PyLong_Check(a[13]))) return none();
     const int mode = static_cast<int>(PyLong_AsLong(a[0]));
     const bool shadows = a[12] == Py_True;
     const Tensor *x = plain(a[1], ScalarType::Byte, -1);
@@ -603,13 +604,14 @@ PyObject *m_linear4(PyObject *, PyObject *const *a, Py_ssize_t n)
         return none();
     for (int k = 5; k < 10; ++k)
         if (!operand(a[k], ScalarType::Half, dev, N, k != 5 && !(rowsum && k == 6), &p[k])) return none();
-    const duq_stream_t st = stream_of(a[13]);
+    const int64_t most = n == 15 ? whole(a[13]) : INT64_MAX;
+    const duq_stream_t st = stream_of(a[n - 1]);
     return guarded([&]() -> PyObject * {
         Tensor y = output(*x, N, ScalarType::Half);
         const uint8_t *px = static_cast<const uint8_t *>(x->const_data_ptr()), *pw = static_cast<const uint8_t *>(w->const_data_ptr());
         const uint32_t m = static_cast<uint32_t>(M), nn = static_cast<uint32_t>(N), k = static_cast<uint32_t>(K);
         const uint64_t bytes = shadows ? 0 : duq_linear4bit_room_bytes(mode, m, nn, k);
-        const Scratch room = g_rooms.take(dev, bytes);
+        const Scratch room = g_rooms.take(dev, static_cast<int64_t>(bytes) <= most ? bytes : 0);
         int e;
         {
             Unlocked u;

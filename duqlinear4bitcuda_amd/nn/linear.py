@@ -231,6 +231,9 @@ class _Linear4bitBase(_MovesTogether):
     # 25.0 / 21.6, 768 x 4096 x 8192 26.9 / 29.2, 384 x 8192 x 8192 32.7 / 32.0, 512 x 8192 x 8192 33.9 / 35.0, 248 x 19968 x 17264 106 / 114, 1024 x 16384 x 4096 64.9 /
     # 63.2, 512 x 1536 x 16384 25.3 / 19.0, 768 x 1536 x 16384 25.0 / 27.4
     fp6_min_tiles = _FP6_MIN_TILES
+    # Device memory that a call of some thousand rows may take for itself to make both operands' 6-bit float shadows, where the layer
+    # holds none and that is faster (0: none, the integer kernel runs; same bits).  A graph's memory holds what its recording took.
+    prefill_room_bytes = _ops.ROOM_BYTES
     _shadow_key = None
 
     def _finish(self, y):
@@ -398,7 +401,8 @@ class Linear4bitSQ(_Linear4bitBase):
                                                       self.weight_scales, bias=self.bias)
         if self.fused:
             return tensor_utils.linear_forward(_ops.EPI_SYM, xq, scales_x, None, self.weight, self.weight_scales,
-                                               bias=self.bias)
+                                               bias=self.bias,
+                                               room_bytes=self.prefill_room_bytes)
         acc = tensor_utils.matmul(xq, self.weight)
         return self._finish(tensor_utils.sym_dequant(acc, scales_x, self.weight_scales))
 
@@ -451,7 +455,8 @@ class Linear4bitASQ(_Linear4bitBase):
                                                       self.weight_scales, self.weight_zeros, bias=self.bias)
         if self.fused:
             return tensor_utils.linear_forward(_ops.EPI_ASYM, xq, scales_x, zeros_x, self.weight, self.weight_scales,
-                                               self.weight_zeros, bias=self.bias)
+                                               self.weight_zeros, bias=self.bias,
+                                               room_bytes=self.prefill_room_bytes)
         acc = tensor_utils.matmul(xq, self.weight)
         return self._finish(tensor_utils.asym_dequant(acc, scales_x, zeros_x, self.weight_scales, self.weight_zeros))
 
@@ -515,7 +520,8 @@ class Linear4bitASQRowSum(_Linear4bitBase):
         if self.fused:
             return tensor_utils.linear_forward_rowsum(x.quantized_x, x.scales_x, x.zeros_x, x.rowsum_x, self.weight,
                                                       self.weight_scales, self.weight_zeros, self.weight_rowsum,
-                                                      bias=self.bias)
+                                                      bias=self.bias,
+                                                      room_bytes=self.prefill_room_bytes)
         acc = tensor_utils.matmul(x.quantized_x, self.weight)
         lead = acc.shape[:-1]
         y = _ops.asym_rowsum_dequant(acc.view(-1, acc.shape[-1]), x.scales_x, x.zeros_x, x.rowsum_x, self.weight_scales,
@@ -677,7 +683,8 @@ class Linear4bitDUSQ(_Linear4bitBase):
                                                       self.weight_scales_1, None, self.weight_scales_2, bias=self.bias)
         if self.fused:
             return tensor_utils.linear_forward(_ops.EPI_SYM_DUAL, xq, scales_x, None, self.weight,
-                                               self.weight_scales_1, None, self.weight_scales_2, bias=self.bias)
+                                               self.weight_scales_1, None, self.weight_scales_2, bias=self.bias,
+                                               room_bytes=self.prefill_room_bytes)
         acc = tensor_utils.matmul(xq, self.weight)
         return self._finish(tensor_utils.sym_dual_dequant(acc, scales_x, self.weight_scales_1, self.weight_scales_2))
 
@@ -737,7 +744,8 @@ class LinearQuant4bitDUASQ(_Linear4bitBase):
         if self.fused:
             return tensor_utils.linear_forward(_ops.EPI_ASYM_DUAL, xq, scales_x, zeros_x, self.weight,
                                                self.weight_scales_1, self.weight_zeros_1, self.weight_scales_2,
-                                               self.weight_zeros_2, bias=self.bias)
+                                               self.weight_zeros_2, bias=self.bias,
+                                               room_bytes=self.prefill_room_bytes)
         acc = tensor_utils.matmul(xq, self.weight)
         return self._finish(tensor_utils.asym_dual_dequant(acc, scales_x, zeros_x, self.weight_scales_1,
                                                            self.weight_zeros_1, self.weight_scales_2,

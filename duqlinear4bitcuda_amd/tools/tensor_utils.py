@@ -259,17 +259,18 @@ def quantize_asym_shifted(x):
     return _ops.quantize_rows_asym_shifted(x)
 
 
-def linear_forward_rowsum(xq, scales_x, zeros_x, rowsum_x, weight, w_scale, w_zeros, w_rowsum_adj, bias=None):
-    """GEMM + exact zero-point correction (+ bias) in one launch on signed-shifted operands."""
+def linear_forward_rowsum(xq, scales_x, zeros_x, rowsum_x, weight, w_scale, w_zeros, w_rowsum_adj, bias=None, room_bytes=_ops.ROOM_BYTES):
+    """GEMM + exact zero-point correction (+ bias) on signed-shifted operands."""
     assert xq.shape[-1] % 32 == 0, "A.shape[-1]: {} must be multiplication of 32".format(xq.shape[-1])
-    return _ops.linear4bit_forward_rowsum(xq, scales_x, zeros_x, rowsum_x, weight, w_scale, w_zeros, w_rowsum_adj, bias)
+    return _ops.linear4bit_forward_rowsum(xq, scales_x, zeros_x, rowsum_x, weight, w_scale, w_zeros, w_rowsum_adj, bias, room_bytes)
 
 
 def linear_forward(mode, xq, scales_x, zeros_x, weight, w_scale_1, w_zeros_1=None, w_scale_2=None, w_zeros_2=None,
-                   bias=None):
-    """GEMM + dequant (+ bias) in one launch; result has xq's leading dims and N columns."""
+                   bias=None, room_bytes=_ops.ROOM_BYTES):
+    """GEMM + dequant (+ bias); result has xq's leading dims and N columns."""
     assert xq.shape[-1] % 32 == 0, "A.shape[-1]: {} must be multiplication of 32".format(xq.shape[-1])
-    return _ops.linear4bit_forward(mode, xq, scales_x, zeros_x, weight, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias)
+    return _ops.linear4bit_forward(mode, xq, scales_x, zeros_x, weight, w_scale_1, w_zeros_1, w_scale_2, w_zeros_2, bias,
+                                   room_bytes)
 
 
 # ---- 6-bit float matrix path (no counterpart in the reference) ---------------------------

@@ -145,3 +145,37 @@ def test_short_of_memory(dev):
     assert torch.cuda.max_memory_allocated() - before >= small + y.nbytes
     _lib.host().forget_refused_rooms()
     assert took() >= need
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cls", ["Linear4bitSQ", "Linear4bitDUSQ", "Linear4bitASQ", "LinearQuant4bitDUASQ", "Linear4bitASQRowSum"])
+def test_a_layer_takes_no_more_than_it_may(dev, cls):
+    from duqlinear4bitcuda_amd import _lib
+    from duqlinear4bitcuda_amd import nn as qnn
+    M, N, K = 3072, 4096, 4096
+    need = _room(0, M, N, K)
+    assert need
+    lin = torch.nn.Linear(K, N, bias=True, device=dev, dtype=torch.float16).requires_grad_(False)
+    x = torch.randn(M, K, device=dev, generator=torch.Generator(device=dev).manual_seed(3)).half()
+    s = lin.weight.abs().amax(1, keepdim=True) / 7
+    if cls in ("Linear4bitSQ", "Linear4bitDUSQ"):
+        layer = getattr(qnn, cls).from_float(lin, *((s,) if cls == "Linear4bitSQ" else (s, s))).to(dev)
+        x = qnn.SymQuantizer()(x)
+    else:
+        layer = getattr(qnn, cls).from_linear(lin, False).to(dev)
+        x = qnn.AsymQuantizer(shifted=cls.endswith("RowSum"))(x)
+    assert layer.prefill_room_bytes == 2 << 30
+    _lib.host().forget_refused_rooms()
+    want = None
+    for most, takes in ((2 << 30, True), (need, True), (need - 1, False), (0, False)):
+        layer.prefill_room_bytes = most
+        layer(x)
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        y = layer(x)
+        torch.cuda.synchronize()
+        took = torch.cuda.max_memory_allocated() - before - y.nbytes
+        assert (took >= need) == takes and (takes or took == 0), (most, took)
+        want = y if want is None else want
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16)), most
