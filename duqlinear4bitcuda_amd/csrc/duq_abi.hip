@@ -482,17 +482,19 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
     if (!aligned(workspace, 16)) return DUQ_E_ALIGN;
     if (workspace_bytes < duq_quantize_product_workspace_bytes(mode, batch_count, M, N, K)) return DUQ_E_SHAPE;
     const bool asym = mode == DUQ_EPI_ASYM;
-    if (duq::product_row_takes(M, N, K))
+    duq::ProductPath path, recorded;
+    path = duq::product_path(asym, batch_count, M, N, K, &recorded);
+    if (path != recorded && recording(as_stream(stream))) path = recorded;
+    if (path == duq::kProductRow)
         return duq::launch_product_row(asym, a, b, batch_count, N, K, clip_a, qmax_a, clip_b, qmax_b, y, as_stream(stream));
-    if (duq::product_tiles_takes(asym, batch_count, M, N, K) &&
-        !(duq::product_tiles_eager_only(batch_count, M, N, K) && recording(as_stream(stream))))
+    if (path == duq::kProductTiles)
         return duq::launch_product_tiles(asym, a, b, batch_count, M, N, K, asym ? 1.0f : clip_a, asym ? 15 : qmax_a, asym ? 1.0f : clip_b,
                                          asym ? 15 : qmax_b, y, as_stream(stream));
     uint8_t *q = static_cast<uint8_t *>(workspace);
     duq_half *s = reinterpret_cast<duq_half *>(q + up16(rows * (K / 2)));
     duq_half *z = asym ? s + up16(rows * 2) / 2 : nullptr;
     // (M >= 32: the workspace has the room of whole tiles of B)
-    if (duq::product_long_takes(batch_count, M, N, K))
+    if (path == duq::kProductLong)
         return duq::launch_product_long(asym, a, b, batch_count, M, N, K, asym ? 1.0f : clip_a, asym ? 15 : qmax_a, asym ? 1.0f : clip_b,
                                         asym ? 15 : qmax_b, y, q, s, z, as_stream(stream));
     if (asym || (clip_a == clip_b && qmax_a == qmax_b)) {
@@ -507,6 +509,14 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
     }
     return duq_batch_linear4bit_forward(mode, q, s, z, q + rows_a * (K / 2), s + rows_a, asym ? z + rows_a : nullptr, nullptr, nullptr,
                                         nullptr, batch_count, M, N, K, y, stream);
+}
+
+int duq_product_path_for(int32_t mode, uint32_t batch_count, uint32_t M, uint32_t N, uint32_t K, int32_t recorded)
+{
+    if ((mode != DUQ_EPI_SYM && mode != DUQ_EPI_ASYM) || batch_count == 0 || M == 0 || N == 0 || K == 0 || K % 64 != 0) return 0;
+    duq::ProductPath in_graph;
+    const duq::ProductPath path = duq::product_path(mode == DUQ_EPI_ASYM, batch_count, M, N, K, &in_graph);
+    return recorded ? in_graph : path;
 }
 
 uint32_t duq_product_long_reads_for(uint32_t N, uint32_t K)

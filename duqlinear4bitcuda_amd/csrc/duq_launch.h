@@ -43,6 +43,19 @@ uint32_t product_long_reads(uint32_t N, uint32_t K);
 int launch_product_long(bool asym, const uint16_t *a, const uint16_t *b, uint32_t batch, uint32_t M, uint32_t N, uint32_t K, float clip_a,
                         int qmax_a, float clip_b, int qmax_b, uint16_t *y, uint8_t *q, uint16_t *s, uint16_t *z, hipStream_t stream);
 
+// What runs a product of activations (duq_quantize_product).  Several kernels may take a shape: the first of these that does.  *recorded: what
+// runs it where the call is being recorded into a graph.
+enum ProductPath { kProductRow = 1, kProductTiles, kProductLong, kProductTwoLaunches };
+inline ProductPath product_path(bool asym, uint32_t batch, uint32_t M, uint32_t N, uint32_t K, ProductPath *recorded)
+{
+    const ProductPath separate = product_long_takes(batch, M, N, K) ? kProductLong : kProductTwoLaunches;
+    const ProductPath path = product_row_takes(M, N, K)                    ? kProductRow
+                             : product_tiles_takes(asym, batch, M, N, K) ? kProductTiles
+                                                                         : separate;
+    *recorded = path == kProductTiles && product_tiles_eager_only(batch, M, N, K) ? separate : path;
+    return path;
+}
+
 // Epilogue description shared by the stand-alone dequant kernels and the fused GEMM.
 // mode: 0 sym, 1 asym, 2 sym-dual, 3 asym-dual, 4 asym with row-sum zero-point correction, 5 the same for the
 // dual-uniform layer (fused GEMM only, shapes of gemm_fuses_dual_rowsum) (DUQ_EPI_* of the public header).

@@ -234,6 +234,10 @@ int duq_quantize_product(int32_t mode, const duq_half *a, const duq_half *b, uin
                          float clip_a, int32_t qmax_a, float clip_b, int32_t qmax_b, duq_half *y, void *workspace,
                          uint64_t workspace_bytes, duq_stream_t stream);
 
+/* What runs duq_quantize_product for a shape, called eagerly or (`recorded` not 0) while a graph is recorded: 1 one row of a, in one launch,
+ * 2 short rows, in one launch, 3 long rows and few columns, a launch for b and one for the rest, 4 quantizers and batched GEMM; 0 for an
+ * empty problem, K % 64 != 0 or another mode.  (No GPU work; for tests and tuning.) */
+int duq_product_path_for(int32_t mode, uint32_t batch_count, uint32_t M, uint32_t N, uint32_t K, int32_t recorded);
 /* How many bytes of a problem's codes of b, whole tiles of 32 rows of K / 2 bytes, a workgroup of the launch for long rows reaches
  * (N <= 256, K <= 4096, else 0; no GPU work; for tests). */
 uint32_t duq_product_long_reads_for(uint32_t N, uint32_t K);

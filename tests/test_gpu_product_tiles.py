@@ -65,6 +65,11 @@ def test_against_separate_launches(dev, n, M, N, K):
     assert torch.equal(m(a, b), hip.batch_linear4bit_forward(hip.EPI_SYM, qa, sa, None, qb, sb))
 
 
+@pytest.mark.parametrize("n,M,N,K", [(12, 1100, 2016, 256), (8, 999, 1500, 256)])
+def test_many_rows_of_256(dev, n, M, N, K):
+    test_against_separate_launches(dev, n, M, N, K)
+
+
 # one tile and a few, which a recording runs as two launches, and more
 @pytest.mark.parametrize("n,M,N,K", [(1, 64, 64, 256), (1, 50, 200, 128), (11, 60, 64, 192), (15, 64, 64, 256), (31, 60, 64, 256), (32, 64, 64, 256), (1, 16, 4096, 128), (8, 300, 300, 128)])
 def test_in_a_recording(dev, n, M, N, K):

@@ -1,4 +1,59 @@
 """Rules of the products of activations (csrc/duq_product.hip, csrc/duq_product_long.hip), asked without a GPU."""
+import pytest
+
+ROW, TILES, LONG, TWO = 1, 2, 3, 4
+
+
+def _path(mode, n, M, N, K, recorded=0):
+    from duqlinear4bitcuda_amd import _lib
+    return _lib.load().duq_product_path_for(mode, n, M, N, K, recorded)
+
+
+def _parametrised(name, module):
+    """The shapes of a parametrised test."""
+    import importlib
+    mark, = (m for m in getattr(importlib.import_module(module), name).pytestmark if m.name == "parametrize" and m.args[0] == "n,M,N,K")
+    return mark.args[1]
+
+
+def test_shapes_of_the_short_row_tests_reach_that_kernel():
+    of = lambda name: _parametrised(name, "tests.test_gpu_product_tiles")
+    for shape in of("test_against_the_oracle") + of("test_against_separate_launches"):
+        want = TWO if shape == (8, 2000, 2008, 256) else TILES   # (rows of 256, large outputs whose rows begin anywhere: not that kernel's)
+        assert _path(0, *shape) == _path(1, *shape) == want, shape
+    for shape in of("test_many_rows_of_256"):
+        assert _path(0, *shape) == _path(1, *shape) == TILES, shape
+    for shape in of("test_in_a_recording"):
+        assert _path(1, *shape) == TILES, shape
+    # a recording keeps two launches for a few tiles: both sides of that are there
+    assert [_path(1, *shape, 1) for shape in of("test_in_a_recording")] == [TWO, TWO, TWO, TWO, TWO, TILES, TWO, TILES]
+
+
+def test_shapes_of_the_long_row_tests_reach_that_kernel():
+    of = lambda name: _parametrised(name, "tests.test_gpu_product_long")
+    for shape in of("test_against_the_oracle_and_separate_launches"):
+        assert _path(0, *shape) == _path(1, *shape) == _path(1, *shape, 1) == LONG, shape
+    assert [_path(1, *shape) for shape in of("test_against_separate_launches")] == [LONG] * 4 + [TWO] * 6 + [LONG]
+    assert _path(1, 8, 300, 80, 704) == LONG
+
+
+@pytest.mark.parametrize("there,beside", [
+    # short rows: their length, one row of a, width, rows of 256 where a and the blocks of columns are few (asymmetric), large unaligned outputs
+    ((8, 500, 500, 256), (8, 500, 500, 320)), ((8, 2, 500, 128), (8, 1, 500, 128)), ((1, 100, 1 << 24, 64), (1, 100, (1 << 24) + 1, 64)),
+    ((8, 1024, 1216, 256), (8, 1025, 1216, 256)), ((41, 1025, 256, 256), (40, 1025, 256, 256)), ((8, 1024, 2047, 256), (9, 1024, 2047, 256)),
+    # long rows: their length, columns, problems, rows of a, tiles
+    ((32, 300, 64, 320), (32, 300, 64, 256)), ((32, 300, 64, 4096), (32, 300, 64, 4160)), ((32, 300, 256, 1024), (32, 300, 257, 1024)),
+    ((2, 2048, 64, 1024), (1, 4096, 64, 1024)), ((64, 32, 32, 1024), (64, 31, 31, 1024)), ((8, 256, 256, 1536), (8, 255, 256, 1536)),
+    ((64, 256, 128, 2048), (64, 255, 128, 2048)), ((64, 32, 16, 2048), (63, 32, 16, 2048)), ((128, 32, 16, 2112), (127, 32, 16, 2112)),
+    ((8, 1024, 256, 2048), (8, 992, 256, 2048)), ((8, 4096, 256, 2112), (8, 4064, 256, 2112))])
+def test_either_side_of_the_thresholds(there, beside):
+    short = there[3] <= 256
+    assert _path(1, *there) == (TILES if short else LONG) and _path(1, *beside) in (ROW, TILES, TWO) and _path(1, *there) != _path(1, *beside)
+
+
+def test_no_path_for_what_is_refused():
+    assert [_path(m, *s) for m, s in ((2, (8, 64, 64, 64)), (1, (0, 64, 64, 64)), (1, (8, 0, 64, 64)), (1, (8, 64, 0, 64)),
+                                      (1, (8, 64, 64, 0)), (1, (8, 64, 64, 96)))] == [0] * 6
 
 
 def test_long_rows_read_their_own_codes_only():
