@@ -193,18 +193,56 @@ __global__ __launch_bounds__(512, 4) void product_tiles_kernel(DUQ_HEAD_DECL, Pr
     }
 }
 
-// All rows of up to 256 elements but for a few where the quantizer launch and the short-row kernel are ahead, asymmetric, us: rows of 256
-// on few blocks of columns, where many workgroups quantize the same rows of B (1 x 4090 x 4096 15.7 / 16.9, 8 x 1215 x 1216 15.4 / 15.8, but 12 x
-// 2046 x 2048 42.1 / 39.0), or with large outputs whose rows do not begin at half lines (32 x 2000 x 1992 94.5 / 97.7); in a recording, where a
-// launch costs the host nothing, a few tiles (1 x 64 x 64 x 256 4.9 / 7.0, 8 x 60 x 64 x 256 6.8 / 7.2, 16 x 60 x 64 x 256 7.2 / 7.4, 1 x 64 x 64 x 128 4.9 /
-// 5.6, 1 x 2 x 4096 x 128 5.1 / 5.8, 1 x 16 x 4096 x 128 5.4 / 5.8; eager the first two and the fourth 7.5 / 6.8, 7.5 / 7.0, 7.4 / 5.4).
+// The rows of B cost a workgroup about as much as a tile: the run of tiles that makes the least of rounds of 256 workgroups, the longest
+// of those that are level; a tenth more where a CU has one workgroup alone.  32 x 2048 x 2048 x 128 in one to eight runs 58.8, 55.3, 56.0,
+// 55.3, 60.7 (six), 62.3 us, 8 x 4000 x 4000 x 128 102, 59.7, 59.3, 58.0, 59.1, 56.6.
+struct TileRuns {
+    uint32_t per, splits;  // tiles of a run, runs of 256 columns
+    uint64_t runs, rounds;
+};
+static TileRuns tile_runs(uint32_t batch, uint32_t M, uint32_t N)
+{
+    TileRuns r{};
+    const uint32_t tiles_m = (M + 63) / 64;
+    const uint64_t blocks = (uint64_t)batch * ((N + 255) / 256);
+    uint64_t least = ~0ull;
+    for (uint32_t s = 1; s <= tiles_m && blocks * (s - 1) < 1024; ++s) {
+        const uint32_t per = (tiles_m + s - 1) / s;
+        const uint64_t rounds = (blocks * ((tiles_m + per - 1) / per) + 255) / 256, cost = rounds * (per + 1) * (rounds == 1 ? 11 : 10);
+        if (cost < least) least = cost, r.per = per, r.rounds = rounds;
+    }
+    r.splits = (tiles_m + r.per - 1) / r.per;
+    r.runs = blocks * r.splits;
+    return r;
+}
+
+// All rows of up to 256 elements but for a few where the quantizer launch and the kernel behind it (for a single problem the GEMM of the
+// layers) are ahead, asymmetric, us, two launches / this one:
+//  rows of 256 on few blocks of columns, where many workgroups quantize the same rows of B, and with wide problems, where as many do those
+//   of A: 1 x 4090 x 4096 15.7 / 16.9, 8 x 1215 x 1216 15.4 / 15.8, 1 x 2048 x 12288 22.2 / 24.6, 2 x 3000 x 11520 44.9 / 52.5, but 12 x 2046 x 2048
+//   42.1 / 39.0;
+//  large outputs whose rows do not begin at half lines: 32 x 2000 x 1992 x 256 94.5 / 97.7; single problems of many rows past 150 Mi outputs: 1 x 8192 x 20480 x
+//   128 69.3 / 73.0;
+//  single problems near square whose runs of three tiles (rows of 192: to five) are too few for the CUs, or just too many for one round: 1 x
+//   3067 x 3072 x 128 10.0 / 10.5, 1 x 2493 x 3328 x 128 9.5 / 10.2, 1 x 3581 x 3584 x 192 12.8 / 13.5, 1 x 4221 x 4224 x 192 15.2 / 15.8, symmetric
+//   1 x 3709 x 3712 x 256 14.0 / 14.5, but 1 x 3453 x 3456 x 128 11.2 / 10.4, 1 x 2813 x 2816 x 128 9.5 / 8.5, 1 x 1021 x 9216 x 128 10.7 / 10.0, 1 x 4093 x
+//   4096 x 192 14.5 / 13.7;
+//  in a recording, where a launch costs the host nothing, a few tiles: 1 x 64 x 64 x 256 4.9 / 7.0, 8 x 60 x 64 x 256 6.8 / 7.2, 16 x 60 x 64 x 256 7.2 /
+//   7.4, 1 x 64 x 64 x 128 4.9 / 5.6, 1 x 2 x 4096 x 128 5.1 / 5.8, 1 x 16 x 4096 x 128 5.4 / 5.8; eager the first two and the fourth 7.5 / 6.8,
+//   7.5 / 7.0, 7.4 / 5.4.
 bool product_tiles_takes(bool asym, uint32_t batch, uint32_t M, uint32_t N, uint32_t K)
 {
     if (K == 0 || K > 256 || K % 64 != 0 || M < 2 || N > (1u << 24)) return false;  // (a tile of outputs: 32-bit offsets)
     const uint64_t blocks = (uint64_t)batch * ((N + 255) / 256);
     if (blocks * ((M + 63) / 64) >= (1u << 30)) return false;
     if (K > 192 && N % 32 != 0 && (uint64_t)M * N * batch > (16u << 20)) return false;
-    return !(asym && K > 192 && M > 1024 && blocks <= 40);
+    if (asym && K > 192 && M > 1024 && (blocks <= 40 || batch == 1 || N > 6144)) return false;
+    if (batch != 1) return true;
+    if (M > 1024 && (uint64_t)M * N > (150u << 20)) return false;
+    if (K <= 64 || M < 2048 || N < 2048 || !(asym || K > 192)) return true;
+    const TileRuns r = tile_runs(batch, M, N);
+    if (r.rounds == 1) return !(r.per >= 3 && r.per <= (K <= 128 ? 3u : 5u) && r.runs <= (r.per == 3 ? 224u : 228u));
+    return !(asym && r.rounds == 2 && r.per == 1);
 }
 
 bool product_tiles_eager_only(uint32_t batch, uint32_t M, uint32_t N, uint32_t K)
@@ -230,19 +268,10 @@ int launch_product_tiles(bool asym, const uint16_t *a, const uint16_t *b, uint32
     // (the rule of gemm_s4_shortk_kernel's stores)
     const bool past = batch > 1 ? N % 32 == 0 || K > 192 : N % 32 == 0 ? K > 128 : K > 192 && (uint64_t)M * N > (128u << 20);
     p.streamed = past || N % 64 == 0 || (uint64_t)M * N * batch <= (16u << 20);
-    // The rows of B cost a workgroup about as much as a tile: the run of tiles that makes the least of rounds of 256 workgroups, the longest
-    // of those that are level; a tenth more where a CU has one workgroup alone.  32 x 2048 x 2048 x 128 in one to eight runs 58.8, 55.3, 56.0,
-    // 55.3, 60.7 (six), 62.3 us, 8 x 4000 x 4000 x 128 102, 59.7, 59.3, 58.0, 59.1, 56.6.
-    const uint32_t tiles_m = (M + 63) / 64;
-    const uint64_t blocks = (uint64_t)batch * p.tiles_n;
-    uint64_t least = ~0ull;
-    for (uint32_t s = 1; s <= tiles_m && blocks * (s - 1) < 1024; ++s) {
-        const uint32_t per = (tiles_m + s - 1) / s;
-        const uint64_t rounds = (blocks * ((tiles_m + per - 1) / per) + 255) / 256, cost = rounds * (per + 1) * (rounds == 1 ? 11 : 10);
-        if (cost < least) least = cost, p.per = per;
-    }
-    p.splits = (tiles_m + p.per - 1) / p.per;
-    p.units = (uint32_t)(blocks * p.splits);
+    const TileRuns r = tile_runs(batch, M, N);
+    p.per = r.per;
+    p.splits = r.splits;
+    p.units = (uint32_t)r.runs;
 #define DUQ_TILES(NP)                                                                                                     \
     do {                                                                                                                  \
         if (asym) DUQ_LAUNCH_HEAD((product_tiles_kernel<NP, true>), dim3(p.units), dim3(512), 0, stream, p);              \

@@ -51,6 +51,19 @@ def test_either_side_of_the_thresholds(there, beside):
     assert _path(1, *there) == (TILES if short else LONG) and _path(1, *beside) in (ROW, TILES, TWO) and _path(1, *there) != _path(1, *beside)
 
 
+# single problems: runs of three to five tiles for most of the CUs but not for all, runs of one in a second round, rows of 256 (asymmetric),
+# outputs past what the last-level cache holds
+@pytest.mark.parametrize("mode,there,beside", [
+    (1, (3453, 3456, 128), (3067, 3072, 128)), (1, (2813, 2816, 128), (2941, 2944, 128)), (1, (3581, 3584, 128), (3197, 3200, 128)),
+    (1, (2047, 4096, 128), (2049, 4096, 128)), (1, (4605, 1792, 128), (4605, 2048, 128)), (1, (3069, 3072, 64), (3069, 3072, 128)),
+    (1, (2397, 3200, 128), (2493, 3328, 128)), (1, (4093, 4096, 192), (3581, 3584, 192)), (1, (4605, 4608, 192), (4029, 4352, 192)),
+    (0, (4093, 4096, 256), (3709, 3712, 256)), (0, (4029, 4352, 192), (4029, 4352, 256)), (1, (1024, 20480, 256), (1025, 20480, 256)),
+    (0, (8192, 19200, 128), (8192, 19201, 128))])
+def test_single_problems(mode, there, beside):
+    assert (_path(mode, 1, *there), _path(mode, 1, *beside)) == (TILES, TWO)
+    assert _path(mode, 2, *beside) == (TWO if mode and beside[2] > 192 and beside[1] > 6144 else TILES)
+
+
 def test_no_path_for_what_is_refused():
     assert [_path(m, *s) for m, s in ((2, (8, 64, 64, 64)), (1, (0, 64, 64, 64)), (1, (8, 0, 64, 64)), (1, (8, 64, 0, 64)),
                                       (1, (8, 64, 64, 0)), (1, (8, 64, 64, 96)))] == [0] * 6
