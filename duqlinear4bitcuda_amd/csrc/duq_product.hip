@@ -265,9 +265,7 @@ int launch_product_tiles(bool asym, const uint16_t *a, const uint16_t *b, uint32
     p.qmax_a = qmax_a;
     p.clip_b = clip_b;
     p.qmax_b = qmax_b;
-    // (the rule of gemm_s4_shortk_kernel's stores)
-    const bool past = batch > 1 ? N % 32 == 0 || K > 192 : N % 32 == 0 ? K > 128 : K > 192 && (uint64_t)M * N > (128u << 20);
-    p.streamed = past || N % 64 == 0 || (uint64_t)M * N * batch <= (16u << 20);
+    p.streamed = streams_short_rows(M, N, K, batch);
     const TileRuns r = tile_runs(batch, M, N);
     p.per = r.per;
     p.splits = r.splits;

@@ -69,7 +69,7 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // -> 78.4, 4078 x 13360 x 832 91.7 -> 82.2, 1999 x 11024 x 4096 80.0 -> 74.0; 6-bit floats 80.3 -> 67.8, 61.6 -> 53.9, 59.2 -> 56.2).  The output
 // is that of all problems of a launch (8 of 2000 x 2008 x 512 43.3 -> 35.1, 16 of 1000 x 1992 x 640 48.2 -> 39.6, 32 of 1000 x 1000 x 1024 51.6
 // -> 43.9, 8 of 2048 x 2056 x 2048 83.1 -> 80.9; the least 5 of 2000 x 2008 x 512 23.0 -> 23.4).
-__device__ __forceinline__ bool few_or_whole_lines(uint32_t M, uint32_t N, uint32_t problems = 1)
+__host__ __device__ __forceinline__ bool few_or_whole_lines(uint32_t M, uint32_t N, uint32_t problems = 1)
 {
     return N % 64 == 0 || (uint64_t)M * N * problems <= (16u << 20);
 }
@@ -83,6 +83,21 @@ __device__ __forceinline__ bool few_or_whole_lines(uint32_t M, uint32_t N, uint3
 __device__ __forceinline__ bool streams_outputs(uint32_t M, uint32_t N, uint32_t problems, uint32_t most)
 {
     return few_or_whole_lines(M, N, problems) || (uint64_t)M * N * problems > most;
+}
+
+// Products of short rows (K up to 256), whose instructions store 512 bytes of a row, two parts of cache lines at most.  Batches: into the L2 only
+// where rows do not begin at half lines and are of 192 elements at most.  Asymmetric, past the L2 / into it, us: 32 x 2000 x
+// 1992 x 64 74.7 / 42.4, x 128 73.2 / 50.0, x 192 70.9 / 58.6, x 256 65.3 / 76.4; 32 x 2000 x 2016 x 128 48.8 / 52.1; the
+// largest loss 10 x 4000 x 4040 x 192 89 / 93.
+// One problem: past it only where rows of more than 128 elements begin at half lines, or the outputs of rows of more than 192
+// are larger than the last-level cache (8192 x 28704 x 256 108 / 151, x 192 91 / 129, x 128 94 / 107, but 8192 x 14368 x 128 47 / 42; 8192 x
+// 28680 x 256 152 / 169, but x 192 136 / 131 and 8192 x 14344 x 256 71 / 66; 8192 x 10248 x 128 49 / 29).
+__host__ __device__ __forceinline__ bool streams_short_rows(uint32_t M, uint32_t N, uint32_t K, uint32_t problems)
+{
+    const bool past = problems > 1   ? N % 32 == 0 || K > 192
+                      : N % 32 == 0 ? K > 128
+                                    : K > 192 && (uint64_t)M * N > (128u << 20);
+    return past || few_or_whole_lines(M, N, problems);
 }
 
 // Stages of the LDS kernels (duq_decode.hip, duq_int8.hip): MT row tiles and NT column tiles of 16 per workgroup of eight
