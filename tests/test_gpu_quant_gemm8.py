@@ -88,3 +88,41 @@ def test_layer_replayed_as_a_graph(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+def test_every_tile_that_the_rule_gives_has_its_kernel():
+    """A tile without one would end the call in an error.  (Eight pieces of four elements or sixteen for a lane, one chunk of columns or
+    several: what there are kernels for, and what the shapes above run.)"""
+    import os
+    import re
+
+    path = os.path.join(os.path.dirname(__file__), "..", "duqlinear4bitcuda_amd", "csrc", "duq_quant_gemm8.hip")
+    there = {(int(r), int(u), int(c), b == "2") for r, u, c, b in re.findall(r"^    DUQ_Q8\((\d+), (\d+), (\d+), (\d+)\)$", open(path).read(), re.M)}
+    kind = lambda rows, cols, chunks, K: (rows, 8 if rows * K <= 16384 else 16, cols, chunks > 1)
+    assert {kind(*t, s[2]) for t, s in SHAPES + MORE} == there and len(there) == 14
+    seen = set()
+    for M in [*range(3, 34), 40, 63, 64, 65, 100, 128, 129, 200, 256, 257, 500, 512, 513, 700, 1000, 1024, 1025, 1536, 2000, 2047, 2048, 2049]:
+        for N in (1, 16, 17, 33, 48, 64, 65, 128, 200, 300, 512, 1000, 2048, 2053, 4096, 4097, 8192, 8193, 12288, 16384, 28672, 65536, 65537):
+            for K in range(32, 4129, 32):
+                tile = _tile(M, N, K)
+                if tile[0]:
+                    seen.add(kind(*tile, K))
+                else:
+                    assert tile == (0, 0, 0)
+    assert seen == there
+
+
+# the rest of the tiles: eight rows of at most 2048 elements, sixteen of more than 1024
+MORE = [((8, 1, 1), (8, 4001, 1024)), ((8, 1, 1), (5, 436, 1600)), ((8, 1, 1), (7, 130, 2048)), ((16, 1, 1), (9, 2053, 1056)), ((16, 1, 1), (33, 1297, 1504))]
+
+
+@pytest.mark.parametrize("tile,shape", MORE)
+def test_more_shapes_reach_their_tile(tile, shape):
+    assert _tile(*shape) == tile
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("i", range(len(MORE)))
+def test_more_tiles_against_the_oracle(hip, dev, monkeypatch, i):  # noqa: F811
+    monkeypatch.setitem(globals(), "SHAPES", MORE)
+    test_tiles_against_the_oracle(hip, dev, i)
