@@ -55,6 +55,7 @@ PROTOTYPES = {
     "duq_gemm_kernel_for": [_c_u32, _c_u32, _c_u32],
     "duq_gemm_stream_tile_for": [_c_u32, _c_u32, _c_u32],
     "duq_quant_gemm_tile_for": [_c_u32, _c_u32, _c_u32],
+    "duq_quantize_linear4bit_path_for": [_c_i32, _c_u32, _c_u32, _c_u32, _c_i32],
     "duq_gemm_plan_for": [_c_i32, _c_u32, _c_u32, _c_u32, _c_p],
     "duq_gemm_bf6_plan_for": [_c_i32, _c_u32, _c_u32, _c_u32, _c_p],
     "duq_quant_gemm8_tile_for": [_c_u32, _c_u32, _c_u32],

@@ -361,6 +361,15 @@ inline bool leaves_few_rows(uint32_t M, uint32_t N, uint32_t K, bool asym, bool 
     if (M > 4 || K <= 2048 || rowsum || !decode_fp16in_one_launch(M, N, K)) return false;
     return K <= 4096 || (K > 6144 && (N <= 2048 || !asym)) || (M <= 3 && N <= 2048 && !asym);
 }
+// The tile that runs a layer's call from binary16 rows, by the layer's quantizer (rows = 0: the rows kernel, or two launches).  A call that
+// brings no room for codes is one launch in a recording too.
+inline QuantGemmShape quant_gemm_tile(uint32_t M, uint32_t N, uint32_t K, bool asym, bool rowsum)
+{
+    QuantGemmShape s = quant_gemm_shape(M, N, K);
+    if (leaves_few_rows(M, N, K, asym, rowsum)) return QuantGemmShape{0, 0, 0};
+    if (decode_fp16in_one_launch(M, N, K)) s.eager_only = false;
+    return s;
+}
 // q_out / s_out / z_out / rs_out as above.
 int launch_quant_gemm(QuantGemmShape s, const uint16_t *x, float clip, int qmax, const uint8_t *B, uint32_t M, uint32_t N, uint32_t K,
                       const Epilogue &epi, uint16_t *y, uint8_t *q_out, uint16_t *s_out, uint16_t *z_out, int32_t *rs_out,

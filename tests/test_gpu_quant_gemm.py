@@ -156,6 +156,29 @@ def test_recorded_calls(hip, dev, M, N, K, launches):  # noqa: F811
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+def test_the_query_says_what_runs():
+    """Over every mode, eager and recorded: two launches only where the caller is asked for room, a tile that is given up in a recording only
+    there, and the rows kernel where three and four rows of a quantizer without sums are ahead on it."""
+    from duqlinear4bitcuda_amd import _lib
+
+    lib = _lib.load()
+    path = lib.duq_quantize_linear4bit_path_for
+    for M in [1, 2, 3, 4, 5, 8, 9, 13, 16, 17, 32, 64, 200, 1000, 2048, 2049]:
+        for N in (1, 1000, 2048, 2049, 4096, 4097, 12288, 12289, 16384, 16385, 28672):
+            for K in (64, 1024, 2048, 2112, 4096, 4160, 6144, 6208, 8192, 8256, 11008):
+                tile = lib.duq_quant_gemm_tile_for(M, N, K)
+                for mode in range(6):
+                    room = lib.duq_quantize_linear4bit_workspace_bytes(M, N, K) if mode in (0, 2) else \
+                        lib.duq_quantize_linear4bit_asym_workspace_bytes(mode, M, N, K)
+                    eager, recorded = path(mode, M, N, K, 0), path(mode, M, N, K, 1)
+                    assert (eager, recorded) in ((1, 1), (2, 2), (2, 3), (3, 3)) and (room or 3 not in (eager, recorded)), (mode, M, N, K)
+                    assert (recorded != eager) == bool(tile >> 24), (mode, M, N, K)
+                    assert (eager == 2) == bool(tile) or (M in (3, 4) and mode < 4 and eager == 1), (mode, M, N, K)
+    assert [path(m, 3, 4096, 4096, 0) for m in range(6)] == [1, 1, 1, 1, 2, 2] and path(0, 3, 4096, 2048, 0) == path(1, 4, 4096, 8192, 0) == 2
+    assert path(1, 3, 12289, 2112, 1) == 1 and path(4, 3, 12289, 2112, 1) == 2   # (no room: no two launches)
+    assert path(6, 3, 64, 64, 0) == path(0, 0, 64, 64, 0) == path(0, 3, 64, 96, 0) == 0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(20, 1000, 1024), (100, 300, 4096), (300, 700, 512), (60, 12001, 512)])
 @pytest.mark.parametrize("mode", range(6))
