@@ -82,8 +82,8 @@ int check_gemm(const void *A, const void *B, uint32_t M, uint32_t N, uint32_t K)
 }
 
 // quantize + GEMM + dequant from binary16 activations: one launch for decode shapes, otherwise the quantizer
-// into `workspace` (codes, scales, then zero points and row sums for the asymmetric modes) followed by the GEMM, or one kernel
-// (quant_gemm_shape), which writes only what `out` asks for.
+// into `workspace` (codes, scales, then zero points and row sums for the asymmetric modes) followed by the GEMM, or one kernel that
+// leaves the same there (quant_gemm_shape).
 // The epilogue mode decides the quantizer: symmetric for DUQ_EPI_SYM / SYM_DUAL, asymmetric for DUQ_EPI_ASYM /
 // ASYM_DUAL, its signed-shifted form for DUQ_EPI_ASYM_ROWSUM.
 struct FusedOut {
@@ -107,7 +107,7 @@ uint64_t staging_bytes(int32_t mode, uint32_t M, uint32_t N, uint32_t K)
 
 int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t qmax, const uint8_t *w, uint32_t M,
                          uint32_t N, uint32_t K, duq_half *y, FusedOut out, void *workspace, uint64_t workspace_bytes,
-                         duq_stream_t stream, FusedOut room = {})
+                         duq_stream_t stream)
 {
     const int32_t mode = e.mode;
     const bool asym = mode == DUQ_EPI_ASYM || mode == DUQ_EPI_ASYM_DUAL || mode >= DUQ_EPI_ASYM_ROWSUM;
@@ -135,44 +135,43 @@ int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t
                                                       rowsum ? out.rowsum : nullptr, as_stream(stream));
     };
     if (no_room) return launch_one();
-    // codes and per-token parameters go to the caller's outputs where given, else to `room` where that has a place, else to the workspace
-    FusedOut at{out.q ? out.q : room.q, out.scale ? out.scale : room.scale, out.zeros, out.rowsum};
+    // codes and per-token parameters go to the caller's outputs where given, else to the workspace
     const bool acc_ws = mode == DUQ_EPI_ASYM_DUAL_ROWSUM && !duq::gemm_fuses_dual_rowsum(M, N, K);
-    const bool need_ws = !at.q || !at.scale || (asym && !at.zeros) || (rowsum && !at.rowsum) || acc_ws;
+    const bool need_ws = !out.q || !out.scale || (asym && !out.zeros) || (rowsum && !out.rowsum) || acc_ws;
     int32_t *acc = nullptr;
     if (need_ws) {
         if (!workspace) return DUQ_E_NULL;
         if (!aligned(workspace, 16)) return DUQ_E_ALIGN;
         if (workspace_bytes < staging_bytes(mode, M, N, K)) return DUQ_E_SHAPE;
-        uint8_t *p = static_cast<uint8_t *>(workspace);
-        if (!at.q) at.q = p;
-        p += up16((uint64_t)M * (K / 2));
-        if (!at.scale) at.scale = reinterpret_cast<duq_half *>(p);
-        p += up16((uint64_t)M * 2);
-        if (asym && !at.zeros) at.zeros = reinterpret_cast<duq_half *>(p);
-        p += up16((uint64_t)M * 2);
-        if (rowsum && !at.rowsum) at.rowsum = reinterpret_cast<int32_t *>(p);
-        p += up16((uint64_t)M * 4);
-        if (acc_ws) acc = reinterpret_cast<int32_t *>(p);
+        uint8_t *at = static_cast<uint8_t *>(workspace);
+        if (!out.q) out.q = at;
+        at += up16((uint64_t)M * (K / 2));
+        if (!out.scale) out.scale = reinterpret_cast<duq_half *>(at);
+        at += up16((uint64_t)M * 2);
+        if (asym && !out.zeros) out.zeros = reinterpret_cast<duq_half *>(at);
+        at += up16((uint64_t)M * 2);
+        if (rowsum && !out.rowsum) out.rowsum = reinterpret_cast<int32_t *>(at);
+        at += up16((uint64_t)M * 4);
+        if (acc_ws) acc = reinterpret_cast<int32_t *>(at);
     }
     if (one_kernel) return launch_one();
     int st;
     if (!asym)
-        st = duq::launch_quantize_rows_sym(x, M, K, clip, qmax, at.q, at.scale, nullptr, as_stream(stream));
+        st = duq::launch_quantize_rows_sym(x, M, K, clip, qmax, out.q, out.scale, nullptr, as_stream(stream));
     else
-        st = duq::launch_quantize_rows_asym(x, M, K, at.q, at.scale, at.zeros, rowsum ? at.rowsum : nullptr, nullptr,
+        st = duq::launch_quantize_rows_asym(x, M, K, out.q, out.scale, out.zeros, rowsum ? out.rowsum : nullptr, nullptr,
                                             as_stream(stream));
     if (st) return st;
-    e.s_row = at.scale;
-    e.z_row = asym ? at.zeros : nullptr;
-    e.rs_row = rowsum ? at.rowsum : nullptr;
+    e.s_row = out.scale;
+    e.z_row = asym ? out.zeros : nullptr;
+    e.rs_row = rowsum ? out.rowsum : nullptr;
     if (acc_ws && !duq::gemm_applies_dual_rowsum(M, N, K)) {  // GEMM into int32, then the stand-alone epilogue
-        if (int st2 = duq::launch_gemm_s4(at.q, w, M, N, K, acc, nullptr, nullptr, as_stream(stream))) return st2;
-        duq::DualRowsumParams dp{acc,       at.q,     w,         K / 2,    at.scale, at.zeros, at.rowsum, e.s_col_1, e.z_col_1,
+        if (int st2 = duq::launch_gemm_s4(out.q, w, M, N, K, acc, nullptr, nullptr, as_stream(stream))) return st2;
+        duq::DualRowsumParams dp{acc,       out.q,     w,         K / 2,    out.scale, out.zeros, out.rowsum, e.s_col_1, e.z_col_1,
                                  e.s_col_2, e.z_col_2, e.rs_col,  e.rs_col_2, e.bias,  M,         N,          y};
         return duq::launch_dual_rowsum_dequant(dp, as_stream(stream));
     }
-    return duq::launch_gemm_s4(at.q, w, M, N, K, nullptr, &e, y, as_stream(stream));
+    return duq::launch_gemm_s4(out.q, w, M, N, K, nullptr, &e, y, as_stream(stream));
 }
 
 }  // namespace
@@ -666,18 +665,19 @@ int duq_quantize_linear4bit_forward_static(int32_t mode, const duq_half *x, floa
     if (mode != DUQ_EPI_SYM && mode != DUQ_EPI_SYM_DUAL) return DUQ_E_MODE;
     if (slot >= DUQ_STATIC_SCRATCH_SLOTS) return DUQ_E_SCRATCH;
     if ((uint64_t)M * (K / 2) > DUQ_STATIC_SCRATCH_CODE_BYTES || M > DUQ_STATIC_SCRATCH_ROWS) return DUQ_E_SCRATCH;
-    FusedOut room{};
+    uint8_t *q = q_out;
+    duq_half *sc = scale_out;
     const bool staged = M != 0 && N != 0 && K != 0 && !duq::decode_fp16in_one_launch(M, N, K) && (!q_out || !scale_out);
     if (staged) {
         unsigned char *ws = nullptr;
         if (int e = static_scratch(as_stream(stream), &ws)) return e;
         ws += (uint64_t)slot * kSlotBytes;
         // codes at the start of the slot, scales behind the largest code block: both offsets keep the 256-byte alignment
-        room.q = ws;
-        room.scale = reinterpret_cast<duq_half *>(ws + DUQ_STATIC_SCRATCH_CODE_BYTES);
+        if (!q) q = ws;
+        if (!sc) sc = reinterpret_cast<duq_half *>(ws + DUQ_STATIC_SCRATCH_CODE_BYTES);
     }
     duq::Epilogue e{mode, nullptr, nullptr, w_scale_1, nullptr, w_scale_2, nullptr, bias, nullptr, nullptr};
-    return quantize_linear_impl(e, x, clip, qmax, w, M, N, K, y, FusedOut{q_out, scale_out, nullptr, nullptr}, nullptr, 0, stream, room);
+    return quantize_linear_impl(e, x, clip, qmax, w, M, N, K, y, FusedOut{q, sc, nullptr, nullptr}, nullptr, 0, stream);
 }
 
 int duq_asym_rowsum_dequant_host(const int32_t *q, const duq_half *scale_row, const duq_half *zeros_row,
