@@ -125,7 +125,7 @@ int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t
     if (rowsum && !e.rs_col) return DUQ_E_NULL;
     if (mode == DUQ_EPI_ASYM_DUAL_ROWSUM && !e.rs_col_2) return DUQ_E_NULL;
     if ((out.q && !aligned(out.q, 16))) return DUQ_E_ALIGN;
-    const duq::QuantGemmShape tile = duq::quant_gemm_tile(M, N, K, asym, rowsum);
+    const duq::QuantGemmShape tile = duq::quant_gemm_tile(M, N, K, mode);
     const bool no_room = duq::decode_fp16in_one_launch(M, N, K);  // (the caller was asked for none)
     const bool one_kernel = tile.rows != 0 && !(tile.eager_only && recording(as_stream(stream)));
     auto launch_one = [&] {
@@ -542,15 +542,14 @@ int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K)
 
 int duq_quant_gemm_tile_for(uint32_t M, uint32_t N, uint32_t K)
 {
-    const duq::QuantGemmShape t = duq::quant_gemm_tile(M, N, K, true, true);
+    const duq::QuantGemmShape t = duq::quant_gemm_tile(M, N, K);
     return (int)(t.rows + 256 * t.cols + 65536 * t.chunks + ((uint32_t)t.eager_only << 24));
 }
 
 int duq_quantize_linear4bit_path_for(int32_t mode, uint32_t M, uint32_t N, uint32_t K, int32_t recorded)
 {
     if (mode < DUQ_EPI_SYM || mode > DUQ_EPI_ASYM_DUAL_ROWSUM || M == 0 || N == 0 || K == 0 || K % 64 != 0) return 0;
-    const bool asym = mode != DUQ_EPI_SYM && mode != DUQ_EPI_SYM_DUAL;
-    const duq::QuantGemmShape t = duq::quant_gemm_tile(M, N, K, asym, mode >= DUQ_EPI_ASYM_ROWSUM);
+    const duq::QuantGemmShape t = duq::quant_gemm_tile(M, N, K, mode);
     if (t.rows && !(t.eager_only && recorded)) return 2;
     return duq::decode_fp16in_one_launch(M, N, K) ? 1 : 3;
 }

@@ -351,24 +351,37 @@ inline QuantGemmShape quant_gemm_shape(uint32_t M, uint32_t N, uint32_t K)
     if (K > 2048 && K <= 4096) offer(16, 1, 4, 4.0f + 0.62f * k, 1.0f);
     return best;
 }
-// Three and four rows of more than 2048 elements whose quantizer delivers no row sums: the rows kernel, which splits a row's quantization over
-// all its wavefronts, is ahead up to 4096 elements, and beyond on narrow layers (graph, us, rows kernel / this one; 3 rows symmetric, 4
-// symmetric, 4 asymmetric, 4 with row sums: N x K 4096 x 2048 3.88 / 3.70, 3.89 / 3.72, 4.11 / 3.89, 4.45 / 4.09; 4096 x 3072 3.88 / 4.12, 3.90 / 4.16, 4.13
-// / 4.34, 4.50 / 4.51; 4096 x 4096 3.96 / 4.37, 3.98 / 4.41, 4.37 / 4.49, 4.95 / 4.62; 1024 x 4160 4.73 / 4.93, 5.17 / 4.94, 5.60 / 5.27, 6.03 / 5.39; 1024 x
-// 8192 4.79 / 5.63, 5.32 / 5.68, 5.89 / 6.16, 6.43 / 6.19; 4096 x 8192 5.91 / 6.14, 6.19 / 6.13, 6.81 / 6.34, 7.43 / 6.39).
-inline bool leaves_few_rows(uint32_t M, uint32_t N, uint32_t K, bool asym, bool rowsum)
+// Three and four rows of more than 2048 elements: the rows kernel, which splits a row's quantization over all its wavefronts, is ahead of the
+// tile where that quantization counts for more than the products, and where the tile is one of sixteen rows for a few.  Up to 4096 elements
+// without row sums 4096 x 3072 3.88 / 4.12 us (rows kernel / tile, three rows, symmetric, in a graph), 4096 x 4096 3.96 / 4.37, asymmetric 4.27 /
+// 4.45.  Its time over the tile's, three rows and four:
+//  symmetric, 3000 columns: 4160 elements 1.02, 1.05; 5120 0.99, 1.04; 5632 0.94, 0.98; 6144 0.95, 0.98
+//  asymmetric, 3000 columns: 4160 0.99, 1.02; 5120 0.97, 1.01; 5632 0.96, 0.99; 6144 0.94, 0.98; 7168 0.88, 0.92
+//  row sums, 1000 columns: 5120 1.00, 1.05; 5632 0.96, 1.03; 6208 0.92, 0.97; 8192 0.93, 0.97 (four rows, 3000 columns 1.01); 13000 columns: 2560
+//   0.94, 3840 0.95, 4032 1.09, 4096 0.98 (called eagerly 0.91); 12288 columns: 3072 1.14
+//  dual row sums, 1500 columns: 3072 1.00, 3456 0.98, 4096 0.95 (4200 columns: 4032 1.23); 300 columns: 6208 0.96, 1.01; 3000 columns: 8192 1.05, 1.08
+inline bool leaves_few_rows(uint32_t M, uint32_t N, uint32_t K, int mode)
 {
-    if (M > 4 || K <= 2048 || rowsum || !decode_fp16in_one_launch(M, N, K)) return false;
-    return K <= 4096 || (K > 6144 && (N <= 2048 || !asym)) || (M <= 3 && N <= 2048 && !asym);
+    if (M > 4 || K <= 2048 || !decode_fp16in_one_launch(M, N, K)) return false;
+    if (mode < 4) return K <= 4096 || M <= 3 || K > 5632;
+    if (mode == 4) {
+        if (K <= 4096) return N > 12288 && (K <= 3840 || K % 2048 == 0);
+        return M <= 3 ? K > 5120 : K > 6144 && N <= 2048;
+    }
+    return K <= 4096 ? K > 3264 && N <= 4096 : M <= 3 && K > 6144 && N <= 2048;
 }
-// The tile that runs a layer's call from binary16 rows, by the layer's quantizer (rows = 0: the rows kernel, or two launches).  A call that
-// brings no room for codes is one launch in a recording too.
-inline QuantGemmShape quant_gemm_tile(uint32_t M, uint32_t N, uint32_t K, bool asym, bool rowsum)
+// The tile of a call from binary16 rows (rows = 0: the rows kernel, or two launches).  A call that brings no room for codes is one launch in a
+// recording too.
+inline QuantGemmShape quant_gemm_tile(uint32_t M, uint32_t N, uint32_t K)
 {
     QuantGemmShape s = quant_gemm_shape(M, N, K);
-    if (leaves_few_rows(M, N, K, asym, rowsum)) return QuantGemmShape{0, 0, 0};
     if (decode_fp16in_one_launch(M, N, K)) s.eager_only = false;
     return s;
+}
+// The same for an epilogue mode.
+inline QuantGemmShape quant_gemm_tile(uint32_t M, uint32_t N, uint32_t K, int mode)
+{
+    return leaves_few_rows(M, N, K, mode) ? QuantGemmShape{0, 0, 0} : quant_gemm_tile(M, N, K);
 }
 // q_out / s_out / z_out / rs_out as above.
 int launch_quant_gemm(QuantGemmShape s, const uint16_t *x, float clip, int qmax, const uint8_t *B, uint32_t M, uint32_t N, uint32_t K,

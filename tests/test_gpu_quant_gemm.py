@@ -73,6 +73,12 @@ def test_few_long_rows(hip, dev, M, N, K):  # noqa: F811
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(3, 4097, 3392), (4, 1000, 4096), (3, 13001, 2560), (4, 12289, 4032), (3, 333, 5696), (4, 2049, 6208), (4, 400, 7168)])
+def test_more_long_rows(hip, dev, M, N, K):  # noqa: F811
+    test_few_long_rows(hip, dev, M, N, K)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(20, 40, 2112), (33, 2700, 2048), (500, 2001, 960), (40, 4000, 4096)])
 def test_rows_that_are_not_finite_beside_rows_that_are(hip, dev, M, N, K):  # noqa: F811
     """A wavefront holds several rows: a zero row, an infinity and a NaN among them, and a scale that underflows."""
@@ -156,7 +162,7 @@ def test_recorded_calls(hip, dev, M, N, K, launches):  # noqa: F811
 
 def test_the_query_says_what_runs():
     """Over every mode, eager and recorded: two launches only where the caller is asked for room, a tile that is given up in a recording only
-    there, and the rows kernel where three and four rows of a quantizer without sums are ahead on it."""
+    there, and the rows kernel where three and four long rows are ahead on it."""
     from duqlinear4bitcuda_amd import _lib
 
     lib = _lib.load()
@@ -170,8 +176,14 @@ def test_the_query_says_what_runs():
                         lib.duq_quantize_linear4bit_asym_workspace_bytes(mode, M, N, K)
                     eager, recorded = path(mode, M, N, K, 0), path(mode, M, N, K, 1)
                     assert (eager, recorded) in ((1, 1), (2, 2), (2, 3), (3, 3)) and (room or 3 not in (eager, recorded)), (mode, M, N, K)
-                    assert (recorded != eager) == bool(tile >> 24), (mode, M, N, K)
-                    assert (eager == 2) == bool(tile) or (M in (3, 4) and mode < 4 and eager == 1), (mode, M, N, K)
-    assert [path(m, 3, 4096, 4096, 0) for m in range(6)] == [1, 1, 1, 1, 2, 2] and path(0, 3, 4096, 2048, 0) == path(1, 4, 4096, 8192, 0) == 2
-    assert path(1, 3, 12289, 2112, 1) == 1 and path(4, 3, 12289, 2112, 1) == 2   # (no room: no two launches)
+                    assert (recorded != eager) == bool(tile >> 24) or eager == 1, (mode, M, N, K)
+                    assert (eager == 2) == bool(tile) or (M in (3, 4) and K > 2048 and eager == 1), (mode, M, N, K)
+    assert [path(m, 3, 4096, 4096, 0) for m in range(6)] == [1, 1, 1, 1, 2, 1] and path(0, 3, 4096, 2048, 0) == path(1, 4, 4096, 5120, 0) == 2
+    assert path(4, 3, 12289, 4032, 1) == path(5, 4, 12289, 2112, 1) == 2   # (no room: no two launches)
+    for mode, there, beside in ((0, (4, 4096, 5632), (4, 4096, 5696)), (1, (4, 4096, 4160), (3, 4096, 4160)), (2, (4, 300, 4160), (4, 300, 4096)),
+                                (4, (3, 12288, 3072), (3, 12289, 3072)), (4, (3, 1000, 5120), (3, 1000, 5184)), (4, (4, 2049, 6208), (4, 2048, 6208)),
+                                (4, (4, 1000, 6144), (4, 1000, 6208)), (4, (4, 13000, 3904), (4, 13000, 3840)), (4, (4, 13000, 4032), (4, 13000, 4096)),
+                                (5, (4, 4097, 4096), (4, 4096, 4096)), (5, (3, 1000, 3264), (3, 1000, 3328)), (5, (4, 1000, 6208), (3, 1000, 6208)),
+                                (5, (3, 2049, 8192), (3, 2048, 8192))):
+        assert (path(mode, *there, 0), path(mode, *beside, 0)) == (2, 1), (mode, there, beside)
     assert path(6, 3, 64, 64, 0) == path(0, 0, 64, 64, 0) == path(0, 3, 64, 96, 0) == 0
