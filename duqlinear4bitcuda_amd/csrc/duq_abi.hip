@@ -82,8 +82,8 @@ int check_gemm(const void *A, const void *B, uint32_t M, uint32_t N, uint32_t K)
 }
 
 // quantize + GEMM + dequant from binary16 activations: one launch for decode shapes, otherwise the quantizer
-// into `workspace` (codes, scales, then zero points and row sums for the asymmetric modes) followed by the GEMM, or one kernel that
-// leaves the same there (quant_gemm_shape).
+// into `workspace` (codes, scales, then zero points and row sums for the asymmetric modes) followed by the GEMM, or one kernel
+// (quant_gemm_shape) that leaves the same there where `staged` says that the caller may look.
 // The epilogue mode decides the quantizer: symmetric for DUQ_EPI_SYM / SYM_DUAL, asymmetric for DUQ_EPI_ASYM /
 // ASYM_DUAL, its signed-shifted form for DUQ_EPI_ASYM_ROWSUM.
 struct FusedOut {
@@ -107,7 +107,7 @@ uint64_t staging_bytes(int32_t mode, uint32_t M, uint32_t N, uint32_t K)
 
 int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t qmax, const uint8_t *w, uint32_t M,
                          uint32_t N, uint32_t K, duq_half *y, FusedOut out, void *workspace, uint64_t workspace_bytes,
-                         duq_stream_t stream)
+                         duq_stream_t stream, bool staged = true)
 {
     const int32_t mode = e.mode;
     const bool asym = mode == DUQ_EPI_ASYM || mode == DUQ_EPI_ASYM_DUAL || mode >= DUQ_EPI_ASYM_ROWSUM;
@@ -143,6 +143,7 @@ int quantize_linear_impl(duq::Epilogue e, const duq_half *x, float clip, int32_t
         if (!workspace) return DUQ_E_NULL;
         if (!aligned(workspace, 16)) return DUQ_E_ALIGN;
         if (workspace_bytes < staging_bytes(mode, M, N, K)) return DUQ_E_SHAPE;
+        if (one_kernel && !staged) return launch_one();
         uint8_t *at = static_cast<uint8_t *>(workspace);
         if (!out.q) out.q = at;
         at += up16((uint64_t)M * (K / 2));
@@ -645,7 +646,7 @@ int duq_quantize_linear4bit_forward_layer(const duq_fused_layer *layer, const du
     duq::Epilogue e{l.mode,      nullptr, nullptr, l.w_scale_1,    sym ? nullptr : l.w_zeros_1, l.w_scale_2,
                     sym ? nullptr : l.w_zeros_2, l.bias,  nullptr, l.w_rowsum_adj, l.w_rowsum_adj_2};
     return quantize_linear_impl(e, x, sym ? l.clip : 1.0f, sym ? l.qmax : DUQ_QMAX_SYM_DEVICE, l.w, M, l.N, l.K, y,
-                                FusedOut{nullptr, nullptr, nullptr, nullptr}, workspace, workspace_bytes, stream);
+                                FusedOut{nullptr, nullptr, nullptr, nullptr}, workspace, workspace_bytes, stream, false);
 }
 
 int duq_static_scratch_init(void)

@@ -353,8 +353,8 @@ inline QuantGemmShape quant_gemm_shape(uint32_t M, uint32_t N, uint32_t K)
 }
 // Three and four rows of more than 2048 elements: the rows kernel, which splits a row's quantization over all its wavefronts, is ahead of the
 // tile where that quantization counts for more than the products, and where the tile is one of sixteen rows for a few.  Up to 4096 elements
-// without row sums 4096 x 3072 3.88 / 4.12 us (rows kernel / tile, three rows, symmetric, in a graph), 4096 x 4096 3.96 / 4.37, asymmetric 4.27 /
-// 4.45.  Its time over the tile's, three rows and four:
+// without row sums 4096 x 3072 3.88 / 4.12 us (rows kernel / tile, three rows, symmetric, in a graph), 4096 x 4096 3.96 / 4.37, asymmetric, four
+// rows 4.37 / 4.49.  Its time over the tile's, three rows and four:
 //  symmetric, 3000 columns: 4160 elements 1.02, 1.05; 5120 0.99, 1.04; 5632 0.94, 0.98; 6144 0.95, 0.98
 //  asymmetric, 3000 columns: 4160 0.99, 1.02; 5120 0.97, 1.01; 5632 0.96, 0.99; 6144 0.94, 0.98; 7168 0.88, 0.92
 //  row sums, 1000 columns: 5120 1.00, 1.05; 5632 0.96, 1.03; 6208 0.92, 0.97; 8192 0.93, 0.97 (four rows, 3000 columns 1.01); 13000 columns: 2560

@@ -332,7 +332,8 @@ int duq_quantize_linear4bit_forward_asym(int32_t mode, const duq_half *x, const 
  * argument).  Shapes that run as ONE launch take no workspace (NULL, 0); the others stage what the quantizer
  * launch hands to the GEMM launch in `workspace`, of duq_quantize_linear4bit_workspace_bytes(M, N, K) bytes for the
  * symmetric modes and duq_quantize_linear4bit_asym_workspace_bytes(mode, M, N, K) for the others, 16-byte aligned
- * (DUQ_E_NULL without one, DUQ_E_SHAPE for one that is too small, before anything is launched).
+ * (DUQ_E_NULL without one, DUQ_E_SHAPE for one that is too small, before anything is launched).  What it holds afterwards is not said:
+ * a shape that one kernel runs after all leaves it alone.
  *   mode  DUQ_EPI_SYM / DUQ_EPI_SYM_DUAL (clip, qmax as duq_quantize_rows_sym) or one of the asymmetric modes of
  *         duq_quantize_linear4bit_forward_asym (clip, qmax ignored); pointers a mode does not use are NULL */
 typedef struct duq_fused_layer {

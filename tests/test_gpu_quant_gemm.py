@@ -1,5 +1,7 @@
 """The kernel that quantizes its rows, multiplies and dequantizes (``csrc/duq_quant_gemm.hip``): the oracle's bits at the edges of
 its tiles, what it hands out of its quantizer, and the rule that picks its tile."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -187,3 +189,41 @@ def test_the_query_says_what_runs():
                                 (5, (3, 2049, 8192), (3, 2048, 8192))):
         assert (path(mode, *there, 0), path(mode, *beside, 0)) == (2, 1), (mode, there, beside)
     assert path(6, 3, 64, 64, 0) == path(0, 0, 64, 64, 0) == path(0, 3, 64, 96, 0) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(20, 1000, 1024), (100, 300, 4096), (300, 700, 512), (60, 12001, 512)])
+@pytest.mark.parametrize("mode", range(6))
+def test_a_layers_workspace_is_left_alone_by_the_one_kernel(hip, dev, M, N, K, mode):  # noqa: F811
+    """The workspace of duq_quantize_linear4bit_forward_layer, where nobody looks for codes, is asked for as where two launches run."""
+    from duqlinear4bitcuda_amd import _lib
+
+    lib = _lib.load()
+    assert _tile(M, N, K)[0]
+    T = lambda v: cases.t(v, dev)
+    x = T(cases.acts_outliers(M, K, seed=M) if mode in (0, 2) else cases.acts_uniform(M, K, seed=M))
+    wq, sw = (T(v) for v in cases.weights_random_nibbles(N, K, seed=5))
+    adj, s2 = torch.arange(N, dtype=torch.int32, device=dev), (sw * 2).contiguous()
+    p = lambda t, used: t.data_ptr() if used else None
+    layer = _lib.FusedLayer(mode, 1.0, 6, N, K, wq.data_ptr(), sw.data_ptr(), p(s2, mode in (1, 3, 4, 5)), p(s2, mode in (2, 3, 5)),
+                            p(sw, mode in (3, 5)), p(adj, mode >= 4), p(adj, mode == 5), None)
+    need = lib.duq_quantize_linear4bit_workspace_bytes(M, N, K) if mode in (0, 2) else \
+        lib.duq_quantize_linear4bit_asym_workspace_bytes(mode, M, N, K)
+    room = torch.full((need,), 0xA5, dtype=torch.uint8, device=dev)
+    y = torch.empty(M, N, dtype=torch.float16, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    call = lambda n: lib.duq_quantize_linear4bit_forward_layer(ctypes.addressof(layer), x.data_ptr(), M, y.data_ptr(), room.data_ptr(), n, stream)
+    assert call(need - 1) == -2 and call(need) == 0
+    torch.cuda.synchronize()
+    assert bool((room == 0xA5).all())
+    if mode in (0, 2):
+        q, s = hip.quantize_rows_sym(x)[:2]
+        want = hip.linear4bit_forward(mode, q, s, None, wq, sw, None, s2 if mode == 2 else None)
+    elif mode in (1, 3):
+        q, s, z = hip.quantize_rows_asym(x)
+        want = hip.linear4bit_forward(mode, q, s, z, wq, sw, s2, s2 if mode == 3 else None, sw if mode == 3 else None)
+    else:
+        q, s, z, r = hip.quantize_rows_asym_shifted(x)
+        want = hip.linear4bit_forward_rowsum(q, s, z, r, wq, sw, s2, adj) if mode == 4 else \
+            hip.linear4bit_forward_dual_rowsum(q, s, z, r, wq, sw, s2, s2, sw, adj, adj)
+    assert cases.bits_equal(y.cpu().numpy(), want.cpu().numpy())
