@@ -378,10 +378,29 @@ inline QuantGemmShape quant_gemm_tile(uint32_t M, uint32_t N, uint32_t K)
     if (decode_fp16in_one_launch(M, N, K)) s.eager_only = false;
     return s;
 }
+// Tiles of several chunks of columns that two launches are ahead of, for calls that bring room for the codes.  Sixteen rows of more than 2048 elements
+// (not in a recording anyway), two launches / this kernel called eagerly, us: 62 x 3467 x 2368 asymmetric 0.87 of its time, 41 x 4107 x 2304 dual row
+// sums 9.07 / 10.42, 64 x 3906 x 3200 symmetric 0.93.  Thirty-two rows, more than two groups of them and more than 256 elements (shorter ones have
+// another kernel behind the quantizer, 651 x 2334 x 192 asymmetric 9.29 / 8.02; so have up to 64 rows, 51 x 29730 x 832 13.85 / 10.13): four chunks
+// are behind where the GEMM's tiles come out even, 363 x 5035 x 576 asymmetric 9.18 / 10.33, 974 x 1824 x 640 symmetric 8.74 / 9.92, 276 x 6397 x 640 row
+// sums 9.96 / 11.14, and ahead where they do not, 143 x 12886 x 960 12.15 / 10.40; the lines are fits of both, by the model of the GEMM's tiles.  The
+// epilogue of the dual row sums takes this kernel twice as long: three chunks 498 x 2093 x 832 11.05 / 11.99, four 313 x 4875 x 640 10.59 / 13.90, but
+// where no GEMM applies it 604 x 2231 x 448 22.68 / 11.16.
+inline bool leaves_chunks(const QuantGemmShape &s, uint32_t M, uint32_t N, uint32_t K, int mode)
+{
+    if (s.chunks < 2 || decode_fp16in_one_launch(M, N, K)) return false;
+    if (s.rows == 16) return true;
+    if (s.chunks < (mode == 5 ? 3 : 4) || M <= 64 || K <= 256 || gemm_kernel_for(M, N, K) != kKernelStream ||
+        (mode == 5 && !gemm_applies_dual_rowsum(M, N, K)))
+        return false;
+    const float us = select_stream_tile(M, N, K, 1, false).us, k = (float)K / 1024.0f;
+    return us < (mode != 5 ? 2.7f : s.chunks == 3 ? 2.9f : 5.1f) + (mode != 5 ? 3.0f : 3.2f) * k;
+}
 // The same for an epilogue mode.
 inline QuantGemmShape quant_gemm_tile(uint32_t M, uint32_t N, uint32_t K, int mode)
 {
-    return leaves_few_rows(M, N, K, mode) ? QuantGemmShape{0, 0, 0} : quant_gemm_tile(M, N, K);
+    const QuantGemmShape s = quant_gemm_tile(M, N, K);
+    return leaves_few_rows(M, N, K, mode) || leaves_chunks(s, M, N, K, mode) ? QuantGemmShape{0, 0, 0} : s;
 }
 // q_out / s_out / z_out / rs_out as above.
 int launch_quant_gemm(QuantGemmShape s, const uint16_t *x, float clip, int qmax, const uint8_t *B, uint32_t M, uint32_t N, uint32_t K,

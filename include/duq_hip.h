@@ -257,8 +257,8 @@ int duq_gemm_kernel_for(uint32_t M, uint32_t N, uint32_t K);
 int duq_gemm_stream_tile_for(uint32_t M, uint32_t N, uint32_t K);
 /* The tile of the kernel that quantizes, multiplies and dequantizes in one launch, for a shape: rows of a workgroup + 256 * tiles of 16
  * columns + 65536 * chunks of those, + 2^24 where a call that is being recorded into a graph runs two launches instead.  0: the rows kernel
- * that quantizes for itself (up to eight rows), or two launches.  Some shapes of three and four rows run the rows kernel all the same, by
- * their mode: duq_quantize_linear4bit_path_for. */
+ * that quantizes for itself (up to eight rows), or two launches.  Some shapes of three and four rows run the rows kernel all the same, and
+ * some of several chunks two launches, by their mode: duq_quantize_linear4bit_path_for. */
 int duq_quant_gemm_tile_for(uint32_t M, uint32_t N, uint32_t K);
 /* What runs duq_quantize_linear4bit_forward (_asym, _layer, _static) for a mode and a shape, called eagerly or (`recorded` not 0) while a graph
  * is recorded: 1 the rows kernel that quantizes for itself, 2 the kernel of duq_quant_gemm_tile_for, 3 quantizer and GEMM; 0 for an empty
