@@ -49,6 +49,7 @@ PROTOTYPES = {
     "duq_linear4bit_forward": [_c_i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_u32, _c_u32,
                                _c_u32, _c_p, _c_p],
     "duq_linear4bit_room_bytes": [_c_i32, _c_u32, _c_u32, _c_u32],  # returns uint64_t
+    "duq_linear4bit_room_pays": [_c_i32, _c_u32, _c_u32, _c_u32],
     "duq_linear4bit_forward_room": [_c_i32] + [_c_p] * 11 + [_c_u32, _c_u32, _c_u32, _c_p, _c_p, ctypes.c_uint64, _c_p],
     "duq_product_path_for": [_c_i32, _c_u32, _c_u32, _c_u32, _c_u32, _c_i32],
     "duq_product_long_reads_for": [_c_u32, _c_u32],  # returns uint32_t

@@ -359,6 +359,11 @@ uint64_t duq_linear4bit_room_bytes(int32_t mode, uint32_t M, uint32_t N, uint32_
     return bytes <= 0x80000000ull ? bytes : 0;
 }
 
+int duq_linear4bit_room_pays(int32_t mode, uint32_t M, uint32_t N, uint32_t K)
+{
+    return duq_linear4bit_room_bytes(mode, M, N, K) != 0 && duq::shadows_are_ahead(M, N, K);
+}
+
 int duq_linear4bit_forward_room(int32_t mode, const uint8_t *xq, const duq_half *scale_x, const duq_half *zeros_x,
                                 const int32_t *rowsum_x, const uint8_t *w, const duq_half *w_scale_1, const duq_half *w_zeros_1,
                                 const duq_half *w_scale_2, const duq_half *w_zeros_2, const int32_t *w_rowsum_adj,

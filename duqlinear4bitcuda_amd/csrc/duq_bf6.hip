@@ -38,6 +38,8 @@
 // conflicts 44 -> 6 % of its cycles.  The smaller tiles are faster with their activations loaded to registers first and stored
 // a body later (2048 x 4096 x 4096 31.5 against 32.6, 505 x 8960 x 4560 36.9 / 38.8): they are asked for a chunk earlier, and
 // there the CU's intake is what is short.
+#include <algorithm>
+
 #include "duq_epilogue.h"
 #include "duq_launch.h"
 #include "duq_tiles.h"
@@ -853,6 +855,23 @@ bool pays_shadows(uint32_t M, uint32_t N, uint32_t K)
     if (M <= 1024 || K < 512 || (uint64_t)M * N < (1u << 22)) return false;
     const float pass = 2.0f + 1.25f * (float)(((double)M + N) * K * 1.7e-7);
     return plan_bf6(M, N, K, false).us + pass < 0.96f * select_stream_tile(M, N, K, 1, false).us;
+}
+
+// That rule's 0.96 holds for rows of 2600 elements and more, and for weights that the last-level cache holds beside the rest: on shorter rows the
+// 6-bit float kernel's model leaves out more of its end than the integer kernel's (measured over model 1.19 against 1.07 at 800 to 1800
+// elements), and a larger shadow comes from memory a second time.  Integer / by shadows, us: 3285 x 5068 x 1152 36.6 / 48.2, 2671 x 3584 x 1664 22.9 /
+// 29.1, 2304 x 14616 x 640 48.6 / 60.5, 2238 x 21032 x 576 53.2 / 56.2, 1489 x 25479 x 11840 325 / 373, 1253 x 23636 x 16448 348 / 410, but 5652 x 14176 x 1664
+// 167 / 130, 1663 x 10675 x 1728 53 / 42, 3882 x 21744 x 14784 931 / 688.  Of 580 shapes that the rule above takes 97 were behind by more than 2 %, by
+// this one 5 of the 394 that it leaves, 1.16 times as fast in the geometric mean (the most lost 2034 x 39106 x 6976 432 / 473); of those
+// that it gives back the most would have been 3130 x 26112 x 704 111 / 89.
+bool shadows_are_ahead(uint32_t M, uint32_t N, uint32_t K)
+{
+    if (!pays_shadows(M, N, K)) return false;
+    float margin = 1.04f;
+    if (K < 2600) margin += 0.12f * std::min(1.0f, (float)(2600 - K) / 1000.0f);
+    if ((uint64_t)N * K > 200000000ull) margin = std::max(margin, 1.12f);
+    const float pass = 2.0f + 1.25f * (float)(((double)M + N) * K * 1.7e-7);
+    return (plan_bf6(M, N, K, false).us + pass) * margin < select_stream_tile(M, N, K, 1, false).us;
 }
 
 int launch_gemm_via_shadows(const uint8_t *xq, const uint8_t *w, uint32_t M, uint32_t N, uint32_t K, const Epilogue &epi, uint16_t *y,

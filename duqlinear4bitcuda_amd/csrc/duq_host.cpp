@@ -610,7 +610,7 @@ PyObject *m_linear4(PyObject *, PyObject *const *a, Py_ssize_t n)
         Tensor y = output(*x, N, ScalarType::Half);
         const uint8_t *px = static_cast<const uint8_t *>(x->const_data_ptr()), *pw = static_cast<const uint8_t *>(w->const_data_ptr());
         const uint32_t m = static_cast<uint32_t>(M), nn = static_cast<uint32_t>(N), k = static_cast<uint32_t>(K);
-        const uint64_t bytes = shadows ? 0 : duq_linear4bit_room_bytes(mode, m, nn, k);
+        const uint64_t bytes = !shadows && duq_linear4bit_room_pays(mode, m, nn, k) ? duq_linear4bit_room_bytes(mode, m, nn, k) : 0;
         const Scratch room = g_rooms.take(dev, static_cast<int64_t>(bytes) <= most ? bytes : 0);
         int e;
         {

@@ -436,7 +436,8 @@ int launch_gemm_bf6(const uint8_t *X, const uint8_t *W, uint32_t M, uint32_t N, 
 // The same product from packed operands that come without shadows (epilogue modes 0 - 4): both are made first, in `room` of
 // shadows_bytes(M, N, K) bytes, 16-byte aligned.  Any N, K % 64 == 0, y at any address.
 uint64_t shadows_bytes(uint32_t M, uint32_t N, uint32_t K);
-bool pays_shadows(uint32_t M, uint32_t N, uint32_t K);
+bool pays_shadows(uint32_t M, uint32_t N, uint32_t K);       // by the kernels' models alone
+bool shadows_are_ahead(uint32_t M, uint32_t N, uint32_t K);  // and with what these leave out
 int launch_gemm_via_shadows(const uint8_t *xq, const uint8_t *w, uint32_t M, uint32_t N, uint32_t K, const Epilogue &epi, uint16_t *y,
                             uint8_t *room, hipStream_t stream);
 

@@ -199,11 +199,12 @@ int duq_linear4bit_forward(int32_t mode, const uint8_t *xq, const duq_half *scal
                            uint32_t M, uint32_t N, uint32_t K, duq_half *y, duq_stream_t stream);
 
 /* No counterpart in the reference.  duq_linear4bit_forward (modes 0 - 3; rowsum_x and w_rowsum_adj NULL) and
- * duq_linear4bit_forward_rowsum (DUQ_EPI_ASYM_ROWSUM), the same bits, with room for 6-bit float shadows of both operands: where
- * duq_linear4bit_room_bytes is not 0, making these and multiplying them is the faster way (prefill of some thousand rows), and
- * `room` is that many bytes of device memory, 16-byte aligned, that the caller provides and may reuse once the call's work
- * has completed on the stream.  room NULL: as without. */
+ * duq_linear4bit_forward_rowsum (DUQ_EPI_ASYM_ROWSUM), the same bits, with room for 6-bit float shadows of both operands: the call makes
+ * these and multiplies them.  `room` is duq_linear4bit_room_bytes bytes of device memory (0: a shape that takes none, and runs without),
+ * 16-byte aligned, that the caller provides and may reuse once the call's work has completed on the stream.  room NULL: as without.
+ * duq_linear4bit_room_pays: 1 where that is the faster way (prefill of some thousand rows), so that it is worth the memory, else 0. */
 uint64_t duq_linear4bit_room_bytes(int32_t mode, uint32_t M, uint32_t N, uint32_t K);
+int duq_linear4bit_room_pays(int32_t mode, uint32_t M, uint32_t N, uint32_t K);
 int duq_linear4bit_forward_room(int32_t mode, const uint8_t *xq, const duq_half *scale_x, const duq_half *zeros_x,
                                 const int32_t *rowsum_x, const uint8_t *w, const duq_half *w_scale_1, const duq_half *w_zeros_1,
                                 const duq_half *w_scale_2, const duq_half *w_zeros_2, const int32_t *w_rowsum_adj,

@@ -179,3 +179,41 @@ def test_a_layer_takes_no_more_than_it_may(dev, cls):
         assert (took >= need) == takes and (takes or took == 0), (most, took)
         want = y if want is None else want
         assert torch.equal(y.view(torch.int16), want.view(torch.int16)), most
+
+
+def _pays(mode, M, N, K):
+    from duqlinear4bitcuda_amd import _lib
+    return _lib.load().duq_linear4bit_room_pays(mode, M, N, K)
+
+
+def test_where_it_pays():
+    """Short rows and weights beyond the last-level cache have to be ahead by more."""
+    for shape in ((4096, 28672, 8192), (1999, 11008, 4096), (3072, 4096, 4096), (3679, 3712, 10240), (1663, 10675, 1728), (5652, 14176, 1664),
+                  (3882, 21744, 14784), (1553, 8561, 7936)):
+        assert _pays(0, *shape) == _pays(4, *shape) == 1, shape
+    for shape in ((3285, 5068, 1152), (2671, 3584, 1664), (2304, 14616, 640), (2238, 21032, 576), (2100, 12000, 1088), (1489, 25479, 11840),
+                  (1253, 23636, 16448), (1025, 30000, 8192)):
+        assert _room(0, *shape) and _pays(0, *shape) == 0, shape
+    assert _pays(5, 4096, 28672, 8192) == _pays(0, 1024, 28672, 8192) == _pays(0, 4096, 28672, 8200) == _pays(0, 0, 4096, 4096) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2100, 12000, 1088), (1323, 16400, 2112), (1025, 30000, 8192), (1651, 3566, 1152), (1712, 25720, 2880)])
+def test_room_that_the_caller_brings(dev, M, N, K):
+    """Whether it pays or not: the shadows' bits where the room is given."""
+    from duqlinear4bitcuda_amd import _HIP as hip
+    from duqlinear4bitcuda_amd import _lib
+    lib = _lib.load()
+    need = _room(0, M, N, K)
+    assert need
+    g = torch.Generator(device=dev).manual_seed(M)
+    a, b = (torch.randint(0, 256, (n, K // 2), dtype=torch.uint8, device=dev, generator=g) for n in (M, N))
+    s, t = (torch.rand(n, device=dev, generator=g).half() / 64 for n in (M, N))
+    room = torch.full((need,), 0xA5, dtype=torch.uint8, device=dev)
+    y = torch.empty(M, N, dtype=torch.float16, device=dev)
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib.duq_linear4bit_forward_room(0, a.data_ptr(), s.data_ptr(), None, None, b.data_ptr(), t.data_ptr(), None, None, None, None, None,
+                                           M, N, K, y.data_ptr(), room.data_ptr(), need, st) == 0
+    want = hip.linear4bit_forward(hip.EPI_SYM, a, s, None, b, t, room_bytes=0)
+    torch.cuda.synchronize()
+    assert not bool((room == 0xA5).all()) and torch.equal(y.view(torch.int16), want.view(torch.int16))
