@@ -112,6 +112,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_s4_rows_kernel(DUQ_HEAD_DECL,
     // parameters of the output this lane will finish
     // activations: lane l needs bytes [i*1024 + l*16, +16) of every row
     v4u xr[MR][XS];
+    // Four rows of 12289 to 16384 elements come out of LDS in two halves: all of them beside the weights are more than
+    // the 128 registers that sixteen wavefronts leave each, and the asymmetric quantizers spilled.  Measured (us, four
+    // rows, 4096 columns x 16384, whole against halves): Linear4bitASQ 11.2 -> 9.9, Linear4bitASQRowSum 11.4 -> 10.4,
+    // LinearQuant4bitDUASQRowSum 12.8 -> 11.1, Linear4bitSQ 9.5 -> 9.6.
+    constexpr bool kHalves = FUSEQ && MR == 4 && XS >= 8 && !MULTI;
     constexpr int WPR = WAVES / MR;           // wavefronts that share a row in the quantize phase
     constexpr int UPL = FUSEQ ? XS * MR * 4 / WAVES : 1;  // 8-element units per lane in the quantize phase
     const uint32_t qrow = wave / WPR, qpart = wave % WPR;
@@ -278,7 +283,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_s4_rows_kernel(DUQ_HEAD_DECL,
 #pragma unroll
         for (int m = 0; m < MR; ++m)
 #pragma unroll
-            for (int i = 0; i < XS; ++i) xr[m][i] = load16(xs + m * XSTRIDE + i * 1024 + lane * 16);
+            for (int i = 0; i < (kHalves ? XS / 2 : XS); ++i) xr[m][i] = load16(xs + m * XSTRIDE + i * 1024 + lane * 16);
         const uint32_t rm = min(my_m, (uint32_t)MR - 1);
         if constexpr (MODE == 5) {
             // the row record from the codes this workgroup just wrote
@@ -304,7 +309,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_s4_rows_kernel(DUQ_HEAD_DECL,
 #pragma unroll
             for (int r = 0; r < R; ++r) acc[m][r] = 0;
 #pragma unroll
-        for (int i = 0; i < XS; ++i)
+        for (int i = 0; i < XS; ++i) {
+            if (kHalves && i == XS / 2) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int m = 0; m < MR; ++m)
+#pragma unroll
+                    for (int h = XS / 2; h < XS; ++h) xr[m][h] = load16(xs + m * XSTRIDE + h * 1024 + lane * 16);
+            }
 #pragma unroll
             for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -312,6 +324,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_s4_rows_kernel(DUQ_HEAD_DECL,
 #pragma unroll
                     for (int d = 0; d < 4; ++d)
                         acc[m][r] = __builtin_amdgcn_sdot8((int)w[r][i][d], (int)xr[m][i][d], acc[m][r], false);
+        }
 
         // ---- the V sums of 64 lanes each: through this wavefront's piece of LDS (a wavefront's LDS operations
         // execute in order: no barrier), V entries per lane back, then log2(LPV) DPP steps

@@ -80,6 +80,13 @@ def test_more_long_rows(hip, dev, M, N, K):  # noqa: F811
     test_few_long_rows(hip, dev, M, N, K)
 
 
+# rows that the rows kernel takes out of LDS in two halves (K > 12288), the last one a piece, a part and the whole of its range
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(3, 37, 12352), (4, 1001, 12352), (4, 300, 14336), (3, 515, 14400), (4, 33, 16320), (4, 1030, 16384)])
+def test_rows_in_two_halves(hip, dev, M, N, K):  # noqa: F811
+    test_few_long_rows(hip, dev, M, N, K)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(20, 40, 2112), (33, 2700, 2048), (500, 2001, 960), (40, 4000, 4096)])
 def test_rows_that_are_not_finite_beside_rows_that_are(hip, dev, M, N, K):  # noqa: F811
