@@ -220,7 +220,9 @@ static TileRuns tile_runs(uint32_t batch, uint32_t M, uint32_t N)
 // layers) are ahead, asymmetric, us, two launches / this one:
 //  rows of 256 on few blocks of columns, where many workgroups quantize the same rows of B, and with wide problems, where as many do those
 //   of A: 1 x 4090 x 4096 15.7 / 16.9, 8 x 1215 x 1216 15.4 / 15.8, 1 x 2048 x 12288 22.2 / 24.6, 2 x 3000 x 11520 44.9 / 52.5, but 12 x 2046 x 2048
-//   42.1 / 39.0;
+//   42.1 / 39.0; and with up to eight problems whose tiles leave more than a quarter of one round of long runs empty (the part of the last tile of
+//   columns past N, and CUs without a run), up to twelve that leave more than 5/16: 6 x 1597 x 1600 17.1 / 18.6, 8 x 1317 x 1328 17.4 / 19.0, 4 x 1934 x
+//   3168 24.0 / 25.7, 12 x 1085 x 1088 17.1 / 18.4, but 6 x 1725 x 1728 19.2 / 18.7, 12 x 1126 x 1144 20.7 / 19.3, 7 x 1533 x 1568 19.5 / 18.6;
 //  large outputs whose rows do not begin at half lines: 32 x 2000 x 1992 x 256 94.5 / 97.7; single problems of many rows past 150 Mi outputs: 1 x 8192 x 20480 x
 //   128 69.3 / 73.0;
 //  single problems near square whose runs of three tiles (rows of 192: to five) are too few for the CUs, or just too many for one round: 1 x
@@ -237,6 +239,11 @@ bool product_tiles_takes(bool asym, uint32_t batch, uint32_t M, uint32_t N, uint
     if (blocks * ((M + 63) / 64) >= (1u << 30)) return false;
     if (K > 192 && N % 32 != 0 && (uint64_t)M * N * batch > (16u << 20)) return false;
     if (asym && K > 192 && M > 1024 && (blocks <= 40 || batch == 1 || N > 6144)) return false;
+    if (asym && K > 192 && M > 1024 && batch <= 12) {
+        const TileRuns r = tile_runs(batch, M, N);
+        const uint64_t outputs = 256ull * r.per * (64 * 256);   // of a round whose CUs all have a run of whole tiles
+        if (r.rounds == 1 && r.per >= 5 && (uint64_t)M * N * batch < outputs / 16 * (batch <= 8 ? 12 : 11)) return false;
+    }
     if (batch != 1) return true;
     if (M > 1024 && (uint64_t)M * N > (150u << 20)) return false;
     if (K <= 64 || M < 2048 || N < 2048 || !(asym || K > 192)) return true;

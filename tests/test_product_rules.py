@@ -64,6 +64,15 @@ def test_single_problems(mode, there, beside):
     assert _path(mode, 2, *beside) == (TWO if mode and beside[2] > 192 and beside[1] > 6144 else TILES)
 
 
+# several problems of rows of 256 (asymmetric): how much of a round of runs of five tiles or more is empty, by the number of problems
+@pytest.mark.parametrize("there,beside", [((6, 1725, 1728, 256), (6, 1597, 1600, 256)), ((8, 1405, 1408, 256), (8, 1400, 1400, 256)),
+                                          ((12, 1126, 1144, 256), (12, 1085, 1088, 256)), ((13, 1085, 1088, 256), (12, 1085, 1088, 256)),
+                                          ((48, 1100, 256, 256), (12, 1059, 1064, 256)), ((10, 1085, 1088, 256), (10, 1289, 1312, 256))])
+def test_several_problems(there, beside):
+    assert (_path(1, *there), _path(1, *beside)) == (TILES, TWO)
+    assert _path(0, *beside) == _path(1, *beside[:3], 192) == TILES
+
+
 def test_no_path_for_what_is_refused():
     assert [_path(m, *s) for m, s in ((2, (8, 64, 64, 64)), (1, (0, 64, 64, 64)), (1, (8, 0, 64, 64)), (1, (8, 64, 0, 64)),
                                       (1, (8, 64, 64, 0)), (1, (8, 64, 64, 96)))] == [0] * 6
