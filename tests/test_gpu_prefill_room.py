@@ -122,9 +122,12 @@ def test_short_of_memory(dev):
     torch.cuda.synchronize()
     gc.collect()
     torch.cuda.empty_cache()
+    # (what earlier tests left in use can keep a segment whose free part is as large as the room: those parts are taken first)
+    held = [torch.empty(block["size"], dtype=torch.uint8, device=dev) for segment in torch.cuda.memory_snapshot()
+            for block in segment["blocks"] if block["state"] == "inactive" and block["size"] >= out]
     free = out + need // 2   # an output, and half a room
     try:
-        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + free) / torch.cuda.get_device_properties(dev).total_memory)
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + free) / torch.cuda.mem_get_info(dev)[1])
         before = torch.cuda.memory_stats()
         for _ in range(5):
             got = None
