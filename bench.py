@@ -325,7 +325,7 @@ def decode_section(dev, quick, eager=True):
     """HBM-bound decode at configuration 2 and around it.  Per shape, HIP-graph timed, with the weights rotated
     over more than 512 MB of distinct buffers so that no launch finds its weights in a cache:
       us            binary16 activations in -> per-token quantize -> GEMM -> fp16 out, the single entry point
-                    (one launch up to eight rows and for nine to sixteen short ones, quantizer + GEMM launches above)
+                    (one launch up to eight rows and for some hundred short ones, quantizer + GEMM launches above)
       gemm_only_us  the GEMM + dequant launch alone on pre-quantized activations
       read_floor_us a kernel that only reads the same N*K/2 weight bytes with the decode access pattern
       module_graph_us  the same step through the drop-in modules, Sequential(SymQuantizer, Linear4bitSQ) on an input
@@ -338,14 +338,16 @@ def decode_section(dev, quick, eager=True):
     import torch
 
     from duqlinear4bitcuda_amd import _HIP as hip
+    from duqlinear4bitcuda_amd import _lib
     from duqlinear4bitcuda_amd.nn import Linear4bitSQ, SymQuantizer
 
+    path_for = _lib.load().duq_quantize_linear4bit_path_for
     out = []
     shapes = list(LLAMA7B_DECODE)
     if not quick:
         shapes += [(8, 4096, 4096), (32, 4096, 4096), (64, 11008, 4096), (1, 4096, 11008), (16, 4096, 11008), (1, 28672, 8192),
                    (1, 8192, 28672), (16, 28672, 8192),
-                   # sixteen rows of 2048 elements: one launch (the MFMA decode kernel quantizes the rows itself)
+                   # sixteen rows of 2048 elements: one launch
                    (16, 2048, 2048), (16, 8192, 2048)]
     for (M, N, K) in shapes:
         wbytes = N * K // 2
@@ -368,11 +370,12 @@ def decode_section(dev, quick, eager=True):
         us_mod_graph = graph_time_us([(lambda m=m: m(x3)) for m in models] * 2)
         us_mod_eager = eager_wall_us(models, x3) if eager else float("nan")
         byts = 2 * M * K + wbytes + 2 * N + 2 * M * N
+        launches = 2 if path_for(hip.EPI_SYM, M, N, K, 1) == 3 else 1   # (as recorded: some shapes are one launch only when called eagerly)
         out.append({"M": M, "N": N, "K": K, "us": round(us, 3), "GBps": round(byts / us / 1e3, 1),
                     "frac_hbm": round(byts / us / 1e3 / PEAK_HBM_GBS, 4),
-                    "launches": 1 if hip.quantize_linear4bit_one_launch(M, N, K) else 2,
+                    "launches": launches,
                     "module_graph_us": round(us_mod_graph, 3), "module_eager_us": round(us_mod_eager, 3) if eager else None,
-                    "module_launches": 1 if hip.quantize_linear4bit_one_launch(M, N, K) else 2,
+                    "module_launches": launches,
                     "module_library_calls": 1 if M <= 1024 else 2,
                     "gemm_only_us": round(us_gemm, 3),
                     "gemm_only_GBps": round((byts - 2 * M * K + M * K // 2 + 2 * M) / us_gemm / 1e3, 1),
@@ -794,8 +797,8 @@ def main():
     stack = None if args.quick or args.no_harness else stack_section(dev)
     rows_7b = [d for d in decode if (d["M"], d["N"], d["K"]) in LLAMA7B_DECODE]
     worst = min(rows_7b, key=lambda d: d["frac_hbm"])
-    roofline_decode = {"bound": "hbm", "kernel": "gemv_s4_rows_kernel (M <= 8, quantizer inside) / quantize_rows_kernel + "
-                                                 "gemm_s4_lds_kernel (N <= 4096), gemm_s4_decode_kernel (wider)",
+    roofline_decode = {"bound": "hbm", "kernel": "gemv_s4_rows_kernel (M <= 4, quantizer inside) / quant_gemm_s4_kernel (M = 16, N = 4096, "
+                                                 "likewise) / quantize_rows_kernel + gemm_s4_decode_kernel (N = 11008)",
                        "what": "worst of the Llama-2-7B decode rows (M in {1,4,16}, K=4096, N in {4096,11008}), binary16 "
                                "activations in, quantize + GEMM + dequant, weights never in a cache",
                        "achieved": worst["GBps"], "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": worst["frac_hbm"],

@@ -515,8 +515,9 @@ def quantize_linear4bit_forward(x, w, w_scale_1, w_scale_2=None, bias=None, clip
                                 return_quantized: bool = False, static: bool = False, slot: int = 0):
     """SymQuantizer + Linear4bitSQ / Linear4bitDUSQ forward (qlinear4bit/nn/quantizer.py:10-16,
     qlinear4bit/nn/linear.py:42-56, 167-176) from binary16 activations ``x`` [..., K]: bit-identical to
-    ``quantize_rows_sym`` followed by ``linear4bit_forward``.  Up to eight rows (and nine to sixteen that hold at
-    most 32768 elements together) are ONE launch; larger inputs run the two launches with the codes staged in a buffer allocated here.  With
+    ``quantize_rows_sym`` followed by ``linear4bit_forward``.  Up to eight rows, and more short ones while their tiles are
+    one round of workgroups, are ONE launch; larger inputs run the two launches, with the codes staged in a buffer allocated here (some of
+    the shapes of one launch, too, leave them there).  With
     ``return_quantized`` also returns (codes uint8 [..., K/2], scales [..., 1]).  ``static=True`` stages in the
     library's static device array instead (``duq_quantize_linear4bit_forward_static``: nothing but the outputs is
     allocated; M * K / 2 <= 8 MiB; calls that may overlap on one GPU must name different ``slot``s, 0..3)."""
@@ -573,7 +574,7 @@ def quantize_linear4bit_forward_asym(mode, x, w, w_scale_1, w_zeros_1, w_scale_2
     (``mode`` EPI_ASYM_ROWSUM with ``w_rowsum_adj``, or EPI_ASYM_DUAL_ROWSUM with ``w_rowsum_adj`` /
     ``w_rowsum_adj_2`` for the dual-uniform layer: the signed-shifted quantizer): bit-identical to
     ``quantize_rows_asym`` (``quantize_rows_asym_shifted``) followed by ``linear4bit_forward``
-    (``linear4bit_forward_rowsum`` / ``linear4bit_forward_dual_rowsum``).  Up to eight rows (sixteen short ones) are
+    (``linear4bit_forward_rowsum`` / ``linear4bit_forward_dual_rowsum``).  Up to eight rows and some hundred short ones are
     ONE launch; larger inputs run the two launches with the
     codes staged in a buffer allocated here.  With ``return_quantized`` also returns (codes, scales [..., 1],
     zeros [..., 1][, rowsum [...]])."""
@@ -710,13 +711,13 @@ class FusedDecode:
             ref = self._structs[key] = (ctypes.addressof(st), st)   # (the struct is kept alive beside its address)
         return ref[0]
 
-    # Rows up to which a module hands binary16 activations to this call.  Up to eight rows, sixteen short ones, it is one
+    # Rows up to which a module hands binary16 activations to this call.  Up to eight rows, and for some hundred short ones, it is one
     # launch; above, the quantizer launch and the GEMM launch of one library call: up to about 700 rows (N = K = 4096)
     # the two kernels take less time than two calls cost on the host (23 us).
     max_rows = 1024
 
     def _staging(self, M: int) -> int:
-        """Bytes the library stages between its two launches at M rows (0: one launch); -1 when M is out of range."""
+        """Bytes the library stages between its two launches at M rows (0: needs no workspace); -1 when M is out of range."""
         b = self._one.get(M)
         if b is None:
             if not 0 < M <= self.max_rows:
@@ -1240,7 +1241,7 @@ def linear8bit_forward(xq, scale_x, zeros_x, w, w_scale, w_zeros, bias=None, til
 
 def quantize_linear8bit_forward(x, w, w_tiled, w_scale, w_zeros, bias=None):
     """AsymQuantizer8bit + linear8bit_forward in one library call (one launch up to eight rows of at most 4096
-    elements, else two, the codes staged in a workspace allocated here): x float32 [..., K] -> float32 [..., N], the bits of the two calls.  ``w`` the weight [N, K]
+    elements and more while their tiles are one round of workgroups, else two, the codes staged in a workspace allocated here): x float32 [..., K] -> float32 [..., N], the bits of the two calls.  ``w`` the weight [N, K]
     int8, ``w_tiled`` its tiled copy from weight_tile_8bit or None."""
     name = "quantize_linear8bit_forward"
     if type(x) is torch.Tensor and x.is_cuda and type(w) is torch.Tensor and w.dim() == 2:

@@ -3,7 +3,7 @@
 // A workgroup quantizes the rows of its tile itself, through the same RowQuant code as the stand-alone quantizer (scale:
 // qlinear4bit/nn/quantizer.py:13, codes: src/kernels/quant.cu:11-45, :99-132), while its whole share of the weights comes to LDS.
 // As two launches a step of few or short rows cost 8.2 us of host time, and in a graph 4.7 at least, more than its work: 46 rows 1231 x
-// 1216 9.2 -> 6.4 called eagerly, 5.0 -> 3.9 in a graph.  What bounds it: every workgroup repeats the quantizer's vector work for its
+// 1216 8.3 -> 5.7 called eagerly, 5.6 -> 4.3 in a graph.  What bounds it: every workgroup repeats the quantizer's vector work for its
 // rows, about 31 instructions per eight elements (2.2 us for the 65536 elements a workgroup can have), behind one trip to memory
 // and its fetch of the rows (128 KB there, 1.2 us); then the launch.  So a tile is as few rows as one round of workgroups allows.
 #include "duq_decode_common.h"

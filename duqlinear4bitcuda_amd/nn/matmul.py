@@ -3,7 +3,8 @@
 int4 x int4 and dequantized.  Rows of ``B`` play the part of weight rows: the result is
 ``A @ B^T`` over the last dimension.
 
-A whole batch runs as ONE fused GEMM + dequant launch, whatever the number of batch entries
+A whole batch runs as ONE fused GEMM + dequant launch behind one that quantizes, whatever the number of batch entries, or
+as one or two that quantize where they multiply (rows of up to 256 elements, one row per entry, long rows and few columns)
 (the reference runs a GEMM per batch entry into a zero-filled int32 tensor, pads B's rows to a
 multiple of 32, then one batched dequant: matmul.py:46-63); the bits are the same.  With
 ``fused = False`` the steps are the reference's: one batched GEMM launch into int32, one

@@ -224,9 +224,9 @@ int duq_batch_linear4bit_forward(int32_t mode, const uint8_t *xq, const duq_half
                                  duq_stream_t stream);
 
 /* The whole forward of AsymQuantMatMul (mode DUQ_EPI_ASYM) and SymQuantMatMul (DUQ_EPI_SYM): both operands quantized per
- * row, in one launch unless the symmetric settings of the two differ, then duq_batch_linear4bit_forward (M = 1, N <= 2^24, K <= 4096,
- * and most shapes of K <= 256: all of it in one launch that leaves the workspace alone; a launch for
- * b and one for the rest where N <= 256 and b is the smaller part); the same bits as those steps (qlinear4bit/nn/matmul.py:38-63, 78-84).
+ * row, in one launch unless the symmetric settings of the two differ, then duq_batch_linear4bit_forward; the same bits as those steps
+ * (qlinear4bit/nn/matmul.py:38-63, 78-84).  All of it in one launch that leaves the workspace alone: M = 1 (N <= 2^24, K <= 4096), and most
+ * shapes of K <= 256.  A launch for b and one for the rest: many shapes of 256 < K <= 4096, N <= 256.  duq_product_path_for says which.
  *   a [batch_count, M, K], b [batch_count, N, K] fp16, 16-byte aligned, K % 64 == 0;  y [batch_count, M, N] fp16
  *   clip, qmax   settings of the symmetric quantizers (not read by DUQ_EPI_ASYM, qmax has to be valid)
  *   workspace    duq_quantize_product_workspace_bytes(...) bytes, 16-byte aligned */
@@ -292,11 +292,13 @@ int duq_probe_read(const void *src, uint64_t bytes, uint32_t *sink, duq_stream_t
  * Up to four rows (K <= 16384, N * K / 2 < 2^32 - 256; from two rows on K <= 8192 or N <= 16384), five to eight rows
  * of at most 4096 elements (8192 with N <= 4096) and nine to sixteen rows that hold at most 32768 elements together (40960
  * with N <= 4096; K <= 4096, N <= 16384) run as ONE launch: every workgroup quantizes the rows itself while its
- * weights are in flight, and `workspace` is not touched.  Any other shape runs two launches
- * (quantizer, then GEMM) and stages the codes and scales in `workspace`, device memory of at least
- * duq_quantize_linear4bit_workspace_bytes(M, N, K) bytes (0 for the one-launch shapes), 16-byte aligned, that the
- * caller provides and may reuse once the call's work has completed on the stream (DUQ_E_NULL / DUQ_E_SHAPE if it
- * is missing or too small; codes and scales go to q_out / scale_out instead when both are given). */
+ * weights are in flight, and `workspace` is not touched.  Any other shape stages the codes and scales in `workspace`,
+ * device memory of at least duq_quantize_linear4bit_workspace_bytes(M, N, K) bytes (0 for the shapes above), 16-byte
+ * aligned, that the caller provides and may reuse once the call's work has completed on the stream (DUQ_E_NULL /
+ * DUQ_E_SHAPE if it is missing or too small; codes and scales go to q_out / scale_out instead when both are given).
+ * It runs two launches (quantizer, then GEMM), or, where its tiles are one round of workgroups (some hundred rows of up to
+ * 1024 elements, fewer longer ones up to 8192: duq_quant_gemm_tile_for, duq_quantize_linear4bit_path_for), one that
+ * leaves the same codes and scales there. */
 uint64_t duq_quantize_linear4bit_workspace_bytes(uint32_t M, uint32_t N, uint32_t K);
 int duq_quantize_linear4bit_forward(int32_t mode, const duq_half *x, float clip, int32_t qmax, const uint8_t *w,
                                     const duq_half *w_scale_1, const duq_half *w_scale_2, const duq_half *bias,
@@ -313,9 +315,9 @@ int duq_quantize_linear4bit_forward(int32_t mode, const duq_half *x, float clip,
  *        DUQ_EPI_ASYM_DUAL_ROWSUM  duq_quantize_rows_asym_shifted, then duq_linear4bit_forward_dual_rowsum
  *                           (w_rowsum_adj = its w_adj_1, w_rowsum_adj_2 = its w_adj_2)
  *   q_out [M,K/2], scale_out [M], zeros_out [M], rowsum_out [M] (row-sum modes): optional (NULL)
- * The shapes that run as ONE launch are those of duq_quantize_linear4bit_forward; the others run quantizer + GEMM
- * and stage codes, scales, zero points (and row sums; in the dual-uniform row-sum mode also the int32 accumulators,
- * for shapes whose GEMM cannot apply that epilogue itself) in `workspace`
+ * The shapes that need no workspace are those of duq_quantize_linear4bit_forward; the others, in two launches or one,
+ * stage codes, scales, zero points (and row sums; in the dual-uniform row-sum mode there is also room for the int32
+ * accumulators, for shapes whose GEMM cannot apply that epilogue itself) in `workspace`
  * (duq_quantize_linear4bit_asym_workspace_bytes(mode, M, N, K) bytes, 16-byte aligned; whatever the caller's own
  * output pointers cover is written there instead). */
 uint64_t duq_quantize_linear4bit_asym_workspace_bytes(int32_t mode, uint32_t M, uint32_t N, uint32_t K);
@@ -330,8 +332,8 @@ int duq_quantize_linear4bit_forward_asym(int32_t mode, const duq_half *x, const 
 /* The two entry points above with the layer's side of the arguments in a struct the caller fills once per layer
  * (no counterpart in the reference): a decode step then passes seven arguments instead of seventeen to twenty, which
  * is what a step costs on the host when it goes through a foreign-function interface (ctypes: about 0.1 us per
- * argument).  Shapes that run as ONE launch take no workspace (NULL, 0); the others stage what the quantizer
- * launch hands to the GEMM launch in `workspace`, of duq_quantize_linear4bit_workspace_bytes(M, N, K) bytes for the
+ * argument).  Shapes for which the query says 0 take no workspace (NULL, 0); the others need one for what the quantizer
+ * launch hands to the GEMM launch, of duq_quantize_linear4bit_workspace_bytes(M, N, K) bytes for the
  * symmetric modes and duq_quantize_linear4bit_asym_workspace_bytes(mode, M, N, K) for the others, 16-byte aligned
  * (DUQ_E_NULL without one, DUQ_E_SHAPE for one that is too small, before anything is launched).  What it holds afterwards is not said:
  * a shape that one kernel runs after all leaves it alone.
@@ -539,7 +541,8 @@ int duq_quant_gemm8_tile_for(uint32_t M, uint32_t N, uint32_t K);
 /* No counterpart in the reference: LinearQuant8bitASQ.forward with its own quantizer (qlinear4bit/nn/linear.py:323-335)
  * in one call: duq_quantize_rows_asym_8bit into `workspace`, then duq_linear8bit_forward(_tiled) on it; the same
  * bits as the two calls.  x [M,K] float32, 16-byte aligned, K % 32 == 0; w the weight as stored and / or w_tiled its
- * tiled copy (one may be NULL).  Up to eight rows of at most 4096 elements are one launch, which quantizes the rows itself and
+ * tiled copy (one may be NULL).  Up to eight rows of at most 4096 elements, and more rows of that length where their tiles are
+ * one round of workgroups (duq_quant_gemm8_tile_for), are one launch, which quantizes the rows itself and
  * reads w_tiled when it is given (up to four rows with both: when w_tiled is 16-byte aligned, else w); up to two rows of
  * 4097..8192 elements read w when it is given; everything else reads w_tiled when it is given.  What is read has to be 16-byte
  * aligned; so has w where up to four rows (two above 4096 elements) come with both.  workspace:
